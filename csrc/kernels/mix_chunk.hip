@@ -1,0 +1,668 @@
+// Linear recurrences with a decay per key channel (wkv, gated linear attention, gated delta rule:
+// mix_wkv.hip and mix_linrec.hip have their definitions) in chunks of 16 tokens on fp32 MFMA tiles.
+//
+// With D_t = diag(a_t), inside a chunk that starts from the state S,
+//
+//   o_t = Qd_t S + sum_{s<=t} A[t,s] u_s          Qd_t = q_t a_1 .. a_t
+//   S  <- a_1 .. a_16 S + sum_s Kd_s u_s          Kd_s = k_s a_{s+1} .. a_16
+//   A[t,s] = sum_c q_t[c] k_s[c] (a_{s+1} .. a_t)[c]
+//
+// (wkv reads before it writes: its products of q end at a_{t-1}, and A[t,t] = sum_c q u k.)  Without
+// the delta rule u_s = v_s.  With it U = T (beta (V - Kk S)), Kk_t = k_t a_1 .. a_t, T the inverse
+// of the unit lower triangle I + beta A_kk, A_kk[t,s] = sum_c k_t k_s a_{s+1} .. a_t for s < t.
+// All decay products are running products of the decays themselves: no logarithm, no quotient, so
+// nothing overflows and nothing cancels however strong the decay.  Pairs of different four-token
+// blocks factor at the block's edge: (a_{block} .. a_t) from the reader's side, (a_{s+1} ..) from
+// the writer's, both at most 1; pairs inside a block multiply their decays directly.
+//
+// What bounds it: the chain over a run's chunks, and inside a chunk the instructions of the waves
+// that share a SIMD.  Token by token the chain was 0.2 - 2.6 us a token (LDS round trips, 64 x 64
+// FMAs on one or four waves); here a chunk's chain is 36 (wkv, gla) or 56 (delta) MFMAs of 16x16x4
+// per wave, 1.4 - 2.1 us.  One workgroup per (run, head, 64 value channels): four consumer waves hold
+// 64 x 16 of the state in accumulators, which are MFMA operands as they lie (a lane holds channels
+// 16 i + 4 grp + r of its column: exactly the K slices that step (i, r) of Qd S takes); the other
+// waves work ahead: decays and their products for chunk c + 3, A for chunk c + 2, T for chunk c + 1,
+// wkv's norm and gate for chunk c - 1; one barrier per chunk.  A state operand never leaves the
+// registers, an fp32 operand is never narrowed.  Measured, two runs of 2,048 tokens in bf16: wkv with
+// 64 heads of 64 x 64 5,353 -> 180 us; delta rule with 32 heads of 64 x 128 741 (decays and scan) ->
+// 277 us; gla in fp32, five ragged runs of up to 1,031, 32 heads, 447 -> 117 us.
+#include <algorithm>
+#include <type_traits>
+
+#include "common.h"
+#include "mix_common.h"
+#include "mix_chunk.h"
+
+namespace rfqmix {
+
+using rfq::f32x4;
+
+namespace {
+constexpr int CT = 16;                  // tokens per chunk
+constexpr int NC = kChunkDim;           // key channels (those past dim are zeros)
+constexpr int RS = NC + 4;              // floats per token row in LDS
+constexpr int TS = CT + 4;              // floats per row of a 16 x 16 tile, of Kd^T
+
+// four consumers, four waves for the decays, four for A (and T), wkv: four for norm and gate
+constexpr int chunk_threads(int mode) { return mode == kChunkWkv ? 1024 : 768; }
+
+__device__ __forceinline__ float ror_add(float v) {   // sum over the 16 lanes of a row
+  v += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x128, 0xf, 0xf, true));
+  v += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x124, 0xf, 0xf, true));
+  v += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x122, 0xf, 0xf, true));
+  v += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x121, 0xf, 0xf, true));
+  return v;
+}
+// What a chunk's producers leave in LDS.
+template <int MODE>
+struct ChunkLds {
+  static constexpr bool DELTA = MODE == kChunkDelta;
+  float qd[4][CT * RS];                 // four chunks in flight between producers and consumers
+  float kk[DELTA ? 4 : 1][DELTA ? CT * RS : 4];
+  float kd[4][NC * TS];                 // Kd^T
+  float dec[4][NC];
+  float beta[4][CT];
+  float aq[4][CT * TS];
+  float ak[2][DELTA ? CT * TS : 4];
+  float tt[2][DELTA ? CT * TS : 4];
+  float q[2][CT * RS], k[2][CT * RS], a[2][CT * RS];      // operands of A: raw,
+  float ql[2][CT * RS], kl[2][CT * RS];                   // times the block's products up to / after
+  float kb[2][DELTA ? CT * RS : 4];
+  float blk[2][4 * NC];                 // product of a block's decays
+  float o[2][MODE == kChunkWkv ? CT * RS : 4];
+};
+
+__device__ __forceinline__ float4 mul4(float4 x, float4 y) {
+  return make_float4(x.x * y.x, x.y * y.y, x.z * y.z, x.w * y.w);
+}
+__device__ __forceinline__ float dot4(float4 x, float4 y) {
+  return x.x * y.x + x.y * y.y + x.z * y.z + x.w * y.w;
+}
+// exp(x) and log(1 + e^-|y|) on the transcendental unit (v_exp_f32, v_log_f32: about one unit in the
+// last place of base 2); log(1 + e) / ((1 + e) - 1) e keeps small e exact
+__device__ __forceinline__ float exp_c(float x) { return __builtin_amdgcn_exp2f(x * 1.44269504088896f); }
+__device__ __forceinline__ float softplus_c(float y) {
+  const float e = exp_c(-fabsf(y)), w = 1.f + e, d = w - 1.f;
+  const float l = __builtin_amdgcn_logf(w) * 0.693147180559945f * (e * __builtin_amdgcn_rcpf(d));
+  return fmaxf(y, 0.f) + (d == 0.f ? e : l);
+}
+__device__ __forceinline__ float sigmoid_c(float x) { return __builtin_amdgcn_rcpf(1.f + exp_c(-x)); }
+
+// An operand in flight across a turn of the loop: its bits as loaded.  `arrived` converts it where it
+// stands: left to the compiler, the conversion moves to the end of the turn that loaded it, or past
+// the next load into the same register, and either way the wave waits there for memory.
+template <typename T>
+__device__ __forceinline__ T load_at(const T* base, uint32_t bytes) {
+  return *reinterpret_cast<const T*>(reinterpret_cast<const char*>(base) + bytes);
+}
+__device__ __forceinline__ float arrived(float bits) {
+  float f;
+  asm volatile("v_mov_b32 %0, %1" : "=v"(f) : "v"(bits));
+  return f;
+}
+__device__ __forceinline__ float arrived(bf16_t bits) {
+  float f;
+  asm volatile("v_lshlrev_b32 %0, 16, %1" : "=v"(f) : "v"(bits));
+  return f;
+}
+__device__ __forceinline__ float4 ld4(const float* p) { return *reinterpret_cast<const float4*>(p); }
+}  // namespace
+
+namespace {
+__device__ __forceinline__ bool finite4(const f32x4& x) {      // no infinity, no NaN among them
+  return fabsf((fabsf(x[0]) + fabsf(x[1])) + (fabsf(x[2]) + fabsf(x[3]))) < __builtin_huge_valf();
+}
+
+// o[t] += sum_{s<=t} m[t][s] x[s] with the pairs s > t left out instead of multiplied by zero: a
+// token's infinity or NaN stays out of the tokens before it.  (Also taken, with the same result,
+// where the sum of four finite values overflows.)
+__device__ __forceinline__ void lower_product(const float* m, const f32x4& x, int col, int grp, f32x4& o) {
+#pragma unroll 1
+  for (int b = 0; b < 4; ++b) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int s = 4 * b + e;
+      const float xs = __shfl(x[e], 16 * b + col, 64);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const float y = o[r] + m[(4 * grp + r) * TS + s] * xs;
+        o[r] = s <= 4 * grp + r ? y : o[r];
+      }
+    }
+  }
+}
+}  // namespace
+
+template <typename TI, typename TG, int MODE>
+__global__ __launch_bounds__(chunk_threads(MODE)) void chunk_recurrence_kernel(const ChunkArgs a) {
+  constexpr bool WKV = MODE == kChunkWkv, DELTA = MODE == kChunkDelta;
+  const int h = blockIdx.y;
+  const int tid = threadIdx.x, lane = tid & 63, col = lane & 15, grp = lane >> 4;
+  int t0 = -1;
+  if (a.min_run <= 1) {
+    t0 = a.run_rows[blockIdx.x];
+  } else {                     // the step's runs of min_run rows or more, counted by every wave for itself
+    int left = blockIdx.x;
+    for (int base = 0; base < a.runs; base += 64) {
+      const int r = base + lane < a.runs ? a.run_rows[base + lane] : -1;
+      const bool fits = r >= 0 && a.row_back[r] == 0 && a.row_fwd[r] + 1 >= a.min_run;
+      uint64_t m = __builtin_amdgcn_ballot_w64(fits);
+      const int c = __builtin_popcountll(m);
+      if (left < c) {
+        for (; left > 0; --left) m &= m - 1;
+        t0 = __builtin_amdgcn_readfirstlane(__shfl(r, __builtin_ctzll(m), 64));
+        break;
+      }
+      left -= c;
+    }
+  }
+  if (t0 < 0 || a.row_back[t0] != 0) return;
+  const int n = a.row_fwd[t0] + 1, nc = (n + CT - 1) / CT;
+  const int code = a.row_state[t0];
+  const int H = a.H, dim = a.dim, vdim = a.vdim;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int role = wave >> 2, w = wave & 3;               // 0 consumers, 1 decays, 2 A and T, 3 wkv's norm and gate
+
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  ChunkLds<MODE>& L = *reinterpret_cast<ChunkLds<MODE>*>(smem);
+  for (int x = tid; x < 4 * CT * TS; x += chunk_threads(MODE)) (&L.aq[0][0])[x] = 0.f;    // pairs s > t stay zero
+  if constexpr (DELTA)
+    for (int x = tid; x < 2 * CT * TS; x += chunk_threads(MODE)) {
+      (&L.ak[0][0])[x] = 0.f;
+      (&L.tt[0][0])[x] = 0.f;
+    }
+
+  // Row offsets inside a chunk in bytes (the launcher bounds 16 rows by 2^31); a chunk's first row
+  // is a wave-uniform pointer.  Rows past the run's end are read as its last row and left out later.
+  auto offsets = [&](uint32_t (&o)[4], int64_t stride, int first, int esz, int c) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) o[i] = (uint32_t)min(first + i, n - 1 - c * CT) * (uint32_t)(stride * esz);
+  };
+  // ---- consumers: 16 value channels, S[16 i + 4 grp + r][column]
+  const int vcol = (int)blockIdx.z * 64 + 16 * w + col;
+  const bool vlive = vcol < vdim;
+  const bool from_state = code >= 0 && a.pos[t0] > 0;
+  const int64_t hsz = (int64_t)dim * vdim;
+  f32x4 st[4];
+  TI vreg[4];
+  uint32_t vo[4];
+  const TI* vb = static_cast<const TI*>(a.v) + t0 * a.vs + (int64_t)h * vdim;
+  auto fetch_v = [&](int c) {
+    if (c * CT + CT > n) offsets(vo, a.vs, 4 * grp, sizeof(TI), c);   // the last, partial chunk
+    const TI* base = vb + (int64_t)c * CT * a.vs;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) vreg[r] = load_at(base, vo[r] + (uint32_t)(min(vcol, vdim - 1) * sizeof(TI)));
+  };
+  // ---- producers: a lane has four tokens of one key channel
+  const int ch = 16 * w + col, chl = min(ch, dim - 1);
+  const bool klive = ch < dim;
+  const int hq = h / a.rep;
+  typedef typename std::conditional<WKV, TI, float>::type TZ;
+  TI rq[4], rk[4];
+  TZ rz[4];
+  TG rb{};
+  TI rg[4] = {};                                          // wkv: four channels' gates of one token
+  uint32_t qo[4], ko[4], zo[4];
+  const TI* qb = static_cast<const TI*>(a.q) + t0 * a.qs + (int64_t)hq * dim;
+  const TI* kb = static_cast<const TI*>(a.k) + t0 * a.ks + (int64_t)hq * dim;
+  const TZ* zb = static_cast<const TZ*>(a.z) + t0 * a.zs + (int64_t)h * dim;
+  const TG* bb = DELTA ? static_cast<const TG*>(a.beta) + t0 * a.bs + h : nullptr;
+  const TI* gb = WKV ? static_cast<const TI*>(a.gate) + t0 * a.gs + (int64_t)h * vdim : nullptr;
+  auto fetch = [&](int c) {
+    if (c * CT + CT > n) {
+      offsets(qo, a.qs, 4 * grp, sizeof(TI), c);
+      offsets(ko, a.ks, 4 * grp, sizeof(TI), c);
+      offsets(zo, a.zs, 4 * grp, sizeof(TZ), c);
+    }
+    const TI *q = qb + (int64_t)c * CT * a.qs, *k = kb + (int64_t)c * CT * a.ks;
+    const TZ* z = zb + (int64_t)c * CT * a.zs;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      rq[i] = load_at(q, qo[i] + (uint32_t)(chl * sizeof(TI)));
+      rk[i] = load_at(k, ko[i] + (uint32_t)(chl * sizeof(TI)));
+      rz[i] = load_at(z, zo[i] + (uint32_t)(chl * sizeof(TZ)));
+    }
+    if constexpr (DELTA) rb = load_at(bb + (int64_t)min(c * CT + col, n - 1) * a.bs, 0);
+  };
+  float4 nw = {}, bonus = {};
+  float zbias = 0.f, rate = 0.f;
+
+  if (role == 0) {
+    offsets(vo, a.vs, 4 * grp, sizeof(TI), 0);
+    const float* rd = a.state + (((int64_t)(code & 1) * a.slots + (code >> 1)) * H + h) * hsz;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int c = 16 * i + 4 * grp + r;
+        st[i][r] = (from_state && vlive && c < dim) ? rd[(int64_t)c * vdim + vcol] : 0.f;
+      }
+    fetch_v(0);
+  } else if (role == 1) {
+    offsets(qo, a.qs, 4 * grp, sizeof(TI), 0);
+    offsets(ko, a.ks, 4 * grp, sizeof(TI), 0);
+    offsets(zo, a.zs, 4 * grp, sizeof(TZ), 0);
+    fetch(0);
+    zbias = a.zbias[h * dim + chl];
+    if constexpr (!WKV) rate = a.rate[h];
+  } else if constexpr (WKV) {
+    const float *np = a.norm_w + h * NC + 4 * col, *up = a.u + h * NC + 4 * col;
+    nw = make_float4(np[0], np[1], np[2], np[3]);
+    bonus = make_float4(up[0], up[1], up[2], up[3]);
+  }
+  __syncthreads();
+
+  // The kinds of wave run loops of their own with the same number of barriers.
+  const int turns = nc + (WKV ? 1 : 0);                   // and three turns ahead of them
+  if (role == 0) {
+    for (int i = 0; i < 3; ++i) __syncthreads();
+    // The operands of the next chunk are there a turn ahead: they are read into registers behind the
+    // products that use the present ones.
+    float4 qa[4], ka[DELTA ? 4 : 1], kh[4], dc[4], aa;
+    auto queries = [&](int b) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        qa[i] = ld4(&L.qd[b][col * RS + 16 * i + 4 * grp]);
+        if constexpr (DELTA) ka[i] = ld4(&L.kk[b][col * RS + 16 * i + 4 * grp]);
+      }
+    };
+    auto keys = [&](int b) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        kh[i] = ld4(&L.kd[b][(16 * i + col) * TS + 4 * grp]);
+        dc[i] = ld4(&L.dec[b][16 * i + 4 * grp]);
+      }
+      aa = ld4(&L.aq[b][col * TS + 4 * grp]);
+    };
+    queries(0);
+    keys(0);
+    for (int it = 0; it < nc; ++it) {
+      const int b = it & 3;
+      float v[4];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) v[r] = arrived(vreg[r]);
+      fetch_v(min(it + 1, nc - 1));
+      if (!vlive || it * CT + CT > n) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) v[r] = vlive && it * CT + 4 * grp + r < n ? v[r] : 0.f;
+      }
+      f32x4 o = (f32x4){0.f, 0.f, 0.f, 0.f}, u;
+      if constexpr (DELTA) {
+        const float4 bt = ld4(&L.beta[b][4 * grp]), ta = ld4(&L.tt[it & 1][col * TS + 4 * grp]);
+        f32x4 y = (f32x4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          y = __builtin_amdgcn_mfma_f32_16x16x4f32(ka[i].x, st[i][0], y, 0, 0, 0);
+          o = __builtin_amdgcn_mfma_f32_16x16x4f32(qa[i].x, st[i][0], o, 0, 0, 0);
+          y = __builtin_amdgcn_mfma_f32_16x16x4f32(ka[i].y, st[i][1], y, 0, 0, 0);
+          o = __builtin_amdgcn_mfma_f32_16x16x4f32(qa[i].y, st[i][1], o, 0, 0, 0);
+          y = __builtin_amdgcn_mfma_f32_16x16x4f32(ka[i].z, st[i][2], y, 0, 0, 0);
+          o = __builtin_amdgcn_mfma_f32_16x16x4f32(qa[i].z, st[i][2], o, 0, 0, 0);
+          y = __builtin_amdgcn_mfma_f32_16x16x4f32(ka[i].w, st[i][3], y, 0, 0, 0);
+          o = __builtin_amdgcn_mfma_f32_16x16x4f32(qa[i].w, st[i][3], o, 0, 0, 0);
+        }
+        const f32x4 x = {bt.x * (v[0] - y[0]), bt.y * (v[1] - y[1]), bt.z * (v[2] - y[2]), bt.w * (v[3] - y[3])};
+        u = (f32x4){0.f, 0.f, 0.f, 0.f};
+        if (__builtin_amdgcn_ballot_w64(!finite4(x)) == 0ull) {
+          u = __builtin_amdgcn_mfma_f32_16x16x4f32(ta.x, x[0], u, 0, 0, 0);
+          u = __builtin_amdgcn_mfma_f32_16x16x4f32(ta.y, x[1], u, 0, 0, 0);
+          u = __builtin_amdgcn_mfma_f32_16x16x4f32(ta.z, x[2], u, 0, 0, 0);
+          u = __builtin_amdgcn_mfma_f32_16x16x4f32(ta.w, x[3], u, 0, 0, 0);
+        } else {
+          lower_product(L.tt[it & 1], x, col, grp, u);
+        }
+      } else {
+        f32x4 o2 = (f32x4){0.f, 0.f, 0.f, 0.f};           // two independent chains
+#pragma unroll
+        for (int i = 0; i < 4; i += 2) {
+          o = __builtin_amdgcn_mfma_f32_16x16x4f32(qa[i].x, st[i][0], o, 0, 0, 0);
+          o2 = __builtin_amdgcn_mfma_f32_16x16x4f32(qa[i + 1].x, st[i + 1][0], o2, 0, 0, 0);
+          o = __builtin_amdgcn_mfma_f32_16x16x4f32(qa[i].y, st[i][1], o, 0, 0, 0);
+          o2 = __builtin_amdgcn_mfma_f32_16x16x4f32(qa[i + 1].y, st[i + 1][1], o2, 0, 0, 0);
+          o = __builtin_amdgcn_mfma_f32_16x16x4f32(qa[i].z, st[i][2], o, 0, 0, 0);
+          o2 = __builtin_amdgcn_mfma_f32_16x16x4f32(qa[i + 1].z, st[i + 1][2], o2, 0, 0, 0);
+          o = __builtin_amdgcn_mfma_f32_16x16x4f32(qa[i].w, st[i][3], o, 0, 0, 0);
+          o2 = __builtin_amdgcn_mfma_f32_16x16x4f32(qa[i + 1].w, st[i + 1][3], o2, 0, 0, 0);
+        }
+        o += o2;
+        u = (f32x4){v[0], v[1], v[2], v[3]};
+      }
+      queries((it + 1) & 3);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        st[i][0] *= dc[i].x;
+        st[i][1] *= dc[i].y;
+        st[i][2] *= dc[i].z;
+        st[i][3] *= dc[i].w;
+      }
+#define CHUNK_STATE(r, f)                                                           \
+do {                                                                              \
+  st[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(kh[0].f, u[r], st[0], 0, 0, 0);    \
+  st[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(kh[1].f, u[r], st[1], 0, 0, 0);    \
+  st[2] = __builtin_amdgcn_mfma_f32_16x16x4f32(kh[2].f, u[r], st[2], 0, 0, 0);    \
+  st[3] = __builtin_amdgcn_mfma_f32_16x16x4f32(kh[3].f, u[r], st[3], 0, 0, 0);    \
+} while (0)
+      if (__builtin_amdgcn_ballot_w64(!finite4(u)) != 0ull) {
+        lower_product(L.aq[b], u, col, grp, o);
+      } else {
+        o = __builtin_amdgcn_mfma_f32_16x16x4f32(aa.x, u[0], o, 0, 0, 0);
+        o = __builtin_amdgcn_mfma_f32_16x16x4f32(aa.y, u[1], o, 0, 0, 0);
+        o = __builtin_amdgcn_mfma_f32_16x16x4f32(aa.z, u[2], o, 0, 0, 0);
+        o = __builtin_amdgcn_mfma_f32_16x16x4f32(aa.w, u[3], o, 0, 0, 0);
+      }
+      CHUNK_STATE(0, x);
+      CHUNK_STATE(1, y);
+      CHUNK_STATE(2, z);
+      CHUNK_STATE(3, w);
+#undef CHUNK_STATE
+      keys((it + 1) & 3);
+      if constexpr (WKV) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) L.o[it & 1][(4 * grp + r) * RS + 16 * w + col] = o[r];
+      } else {
+        float* rw = a.raw + ((int64_t)(t0 + it * CT + 4 * grp) * H + h) * vdim + vcol;
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          if (vlive && it * CT + 4 * grp + r < n) rw[(int64_t)r * H * vdim] = o[r] * a.q_scale;
+      }
+      __syncthreads();
+    }
+    if constexpr (WKV) __syncthreads();
+  } else if (role == 1) {
+    for (int it = -3; it < turns; ++it) {
+      float q[4], k[4], d[4], bt = 0.f;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        q[i] = arrived(rq[i]);
+        k[i] = arrived(rk[i]);
+        d[i] = arrived(rz[i]) + zbias;
+      }
+      if constexpr (DELTA) bt = arrived(rb);
+      fetch(min(it + 4, nc - 1));
+      if (const int c = it + 3; c < nc) {                 // decays and their products of chunk c
+        const int b = c & 3, e = c & 1;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) d[i] = WKV ? exp_c(-exp_c(d[i])) : exp_c(-rate * softplus_c(a.zsign * d[i]));
+        if constexpr (DELTA)
+          if (w == 0 && grp == 0) L.beta[b][col] = c * CT + col < n ? sigmoid_c(bt) : 0.f;
+        if (dim < NC || c * CT + CT > n) {
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const bool ok = klive && c * CT + 4 * grp + i < n;
+            q[i] = ok ? q[i] : 0.f;
+            k[i] = ok ? k[i] : 0.f;
+            d[i] = ok ? d[i] : 1.f;
+          }
+        }
+        float up[4], after[4];                            // products inside the block: up to t, after t
+        up[0] = d[0];
+        up[1] = up[0] * d[1];
+        up[2] = up[1] * d[2];
+        up[3] = up[2] * d[3];
+        after[3] = 1.f;
+        after[2] = d[3];
+        after[1] = d[2] * after[2];
+        after[0] = d[1] * after[1];
+        // the products of the blocks grp ^ 1, grp ^ 2, grp ^ 3 from the lanes that hold them
+        const float b1 = __shfl_xor(up[3], 16, 64), b2 = __shfl_xor(up[3], 32, 64), b3 = __shfl_xor(b1, 32, 64);
+        const float b23 = b2 * b3;
+        const float pre = ((grp & 1) ? b1 : 1.f) * ((grp & 2) ? b23 : 1.f);
+        const float post = ((grp & 1) ? 1.f : b1) * ((grp & 2) ? 1.f : b23);
+        if (grp == 0) L.dec[b][ch] = up[3] * post;
+        L.blk[e][grp * NC + ch] = up[3];
+        float4 kd;
+        float* kdp = reinterpret_cast<float*>(&kd);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int at = (4 * grp + i) * RS + ch;
+          const float ql = WKV ? (i == 0 ? q[0] : q[i] * up[i - 1]) : q[i] * up[i];
+          const float kl = k[i] * after[i];
+          L.qd[b][at] = ql * pre;
+          kdp[i] = kl * post;
+          L.q[e][at] = q[i];
+          L.k[e][at] = k[i];
+          L.a[e][at] = d[i];
+          L.ql[e][at] = ql;
+          L.kl[e][at] = kl;
+          if constexpr (DELTA) {
+            const float kb = k[i] * up[i];
+            L.kb[e][at] = kb;
+            L.kk[b][at] = kb * pre;
+          }
+        }
+        *reinterpret_cast<float4*>(&L.kd[b][ch * TS + 4 * grp]) = kd;
+      }
+      __syncthreads();
+    }
+  } else if (role == 2) {
+    for (int it = -3; it < turns; ++it) {
+      if constexpr (DELTA) {
+        const int c = it + 1;
+        if (w == 3 && c >= 0 && c < nc && lane < CT) {    // T: column `lane` by forward substitution
+          const float* m = L.ak[c & 1];
+          const float* bt = L.beta[c & 3];
+          float x[CT];
+#pragma unroll
+          for (int t = 0; t < CT; ++t) {
+            float p[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int s4 = 0; s4 < (t + 3) / 4; ++s4) {
+              const float4 r = ld4(m + t * TS + 4 * s4);
+              if (4 * s4 < t) p[0] += r.x * x[4 * s4];
+              if (4 * s4 + 1 < t) p[1] += r.y * x[4 * s4 + 1];
+              if (4 * s4 + 2 < t) p[2] += r.z * x[4 * s4 + 2];
+              if (4 * s4 + 3 < t) p[3] += r.w * x[4 * s4 + 3];
+            }
+            x[t] = (t == lane ? 1.f : 0.f) - bt[t] * ((p[0] + p[1]) + (p[2] + p[3]));
+            L.tt[c & 1][t * TS + lane] = x[t];
+          }
+        }
+      }
+      if (const int c = it + 2; c >= 0 && c < nc) {
+        // A of chunk c.  Pairs of blocks `far` apart: one 16 x 16 product of the readers' rows with
+        // the writers' rows times the blocks between them, of which those pairs are kept.  The delta
+        // rule's keys as readers take the same columns: beside q's rows where they fit (rows 0..7 q,
+        // 8..15 k of the last two blocks), else in a product of their own.
+        const int b = c & 1;
+        auto product = [&](auto far_c, auto rows_c) {     // rows: 0 q, 1 k, 2 both
+          constexpr int far = far_c, rows = rows_c;
+          const float* src = rows == 1 || (rows == 2 && col >= 8) ? L.kb[DELTA ? b : 0] : L.ql[b];
+          const int tr = rows == 2 ? 8 + (col & 7) : col;
+          float4 q[4], k[4], g[4], g2[4];
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const int at = 16 * i + 4 * grp;
+            q[i] = ld4(src + tr * RS + at);
+            k[i] = ld4(&L.kl[b][col * RS + at]);
+            if constexpr (far > 1) g[i] = ld4(&L.blk[b][min((col >> 2) + 1, 3) * NC + at]);
+            if constexpr (far > 2) g2[i] = ld4(&L.blk[b][min((col >> 2) + 2, 3) * NC + at]);
+          }
+          f32x4 x = (f32x4){0.f, 0.f, 0.f, 0.f}, y = x;
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            if constexpr (far > 1) k[i] = mul4(k[i], g[i]);
+            if constexpr (far > 2) k[i] = mul4(k[i], g2[i]);
+            x = __builtin_amdgcn_mfma_f32_16x16x4f32(q[i].x, k[i].x, x, 0, 0, 0);
+            y = __builtin_amdgcn_mfma_f32_16x16x4f32(q[i].y, k[i].y, y, 0, 0, 0);
+            x = __builtin_amdgcn_mfma_f32_16x16x4f32(q[i].z, k[i].z, x, 0, 0, 0);
+            y = __builtin_amdgcn_mfma_f32_16x16x4f32(q[i].w, k[i].w, y, 0, 0, 0);
+          }
+          x += y;
+          const int tb = rows == 2 ? 2 + (grp & 1) : grp;  // this lane's block of rows, its column's block
+          float* to = rows == 1 || (rows == 2 && grp >= 2) ? L.ak[DELTA ? b : 0] : L.aq[c & 3];
+          if (tb - (col >> 2) == far) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) to[(4 * tb + r) * TS + col] = x[r];
+          }
+        };
+        constexpr std::integral_constant<int, 0> i0{};
+        constexpr std::integral_constant<int, 1> i1{};
+        constexpr std::integral_constant<int, 2> i2{};
+        constexpr std::integral_constant<int, 3> i3{};
+        if constexpr (DELTA) {
+          if (w == 0) product(i1, i0);
+          else if (w == 1) product(i1, i1);
+          else if (w == 2) { product(i2, i2); product(i3, i2); }
+        } else {
+          if (w == 0) product(i1, i0);
+          else if (w == 1) product(i2, i0);
+          else if (w == 2) product(i3, i0);
+        }
+        if (w == (DELTA ? 0 : 3)) {
+          // pairs inside a block: sixteen lanes per block, four key channels each
+          float4 q[4], k[4], d[4];
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const int at = (4 * grp + i) * RS + 4 * col;
+            q[i] = ld4(&L.q[b][at]);
+            k[i] = ld4(&L.k[b][at]);
+            d[i] = ld4(&L.a[b][at]);
+          }
+          float acc[10], ack[6];                          // (0,0) (1,0) (1,1) (2,0) .. (3,3); without s = t
+          if constexpr (WKV) {
+            acc[1] = dot4(q[1], k[0]);
+            acc[4] = dot4(q[2], k[1]);
+            acc[8] = dot4(q[3], k[2]);
+            const float4 e1 = mul4(d[1], k[0]);
+            acc[3] = dot4(q[2], e1);
+            acc[7] = dot4(q[3], mul4(d[2], k[1]));
+            acc[6] = dot4(q[3], mul4(d[2], e1));
+#pragma unroll
+            for (int i = 0; i < 4; ++i) acc[i * (i + 3) / 2] = dot4(mul4(q[i], bonus), k[i]);
+          } else {
+            const float4 e10 = mul4(d[1], k[0]), e21 = mul4(d[2], k[1]), e32 = mul4(d[3], k[2]);
+            const float4 e20 = mul4(d[2], e10), e31 = mul4(d[3], e21), e30 = mul4(d[3], e20);
+            acc[1] = dot4(q[1], e10);
+            acc[3] = dot4(q[2], e20);
+            acc[4] = dot4(q[2], e21);
+            acc[6] = dot4(q[3], e30);
+            acc[7] = dot4(q[3], e31);
+            acc[8] = dot4(q[3], e32);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) acc[i * (i + 3) / 2] = dot4(q[i], k[i]);
+            if constexpr (DELTA) {
+              ack[0] = dot4(k[1], e10);
+              ack[1] = dot4(k[2], e20);
+              ack[2] = dot4(k[2], e21);
+              ack[3] = dot4(k[3], e30);
+              ack[4] = dot4(k[3], e31);
+              ack[5] = dot4(k[3], e32);
+            }
+          }
+          float* ao = &L.aq[c & 3][4 * grp * TS + 4 * grp];
+#pragma unroll
+          for (int i = 0; i < 10; ++i) acc[i] = ror_add(acc[i]);
+          if (col == 0) {
+            ao[0] = acc[0];
+            *reinterpret_cast<float2*>(ao + TS) = make_float2(acc[1], acc[2]);
+            *reinterpret_cast<float2*>(ao + 2 * TS) = make_float2(acc[3], acc[4]);
+            ao[2 * TS + 2] = acc[5];
+            *reinterpret_cast<float4*>(ao + 3 * TS) = make_float4(acc[6], acc[7], acc[8], acc[9]);
+          }
+          if constexpr (DELTA) {
+            float* ko4 = &L.ak[b][4 * grp * TS + 4 * grp];
+#pragma unroll
+            for (int i = 0; i < 6; ++i) ack[i] = ror_add(ack[i]);
+            if (col == 0) {
+              ko4[TS] = ack[0];
+              *reinterpret_cast<float2*>(ko4 + 2 * TS) = make_float2(ack[1], ack[2]);
+              *reinterpret_cast<float2*>(ko4 + 3 * TS) = make_float2(ack[3], ack[4]);
+              ko4[3 * TS + 2] = ack[5];
+            }
+          }
+        }
+      }
+      __syncthreads();
+    }
+  } else if constexpr (WKV) {
+    for (int it = -3; it < turns; ++it) {
+      float g[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) g[e] = arrived(rg[e]);
+      const int tn = min(max(it, 0) * CT + 4 * w + grp, n - 1);  // the gates of chunk it, for the next turn
+      const TI* gr = gb + tn * a.gs + 4 * col;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) rg[e] = load_at(gr + e, 0);
+      if (it >= 1) {                                    // norm and gate of chunk it - 1
+        const int tl = 4 * w + grp, t = (it - 1) * CT + tl;
+        const float4 o4 = ld4(&L.o[(it - 1) & 1][tl * RS + 4 * col]);
+        const float inv = 1.0f / sqrtf(ror_add(dot4(o4, o4)) / (float)NC + a.eps);
+        const float y[4] = {o4.x * nw.x, o4.y * nw.y, o4.z * nw.z, o4.w * nw.w};
+        TI* op = static_cast<TI*>(a.out) + ((int64_t)(t0 + t) * H + h) * NC + 4 * col;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const float z = y[e] * inv * (g[e] * sigmoid_c(g[e]));
+          if (t < n) stf(op + e, z);
+        }
+      }
+      __syncthreads();
+    }
+  }
+
+  if (role == 0 && code >= 0 && vlive) {
+    float* wr = a.state + (((int64_t)(1 - (code & 1)) * a.slots + (code >> 1)) * H + h) * hsz;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int c = 16 * i + 4 * grp + r;
+        if (c < dim) wr[(int64_t)c * vdim + vcol] = st[i][r];
+      }
+  }
+}
+
+// ------------------------------------------------------------------ launcher
+// A workgroup costs some 9 us before its first chunk is out and 1.4 - 2 us a chunk, one to a CU; the
+// token-by-token kernels some 6 us and 0.2 (64 runs) - 2.6 us a token, many to a CU.  Two rounds of
+// workgroups or fewer: chunks from 8 rows a run on (wkv, one run: 8 rows 21 us against 37; the
+// others have a launch more, they gain from 24 on: delta 16 rows 73 us against 67, 40 rows 72
+// against 129).  More rounds: no gain below some 24 (wkv, 64 runs of 16:
+// 145 us against 130, of 32: 189 against 201) or 40 rows (delta, 64 runs of 32: 261 against 212), so the
+// runs of a step, decode rows beside prompts as a rule, are shared by their length (wkv, 64 decode
+// rows beside a prompt of 200: 102 us, one kernel for all of them 594).
+int chunk_min_run(int mode, int T, const ChunkArgs& a) {
+  constexpr int kNever = INT32_MAX;
+  const int kLong = mode == kChunkWkv ? 24 : 40;
+  if (a.run_rows == nullptr || a.dim > NC || (mode == kChunkWkv && (a.dim != NC || a.vdim != NC))) return kNever;
+  for (int64_t st : {a.qs, a.ks, a.vs, a.zs})             // a chunk's rows in 32-bit byte offsets
+    if (st < 0 || st >= (1ll << 24)) return kNever;
+  const int64_t groups = (int64_t)a.runs * a.H * ((a.vdim + 63) / 64);
+  if (groups <= 512 && T >= (mode == kChunkWkv ? 8 : 24) * a.runs) return 1;
+  return T - a.runs + 1 >= kLong ? kLong : kNever;        // no run can be longer than that
+}
+
+template <typename TI, typename TG, int MODE>
+static void launch_chunk_one(int T, const ChunkArgs& a, hipStream_t s) {
+  static bool attr = false;
+  if (!attr) {          // dynamic LDS above 64 KB has to be allowed per kernel, once
+    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&chunk_recurrence_kernel<TI, TG, MODE>),
+                              hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+    attr = true;
+  }
+  static_assert(sizeof(ChunkLds<MODE>) <= 160 * 1024, "LDS of a CU");
+  // No more long runs than rows allow.  An odd number: workgroups go to the eight XCDs in turn, and
+  // those of the first few runs are all that work (64 decode rows beside a prompt of 600, wkv: 198 us
+  // with 8 columns, all of them on one XCD, 145 with 13).
+  const int gx = a.min_run <= 1 ? a.runs : std::min(a.runs, T / a.min_run) | 1;
+  hipLaunchKernelGGL((chunk_recurrence_kernel<TI, TG, MODE>),
+                     dim3(gx, a.H, (a.vdim + 63) / 64), dim3(chunk_threads(MODE)), sizeof(ChunkLds<MODE>), s, a);
+}
+
+void launch_chunk(int mode, bool in_f32, bool act_f32, int T, const ChunkArgs& a, hipStream_t s) {
+  if (a.runs == 0) return;
+  if (mode == kChunkWkv) {
+    if (in_f32) launch_chunk_one<float, float, kChunkWkv>(T, a, s);
+    else launch_chunk_one<bf16_t, bf16_t, kChunkWkv>(T, a, s);
+  } else if (mode == kChunkGla) {
+    if (in_f32) launch_chunk_one<float, float, kChunkGla>(T, a, s);
+    else launch_chunk_one<bf16_t, float, kChunkGla>(T, a, s);
+  } else if (in_f32) {
+    if (act_f32) launch_chunk_one<float, float, kChunkDelta>(T, a, s);
+    else launch_chunk_one<float, bf16_t, kChunkDelta>(T, a, s);
+  } else {
+    if (act_f32) launch_chunk_one<bf16_t, float, kChunkDelta>(T, a, s);
+    else launch_chunk_one<bf16_t, bf16_t, kChunkDelta>(T, a, s);
+  }
+}
+
+}  // namespace rfqmix

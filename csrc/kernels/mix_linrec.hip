@@ -17,10 +17,14 @@
 // The state pool is double buffered: a run reads its sequence's half and writes the other, and
 // a run that starts at position 0 reads nothing (the slot may hold another sequence's rest).
 //
-// One workgroup per (run, head); thread j owns value channel j: column j of S lives in
+// Long runs with up to 64 key channels go in chunks (mix_chunk.hip).  Below: token by token.  One
+// workgroup per (run, head); thread j owns value channel j: column j of S lives in
 // registers when dim is a compile-time size, else in LDS.  q, k and the decay of a token reach
 // all threads through LDS (one 16-byte read per key channel); the next token's operands are
 // loaded while the current one is summed.
+#include <algorithm>
+
+#include "mix_chunk.h"
 #include "mix_common.h"
 #include "mix_linrec.h"
 
@@ -37,15 +41,16 @@ __global__ __launch_bounds__(256) void gated_linrec_kernel(
     int64_t z_stride, const float* __restrict__ rate, const float* __restrict__ zbias,
     float zsign, const TG* __restrict__ beta, int64_t b_stride, const TG* __restrict__ gate,
     int64_t g_stride, int gate_sigmoid, const float* __restrict__ norm_w, float eps,
-    float q_scale, int decay_ready, float* __restrict__ raw, float* __restrict__ state,
+    float q_scale, float* __restrict__ raw, float* __restrict__ state,
     const int32_t* __restrict__ row_state,
     const int32_t* __restrict__ row_back, const int32_t* __restrict__ row_fwd,
     const int32_t* __restrict__ pos, const int32_t* __restrict__ run_rows, TG* __restrict__ out,
-    int64_t o_stride, int H, int rep, int dim, int vdim, int slots) {
+    int64_t o_stride, int H, int rep, int dim, int vdim, int slots, int below) {
   const int t0 = run_rows != nullptr ? run_rows[blockIdx.x] : (int)blockIdx.x;
   const int h = blockIdx.y;
   if (t0 < 0 || row_back[t0] != 0) return;
   const int n = row_fwd[t0] + 1;
+  if (n >= below) return;                              // a run of the chunked kernel
   const int code = row_state[t0];
   const int j = threadIdx.x;
   const bool vlive = j < vdim, klive = j < dim;
@@ -78,7 +83,7 @@ __global__ __launch_bounds__(256) void gated_linrec_kernel(
     nq = ldf(q + (int64_t)t0 * q_stride + qc);
     nk = ldf(k + (int64_t)t0 * k_stride + qc);
     na = z[(int64_t)t0 * z_stride + zc];
-    if (!decay_ready) na = expf(-my_rate * softplus_f(zsign * (na + my_zb)));
+    na = expf(-my_rate * softplus_f(zsign * (na + my_zb)));
   }
   if (vlive) {
     nv = ldf(v + (int64_t)t0 * v_stride + vc);
@@ -165,7 +170,7 @@ __global__ __launch_bounds__(256) void gated_linrec_kernel(
       }
       o *= q_scale;
     }
-    if (a + 1 < n && klive && !decay_ready) na = expf(-my_rate * softplus_f(zsign * (na + my_zb)));
+    if (a + 1 < n && klive) na = expf(-my_rate * softplus_f(zsign * (na + my_zb)));
     if (raw != nullptr) {              // long steps: norm and gate follow in a row-parallel kernel
       if (vlive) raw[(int64_t)(t0 + a) * H * vdim + vc] = o;
       continue;
@@ -187,36 +192,19 @@ __global__ __launch_bounds__(256) void gated_linrec_kernel(
   }
 }
 
-// z[t, h, c] <- exp(-rate_h softplus(zsign (z + zbias[h, c]))) in place: the decays of a long
-// step are formed by all threads of the chip at once instead of inside the token-by-token scan.
-__global__ __launch_bounds__(256) void decay_from_logits_kernel(
-    float* __restrict__ z, int64_t z_stride, const float* __restrict__ rate,
-    const float* __restrict__ zbias, float zsign, int HD, int dim) {
-  const int t = blockIdx.x;
-  float* zr = z + (int64_t)t * z_stride;
-  for (int c = blockIdx.y * blockDim.x + threadIdx.x; c < HD; c += gridDim.y * blockDim.x)
-    zr[c] = expf(-rate[c / dim] * softplus_f(zsign * (zr[c] + zbias[c])));
-}
-
-void launch_decay_from_logits(float* z, int64_t z_stride, const float* rate, const float* zbias,
-                              float zsign, int T, int H, int dim, hipStream_t s) {
-  if (T == 0) return;
-  const int HD = H * dim;
-  hipLaunchKernelGGL(decay_from_logits_kernel, dim3(T, (HD + 1023) / 1024), dim3(256), 0, s, z,
-                     z_stride, rate, zbias, zsign, HD, dim);
-}
-
 // out[t, h, :] = raw / sqrt(mean(raw^2) + eps) * norm_w * act(gate): the scan's read-outs of a
 // long step, a wave per (row, head).
 template <typename TG>
 __global__ __launch_bounds__(256) void linrec_finish_kernel(
     const float* __restrict__ raw, const TG* __restrict__ gate, int64_t g_stride,
     int gate_sigmoid, const float* __restrict__ norm_w, float eps, TG* __restrict__ out,
-    int64_t o_stride, int T, int H, int vdim) {
+    int64_t o_stride, const int32_t* __restrict__ row_back, const int32_t* __restrict__ row_fwd,
+    int min_run, int T, int H, int vdim) {
   const int lane = threadIdx.x & 63;
   const int64_t item = (int64_t)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
   if (item >= (int64_t)T * H) return;
   const int64_t t = item / H;
+  if (min_run > 1 && row_back[t] + row_fwd[t] + 1 < min_run) return;   // its own kernel finished it
   const int h = (int)(item - t * H);
   const float* r = raw + item * vdim;
   float ss = 0.f;
@@ -230,7 +218,7 @@ __global__ __launch_bounds__(256) void linrec_finish_kernel(
   }
 }
 
-// The scan of a long step: decays formed ahead (z holds them), read-outs to `raw` for the
+// The scan of a long step: decays formed while its operands are staged, read-outs to `raw` for the
 // row-parallel norm and gate.  One workgroup of four waves per (run, head, 64 value channels).  Four
 // neighbouring lanes share a value channel: each holds a quarter of the key channels of its column
 // of S in registers, and the sums over all of them finish with two DPP adds inside the quad.  The
@@ -268,11 +256,11 @@ template <typename TI, typename TG, int NR, bool DELTA>
 __global__ __launch_bounds__(256) void gated_linrec_scan_kernel(
     const TI* __restrict__ q, const TI* __restrict__ k, const TI* __restrict__ v,
     int64_t q_stride, int64_t k_stride, int64_t v_stride, const float* __restrict__ z,
-    int64_t z_stride, const TG* __restrict__ beta, int64_t b_stride, float q_scale,
-    float* __restrict__ raw, float* __restrict__ state, const int32_t* __restrict__ row_state,
+    int64_t z_stride, const float* __restrict__ rate, const float* __restrict__ zbias, float zsign,
+    const TG* __restrict__ beta, int64_t b_stride, float q_scale, float* __restrict__ raw, float* __restrict__ state, const int32_t* __restrict__ row_state,
     const int32_t* __restrict__ row_back, const int32_t* __restrict__ row_fwd,
     const int32_t* __restrict__ pos, const int32_t* __restrict__ run_rows, int H, int rep, int dim,
-    int vdim, int slots, int vec) {
+    int vdim, int slots, int vec, int above, int below) {
   constexpr int NK = NR / 4;                           // key channels per lane
   constexpr int P4 = NR / 4;                           // 16-byte pieces per row of q, k, decay
   constexpr int NL = (SCAN_ROWS * P4 + 255) / 256;     // pieces per thread
@@ -281,6 +269,7 @@ __global__ __launch_bounds__(256) void gated_linrec_scan_kernel(
   const int h = blockIdx.y;
   if (t0 < 0 || row_back[t0] != 0) return;
   const int n = row_fwd[t0] + 1;
+  if (n <= above || n >= below) return;                // runs of the other kernels
   const int code = row_state[t0];
   const int tid = threadIdx.x, lane = tid & 63, ks = lane & 3;
   const int v0 = blockIdx.z * 64;
@@ -303,8 +292,14 @@ __global__ __launch_bounds__(256) void gated_linrec_scan_kernel(
     sreg[i] = (from_state && vlive && ch < dim) ? rd[(int64_t)ch * vdim + j] : 0.f;
   }
 
-  float4 rq[NL], rk[NL], ra[NL], rv;
+  float4 rq[NL], rk[NL], ra[NL], zb[NL], rv;
   float rb = 0.f;
+  const float my_rate = rate[h];
+#pragma unroll
+  for (int u = 0; u < NL; ++u) {
+    const int x = tid + u * 256, c = (x - x / P4 * P4) * 4;
+    zb[u] = row4(zbias + (int64_t)h * dim, c, dim, false);
+  }
   auto fetch = [&](int a0) {
     const int rows = min(SCAN_ROWS, n - a0);
 #pragma unroll
@@ -332,7 +327,12 @@ __global__ __launch_bounds__(256) void gated_linrec_scan_kernel(
       const int x = tid + u * 256, r = x / P4, c = (x - r * P4) * 4;
       if (x < SCAN_ROWS * P4 && r < rows) {
         float* o = ops + r * RS + c;
-        *reinterpret_cast<float4*>(o) = ra[u];
+        float4 d = ra[u];
+        d.x = expf(-my_rate * softplus_f(zsign * (d.x + zb[u].x)));
+        d.y = expf(-my_rate * softplus_f(zsign * (d.y + zb[u].y)));
+        d.z = expf(-my_rate * softplus_f(zsign * (d.z + zb[u].z)));
+        d.w = expf(-my_rate * softplus_f(zsign * (d.w + zb[u].w)));
+        *reinterpret_cast<float4*>(o) = d;
         *reinterpret_cast<float4*>(o + NR) = rk[u];
         *reinterpret_cast<float4*>(o + 2 * NR) = rq[u];
       }
@@ -409,7 +409,7 @@ __global__ __launch_bounds__(256) void gated_linrec_scan_kernel(
 
 // ------------------------------------------------------------------ launchers
 template <typename TI, typename TG, int NR, bool DELTA>
-static void launch_linrec_scan(const LinrecArgs& a, hipStream_t s) {
+static void launch_linrec_scan(const LinrecArgs& a, int above, hipStream_t s) {
   auto al = [](const void* p, int64_t stride, int64_t head, size_t esz) {
     return reinterpret_cast<uintptr_t>(p) % (4 * esz) == 0 && stride % 4 == 0 && head % 4 == 0;
   };
@@ -418,8 +418,9 @@ static void launch_linrec_scan(const LinrecArgs& a, hipStream_t s) {
   const dim3 grid(a.run_rows != nullptr ? a.runs : a.T, a.H, (a.vdim + 63) / 64);
   hipLaunchKernelGGL((gated_linrec_scan_kernel<TI, TG, NR, DELTA>), grid, dim3(256), 0, s,
                      (const TI*)a.q, (const TI*)a.k, (const TI*)a.v, a.qs, a.ks, a.vs, a.z, a.zs,
-                     (const TG*)a.beta, a.bs, a.q_scale, a.raw, a.state, a.row_state, a.row_back,
-                     a.row_fwd, a.pos, a.run_rows, a.H, a.rep, a.dim, a.vdim, a.slots, (int)vec);
+                     a.rate, a.zbias, a.zsign, (const TG*)a.beta, a.bs, a.q_scale, a.raw, a.state,
+                     a.row_state, a.row_back, a.row_fwd, a.pos, a.run_rows, a.H, a.rep, a.dim, a.vdim,
+                     a.slots, (int)vec, above, a.below);
 }
 
 template <typename TI, typename TG, int NR, bool DELTA>
@@ -436,17 +437,17 @@ static void launch_linrec_one(const LinrecArgs& a, hipStream_t s) {
                      dim3(a.run_rows != nullptr ? a.runs : a.T, a.H), dim3(threads), lds, s,
                      (const TI*)a.q, (const TI*)a.k, (const TI*)a.v, a.qs, a.ks, a.vs, a.z, a.zs,
                      a.rate, a.zbias, a.zsign, (const TG*)a.beta, a.bs, (const TG*)a.gate, a.gs,
-                     a.gate_sigmoid, a.norm_w, a.eps, a.q_scale, a.decay_ready, a.raw, a.state,
+                     a.gate_sigmoid, a.norm_w, a.eps, a.q_scale, a.raw, a.state,
                      a.row_state, a.row_back,
-                     a.row_fwd, a.pos, a.run_rows, (TG*)a.out, a.os, a.H, a.rep, a.dim, a.vdim, a.slots);
+                     a.row_fwd, a.pos, a.run_rows, (TG*)a.out, a.os, a.H, a.rep, a.dim, a.vdim, a.slots, a.below);
 }
 
 template <typename TI, typename TG, bool DELTA>
-static void launch_linrec_dim(const LinrecArgs& a, hipStream_t s) {
-  if (a.raw != nullptr && a.decay_ready && a.dim <= 128) {
-    if (a.dim <= 32) launch_linrec_scan<TI, TG, 32, DELTA>(a, s);
-    else if (a.dim <= 64) launch_linrec_scan<TI, TG, 64, DELTA>(a, s);
-    else launch_linrec_scan<TI, TG, 128, DELTA>(a, s);
+static void launch_linrec_dim(const LinrecArgs& a, int above, hipStream_t s) {
+  if (a.raw != nullptr && a.dim <= 128) {
+    if (a.dim <= 32) launch_linrec_scan<TI, TG, 32, DELTA>(a, above, s);
+    else if (a.dim <= 64) launch_linrec_scan<TI, TG, 64, DELTA>(a, above, s);
+    else launch_linrec_scan<TI, TG, 128, DELTA>(a, above, s);
     return;
   }
   if (a.dim == 32) launch_linrec_one<TI, TG, 32, DELTA>(a, s);
@@ -463,30 +464,65 @@ bool linrec_ok(int dim, int vdim) {
 }
 
 // in_f32: q, k, v are fp32 (else bf16); act_f32: beta, gate and out are fp32 (else bf16).
-void launch_gated_linrec(bool in_f32, bool act_f32, bool delta, const LinrecArgs& a,
+void launch_gated_linrec(bool in_f32, bool act_f32, bool delta, const LinrecArgs& args,
                          hipStream_t s) {
+  LinrecArgs a = args;
   if (a.T == 0 || (a.run_rows != nullptr && a.runs == 0)) return;
-#define LINREC_GO(TI, TG)                                   \
-  do {                                                      \
-    if (delta) launch_linrec_dim<TI, TG, true>(a, s);       \
-    else launch_linrec_dim<TI, TG, false>(a, s);            \
+  int above = 0;                // runs of up to that many rows are finished by their own kernel
+  if (a.raw != nullptr) {       // a step's long runs go to the chunked kernel
+    ChunkArgs c{};
+    c.q = a.q; c.k = a.k; c.v = a.v; c.z = a.z; c.beta = a.beta;
+    c.qs = a.qs; c.ks = a.ks; c.vs = a.vs; c.zs = a.zs; c.bs = a.bs;
+    c.rate = a.rate; c.zbias = a.zbias; c.zsign = a.zsign; c.q_scale = a.q_scale;
+    c.raw = a.raw; c.state = a.state;
+    c.row_state = a.row_state; c.row_back = a.row_back; c.row_fwd = a.row_fwd; c.pos = a.pos;
+    c.run_rows = a.run_rows; c.runs = a.runs; c.H = a.H; c.rep = a.rep; c.dim = a.dim; c.vdim = a.vdim;
+    c.slots = a.slots;
+    const int mode = delta ? kChunkDelta : kChunkGla;
+    a.below = c.min_run = chunk_min_run(mode, a.T, c);
+    if (c.min_run < INT32_MAX) launch_chunk(mode, in_f32, act_f32, a.T, c, s);
+    // Below them: the scan's fixed cost is the larger one (64 decode rows, gla: 41 us against 72),
+    // its tokens are the cheaper ones where each has two sums (delta, 64 runs of 8: 106 us against
+    // 177; gla 89 against 82).
+    if (a.run_rows != nullptr && a.dim <= kChunkDim) 
+      above = delta && a.T > 2 * a.runs ? std::min(3, a.below - 1) : a.below - 1;
+  }
+#define LINREC_GO(TI, TG)                                              \
+  do {                                                                 \
+    if (delta) launch_linrec_dim<TI, TG, true>(b, above, s);           \
+    else launch_linrec_dim<TI, TG, false>(b, above, s);                \
   } while (0)
-  if (in_f32 && act_f32) LINREC_GO(float, float);
-  else if (in_f32) LINREC_GO(float, bf16_t);
-  else if (!act_f32) LINREC_GO(bf16_t, bf16_t);
-  else LINREC_GO(bf16_t, float);
+#define LINREC_ALL()                                                   \
+  do {                                                                 \
+    if (in_f32 && act_f32) LINREC_GO(float, float);                    \
+    else if (in_f32) LINREC_GO(float, bf16_t);                         \
+    else if (!act_f32) LINREC_GO(bf16_t, bf16_t);                      \
+    else LINREC_GO(bf16_t, float);                                     \
+  } while (0)
+  if (above > 0 || a.raw == nullptr) {
+    LinrecArgs b = a;
+    b.raw = nullptr;
+    if (above > 0) b.below = above + 1;
+    LINREC_ALL();
+  }
+  if (a.raw != nullptr && above + 1 < a.below) {
+    const LinrecArgs& b = a;
+    LINREC_ALL();
+  }
+#undef LINREC_ALL
 #undef LINREC_GO
-  if (a.raw != nullptr) {
+  const float* raw = a.raw;
+  if (raw != nullptr && (a.below < INT32_MAX || above + 1 < a.below)) {     // chunks or the scan wrote to it
     const int64_t items = (int64_t)a.T * a.H;
     const dim3 grid((unsigned)((items + 3) / 4));
     if (act_f32)
-      hipLaunchKernelGGL(linrec_finish_kernel<float>, grid, dim3(256), 0, s, a.raw,
+      hipLaunchKernelGGL(linrec_finish_kernel<float>, grid, dim3(256), 0, s, raw,
                          (const float*)a.gate, a.gs, a.gate_sigmoid, a.norm_w, a.eps,
-                         (float*)a.out, a.os, a.T, a.H, a.vdim);
+                         (float*)a.out, a.os, a.row_back, a.row_fwd, above + 1, a.T, a.H, a.vdim);
     else
-      hipLaunchKernelGGL(linrec_finish_kernel<bf16_t>, grid, dim3(256), 0, s, a.raw,
+      hipLaunchKernelGGL(linrec_finish_kernel<bf16_t>, grid, dim3(256), 0, s, raw,
                          (const bf16_t*)a.gate, a.gs, a.gate_sigmoid, a.norm_w, a.eps,
-                         (bf16_t*)a.out, a.os, a.T, a.H, a.vdim);
+                         (bf16_t*)a.out, a.os, a.row_back, a.row_fwd, above + 1, a.T, a.H, a.vdim);
   }
 }
 

@@ -9,6 +9,7 @@
 // (-1: none), row_back = index of the row inside its run, row_fwd = rows of the run after it.
 // State pools are double buffered: a run reads its sequence's half and writes the other, and
 // a run that starts at position 0 reads nothing (the slot may hold another sequence's rest).
+#include "mix_chunk.h"
 #include "mix_common.h"
 
 namespace rfqmix {
@@ -40,8 +41,8 @@ __global__ __launch_bounds__(256) void token_shift_mix_kernel(
   }
 }
 
-// One workgroup per (row, head); only a run's first row works: it walks the run token by
-// token.  Thread j owns value channel j: column j of S lives in LDS (st[i * N + j]: lanes hit
+// Token by token (long runs of 64 x 64 heads go in chunks: mix_chunk.hip).  One workgroup per
+// (row, head); only a run's first row works: it walks the run.  Thread j owns value channel j: column j of S lives in LDS (st[i * N + j]: lanes hit
 // consecutive banks), or in registers when N is the compile-time NR.  r, k and the decay of
 // the next token are fetched while the current one is computed.
 template <typename T, int NR>
@@ -53,13 +54,14 @@ __global__ __launch_bounds__(256) void wkv_recurrence_kernel(
     float* __restrict__ state, const int32_t* __restrict__ row_state,
     const int32_t* __restrict__ row_back, const int32_t* __restrict__ row_fwd,
     const int32_t* __restrict__ pos, const int32_t* __restrict__ run_rows, T* __restrict__ out,
-    int H, int N, int slots) {
+    int H, int N, int slots, int below) {
   // with a list of the runs' first rows the grid holds only workgroups that work (-1: no run);
   // without one, a workgroup per row, of which the runs' first rows work
   const int t0 = run_rows != nullptr ? run_rows[blockIdx.x] : (int)blockIdx.x;
   const int h = blockIdx.y;
   if (t0 < 0 || row_back[t0] != 0) return;
   const int n = row_fwd[t0] + 1;
+  if (n >= below) return;            // a run of the chunked kernel
   const int code = row_state[t0];
   const int j = threadIdx.x;
   const bool live = j < N;
@@ -166,7 +168,7 @@ static void launch_wkv_one(const void* r, const void* k, const void* v, const vo
                            float eps, float* state, const int32_t* row_state,
                            const int32_t* row_back, const int32_t* row_fwd, const int32_t* pos,
                            const int32_t* run_rows, int runs, void* out, int Trows, int H, int N,
-                           int slots, hipStream_t s) {
+                           int slots, int below, hipStream_t s) {
   const int threads = (N + 63) / 64 * 64;
   const size_t lds = (size_t)(8 * N + 16 + (NR > 0 ? 0 : N * N)) * 4;
   static bool attr = false;
@@ -178,7 +180,7 @@ static void launch_wkv_one(const void* r, const void* k, const void* v, const vo
   hipLaunchKernelGGL((wkv_recurrence_kernel<T, NR>), dim3(run_rows != nullptr ? runs : Trows, H),
                      dim3(threads), lds, s, (const T*)r, (const T*)k, (const T*)v, (const T*)zw,
                      (const T*)gate, rs, ks, vs, zs, gs, w0, u, norm_w, eps, state, row_state,
-                     row_back, row_fwd, pos, run_rows, (T*)out, H, N, slots);
+                     row_back, row_fwd, pos, run_rows, (T*)out, H, N, slots, below);
 }
 
 // Whether the head size fits (threads <= 256; the state matrix of a head in LDS).
@@ -192,10 +194,20 @@ void launch_wkv_recurrence(bool f32, const void* r, const void* k, const void* v
                            const int32_t* run_rows, int runs, void* out, int Trows, int H, int N,
                            int slots, hipStream_t s) {
   if (Trows == 0 || (run_rows != nullptr && runs == 0)) return;
+  ChunkArgs a{};
+  a.q = r; a.k = k; a.v = v; a.z = zw; a.gate = gate;
+  a.qs = rs; a.ks = ks; a.vs = vs; a.zs = zs; a.gs = gs;
+  a.zbias = w0; a.u = u; a.norm_w = norm_w; a.eps = eps; a.q_scale = 1.f;
+  a.out = out; a.state = state;
+  a.row_state = row_state; a.row_back = row_back; a.row_fwd = row_fwd; a.pos = pos; a.run_rows = run_rows;
+  a.runs = runs; a.H = H; a.rep = 1; a.dim = a.vdim = N; a.slots = slots;
+  const int below = a.min_run = chunk_min_run(kChunkWkv, Trows, a);
+  if (below < INT32_MAX) launch_chunk(kChunkWkv, f32, f32, Trows, a, s);
+  if (below == 1) return;
 #define WKV_GO(TT, NRR)                                                                         \
   launch_wkv_one<TT, NRR>(r, k, v, zw, gate, rs, ks, vs, zs, gs, w0, u, norm_w, eps, state,     \
                           row_state, row_back, row_fwd, pos, run_rows, runs, out, Trows, H, N,  \
-                          slots, s)
+                          slots, below, s)
   if (f32) {
     if (N == 64) WKV_GO(float, 64); else WKV_GO(float, 0);
   } else {

@@ -1355,27 +1355,29 @@ def conv_act_heads(x, w, state, row_state, row_back, row_fwd, positions, n_unit:
     return out
 
 
-LINREC_DECAY_ROWS = 128     # steps with more rows form the decays before the scan
+LINREC_SCAN_ROWS = 128      # steps with more rows leave norm and gate to a row-parallel kernel
+CHUNK_DIM = 64              # most key channels of the chunked recurrences (csrc/kernels/mix_chunk.hip)
+CHUNK_RUN = 40              # steps that can hold a run of that many rows may use them
 
 
 def gated_linear_recurrence(q, k, v, z, rate, zbias, zsign: float, beta, gate, gate_sigmoid: bool,
                             norm_w, eps: float, q_scale: float, state, row_state, row_back,
                             row_fwd, positions, out, run_rows=None):
     """``run_rows`` (int32): the first row of every run of the step (-1: none); the kernel
-    launches one workgroup per (run, head).  On the GPU a step of more than
-    LINREC_DECAY_ROWS rows first turns ``z`` into the decays IN PLACE with a row-parallel
-    kernel and leaves norm and gate to another one, so that the token-by-token scan holds
-    neither transcendental work nor a reduction over the head."""
+    launches one workgroup per (run, head).  On the GPU the long runs of a step with up to
+    CHUNK_DIM key channels go in chunks of 16 tokens, the short ones token by token; norm and
+    gate of such a step, and of any other with more than LINREC_SCAN_ROWS rows, are left to a
+    row-parallel kernel, so that neither loop holds a reduction over the head."""
     if _gpu(q):
-        ready = q.shape[0] > LINREC_DECAY_ROWS
+        T, runs = q.shape[0], -1 if run_rows is None else run_rows.numel()
         raw = None
-        if ready:
-            _native.mix_ops().decay_from_logits(z, rate, zbias, float(zsign), int(state.shape[2]))
+        if T > LINREC_SCAN_ROWS and T != runs or T >= 24 * runs > 0 and state.shape[2] <= CHUNK_DIM or \
+                runs >= 0 and state.shape[2] <= CHUNK_DIM and T - runs + 1 >= CHUNK_RUN:
             raw = torch.empty(out.shape, dtype=torch.float32, device=out.device)
         _native.mix_ops().gated_linear_recurrence(
             q, k, v, z, rate, zbias, float(zsign), beta, gate, bool(gate_sigmoid), norm_w,
             float(eps), float(q_scale), state, row_state, row_back, row_fwd, positions, run_rows,
-            out, ready, raw)
+            out, raw)
     else:
         ref.gated_linear_recurrence(q, k, v, z, rate, zbias, zsign, beta, gate, gate_sigmoid,
                                     norm_w, eps, q_scale, state, row_state, row_back, row_fwd,
