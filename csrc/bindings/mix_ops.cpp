@@ -86,11 +86,14 @@ int launch_attn_keep_decode(bool, const float*, const void*, const void*, int64_
                             const float*, const void*, int64_t, int, void*, int64_t, float, int,
                             int, bool, int, int, int, int, int, float, float, hipStream_t);
 bool keep_mfma_ok(int, int, int, bool);
+void launch_attn_keep_split(const float*, const void*, const void*, int64_t, const int32_t*, int, const int32_t*,
+                            const int32_t*, const int32_t*, int, int, const float*, const void*, int64_t, int, void*,
+                            int64_t, float, int, int, bool, int, int, int, int, bool, float, float, hipStream_t);
 bool launch_attn_keep_mfma(const float*, const void*, const void*, int64_t, const int32_t*, int,
                            const int32_t*, const int32_t*, const int32_t*, const int32_t*,
                            const int32_t*, int, const float*, const void*, int64_t, int, void*,
-                           int64_t, float, int, int, bool, int, int, int, int, int, bool, int, int,
-                           float, float, hipStream_t);
+                           int64_t, float, int, int, bool, int, int, int, int, int, bool, float, float,
+                           hipStream_t);
 bool streams_norm_ok(int, int64_t);
 void launch_streams_norm(bool, float*, const int32_t*, const void*, int, const void*, int64_t,
                          const float*, const float*, const float*, const float*, float, bool, void*,
@@ -802,10 +805,17 @@ void attn_keep_window(const Tensor& q, const Tensor& k_cache, const Tensor& v_ca
                      reinterpret_cast<uintptr_t>(out.data_ptr()) % 8 == 0 &&
                      (gw == 1 || (gs % 4 == 0 && reinterpret_cast<uintptr_t>(gp) % 8 == 0));
   TORCH_CHECK(short_rows >= 0 && short_rows <= 65535 && G <= 65535, "attn_keep_window: short_rows");
-  if (short_rows > 0 && !(tiles && H / G >= 16)) {
-    // sequences of at most short_rows rows each (decode section): one workgroup per
-    // (sequence, key/value head) on the FMA kernel; groups of 16 heads or more fill the MFMA
-    // tiles' columns and run there; falls through if the LDS is too small
+  if (short_rows > 0 && tiles) {
+    // sequences of at most short_rows rows each (decode section): their pages split over waves
+    return rfqmix::launch_attn_keep_split(
+        f32p(q, "q"), k_cache.data_ptr(), v_cache.data_ptr(), vrs, i32p(bt, "block_tables", 0),
+        (int)bt.size(1), i32p(q_start, "q_start", NB), i32p(q_len, "q_len", NB), i32p(kv_len, "kv_len", NB),
+        NB, (int)short_rows, hb, gp, gs, gw, out.data_ptr(), out.stride(0), (float)scale, (int)window,
+        (int)keep_first, sigmoid, H, G, E, (int)vdim, shared, (float)softcap, (float)out_mult, stream());
+  }
+  if (short_rows > 0) {
+    // the same on the FMA kernel, one workgroup per (sequence, key/value head); falls through if
+    // the LDS is too small
     const int kt = rfqmix::launch_attn_keep_decode(
         f32, f32p(q, "q"), k_cache.data_ptr(), v_cache.data_ptr(), vrs, i32p(bt, "block_tables", 0),
         (int)bt.size(1), i32p(q_start, "q_start", NB), i32p(q_len, "q_len", NB),
@@ -820,8 +830,7 @@ void attn_keep_window(const Tensor& q, const Tensor& k_cache, const Tensor& v_ca
         (int)bt.size(1), i32p(q_start, "q_start", NB), i32p(q_len, "q_len", NB),
         i32p(kv_len, "kv_len", NB), i32p(work_seq, "work_seq", W), i32p(work_qblk, "work_qblk", W),
         W, hb, gp, gs, gw, out.data_ptr(), out.stride(0), (float)scale, (int)window, (int)keep_first,
-        sigmoid, H, G, E, (int)vdim, BS, shared, NB, (int)short_rows, (float)softcap, (float)out_mult,
-        stream());
+        sigmoid, H, G, E, (int)vdim, BS, shared, (float)softcap, (float)out_mult, stream());
     return;
   }
   const bool ok = rfqmix::launch_attn_keep_window(

@@ -1,0 +1,92 @@
+"""Decode rows of attn_keep_window with the pages split over waves (csrc/kernels/mix_keep_split.hip):
+contexts around pages and waves, head groups around the sixteen columns, every option."""
+import pytest
+import torch
+
+from replisense_rfq_amd import ops
+from replisense_rfq_amd.ops import reference as ref
+
+pytestmark = pytest.mark.gpu
+DEV, BS = "cuda", 32
+# (cached tokens, rows): shorter than a page, page edges, one piece per wave and one more, a short
+# extend, a padding sequence without rows
+SEQS = [(1, 1), (31, 1), (32, 1), (33, 1), (129, 1), (257, 1), (300, 5), (40, 0), (700, 1), (70, 33)]
+
+
+def _check(H, G, E, vd, shared, seqs=SEQS, spoil=None, **opt):
+    g = torch.Generator().manual_seed(H + E + vd)
+    need = [(n + BS - 1) // BS for n, _ in seqs]
+    perm = torch.randperm(sum(need), generator=g).tolist()
+    tables, at = [], 0
+    for nb in need:
+        tables.append(perm[at:at + nb] + [sum(need)] * (max(need) - nb))
+        at += nb
+    nb = sum(need) + 1
+    k = torch.randn(nb, G, BS, E, generator=g).bfloat16()
+    v = k if shared else torch.randn(nb, G, BS, vd, generator=g).bfloat16()
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32)  # noqa: E731
+    ql, kl, bt = i32([r for _, r in seqs]), i32([n for n, _ in seqs]), i32(tables)
+    for i, (n, r) in enumerate(seqs):            # what was never written may be anything
+        if n % BS:
+            for x in (k, v):
+                x[tables[i][n // BS], :, n % BS:] = float("nan")
+        if spoil is not None and n > spoil and opt.get("window"):
+            for x in (k, v):                     # a key that no row sees any more
+                x[tables[i][spoil // BS], :, spoil % BS] = float("inf")
+    qs, T = torch.cumsum(ql, 0).int() - ql, int(ql.sum())
+    q = torch.randn(T, H, E, generator=g) * 2
+    gate = opt.pop("gate", None)
+    gate = None if gate is None else torch.randn(T, H * (vd if gate == "output" else 1), generator=g).bfloat16()
+    bias = torch.randn(H, generator=g) - 1 if opt.pop("bias", False) else None
+    out = torch.zeros(T, H * vd, dtype=torch.bfloat16)
+    args = lambda d: (vd, *(x.to(d) for x in (bt, qs, ql, kl)))  # noqa: E731
+    kc, vc = (torch.nan_to_num(x.float(), nan=0.0, posinf=0.0).bfloat16() for x in (k, v))
+    ref.attn_keep_window(q, kc, vc, *args("cpu"), bias, gate, out, E ** -0.5, opt.get("window", 0),
+                         opt.get("keep_first", 0), opt.get("sigmoid", False), opt.get("softcap", 0.0),
+                         opt.get("out_mult", 1.0))
+    got = torch.full_like(out, 7.0).to(DEV)
+    kd = k.to(DEV)
+    m = lambda x: None if x is None else x.to(DEV)  # noqa: E731
+    zero = torch.zeros(len(seqs), dtype=torch.int32, device=DEV)
+    ops.attn_keep_window(q.to(DEV), kd, kd if shared else v.to(DEV), *args(DEV), zero, zero, m(bias), m(gate), got,
+                         E ** -0.5, short_rows=max(r for _, r in seqs), **opt)
+    # both sides round to bf16, whose neighbouring values are up to 2^-7 of the value apart: where the
+    # fp32 results lie on two sides of a tie they end one spacing apart.  Queries of keys wider than
+    # 320 entries enter the products as bf16: four times that.
+    tol = 2.0 ** -7 if E <= 320 else 2.0 ** -5
+    err = (got.cpu().float() - out.float()).abs()
+    assert float(err.max()) <= tol * max(1.0, float(out.float().abs().max()))
+    assert float((err / out.float().abs().clamp_min(0.25)).mean()) <= tol
+
+
+@pytest.mark.parametrize("H,G", [(4, 4), (6, 2), (32, 8), (32, 2), (17, 1), (40, 1)])
+def test_head_groups_around_the_columns(H, G):
+    _check(H, G, 128, 128, False, softcap=30.0, out_mult=0.6)
+
+
+@pytest.mark.parametrize("E,vd", [(32, 32), (64, 128), (96, 64), (128, 32)])
+def test_plain_sizes(E, vd):
+    _check(8, 2, E, vd, False, bias=True, gate="output")
+
+
+@pytest.mark.parametrize("E,vd,H", [(96, 64, 8), (128, 64, 4), (128, 96, 16), (160, 128, 8), (192, 128, 20),
+                                    (320, 256, 16), (576, 512, 32), (576, 512, 5)])
+def test_shared_sizes(E, vd, H):
+    _check(H, 1, E, vd, True, bias=True, gate="head")
+
+
+@pytest.mark.parametrize("sigmoid", [False, True])
+@pytest.mark.parametrize("window,keep", [(1, 0), (33, 0), (64, 5), (100, 64), (512, 40)])
+def test_windows_and_kept_tokens(window, keep, sigmoid):
+    _check(32, 8, 128, 128, False, window=window, keep_first=keep, sigmoid=sigmoid, bias=True)
+    _check(16, 1, 576, 512, True, window=window, keep_first=keep, bias=True)
+
+
+def test_many_sequences_take_four_waves():
+    _check(32, 8, 128, 128, False, seqs=[(1 + 37 * i % 400, 1) for i in range(40)], softcap=20.0)
+
+
+def test_a_key_outside_the_window_may_hold_infinities():
+    seqs = [(200, 1), (333, 1), (129, 1)]
+    _check(32, 8, 128, 128, False, seqs=seqs, spoil=20, window=64, keep_first=4)
+    _check(16, 1, 576, 512, True, seqs=seqs, spoil=20, window=64, keep_first=4)
