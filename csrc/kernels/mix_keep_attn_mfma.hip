@@ -1,27 +1,34 @@
-// attn_keep_window on MFMA tiles (bf16 pages of 32 tokens, key width a multiple of 32, value
-// width a multiple of 16).  Semantics of mix_keep_attn.hip: sliding window with kept first
+// attn_keep_window on MFMA tiles, prompt rows (bf16 pages of 32 tokens, key width a multiple of 32,
+// value width a multiple of 32).  Semantics of mix_keep_attn.hip: sliding window with kept first
 // tokens; softmax, softmax with a sink, or unnormalised sigmoid weights; optional output gate
 // (a column per head, or gate_w = vdim: one per output, rows 8-byte aligned);
 // the values may be the leading entries of the key rows themselves (latent attention).
-//
-// One workgroup per (work item, HPW heads of one key/value head); a work item is (sequence,
-// block of 32 queries).  Its 2 HPW waves are (16 queries) x (head): a wave keeps the running
-// maximum and sum of its 16 query columns and the weighted values O^T [vdim x 16] in
-// registers.  A key tile is one page: the head group's key rows go to LDS as they lie in the
-// page, its value rows likewise (read back transposed, ds_read_tr16_b64); with shared pages
-// the key rows are staged once and read both ways.  The next page's pieces are loaded into
-// registers while the current one is multiplied.  Pages between the kept first tokens and the
-// window are never read.
-//
 // Decode rows have a kernel of their own (mix_keep_split.hip).
+//
+// One workgroup per (work item, HPW heads of one key/value head); a work item is (sequence, block of
+// 32 queries).  Its 2 HPW waves are (16 queries) x (head): a wave keeps the running maximum and sum of
+// its 16 query columns and the weighted values O^T [vdim x 16] in registers.  A key tile is one page,
+// staged in LDS for all heads of the workgroup, the next page while this one is multiplied; one barrier
+// per page.  Pages between the kept first tokens and the window are never read.
 //
 //   S^T[key, query] = K[key, :] . Q[query, :]   v_mfma_f32_16x16x32_bf16, A = key rows from LDS,
 //                     B = the queries in registers as bf16 hi (+ lo for keys of up to 320
-//                     entries: they arrive in fp32 and are not rounded a second time)
-//   scale, mask, weights per query column in fp32
-//   O^T[dv, query] += V^T[dv, keys] . P^T[keys, query]   A = two transposed reads of V, B = the
-//                     weights straight from the score registers as bf16 hi + lo parts (two
-//                     MFMAs), so the weights keep fp32's precision
+//                     entries: they arrive in fp32 and are not rounded a second time), already
+//                     times the scale and log2 e
+//   cap, mask, weights per query column in fp32, base 2
+//   O^T[dv, query] += V^T[dv, keys] . P^T[keys, query]   A = two transposed reads of V
+//                     (ds_read_tr16_b64), B = the weights straight from the score registers as bf16
+//                     hi + lo parts (two MFMAs), so the weights keep fp32's precision
+//
+// What bounds it: the vector instructions between the products, and their latency.  Pages without an
+// edge inside skip the masks, the maximum moves only when a score passes it by 2^11 (so the
+// accumulators are rarely rescaled), rows meet by lane swaps instead of LDS, one barrier a page, and a
+// sequence's last blocks, which see the most keys, start first.  Measured with the append before it,
+// without -> with these: prompts of 2,048 and 600 tokens (32 heads over 8 of 128, softcap) 234 -> 223 us,
+// three ragged prompts with sigmoid weights and a window of 512 125 -> 87 us, one prompt of 2,048 with
+// 64 heads and a window 268 -> 174 us.  What is left of the first is the longest block's chain of 64
+// pages.  32 x 32 tiles, a wave per 32 queries, took 217 and 116 us there and lost 20 % on prompts of a
+// few hundred tokens; two waves sharing such a wave's pages 251 and 119.
 #include "common.h"
 #include "mix_common.h"
 
@@ -36,6 +43,8 @@ namespace {
 constexpr int WQB = 32;                 // queries per work item
 constexpr int WBS = 32;                 // keys per tile = page size
 constexpr float kNegInfW = -__builtin_huge_valf();
+constexpr float kLog2e = 1.44269504088896f;
+constexpr float kDeferW = 11.f;         // base 2
 
 __device__ __forceinline__ void split_bf16w(const float* f, s16x8& hi, s16x8& lo) {
   float r[8];
@@ -44,266 +53,28 @@ __device__ __forceinline__ void split_bf16w(const float* f, s16x8& hi, s16x8& lo
   for (int i = 0; i < 8; ++i) r[i] = f[i] - rfq::bf2f_s(hi[i]);
   lo = rfq::pack8(r);
 }
-}  // namespace
 
-// DK = E / 32, DV = vdim / 16, HPW heads per workgroup, SHARED: values = leading entries of the
-// key rows, QLO: the queries' lo parts are multiplied too.
-template <int DK, int DV, int HPW, bool SHARED, bool QLO>
-__global__ __launch_bounds__(128 * HPW) void attn_keep_mfma_kernel(
-    const float* __restrict__ q, const bf16_t* __restrict__ k_cache,
-    const bf16_t* __restrict__ v_cache, int64_t vrs, const int32_t* __restrict__ block_tables,
-    int maxb, const int32_t* __restrict__ q_start, const int32_t* __restrict__ q_len,
-    const int32_t* __restrict__ kv_len, const int32_t* __restrict__ work_seq,
-    const int32_t* __restrict__ work_qblk, const float* __restrict__ head_bias,
-    const bf16_t* __restrict__ gate, int64_t gate_stride, int gate_w,
-    bf16_t* __restrict__ out, int64_t out_stride, float scale, int window, int keep_first, int sigmoid, int H, int G,
-    float softcap, float out_mult) {
-  constexpr int E = 32 * DK, vdim = 16 * DV, NT = 128 * HPW;
-  constexpr int KRS = E + 8;                       // shorts per key row in LDS (+ 16 bytes)
-  constexpr int VRS = SHARED ? KRS : vdim + 8;     // shorts per value row
-  const int s = work_seq[blockIdx.x];
-  if (s < 0) return;
-  const int ql = q_len[s];
-  const int32_t* bt = block_tables + (int64_t)s * maxb;
-  const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
-  const int col = lane & 15, grp = lane >> 4;
-  const int rep = H / G;
-  const int g = ((int)blockIdx.y * HPW) / rep;
-  const int hh = (int)blockIdx.y * HPW + (wid >> 1);   // columns: 16 queries of this head
-  const int i0 = work_qblk[blockIdx.x] * WQB;
-  if (i0 >= ql) return;
-  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-  short* Ks = reinterpret_cast<short*>(smem);      // [32][KRS]
-  short* Vs = SHARED ? Ks : Ks + WBS * KRS;        // [32][VRS]
-
-  const int nq = min(WQB, ql - i0);
-  const int p0 = kv_len[s] - ql + i0;
-  const int plast = p0 + nq - 1;
-  const int jwin = window > 0 ? max(0, p0 - window + 1) : 0;
-  const int kf = window > 0 ? min(keep_first, jwin) : 0;     // kept keys before the window
-  const int row = (wid & 1) * 16 + col;            // this lane's query of the block
-  const int pi = p0 + row;
-  const bool qlive = row < nq;
-  const int64_t t = q_start[s] + i0 + row;
-
-  s16x8 qhi[DK], qlo[QLO ? DK : 1];
-  {
-    const float* qp = q + (t * H + hh) * E + grp * 8;
-#pragma unroll
-    for (int ks = 0; ks < DK; ++ks) {
-      float f[8];
-      if (qlive) {
-        const float4 a = *reinterpret_cast<const float4*>(qp + ks * 32);
-        const float4 b = *reinterpret_cast<const float4*>(qp + ks * 32 + 4);
-        f[0] = a.x; f[1] = a.y; f[2] = a.z; f[3] = a.w; f[4] = b.x; f[5] = b.y; f[6] = b.z; f[7] = b.w;
-      } else {
-#pragma unroll
-        for (int e = 0; e < 8; ++e) f[e] = 0.f;
-      }
-      if constexpr (QLO) {
-        split_bf16w(f, qhi[ks], qlo[ks]);
-      } else {
-        qhi[ks] = rfq::pack8(f);
-      }
-    }
-  }
-  f32x4 o[DV];
-#pragma unroll
-  for (int m = 0; m < DV; ++m) o[m] = (f32x4){0.f, 0.f, 0.f, 0.f};
-  const float hb = head_bias != nullptr ? head_bias[hh] : 0.f;
-  const bool sink = !sigmoid && head_bias != nullptr;
-  float mrun = sink ? hb : kNegInfW, lrun = sink ? 1.f : 0.f;
-
-  constexpr int NKV = (WBS * E / 8 + NT - 1) / NT;
-  constexpr int NVV = SHARED ? 1 : (WBS * vdim / 8 + NT - 1) / NT;
-  s16x8 kreg[NKV], vreg[NVV];
-  auto fetch = [&](int pg) {
-    const int64_t page = bt[pg];
-    const s16x8* kp = reinterpret_cast<const s16x8*>(k_cache + ((page * G + g) * WBS) * (int64_t)E);
-#pragma unroll
-    for (int a = 0; a < NKV; ++a) {
-      const int x = tid + a * NT;
-      if (x < WBS * E / 8) kreg[a] = kp[x];
-    }
-    if constexpr (!SHARED) {
-      const bf16_t* vb = v_cache + ((page * G + g) * WBS) * vrs;
-#pragma unroll
-      for (int a = 0; a < NVV; ++a) {
-        const int x = tid + a * NT;
-        if (x < WBS * vdim / 8) {
-          const int jj = x / (vdim / 8), c = x - jj * (vdim / 8);
-          vreg[a] = *reinterpret_cast<const s16x8*>(vb + jj * vrs + c * 8);
-        }
-      }
-    }
-  };
-  // pages [0 .. pg_keep] hold the kept first tokens, pages [pg_win .. pg_last] the window
-  const int pg_last = plast / WBS;
-  const int pg_keep = kf > 0 ? (kf - 1) / WBS : -1;
-  const int pg_win = jwin / WBS;
-  auto next_page = [&](int pg) { return (pg == pg_keep && pg_win > pg) ? pg_win : pg + 1; };
-  int pg = kf > 0 ? 0 : pg_win;
-  fetch(pg);
-  while (pg <= pg_last) {
-    const int jb = pg * WBS;
-    const int pg_next = next_page(pg);
-    __syncthreads();                                     // the last tile's reads are done
-#pragma unroll
-    for (int a = 0; a < NKV; ++a) {
-      const int x = tid + a * NT;
-      if (x < WBS * E / 8) {
-        const int jj = x / (E / 8), c = x - jj * (E / 8);
-        s16x8 v = kreg[a];
-        if (SHARED && jb + jj > plast) v = (s16x8){0, 0, 0, 0, 0, 0, 0, 0};   // rows never written
-        *reinterpret_cast<s16x8*>(Ks + jj * KRS + c * 8) = v;
-      }
-    }
-    if constexpr (!SHARED) {
-#pragma unroll
-      for (int a = 0; a < NVV; ++a) {
-        const int x = tid + a * NT;
-        if (x < WBS * vdim / 8) {
-          const int jj = x / (vdim / 8), c = x - jj * (vdim / 8);
-          s16x8 v = vreg[a];
-          if (jb + jj > plast) v = (s16x8){0, 0, 0, 0, 0, 0, 0, 0};
-          *reinterpret_cast<s16x8*>(Vs + jj * VRS + c * 8) = v;
-        }
-      }
-    }
-    __syncthreads();
-    if (pg_next <= pg_last) fetch(pg_next);              // in flight during this tile's MFMAs
-    // scores of the two 16-key halves
-    f32x4 sc[2];
-#pragma unroll
-    for (int kt = 0; kt < 2; ++kt) {
-      sc[kt] = (f32x4){0.f, 0.f, 0.f, 0.f};
-      const short* kr = Ks + (kt * 16 + col) * KRS + grp * 8;
-#pragma unroll
-      for (int ks = 0; ks < DK; ++ks) {
-        const s16x8 kfr = *reinterpret_cast<const s16x8*>(kr + ks * 32);
-        sc[kt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(kfr), as_bf16x8(qhi[ks]), sc[kt], 0, 0, 0);
-        if constexpr (QLO)
-          sc[kt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(kfr), as_bf16x8(qlo[ks]), sc[kt], 0, 0, 0);
-      }
-    }
-    // the scaled scores, capped where a cap is given: c tanh(s / c) = c - 2 c / (exp(2 s / c) + 1)
-#pragma unroll
-    for (int kt = 0; kt < 2; ++kt) sc[kt] *= scale;
-    if (softcap > 0.f) {
-      const float two_c = 2.f * softcap, inv = 2.f / softcap;
-#pragma unroll
-      for (int kt = 0; kt < 2; ++kt)
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-          sc[kt][i] = softcap - two_c * __builtin_amdgcn_rcpf(__expf(sc[kt][i] * inv) + 1.f);
-    }
-    float pv[8];
-    float alpha = 1.f;
-    if (sigmoid) {
-#pragma unroll
-      for (int kt = 0; kt < 2; ++kt)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const int j = jb + kt * 16 + grp * 4 + i;
-          const bool ok = qlive && j <= pi && (window <= 0 || pi - j < window || j < keep_first);
-          pv[kt * 4 + i] = ok ? 1.0f / (1.0f + __expf(-(sc[kt][i] + hb))) : 0.f;
-        }
-    } else {
-      float mx = kNegInfW;
-#pragma unroll
-      for (int kt = 0; kt < 2; ++kt)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const int j = jb + kt * 16 + grp * 4 + i;
-          const bool ok = qlive && j <= pi && (window <= 0 || pi - j < window || j < keep_first);
-          sc[kt][i] = ok ? sc[kt][i] : kNegInfW;
-          mx = fmaxf(mx, sc[kt][i]);
-        }
-      mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-      mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-      const float mn = fmaxf(mrun, mx);
-      float sum = 0.f;
-#pragma unroll
-      for (int kt = 0; kt < 2; ++kt)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const float e = sc[kt][i] == kNegInfW ? 0.f : __expf(sc[kt][i] - mn);
-          pv[kt * 4 + i] = e;
-          sum += e;
-        }
-      sum += __shfl_xor(sum, 16, 64);
-      sum += __shfl_xor(sum, 32, 64);
-      alpha = mrun == kNegInfW ? 0.f : __expf(mrun - mn);
-      lrun = lrun * alpha + sum;
-      mrun = mn;
-    }
-    s16x8 phi, plo;
-    split_bf16w(pv, phi, plo);
-    // the accumulators are rescaled only on pages that moved some column's running maximum
-    // (wave-uniform test; a factor of exactly 1 changes nothing)
-    if (__builtin_amdgcn_ballot_w64(alpha != 1.f) != 0ull) {
-#pragma unroll
-      for (int m = 0; m < DV; ++m) o[m] *= alpha;
-    }
-    // transposed reads: a 16-lane group takes 4 key rows x 16 value columns, lane `col`
-    // receives its column (keys 4 grp .. 4 grp + 3 of each 16-key half)
-    const short* v0 = Vs + (4 * grp + (col >> 2)) * VRS + 4 * (col & 3);
-    const short* v1 = v0 + 16 * VRS;
-#pragma unroll
-    for (int m = 0; m < DV; ++m) {
-      const s16x4 a0 = rfq::ds_read_tr16(v0 + 16 * m);
-      const s16x4 a1 = rfq::ds_read_tr16(v1 + 16 * m);
-      const s16x8 a = (s16x8){a0[0], a0[1], a0[2], a0[3], a1[0], a1[1], a1[2], a1[3]};
-      o[m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(a), as_bf16x8(phi), o[m], 0, 0, 0);
-      o[m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(a), as_bf16x8(plo), o[m], 0, 0, 0);
-    }
-    pg = pg_next;
-  }
-  // lane (col, grp) holds value channels 16 m + 4 grp .. + 3 of its column: 8-byte stores
-  if (qlive) {
-    float mul = sigmoid ? out_mult : (lrun > 0.f ? out_mult / lrun : 0.f);
-    if (gate != nullptr && gate_w == 1) mul /= 1.0f + __expf(-ldf(gate + t * gate_stride + hh));
-    // a gate column per output: four neighbouring logits per 16-channel block, 8-byte reads
-    const bf16_t* grow = gate != nullptr && gate_w > 1
-                             ? gate + t * gate_stride + (int64_t)hh * vdim + grp * 4 : nullptr;
-    bf16_t* orow = out + t * out_stride + (int64_t)hh * vdim + grp * 4;
-#pragma unroll
-    for (int m = 0; m < DV; ++m) {
-      if (grow != nullptr) {
-        const uint2 gu = *reinterpret_cast<const uint2*>(grow + m * 16);
-        o[m][0] /= 1.0f + __expf(-__uint_as_float(gu.x << 16));
-        o[m][1] /= 1.0f + __expf(-__uint_as_float(gu.x & 0xffff0000u));
-        o[m][2] /= 1.0f + __expf(-__uint_as_float(gu.y << 16));
-        o[m][3] /= 1.0f + __expf(-__uint_as_float(gu.y & 0xffff0000u));
-      }
-      bf16_t b[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) stf(&b[i], o[m][i] * mul);
-      *reinterpret_cast<uint2*>(orow + m * 16) =
-          make_uint2((uint32_t)b[0] | ((uint32_t)b[1] << 16), (uint32_t)b[2] | ((uint32_t)b[3] << 16));
-    }
-  }
+// the value of the lane 32 away beside one's own
+__device__ __forceinline__ float other_half_max(float x) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+__device__ __forceinline__ float both_halves_sum(float x) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
 
-// ------------------------------------------------------------------ launcher
-namespace {
-bool plain_sizes(int DK, int DV) { return DK >= 1 && DK <= 4 && (DV == 2 || DV == 4 || DV == 8); }
-bool shared_sizes(int DK, int DV) {
-  return (DK == 3 && DV == 4) || (DK == 4 && (DV == 4 || DV == 6)) || (DK == 5 && DV == 8) ||
-         (DK == 6 && DV == 8) || (DK == 10 && DV == 16) || (DK == 18 && DV == 32);
+template <int DK, int DV, bool SHARED>
+constexpr int keep_page_shorts() {
+  return WBS * (32 * DK + 8) + (SHARED ? 0 : WBS * (16 * DV + 8));
 }
 }  // namespace
-
-bool keep_mfma_ok(int E, int vdim, int BS, bool shared) {
-  if (BS != WBS || E % 32 != 0 || vdim % 16 != 0) return false;
-  return shared ? shared_sizes(E / 32, vdim / 16) : plain_sizes(E / 32, vdim / 16);
-}
 
 struct KeepArgs {
   const float* q;
   const void *k_cache, *v_cache;
   int64_t vrs;
-  const int32_t *bt;
+  const int32_t* bt;
   int maxb;
   const int32_t *q_start, *q_len, *kv_len, *work_seq, *work_qblk;
   int W;
@@ -321,31 +92,485 @@ struct KeepArgs {
   hipStream_t s;
 };
 
-template <int DK, int DV, int HPW, bool SHARED>
-static void launch_keep_mfma_one(const KeepArgs& a) {
-  constexpr bool QLO = DK <= 10;       // wider keys: the queries' registers go to the accumulators
-  constexpr int E = 32 * DK, vdim = 16 * DV;
-  const size_t lds = (size_t)(WBS * (E + 8) + (SHARED ? 0 : WBS * (vdim + 8))) * 2;
-  static bool attr = false;
-  if (!attr) {
-    (void)hipFuncSetAttribute(
-        reinterpret_cast<const void*>(&attn_keep_mfma_kernel<DK, DV, HPW, SHARED, QLO>),
-        hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
-    attr = true;
+// the same over lanes 16 away
+__device__ __forceinline__ float other_row_max(float x) {
+  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+__device__ __forceinline__ float both_rows_sum(float x) {
+  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+
+// lane (col, grp) holds value channels 16 m + 4 grp .. + 3 of its query: 8-byte stores
+template <int DV, int MODE>
+__device__ __forceinline__ void store_rows(const KeepArgs& a, f32x4 (&o)[DV], float lrun, int64_t t, int hh, int grp,
+                                           bool qlive) {
+  constexpr int vdim = 16 * DV;
+  const float l = both_halves_sum(both_rows_sum(lrun));
+  if (!qlive) return;
+  const bf16_t* gate = static_cast<const bf16_t*>(a.gate);
+  float mul = MODE == 2 ? a.out_mult : (l > 0.f ? a.out_mult / l : 0.f);
+  if (gate != nullptr && a.gate_w == 1) mul /= 1.0f + __expf(-ldf(gate + t * a.gate_stride + hh));
+  // a gate column per output: four neighbouring logits, 8-byte reads
+  const bf16_t* grow = gate != nullptr && a.gate_w > 1 ? gate + t * a.gate_stride + (int64_t)hh * vdim + grp * 4 : nullptr;
+  bf16_t* orow = static_cast<bf16_t*>(a.out) + t * a.out_stride + (int64_t)hh * vdim + grp * 4;
+#pragma unroll
+  for (int m = 0; m < DV; ++m) {
+    float y[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) y[i] = o[m][i] * mul;
+    if (grow != nullptr) {
+      const uint2 gu = *reinterpret_cast<const uint2*>(grow + m * 16);
+      y[0] /= 1.0f + __expf(-__uint_as_float(gu.x << 16));
+      y[1] /= 1.0f + __expf(-__uint_as_float(gu.x & 0xffff0000u));
+      y[2] /= 1.0f + __expf(-__uint_as_float(gu.y << 16));
+      y[3] /= 1.0f + __expf(-__uint_as_float(gu.y & 0xffff0000u));
+    }
+    *reinterpret_cast<uint2*>(orow + m * 16) = make_uint2(rfq::pack_bf16x2(y[0], y[1]), rfq::pack_bf16x2(y[2], y[3]));
   }
-  const dim3 grid(a.W, a.H / HPW);
-  hipLaunchKernelGGL((attn_keep_mfma_kernel<DK, DV, HPW, SHARED, QLO>), grid,
-                     dim3(128 * HPW), lds, a.s, a.q, (const bf16_t*)a.k_cache,
-                     (const bf16_t*)a.v_cache, a.vrs, a.bt, a.maxb, a.q_start, a.q_len, a.kv_len,
-                     a.work_seq, a.work_qblk, a.head_bias, (const bf16_t*)a.gate, a.gate_stride,
-                     a.gate_w, (bf16_t*)a.out, a.out_stride, a.scale, a.window, a.keep_first, (int)a.sigmoid,
-                     a.H, a.G, a.softcap, a.out_mult);
+}
+
+// DK = E / 32, DV = vdim / 16, HPW heads per workgroup, SHARED: values = leading entries of the
+// key rows, MODE: 0 softmax, 1 softmax of capped scores, 2 sigmoid.
+template <int DK, int DV, int HPW, bool SHARED, int MODE>
+__global__ __launch_bounds__(128 * HPW) void attn_keep_mfma_kernel(const KeepArgs a) {
+  constexpr int E = 32 * DK, vdim = 16 * DV, NT = 128 * HPW;
+  constexpr int KRS = E + 8;                       // shorts per key row in LDS (+ 16 bytes)
+  constexpr int VRS = SHARED ? KRS : vdim + 8;     // shorts per value row
+  constexpr int PGS = keep_page_shorts<DK, DV, SHARED>();
+  const int item = gridDim.x - 1 - blockIdx.x;     // a sequence's later blocks see the most keys: they start first
+  const int s = a.work_seq[item];
+  if (s < 0) return;
+  const int ql = a.q_len[s];
+  const int i0 = a.work_qblk[item] * WQB;
+  if (i0 >= ql) return;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int col = lane & 15, grp = lane >> 4;
+  const int g = ((int)blockIdx.y * HPW) / (a.H / a.G);
+  const int hh = (int)blockIdx.y * HPW + (wid >> 1);
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  short* const pages = reinterpret_cast<short*>(smem);       // two of them
+
+  const int nq = min(WQB, ql - i0);
+  const int p0 = a.kv_len[s] - ql + i0, plast = p0 + nq - 1;
+  const int window = a.window, keep_first = a.keep_first;
+  const int jwin = window > 0 ? max(0, p0 - window + 1) : 0;
+  const int kf = window > 0 ? min(keep_first, jwin) : 0;     // kept keys before the window
+  const int row = (wid & 1) * 16 + col, pi = p0 + row;       // this lane's query
+  const bool qlive = row < nq;
+  const int64_t t = a.q_start[s] + i0 + (qlive ? row : 0);
+  typedef const __attribute__((address_space(4))) int32_t const_i32;
+  const_i32* bt = (const_i32*)(uintptr_t)(a.bt + (int64_t)s * a.maxb);
+
+  // scores arrive as exponents of 2: s log2 e; 2 s log2 e / cap; -s log2 e (sigmoid)
+  const float qmul = a.scale * (MODE == 1 ? 2.f * kLog2e / a.softcap : MODE == 2 ? -kLog2e : kLog2e);
+  const float cap2 = MODE == 1 ? a.softcap * kLog2e : 0.f;
+  s16x8 qhi[DK], qlo[DK];
+  {
+    const float* qp = a.q + (t * a.H + hh) * E + grp * 8;
+#pragma unroll
+    for (int ks = 0; ks < DK; ++ks) {
+      const float4 x = *reinterpret_cast<const float4*>(qp + ks * 32);
+      const float4 y = *reinterpret_cast<const float4*>(qp + ks * 32 + 4);
+      const float f[8] = {x.x * qmul, x.y * qmul, x.z * qmul, x.w * qmul, y.x * qmul, y.y * qmul, y.z * qmul, y.w * qmul};
+      split_bf16w(f, qhi[ks], qlo[ks]);
+    }
+  }
+  f32x4 o[DV];
+#pragma unroll
+  for (int m = 0; m < DV; ++m) o[m] = (f32x4){0.f, 0.f, 0.f, 0.f};
+  const float hb = a.head_bias != nullptr ? a.head_bias[hh] * kLog2e : 0.f;
+  const bool sink = MODE != 2 && a.head_bias != nullptr;
+  // the sink is one more entry of the row: it starts the maximum, and one lane's part of the sum
+  float mrun = sink ? hb : kNegInfW, lrun = sink && grp == 0 ? 1.f : 0.f;
+
+  // ---- staging
+  constexpr int NKV = (WBS * E / 8 + NT - 1) / NT;
+  constexpr int NVV = SHARED ? 1 : (WBS * vdim / 8 + NT - 1) / NT;
+  s16x8 kreg[NKV], vreg[NVV];
+  auto fetch = [&](int page) {
+    const int64_t at = ((int64_t)page * a.G + g) * WBS;      // the page's first slot
+    const bf16_t* kb = static_cast<const bf16_t*>(a.k_cache) + at * E;
+#pragma unroll
+    for (int i = 0; i < NKV; ++i) {
+      const int x = tid + i * NT;
+      if (x < WBS * E / 8) kreg[i] = reinterpret_cast<const s16x8*>(kb)[x];
+    }
+    if constexpr (!SHARED) {
+      const bf16_t* vb = static_cast<const bf16_t*>(a.v_cache) + at * a.vrs;
+#pragma unroll
+      for (int i = 0; i < NVV; ++i) {
+        const int x = tid + i * NT;
+        if (x < WBS * vdim / 8) {
+          const int jj = x / (vdim / 8), c = x - jj * (vdim / 8);
+          vreg[i] = *reinterpret_cast<const s16x8*>(vb + jj * a.vrs + c * 8);
+        }
+      }
+    }
+  };
+  // Rows past the sequence's end were never written and may hold anything: zeros.
+  auto stage = [&](int jb, int buf) {
+    short* Ks = pages + buf * PGS;
+    short* Vs = SHARED ? Ks : Ks + WBS * KRS;
+    const bool tail = jb + WBS - 1 > plast;
+#pragma unroll
+    for (int i = 0; i < NKV; ++i) {
+      const int x = tid + i * NT;
+      if (x < WBS * E / 8) {
+        const int jj = x / (E / 8), c = x - jj * (E / 8);
+        s16x8 v = kreg[i];
+        if (SHARED && tail && jb + jj > plast) v = (s16x8){0, 0, 0, 0, 0, 0, 0, 0};
+        *reinterpret_cast<s16x8*>(Ks + jj * KRS + c * 8) = v;
+      }
+    }
+    if constexpr (!SHARED) {
+#pragma unroll
+      for (int i = 0; i < NVV; ++i) {
+        const int x = tid + i * NT;
+        if (x < WBS * vdim / 8) {
+          const int jj = x / (vdim / 8), c = x - jj * (vdim / 8);
+          s16x8 v = vreg[i];
+          if (tail && jb + jj > plast) v = (s16x8){0, 0, 0, 0, 0, 0, 0, 0};
+          *reinterpret_cast<s16x8*>(Vs + jj * VRS + c * 8) = v;
+        }
+      }
+    }
+  };
+  const int kat = col * KRS + grp * 8;
+  // transposed reads: a 16-lane group takes 4 key rows x 16 value columns, lane `col` receives its
+  // column (keys 4 grp .. 4 grp + 3 of each 16-key half)
+  const int vat = (4 * grp + (col >> 2)) * VRS + 4 * (col & 3);
+
+  // pages [0 .. pg_keep] hold the kept first tokens, pages [pg_win .. pg_last] the window
+  const int pg_last = plast / WBS;
+  const int pg_keep = kf > 0 ? (kf - 1) / WBS : -1;
+  const int pg_win = jwin / WBS;
+  auto next_page = [&](int pg) { return (pg == pg_keep && pg_win > pg) ? pg_win : pg + 1; };
+  int pg = kf > 0 ? 0 : pg_win, buf = 0;
+  fetch(bt[pg]);
+  stage(pg * WBS, 0);
+  int pn = next_page(pg);
+  if (pn <= pg_last) fetch(bt[pn]);
+  __syncthreads();
+  while (pg <= pg_last) {
+    const int jb = pg * WBS;
+    const short* Ks = pages + buf * PGS;
+    const short* Vs = SHARED ? Ks : Ks + WBS * KRS;
+    f32x4 sc[2][2];                                          // two chains per half page
+#pragma unroll
+    for (int kt = 0; kt < 2; ++kt) {
+      sc[kt][0] = sc[kt][1] = (f32x4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int ks = 0; ks < DK; ++ks) {
+        const s16x8 k = *reinterpret_cast<const s16x8*>(Ks + kat + kt * 16 * KRS + ks * 32);
+        sc[kt][0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(k), as_bf16x8(qhi[ks]), sc[kt][0], 0, 0, 0);
+        sc[kt][1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(k), as_bf16x8(qlo[ks]), sc[kt][1], 0, 0, 0);
+      }
+    }
+    float p[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      float x = sc[i >> 2][0][i & 3] + sc[i >> 2][1][i & 3];
+      if constexpr (MODE == 1) x = cap2 - 2.f * cap2 * __builtin_amdgcn_rcpf(__builtin_amdgcn_exp2f(x) + 1.f);
+      if constexpr (MODE == 2) x = __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(x - hb));
+      p[i] = x;
+    }
+    if (!(jb + WBS - 1 <= p0 && (window <= 0 || plast - jb < window || jb + WBS <= keep_first))) {
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {                          // an edge inside the page
+        const int j = jb + (i >> 2) * 16 + grp * 4 + (i & 3);
+        const bool ok = j <= pi && (window <= 0 || pi - j < window || j < keep_first);
+        p[i] = ok ? p[i] : MODE == 2 ? 0.f : kNegInfW;
+      }
+    }
+    if constexpr (MODE != 2) {
+      float mx = fmaxf(fmaxf(fmaxf(p[0], p[1]), fmaxf(p[2], p[3])), fmaxf(fmaxf(p[4], p[5]), fmaxf(p[6], p[7])));
+      mx = other_half_max(other_row_max(mx));
+      const bool moves = mx > mrun + kDeferW;                // also for the first keys: mrun = -inf
+      if (__builtin_amdgcn_ballot_w64(moves) != 0ull) {
+        const float mn = moves ? mx : mrun;
+        const float alpha = moves ? __builtin_amdgcn_exp2f(mrun - mn) : 1.f;
+        mrun = mn;
+        lrun *= alpha;
+#pragma unroll
+        for (int m = 0; m < DV; ++m) o[m] *= alpha;
+      }
+      const float mu = mrun == kNegInfW ? 0.f : mrun;        // no visible key so far: every weight 0
+      float l0 = 0.f, l1 = 0.f;
+#pragma unroll
+      for (int i = 0; i < 8; i += 2) {
+        p[i] = __builtin_amdgcn_exp2f(p[i] - mu);
+        p[i + 1] = __builtin_amdgcn_exp2f(p[i + 1] - mu);
+        l0 += p[i];
+        l1 += p[i + 1];
+      }
+      lrun += l0 + l1;
+    }
+    s16x8 phi, plo;
+    split_bf16w(p, phi, plo);
+    constexpr int MG = DV % 4 == 0 ? 4 : 2;                  // value blocks taken together
+#pragma unroll
+    for (int m = 0; m < DV; m += MG) {
+      s16x8 v[MG];
+#pragma unroll
+      for (int u = 0; u < MG; ++u) {
+        const s16x4 a0 = rfq::ds_read_tr16(Vs + vat + 16 * (m + u));
+        const s16x4 a1 = rfq::ds_read_tr16(Vs + vat + 16 * VRS + 16 * (m + u));
+        v[u] = (s16x8){a0[0], a0[1], a0[2], a0[3], a1[0], a1[1], a1[2], a1[3]};
+      }
+#pragma unroll
+      for (int u = 0; u < MG; ++u)
+        o[m + u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(v[u]), as_bf16x8(phi), o[m + u], 0, 0, 0);
+#pragma unroll
+      for (int u = 0; u < MG; ++u)
+        o[m + u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(v[u]), as_bf16x8(plo), o[m + u], 0, 0, 0);
+    }
+    pg = pn;
+    if (pg <= pg_last) {
+      stage(pg * WBS, buf ^ 1);          // it has been on its way since the last page
+      pn = next_page(pg);
+      if (pn <= pg_last) fetch(bt[pn]);
+    }
+    __syncthreads();
+    buf ^= 1;
+  }
+  store_rows<DV, MODE>(a, o, lrun, t, hh, grp, qlive);
+}
+
+// Wide latents: keys of 320 or 576 entries whose first 256 or 512 are the values.  32 queries' results
+// (256 registers at 512 values) and the queries themselves (144) leave no room for the rest, so a wave
+// has 16 queries on 16x16x32 tiles, two waves a head, and the page's LDS reads are what bounds it (K
+// rows 36 x 1 KB, V 64 x 512 B a wave and page: 4,350 clocks for eight waves against 3,200 of MFMA).
+// One prompt of 2,048 over 576 (32 heads) took 904 us a pass on the kernel above, 420 here; four of
+// them with 64 heads 3,249 and 1,414.  Pages come by LDS-DMA, the next one during this one; their rows lie unpadded, 16-byte pieces
+// permuted inside each 128 bytes by wide_swizzle(row).
+// Sixteen rows of one piece (a K read) and four neighbouring rows of a pair of pieces beside the next
+// four (a transposed V read) then lie on different banks: the row's parity picks a half of them, bits
+// 1 and 2 the pair, bit 3 the order inside it.
+__device__ __forceinline__ int wide_swizzle(int r) { return ((r >> 1) & 1) << 2 | ((r >> 2) & 1) << 1 | ((r >> 3) & 1); }
+
+template <int DK, int DV, int HPW, int MODE>
+__global__ __launch_bounds__(128 * HPW, 2) void attn_keep_wide_kernel(const KeepArgs a) {
+  constexpr int E = 32 * DK, vdim = 16 * DV, NWV = 2 * HPW, NP = WBS * E / 512, ND = (NP + NWV - 1) / NWV;
+  constexpr bool QLO = DK <= 10;
+  static_assert(E % 64 == 0 && DV % 4 == 0, "whole 128-byte lines");
+  const int item = gridDim.x - 1 - blockIdx.x;     // a sequence's later blocks see the most keys: they start first
+  const int s = a.work_seq[item];
+  if (s < 0) return;
+  const int ql = a.q_len[s];
+  const int i0 = a.work_qblk[item] * WQB;
+  if (i0 >= ql) return;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int col = lane & 15, grp = lane >> 4;
+  const int g = ((int)blockIdx.y * HPW) / (a.H / a.G);
+  const int hh = (int)blockIdx.y * HPW + (wid >> 1);
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  short* const pages = reinterpret_cast<short*>(smem);       // a ring of three
+
+  const int nq = min(WQB, ql - i0);
+  const int p0 = a.kv_len[s] - ql + i0, plast = p0 + nq - 1;
+  const int window = a.window, keep_first = a.keep_first;
+  const int jwin = window > 0 ? max(0, p0 - window + 1) : 0;
+  const int kf = window > 0 ? min(keep_first, jwin) : 0;
+  const int row = (wid & 1) * 16 + col, pi = p0 + row;       // this lane's query
+  const bool qlive = row < nq;
+  const int64_t t = a.q_start[s] + i0 + (qlive ? row : 0);
+  typedef const __attribute__((address_space(4))) int32_t const_i32;
+  const_i32* bt = (const_i32*)(uintptr_t)(a.bt + (int64_t)s * a.maxb);
+
+  const float qmul = a.scale * (MODE == 1 ? 2.f * kLog2e / a.softcap : MODE == 2 ? -kLog2e : kLog2e);
+  const float cap2 = MODE == 1 ? a.softcap * kLog2e : 0.f;
+  s16x8 qhi[DK], qlo[QLO ? DK : 1];
+  {
+    const float* qp = a.q + (t * a.H + hh) * E + grp * 8;
+#pragma unroll
+    for (int ks = 0; ks < DK; ++ks) {
+      const float4 x = *reinterpret_cast<const float4*>(qp + ks * 32);
+      const float4 y = *reinterpret_cast<const float4*>(qp + ks * 32 + 4);
+      const float f[8] = {x.x * qmul, x.y * qmul, x.z * qmul, x.w * qmul, y.x * qmul, y.y * qmul, y.z * qmul, y.w * qmul};
+      if constexpr (QLO) split_bf16w(f, qhi[ks], qlo[ks]);
+      else qhi[ks] = rfq::pack8(f);
+    }
+  }
+  f32x4 o[DV];
+#pragma unroll
+  for (int m = 0; m < DV; ++m) o[m] = (f32x4){0.f, 0.f, 0.f, 0.f};
+  const float hb = a.head_bias != nullptr ? a.head_bias[hh] * kLog2e : 0.f;
+  const bool sink = MODE != 2 && a.head_bias != nullptr;
+  float mrun = sink ? hb : kNegInfW, lrun = sink && grp == 0 ? 1.f : 0.f;      // sums: a quarter per lane
+
+  int src[ND];                                               // this lane's source pieces, in shorts
+#pragma unroll
+  for (int i = 0; i < ND; ++i) {
+    const int p = (wid + i * NWV) * 64 + lane, r = p / (E / 8), c = p - r * (E / 8);
+    src[i] = r * E + ((c & ~7) | ((c & 7) ^ wide_swizzle(r))) * 8;
+  }
+  auto fetch = [&](int page, int buf) {
+    const bf16_t* kb = static_cast<const bf16_t*>(a.k_cache) + ((int64_t)page * a.G + g) * WBS * E;
+#pragma unroll
+    for (int i = 0; i < ND; ++i) {
+      const int piece = wid + i * NWV;
+      if (piece < NP) rfq::glds16(kb + src[i], reinterpret_cast<bf16_t*>(pages + buf * WBS * E + piece * 512));
+    }
+  };
+  // The page has landed for everyone, who is done with the one before the last; rows past the sequence's end were never written: zeros.
+  auto landed = [&](int jb, int buf) {
+    __builtin_amdgcn_s_waitcnt(0x0F70);                      // vmcnt(0)
+    __syncthreads();
+    if (jb + WBS - 1 > plast) {
+      for (int x = max(0, plast + 1 - jb) * (E / 8) + tid; x < WBS * (E / 8); x += 64 * NWV)
+        *reinterpret_cast<s16x8*>(pages + buf * WBS * E + x * 8) = (s16x8){0, 0, 0, 0, 0, 0, 0, 0};
+      __syncthreads();
+    }
+  };
+  // keys: row col (+ 16), entries 32 ks + 8 grp ..; values, transposed: rows 4 grp + col / 4 (+ 16),
+  // channels 16 m + 4 (col % 4) ..
+  const int ksw = wide_swizzle(col), vrow = 4 * grp + (col >> 2), vsw = wide_swizzle(vrow);
+  int kat[2], vat[4];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) kat[i] = col * E + ((4 * i + grp) ^ ksw) * 8;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) vat[i] = vrow * E + ((2 * i + ((col >> 1) & 1)) ^ vsw) * 8 + (col & 1) * 4;
+
+  const int pg_last = plast / WBS;
+  const int pg_keep = kf > 0 ? (kf - 1) / WBS : -1;
+  const int pg_win = jwin / WBS;
+  auto next_page = [&](int pg) { return (pg == pg_keep && pg_win > pg) ? pg_win : pg + 1; };
+  s16x8 phi, plo;
+  auto weigh = [&](const short* P) {                         // O += V^T P^T
+#pragma unroll
+    for (int m = 0; m < DV; m += 4) {
+      s16x8 v[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const short* vp = P + vat[u] + (m >> 2) * 64;
+        const s16x4 a0 = rfq::ds_read_tr16(vp), a1 = rfq::ds_read_tr16(vp + 16 * E);
+        v[u] = (s16x8){a0[0], a0[1], a0[2], a0[3], a1[0], a1[1], a1[2], a1[3]};
+      }
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+        o[m + u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(v[u]), as_bf16x8(phi), o[m + u], 0, 0, 0);
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+        o[m + u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(v[u]), as_bf16x8(plo), o[m + u], 0, 0, 0);
+    }
+  };
+  int pg = kf > 0 ? 0 : pg_win, buf = 0;
+  fetch(bt[pg], 0);
+  int ahead = bt[min(next_page(pg), pg_last)];                 // the next page's number, read a page early
+  while (pg <= pg_last) {
+    const int jb = pg * WBS, pn = next_page(pg), nbuf = buf == 2 ? 0 : buf + 1;
+    landed(jb, buf);
+    if (pn <= pg_last) fetch(ahead, nbuf);
+    ahead = bt[min(next_page(pn), pg_last)];
+    const short* P = pages + buf * WBS * E;
+    f32x4 sc[2][2];                                          // two chains per half page
+#pragma unroll
+    for (int kt = 0; kt < 2; ++kt) {
+      sc[kt][0] = sc[kt][1] = (f32x4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int ks = 0; ks < DK; ++ks) {
+        const s16x8 k = *reinterpret_cast<const s16x8*>(P + kat[ks & 1] + kt * 16 * E + (ks >> 1) * 64);
+        f32x4& acc = sc[kt][ks & 1];
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(k), as_bf16x8(qhi[ks]), acc, 0, 0, 0);
+        if constexpr (QLO) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(k), as_bf16x8(qlo[ks]), acc, 0, 0, 0);
+      }
+    }
+    float p[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      float x = sc[i >> 2][0][i & 3] + sc[i >> 2][1][i & 3];
+      if constexpr (MODE == 1) x = cap2 - 2.f * cap2 * __builtin_amdgcn_rcpf(__builtin_amdgcn_exp2f(x) + 1.f);
+      if constexpr (MODE == 2) x = __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(x - hb));
+      p[i] = x;
+    }
+    if (!(jb + WBS - 1 <= p0 && (window <= 0 || plast - jb < window || jb + WBS <= keep_first))) {
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {                          // an edge inside the page
+        const int j = jb + (i >> 2) * 16 + grp * 4 + (i & 3);
+        const bool ok = j <= pi && (window <= 0 || pi - j < window || j < keep_first);
+        p[i] = ok ? p[i] : MODE == 2 ? 0.f : kNegInfW;
+      }
+    }
+    if constexpr (MODE != 2) {
+      float mx = fmaxf(fmaxf(fmaxf(p[0], p[1]), fmaxf(p[2], p[3])), fmaxf(fmaxf(p[4], p[5]), fmaxf(p[6], p[7])));
+      mx = other_half_max(other_row_max(mx));
+      const bool moves = mx > mrun + kDeferW;                // also for the first keys: mrun = -inf
+      if (__builtin_amdgcn_ballot_w64(moves) != 0ull) {
+        const float mn = moves ? mx : mrun;
+        const float alpha = moves ? __builtin_amdgcn_exp2f(mrun - mn) : 1.f;
+        mrun = mn;
+        lrun *= alpha;
+#pragma unroll
+        for (int m = 0; m < DV; ++m) o[m] *= alpha;
+      }
+      const float mu = mrun == kNegInfW ? 0.f : mrun;        // no visible key so far: every weight 0
+      float l0 = 0.f, l1 = 0.f;
+#pragma unroll
+      for (int i = 0; i < 8; i += 2) {
+        p[i] = __builtin_amdgcn_exp2f(p[i] - mu);
+        p[i + 1] = __builtin_amdgcn_exp2f(p[i + 1] - mu);
+        l0 += p[i];
+        l1 += p[i + 1];
+      }
+      lrun += l0 + l1;
+    }
+    split_bf16w(p, phi, plo);
+    weigh(P);
+    pg = pn;
+    buf = nbuf;
+  }
+  store_rows<DV, MODE>(a, o, lrun, t, hh, grp, qlive);
+}
+
+// ------------------------------------------------------------------ launcher
+namespace {
+bool plain_sizes(int DK, int DV) { return DK >= 1 && DK <= 4 && (DV == 2 || DV == 4 || DV == 8); }
+bool shared_sizes(int DK, int DV) {
+  return (DK == 3 && DV == 4) || (DK == 4 && (DV == 4 || DV == 6)) || (DK == 5 && DV == 8) ||
+         (DK == 6 && DV == 8) || (DK == 10 && DV == 16) || (DK == 18 && DV == 32);
+}
+}  // namespace
+
+bool keep_mfma_ok(int E, int vdim, int BS, bool shared) {
+  if (BS != WBS || E % 32 != 0 || vdim % 16 != 0) return false;
+  return shared ? shared_sizes(E / 32, vdim / 16) : plain_sizes(E / 32, vdim / 16);
+}
+
+template <int DK, int DV, int HPW, bool SHARED, int MODE>
+static void launch_keep_mfma_one(const KeepArgs& a) {
+  constexpr bool WIDE = SHARED && DK >= 10;
+  constexpr size_t lds = (size_t)(WIDE ? 3 * WBS * 32 * DK : 2 * keep_page_shorts<DK, DV, SHARED>()) * sizeof(short);
+  static_assert(lds <= 160 * 1024, "LDS of a CU");
+  static bool attr = false;
+  auto run = [&](auto kernel, int threads) {
+    if (!attr) {
+      (void)hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                160 * 1024);
+      attr = true;
+    }
+    hipLaunchKernelGGL(kernel, dim3(a.W, a.H / HPW), dim3(threads), lds, a.s, a);
+  };
+  if constexpr (WIDE) run(&attn_keep_wide_kernel<DK, DV, HPW, MODE>, 128 * HPW);
+  else run(&attn_keep_mfma_kernel<DK, DV, HPW, SHARED, MODE>, 128 * HPW);
+}
+
+template <int DK, int DV, int HPW, bool SHARED>
+static void launch_keep_mfma_mode(const KeepArgs& a) {
+  if (a.sigmoid) launch_keep_mfma_one<DK, DV, HPW, SHARED, 2>(a);
+  else if (a.softcap > 0.f) launch_keep_mfma_one<DK, DV, HPW, SHARED, 1>(a);
+  else launch_keep_mfma_one<DK, DV, HPW, SHARED, 0>(a);
 }
 
 template <int DK, int DV, bool SHARED>
 static void launch_keep_mfma_heads(const KeepArgs& a) {
-  if ((a.H / a.G) % 2 == 0) launch_keep_mfma_one<DK, DV, 2, SHARED>(a);
-  else launch_keep_mfma_one<DK, DV, 1, SHARED>(a);
+  const int rep = a.H / a.G;
+  if (rep % 4 == 0) launch_keep_mfma_mode<DK, DV, 4, SHARED>(a);
+  else if (rep % 2 == 0) launch_keep_mfma_mode<DK, DV, 2, SHARED>(a);
+  else launch_keep_mfma_mode<DK, DV, 1, SHARED>(a);
 }
 
 bool launch_attn_keep_mfma(const float* q, const void* k_cache, const void* v_cache, int64_t vrs,

@@ -1,5 +1,6 @@
-"""Decode rows of attn_keep_window with the pages split over waves (csrc/kernels/mix_keep_split.hip):
-contexts around pages and waves, head groups around the sixteen columns, every option."""
+"""attn_keep_window on MFMA tiles: decode rows with the pages split over waves
+(csrc/kernels/mix_keep_split.hip) and prompt rows (mix_keep_attn_mfma.hip).  Contexts around pages and
+waves, head groups around columns and workgroups, every option."""
 import pytest
 import torch
 
@@ -13,7 +14,7 @@ DEV, BS = "cuda", 32
 SEQS = [(1, 1), (31, 1), (32, 1), (33, 1), (129, 1), (257, 1), (300, 5), (40, 0), (700, 1), (70, 33)]
 
 
-def _check(H, G, E, vd, shared, seqs=SEQS, spoil=None, **opt):
+def _check(H, G, E, vd, shared, seqs=SEQS, spoil=None, prompt=False, **opt):
     g = torch.Generator().manual_seed(H + E + vd)
     need = [(n + BS - 1) // BS for n, _ in seqs]
     perm = torch.randperm(sum(need), generator=g).tolist()
@@ -47,9 +48,10 @@ def _check(H, G, E, vd, shared, seqs=SEQS, spoil=None, **opt):
     got = torch.full_like(out, 7.0).to(DEV)
     kd = k.to(DEV)
     m = lambda x: None if x is None else x.to(DEV)  # noqa: E731
-    zero = torch.zeros(len(seqs), dtype=torch.int32, device=DEV)
-    ops.attn_keep_window(q.to(DEV), kd, kd if shared else v.to(DEV), *args(DEV), zero, zero, m(bias), m(gate), got,
-                         E ** -0.5, short_rows=max(r for _, r in seqs), **opt)
+    items = [(i, b) for i, (_, r) in enumerate(seqs) for b in range((r + 31) // 32)] + [(-1, 0)]   # -1: padding
+    ws, wq = (i32([x[j] for x in items]).to(DEV) for j in (0, 1))
+    ops.attn_keep_window(q.to(DEV), kd, kd if shared else v.to(DEV), *args(DEV), ws, wq, m(bias), m(gate), got,
+                         E ** -0.5, short_rows=0 if prompt else max(r for _, r in seqs), **opt)
     # both sides round to bf16, whose neighbouring values are up to 2^-7 of the value apart: where the
     # fp32 results lie on two sides of a tie they end one spacing apart.  Queries of keys wider than
     # 320 entries enter the products as bf16: four times that.
@@ -90,3 +92,41 @@ def test_a_key_outside_the_window_may_hold_infinities():
     seqs = [(200, 1), (333, 1), (129, 1)]
     _check(32, 8, 128, 128, False, seqs=seqs, spoil=20, window=64, keep_first=4)
     _check(16, 1, 576, 512, True, seqs=seqs, spoil=20, window=64, keep_first=4)
+
+
+PROMPTS = [(1, 1), (31, 31), (32, 32), (33, 33), (100, 70), (300, 45), (40, 0), (161, 97)]
+
+
+@pytest.mark.parametrize("H,G,E,vd,shared", [(4, 4, 128, 128, False), (6, 3, 64, 32, False), (8, 2, 96, 128, False),
+                                             (3, 1, 32, 64, False), (8, 1, 96, 64, True), (6, 1, 128, 96, True),
+                                             (5, 1, 160, 128, True), (4, 1, 192, 128, True), (8, 1, 320, 256, True),
+                                             (6, 1, 576, 512, True), (3, 1, 576, 512, True), (16, 1, 576, 512, True)])
+def test_prompt_rows(H, G, E, vd, shared):
+    _check(H, G, E, vd, shared, seqs=PROMPTS, prompt=True, bias=True, gate="head")
+    _check(H, G, E, vd, shared, seqs=PROMPTS, prompt=True, softcap=20.0, out_mult=0.6, gate="output")
+    _check(H, G, E, vd, shared, seqs=PROMPTS, prompt=True, window=37, keep_first=5, sigmoid=True, bias=True)
+    _check(H, G, E, vd, shared, seqs=PROMPTS, prompt=True, window=64, keep_first=40)
+
+
+def test_prompt_rows_with_rising_scores():
+    """Every page moves the maximum by far: the accumulators are rescaled each time."""
+    for shared, E, vd in ((False, 128, 128), (True, 576, 512)):
+        g = torch.Generator().manual_seed(1)
+        n, nb = 160, 6
+        k = torch.randn(nb, 1, BS, E, generator=g)
+        k *= (torch.arange(nb * BS).view(nb, 1, BS, 1) // BS + 1)
+        k = k.bfloat16()
+        v = k if shared else torch.randn(nb, 1, BS, vd, generator=g).bfloat16()
+        q = torch.randn(n, 4, E, generator=g) * 3
+        i32 = lambda x: torch.tensor(x, dtype=torch.int32)  # noqa: E731
+        meta = (vd, i32([[0, 1, 2, 3, 4]]), i32([0]), i32([n]), i32([n]))
+        out = torch.zeros(n, 4 * vd, dtype=torch.bfloat16)
+        qb = q.bfloat16().float() if shared else q      # wide queries enter the products as bf16
+        ref.attn_keep_window(qb, k, v, *meta, None, None, out, 0.5, 0, 0, False)
+        got = torch.empty_like(out).to(DEV)
+        kd = k.to(DEV)
+        ops.attn_keep_window(qb.to(DEV), kd, kd if shared else v.to(DEV), vd, *(x.to(DEV) for x in meta[1:]),
+                             i32([0] * 5).to(DEV), i32(list(range(5))).to(DEV), None, None, got, 0.5)
+        err = (got.cpu().float() - out.float()).abs()
+        # scores of some hundreds, their bf16 hi + lo products to 2^-16: weights to about 1 %
+        assert float(err.mean()) <= 0.02 * float(out.float().abs().mean())
