@@ -105,7 +105,6 @@ __device__ __forceinline__ float arrived(bf16_t bits) {
   asm volatile("v_lshlrev_b32 %0, 16, %1" : "=v"(f) : "v"(bits));
   return f;
 }
-__device__ __forceinline__ float4 ld4(const float* p) { return *reinterpret_cast<const float4*>(p); }
 }  // namespace
 
 namespace {

@@ -33,6 +33,35 @@ __device__ __forceinline__ float wave_max(float v) {
   return v;
 }
 
+// Sum over each aligned group of L neighbouring lanes (L = 4, 8, .. 64, the same for the whole wave);
+// every lane of the group receives it.  The first four steps stay inside a row of 16 lanes.
+__device__ __forceinline__ float group_sum(float v, int L) {
+  v += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0xB1, 0xf, 0xf, true));              // lanes 1 0 3 2
+  v += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x4E, 0xf, 0xf, true));              // lanes 2 3 0 1
+  if (L > 4) v += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x141, 0xf, 0xf, true));  // half rows mirrored
+  if (L > 8) v += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x140, 0xf, 0xf, true));  // rows mirrored
+  if (L > 16) v += __shfl_xor(v, 16, 64);
+  if (L > 32) v += __shfl_xor(v, 32, 64);
+  return v;
+}
+
+// four neighbouring entries, 16- or 8-byte aligned
+__device__ __forceinline__ float4 ld4(const float* p) { return *reinterpret_cast<const float4*>(p); }
+__device__ __forceinline__ float4 ld4(const bf16_t* p) {
+  const uint2 w = *reinterpret_cast<const uint2*>(p);
+  return make_float4(__uint_as_float(w.x << 16), __uint_as_float(w.x & 0xffff0000u),
+                     __uint_as_float(w.y << 16), __uint_as_float(w.y & 0xffff0000u));
+}
+__device__ __forceinline__ void st4(float* p, float4 v) { *reinterpret_cast<float4*>(p) = v; }
+__device__ __forceinline__ void st4(bf16_t* p, float4 v) {
+  union { bf16_t h[4]; uint2 w; } u;
+  stf(u.h, v.x);
+  stf(u.h + 1, v.y);
+  stf(u.h + 2, v.z);
+  stf(u.h + 3, v.w);
+  *reinterpret_cast<uint2*>(p) = u.w;
+}
+
 // Block-wide sum for blockDim.x a multiple of 64, at most 1024.  scratch >= 16 floats.
 __device__ __forceinline__ float block_sum(float v, float* scratch) {
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;

@@ -29,19 +29,6 @@ __global__ __launch_bounds__(256) void embed_sinusoid_kernel(
   }
 }
 
-__device__ __forceinline__ float4 ld4(const float* p) { return *reinterpret_cast<const float4*>(p); }
-__device__ __forceinline__ float4 ld4(const bf16_t* p) {
-  const uint2 v = *reinterpret_cast<const uint2*>(p);
-  return make_float4(__uint_as_float(v.x << 16), __uint_as_float(v.x & 0xffff0000u),
-                     __uint_as_float(v.y << 16), __uint_as_float(v.y & 0xffff0000u));
-}
-__device__ __forceinline__ void st4(float* p, float4 v) { *reinterpret_cast<float4*>(p) = v; }
-__device__ __forceinline__ void st4(bf16_t* p, float4 v) {
-  bf16_t t[4];
-  stf(t, v.x); stf(t + 1, v.y); stf(t + 2, v.z); stf(t + 3, v.w);
-  *reinterpret_cast<uint2*>(p) = *reinterpret_cast<const uint2*>(t);
-}
-
 __device__ __forceinline__ void ld8(const float* p, float* f) {
   const float4 a = ld4(p), b = ld4(p + 4);
   f[0] = a.x; f[1] = a.y; f[2] = a.z; f[3] = a.w; f[4] = b.x; f[5] = b.y; f[6] = b.z; f[7] = b.w;
