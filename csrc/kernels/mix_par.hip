@@ -256,13 +256,6 @@ __global__ __launch_bounds__(256) void conv_act_heads_kernel(
 // Four channels per thread (2 to 4 taps; C, dim, the row stride and the chunk multiples of 4,
 // 16-byte aligned rows): one 8- or 16-byte load per tap row, the four channels' taps as 4 * taps
 // contiguous floats, 16-byte state accesses and stores.
-__device__ __forceinline__ float4 ld4any(const float* p) { return *reinterpret_cast<const float4*>(p); }
-__device__ __forceinline__ float4 ld4any(const bf16_t* p) {
-  const uint2 w = *reinterpret_cast<const uint2*>(p);
-  return make_float4(__uint_as_float(w.x << 16), __uint_as_float(w.x & 0xffff0000u),
-                     __uint_as_float(w.y << 16), __uint_as_float(w.y & 0xffff0000u));
-}
-
 template <typename T, int TAPS>
 __global__ __launch_bounds__(256) void conv_act_heads_vec_kernel(
     const T* __restrict__ x, int64_t x_stride, const float* __restrict__ w,
@@ -283,18 +276,18 @@ __global__ __launch_bounds__(256) void conv_act_heads_vec_kernel(
   const int n = i + f + 1;
   for (int cc = threadIdx.x * 4; cc < nc; cc += blockDim.x * 4) {
     const int c = c0 + cc;
-    const float4 x0 = ld4any(xr + c);
+    const float4 x0 = ld4(xr + c);
     float wc[4 * TAPS];                                  // [4][taps], read in 16-byte pieces
 #pragma unroll
     for (int k = 0; k < TAPS; ++k)
-      *reinterpret_cast<float4*>(wc + 4 * k) = ld4any(w + (int64_t)c * taps + 4 * k);
+      *reinterpret_cast<float4*>(wc + 4 * k) = ld4(w + (int64_t)c * taps + 4 * k);
     float a0 = wc[taps - 1] * x0.x, a1 = wc[2 * taps - 1] * x0.y;
     float a2 = wc[3 * taps - 1] * x0.z, a3 = wc[4 * taps - 1] * x0.w;
 #pragma unroll
     for (int dl = 1; dl < taps; ++dl) {
       float4 src;
-      if (dl <= i) src = ld4any(xr - (int64_t)dl * x_stride + c);
-      else if (p - dl >= 0 && rd != nullptr) src = ld4any(rd + (int64_t)(K + i - dl) * C + c);
+      if (dl <= i) src = ld4(xr - (int64_t)dl * x_stride + c);
+      else if (p - dl >= 0 && rd != nullptr) src = ld4(rd + (int64_t)(K + i - dl) * C + c);
       else continue;
       const int k = taps - 1 - dl;
       a0 += wc[k] * src.x;
@@ -309,7 +302,7 @@ __global__ __launch_bounds__(256) void conv_act_heads_vec_kernel(
       if (f < K) *reinterpret_cast<float4*>(wr + (int64_t)(K - 1 - f) * C + c) = x0;
       if (i == 0)
         for (int e = 0; e < K - n; ++e)
-          *reinterpret_cast<float4*>(wr + (int64_t)e * C + c) = ld4any(rd + (int64_t)(e + n) * C + c);
+          *reinterpret_cast<float4*>(wr + (int64_t)e * C + c) = ld4(rd + (int64_t)(e + n) * C + c);
     }
   }
   float* o = out + (int64_t)t * C + c0;
@@ -333,6 +326,72 @@ __global__ __launch_bounds__(256) void conv_act_heads_vec_kernel(
     for (int e = lane; e < dim; e += 64) o[hd * dim + e] = ys[hd * dim + e] * r;
   }
   for (int cc = unit_here * dim + threadIdx.x; cc < nc; cc += blockDim.x) o[cc] = ys[cc];
+}
+
+// The same for heads of 16, 32, 64, 128 or 256 channels: a wave has 256 channels, four a lane, so a head
+// is a group of dim / 4 lanes and its sum needs no LDS; a thread takes R rows below one another, whose
+// earlier inputs and taps stay in registers.  (Positions rise by one inside a run, so what precedes a
+// row is what preceded the row above, shifted.)  Bound by memory and the fp32 divides: 4,096 rows of 8,192
+// channels, 4 taps, from bf16 took 97 us with a row a block, its taps read again for each and the heads'
+// sums through LDS; 49 us here (4.1 TB/s).
+template <typename T, int TAPS, int R>
+__global__ __launch_bounds__(256) void conv_act_heads_rows_kernel(
+    const T* __restrict__ x, int64_t x_stride, const float* __restrict__ w,
+    float* __restrict__ state, const int32_t* __restrict__ row_state,
+    const int32_t* __restrict__ row_back, const int32_t* __restrict__ row_fwd,
+    const int32_t* __restrict__ pos, float* __restrict__ out, int Trows, int C, int slots,
+    int n_unit, int dim, float unit_eps) {
+  constexpr int K = TAPS - 1;
+  const int t0 = blockIdx.x * R, c = (blockIdx.y * 256 + threadIdx.x) * 4;
+  if (c >= C) return;                                    // whole heads: C is a multiple of dim
+  const bool unit = c < n_unit * dim;
+  float wc[4 * TAPS];                                    // [4][taps], read in 16-byte pieces
+#pragma unroll
+  for (int k = 0; k < TAPS; ++k) *reinterpret_cast<float4*>(wc + 4 * k) = ld4(w + (int64_t)c * TAPS + 4 * k);
+  float4 xs[R], h[K];                                    // h[dl - 1]: the input dl rows above
+#pragma unroll
+  for (int r = 0; r < R; ++r) xs[r] = ld4(x + (int64_t)min(t0 + r, Trows - 1) * x_stride + c);
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    const int t = t0 + r;
+    if (t >= Trows) break;
+    const int code = row_state[t], i = row_back[t], f = row_fwd[t];
+    const float* rd = code >= 0 ? state + ((int64_t)((code & 1) * slots + (code >> 1)) * K) * C + c : nullptr;
+    float* wr = code >= 0 ? state + ((int64_t)((1 - (code & 1)) * slots + (code >> 1)) * K) * C + c : nullptr;
+    if (r == 0 || i == 0) {
+      const int p = pos[t];
+#pragma unroll
+      for (int dl = 1; dl <= K; ++dl) {
+        h[dl - 1] = make_float4(0.f, 0.f, 0.f, 0.f);
+        if (dl <= i) h[dl - 1] = ld4(x + (int64_t)(t - dl) * x_stride + c);
+        else if (p - dl >= 0 && rd != nullptr) h[dl - 1] = ld4(rd + (int64_t)(K + i - dl) * C);
+      }
+    }
+    const float4 x0 = xs[r];
+    float a0 = wc[K] * x0.x, a1 = wc[TAPS + K] * x0.y, a2 = wc[2 * TAPS + K] * x0.z, a3 = wc[3 * TAPS + K] * x0.w;
+#pragma unroll
+    for (int dl = 1; dl <= K; ++dl) {
+      a0 += wc[K - dl] * h[dl - 1].x;
+      a1 += wc[TAPS + K - dl] * h[dl - 1].y;
+      a2 += wc[2 * TAPS + K - dl] * h[dl - 1].z;
+      a3 += wc[3 * TAPS + K - dl] * h[dl - 1].w;
+    }
+    float4 y = make_float4(a0 / (1.0f + expf(-a0)), a1 / (1.0f + expf(-a1)), a2 / (1.0f + expf(-a2)),
+                           a3 / (1.0f + expf(-a3)));
+    if (n_unit > 0) {
+      const float m = 1.0f / sqrtf(group_sum(y.x * y.x + y.y * y.y + y.z * y.z + y.w * y.w, dim >> 2) + unit_eps);
+      if (unit) y = make_float4(y.x * m, y.y * m, y.z * m, y.w * m);
+    }
+    st4(out + (int64_t)t * C + c, y);
+    if (wr != nullptr) {
+      if (f < K) st4(wr + (int64_t)(K - 1 - f) * C, x0);
+      if (i == 0)
+        for (int e = 0; e < K - (f + 1); ++e) st4(wr + (int64_t)e * C, ld4(rd + (int64_t)(e + f + 1) * C));
+    }
+#pragma unroll
+    for (int dl = K; dl > 1; --dl) h[dl - 1] = h[dl - 2];
+    h[0] = x0;
+  }
 }
 
 // One thread per row: the `top` largest of z + bias (ties to the lower index), weights =
@@ -450,13 +509,30 @@ void launch_conv_act_heads(bool f32, const void* x, int64_t stride, const float*
   hipLaunchKernelGGL(KERNEL<TT>, grid, dim3(256), lds, s, (const TT*)x, stride, w, state,      \
                      row_state, row_back, row_fwd, pos, out, C, taps, slots, n_unit, dim,       \
                      unit_eps, chunk)
+  // heads that are a group of a wave's lanes; eight rows together once that still leaves 1,024 workgroups
+  const bool group = vec && C % dim == 0 && (dim == 16 || dim == 32 || dim == 64 || dim == 128 || dim == 256);
+  const int cols = (C + 1023) / 1024;
+  const bool rows8 = (int64_t)T_ * cols >= 8192;
+#define CONV_ROWS1(TT, TAPS, R)                                                                 \
+  hipLaunchKernelGGL((conv_act_heads_rows_kernel<TT, TAPS, R>), dim3((T_ + R - 1) / R, cols),    \
+                     dim3(256), 0, s, (const TT*)x, stride, w, state, row_state, row_back,       \
+                     row_fwd, pos, out, T_, C, slots, n_unit, dim, unit_eps)
+#define CONV_ROWS(TT)                                                                           \
+  do {                                                                                          \
+    if (taps == 2) { if (rows8) CONV_ROWS1(TT, 2, 8); else CONV_ROWS1(TT, 2, 1); }               \
+    else if (taps == 3) { if (rows8) CONV_ROWS1(TT, 3, 8); else CONV_ROWS1(TT, 3, 1); }          \
+    else { if (rows8) CONV_ROWS1(TT, 4, 8); else CONV_ROWS1(TT, 4, 1); }                         \
+  } while (0)
 #define CONV_VEC(TT)                                                                            \
   do {                                                                                          \
     if (taps == 2) hipLaunchKernelGGL((conv_act_heads_vec_kernel<TT, 2>), grid, dim3(256), lds, s, (const TT*)x, stride, w, state, row_state, row_back, row_fwd, pos, out, C, taps, slots, n_unit, dim, unit_eps, chunk); \
     else if (taps == 3) hipLaunchKernelGGL((conv_act_heads_vec_kernel<TT, 3>), grid, dim3(256), lds, s, (const TT*)x, stride, w, state, row_state, row_back, row_fwd, pos, out, C, taps, slots, n_unit, dim, unit_eps, chunk); \
     else hipLaunchKernelGGL((conv_act_heads_vec_kernel<TT, 4>), grid, dim3(256), lds, s, (const TT*)x, stride, w, state, row_state, row_back, row_fwd, pos, out, C, taps, slots, n_unit, dim, unit_eps, chunk); \
   } while (0)
-  if (vec) {
+  if (group) {
+    if (f32) CONV_ROWS(float);
+    else CONV_ROWS(bf16_t);
+  } else if (vec) {
     if (f32) CONV_VEC(float);
     else CONV_VEC(bf16_t);
   } else {
@@ -464,6 +540,8 @@ void launch_conv_act_heads(bool f32, const void* x, int64_t stride, const float*
     else CONV_GO(conv_act_heads_kernel, bf16_t);
   }
 #undef CONV_GO
+#undef CONV_ROWS1
+#undef CONV_ROWS
 #undef CONV_VEC
 }
 

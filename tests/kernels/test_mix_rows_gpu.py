@@ -1,4 +1,6 @@
-"""Row kernels that take several channels a lane and several rows a thread (csrc/kernels/mix_wkv.hip) against the row-by-row reference: runs that begin and end inside a thread's rows, the last rows and columns of a grid."""
+"""Row kernels that take several channels a lane and several rows a thread (csrc/kernels/mix_par.hip,
+mix_wkv.hip) against the row-by-row reference: runs that begin and end inside a thread's rows, runs
+shorter than the taps, head sizes, the last rows and columns of a grid."""
 import pytest
 import torch
 
@@ -23,6 +25,29 @@ def _rows(lens, start=23):
 def _lens(total):
     lens = [1, 2, 3, 8, 1, 9, 15, 1, 1, 4]
     return lens + [total - sum(lens)]
+
+
+# 8,192 (rows x columns of 1,024 channels) and more are taken eight rows together, fewer singly
+@pytest.mark.parametrize("together", [False, True])
+@pytest.mark.parametrize("taps,dim,heads,n_unit", [(2, 16, 3, 2), (3, 32, 40, 40), (4, 64, 64, 32), (4, 128, 32, 16),
+                                                   (2, 256, 16, 3), (4, 128, 3, 0)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_convolution_by_groups_of_lanes(dtype, taps, dim, heads, n_unit, together):
+    g = torch.Generator().manual_seed(dim + taps)
+    T = 8192 // -(-heads * dim // 1024) + 3 if together else 50
+    C, lens = heads * dim, _lens(T)
+    wide = torch.randn(T, C + 8, generator=g).to(dtype)
+    w = torch.randn(C, taps, generator=g)
+    state = torch.randn(2 * len(lens), taps - 1, C, generator=g)
+    rows = _rows(lens)
+    got_s, want_s = state.to(DEV), state.clone()
+    got, want = torch.empty(T, C, device=DEV), torch.empty(T, C)
+    ops.conv_act_heads(wide.to(DEV)[:, 8:], w.to(DEV), got_s, *(r.to(DEV) for r in rows), n_unit, dim, 1e-6, got)
+    ref.conv_act_heads(wide[:, 8:], w, want_s, *rows, n_unit, dim, 1e-6, want)
+    # up to four products of at most 25 and their sum to 2^-24 each: 100 * 5 * 2^-24 = 3e-5; a unit
+    # vector's sum of 256 squares adds less
+    torch.testing.assert_close(got.cpu(), want, atol=3e-5, rtol=1e-5)
+    assert torch.equal(got_s.cpu(), want_s)
 
 
 @pytest.mark.parametrize("T,d", [(47, 4), (50, 2052), (1371, 2052), (4099, 64)])     # the last two: four rows a thread
