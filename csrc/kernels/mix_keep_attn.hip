@@ -23,6 +23,8 @@
 // sums in fp32): work items (sequence, block of QB queries) x head for prompt portions, one
 // workgroup per (sequence, key/value head) over one pass through the pages for decode rows.
 // MFMA tiles for bf16 pages are in mix_keep_attn_mfma.hip.
+#include <algorithm>
+
 #include "mix_common.h"
 
 namespace rfqmix {
@@ -89,6 +91,32 @@ __device__ __forceinline__ void st_chunk(bf16_t* p, const float* f) {
     stf(p, f[0]);
   }
 }
+// A chunk as loaded, for operands that several loads bring in together: converted at its use.
+template <int CW>
+struct Bits {
+  uint32_t u[CW];
+  __device__ __forceinline__ void load(const float* p) {
+    if constexpr (CW == 8) {
+      *reinterpret_cast<uint4*>(u) = *reinterpret_cast<const uint4*>(p);
+      *reinterpret_cast<uint4*>(u + 4) = *reinterpret_cast<const uint4*>(p + 4);
+    } else {
+      u[0] = __float_as_uint(*p);
+    }
+  }
+  __device__ __forceinline__ void load(const bf16_t* p) {
+    if constexpr (CW == 8) *reinterpret_cast<uint4*>(u) = *reinterpret_cast<const uint4*>(p);
+    else u[0] = *p;
+  }
+  template <typename T>
+  __device__ __forceinline__ void get(float* f) const {
+#pragma unroll
+    for (int i = 0; i < CW; ++i) {
+      if constexpr (sizeof(T) == 4) f[i] = __uint_as_float(u[i]);
+      else if constexpr (CW == 8) f[i] = __uint_as_float(i & 1 ? u[i >> 1] & 0xffff0000u : u[i >> 1] << 16);
+      else f[i] = __uint_as_float(u[0] << 16);
+    }
+  }
+};
 }  // namespace
 
 // One workgroup per row; the row passes through LDS as floats.  CW = 8: every width, stride and
@@ -98,9 +126,9 @@ __device__ __forceinline__ void st_chunk(bf16_t* p, const float* f) {
 // rows go to the other half).
 // q_from > 0 (no convolution): a head of q holds q_from + qw entries in proj, of which only the
 // last qw are read; everything below sees heads of qw entries.
-// LDS (floats): row[W] | fac[H + G] | cs[2 nrot] | scratch[16]
+// LDS (floats): row[W] | fac[H + G] | cs[2 nrot] | scratch[2 per wave]
 template <typename T, int CW>
-__global__ __launch_bounds__(256) void qk_norm_rotary_append_kernel(
+__global__ __launch_bounds__(1024) void qk_norm_rotary_append_kernel(
     const T* __restrict__ proj, int64_t stride, const float* __restrict__ bias,
     const float* __restrict__ q_norm_w, const float* __restrict__ k_norm_w, int norm_all,
     int k_norm_n, float eps, const int32_t* __restrict__ pos, const float* __restrict__ inv_freq,
@@ -145,6 +173,21 @@ __global__ __launch_bounds__(256) void qk_norm_rotary_append_kernel(
     else ld_chunk<CW>(src_k + c, f);
     if (conv_w != nullptr) {
       float u[CW], w[CW];
+      // up to three rows above and their weights on the way together, later ones one by one
+      constexpr int NR = 3;
+      Bits<CW> raw[NR];
+      float wr4[NR][CW];
+      int have = 0;                    // rows above that exist
+#pragma unroll
+      for (int dl = 1; dl <= NR; ++dl) {
+        if (dl > K) break;
+        if (dl <= back) raw[dl - 1].load(src - (int64_t)dl * stride + c);
+        else if (pt - dl >= 0 && rd != nullptr) raw[dl - 1].load(rd + (int64_t)(K + back - dl) * W + c);
+        else break;
+        ld_chunk<CW>(conv_w + (int64_t)(K - dl) * W + c, wr4[dl - 1]);
+        have = dl;
+      }
+      ld_chunk<CW>(conv_w + (int64_t)K * W + c, w);
       if (wr != nullptr) {
         if (fwd < K) st_chunk<CW>(wr + (int64_t)(K - 1 - fwd) * W + c, f);
         if (back == 0)                 // a run shorter than the taps: older inputs move up
@@ -153,10 +196,17 @@ __global__ __launch_bounds__(256) void qk_norm_rotary_append_kernel(
             st_chunk<CW>(wr + (int64_t)e * W + c, u);
           }
       }
-      ld_chunk<CW>(conv_w + (int64_t)K * W + c, w);
 #pragma unroll
       for (int i = 0; i < CW; ++i) f[i] *= w[i];
-      for (int dl = 1; dl <= K; ++dl) {
+#pragma unroll
+      for (int dl = 1; dl <= NR; ++dl) {
+        if (dl > have) break;
+        if (dl <= back) raw[dl - 1].template get<T>(u);
+        else raw[dl - 1].template get<float>(u);
+#pragma unroll
+        for (int i = 0; i < CW; ++i) f[i] += wr4[dl - 1][i] * u[i];
+      }
+      for (int dl = NR + 1; dl <= K; ++dl) {
         if (dl <= back) ld_chunk<CW>(src - (int64_t)dl * stride + c, u);
         else if (pt - dl >= 0 && rd != nullptr) ld_chunk<CW>(rd + (int64_t)(K + back - dl) * W + c, u);
         else break;
@@ -181,30 +231,29 @@ __global__ __launch_bounds__(256) void qk_norm_rotary_append_kernel(
     }
   }
   const float p = (float)pos[t];
-  for (int i = tid; i < nrot; i += nthr) {
+  for (int i = nthr - 1 - tid; i < nrot; i += nthr) {    // the last wave as a rule has no chunk of the row
     float sn, c;
     sincosf(p * inv_freq[i], &sn, &c);
     cs[2 * i] = c * rot_mult;
     cs[2 * i + 1] = sn * rot_mult;
   }
-  // norm factors: fac[0], fac[1] (whole projections) or one per head
+  // norm factors: fq, fk (whole projections) or one per head
+  float fq = 1.f, fk = 1.f;
   if (norm_all) {
     sq = wave_sum(sq);
     sk = wave_sum(sk);
     if (lane == 0) {
       scratch[wid] = sq;
-      scratch[8 + wid] = sk;
+      scratch[nw + wid] = sk;
     }
     __syncthreads();
-    if (tid == 0) {
-      float a = 0.f, b = 0.f;
-      for (int w = 0; w < nw; ++w) {
-        a += scratch[w];
-        b += scratch[8 + w];
-      }
-      fac[0] = q_norm_w != nullptr ? 1.0f / sqrtf(a / (float)nq + eps) : 1.f;
-      fac[1] = k_norm_w != nullptr && nk > 0 ? 1.0f / sqrtf(b / (float)nk + eps) : 1.f;
+    float a = 0.f, b = 0.f;
+    for (int w = 0; w < nw; ++w) {
+      a += scratch[w];
+      b += scratch[nw + w];
     }
+    fq = q_norm_w != nullptr ? 1.0f / sqrtf(a / (float)nq + eps) : 1.f;
+    fk = k_norm_w != nullptr && nk > 0 ? 1.0f / sqrtf(b / (float)nk + eps) : 1.f;
   } else {
     __syncthreads();
     // sixteen lanes per head: sixteen heads of the row are summed at a time
@@ -221,8 +270,8 @@ __global__ __launch_bounds__(256) void qk_norm_rotary_append_kernel(
       for (int o = 8; o > 0; o >>= 1) ss += __shfl_xor(ss, o, 64);
       if (sub == 0) fac[hd] = normed ? 1.0f / sqrtf(ss / (float)n + eps) : 1.f;
     }
+    __syncthreads();
   }
-  __syncthreads();
   const int32_t slot = slots[t];
   const bool keep = G > 0 && slot >= 0 && slot < pool_slots;
   const int64_t page_row = keep ? ((int64_t)(slot / BS) * G) * BS + slot % BS : 0;   // + g * BS
@@ -259,7 +308,7 @@ __global__ __launch_bounds__(256) void qk_norm_rotary_append_kernel(
     const int hd = y / width, e = y - hd * width;
     const float* wv = isq ? q_norm_w : k_norm_w;
     const int nn = wv == nullptr ? 0 : (norm_all || isq ? width : k_norm_n);   // normed entries of a head
-    const float fc = norm_all ? fac[isq ? 0 : 1] : fac[isq ? hd : H + hd];
+    const float fc = norm_all ? (isq ? fq : fk) : fac[isq ? hd : H + hd];
     const float* wp = wv == nullptr ? nullptr : (norm_all ? wv + (y - e) : wv);  // the head's weights
     const int r0 = e - (isq ? q_rot_off : k_rot_off);
     float v[CW];
@@ -717,8 +766,8 @@ bool launch_qk_norm_rotary_append(bool f32, const void* proj, int64_t stride, co
                                   const int32_t* row_state, const int32_t* row_back,
                                   const int32_t* row_fwd, hipStream_t s) {
   const size_t W = (size_t)H * qw + (size_t)G * kw + (v_mode == 0 ? (size_t)G * vdim : 0);
-  const size_t lds = (W + 4 + H + G + 4 + 2 * (size_t)nrot + 16) * sizeof(float);
-  if (lds > (size_t)kLdsMax) return false;
+  const size_t base = W + 4 + H + G + 4 + 2 * (size_t)nrot;
+  if ((base + 16) * sizeof(float) > (size_t)kLdsMax) return false;
   if (T == 0) return true;
   static bool attr = false;
   if (!attr) {
@@ -735,8 +784,16 @@ bool launch_qk_norm_rotary_append(bool f32, const void* proj, int64_t stride, co
                    al16(k_norm_w) && al16(k_cache) && al16(v_cache) && al16(q_out) && al16(v_in) &&
                    al16(v_out) && al16(conv_w) && al16(conv_state) && q_ts % 8 == 0 && q_hs % 8 == 0 &&
                    q_from % 8 == 0;
+  // Up to a row per CU its chain of loads is what counts: a chunk per thread, a wave for the sines
+  // beside them (32 + 8 + 8 heads of 128, convolved: one row 10.7 -> 8.2 us, 64 rows 14.2 -> 11.4).
+  // More rows share a CU and fill it from blocks of 256 (512 rows: a pass of 23.7 us against 24.8;
+  // 2,648 rows: 40 us against 73), as does a row that leaves no LDS for more waves' sums.
+  const size_t want = (W / (vec ? 8 : 1) + 63) / 64 * 64 + (nrot > 0 ? 64 : 0);
+  int threads = T <= 256 ? (int)std::min<size_t>(1024, std::max<size_t>(want, 256)) : 256;
+  if ((base + 2 * threads / 64) * sizeof(float) > (size_t)kLdsMax) threads = 256;
+  const size_t lds = (base + 2 * threads / 64) * sizeof(float);
 #define QKN_GO(TT, CW)                                                                          \
-  hipLaunchKernelGGL((qk_norm_rotary_append_kernel<TT, CW>), dim3(T), dim3(256), lds, s,       \
+  hipLaunchKernelGGL((qk_norm_rotary_append_kernel<TT, CW>), dim3(T), dim3(threads), lds, s,   \
                      (const TT*)proj, stride, bias, q_norm_w, k_norm_w, (int)norm_all, k_norm_n, \
                      eps, pos, inv_freq, nrot, rot_mult, q_rot_off, k_rot_off, slots,           \
                      (TT*)k_cache, (TT*)v_cache, H, G, qw, kw, vdim, v_mode, BS, pool_slots,    \

@@ -1,6 +1,6 @@
-"""Row kernels that take several channels a lane and several rows a thread (csrc/kernels/mix_par.hip,
-mix_wkv.hip) against the row-by-row reference: runs that begin and end inside a thread's rows, runs
-shorter than the taps, head sizes, the last rows and columns of a grid."""
+"""Row kernels that take several channels a lane or several rows a thread (csrc/kernels/mix_par.hip,
+mix_wkv.hip, mix_keep_attn.hip) against the row-by-row reference: runs that begin and end inside a
+thread's rows, runs shorter than the taps, head sizes, the last rows and columns of a grid."""
 import pytest
 import torch
 
@@ -64,3 +64,32 @@ def test_token_shift_four_channels_a_lane(dtype, T, d):
     # a + (b - a) mu with terms up to 50, two roundings of 2^-24; bf16: the neighbouring value
     torch.testing.assert_close(got.cpu(), want, atol=1e-5, rtol=2.0 ** -7 if dtype == torch.bfloat16 else 1e-6)
     assert torch.equal(got_p.cpu(), want_p)
+
+
+# 256 rows: a thread per chunk of a row and a wave for the sines; 257: blocks of 256 threads
+@pytest.mark.parametrize("T", [256, 257])
+@pytest.mark.parametrize("H,G,dim", [(2, 1, 16), (40, 8, 128), (72, 8, 128), (3, 1, 10)])
+@pytest.mark.parametrize("taps,norm_all", [(0, True), (0, False), (1, True), (4, False), (4, True), (6, True)])
+def test_norm_and_rotation_by_number_of_rows(taps, norm_all, H, G, dim, T):
+    g = torch.Generator().manual_seed(H + taps)
+    W, lens, page = (H + 2 * G) * dim, _lens(T), 32
+    proj, state = torch.randn(T, W, generator=g), torch.randn(2 * len(lens), max(taps - 1, 0), W, generator=g)
+    qn, kn = (torch.randn(n * dim if norm_all else dim, generator=g) for n in (H, G))
+    w, freq = torch.randn(max(taps, 1), W, generator=g), 1000.0 ** -torch.linspace(0, 1, dim // 2)
+    rows = _rows(lens)
+    slots = torch.randperm(9 * page, generator=g)[:T].to(torch.int32)
+    slots[5] = -1
+
+    def call(dev, f, st):
+        m = lambda x: x.to(dev)  # noqa: E731
+        q, kc, vc = torch.empty(T, H, dim, device=dev), *(torch.full((9, G, page, dim), 7.0, device=dev) for _ in range(2))
+        rs, rb, rf, pos = (m(r) for r in rows)
+        f(m(proj), None, m(qn), m(kn), norm_all, dim, 1e-5, pos, m(freq), 1.5, 0, 0, m(slots), kc, vc, H, G, dim, dim,
+          dim, 0, q, conv=(m(w), st, rs, rb, rf) if taps else None)
+        return q, kc, vc, st
+
+    got, want = call(DEV, ops.qk_norm_rotary_append, state.to(DEV)), call("cpu", ref.qk_norm_rotary_append, state.clone())
+    # a normed entry times weight and sine, up to 30, after some ten roundings of 2^-24; values: sums
+    # of up to six products of at most 25
+    for a, b in zip(got, want):
+        torch.testing.assert_close(a.cpu(), b, atol=3e-5, rtol=1e-5)
