@@ -132,6 +132,9 @@ __global__ __launch_bounds__(256) void gated_linrec_kernel(
           }
         }
         const float u = bj * (vj - acc);
+        // the channels' operands are read from LDS again: kept from the sum above they are four times
+        // the state's registers, spilled
+        asm volatile("" ::: "memory");
         if (NR > 0) {
           float po[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
