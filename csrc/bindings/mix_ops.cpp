@@ -51,6 +51,8 @@ void launch_token_shift_mix(bool, const float*, const float*, float*, const int3
                             const int32_t*, const int32_t*, const int32_t*, void*, int, int, int,
                             int, hipStream_t);
 bool wkv_ok(int);
+bool rank_product_ok(int64_t, int64_t, int64_t);
+void launch_rank_product(bool, const void*, int64_t, const void*, int64_t, void*, int, int, int, hipStream_t);
 bool latent_mfma_ok(int, int);
 bool launch_attn_latent_mfma(const void*, int64_t, int64_t, const void*, const int32_t*, int,
                              const int32_t*, const int32_t*, const int32_t*, const int32_t*,
@@ -433,6 +435,28 @@ void token_shift_mix(const Tensor& x, const Tensor& mu, const Tensor& prev, cons
                                  i32p(row_state, "row_state", T), i32p(row_back, "row_back", T),
                                  i32p(row_fwd, "row_fwd", T), i32p(pos, "positions", T),
                                  out.data_ptr(), T, d, NS, (int)prev.size(0) / 2, stream());
+}
+
+bool rank_product_fits(const Tensor& x, const Tensor& w) {
+  return x.dim() == 2 && w.dim() == 2 && x.scalar_type() == at::kBFloat16 && w.scalar_type() == at::kBFloat16 &&
+         x.device() == w.device() && x.size(1) == w.size(1) &&
+         rfqmix::rank_product_ok(x.size(0), w.size(0), x.size(1)) && x.stride(1) == 1 && w.stride(1) == 1 &&
+         x.stride(0) % 8 == 0 && w.stride(0) % 8 == 0 && reinterpret_cast<uintptr_t>(x.data_ptr()) % 16 == 0 &&
+         reinterpret_cast<uintptr_t>(w.data_ptr()) % 16 == 0;
+}
+
+// x . w^T: the short and small products here, all others with the library
+Tensor matmul_short(const Tensor& x, const Tensor& w, bool out_f32) {
+  if (!rank_product_fits(x, w))
+    return out_f32 ? at::mm(x, w.t(), at::kFloat) : at::matmul(x, w.t());
+  Tensor y = at::empty({x.size(0), w.size(0)}, x.options().dtype(out_f32 ? at::kFloat : at::kBFloat16));
+  rfqmix::launch_rank_product(out_f32, x.data_ptr(), x.stride(0), w.data_ptr(), w.stride(0), y.data_ptr(),
+                              (int)x.size(0), (int)w.size(0), (int)x.size(1), stream());
+  return y;
+}
+
+Tensor matmul_short_meta(const Tensor& x, const Tensor& w, bool out_f32) {
+  return at::empty({x.size(0), w.size(0)}, x.options().dtype(out_f32 ? at::kFloat : x.scalar_type()));
 }
 
 void wkv_recurrence(const Tensor& r, const Tensor& k, const Tensor& v, const Tensor& zw,
@@ -1162,6 +1186,7 @@ TORCH_LIBRARY(rfq_mix, m) {
   m.def("latent_norm_append(Tensor x, Tensor w, float eps, Tensor slots, Tensor(a!) pool) -> ()");
   m.def("silu_mul_any(Tensor gate_up, Tensor(a!) out) -> ()");
   m.def("softcap(Tensor(a!) x, float cap) -> ()");
+  m.def("matmul_short(Tensor x, Tensor w, bool out_f32) -> Tensor");
   m.def("token_shift_mix(Tensor x, Tensor mu, Tensor(a!) prev, Tensor row_state, Tensor row_back, Tensor row_fwd, Tensor pos, Tensor(b!) out) -> ()");
   m.def("wkv_recurrence(Tensor r, Tensor k, Tensor v, Tensor zw, Tensor w0, Tensor u, Tensor gate, Tensor norm_w, float eps, Tensor(a!) state, Tensor row_state, Tensor row_back, Tensor row_fwd, Tensor pos, Tensor? run_rows, Tensor(b!) out) -> ()");
   m.def("moe_route_grouped(Tensor z, Tensor correction, int top, int groups, int keep, Tensor(a!) ids, Tensor(b!) weights) -> ()");
@@ -1205,6 +1230,7 @@ TORCH_LIBRARY_IMPL(rfq_mix, CUDA, m) {
   m.impl("silu_mul_any", &silu_mul_any);
   m.impl("softcap", &softcap);
   m.impl("token_shift_mix", &token_shift_mix);
+  m.impl("matmul_short", &matmul_short);
   m.impl("wkv_recurrence", &wkv_recurrence);
   m.impl("moe_route_grouped", &moe_route_grouped);
   m.impl("moe_pair_up", &moe_pair_up);
@@ -1220,3 +1246,5 @@ TORCH_LIBRARY_IMPL(rfq_mix, CUDA, m) {
   m.impl("moe_route_topk", &moe_route_topk);
   m.impl("gelu_rows", &gelu_rows);
 }
+
+TORCH_LIBRARY_IMPL(rfq_mix, Meta, m) { m.impl("matmul_short", &matmul_short_meta); }

@@ -1007,9 +1007,23 @@ def reset_plans() -> None:
 _MM_OUT_DTYPE = None      # whether torch.mm takes out_dtype on this build (probed once)
 
 
+SHORT_K = 128       # matmul_nt: bf16 products of up to as many terms have a kernel (mix_rank.hip)
+
+
+def _plain(x, w) -> bool:
+    """No derivative of x . w^T is asked for, backward or forward."""
+    return (not (torch.is_grad_enabled() and (x.requires_grad or w.requires_grad))
+            and torch.autograd.forward_ad._current_level < 0)
+
+
 def matmul_nt(x, w, out_dtype=None):
     """x[M, K] . w[N, K]^T on the vendor library (fp32 accumulation; true fp32 for fp32
-    operands); ``out_dtype`` float32 keeps the accumulator's precision for bf16 operands."""
+    operands); ``out_dtype`` float32 keeps the accumulator's precision for bf16 operands.  Short
+    bf16 products (a low-rank projection's second factor) of few rows run on a kernel: the
+    library's host work, 20 us a call, is what bounds them."""
+    if (x.is_cuda and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and x.dim() == 2 and w.dim() == 2
+            and 32 <= w.shape[1] <= SHORT_K and out_dtype in (None, torch.bfloat16, torch.float32) and _plain(x, w)):
+        return _native.mix_ops().matmul_short(x, w, out_dtype == torch.float32)
     if out_dtype is None or out_dtype == x.dtype:
         return x @ w.t()
     if x.shape[0] == 0:
