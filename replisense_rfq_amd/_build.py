@@ -41,6 +41,9 @@ RT_SO = PKG_DIR / f"_runtime{sysconfig.get_config_var('EXT_SUFFIX') or '.so'}"
 KERNEL_FLAGS = [
     f"--offload-arch={ARCH}", "-O3", "-fPIC", "-std=c++17", "-mcode-object-version=5",
     "-ffp-contract=fast", "-munsafe-fp-atomics", "-Wno-unused-result",
+    # trap of this hardware generation: some packed-fp32 forms the compiler picks by itself
+    # have given wrong results, so the libraries are built without them
+    "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
 ]
 
 
@@ -90,9 +93,7 @@ def _link(out: Path, objs, libs, key_extra: str):
 
 
 MIX_SO = PKG_DIR / "_C_mix.so"
-# trap of this hardware generation: some packed-fp32 forms the compiler picks by itself
-# have given wrong results, so the new library is built without them
-MIX_FLAGS = KERNEL_FLAGS + ["-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]
+MIX_FLAGS = KERNEL_FLAGS
 
 
 def _bind_flags(tdir, abi):
