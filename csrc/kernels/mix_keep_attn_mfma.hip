@@ -110,7 +110,7 @@ __device__ __forceinline__ void store_rows(const KeepArgs& a, f32x4 (&o)[DV], fl
   const float l = both_halves_sum(both_rows_sum(lrun));
   if (!qlive) return;
   const bf16_t* gate = static_cast<const bf16_t*>(a.gate);
-  float mul = MODE == 2 ? a.out_mult : (l > 0.f ? a.out_mult / l : 0.f);
+  float mul = MODE >= 2 ? a.out_mult : (l > 0.f ? a.out_mult / l : 0.f);
   if (gate != nullptr && a.gate_w == 1) mul /= 1.0f + __expf(-ldf(gate + t * a.gate_stride + hh));
   // a gate column per output: four neighbouring logits, 8-byte reads
   const bf16_t* grow = gate != nullptr && a.gate_w > 1 ? gate + t * a.gate_stride + (int64_t)hh * vdim + grp * 4 : nullptr;
@@ -132,7 +132,7 @@ __device__ __forceinline__ void store_rows(const KeepArgs& a, f32x4 (&o)[DV], fl
 }
 
 // DK = E / 32, DV = vdim / 16, HPW heads per workgroup, SHARED: values = leading entries of the
-// key rows, MODE: 0 softmax, 1 softmax of capped scores, 2 sigmoid.
+// key rows, MODE: 0 softmax, 1 softmax of capped scores, 2 sigmoid, 3 sigmoid of capped scores.
 template <int DK, int DV, int HPW, bool SHARED, int MODE>
 __global__ __launch_bounds__(128 * HPW) void attn_keep_mfma_kernel(const KeepArgs a) {
   constexpr int E = 32 * DK, vdim = 16 * DV, NT = 128 * HPW;
@@ -164,9 +164,9 @@ __global__ __launch_bounds__(128 * HPW) void attn_keep_mfma_kernel(const KeepArg
   typedef const __attribute__((address_space(4))) int32_t const_i32;
   const_i32* bt = (const_i32*)(uintptr_t)(a.bt + (int64_t)s * a.maxb);
 
-  // scores arrive as exponents of 2: s log2 e; 2 s log2 e / cap; -s log2 e (sigmoid)
-  const float qmul = a.scale * (MODE == 1 ? 2.f * kLog2e / a.softcap : MODE == 2 ? -kLog2e : kLog2e);
-  const float cap2 = MODE == 1 ? a.softcap * kLog2e : 0.f;
+  // scores arrive as exponents of 2: s log2 e; 2 s log2 e / cap; -s log2 e (sigmoid, no cap)
+  const float qmul = a.scale * (MODE % 2 == 1 ? 2.f * kLog2e / a.softcap : MODE == 2 ? -kLog2e : kLog2e);
+  const float cap2 = MODE % 2 == 1 ? a.softcap * kLog2e : 0.f;
   s16x8 qhi[DK], qlo[DK];
   {
     const float* qp = a.q + (t * a.H + hh) * E + grp * 8;
@@ -182,7 +182,7 @@ __global__ __launch_bounds__(128 * HPW) void attn_keep_mfma_kernel(const KeepArg
 #pragma unroll
   for (int m = 0; m < DV; ++m) o[m] = (f32x4){0.f, 0.f, 0.f, 0.f};
   const float hb = a.head_bias != nullptr ? a.head_bias[hh] * kLog2e : 0.f;
-  const bool sink = MODE != 2 && a.head_bias != nullptr;
+  const bool sink = MODE < 2 && a.head_bias != nullptr;
   // the sink is one more entry of the row: it starts the maximum, and one lane's part of the sum
   float mrun = sink ? hb : kNegInfW, lrun = sink && grp == 0 ? 1.f : 0.f;
 
@@ -273,8 +273,8 @@ __global__ __launch_bounds__(128 * HPW) void attn_keep_mfma_kernel(const KeepArg
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
       float x = sc[i >> 2][0][i & 3] + sc[i >> 2][1][i & 3];
-      if constexpr (MODE == 1) x = cap2 - 2.f * cap2 * __builtin_amdgcn_rcpf(__builtin_amdgcn_exp2f(x) + 1.f);
-      if constexpr (MODE == 2) x = __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(x - hb));
+      if constexpr (MODE % 2 == 1) x = cap2 - 2.f * cap2 * __builtin_amdgcn_rcpf(__builtin_amdgcn_exp2f(x) + 1.f);
+      if constexpr (MODE >= 2) x = __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f((MODE == 3 ? -x : x) - hb));
       p[i] = x;
     }
     if (!(jb + WBS - 1 <= p0 && (window <= 0 || plast - jb < window || jb + WBS <= keep_first))) {
@@ -282,10 +282,10 @@ __global__ __launch_bounds__(128 * HPW) void attn_keep_mfma_kernel(const KeepArg
       for (int i = 0; i < 8; ++i) {                          // an edge inside the page
         const int j = jb + (i >> 2) * 16 + grp * 4 + (i & 3);
         const bool ok = j <= pi && (window <= 0 || pi - j < window || j < keep_first);
-        p[i] = ok ? p[i] : MODE == 2 ? 0.f : kNegInfW;
+        p[i] = ok ? p[i] : MODE >= 2 ? 0.f : kNegInfW;
       }
     }
-    if constexpr (MODE != 2) {
+    if constexpr (MODE < 2) {
       float mx = fmaxf(fmaxf(fmaxf(p[0], p[1]), fmaxf(p[2], p[3])), fmaxf(fmaxf(p[4], p[5]), fmaxf(p[6], p[7])));
       mx = other_half_max(other_row_max(mx));
       const bool moves = mx > mrun + kDeferW;                // also for the first keys: mrun = -inf
@@ -381,8 +381,8 @@ __global__ __launch_bounds__(128 * HPW, 2) void attn_keep_wide_kernel(const Keep
   typedef const __attribute__((address_space(4))) int32_t const_i32;
   const_i32* bt = (const_i32*)(uintptr_t)(a.bt + (int64_t)s * a.maxb);
 
-  const float qmul = a.scale * (MODE == 1 ? 2.f * kLog2e / a.softcap : MODE == 2 ? -kLog2e : kLog2e);
-  const float cap2 = MODE == 1 ? a.softcap * kLog2e : 0.f;
+  const float qmul = a.scale * (MODE % 2 == 1 ? 2.f * kLog2e / a.softcap : MODE == 2 ? -kLog2e : kLog2e);
+  const float cap2 = MODE % 2 == 1 ? a.softcap * kLog2e : 0.f;
   s16x8 qhi[DK], qlo[QLO ? DK : 1];
   {
     const float* qp = a.q + (t * a.H + hh) * E + grp * 8;
@@ -399,7 +399,7 @@ __global__ __launch_bounds__(128 * HPW, 2) void attn_keep_wide_kernel(const Keep
 #pragma unroll
   for (int m = 0; m < DV; ++m) o[m] = (f32x4){0.f, 0.f, 0.f, 0.f};
   const float hb = a.head_bias != nullptr ? a.head_bias[hh] * kLog2e : 0.f;
-  const bool sink = MODE != 2 && a.head_bias != nullptr;
+  const bool sink = MODE < 2 && a.head_bias != nullptr;
   float mrun = sink ? hb : kNegInfW, lrun = sink && grp == 0 ? 1.f : 0.f;      // sums: a quarter per lane
 
   int src[ND];                                               // this lane's source pieces, in shorts
@@ -483,8 +483,8 @@ __global__ __launch_bounds__(128 * HPW, 2) void attn_keep_wide_kernel(const Keep
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
       float x = sc[i >> 2][0][i & 3] + sc[i >> 2][1][i & 3];
-      if constexpr (MODE == 1) x = cap2 - 2.f * cap2 * __builtin_amdgcn_rcpf(__builtin_amdgcn_exp2f(x) + 1.f);
-      if constexpr (MODE == 2) x = __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(x - hb));
+      if constexpr (MODE % 2 == 1) x = cap2 - 2.f * cap2 * __builtin_amdgcn_rcpf(__builtin_amdgcn_exp2f(x) + 1.f);
+      if constexpr (MODE >= 2) x = __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f((MODE == 3 ? -x : x) - hb));
       p[i] = x;
     }
     if (!(jb + WBS - 1 <= p0 && (window <= 0 || plast - jb < window || jb + WBS <= keep_first))) {
@@ -492,10 +492,10 @@ __global__ __launch_bounds__(128 * HPW, 2) void attn_keep_wide_kernel(const Keep
       for (int i = 0; i < 8; ++i) {                          // an edge inside the page
         const int j = jb + (i >> 2) * 16 + grp * 4 + (i & 3);
         const bool ok = j <= pi && (window <= 0 || pi - j < window || j < keep_first);
-        p[i] = ok ? p[i] : MODE == 2 ? 0.f : kNegInfW;
+        p[i] = ok ? p[i] : MODE >= 2 ? 0.f : kNegInfW;
       }
     }
-    if constexpr (MODE != 2) {
+    if constexpr (MODE < 2) {
       float mx = fmaxf(fmaxf(fmaxf(p[0], p[1]), fmaxf(p[2], p[3])), fmaxf(fmaxf(p[4], p[5]), fmaxf(p[6], p[7])));
       mx = other_half_max(other_row_max(mx));
       const bool moves = mx > mrun + kDeferW;                // also for the first keys: mrun = -inf
@@ -560,8 +560,10 @@ static void launch_keep_mfma_one(const KeepArgs& a) {
 
 template <int DK, int DV, int HPW, bool SHARED>
 static void launch_keep_mfma_mode(const KeepArgs& a) {
-  if (a.sigmoid) launch_keep_mfma_one<DK, DV, HPW, SHARED, 2>(a);
-  else if (a.softcap > 0.f) launch_keep_mfma_one<DK, DV, HPW, SHARED, 1>(a);
+  const bool cap = a.softcap > 0.f;
+  if (a.sigmoid && cap) launch_keep_mfma_one<DK, DV, HPW, SHARED, 3>(a);
+  else if (a.sigmoid) launch_keep_mfma_one<DK, DV, HPW, SHARED, 2>(a);
+  else if (cap) launch_keep_mfma_one<DK, DV, HPW, SHARED, 1>(a);
   else launch_keep_mfma_one<DK, DV, HPW, SHARED, 0>(a);
 }
 

@@ -1,0 +1,62 @@
+"""attn_keep_window on MFMA tiles against 64-bit attention: options together, and the precision of
+queries, scores and weights, seen through values that cancel."""
+import pytest
+import torch
+
+from replisense_rfq_amd import ops
+
+pytestmark = pytest.mark.gpu
+DEV, BS = "cuda", 32
+
+
+def _exact(q, k, v, bias, scale, window, keep_first, sigmoid, softcap):
+    """q [T, H, E], k [L, G, E], v [L, G, vd]; the rows are the sequence's last T.  64 bits."""
+    T, H, L, rep = q.shape[0], q.shape[1], k.shape[0], q.shape[1] // k.shape[1]
+    k, v = (x.double().repeat_interleave(rep, 1) for x in (k, v))
+    i, j = torch.arange(L - T, L)[:, None], torch.arange(L)[None]
+    ok = (j <= i) & ((i - j < window) | (j < keep_first) if window else True)
+    s = torch.stack([q.double()[:, h] @ k[:, h].t() for h in range(H)]) * scale
+    if softcap:
+        s = softcap * torch.tanh(s / softcap)
+    b = None if bias is None else bias.double()[:, None, None]
+    if sigmoid:
+        w = torch.sigmoid(s + b) * ok
+    else:
+        s = s.masked_fill(~ok, float("-inf"))
+        w = torch.softmax(s if b is None else torch.cat([s, b.expand(H, T, 1)], -1), -1)[..., :L]
+    return torch.stack([w[h] @ v[:, h] for h in range(H)], 1)
+
+
+def _both(q, k, v, prompt, bias=None, scale=1.0, window=0, keep_first=0, sigmoid=False, softcap=0.0):
+    """(ops.attn_keep_window, 64 bits), [T, H, vd]; v None: the keys' leading entries."""
+    T, H, E = q.shape
+    L, G = k.shape[:2]
+    nb = (L + BS - 1) // BS
+    pages = lambda x: torch.cat([x, torch.zeros(nb * BS - L, *x.shape[1:], dtype=x.dtype)]) \
+        .view(nb, BS, G, -1).transpose(1, 2).flip(0).contiguous().to(DEV)  # noqa: E731
+    i32 = lambda *x: torch.tensor(x, dtype=torch.int32, device=DEV)  # noqa: E731
+    kd = pages(k)
+    vd = E - 64 if v is None else v.shape[2]
+    out = torch.empty(T, H * vd, dtype=torch.bfloat16, device=DEV)
+    blocks = range((T + 31) // 32)
+    ops.attn_keep_window(q.to(DEV), kd, kd if v is None else pages(v), vd, i32(*range(nb - 1, -1, -1))[None], i32(0),
+                         i32(T), i32(L), i32(*[0 for _ in blocks]), i32(*blocks), None if bias is None else bias.to(DEV),
+                         None, out, scale, window=window, keep_first=keep_first, sigmoid=sigmoid, softcap=softcap,
+                         short_rows=0 if prompt else T)
+    want = _exact(q, k, k[..., :vd] if v is None else v, bias, scale, window, keep_first, sigmoid, softcap)
+    return out.view(T, H, vd).double().cpu(), want
+
+
+@pytest.mark.parametrize("prompt", [True, False])
+@pytest.mark.parametrize("H,G,E,vd", [(8, 2, 128, 128), (3, 3, 64, 32), (8, 1, 320, 0), (4, 1, 576, 0)])
+def test_sigmoid_weights_of_capped_scores(H, G, E, vd, prompt):
+    """The cap binds: scores of 6 rms under a cap of 4, weights of some hundred keys."""
+    g = torch.Generator().manual_seed(E + H)
+    T, L = (70, 150) if prompt else (2, 150)
+    q, k = torch.randn(T, H, E, generator=g) * 6, torch.randn(L, G, E, generator=g).bfloat16()
+    v = torch.randn(L, G, vd, generator=g).bfloat16() if vd else None
+    got, want = _both(q, k, v, prompt, torch.randn(H, generator=g) - 1, E ** -0.5, 90, 5, True, 4.0)
+    # half a bf16 step of the result, and of the wide queries: 2^-9 of scores of 6, whose weights
+    # of 150 keys add up in quadrature
+    err, rms = (got - want).abs(), want.square().mean().sqrt()
+    assert bool((err <= 2.0 ** -8 * want.abs() + 2.0 ** -5 * rms).all())
