@@ -344,7 +344,7 @@ __global__ __launch_bounds__(128 * HPW) void attn_keep_mfma_kernel(const KeepArg
 // has 16 queries on 16x16x32 tiles, two waves a head, and the page's LDS reads are what bounds it (K
 // rows 36 x 1 KB, V 64 x 512 B a wave and page: 4,350 clocks for eight waves against 3,200 of MFMA).
 // One prompt of 2,048 over 576 (32 heads) took 904 us a pass on the kernel above, 420 here; four of
-// them with 64 heads 3,249 and 1,414.  Pages come by LDS-DMA, the next one during this one; their rows lie unpadded, 16-byte pieces
+// them with 64 heads 3,249 and 1,402.  Pages come by LDS-DMA, the next one during this one; their rows lie unpadded, 16-byte pieces
 // permuted inside each 128 bytes by wide_swizzle(row).
 // Sixteen rows of one piece (a K read) and four neighbouring rows of a pair of pieces beside the next
 // four (a transposed V read) then lie on different banks: the row's parity picks a half of them, bits
@@ -402,18 +402,22 @@ __global__ __launch_bounds__(128 * HPW, 2) void attn_keep_wide_kernel(const Keep
   const bool sink = MODE < 2 && a.head_bias != nullptr;
   float mrun = sink ? hb : kNegInfW, lrun = sink && grp == 0 ? 1.f : 0.f;      // sums: a quarter per lane
 
-  int src[ND];                                               // this lane's source pieces, in shorts
+  uint32_t src[ND];                                          // this lane's source pieces, bytes from the page's first
 #pragma unroll
   for (int i = 0; i < ND; ++i) {
     const int p = (wid + i * NWV) * 64 + lane, r = p / (E / 8), c = p - r * (E / 8);
-    src[i] = r * E + ((c & ~7) | ((c & 7) ^ wide_swizzle(r))) * 8;
+    src[i] = (r * E + ((c & ~7) | ((c & 7) ^ wide_swizzle(r))) * 8) * 2;
   }
   auto fetch = [&](int page, int buf) {
-    const bf16_t* kb = static_cast<const bf16_t*>(a.k_cache) + ((int64_t)page * a.G + g) * WBS * E;
+    const char* kb = static_cast<const char*>(a.k_cache) + ((int64_t)page * a.G + g) * WBS * E * 2;
 #pragma unroll
     for (int i = 0; i < ND; ++i) {
       const int piece = wid + i * NWV;
-      if (piece < NP) rfq::glds16(kb + src[i], reinterpret_cast<bf16_t*>(pages + buf * WBS * E + piece * 512));
+      uint32_t at = src[i];
+      asm("" : "+v"(at));      // widened here: hoisted out of the loop the offsets are pairs of registers, spilled
+      if ((i + 1) * NWV <= NP || piece < NP)
+        rfq::glds16(reinterpret_cast<const bf16_t*>(kb + at),
+                    reinterpret_cast<bf16_t*>(pages + buf * WBS * E + piece * 512));
     }
   };
   // The page has landed for everyone, who is done with the one before the last; rows past the sequence's end were never written: zeros.
