@@ -13,8 +13,8 @@
 //
 //   S^T[key, query] = K[key, :] . Q[query, :]   v_mfma_f32_16x16x32_bf16, A = key rows from LDS,
 //                     B = the queries in registers as bf16 hi (+ lo for keys of up to 320
-//                     entries: they arrive in fp32 and are not rounded a second time), already
-//                     times the scale and log2 e
+//                     entries: they arrive in fp32 and are not rounded a second time), up to 192
+//                     entries already times the scale and log2 e
 //   cap, mask, weights per query column in fp32, base 2
 //   O^T[dv, query] += V^T[dv, keys] . P^T[keys, query]   A = two transposed reads of V
 //                     (ds_read_tr16_b64), B = the weights straight from the score registers as bf16
@@ -381,7 +381,8 @@ __global__ __launch_bounds__(128 * HPW, 2) void attn_keep_wide_kernel(const Keep
   typedef const __attribute__((address_space(4))) int32_t const_i32;
   const_i32* bt = (const_i32*)(uintptr_t)(a.bt + (int64_t)s * a.maxb);
 
-  const float qmul = a.scale * (MODE % 2 == 1 ? 2.f * kLog2e / a.softcap : MODE == 2 ? -kLog2e : kLog2e);
+  const float qmul = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(
+      a.scale * (MODE % 2 == 1 ? 2.f * kLog2e / a.softcap : MODE == 2 ? -kLog2e : kLog2e))));
   const float cap2 = MODE % 2 == 1 ? a.softcap * kLog2e : 0.f;
   s16x8 qhi[DK], qlo[QLO ? DK : 1];
   {
@@ -390,7 +391,7 @@ __global__ __launch_bounds__(128 * HPW, 2) void attn_keep_wide_kernel(const Keep
     for (int ks = 0; ks < DK; ++ks) {
       const float4 x = *reinterpret_cast<const float4*>(qp + ks * 32);
       const float4 y = *reinterpret_cast<const float4*>(qp + ks * 32 + 4);
-      const float f[8] = {x.x * qmul, x.y * qmul, x.z * qmul, x.w * qmul, y.x * qmul, y.y * qmul, y.z * qmul, y.w * qmul};
+      const float f[8] = {x.x, x.y, x.z, x.w, y.x, y.y, y.z, y.w};   // as they are: bf16 values stay exact
       if constexpr (QLO) split_bf16w(f, qhi[ks], qlo[ks]);
       else qhi[ks] = rfq::pack8(f);
     }
@@ -486,7 +487,7 @@ __global__ __launch_bounds__(128 * HPW, 2) void attn_keep_wide_kernel(const Keep
     float p[8];
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
-      float x = sc[i >> 2][0][i & 3] + sc[i >> 2][1][i & 3];
+      float x = (sc[i >> 2][0][i & 3] + sc[i >> 2][1][i & 3]) * qmul;
       if constexpr (MODE % 2 == 1) x = cap2 - 2.f * cap2 * __builtin_amdgcn_rcpf(__builtin_amdgcn_exp2f(x) + 1.f);
       if constexpr (MODE >= 2) x = __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f((MODE == 3 ? -x : x) - hb));
       p[i] = x;

@@ -60,3 +60,28 @@ def test_sigmoid_weights_of_capped_scores(H, G, E, vd, prompt):
     # of 150 keys add up in quadrature
     err, rms = (got - want).abs(), want.square().mean().sqrt()
     assert bool((err <= 2.0 ** -8 * want.abs() + 2.0 ** -5 * rms).all())
+
+
+def _cancelling(T, L, H, G, E, vd, step, seed):
+    """Queries of 4,108 and a little more (``step``: of 4,096 and a multiple of it), keys +-1 in pairs
+    that cancel: the scores are the differences of the small parts."""
+    g = torch.Generator().manual_seed(seed)
+    small = torch.randn(T, H, E, generator=g)
+    small = (small * 4).round() * step if step else 12.0 + small / 4
+    s = torch.randint(0, 2, (L, G, E // 2), generator=g) * 2.0 - 1.0
+    k = torch.stack([s, -s], -1).reshape(L, G, E).bfloat16()
+    v = torch.randn(L, G, vd, generator=g).bfloat16() if vd else None
+    return 4096.0 + small, k, v
+
+
+def _near(got, want, part):
+    """Half a bf16 step of the value, and ``part`` of the results' rms."""
+    err, rms = (got - want).abs(), want.square().mean().sqrt()
+    assert bool((err <= 2.0 ** -8 * want.abs() + part * rms).all()), float(((err - 2.0 ** -8 * want.abs()) / rms).max())
+
+
+@pytest.mark.parametrize("H,E", [(4, 576), (6, 576), (3, 576), (8, 320)])
+def test_wide_prompt_queries_enter_as_they_are(H, E):
+    """Queries that bf16 holds exactly are not rounded again, whatever the scale."""
+    q, k, _ = _cancelling(70, 150, H, 1, E, 0, 32, E)
+    _near(*_both(q, k, None, True, scale=(2 * E) ** -0.5 / 32.0), 2.0 ** -8)
