@@ -365,8 +365,9 @@ __global__ __launch_bounds__(128 * HPW, 2) void attn_keep_wide_kernel(const Keep
   const int tid = threadIdx.x, lane = tid & 63;
   const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int col = lane & 15, grp = lane >> 4;
-  const int g = ((int)blockIdx.y * HPW) / (a.H / a.G);
-  const int hh = (int)blockIdx.y * HPW + (wid >> 1);
+  const int rep = a.H / a.G, per = (rep + HPW - 1) / HPW;     // workgroups of a key head, the last partly idle
+  const int g = (int)blockIdx.y / per, hd = ((int)blockIdx.y - g * per) * HPW + (wid >> 1);
+  const int hh = g * rep + min(hd, rep - 1);                 // past the last head: it once more, not stored
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   short* const pages = reinterpret_cast<short*>(smem);       // a ring of three
 
@@ -376,7 +377,7 @@ __global__ __launch_bounds__(128 * HPW, 2) void attn_keep_wide_kernel(const Keep
   const int jwin = window > 0 ? max(0, p0 - window + 1) : 0;
   const int kf = window > 0 ? min(keep_first, jwin) : 0;
   const int row = (wid & 1) * 16 + col, pi = p0 + row;       // this lane's query
-  const bool qlive = row < nq;
+  const bool qlive = row < nq && hd < rep;
   const int64_t t = a.q_start[s] + i0 + (qlive ? row : 0);
   typedef const __attribute__((address_space(4))) int32_t const_i32;
   const_i32* bt = (const_i32*)(uintptr_t)(a.bt + (int64_t)s * a.maxb);
@@ -557,7 +558,8 @@ static void launch_keep_mfma_one(const KeepArgs& a) {
                                 160 * 1024);
       attr = true;
     }
-    hipLaunchKernelGGL(kernel, dim3(a.W, a.H / HPW), dim3(threads), lds, a.s, a);
+    const int rep = a.H / a.G;
+    hipLaunchKernelGGL(kernel, dim3(a.W, a.G * ((rep + HPW - 1) / HPW)), dim3(threads), lds, a.s, a);
   };
   if constexpr (WIDE) run(&attn_keep_wide_kernel<DK, DV, HPW, MODE>, 128 * HPW);
   else run(&attn_keep_mfma_kernel<DK, DV, HPW, SHARED, MODE>, 128 * HPW);
@@ -575,7 +577,11 @@ static void launch_keep_mfma_mode(const KeepArgs& a) {
 template <int DK, int DV, bool SHARED>
 static void launch_keep_mfma_heads(const KeepArgs& a) {
   const int rep = a.H / a.G;
-  if (rep % 4 == 0) launch_keep_mfma_mode<DK, DV, 4, SHARED>(a);
+  // Odd groups of wide keys take four heads together too, the last workgroup's spare waves idle: a CU holds
+  // one workgroup of any size (the pages' LDS), and one head is two waves.  576 entries, sixteen chunks of
+  // 230 rows after 416 with 3 heads 178 us a pass -> 101, four prompts of 2,048 582 -> 238.
+  constexpr bool WIDE = SHARED && DK >= 10;
+  if (rep % 4 == 0 || (WIDE && rep % 2 == 1 && rep > 1)) launch_keep_mfma_mode<DK, DV, 4, SHARED>(a);
   else if (rep % 2 == 0) launch_keep_mfma_mode<DK, DV, 2, SHARED>(a);
   else launch_keep_mfma_mode<DK, DV, 1, SHARED>(a);
 }

@@ -85,3 +85,12 @@ def test_wide_prompt_queries_enter_as_they_are(H, E):
     """Queries that bf16 holds exactly are not rounded again, whatever the scale."""
     q, k, _ = _cancelling(70, 150, H, 1, E, 0, 32, E)
     _near(*_both(q, k, None, True, scale=(2 * E) ** -0.5 / 32.0), 2.0 ** -8)
+
+
+@pytest.mark.parametrize("H,G,E", [(3, 1, 576), (5, 1, 320), (14, 2, 320), (9, 3, 576), (2, 1, 576), (3, 3, 320)])
+def test_wide_prompts_of_heads_that_leave_waves_idle(H, G, E):
+    """Groups of 3, 5, 7, 3, 2 and 1 heads: nothing is written past a group's last one."""
+    g = torch.Generator().manual_seed(H)
+    q, k = torch.randn(70, H, E, generator=g), torch.randn(150, G, E, generator=g).bfloat16()
+    got, want = _both(q.bfloat16().float(), k, None, True, torch.randn(H, generator=g), E ** -0.5)
+    _near(got, want, 2.0 ** -9)
