@@ -369,7 +369,7 @@ __global__ __launch_bounds__(128 * HPW, 2) void attn_keep_wide_kernel(const Keep
   const int g = (int)blockIdx.y / per, hd = ((int)blockIdx.y - g * per) * HPW + (wid >> 1);
   const int hh = g * rep + min(hd, rep - 1);                 // past the last head: it once more, not stored
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-  short* const pages = reinterpret_cast<short*>(smem);       // a ring of three
+  short* const pages = reinterpret_cast<short*>(smem);       // two of them
 
   const int nq = min(WQB, ql - i0);
   const int p0 = a.kv_len[s] - ql + i0, plast = p0 + nq - 1;
@@ -422,7 +422,8 @@ __global__ __launch_bounds__(128 * HPW, 2) void attn_keep_wide_kernel(const Keep
                     reinterpret_cast<bf16_t*>(pages + buf * WBS * E + piece * 512));
     }
   };
-  // The page has landed for everyone, who is done with the one before the last; rows past the sequence's end were never written: zeros.
+  // The page has landed for everyone, and everyone is done with the one before it, whose place the next
+  // takes; rows past the sequence's end were never written: zeros.
   auto landed = [&](int jb, int buf) {
     __builtin_amdgcn_s_waitcnt(0x0F70);                      // vmcnt(0)
     __syncthreads();
@@ -468,9 +469,9 @@ __global__ __launch_bounds__(128 * HPW, 2) void attn_keep_wide_kernel(const Keep
   fetch(bt[pg], 0);
   int ahead = bt[min(next_page(pg), pg_last)];                 // the next page's number, read a page early
   while (pg <= pg_last) {
-    const int jb = pg * WBS, pn = next_page(pg), nbuf = buf == 2 ? 0 : buf + 1;
+    const int jb = pg * WBS, pn = next_page(pg);
     landed(jb, buf);
-    if (pn <= pg_last) fetch(ahead, nbuf);
+    if (pn <= pg_last) fetch(ahead, buf ^ 1);
     ahead = bt[min(next_page(pn), pg_last)];
     const short* P = pages + buf * WBS * E;
     f32x4 sc[2][2];                                          // two chains per half page
@@ -527,7 +528,7 @@ __global__ __launch_bounds__(128 * HPW, 2) void attn_keep_wide_kernel(const Keep
     split_bf16w(p, phi, plo);
     weigh(P);
     pg = pn;
-    buf = nbuf;
+    buf ^= 1;
   }
   store_rows<DV, MODE>(a, o, lrun, t, hh, grp, qlive);
 }
@@ -549,7 +550,7 @@ bool keep_mfma_ok(int E, int vdim, int BS, bool shared) {
 template <int DK, int DV, int HPW, bool SHARED, int MODE>
 static void launch_keep_mfma_one(const KeepArgs& a) {
   constexpr bool WIDE = SHARED && DK >= 10;
-  constexpr size_t lds = (size_t)(WIDE ? 3 * WBS * 32 * DK : 2 * keep_page_shorts<DK, DV, SHARED>()) * sizeof(short);
+  constexpr size_t lds = (size_t)2 * (WIDE ? WBS * 32 * DK : keep_page_shorts<DK, DV, SHARED>()) * sizeof(short);
   static_assert(lds <= 160 * 1024, "LDS of a CU");
   static bool attr = false;
   auto run = [&](auto kernel, int threads) {
@@ -577,9 +578,9 @@ static void launch_keep_mfma_mode(const KeepArgs& a) {
 template <int DK, int DV, bool SHARED>
 static void launch_keep_mfma_heads(const KeepArgs& a) {
   const int rep = a.H / a.G;
-  // Odd groups of wide keys take four heads together too, the last workgroup's spare waves idle: a CU holds
-  // one workgroup of any size (the pages' LDS), and one head is two waves.  576 entries, sixteen chunks of
-  // 230 rows after 416 with 3 heads 178 us a pass -> 101, four prompts of 2,048 582 -> 238.
+  // Odd groups of wide keys take four heads together too, the last workgroup's spare waves idle: one head is
+  // two waves, and the pages' LDS lets a CU hold two workgroups.  576 entries with 3 heads, sixteen chunks
+  // of 230 rows after 416: 120 us a pass with a head a workgroup, 101 so; four prompts of 2,048: 434, 238.
   constexpr bool WIDE = SHARED && DK >= 10;
   if (rep % 4 == 0 || (WIDE && rep % 2 == 1 && rep > 1)) launch_keep_mfma_mode<DK, DV, 4, SHARED>(a);
   else if (rep % 2 == 0) launch_keep_mfma_mode<DK, DV, 2, SHARED>(a);
