@@ -94,3 +94,16 @@ def test_wide_prompts_of_heads_that_leave_waves_idle(H, G, E):
     q, k = torch.randn(70, H, E, generator=g), torch.randn(150, G, E, generator=g).bfloat16()
     got, want = _both(q.bfloat16().float(), k, None, True, torch.randn(H, generator=g), E ** -0.5)
     _near(got, want, 2.0 ** -9)
+
+
+@pytest.mark.parametrize("prompt", [True, False])
+@pytest.mark.parametrize("H,G,E,vd", [(8, 2, 128, 128), (16, 1, 128, 128), (4, 1, 576, 0), (16, 1, 576, 0)])
+@pytest.mark.parametrize("opt", [{}, {"sigmoid": True}, {"softcap": 20.0}])
+def test_a_query_that_is_no_number_shows(H, G, E, vd, prompt, opt):
+    g = torch.Generator().manual_seed(3)
+    q, k = torch.randn(1, H, E, generator=g), torch.randn(150, G, E, generator=g).bfloat16()
+    v = torch.randn(150, G, vd, generator=g).bfloat16() if vd else None
+    q[0, 1, 5] = float("nan")
+    for bias in (torch.zeros(H), None)[:1 if opt.get("sigmoid") else 2]:
+        got, _ = _both(q, k, v, prompt, bias, E ** -0.5, **opt)
+        assert bool(got[0, 1].isnan().all()) and bool(got[0, [0, *range(2, H)]].isfinite().all())
