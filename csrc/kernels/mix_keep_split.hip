@@ -44,6 +44,14 @@ __device__ __forceinline__ void split_hl(const float* f, s16x8& hi, s16x8& lo) {
   lo = rfq::pack8(r);
 }
 
+// Lanes read here what others of their wave wrote to LDS.  The hardware keeps a wave's LDS accesses in
+// order, this keeps the compiler's; no instruction comes of it.
+__device__ __forceinline__ void wave_lds_order() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // keys per turn: a page, or half of one where queries and results of a wide latent fill the registers
 template <int DK, bool SHARED>
 constexpr int turn_keys() { return SHARED && DK >= 10 ? 16 : PG; }
@@ -204,6 +212,7 @@ __global__ __launch_bounds__(64 * NW, SHARED && DK >= 10 ? 1 : 2) void attn_keep
       }
 #pragma unroll
       for (int x = 0; x < NS; ++x) *reinterpret_cast<s16x8*>(St + piece_row(x) * SR + piece_at(x)) = sreg[set][x];
+      wave_lds_order();
       f32x4 sc[KT], sd[KT];
 #pragma unroll
       for (int kt = 0; kt < KT; ++kt) {
@@ -317,6 +326,7 @@ __global__ __launch_bounds__(64 * NW, SHARED && DK >= 10 ? 1 : 2) void attn_keep
             o[m + u] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(v[u], plo, o[m + u], 0, 0, 0);
         }
       }
+      wave_lds_order();                                    // the next turn's rows, or the partial results, take their place
     };
     if constexpr (AHEAD == 2) {
       int i = w;
