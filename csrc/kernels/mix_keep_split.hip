@@ -343,7 +343,8 @@ __global__ __launch_bounds__(64 * NW, SHARED && DK >= 10 ? 1 : 2) void attn_keep
     for (int m = 0; m < DV; ++m)
       *reinterpret_cast<f32x4*>(part + col * (vdim + 4) + 16 * m + 4 * grp) = o[m];
     if (grp == 0) {
-      ml[w * 16 + col] = mrun;
+      // scores that are no numbers leave the maximum at -inf, which marks a wave without visible keys
+      ml[w * 16 + col] = lrun != 0.f && mrun == kNegInfS ? 0.f : mrun;
       ml[(NW + w) * 16 + col] = lrun;
     }
     __syncthreads();
@@ -362,17 +363,17 @@ __global__ __launch_bounds__(64 * NW, SHARED && DK >= 10 ? 1 : 2) void attn_keep
         float l = sink ? __expf(hs - top) : 0.f;
 #pragma unroll
         for (int u = 0; u < NW; ++u) {
-          const float lu = ml[(NW + u) * 16 + cc];
-          l += lu == 0.f ? 0.f : lu * __expf(ml[u * 16 + cc] - top);
+          const float mu = ml[u * 16 + cc];
+          l += mu == kNegInfS ? 0.f : ml[(NW + u) * 16 + cc] * __expf(mu - top);
         }
         mul = l > 0.f ? a.out_mult / l : 0.f;
       }
       float y[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int u = 0; u < NW; ++u) {
-        // a wave without visible keys has the sum 0; one whose scores are no numbers has the maximum -inf too
-        if (!a.sigmoid && ml[(NW + u) * 16 + cc] == 0.f) continue;
-        const float f = a.sigmoid ? 1.f : __expf(ml[u * 16 + cc] - top);
+        const float mu = ml[u * 16 + cc];
+        if (!a.sigmoid && mu == kNegInfS) continue;        // a wave without visible keys
+        const float f = a.sigmoid ? 1.f : __expf(mu - top);
         const float4 p = *reinterpret_cast<const float4*>(
             smem + (size_t)u * wave_lds<DK, DV, SHARED>() + (size_t)(cc * (vdim + 4) + dv) * 4);
         y[0] += f * p.x; y[1] += f * p.y; y[2] += f * p.z; y[3] += f * p.w;
