@@ -12,7 +12,9 @@
 //
 // The 16 MFMA columns are (row, head) pairs of one key/value head, so the rows of a short extend and
 // the heads of a group share one pass.
-//   S^T[key, column] = K . Q^T, the fp32 queries as bf16 hi + lo; O^T = V^T . P^T, the weights likewise
+//   S^T[key, column] = K . Q^T, the fp32 queries as sums of bf16; O^T = V^T . P^T, the weights likewise
+// Groups of fewer than 16 heads take three parts of each, all of fp32's bits; wider ones two parts of the
+// weights, and of the queries two for keys of up to 320 entries, one above.
 //
 // SHARED (latent attention): a page's rows are keys and, their leading entries, values: staged once
 // in LDS, read as they lie for S and transposed for O.
@@ -36,13 +38,24 @@ constexpr float kNegInfS = -__builtin_huge_valf();
 // stay below e^8): most turns then leave the accumulators alone.
 constexpr float kDefer = 8.f;
 
-__device__ __forceinline__ void split_hl(const float* f, s16x8& hi, s16x8& lo) {
+// f as a sum of N bf16 values: three hold all 24 bits, two 16.  INF: f may be infinite, as one of them.
+template <bool INF, int N>
+__device__ __forceinline__ void split_parts(const float* f, s16x8 (&p)[N]) {
   float r[8];
-  hi = rfq::pack8(f);
 #pragma unroll
-  for (int i = 0; i < 8; ++i) r[i] = f[i] - rfq::bf2f_s(hi[i]);
-  lo = rfq::pack8(r);
+  for (int i = 0; i < 8; ++i) r[i] = f[i];
+#pragma unroll
+  for (int n = 0; n < N; ++n) {
+    p[n] = rfq::pack8(r);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const float h = rfq::bf2f_s(p[n][i]);
+      r[i] = INF && fabsf(h) == -kNegInfS ? 0.f : r[i] - h;
+    }
+  }
 }
+template <bool EXACT>
+__device__ __forceinline__ float exp_of(float x) { return EXACT ? expf(x) : __expf(x); }
 
 // Lanes read here what others of their wave wrote to LDS.  The hardware keeps a wave's LDS accesses in
 // order, this keeps the compiler's; no instruction comes of it.
@@ -60,10 +73,17 @@ template <int DK, bool SHARED>
 constexpr int turns_ahead() { return SHARED && DK >= 10 ? 2 : 1; }
 template <int DK, int DV, bool SHARED>
 constexpr int stage_row() { return SHARED ? 32 * DK + 8 : 16 * DV + 8; }      // shorts per staged row
-// a wave's LDS: its staged page, later its 16 x vdim partial results (rows of vdim + 4 floats)
-template <int DK, int DV, bool SHARED>
+// bf16 parts of a query entry
+template <int DK, bool EXACT>
+constexpr int query_parts() { return EXACT ? 3 : DK <= 10 ? 2 : 1; }
+// the partial results meet in as many passes: beside three parts of a wide latent's queries one is too large
+template <int DV, bool EXACT>
+constexpr int merge_passes() { return EXACT && DV > 16 ? 2 : 1; }
+// a wave's LDS: its staged page, later a pass of its 16 x vdim partial results (4 floats between rows)
+template <int DK, int DV, bool SHARED, bool EXACT>
 constexpr int wave_lds() {
-  return std::max(turn_keys<DK, SHARED>() * stage_row<DK, DV, SHARED>() * 2, 16 * (16 * DV + 4) * 4);
+  return std::max(turn_keys<DK, SHARED>() * stage_row<DK, DV, SHARED>() * 2,
+                  16 * (16 * DV / merge_passes<DV, EXACT>() + 4) * 4);
 }
 }  // namespace
 
@@ -84,14 +104,16 @@ struct KeepSplitArgs {
   int window, keep_first, sigmoid, H, G;
 };
 
-template <int DK, int DV, bool SHARED, int NW>
+// EXACT (groups of fewer than 16 heads): queries, weights and their functions in full fp32.
+template <int DK, int DV, bool SHARED, int NW, bool EXACT>
 __global__ __launch_bounds__(64 * NW, SHARED && DK >= 10 ? 1 : 2) void attn_keep_split_kernel(const KeepSplitArgs a) {
   constexpr int E = 32 * DK, vdim = 16 * DV, SR = stage_row<DK, DV, SHARED>();
   constexpr int KS = turn_keys<DK, SHARED>(), KT = KS / 16, AHEAD = turns_ahead<DK, SHARED>();
   constexpr bool QLDS = AHEAD == 2;
   constexpr int QR = E + 8;                              // shorts per query row in LDS
   constexpr int MG = DV % 4 == 0 ? 4 : 2;                // value blocks taken together
-  constexpr bool QLO = DK <= 10;                         // wider keys: as in the prompt kernel
+  constexpr int QP = query_parts<DK, EXACT>(), PP = EXACT ? 3 : 2;   // parts of a query entry, of a weight
+  constexpr int WL = wave_lds<DK, DV, SHARED, EXACT>(), MP = merge_passes<DV, EXACT>(), VP = vdim / MP;
   const int s = blockIdx.x, g = blockIdx.y;
   const int ql = a.q_len[s], kvl = a.kv_len[s];
   const int rep = a.H / a.G;
@@ -105,10 +127,10 @@ __global__ __launch_bounds__(64 * NW, SHARED && DK >= 10 ? 1 : 2) void attn_keep
   const int64_t t_first = a.q_start[s];
 
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-  short* St = reinterpret_cast<short*>(smem + (size_t)w * wave_lds<DK, DV, SHARED>());
-  float* part = reinterpret_cast<float*>(St);            // [16][vdim + 4]
-  float* ml = reinterpret_cast<float*>(smem + (size_t)NW * wave_lds<DK, DV, SHARED>());   // [NW][16] m, [NW][16] l
-  short* Qs = reinterpret_cast<short*>(ml + 2 * NW * 16);                                 // QLDS: [QLO ? 2 : 1][16][QR]
+  short* St = reinterpret_cast<short*>(smem + (size_t)w * WL);
+  float* part = reinterpret_cast<float*>(St);            // [16][VP + 4]
+  float* ml = reinterpret_cast<float*>(smem + (size_t)NW * WL);   // [NW][16] m, [NW][16] l
+  short* Qs = reinterpret_cast<short*>(ml + 2 * NW * 16);       // QLDS: [QP][16][QR]
 
   for (int ct = blockIdx.z; ct < tiles; ct += gridDim.z) {
     const int c = ct * 16 + col;                         // this lane's (row, head)
@@ -125,17 +147,17 @@ __global__ __launch_bounds__(64 * NW, SHARED && DK >= 10 ? 1 : 2) void attn_keep
     const int n_turns = n_keep + k_last - k_win + 1;
     auto keys_at = [&](int i) { return (i < n_keep ? i : k_win + i - n_keep) * KS; };
 
-    s16x8 qhi[QLDS ? 1 : DK], qlo[QLO && !QLDS ? DK : 1];
+    s16x8 qr[QLDS ? 1 : DK][QP];
     if constexpr (QLDS) {
       for (int x = tid; x < 16 * (E / 8); x += 64 * NW) {
         const int cc = x / (E / 8), e = (x - cc * (E / 8)) * 8, cx = min(ct * 16 + cc, ql * rep - 1), r = cx / rep;
         const float* qp = a.q + ((t_first + r) * a.H + g * rep + cx - r * rep) * E + e;
         const float4 u = *reinterpret_cast<const float4*>(qp), v = *reinterpret_cast<const float4*>(qp + 4);
         const float f[8] = {u.x, u.y, u.z, u.w, v.x, v.y, v.z, v.w};
-        s16x8 hi, lo;
-        split_hl(f, hi, lo);
-        *reinterpret_cast<s16x8*>(Qs + cc * QR + e) = hi;
-        if constexpr (QLO) *reinterpret_cast<s16x8*>(Qs + (16 + cc) * QR + e) = lo;
+        s16x8 p[QP];
+        split_parts<EXACT>(f, p);
+#pragma unroll
+        for (int n = 0; n < QP; ++n) *reinterpret_cast<s16x8*>(Qs + (16 * n + cc) * QR + e) = p[n];
       }
       __syncthreads();
     } else {
@@ -149,8 +171,7 @@ __global__ __launch_bounds__(64 * NW, SHARED && DK >= 10 ? 1 : 2) void attn_keep
         const float4 x = *reinterpret_cast<const float4*>(qp + at);
         const float4 y = *reinterpret_cast<const float4*>(qp + at + 4);
         f[0] = x.x; f[1] = x.y; f[2] = x.z; f[3] = x.w; f[4] = y.x; f[5] = y.y; f[6] = y.z; f[7] = y.w;
-        if constexpr (QLO) split_hl(f, qhi[ks], qlo[ks]);
-        else qhi[ks] = rfq::pack8(f);
+        split_parts<EXACT>(f, qr[ks]);
       }
     }
     f32x4 o[DV];
@@ -223,16 +244,13 @@ __global__ __launch_bounds__(64 * NW, SHARED && DK >= 10 ? 1 : 2) void attn_keep
           if constexpr (SHARED) kfr = *reinterpret_cast<const s16x8*>(St + (kt * 16 + col) * SR + grp * 8 + ks * 32);
           else kfr = kreg[kt][ks];
           f32x4& acc = ks % 2 == 0 ? sc[kt] : sd[kt];      // two chains
-          s16x8 hi, lo;
-          if constexpr (QLDS) {
-            hi = *reinterpret_cast<const s16x8*>(Qs + col * QR + grp * 8 + ks * 32);
-            if constexpr (QLO) lo = *reinterpret_cast<const s16x8*>(Qs + (16 + col) * QR + grp * 8 + ks * 32);
-          } else {
-            hi = qhi[ks];
-            if constexpr (QLO) lo = qlo[ks];
+#pragma unroll
+          for (int n = 0; n < QP; ++n) {
+            s16x8 q;
+            if constexpr (QLDS) q = *reinterpret_cast<const s16x8*>(Qs + (16 * n + col) * QR + grp * 8 + ks * 32);
+            else q = qr[ks][n];
+            acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(kfr), as_bf16x8(q), acc, 0, 0, 0);
           }
-          acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(kfr), as_bf16x8(hi), acc, 0, 0, 0);
-          if constexpr (QLO) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(kfr), as_bf16x8(lo), acc, 0, 0, 0);
         }
       }
       fetch(first_key(i + AHEAD * NW), page, set);           // in flight during the rest of this turn
@@ -256,7 +274,7 @@ __global__ __launch_bounds__(64 * NW, SHARED && DK >= 10 ? 1 : 2) void attn_keep
           const int j = jb + kt * 16 + grp * 4 + e;
           const bool ok = live && j <= pi && (a.window <= 0 || pi - j < a.window || j < a.keep_first);
           if (a.sigmoid) {
-            pv[kt * 4 + e] = ok ? 1.0f / (1.0f + __expf(-(sc[kt][e] + hb))) : 0.f;
+            pv[kt * 4 + e] = ok ? 1.0f / (1.0f + exp_of<EXACT>(-(sc[kt][e] + hb))) : 0.f;
           } else {
             sc[kt][e] = ok ? sc[kt][e] : kNegInfS;
             mx = fmaxf(mx, sc[kt][e]);
@@ -272,13 +290,13 @@ __global__ __launch_bounds__(64 * NW, SHARED && DK >= 10 ? 1 : 2) void attn_keep
         for (int kt = 0; kt < KT; ++kt)
 #pragma unroll
           for (int e = 0; e < 4; ++e) {
-            const float p = sc[kt][e] == kNegInfS ? 0.f : __expf(sc[kt][e] - mn);
+            const float p = sc[kt][e] == kNegInfS ? 0.f : exp_of<EXACT>(sc[kt][e] - mn);
             pv[kt * 4 + e] = p;
             sum += p;
           }
         sum += __shfl_xor(sum, 16, 64);
         sum += __shfl_xor(sum, 32, 64);
-        alpha = mrun == kNegInfS ? 0.f : __expf(mrun - mn);
+        alpha = mrun == kNegInfS ? 0.f : exp_of<EXACT>(mrun - mn);
         lrun = lrun * alpha + sum;
         mrun = mn;
       }
@@ -288,10 +306,10 @@ __global__ __launch_bounds__(64 * NW, SHARED && DK >= 10 ? 1 : 2) void attn_keep
       }
       const short* v0 = St + (4 * grp + (col >> 2)) * SR + 4 * (col & 3);
       if constexpr (KT == 2) {
-        s16x8 phi, plo;
-        split_hl(pv, phi, plo);
+        s16x8 pp[PP];
+        split_parts<false>(pv, pp);
 #pragma unroll
-        for (int m = 0; m < DV; m += MG) {                 // a value block's two products MG - 1 others apart
+        for (int m = 0; m < DV; m += MG) {                 // a value block's products MG - 1 others apart
           s16x8 v[MG];
 #pragma unroll
           for (int u = 0; u < MG; ++u) {
@@ -300,18 +318,21 @@ __global__ __launch_bounds__(64 * NW, SHARED && DK >= 10 ? 1 : 2) void attn_keep
             v[u] = (s16x8){a0[0], a0[1], a0[2], a0[3], a1[0], a1[1], a1[2], a1[3]};
           }
 #pragma unroll
-          for (int u = 0; u < MG; ++u)
-            o[m + u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(v[u]), as_bf16x8(phi), o[m + u], 0, 0, 0);
+          for (int n = 0; n < PP; ++n)
 #pragma unroll
-          for (int u = 0; u < MG; ++u)
-            o[m + u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(v[u]), as_bf16x8(plo), o[m + u], 0, 0, 0);
+            for (int u = 0; u < MG; ++u)
+              o[m + u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(v[u]), as_bf16x8(pp[n]), o[m + u], 0, 0, 0);
         }
       } else {
-        s16x4 phi, plo;
+        s16x4 pp[PP];
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          phi[e] = (short)rfq::f2bf(pv[e]);
-          plo[e] = (short)rfq::f2bf(pv[e] - rfq::bf2f_s(phi[e]));
+          float r = pv[e];
+#pragma unroll
+          for (int n = 0; n < PP; ++n) {
+            pp[n][e] = (short)rfq::f2bf(r);
+            r -= rfq::bf2f_s(pp[n][e]);
+          }
         }
 #pragma unroll
         for (int m = 0; m < DV; m += MG) {
@@ -319,11 +340,10 @@ __global__ __launch_bounds__(64 * NW, SHARED && DK >= 10 ? 1 : 2) void attn_keep
 #pragma unroll
           for (int u = 0; u < MG; ++u) v[u] = rfq::ds_read_tr16(v0 + 16 * (m + u));
 #pragma unroll
-          for (int u = 0; u < MG; ++u)
-            o[m + u] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(v[u], phi, o[m + u], 0, 0, 0);
+          for (int n = 0; n < PP; ++n)
 #pragma unroll
-          for (int u = 0; u < MG; ++u)
-            o[m + u] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(v[u], plo, o[m + u], 0, 0, 0);
+            for (int u = 0; u < MG; ++u)
+              o[m + u] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(v[u], pp[n], o[m + u], 0, 0, 0);
         }
       }
       wave_lds_order();                                    // the next turn's rows, or the partial results, take their place
@@ -338,87 +358,91 @@ __global__ __launch_bounds__(64 * NW, SHARED && DK >= 10 ? 1 : 2) void attn_keep
     } else {
       for (int i = w; i < n_turns; i += NW) turn(i, even);
     }
-    // ---- the waves' parts meet: [16 columns][vdim] each, beside their maxima and sums
+    // ---- the waves' parts meet: [16 columns][VP] each, beside their maxima and sums
 #pragma unroll
-    for (int m = 0; m < DV; ++m)
-      *reinterpret_cast<f32x4*>(part + col * (vdim + 4) + 16 * m + 4 * grp) = o[m];
-    if (grp == 0) {
-      // scores that are no numbers leave the maximum at -inf, which marks a wave without visible keys
-      ml[w * 16 + col] = lrun != 0.f && mrun == kNegInfS ? 0.f : mrun;
-      ml[(NW + w) * 16 + col] = lrun;
-    }
-    __syncthreads();
-    for (int x = tid; x < 16 * (vdim / 4); x += 64 * NW) {
-      const int cc = x / (vdim / 4), dv = (x - cc * (vdim / 4)) * 4, cx = ct * 16 + cc;
-      if (cx >= ql * rep) break;
-      const int r = cx / rep, hx = g * rep + cx - r * rep;
-      const int64_t t = t_first + r;
-      float mul = a.out_mult, top = kNegInfS;
-      if (!a.sigmoid) {
-        const bool sink = a.head_bias != nullptr;
-        const float hs = sink ? a.head_bias[hx] : kNegInfS;
-        top = hs;
+    for (int mp = 0; mp < MP; ++mp) {
+      if (mp > 0) __syncthreads();
 #pragma unroll
-        for (int u = 0; u < NW; ++u) top = fmaxf(top, ml[u * 16 + cc]);
-        float l = sink ? __expf(hs - top) : 0.f;
+      for (int m = 0; m < DV / MP; ++m)
+        *reinterpret_cast<f32x4*>(part + col * (VP + 4) + 16 * m + 4 * grp) = o[mp * (DV / MP) + m];
+      if (grp == 0) {
+        // scores that are no numbers leave the maximum at -inf, which marks a wave without visible keys
+        ml[w * 16 + col] = lrun != 0.f && mrun == kNegInfS ? 0.f : mrun;
+        ml[(NW + w) * 16 + col] = lrun;
+      }
+      __syncthreads();
+      for (int x = tid; x < 16 * (VP / 4); x += 64 * NW) {
+        const int cc = x / (VP / 4), dp = (x - cc * (VP / 4)) * 4, dv = mp * VP + dp, cx = ct * 16 + cc;
+        if (cx >= ql * rep) break;
+        const int r = cx / rep, hx = g * rep + cx - r * rep;
+        const int64_t t = t_first + r;
+        float mul = a.out_mult, top = kNegInfS;
+        if (!a.sigmoid) {
+          const bool sink = a.head_bias != nullptr;
+          const float hs = sink ? a.head_bias[hx] : kNegInfS;
+          top = hs;
+#pragma unroll
+          for (int u = 0; u < NW; ++u) top = fmaxf(top, ml[u * 16 + cc]);
+          float l = sink ? exp_of<EXACT>(hs - top) : 0.f;
+#pragma unroll
+          for (int u = 0; u < NW; ++u) {
+            const float mu = ml[u * 16 + cc];
+            l += mu == kNegInfS ? 0.f : ml[(NW + u) * 16 + cc] * exp_of<EXACT>(mu - top);
+          }
+          mul = l > 0.f ? a.out_mult / l : 0.f;
+        }
+        float y[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int u = 0; u < NW; ++u) {
           const float mu = ml[u * 16 + cc];
-          l += mu == kNegInfS ? 0.f : ml[(NW + u) * 16 + cc] * __expf(mu - top);
+          if (!a.sigmoid && mu == kNegInfS) continue;        // a wave without visible keys
+          const float f = a.sigmoid ? 1.f : exp_of<EXACT>(mu - top);
+          const float4 p = *reinterpret_cast<const float4*>(
+              smem + (size_t)u * WL + (size_t)(cc * (VP + 4) + dp) * 4);
+          y[0] += f * p.x; y[1] += f * p.y; y[2] += f * p.z; y[3] += f * p.w;
         }
-        mul = l > 0.f ? a.out_mult / l : 0.f;
-      }
-      float y[4] = {0.f, 0.f, 0.f, 0.f};
+        if (a.gate != nullptr && a.gate_w == 1) mul /= 1.0f + exp_of<EXACT>(-ldf(a.gate + t * a.gate_stride + hx));
+        bf16_t b[4];
 #pragma unroll
-      for (int u = 0; u < NW; ++u) {
-        const float mu = ml[u * 16 + cc];
-        if (!a.sigmoid && mu == kNegInfS) continue;        // a wave without visible keys
-        const float f = a.sigmoid ? 1.f : __expf(mu - top);
-        const float4 p = *reinterpret_cast<const float4*>(
-            smem + (size_t)u * wave_lds<DK, DV, SHARED>() + (size_t)(cc * (vdim + 4) + dv) * 4);
-        y[0] += f * p.x; y[1] += f * p.y; y[2] += f * p.z; y[3] += f * p.w;
+        for (int e = 0; e < 4; ++e) {
+          float v = y[e] * mul;
+          if (a.gate != nullptr && a.gate_w > 1)
+            v /= 1.0f + exp_of<EXACT>(-ldf(a.gate + t * a.gate_stride + (int64_t)hx * vdim + dv + e));
+          stf(&b[e], v);
+        }
+        *reinterpret_cast<uint2*>(a.out + t * a.out_stride + (int64_t)hx * vdim + dv) =
+            make_uint2((uint32_t)b[0] | ((uint32_t)b[1] << 16), (uint32_t)b[2] | ((uint32_t)b[3] << 16));
       }
-      if (a.gate != nullptr && a.gate_w == 1) mul /= 1.0f + __expf(-ldf(a.gate + t * a.gate_stride + hx));
-      bf16_t b[4];
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        float v = y[e] * mul;
-        if (a.gate != nullptr && a.gate_w > 1)
-          v /= 1.0f + __expf(-ldf(a.gate + t * a.gate_stride + (int64_t)hx * vdim + dv + e));
-        stf(&b[e], v);
-      }
-      *reinterpret_cast<uint2*>(a.out + t * a.out_stride + (int64_t)hx * vdim + dv) =
-          make_uint2((uint32_t)b[0] | ((uint32_t)b[1] << 16), (uint32_t)b[2] | ((uint32_t)b[3] << 16));
     }
     __syncthreads();                                       // the next column tile reuses the LDS
   }
 }
 
 // ------------------------------------------------------------------ launcher
-template <int DK, int DV, bool SHARED, int NW>
+template <int DK, int DV, bool SHARED, int NW, bool EXACT>
 static void launch_split_one(const KeepSplitArgs& a, int NA, int short_rows, hipStream_t s) {
-  constexpr size_t lds = (size_t)NW * wave_lds<DK, DV, SHARED>() + 2 * NW * 16 * sizeof(float) +
-                         (turns_ahead<DK, SHARED>() == 2 ? (DK <= 10 ? 2 : 1) * 16 * (32 * DK + 8) * 2 : 0);
+  constexpr size_t lds = (size_t)NW * wave_lds<DK, DV, SHARED, EXACT>() + 2 * NW * 16 * sizeof(float) +
+                         (turns_ahead<DK, SHARED>() == 2 ? query_parts<DK, EXACT>() * 16 * (32 * DK + 8) * 2 : 0);
   static_assert(lds <= 160 * 1024, "LDS of a CU");
   static bool attr = false;
   if (!attr) {          // dynamic LDS above 64 KB has to be allowed per kernel, once
-    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&attn_keep_split_kernel<DK, DV, SHARED, NW>),
+    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&attn_keep_split_kernel<DK, DV, SHARED, NW, EXACT>),
                               hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
     attr = true;
   }
   const int tiles = (short_rows * (a.H / a.G) + 15) / 16;
-  hipLaunchKernelGGL((attn_keep_split_kernel<DK, DV, SHARED, NW>), dim3(NA, a.G, tiles < 4 ? tiles : 4),
+  hipLaunchKernelGGL((attn_keep_split_kernel<DK, DV, SHARED, NW, EXACT>), dim3(NA, a.G, tiles < 4 ? tiles : 4),
                      dim3(64 * NW), lds, s, a);
 }
 
 // Eight waves to a workgroup where sequences and heads alone leave CUs idle: a wave's chain of
 // pages is the time then.  The wide latent's staged page leaves room for four.
-template <int DK, int DV, bool SHARED>
+template <int DK, int DV, bool SHARED, bool EXACT>
 static void launch_split_waves(const KeepSplitArgs& a, int NA, int short_rows, hipStream_t s) {
   if constexpr (!(SHARED && DK >= 10)) {
-    if (NA * a.G < 256) return launch_split_one<DK, DV, SHARED, 8>(a, NA, short_rows, s);
+    if (NA * a.G < 256) return launch_split_one<DK, DV, SHARED, 8, EXACT>(a, NA, short_rows, s);
   }
-  launch_split_one<DK, DV, SHARED, 4>(a, NA, short_rows, s);
+  launch_split_one<DK, DV, SHARED, 4, EXACT>(a, NA, short_rows, s);
 }
 
 // The sizes are those of keep_mfma_ok, which the caller has asked.
@@ -432,7 +456,10 @@ void launch_attn_keep_split(const float* q, const void* k_cache, const void* v_c
                         head_bias, (const bf16_t*)gate, gate_stride, gate_w, (bf16_t*)out, out_stride,
                         scale, softcap, out_mult, window, keep_first, (int)sigmoid, H, G};
   const int DK = E / 32, DV = vdim / 16;
-#define SPLIT_GO(dk, dv, sh) return launch_split_waves<dk, dv, sh>(a, NA, short_rows, s)
+  const bool exact = H / G < 16;
+#define SPLIT_GO(dk, dv, sh)                                                         \
+  return exact ? launch_split_waves<dk, dv, sh, true>(a, NA, short_rows, s)          \
+               : launch_split_waves<dk, dv, sh, false>(a, NA, short_rows, s)
   if (shared) {
     if (DK == 3) SPLIT_GO(3, 4, true);
     if (DK == 4 && DV == 4) SPLIT_GO(4, 4, true);

@@ -107,3 +107,36 @@ def test_a_query_that_is_no_number_shows(H, G, E, vd, prompt, opt):
     for bias in (torch.zeros(H), None)[:1 if opt.get("sigmoid") else 2]:
         got, _ = _both(q, k, v, prompt, bias, E ** -0.5, **opt)
         assert bool(got[0, 1].isnan().all()) and bool(got[0, [0, *range(2, H)]].isfinite().all())
+
+
+# Fewer than 16 heads share a key head: fp32 queries, weights and scores.
+GROUPS = [(8, 2, 128, 128), (3, 3, 64, 32), (15, 1, 96, 64), (4, 1, 320, 0), (15, 1, 576, 0), (5, 1, 576, 0)]
+
+
+@pytest.mark.parametrize("H,G,E,vd", GROUPS)
+def test_decode_weights_keep_32_bits(H, G, E, vd):
+    """Values that cancel in neighbouring keys, scores of rms 2^-12: the results are differences of
+    nearly equal weights.  Weights to 2^-24: 2^-12 of the results each way; to 16 bits: 2^-6."""
+    g = torch.Generator().manual_seed(E + 1)
+    L = 160
+    k, q = torch.randn(L, G, E, generator=g).bfloat16(), torch.randn(2, H, E, generator=g)
+    if vd:
+        v = torch.randn(L // 2, G, vd, generator=g).bfloat16()
+        v = torch.stack([v, -v], 1).view(L, G, vd)
+    else:                                       # the keys are the values: they differ in the last 64 entries
+        v = None
+        k[1::2, :, :E - 64] = -k[0::2, :, :E - 64]
+        q[..., :E - 64] = 0.0
+    n = 64 if v is None else E
+    got, want = _both(q, k, v, False, scale=2.0 ** -12 * n ** -0.5)
+    _near(got[1:], want[1:], 2.0 ** -8)         # the last row: an even number of keys
+
+
+@pytest.mark.parametrize("H,G,E,vd", GROUPS)
+def test_an_infinite_query_under_a_cap(H, G, E, vd):
+    """The head's scores are +-cap, whatever the other entries."""
+    g = torch.Generator().manual_seed(E + 3)
+    q, k = torch.randn(1, H, E, generator=g), torch.randn(150, G, E, generator=g).bfloat16()
+    v = torch.randn(150, G, vd, generator=g).bfloat16() if vd else None
+    q[0, 1, 3] = float("inf")
+    _near(*_both(q, k, v, False, scale=E ** -0.5, softcap=3.0), 2.0 ** -9)
