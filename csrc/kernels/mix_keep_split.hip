@@ -56,6 +56,19 @@ __device__ __forceinline__ void split_parts(const float* f, s16x8 (&p)[N]) {
 }
 template <bool EXACT>
 __device__ __forceinline__ float exp_of(float x) { return EXACT ? expf(x) : __expf(x); }
+// tanh to 1.6 units in the last place, without tanhf's branches (64 sequences of 300 - 900 tokens: 58.5 us a
+// pass with it, 57.5 with this, 56.4 with the wide groups' form).  Below 0.7 an odd
+// polynomial, fitted to a relative error of 1.6e-8; above, 1 - 2 / (exp(2 |x|) + 1).
+__device__ __forceinline__ float tanh_of(float x) {
+  const float u = x * x, ax = fabsf(x);
+  float p = -0.0051386617f;
+  p = p * u + 0.02009197f;
+  p = p * u - 0.05355886f;
+  p = p * u + 0.13329111f;
+  p = p * u - 0.3333319f;
+  const float big = 1.f - 2.f * __builtin_amdgcn_rcpf(__builtin_amdgcn_exp2f(ax * 2.88539008f) + 1.f);
+  return ax < 0.7f ? x + x * u * p : copysignf(big, x);
+}
 
 // Lanes read here what others of their wave wrote to LDS.  The hardware keeps a wave's LDS accesses in
 // order, this keeps the compiler's; no instruction comes of it.
@@ -257,13 +270,15 @@ __global__ __launch_bounds__(64 * NW, SHARED && DK >= 10 ? 1 : 2) void attn_keep
       page = page_of(i + (AHEAD + 1) * NW);
 #pragma unroll
       for (int kt = 0; kt < KT; ++kt) sc[kt] = (sc[kt] + sd[kt]) * a.scale;
-      if (a.softcap > 0.f) {                               // c tanh(s / c) = c - 2 c / (exp(2 s / c) + 1)
-        const float two_c = 2.f * a.softcap, inv = 2.f / a.softcap;
+      if (a.softcap > 0.f) {
+        // wide groups: c tanh(s / c) = c - 2 c / (exp(2 s / c) + 1), off by some 2^-23 of c
+        const float two_c = 2.f * a.softcap, inv1 = 1.f / a.softcap, inv = 2.f * inv1;
 #pragma unroll
         for (int kt = 0; kt < KT; ++kt)
 #pragma unroll
           for (int e = 0; e < 4; ++e)
-            sc[kt][e] = a.softcap - two_c * __builtin_amdgcn_rcpf(__expf(sc[kt][e] * inv) + 1.f);
+            sc[kt][e] = EXACT ? a.softcap * tanh_of(sc[kt][e] * inv1)
+                              : a.softcap - two_c * __builtin_amdgcn_rcpf(__expf(sc[kt][e] * inv) + 1.f);
       }
       float pv[4 * KT];
       float mx = kNegInfS;

@@ -140,3 +140,12 @@ def test_an_infinite_query_under_a_cap(H, G, E, vd):
     v = torch.randn(150, G, vd, generator=g).bfloat16() if vd else None
     q[0, 1, 3] = float("inf")
     _near(*_both(q, k, v, False, scale=E ** -0.5, softcap=3.0), 2.0 ** -9)
+
+
+@pytest.mark.parametrize("H,G,E,vd", GROUPS)
+def test_decode_scores_under_a_wide_cap(H, G, E, vd):
+    """A cap far above the scores leaves them as they are."""
+    g = torch.Generator().manual_seed(E + 2)
+    q, k = torch.randn(2, H, E, generator=g) * 2, torch.randn(150, G, E, generator=g).bfloat16()
+    v = torch.randn(150, G, vd, generator=g).bfloat16() if vd else None
+    _near(*_both(q, k, v, False, scale=E ** -0.5, softcap=2.0 ** 17), 2.0 ** -9)
