@@ -1012,8 +1012,9 @@ SHORT_K = 128       # matmul_nt: bf16 products of up to as many terms have a ker
 
 def _plain(x, w) -> bool:
     """No derivative of x . w^T is asked for, backward or forward."""
+    dual = torch.autograd.forward_ad.unpack_dual
     return (not (torch.is_grad_enabled() and (x.requires_grad or w.requires_grad))
-            and torch.autograd.forward_ad._current_level < 0)
+            and dual(x).tangent is None and dual(w).tangent is None)
 
 
 def matmul_nt(x, w, out_dtype=None):
