@@ -437,20 +437,19 @@ void token_shift_mix(const Tensor& x, const Tensor& mu, const Tensor& prev, cons
                                  out.data_ptr(), T, d, NS, (int)prev.size(0) / 2, stream());
 }
 
-bool rank_product_fits(const Tensor& x, const Tensor& w) {
-  return x.dim() == 2 && w.dim() == 2 && x.scalar_type() == at::kBFloat16 && w.scalar_type() == at::kBFloat16 &&
-         x.device() == w.device() && x.size(1) == w.size(1) &&
-         rfqmix::rank_product_ok(x.size(0), w.size(0), x.size(1)) && x.stride(1) == 1 && w.stride(1) == 1 &&
-         x.stride(0) % 8 == 0 && w.stride(0) % 8 == 0 && reinterpret_cast<uintptr_t>(x.data_ptr()) % 16 == 0 &&
-         reinterpret_cast<uintptr_t>(w.data_ptr()) % 16 == 0;
-}
-
-// x . w^T: the short and small products here, all others with the library
+// x . w^T for the short and small products; the caller sends no others.  Memory from elsewhere may
+// begin at any address: such an operand is copied.
 Tensor matmul_short(const Tensor& x, const Tensor& w, bool out_f32) {
-  if (!rank_product_fits(x, w))
-    return out_f32 ? at::mm(x, w.t(), at::kFloat) : at::matmul(x, w.t());
+  TORCH_CHECK(x.is_cuda() && x.dim() == 2 && w.dim() == 2 && x.scalar_type() == at::kBFloat16 &&
+              w.scalar_type() == at::kBFloat16 && x.device() == w.device() && x.size(1) == w.size(1) &&
+              rfqmix::rank_product_ok(x.size(0), w.size(0), x.size(1)), "matmul_short: x [M, K], w [N, K] bf16");
+  auto rows = [](const Tensor& t) {
+    TORCH_CHECK(t.stride(1) == 1 && t.stride(0) % 8 == 0, "matmul_short: rows of whole 16-byte pieces");
+    return reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0 ? t : t.clone(at::MemoryFormat::Contiguous);
+  };
+  const Tensor xr = rows(x), wr = rows(w);
   Tensor y = at::empty({x.size(0), w.size(0)}, x.options().dtype(out_f32 ? at::kFloat : at::kBFloat16));
-  rfqmix::launch_rank_product(out_f32, x.data_ptr(), x.stride(0), w.data_ptr(), w.stride(0), y.data_ptr(),
+  rfqmix::launch_rank_product(out_f32, xr.data_ptr(), xr.stride(0), wr.data_ptr(), wr.stride(0), y.data_ptr(),
                               (int)x.size(0), (int)w.size(0), (int)x.size(1), stream());
   return y;
 }

@@ -30,3 +30,48 @@ def test_forward_derivatives_pass():
     t = torch.randn_like(x)
     _, dy = torch.func.jvp(lambda y: ops.matmul_nt(y, w), (x,), (t,))
     torch.testing.assert_close(dy, t @ w.t())
+
+
+# what the kernel refuses: no rows, sums and columns that are no whole tiles, too many entries, strides,
+# unaligned rows; (rows, sums, columns)
+REFUSED = [(0, 64, 8), (5, 40, 8), (5, 24, 8), (5, 160, 8), (5, 64, 6), (5, 64, 2), (513, 64, 4096)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("out_dtype", [None, torch.float32])
+def test_what_the_kernel_refuses_takes_the_general_path(monkeypatch, out_dtype):
+    """The general path copes with a torch whose mm has no out_dtype, and with no rows."""
+    def mm(*args, **more):
+        raise TypeError("out_dtype")
+
+    monkeypatch.setattr(ops, "_MM_OUT_DTYPE", None)
+    monkeypatch.setattr(torch, "mm", mm)
+    op = ops._native.mix_ops()
+    monkeypatch.setattr(ops._native, "mix_ops", lambda: types.SimpleNamespace(matmul_short=mm))
+    g = torch.Generator().manual_seed(1)
+    for M, K, N in REFUSED:
+        wide = torch.randn(M, K + 8, generator=g).to(DEV, torch.bfloat16)
+        for x in (wide[:, :K], wide[:, 3:K + 3]) if K == 64 else (wide[:, :K],):
+            w = torch.randn(N, K, generator=g).to(DEV, torch.bfloat16)
+            y = ops.matmul_nt(x, w, out_dtype)
+            want = x.float() @ w.float().t()
+            assert y.shape == want.shape and y.dtype == (out_dtype or torch.bfloat16)
+            torch.testing.assert_close(y.float(), want, atol=1e-3, rtol=2.0 ** -8)
+    x, w = (torch.randn(n, 64, generator=g).to(DEV, torch.bfloat16) for n in (8, 12))
+    for a, b in ((x.t().contiguous().t(), w), (x, w.t().contiguous().t()), (x.repeat(1, 2)[:, 1:65], w),
+                 (torch.randn(8, 68, generator=g).to(DEV, torch.bfloat16)[:, :64], w)):
+        torch.testing.assert_close(ops.matmul_nt(a, b, out_dtype).float(), a.float() @ b.float().t(), atol=1e-3,
+                                   rtol=2.0 ** -8)
+    assert ops._MM_OUT_DTYPE is (False if out_dtype else None)
+    monkeypatch.setattr(ops._native, "mix_ops", lambda: op)
+    torch.testing.assert_close(ops.matmul_nt(x, w, torch.float32), x.float() @ w.float().t(), atol=1e-4, rtol=1e-4)
+
+
+@pytest.mark.gpu
+def test_memory_that_begins_at_an_odd_address():
+    """Rows of a tensor from elsewhere: whole strides, an offset of nought, an unaligned address."""
+    buf, w = torch.randn(8 * 64 + 1, device=DEV, dtype=torch.bfloat16), torch.randn(12, 64, device=DEV, dtype=torch.bfloat16)
+    x = torch.from_dlpack(buf[1:].view(8, 64))
+    assert x.storage_offset() == 0 and x.data_ptr() % 16 == 2
+    for a, b in ((x, w), (w, x)):
+        torch.testing.assert_close(ops.matmul_nt(a, b, torch.float32), a.float() @ b.float().t(), atol=1e-4, rtol=1e-4)
