@@ -5,6 +5,7 @@
 // host against what the kernels index before anything is launched.
 #include <torch/library.h>
 #include <ATen/ATen.h>
+#include <c10/core/DeviceGuard.h>
 #include <c10/hip/HIPStream.h>
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -443,6 +444,7 @@ Tensor matmul_short(const Tensor& x, const Tensor& w, bool out_f32) {
   TORCH_CHECK(x.is_cuda() && x.dim() == 2 && w.dim() == 2 && x.scalar_type() == at::kBFloat16 &&
               w.scalar_type() == at::kBFloat16 && x.device() == w.device() && x.size(1) == w.size(1) &&
               rfqmix::rank_product_ok(x.size(0), w.size(0), x.size(1)), "matmul_short: x [M, K], w [N, K] bf16");
+  const c10::DeviceGuard on(x.device());
   auto rows = [](const Tensor& t) {
     TORCH_CHECK(t.stride(1) == 1 && t.stride(0) % 8 == 0, "matmul_short: rows of whole 16-byte pieces");
     return reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0 ? t : t.clone(at::MemoryFormat::Contiguous);
@@ -452,6 +454,13 @@ Tensor matmul_short(const Tensor& x, const Tensor& w, bool out_f32) {
   rfqmix::launch_rank_product(out_f32, xr.data_ptr(), xr.stride(0), wr.data_ptr(), wr.stride(0), y.data_ptr(),
                               (int)x.size(0), (int)w.size(0), (int)x.size(1), stream());
   return y;
+}
+
+// under vmap: the library's product, which has a batched form; in fp32, as batched bf16 products with a
+// transposed right side are not safe on this hardware
+Tensor matmul_short_batched(const Tensor& x, const Tensor& w, bool out_f32) {
+  const Tensor y = at::matmul(x.to(at::kFloat), w.to(at::kFloat).t());
+  return out_f32 ? y : y.to(at::kBFloat16);
 }
 
 Tensor matmul_short_meta(const Tensor& x, const Tensor& w, bool out_f32) {
@@ -1246,4 +1255,5 @@ TORCH_LIBRARY_IMPL(rfq_mix, CUDA, m) {
   m.impl("gelu_rows", &gelu_rows);
 }
 
+TORCH_LIBRARY_IMPL(rfq_mix, FuncTorchBatched, m) { m.impl("matmul_short", &matmul_short_batched); }
 TORCH_LIBRARY_IMPL(rfq_mix, Meta, m) { m.impl("matmul_short", &matmul_short_meta); }

@@ -1,5 +1,6 @@
 """Which products of ops.matmul_nt go to the kernel for short ones, and which stay with the library."""
 import types
+import warnings
 
 import pytest
 import torch
@@ -75,3 +76,17 @@ def test_memory_that_begins_at_an_odd_address():
     assert x.storage_offset() == 0 and x.data_ptr() % 16 == 2
     for a, b in ((x, w), (w, x)):
         torch.testing.assert_close(ops.matmul_nt(a, b, torch.float32), a.float() @ b.float().t(), atol=1e-4, rtol=1e-4)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("out_dtype", [None, torch.float32])
+def test_a_batch_of_products_is_one(out_dtype):
+    """vmap: no loop over the batch, which torch announces with a warning."""
+    x, w = (torch.randn(3, n, 64, device=DEV, dtype=torch.bfloat16) for n in (8, 12))
+    want = torch.stack([a.float() @ b.float().t() for a, b in zip(x, w)])
+    with warnings.catch_warnings():
+        warnings.simplefilter("error")
+        for y, ref in ((torch.vmap(lambda a, b: ops.matmul_nt(a, b, out_dtype))(x, w), want),
+                       (torch.vmap(lambda a: ops.matmul_nt(a, w[0], out_dtype))(x), x.float() @ w[0].float().t())):
+            assert y.dtype == (out_dtype or torch.bfloat16)
+            torch.testing.assert_close(y.float(), ref, atol=1e-3, rtol=2.0 ** -8)
