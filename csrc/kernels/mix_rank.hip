@@ -1,10 +1,12 @@
 // Y[M, N] = X[M, K] . W[N, K]^T for short K (32, 64, 96 or 128; bf16 operands, fp32 sums, Y in bf16 or
 // fp32): the second factor of a low-rank projection.
 //
-// For products of up to 2^21 entries, where a launch and the host's work before it are what counts: 64
-// rows to 2,048 columns from K = 64 take 3.9 us on the device against 5.2 with the library, whose host
-// work of some 20 us a call is what bounded a decode step (64 rows of a delta rule layer: 64.7 -> 49.1 us
-// a pass).  Larger ones stay with the library: 4,096 rows 12.7 us there, 15.4 here.
+// For products where a launch and the host's work before it are what counts: an eager call takes 5 us
+// against the library's 19, which bounded a decode step (64 rows of a delta rule layer: 64.7 -> 49.1 us
+// a pass).  The lines lie where the device's time, all that a graph sees, is the library's: 2^21 entries
+// (512 x 4,096, 4,096 x 512, 64 x 32,768: K = 32 3.1 - 3.9 us against 4.3 - 5.0, 64 4.6 - 5.3 against
+// 4.6 - 5.6, 96 4.3 - 5.1 against 4.7 - 5.9), 2^20 for K = 128 (64 x 16,384 in bf16 4.3 us on both sides,
+// at 2^21 6.7 against 4.9).  4,096 rows of 2,048 columns, K = 64: 15.4 us against 12.7.
 //
 // No LDS: a wave has the W rows of 64 columns, all K of them, and 16 rows of X straight from memory in
 // 16-byte pieces.  Y comes out transposed in the accumulators (A = W, B = X), so a lane holds
@@ -68,7 +70,7 @@ __global__ __launch_bounds__(256) void rank_product_kernel(const bf16_t* __restr
 
 // ------------------------------------------------------------------ launcher
 bool rank_product_ok(int64_t M, int64_t N, int64_t K) {
-  return M >= 1 && K >= 32 && K <= 128 && K % 32 == 0 && N >= 4 && N % 4 == 0 && M <= (1 << 21) / N;
+  return M >= 1 && K >= 32 && K <= 128 && K % 32 == 0 && N >= 4 && N % 4 == 0 && M <= (1 << (K > 96 ? 20 : 21)) / N;
 }
 
 void launch_rank_product(bool out_f32, const void* x, int64_t xs, const void* w, int64_t ws, void* y, int M, int N,

@@ -1007,7 +1007,7 @@ def reset_plans() -> None:
 _MM_OUT_DTYPE = None      # whether torch.mm takes out_dtype on this build (probed once)
 
 
-SHORT_K, SHORT_ENTRIES = 128, 1 << 21   # matmul_nt: the short bf16 products that have a kernel (mix_rank.hip)
+SHORT_K = 128       # matmul_nt: bf16 products of up to as many terms have a kernel (mix_rank.hip)
 
 
 def _plain(x, w) -> bool:
@@ -1021,7 +1021,7 @@ def _short(x, w) -> bool:
     """The sizes and strides that rfq_mix.matmul_short takes."""
     M, K, N = x.shape[0], x.shape[1], w.shape[0]
     return (32 <= K <= SHORT_K and K % 32 == 0 and w.shape[1] == K and M >= 1 and N >= 4 and N % 4 == 0
-            and M * N <= SHORT_ENTRIES and x.device == w.device and x.stride(1) == 1 and w.stride(1) == 1
+            and M * N <= 1 << (20 if K > 96 else 21) and x.device == w.device and x.stride(1) == 1 and w.stride(1) == 1
             and x.stride(0) % 8 == 0 and w.stride(0) % 8 == 0
             and x.storage_offset() % 8 == 0 and w.storage_offset() % 8 == 0)
 

@@ -33,6 +33,13 @@ def test_forward_derivatives_pass():
     torch.testing.assert_close(dy, t @ w.t())
 
 
+@pytest.mark.parametrize("M,K,N,short", [(512, 96, 4096, True), (513, 64, 4096, False), (512, 128, 2048, True),
+                                         (512, 128, 2052, False), (2049, 128, 512, False)])
+def test_the_largest_product_of_a_kernel(M, K, N, short):
+    """Where the library's kernel is as fast: 2^21 entries, 2^20 with 128 terms."""
+    assert ops._short(torch.empty(M, K, dtype=torch.bfloat16), torch.empty(N, K, dtype=torch.bfloat16)) is short
+
+
 # what the kernel refuses: no rows, sums and columns that are no whole tiles, too many entries, strides,
 # unaligned rows; (rows, sums, columns)
 REFUSED = [(0, 64, 8), (5, 40, 8), (5, 24, 8), (5, 160, 8), (5, 64, 6), (5, 64, 2), (513, 64, 4096)]
