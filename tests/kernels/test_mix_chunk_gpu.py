@@ -132,3 +132,62 @@ def test_wkv_non_finite_value_stays_out_of_earlier_tokens():
     (out, _), (out_w, _) = _wkv(torch.float32, -2.0, (first + 9, 3, float("inf")))
     _close(out[:first + 9], out_w[:first + 9], 1e-5)
     _close(out[sum(LENS[:8]):], out_w[sum(LENS[:8]):], 1e-5)
+
+
+@pytest.mark.parametrize("mode", ["gla", "delta"])
+def test_decays_and_steps_keep_32_bits(mode):
+    """One write, one decay, no reads: the state is beta_0 a_0 and known to a few units in the last place.
+    Arguments of the exponentials are whole numbers, or a tiny softplus times a rate that fp32 holds."""
+    dim, H, n = 64, 2, 40
+    T, off = n, torch.arange(dim, dtype=torch.float32)
+    z = torch.full((T, H, dim), -200.0)                      # softplus and, times any rate, the logarithm 0
+    z[1, 0], z[1, 1] = 20.0 + off, -off                      # decays e^-20 .. e^-83; softplus(0 .. -63)
+    rate = torch.tensor([1.0, 2.0 ** 10])
+    q, v = torch.zeros(T, H, dim), torch.zeros(T, H, dim)
+    k, v[0] = q.clone(), 1.0
+    k[0] = 1.0 if mode == "gla" else dim ** -0.5
+    beta = torch.zeros(T, H)
+    beta[0] = torch.tensor([-27.0, -51.0])
+    rows, runs = _rows([n], 0)
+    state = torch.zeros(2, H, dim, dim)
+    m = lambda x: x.to(DEV)  # noqa: E731
+    out, st = torch.empty(T, H * dim, device=DEV), m(state)
+    ops.gated_linear_recurrence(m(q), m(k), m(v), m(z.view(T, -1)), m(rate), torch.zeros(H * dim, device=DEV), 1.0,
+                                m(beta) if mode == "delta" else None, torch.zeros(T, H * dim, device=DEV), True,
+                                torch.ones(dim, device=DEV), 1e-5, 1.0, st, *(m(r) for r in rows), out,
+                                run_rows=m(torch.tensor([0], dtype=torch.int32)))
+    a = torch.exp(-rate.double()[:, None] * torch.log1p(torch.exp(z[1].double())))
+    want = a * k[0].double() * (torch.sigmoid(beta[0].double())[:, None] if mode == "delta" else 1.0)
+    got = st[1].double().cpu()                               # row_state 0: slot 0, written half 1
+    # a unit in the last place (2^-23) for each of exponential, logarithm and quotient, their products'
+    # roundings; head 1's argument passes its own three on to the exponential, times itself
+    x = rate.double()[:, None] * torch.log1p(torch.exp(z[1].double()))
+    tol = torch.stack([torch.full_like(x[0], 6.0), 6.0 + 4.0 * x[1]]) * 2.0 ** -23
+    seen = want > 1e-30
+    err = ((got - want[:, :, None]).abs() / want[:, :, None])[seen]
+    assert bool(seen[0].any()) and bool(seen[1].any())
+    assert bool((err <= tol[seen][:, None]).all()), float((err / tol[seen][:, None]).max())
+
+
+def test_wkv_decays_and_gates_keep_32_bits():
+    """The same for wkv: e^z is known to a unit or two in its last place, which the decay takes times itself;
+    every value is read alike, so that the norm leaves one and the gate shows."""
+    T, H, N = 40, 2, 64
+    z, zero = torch.full((T, H, N), -200.0), torch.zeros(T, H * N)
+    z[1] = torch.linspace(-4.0, 4.0, H * N).view(H, N)
+    k, v, r = zero.clone(), zero.clone(), zero.clone()
+    k[0], v[0], r[1] = 1.0, 1.0, 1.0
+    gate = torch.linspace(-60.0, 60.0, T * H * N).view(T, -1)
+    rows, runs = _rows([T], 0)
+    st, out = torch.zeros(2, H, N, N, device=DEV), torch.empty(T, H * N, device=DEV)
+    m = lambda x: x.to(DEV)  # noqa: E731
+    ops.wkv_recurrence(m(r), m(k), m(v), m(z.view(T, -1)), m(zero[0]), m(zero[0].view(H, N)), m(gate),
+                       torch.ones(H * N, device=DEV), 0.0, st, *(m(x) for x in rows), out,
+                       run_rows=torch.zeros(1, dtype=torch.int32, device=DEV))
+    x = torch.exp(z[1].double())
+    err = (st[1].double().cpu() * torch.exp(x)[:, :, None] - 1).abs()
+    assert bool((err <= (4 + 3 * x[:, :, None]) * 2.0 ** -23).all()), float((err / (4 + 3 * x[:, :, None])).max() * 2 ** 23)
+    g = gate[1].double()
+    want = g * torch.sigmoid(g)
+    err = (out[1].double().cpu() - want).abs() / want.abs()
+    assert bool((err <= 8 * 2.0 ** -23).all()), float(err.max() * 2 ** 23)      # and the norm's square root and quotient
