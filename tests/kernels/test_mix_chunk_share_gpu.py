@@ -1,0 +1,103 @@
+"""Steps whose runs are shared by their length between the recurrences' kernels: many short runs beside
+longer ones, each kernel's first and last length among them, entries without a run."""
+import pytest
+import torch
+
+from replisense_rfq_amd import ops
+from replisense_rfq_amd.ops import reference as ref
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+# more than two waves' worth of one-row runs, then both sides of every line: 3 and 4 (delta rule, scan),
+# 24 (few workgroups), 40 (gla), 48 (wkv), 80 (delta)
+LENS = [1] * 70 + [24, 3, 4, 23] + [1] * 60 + [39, 40, 41, 200, 47, 48, 79, 80, 81, 2]
+
+
+def _step():
+    g = torch.Generator().manual_seed(1)
+    lens = [LENS[i] for i in torch.randperm(len(LENS), generator=g)]
+    rs, rb, rf, pos, runs = [], [], [], [], []
+    for i, n in enumerate(lens):
+        runs.append(len(rs))
+        rs += [-1 if i % 11 == 10 else 2 * i + i % 2] * n        # some without a state
+        rb += range(n)
+        rf += range(n - 1, -1, -1)
+        pos += range(17 * (i % 3), 17 * (i % 3) + n)
+        if i % 9 == 4:
+            runs.append(-1)                                      # no run
+    i32 = lambda x: torch.tensor(list(x), dtype=torch.int32)  # noqa: E731
+    return lens, [i32(x) for x in (rs, rb, rf, pos)], i32(runs)
+
+
+def _close(got, want, tol):
+    """Row by row: a row that a kernel left out, or finished twice, is one among hundreds."""
+    got, want = got.double().cpu().flatten(1), want.double().flatten(1)
+    size = want.square().mean().sqrt()
+    err = (got - want).abs().amax(1)
+    assert bool((err <= tol * torch.maximum(want.abs().amax(1), size)).all()), (err / size).topk(5)
+
+
+# two heads: chunks from 24 rows on; twenty: more workgroups than that is worth, chunks from 40, 48 or 80 on
+@pytest.mark.parametrize("H", [2, 20])
+@pytest.mark.parametrize("mode", ["gla", "delta"])
+@pytest.mark.parametrize("dim,vdim", [(64, 64), (32, 80)])
+def test_linear_recurrence_of_many_lengths(mode, H, dim, vdim):
+    lens, rows, runs = _step()
+    g, T = torch.Generator().manual_seed(H + dim), sum(lens)
+    r = lambda *s: torch.randn(*s, generator=g)  # noqa: E731
+    q, k = (torch.nn.functional.normalize(r(T, H, dim), dim=-1) for _ in range(2))
+    v, z, gate, rate, zb, nw = r(T, H, vdim), r(T, H * dim) * 2, r(T, H * vdim), torch.rand(H, generator=g) + 0.1, \
+        r(H * dim), r(vdim)
+    beta = r(T, H) if mode == "delta" else None
+    st = r(2 * len(lens), H, dim, vdim) * 0.3
+    m = lambda x: None if x is None else x.to(DEV)  # noqa: E731
+
+    def call(f, to, s, **more):
+        out = to(torch.full((T, H * vdim), 7.0))
+        f(to(q), to(k), to(v), to(z), to(rate), to(zb), 1.0, None if beta is None else to(beta), to(gate), mode == "delta",
+          to(nw), 1e-5, dim ** -0.5, s, *(to(x) for x in rows), out, **more)
+        return out, s
+
+    want, st_w = call(ref.gated_linear_recurrence, lambda x: x, st.clone())
+    got, st_g = call(ops.gated_linear_recurrence, m, m(st), run_rows=m(runs))
+    # the norm divides by a row's own rms, which may be a tenth of the usual: ten times the sums' 1e-5
+    _close(got, want, 1e-4)
+    _close(st_g, st_w, 2e-5)
+
+
+@pytest.mark.parametrize("H", [2, 20])
+def test_wkv_of_many_lengths(H):
+    lens, rows, runs = _step()
+    g, T, N = torch.Generator().manual_seed(H), sum(lens), 64
+    x = [torch.randn(T, H * N, generator=g) for _ in range(5)]
+    w0, u, nw = torch.randn(H * N, generator=g) - 2, torch.randn(H, N, generator=g), torch.randn(H * N, generator=g)
+    st = torch.randn(2 * len(lens), H, N, N, generator=g) * 0.3
+
+    def call(f, to, s, **more):
+        out = to(torch.full((T, H * N), 7.0))
+        f(*(to(t) for t in x[:4]), to(w0), to(u), to(x[4]), to(nw), 1e-5, s, *(to(t) for t in rows), out, **more)
+        return out, s
+
+    want, st_w = call(ref.wkv_recurrence, lambda t: t, st.clone())
+    got, st_g = call(ops.wkv_recurrence, lambda t: t.to(DEV), st.to(DEV), run_rows=runs.to(DEV))
+    _close(got, want, 1e-4)
+    _close(st_g, st_w, 2e-5)
+
+
+def test_a_list_of_runs_changes_nothing():
+    """64 heads, two runs of 2,048 and short ones: with the list in chunks, without it token by token."""
+    H, N, lens = 64, 64, [2048, 1, 1, 2048, 1]
+    g, T = torch.Generator().manual_seed(2), sum(lens)
+    x = [(torch.randn(T, H * N, generator=g) * 0.5).to(DEV) for _ in range(5)]
+    w0, u, nw = (torch.randn(H * N, generator=g) - 2).to(DEV), torch.randn(H, N, generator=g).to(DEV), torch.ones(H * N, device=DEV)
+    i32 = lambda t: torch.tensor(t, dtype=torch.int32, device=DEV)  # noqa: E731
+    rows = [i32([2 * i for i, n in enumerate(lens) for _ in range(n)]), i32([j for n in lens for j in range(n)]),
+            i32([n - 1 - j for n in lens for j in range(n)]), i32([j for n in lens for j in range(n)])]
+    first = i32([sum(lens[:i]) for i in range(len(lens))])
+    res = []
+    for runs in (first, None):
+        st, out = torch.zeros(10, H, N, N, device=DEV), torch.empty(T, H * N, device=DEV)
+        ops.wkv_recurrence(*x[:4], w0, u, x[4], nw, 1e-5, st, *rows, out, run_rows=runs)
+        res.append((out.cpu(), st.cpu()))
+    _close(res[0][0], res[1][0], 1e-4)
+    _close(res[0][1], res[1][1], 2e-5)
