@@ -62,6 +62,23 @@ __device__ __forceinline__ void st4(bf16_t* p, float4 v) {
   *reinterpret_cast<uint2*>(p) = u.w;
 }
 
+// exp(x) for x <= 87, to about a unit in the last place: v_exp_f32 takes base 2, and the product's rounding,
+// which grows with |x|, and the rest of log2 e follow as a factor near one.  Below e^-200: 0.  NaN stays NaN.
+__device__ __forceinline__ float exp_c(float x) {
+  x = x < -200.f ? -200.f : x;
+  const float t = x * 1.44269502f, e = __builtin_amdgcn_exp2f(t);
+  const float rest = fmaf(x, 1.92596299e-8f, fmaf(x, 1.44269502f, -t));
+  return fmaf(e * 0.693147181f, rest, e);
+}
+// log(1 + e^y): log(1 + e) = 2 atanh(e / (2 + e)), the odd series fitted to a relative error of 5e-9
+__device__ __forceinline__ float softplus_c(float y) {
+  const float e = exp_c(-fabsf(y)), d = 2.f + e, r = __builtin_amdgcn_rcpf(d), s0 = e * r;
+  const float s = fmaf(fmaf(-s0, d, e), r, s0), u = s * s;
+  const float p = fmaf(fmaf(fmaf(0.140123978f, u, 0.139995337f), u, 0.200108513f), u, 0.333332062f);
+  return fmaf(2.f, fmaf(s * u, p, s), fmaxf(y, 0.f));
+}
+__device__ __forceinline__ float sigmoid_c(float x) { return 1.0f / (1.0f + exp_c(x < -87.f ? 87.f : -x)); }
+
 // Block-wide sum for blockDim.x a multiple of 64, at most 1024.  scratch >= 16 floats.
 __device__ __forceinline__ float block_sum(float v, float* scratch) {
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;

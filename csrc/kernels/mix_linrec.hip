@@ -30,10 +30,6 @@
 
 namespace rfqmix {
 
-__device__ __forceinline__ float softplus_f(float y) {
-  return fmaxf(y, 0.f) + log1pf(expf(-fabsf(y)));
-}
-
 template <typename TI, typename TG, int NR, bool DELTA>
 __global__ __launch_bounds__(256) void gated_linrec_kernel(
     const TI* __restrict__ q, const TI* __restrict__ k, const TI* __restrict__ v,
@@ -83,7 +79,7 @@ __global__ __launch_bounds__(256) void gated_linrec_kernel(
     nq = ldf(q + (int64_t)t0 * q_stride + qc);
     nk = ldf(k + (int64_t)t0 * k_stride + qc);
     na = z[(int64_t)t0 * z_stride + zc];
-    na = expf(-my_rate * softplus_f(zsign * (na + my_zb)));
+    na = exp_c(-my_rate * softplus_c(zsign * (na + my_zb)));
   }
   if (vlive) {
     nv = ldf(v + (int64_t)t0 * v_stride + vc);
@@ -95,7 +91,7 @@ __global__ __launch_bounds__(256) void gated_linrec_kernel(
     const float4* cur = ops + (a & 1) * dim;
     if (klive) ops[(a & 1) * dim + j] = make_float4(nq, nk, na, 0.f);
     const float vj = nv, gj = ng;
-    const float bj = DELTA ? 1.0f / (1.0f + expf(-nb)) : 1.f;
+    const float bj = DELTA ? sigmoid_c(nb) : 1.f;
     __syncthreads();
     if (a + 1 < n) {                   // the next token's operands, in flight during the sums
       const int64_t t = t0 + a + 1;
@@ -173,7 +169,7 @@ __global__ __launch_bounds__(256) void gated_linrec_kernel(
       }
       o *= q_scale;
     }
-    if (a + 1 < n && klive) na = expf(-my_rate * softplus_f(zsign * (na + my_zb)));
+    if (a + 1 < n && klive) na = exp_c(-my_rate * softplus_c(zsign * (na + my_zb)));
     if (raw != nullptr) {              // long steps: norm and gate follow in a row-parallel kernel
       if (vlive) raw[(int64_t)(t0 + a) * H * vdim + vc] = o;
       continue;
@@ -359,17 +355,17 @@ __global__ __launch_bounds__(256) void gated_linrec_scan_kernel(
       if (x < SCAN_ROWS * P4 && r < rows) {
         float* o = ops + r * RS + c;
         float4 d = ra[u];
-        d.x = expf(-my_rate * softplus_f(zsign * (d.x + zb[u].x)));
-        d.y = expf(-my_rate * softplus_f(zsign * (d.y + zb[u].y)));
-        d.z = expf(-my_rate * softplus_f(zsign * (d.z + zb[u].z)));
-        d.w = expf(-my_rate * softplus_f(zsign * (d.w + zb[u].w)));
+        d.x = exp_c(-my_rate * softplus_c(zsign * (d.x + zb[u].x)));
+        d.y = exp_c(-my_rate * softplus_c(zsign * (d.y + zb[u].y)));
+        d.z = exp_c(-my_rate * softplus_c(zsign * (d.z + zb[u].z)));
+        d.w = exp_c(-my_rate * softplus_c(zsign * (d.w + zb[u].w)));
         *reinterpret_cast<float4*>(o) = d;
         *reinterpret_cast<float4*>(o + NR) = rk[u];
         *reinterpret_cast<float4*>(o + 2 * NR) = rq[u];
       }
     }
     if ((tid >> 4) < rows) *reinterpret_cast<float4*>(ops + (tid >> 4) * RS + 3 * NR + (tid & 15) * 4) = rv;
-    if (DELTA && tid < rows) bet[tid] = 1.0f / (1.0f + expf(-rb));
+    if (DELTA && tid < rows) bet[tid] = sigmoid_c(rb);
     __syncthreads();
     if (a0 + SCAN_ROWS < n) fetch(a0 + SCAN_ROWS);     // in flight during the sums
     float4 ca[NK / 4], ck[NK / 4], cq[NK / 4];         // a token's operands, read one token ahead
@@ -515,7 +511,7 @@ void launch_gated_linrec(bool in_f32, bool act_f32, bool delta, const LinrecArgs
     // Below them: the scan's fixed cost is the larger one (64 decode rows, gla: 41 us against 72),
     // its tokens are the cheaper ones where each has two sums (delta, 64 runs of 8: 106 us against
     // 177; gla 89 against 82).
-    if (a.run_rows != nullptr && a.dim <= kChunkDim) 
+    if (a.run_rows != nullptr && a.dim <= kChunkDim)
       above = delta && a.T > 2 * a.runs ? std::min(3, a.below - 1) : a.below - 1;
   }
 #define LINREC_GO(TI, TG)                                              \

@@ -134,11 +134,13 @@ def test_wkv_non_finite_value_stays_out_of_earlier_tokens():
     _close(out[sum(LENS[:8]):], out_w[sum(LENS[:8]):], 1e-5)
 
 
+# 40 rows: chunks; 6: token by token; 200 without a list of runs: the scan
+@pytest.mark.parametrize("n", [40, 6, 200])
 @pytest.mark.parametrize("mode", ["gla", "delta"])
-def test_decays_and_steps_keep_32_bits(mode):
+def test_decays_and_steps_keep_32_bits(mode, n):
     """One write, one decay, no reads: the state is beta_0 a_0 and known to a few units in the last place.
     Arguments of the exponentials are whole numbers, or a tiny softplus times a rate that fp32 holds."""
-    dim, H, n = 64, 2, 40
+    dim, H = 64, 2
     T, off = n, torch.arange(dim, dtype=torch.float32)
     z = torch.full((T, H, dim), -200.0)                      # softplus and, times any rate, the logarithm 0
     z[1, 0], z[1, 1] = 20.0 + off, -off                      # decays e^-20 .. e^-83; softplus(0 .. -63)
@@ -155,7 +157,7 @@ def test_decays_and_steps_keep_32_bits(mode):
     ops.gated_linear_recurrence(m(q), m(k), m(v), m(z.view(T, -1)), m(rate), torch.zeros(H * dim, device=DEV), 1.0,
                                 m(beta) if mode == "delta" else None, torch.zeros(T, H * dim, device=DEV), True,
                                 torch.ones(dim, device=DEV), 1e-5, 1.0, st, *(m(r) for r in rows), out,
-                                run_rows=m(torch.tensor([0], dtype=torch.int32)))
+                                run_rows=m(torch.tensor([0], dtype=torch.int32)) if n < 200 else None)
     a = torch.exp(-rate.double()[:, None] * torch.log1p(torch.exp(z[1].double())))
     want = a * k[0].double() * (torch.sigmoid(beta[0].double())[:, None] if mode == "delta" else 1.0)
     got = st[1].double().cpu()                               # row_state 0: slot 0, written half 1
