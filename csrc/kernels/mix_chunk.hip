@@ -126,30 +126,11 @@ __device__ __forceinline__ void lower_product(const float* m, const f32x4& x, in
 }
 }  // namespace
 
+// 64 value channels, from z64 on, of head h of the run that begins at row t0.
 template <typename TI, typename TG, int MODE>
-__global__ __launch_bounds__(chunk_threads(MODE)) void chunk_recurrence_kernel(const ChunkArgs a) {
+__device__ __forceinline__ void chunk_run(const ChunkArgs& a, const int t0, const int h, const int z64, const int tid) {
   constexpr bool WKV = MODE == kChunkWkv, DELTA = MODE == kChunkDelta;
-  const int h = blockIdx.y;
-  const int tid = threadIdx.x, lane = tid & 63, col = lane & 15, grp = lane >> 4;
-  int t0 = -1;
-  if (a.min_run <= 1) {
-    t0 = a.run_rows[blockIdx.x];
-  } else {                     // the step's runs of min_run rows or more, counted by every wave for itself
-    int left = blockIdx.x;
-    for (int base = 0; base < a.runs; base += 64) {
-      const int r = base + lane < a.runs ? a.run_rows[base + lane] : -1;
-      const bool fits = r >= 0 && a.row_back[r] == 0 && a.row_fwd[r] + 1 >= a.min_run;
-      uint64_t m = __builtin_amdgcn_ballot_w64(fits);
-      const int c = __builtin_popcountll(m);
-      if (left < c) {
-        for (; left > 0; --left) m &= m - 1;
-        t0 = __builtin_amdgcn_readfirstlane(__shfl(r, __builtin_ctzll(m), 64));
-        break;
-      }
-      left -= c;
-    }
-  }
-  if (t0 < 0 || a.row_back[t0] != 0) return;
+  const int lane = tid & 63, col = lane & 15, grp = lane >> 4;
   const int n = a.row_fwd[t0] + 1, nc = (n + CT - 1) / CT;
   const int code = a.row_state[t0];
   const int H = a.H, dim = a.dim, vdim = a.vdim;
@@ -172,7 +153,7 @@ __global__ __launch_bounds__(chunk_threads(MODE)) void chunk_recurrence_kernel(c
     for (int i = 0; i < 4; ++i) o[i] = (uint32_t)min(first + i, n - 1 - c * CT) * (uint32_t)(stride * esz);
   };
   // ---- consumers: 16 value channels, S[16 i + 4 grp + r][column]
-  const int vcol = (int)blockIdx.z * 64 + 16 * w + col;
+  const int vcol = z64 + 16 * w + col;
   const bool vlive = vcol < vdim;
   const bool from_state = code >= 0 && a.pos[t0] > 0;
   const int64_t hsz = (int64_t)dim * vdim;
@@ -604,41 +585,88 @@ do {                                                                            
   }
 }
 
+// A workgroup per entry of the list, head and 64 value channels.
+template <typename TI, typename TG, int MODE>
+__global__ __launch_bounds__(chunk_threads(MODE)) void chunk_recurrence_kernel(const ChunkArgs a) {
+  const int t0 = a.run_rows[blockIdx.x];
+  if (t0 >= 0 && a.row_back[t0] == 0) chunk_run<TI, TG, MODE>(a, t0, blockIdx.y, blockIdx.z * 64, threadIdx.x);
+}
+
+// Workgroups, one to a CU at most, that share the runs of min_run rows or more, which every wave counts for
+// itself: one for every run that the step has room for costs 16 us where there is none (64 runs of 16, wkv).
+template <typename TI, typename TG, int MODE>
+__global__ __launch_bounds__(chunk_threads(MODE)) void chunk_recurrence_share_kernel(const ChunkArgs a) {
+  const int lane = threadIdx.x & 63, cols = (a.vdim + 63) >> 6, per = a.H * cols;
+#pragma unroll 1
+  for (int item = blockIdx.x;; item += gridDim.x) {
+    int left = item / per, t0 = -1;
+    const int part = item - left * per, z = part / a.H;
+    for (int base = 0; base < a.runs; base += 64) {
+      const int r = base + lane < a.runs ? a.run_rows[base + lane] : -1;
+      const bool fits = r >= 0 && a.row_back[r] == 0 && a.row_fwd[r] + 1 >= a.min_run;
+      uint64_t m = __builtin_amdgcn_ballot_w64(fits);
+      const int c = __builtin_popcountll(m);
+      if (left < c) {
+        for (; left > 0; --left) m &= m - 1;
+        t0 = __builtin_amdgcn_readfirstlane(__shfl(r, __builtin_ctzll(m), 64));
+        break;
+      }
+      left -= c;
+    }
+    if (t0 < 0) return;
+    // The last barrier of a run lies behind every wave's last read of LDS: the next run's first writes need no
+    // other.
+    // thread and arguments are taken anew for every run: what the compiler derives from them would stay in
+    // registers over the loop, 55 of them spilled
+    typedef const __attribute__((address_space(4))) ChunkArgs const_args;
+    const_args* p = (const_args*)__builtin_amdgcn_kernarg_segment_ptr();
+    int tid = threadIdx.x;
+    asm volatile("" : "+v"(tid), "+s"(p));
+    chunk_run<TI, TG, MODE>(*(const ChunkArgs*)p, t0, part - z * a.H, z * 64, tid);
+  }
+}
+
 // ------------------------------------------------------------------ launcher
-// A workgroup costs some 9 us before its first chunk is out and 1.4 - 2 us a chunk, one to a CU; the
-// token-by-token kernels some 6 us and 0.2 (64 runs) - 2.6 us a token, many to a CU.  Two rounds of
-// workgroups or fewer: chunks from 8 rows a run on (wkv, one run: 8 rows 21 us against 37; the
-// others have a launch more, they gain from 24 on: delta 16 rows 73 us against 67, 40 rows 72
-// against 129).  More rounds: no gain below some 24 (wkv, 64 runs of 16:
-// 145 us against 130, of 32: 189 against 201) or 40 rows (delta, 64 runs of 32: 261 against 212), so the
-// runs of a step, decode rows beside prompts as a rule, are shared by their length (wkv, 64 decode
-// rows beside a prompt of 200: 102 us, one kernel for all of them 594).
+// A workgroup costs some 8 us before its first chunk is out and 1.4 - 2.3 us a chunk, one to a CU; the
+// token-by-token kernels some 6 us and 0.2 (64 runs) - 2.6 us a token, many to a CU.  Times below are of whole
+// steps, 32 heads of 64 x 128 (wkv: 64 of 64 x 64), chunks against tokens.
+// Two workgroups to a CU or fewer: everything in chunks from 8 rows a run on (one run of 8: gla 14 us against 25,
+// delta 14 against 28, wkv 8 against 24).
+// More: a step's runs, decode rows beside prompts as a rule, are shared by their length (64 decode rows beside
+// a prompt of 200: gla 59 us, wkv 52, tokens alone 123 and 515), from 24 rows where the step has room for no
+// more than 2,048 workgroups of such runs, delta rule 512 (16 runs of 24: gla 47 against 74, wkv 40 against 73,
+// delta 55 against 46).  Beyond that the CUs' rounds add up: from 48 for wkv (64 runs of 41: 180 against 162, of
+// 64: 210 against 247), 40 for gla (205 against 201, of 64: 235 against 345), 24 with up to 64 value channels
+// (64 runs of 24: 83 against 98), 80 for the delta rule (64 runs of 64: 282 against 249, of 96: 358 against 387).
 int chunk_min_run(int mode, int T, const ChunkArgs& a) {
   constexpr int kNever = INT32_MAX;
-  const int kLong = mode == kChunkWkv ? 24 : 40;
   if (a.run_rows == nullptr || a.dim > NC || (mode == kChunkWkv && (a.dim != NC || a.vdim != NC))) return kNever;
   for (int64_t st : {a.qs, a.ks, a.vs, a.zs})             // a chunk's rows in 32-bit byte offsets
     if (st < 0 || st >= (1ll << 24)) return kNever;
-  const int64_t groups = (int64_t)a.runs * a.H * ((a.vdim + 63) / 64);
-  if (groups <= 512 && T >= (mode == kChunkWkv ? 8 : 24) * a.runs) return 1;
-  return T - a.runs + 1 >= kLong ? kLong : kNever;        // no run can be longer than that
+  const int64_t per = (int64_t)a.H * ((a.vdim + 63) / 64);
+  if (a.runs * per <= 512 && T >= 8 * a.runs) return 1;
+  const int few = 24, many = mode == kChunkWkv ? 48 : mode == kChunkDelta ? 80 : a.vdim > 64 ? 40 : 24;
+  const int from = std::min(a.runs, T / few) * per <= (mode == kChunkDelta ? 512 : 2048) ? few : many;
+  return T - a.runs + 1 >= from ? from : kNever;          // no run can be longer than that
 }
 
 template <typename TI, typename TG, int MODE>
 static void launch_chunk_one(int T, const ChunkArgs& a, hipStream_t s) {
   static bool attr = false;
   if (!attr) {          // dynamic LDS above 64 KB has to be allowed per kernel, once
-    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&chunk_recurrence_kernel<TI, TG, MODE>),
-                              hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+    for (auto* k : {&chunk_recurrence_kernel<TI, TG, MODE>, &chunk_recurrence_share_kernel<TI, TG, MODE>})
+      (void)hipFuncSetAttribute(reinterpret_cast<const void*>(k), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
     attr = true;
   }
   static_assert(sizeof(ChunkLds<MODE>) <= 160 * 1024, "LDS of a CU");
-  // No more long runs than rows allow.  An odd number: workgroups go to the eight XCDs in turn, and
-  // those of the first few runs are all that work (64 decode rows beside a prompt of 600, wkv: 198 us
-  // with 8 columns, all of them on one XCD, 145 with 13).
-  const int gx = a.min_run <= 1 ? a.runs : std::min(a.runs, T / a.min_run) | 1;
-  hipLaunchKernelGGL((chunk_recurrence_kernel<TI, TG, MODE>),
-                     dim3(gx, a.H, (a.vdim + 63) / 64), dim3(chunk_threads(MODE)), sizeof(ChunkLds<MODE>), s, a);
+  const int cols = (a.vdim + 63) / 64;
+  if (a.min_run <= 1)
+    hipLaunchKernelGGL((chunk_recurrence_kernel<TI, TG, MODE>), dim3(a.runs, a.H, cols), dim3(chunk_threads(MODE)),
+                       sizeof(ChunkLds<MODE>), s, a);
+  else                        // no more long runs than rows allow
+    hipLaunchKernelGGL((chunk_recurrence_share_kernel<TI, TG, MODE>),
+                       dim3((unsigned)std::min<int64_t>((int64_t)std::min(a.runs, T / a.min_run) * a.H * cols, 256)),
+                       dim3(chunk_threads(MODE)), sizeof(ChunkLds<MODE>), s, a);
 }
 
 void launch_chunk(int mode, bool in_f32, bool act_f32, int T, const ChunkArgs& a, hipStream_t s) {

@@ -512,7 +512,7 @@ void launch_gated_linrec(bool in_f32, bool act_f32, bool delta, const LinrecArgs
     // its tokens are the cheaper ones where each has two sums (delta, 64 runs of 8: 106 us against
     // 177; gla 89 against 82).
     if (a.run_rows != nullptr && a.dim <= kChunkDim)
-      above = delta && a.T > 2 * a.runs ? std::min(3, a.below - 1) : a.below - 1;
+      above = delta && a.T > std::max(2 * a.runs, 128) ? std::min(3, a.below - 1) : a.below - 1;
   }
 #define LINREC_GO(TI, TG)                                              \
   do {                                                                 \

@@ -1381,7 +1381,7 @@ def conv_act_heads(x, w, state, row_state, row_back, row_fwd, positions, n_unit:
 
 LINREC_SCAN_ROWS = 128      # steps with more rows leave norm and gate to a row-parallel kernel
 CHUNK_DIM = 64              # most key channels of the chunked recurrences (csrc/kernels/mix_chunk.hip)
-CHUNK_RUN = 40              # steps that can hold a run of that many rows may use them
+CHUNK_RUN = 24              # steps that can hold a run of that many rows may use them
 
 
 def gated_linear_recurrence(q, k, v, z, rate, zbias, zsign: float, beta, gate, gate_sigmoid: bool,
@@ -1395,7 +1395,7 @@ def gated_linear_recurrence(q, k, v, z, rate, zbias, zsign: float, beta, gate, g
     if _gpu(q):
         T, runs = q.shape[0], -1 if run_rows is None else run_rows.numel()
         raw = None
-        if T > LINREC_SCAN_ROWS and T != runs or T >= 24 * runs > 0 and state.shape[2] <= CHUNK_DIM or \
+        if T > LINREC_SCAN_ROWS and T != runs or T >= 8 * runs > 0 and state.shape[2] <= CHUNK_DIM or \
                 runs >= 0 and state.shape[2] <= CHUNK_DIM and T - runs + 1 >= CHUNK_RUN:
             raw = torch.empty(out.shape, dtype=torch.float32, device=out.device)
         _native.mix_ops().gated_linear_recurrence(
