@@ -90,8 +90,9 @@ int launch_attn_keep_decode(bool, const float*, const void*, const void*, int64_
                             int, bool, int, int, int, int, int, float, float, hipStream_t);
 bool keep_mfma_ok(int, int, int, bool);
 void launch_attn_keep_split(const float*, const void*, const void*, int64_t, const int32_t*, int, const int32_t*,
-                            const int32_t*, const int32_t*, int, int, const float*, const void*, int64_t, int, void*,
-                            int64_t, float, int, int, bool, int, int, int, int, bool, float, float, hipStream_t);
+                            const int32_t*, const int32_t*, int, int, int, const float*, const void*, int64_t, int,
+                            void*, int64_t, float, int, int, bool, int, int, int, int, bool, float, float,
+                            hipStream_t);
 bool launch_attn_keep_mfma(const float*, const void*, const void*, int64_t, const int32_t*, int,
                            const int32_t*, const int32_t*, const int32_t*, const int32_t*,
                            const int32_t*, int, const float*, const void*, int64_t, int, void*,
@@ -842,7 +843,7 @@ void attn_keep_window(const Tensor& q, const Tensor& k_cache, const Tensor& v_ca
     return rfqmix::launch_attn_keep_split(
         f32p(q, "q"), k_cache.data_ptr(), v_cache.data_ptr(), vrs, i32p(bt, "block_tables", 0),
         (int)bt.size(1), i32p(q_start, "q_start", NB), i32p(q_len, "q_len", NB), i32p(kv_len, "kv_len", NB),
-        NB, (int)short_rows, hb, gp, gs, gw, out.data_ptr(), out.stride(0), (float)scale, (int)window,
+        T, NB, (int)short_rows, hb, gp, gs, gw, out.data_ptr(), out.stride(0), (float)scale, (int)window,
         (int)keep_first, sigmoid, H, G, E, (int)vdim, shared, (float)softcap, (float)out_mult, stream());
   }
   if (short_rows > 0) {

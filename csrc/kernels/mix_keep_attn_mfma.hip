@@ -29,6 +29,8 @@
 // 64 heads and a window 268 -> 174 us.  What is left of the first is the longest block's chain of 64
 // pages.  32 x 32 tiles, a wave per 32 queries, took 217 and 116 us there and lost 20 % on prompts of a
 // few hundred tokens; two waves sharing such a wave's pages 251 and 119.
+#include <algorithm>
+
 #include "common.h"
 #include "mix_common.h"
 
@@ -348,39 +350,47 @@ __global__ __launch_bounds__(128 * HPW, HPW == 2 ? 3 : 1) void attn_keep_mfma_ke
 // One prompt of 2,048 over 576 (32 heads) took 904 us a pass on the kernel above, 420 here; four of
 // them with 64 heads 3,249 and 1,402.  Pages come by LDS-DMA, the next one during this one; their rows lie unpadded, 16-byte pieces
 // permuted inside each 128 bytes by wide_swizzle(row).
+// DEC: decode rows.  A wave's columns are 16 heads of one row, so that a workgroup reads a page once for up to
+// 128 heads; the pages come one after another, which pays once every CU has a workgroup (launch_split_waves).
+// 256 sequences of 300 tokens with 64 heads of 576 entries 44 us, 32 of 500 with four rows each 50; split over
+// waves 116 and 129.
 // Sixteen rows of one piece (a K read) and four neighbouring rows of a pair of pieces beside the next
 // four (a transposed V read) then lie on different banks: the row's parity picks a half of them, bits
 // 1 and 2 the pair, bit 3 the order inside it.
 __device__ __forceinline__ int wide_swizzle(int r) { return ((r >> 1) & 1) << 2 | ((r >> 2) & 1) << 1 | ((r >> 3) & 1); }
 
-template <int DK, int DV, int HPW, int MODE>
-__global__ __launch_bounds__(128 * HPW, 2) void attn_keep_wide_kernel(const KeepArgs a) {
+template <int DK, int DV, int HPW, int MODE, bool DEC>
+__global__ __launch_bounds__(128 * HPW, DEC && HPW == 1 ? 1 : 2) void attn_keep_wide_kernel(const KeepArgs a) {
   constexpr int E = 32 * DK, vdim = 16 * DV, NWV = 2 * HPW, NP = WBS * E / 512, ND = (NP + NWV - 1) / NWV;
   constexpr bool QLO = DK <= 10;
   static_assert(E % 64 == 0 && DV % 4 == 0, "whole 128-byte lines");
   const int item = gridDim.x - 1 - blockIdx.x;     // a sequence's later blocks see the most keys: they start first
-  const int s = a.work_seq[item];
+  const int s = DEC ? item : a.work_seq[item];
   if (s < 0) return;
   const int ql = a.q_len[s];
-  const int i0 = a.work_qblk[item] * WQB;
+  const int i0 = DEC ? 0 : a.work_qblk[item] * WQB;
   if (i0 >= ql) return;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int col = lane & 15, grp = lane >> 4;
-  const int rep = a.H / a.G, per = (rep + HPW - 1) / HPW;     // workgroups of a key head, the last partly idle
-  const int g = (int)blockIdx.y / per, hd = ((int)blockIdx.y - g * per) * HPW + (wid >> 1);
+  constexpr int HW = DEC ? 16 * NWV : HPW;                    // heads of a workgroup
+  const int rep = a.H / a.G, per = (rep + HW - 1) / HW;       // workgroups of a key head, the last partly idle
+  const int g = (int)blockIdx.y / per, h0 = ((int)blockIdx.y - g * per) * HW;
+  const int hd = DEC ? h0 + wid * 16 + col : h0 + (wid >> 1);
+  const bool idle = DEC && h0 + wid * 16 >= rep;             // a wave that only copies pages
   const int hh = g * rep + min(hd, rep - 1);                 // past the last head: it once more, not stored
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   short* const pages = reinterpret_cast<short*>(smem);       // two of them
 
-  const int nq = min(WQB, ql - i0);
-  const int p0 = a.kv_len[s] - ql + i0, plast = p0 + nq - 1;
+  for (int r = DEC ? (int)blockIdx.z : 0; r < (DEC ? ql : 1); r += DEC ? (int)gridDim.z : 1) {
+  const int nq = DEC ? 1 : min(WQB, ql - i0);
+  const int p0 = a.kv_len[s] - ql + (DEC ? r : i0), plast = p0 + nq - 1;
   const int window = a.window, keep_first = a.keep_first;
   const int jwin = window > 0 ? max(0, p0 - window + 1) : 0;
   const int kf = window > 0 ? min(keep_first, jwin) : 0;
-  const int row = (wid & 1) * 16 + col, pi = p0 + row;       // this lane's query
+  const int row = DEC ? 0 : (wid & 1) * 16 + col, pi = p0 + row;       // this lane's query
   const bool qlive = row < nq && hd < rep;
-  const int64_t t = a.q_start[s] + i0 + (qlive ? row : 0);
+  const int64_t t = a.q_start[s] + (DEC ? r : i0) + (qlive ? row : 0);
   typedef const __attribute__((address_space(4))) int32_t const_i32;
   const_i32* bt = (const_i32*)(uintptr_t)(a.bt + (int64_t)s * a.maxb);
 
@@ -434,6 +444,12 @@ __global__ __launch_bounds__(128 * HPW, 2) void attn_keep_wide_kernel(const Keep
         *reinterpret_cast<s16x8*>(pages + buf * WBS * E + x * 8) = (s16x8){0, 0, 0, 0, 0, 0, 0, 0};
       __syncthreads();
     }
+    if (DEC && jb < jwin && jb + WBS > kf) {                 // out of the row's sight: may hold infinities
+      const int end = min(jwin - jb, WBS) * (E / 8);
+      for (int x = max(0, kf - jb) * (E / 8) + tid; x < end; x += 64 * NWV)
+        *reinterpret_cast<s16x8*>(pages + buf * WBS * E + x * 8) = (s16x8){0, 0, 0, 0, 0, 0, 0, 0};
+      __syncthreads();
+    }
   };
   // keys: row col (+ 16), entries 32 ks + 8 grp ..; values, transposed: rows 4 grp + col / 4 (+ 16),
   // channels 16 m + 4 (col % 4) ..
@@ -475,6 +491,11 @@ __global__ __launch_bounds__(128 * HPW, 2) void attn_keep_wide_kernel(const Keep
     landed(jb, buf);
     if (pn <= pg_last) fetch(ahead, buf ^ 1);
     ahead = bt[min(next_page(pn), pg_last)];
+    if (idle) {
+      pg = pn;
+      buf ^= 1;
+      continue;
+    }
     const short* P = pages + buf * WBS * E;
     f32x4 sc[2][2];                                          // two chains per half page
 #pragma unroll
@@ -533,6 +554,8 @@ __global__ __launch_bounds__(128 * HPW, 2) void attn_keep_wide_kernel(const Keep
     buf ^= 1;
   }
   store_rows<DV, MODE>(a, o, lrun, t, hh, grp, qlive);
+  if constexpr (DEC) __syncthreads();                        // the next row's pages take this one's places
+  }
 }
 
 // ------------------------------------------------------------------ launcher
@@ -564,7 +587,7 @@ static void launch_keep_mfma_one(const KeepArgs& a) {
     const int rep = a.H / a.G;
     hipLaunchKernelGGL(kernel, dim3(a.W, a.G * ((rep + HPW - 1) / HPW)), dim3(threads), lds, a.s, a);
   };
-  if constexpr (WIDE) run(&attn_keep_wide_kernel<DK, DV, HPW, MODE>, 128 * HPW);
+  if constexpr (WIDE) run(&attn_keep_wide_kernel<DK, DV, HPW, MODE, false>, 128 * HPW);
   else run(&attn_keep_mfma_kernel<DK, DV, HPW, SHARED, MODE>, 128 * HPW);
 }
 
@@ -587,6 +610,52 @@ static void launch_keep_mfma_heads(const KeepArgs& a) {
   if (rep % 4 == 0 || (WIDE && rep % 2 == 1 && rep > 1)) launch_keep_mfma_mode<DK, DV, 4, SHARED>(a);
   else if (rep % 2 == 0) launch_keep_mfma_mode<DK, DV, 2, SHARED>(a);
   else launch_keep_mfma_mode<DK, DV, 1, SHARED>(a);
+}
+
+template <int DK, int DV, int HPW, int MODE>
+static void launch_keep_rows_one(const KeepArgs& a, int NA, int rows) {
+  constexpr size_t lds = (size_t)2 * WBS * 32 * DK * sizeof(short);
+  static bool attr = false;
+  if (!attr) {
+    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&attn_keep_wide_kernel<DK, DV, HPW, MODE, true>),
+                              hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+    attr = true;
+  }
+  const int per = (a.H / a.G + 32 * HPW - 1) / (32 * HPW);
+  hipLaunchKernelGGL((attn_keep_wide_kernel<DK, DV, HPW, MODE, true>), dim3(NA, a.G * per, rows), dim3(128 * HPW), lds,
+                     a.s, a);
+}
+
+template <int DK, int DV, int HPW>
+static void launch_keep_rows_mode(const KeepArgs& a, int NA, int rows) {
+  const bool cap = a.softcap > 0.f;
+  if (a.sigmoid && cap) launch_keep_rows_one<DK, DV, HPW, 3>(a, NA, rows);
+  else if (a.sigmoid) launch_keep_rows_one<DK, DV, HPW, 2>(a, NA, rows);
+  else if (cap) launch_keep_rows_one<DK, DV, HPW, 1>(a, NA, rows);
+  else launch_keep_rows_one<DK, DV, HPW, 0>(a, NA, rows);
+}
+
+void launch_attn_keep_wide_rows(const float* q, const void* k_cache, int64_t vrs, const int32_t* bt, int maxb,
+                                const int32_t* q_start, const int32_t* q_len, const int32_t* kv_len, int T, int NA,
+                                const float* head_bias, const void* gate, int64_t gate_stride, int gate_w, void* out,
+                                int64_t out_stride, float scale, int window, int keep_first, bool sigmoid, int H, int G,
+                                int E, float softcap, float out_mult, hipStream_t s) {
+  const KeepArgs a{q, k_cache, k_cache, vrs, bt, maxb, q_start, q_len, kv_len, nullptr, nullptr,
+                   0, head_bias, gate, gate_stride, gate_w, out, out_stride, scale, window, keep_first,
+                   sigmoid, H, G, softcap, out_mult, s};
+  // Rows side by side: as many as the sequences have on the average, or four, the others follow.  Heads: as
+  // few a workgroup as leave no more workgroups than fit the chip, two to a CU.
+  const int rep = H / G, rows = std::min(std::max((T + NA - 1) / NA, 4), T);
+  auto wgs = [&](int heads) { return (int64_t)T * G * ((rep + heads - 1) / heads); };
+#define ROWS_GO(dk, dv)                                                                        \
+  do {                                                                                         \
+    if (rep <= 32 || wgs(32) <= 512) launch_keep_rows_mode<dk, dv, 1>(a, NA, rows);            \
+    else if (rep <= 64 || wgs(64) <= 512) launch_keep_rows_mode<dk, dv, 2>(a, NA, rows);       \
+    else launch_keep_rows_mode<dk, dv, 4>(a, NA, rows);                                        \
+  } while (0)
+  if (E == 576) ROWS_GO(18, 32);
+  else ROWS_GO(10, 16);
+#undef ROWS_GO
 }
 
 bool launch_attn_keep_mfma(const float* q, const void* k_cache, const void* v_cache, int64_t vrs,

@@ -90,15 +90,19 @@ constexpr int stage_row() { return SHARED ? 32 * DK + 8 : 16 * DV + 8; }      //
 template <int DK, bool EXACT>
 constexpr int query_parts() { return EXACT ? 3 : DK <= 10 ? 2 : 1; }
 // the partial results meet in as many passes: beside three parts of a wide latent's queries one is too large
-template <int DV, bool EXACT>
+template <int DV, int NW, bool EXACT>
 constexpr int merge_passes() { return EXACT && DV > 16 ? 2 : 1; }
 // a wave's LDS: its staged page, later a pass of its 16 x vdim partial results (4 floats between rows)
-template <int DK, int DV, bool SHARED, bool EXACT>
+template <int DK, int DV, bool SHARED, int NW, bool EXACT>
 constexpr int wave_lds() {
   return std::max(turn_keys<DK, SHARED>() * stage_row<DK, DV, SHARED>() * 2,
-                  16 * (16 * DV / merge_passes<DV, EXACT>() + 4) * 4);
+                  16 * (16 * DV / merge_passes<DV, NW, EXACT>() + 4) * 4);
 }
 }  // namespace
+
+void launch_attn_keep_wide_rows(const float*, const void*, int64_t, const int32_t*, int, const int32_t*, const int32_t*,
+                                const int32_t*, int, int, const float*, const void*, int64_t, int, void*, int64_t, float,
+                                int, int, bool, int, int, int, float, float, hipStream_t);   // mix_keep_attn_mfma.hip
 
 struct KeepSplitArgs {
   const float* q;
@@ -126,7 +130,7 @@ __global__ __launch_bounds__(64 * NW, SHARED && DK >= 10 ? 1 : 2) void attn_keep
   constexpr int QR = E + 8;                              // shorts per query row in LDS
   constexpr int MG = DV % 4 == 0 ? 4 : 2;                // value blocks taken together
   constexpr int QP = query_parts<DK, EXACT>(), PP = EXACT ? 3 : 2;   // parts of a query entry, of a weight
-  constexpr int WL = wave_lds<DK, DV, SHARED, EXACT>(), MP = merge_passes<DV, EXACT>(), VP = vdim / MP;
+  constexpr int WL = wave_lds<DK, DV, SHARED, NW, EXACT>(), MP = merge_passes<DV, NW, EXACT>(), VP = vdim / MP;
   const int s = blockIdx.x, g = blockIdx.y;
   const int ql = a.q_len[s], kvl = a.kv_len[s];
   const int rep = a.H / a.G;
@@ -435,8 +439,8 @@ __global__ __launch_bounds__(64 * NW, SHARED && DK >= 10 ? 1 : 2) void attn_keep
 
 // ------------------------------------------------------------------ launcher
 template <int DK, int DV, bool SHARED, int NW, bool EXACT>
-static void launch_split_one(const KeepSplitArgs& a, int NA, int short_rows, hipStream_t s) {
-  constexpr size_t lds = (size_t)NW * wave_lds<DK, DV, SHARED, EXACT>() + 2 * NW * 16 * sizeof(float) +
+static void launch_split_one(const KeepSplitArgs& a, int NA, int z, hipStream_t s) {
+  constexpr size_t lds = (size_t)NW * wave_lds<DK, DV, SHARED, NW, EXACT>() + 2 * NW * 16 * sizeof(float) +
                          (turns_ahead<DK, SHARED>() == 2 ? query_parts<DK, EXACT>() * 16 * (32 * DK + 8) * 2 : 0);
   static_assert(lds <= 160 * 1024, "LDS of a CU");
   static bool attr = false;
@@ -445,36 +449,56 @@ static void launch_split_one(const KeepSplitArgs& a, int NA, int short_rows, hip
                               hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
     attr = true;
   }
-  const int tiles = (short_rows * (a.H / a.G) + 15) / 16;
-  hipLaunchKernelGGL((attn_keep_split_kernel<DK, DV, SHARED, NW, EXACT>), dim3(NA, a.G, tiles < 4 ? tiles : 4),
+  hipLaunchKernelGGL((attn_keep_split_kernel<DK, DV, SHARED, NW, EXACT>), dim3(NA, a.G, z),
                      dim3(64 * NW), lds, s, a);
 }
 
-// Eight waves to a workgroup where sequences and heads alone leave CUs idle: a wave's chain of
-// pages is the time then.  The wide latent's staged page leaves room for four.
+// Eight waves to a workgroup where sequences and heads alone leave CUs idle: a wave's chain of pages is the
+// time then.  The wide latent's staged page leaves room for four, one workgroup to a CU; once there are more
+// workgroups than CUs the prompts' kernel takes its rows, which reads a page once for all heads, not for every
+// 16 of them (64 heads of 576: 128 sequences of 600 tokens 78 us split, 54 there; 64 of them 40 and 53).  Many
+// workgroups of large groups in plain sizes: two waves, or one, whose partial results need no merge (512
+// sequences of 100 tokens, 32 heads over 2 of 128: 23 us with four waves, 20 with one; of 1,000: 100 and 99).
+// Column tiles side by side: as many as the sequences have on the average, more where CUs would idle (one
+// sequence of 600 tokens with 33 rows, 64 heads: 1,130 us with four side by side, 38 with all).
 template <int DK, int DV, bool SHARED, bool EXACT>
-static void launch_split_waves(const KeepSplitArgs& a, int NA, int short_rows, hipStream_t s) {
-  if constexpr (!(SHARED && DK >= 10)) {
-    if (NA * a.G < 256) return launch_split_one<DK, DV, SHARED, 8, EXACT>(a, NA, short_rows, s);
+static void launch_split_waves(const KeepSplitArgs& a, int T, int NA, int tiles, hipStream_t s) {
+  const int64_t work = (int64_t)a.G * (((int64_t)T * (a.H / a.G) + 15) / 16), wgs = (int64_t)NA * a.G;
+  const int z = (int)std::min<int64_t>(tiles, std::max((work + wgs - 1) / wgs, 256 / wgs));
+  if constexpr (SHARED && DK >= 10) {
+    if constexpr (!EXACT) {
+      if (work > 256)
+        return launch_attn_keep_wide_rows(a.q, a.k_cache, a.vrs, a.bt, a.maxb, a.q_start, a.q_len, a.kv_len, T, NA,
+                                          a.head_bias, a.gate, a.gate_stride, a.gate_w, a.out, a.out_stride, a.scale,
+                                          a.window, a.keep_first, a.sigmoid != 0, a.H, a.G, 32 * DK, a.softcap,
+                                          a.out_mult, s);
+    }
+  } else {
+    if (wgs < 256) return launch_split_one<DK, DV, SHARED, 8, EXACT>(a, NA, z, s);
+    if constexpr (!EXACT) {
+      if (work >= 1024) return launch_split_one<DK, DV, SHARED, 1, EXACT>(a, NA, z, s);
+      if (work >= 512) return launch_split_one<DK, DV, SHARED, 2, EXACT>(a, NA, z, s);
+    }
   }
-  launch_split_one<DK, DV, SHARED, 4, EXACT>(a, NA, short_rows, s);
+  launch_split_one<DK, DV, SHARED, 4, EXACT>(a, NA, z, s);
 }
 
 // The sizes are those of keep_mfma_ok, which the caller has asked.
 void launch_attn_keep_split(const float* q, const void* k_cache, const void* v_cache, int64_t vrs, const int32_t* bt,
-                            int maxb, const int32_t* q_start, const int32_t* q_len, const int32_t* kv_len, int NA,
-                            int short_rows, const float* head_bias, const void* gate, int64_t gate_stride, int gate_w,
+                            int maxb, const int32_t* q_start, const int32_t* q_len, const int32_t* kv_len, int T,
+                            int NA, int short_rows, const float* head_bias, const void* gate, int64_t gate_stride, int gate_w,
                             void* out, int64_t out_stride, float scale, int window, int keep_first, bool sigmoid,
                             int H, int G, int E, int vdim, bool shared, float softcap, float out_mult, hipStream_t s) {
-  if (NA == 0) return;
+  if (NA == 0 || T == 0) return;
   const KeepSplitArgs a{q, (const bf16_t*)k_cache, (const bf16_t*)v_cache, vrs, bt, maxb, q_start, q_len, kv_len,
                         head_bias, (const bf16_t*)gate, gate_stride, gate_w, (bf16_t*)out, out_stride,
                         scale, softcap, out_mult, window, keep_first, (int)sigmoid, H, G};
   const int DK = E / 32, DV = vdim / 16;
   const bool exact = H / G < 16;
+  const int tiles = (int)(((int64_t)std::min(short_rows, T) * (H / G) + 15) / 16);   // at most, of a sequence
 #define SPLIT_GO(dk, dv, sh)                                                         \
-  return exact ? launch_split_waves<dk, dv, sh, true>(a, NA, short_rows, s)          \
-               : launch_split_waves<dk, dv, sh, false>(a, NA, short_rows, s)
+  return exact ? launch_split_waves<dk, dv, sh, true>(a, T, NA, tiles, s)          \
+               : launch_split_waves<dk, dv, sh, false>(a, T, NA, tiles, s)
   if (shared) {
     if (DK == 3) SPLIT_GO(3, 4, true);
     if (DK == 4 && DV == 4) SPLIT_GO(4, 4, true);
