@@ -18,14 +18,14 @@
 // What bounds it: the chain over a run's chunks, and inside a chunk the instructions of the waves
 // that share a SIMD.  Token by token the chain was 0.2 - 2.6 us a token (LDS round trips, 64 x 64
 // FMAs on one or four waves); here a chunk's chain is 36 (wkv, gla) or 56 (delta) MFMAs of 16x16x4
-// per wave, 1.4 - 2.1 us.  One workgroup per (run, head, 64 value channels): four consumer waves hold
+// per wave, 1.6 - 2.3 us.  One workgroup per (run, head, 64 value channels): four consumer waves hold
 // 64 x 16 of the state in accumulators, which are MFMA operands as they lie (a lane holds channels
 // 16 i + 4 grp + r of its column: exactly the K slices that step (i, r) of Qd S takes); the other
 // waves work ahead: decays and their products for chunk c + 3, A for chunk c + 2, T for chunk c + 1,
 // wkv's norm and gate for chunk c - 1; one barrier per chunk.  A state operand never leaves the
 // registers, an fp32 operand is never narrowed.  Measured, two runs of 2,048 tokens in bf16: wkv with
-// 64 heads of 64 x 64 5,353 -> 180 us; delta rule with 32 heads of 64 x 128 741 (decays and scan) ->
-// 277 us; gla in fp32, five ragged runs of up to 1,031, 32 heads, 447 -> 117 us.
+// 64 heads of 64 x 64 5,353 -> 203 us; delta rule with 32 heads of 64 x 128 741 (decays and scan) ->
+// 301 us; gla in fp32, five ragged runs of up to 1,031, 32 heads, 447 -> 121 us.
 #include <algorithm>
 #include <type_traits>
 
@@ -627,7 +627,7 @@ __global__ __launch_bounds__(chunk_threads(MODE)) void chunk_recurrence_share_ke
 }
 
 // ------------------------------------------------------------------ launcher
-// A workgroup costs some 8 us before its first chunk is out and 1.4 - 2.3 us a chunk, one to a CU; the
+// A workgroup costs some 8 us before its first chunk is out and 1.6 - 2.3 us a chunk, one to a CU; the
 // token-by-token kernels some 6 us and 0.2 (64 runs) - 2.6 us a token, many to a CU.  Times below are of whole
 // steps, 32 heads of 64 x 128 (wkv: 64 of 64 x 64), chunks against tokens.
 // Two workgroups to a CU or fewer: everything in chunks from 8 rows a run on (one run of 8: gla 14 us against 25,

@@ -25,7 +25,7 @@
 // accumulators are rarely rescaled), rows meet by lane swaps instead of LDS, one barrier a page, and a
 // sequence's last blocks, which see the most keys, start first.  Measured with the append before it,
 // without -> with these: prompts of 2,048 and 600 tokens (32 heads over 8 of 128, softcap) 234 -> 223 us,
-// three ragged prompts with sigmoid weights and a window of 512 125 -> 87 us, one prompt of 2,048 with
+// five ragged prompts with sigmoid weights and a window of 1,024 125 -> 87 us, one prompt of 2,048 with
 // 64 heads and a window 268 -> 174 us.  What is left of the first is the longest block's chain of 64
 // pages.  32 x 32 tiles, a wave per 32 queries, took 217 and 116 us there and lost 20 % on prompts of a
 // few hundred tokens; two waves sharing such a wave's pages 251 and 119.

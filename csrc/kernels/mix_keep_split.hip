@@ -8,7 +8,7 @@
 // tiles, 121 us.  Here every wave takes every NW-th piece: its key rows go from memory straight into
 // MFMA operands, its value rows through the wave's own piece of LDS (read back transposed), the next
 // rows are in flight meanwhile, and no wave waits for another until the partial results (running
-// maximum, sum, weighted values) meet in LDS at the end.  Measured: 34 us (4.9 TB/s), 13 us and 53 us.
+// maximum, sum, weighted values) meet in LDS at the end.  Measured: 37 us (4.5 TB/s), 15 us and 54 us.
 //
 // The 16 MFMA columns are (row, head) pairs of one key/value head, so the rows of a short extend and
 // the heads of a group share one pass.

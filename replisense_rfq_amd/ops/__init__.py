@@ -1470,10 +1470,11 @@ def attn_keep_window(q, k_cache, v_cache, vdim: int, block_tables, q_start, q_le
                      keep_first: int = 0, sigmoid: bool = False, short_rows: int = 0,
                      mfma: bool | None = None, softcap: float = 0.0, out_mult: float = 1.0):
     """Work items (sequence, block of KEEP_QBLK queries) as for attn_mixq_prefill.
-    ``short_rows`` > 0: every sequence has at most that many rows (a decode section); the
-    kernel then runs one workgroup per (sequence, key/value head) over one pass through the
-    pages where the sizes fit its LDS.  Otherwise bf16 pages whose sizes the MFMA tiles cover
-    run on them unless ``mfma`` is False (the FMA work-item kernel).  ``gate``: logits [T, H]
+    ``short_rows`` > 0: every sequence has at most that many rows (a decode section); bf16 pages
+    whose sizes the MFMA tiles cover are then split over waves, others take one workgroup per
+    (sequence, key/value head) over one pass through the pages where the sizes fit its LDS.  Prompt
+    sections run on MFMA tiles where those cover the sizes, unless ``mfma`` is False (the FMA
+    work-item kernel).  ``gate``: logits [T, H]
     (one per head) or [T, H vdim] (one per output).  ``softcap`` > 0: softcap tanh(score / softcap);
     the output is multiplied by ``out_mult``."""
     if _gpu(q):

@@ -149,3 +149,25 @@ def test_decode_scores_under_a_wide_cap(H, G, E, vd):
     q, k = torch.randn(2, H, E, generator=g) * 2, torch.randn(150, G, E, generator=g).bfloat16()
     v = torch.randn(150, G, vd, generator=g).bfloat16() if vd else None
     _near(*_both(q, k, v, False, scale=E ** -0.5, softcap=2.0 ** 17), 2.0 ** -9)
+
+
+# prompts, and decode rows of 16 heads a key head or more: weights in two parts, 16 bits
+@pytest.mark.parametrize("H,G,E,vd,prompt", [(8, 2, 128, 128, True), (4, 4, 64, 32, True), (6, 1, 192, 0, True), (8, 1, 320, 0, True),
+                                             (4, 1, 576, 0, True), (32, 2, 128, 128, False), (16, 1, 192, 0, False),
+                                             (20, 1, 320, 0, False), (16, 1, 576, 0, False)])
+def test_weights_keep_16_bits(H, G, E, vd, prompt):
+    """The values of neighbouring keys cancel, scores of rms 2^-6: the results are 2^-6 of what goes in.  Two
+    parts of a weight, 2^-17: 2^-11 of the results; one, 2^-9: an eighth of them.  The last row has an even
+    number of keys."""
+    g = torch.Generator().manual_seed(E + 7)
+    T, L = (34, 160) if prompt else (2, 160)
+    k, q = torch.randn(L, G, E, generator=g).bfloat16(), torch.randn(T, H, E, generator=g).bfloat16().float()
+    if vd:
+        v = torch.randn(L // 2, G, vd, generator=g).bfloat16()
+        v, n = torch.stack([v, -v], 1).view(L, G, vd), E
+    else:                                       # the keys are the values: they differ in the last 64 entries
+        v, n = None, 64
+        k[1::2, :, :E - 64] = -k[0::2, :, :E - 64]
+        q[..., :E - 64] = 0.0
+    got, want = _both(q, k, v, prompt, scale=2.0 ** -6 * n ** -0.5)
+    _near(got[-1:], want[-1:], 2.0 ** -7)
