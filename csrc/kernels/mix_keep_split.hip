@@ -464,7 +464,7 @@ static void launch_split_one(const KeepSplitArgs& a, int NA, int z, hipStream_t 
 template <int DK, int DV, bool SHARED, bool EXACT>
 static void launch_split_waves(const KeepSplitArgs& a, int T, int NA, int tiles, hipStream_t s) {
   const int64_t work = (int64_t)a.G * (((int64_t)T * (a.H / a.G) + 15) / 16), wgs = (int64_t)NA * a.G;
-  const int z = (int)std::min<int64_t>(tiles, std::max((work + wgs - 1) / wgs, 256 / wgs));
+  const int z = (int)std::min<int64_t>(std::min(tiles, 65535), std::max((work + wgs - 1) / wgs, 256 / wgs));
   if constexpr (SHARED && DK >= 10) {
     if constexpr (!EXACT) {
       if (work > 256)

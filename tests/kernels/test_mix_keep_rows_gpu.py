@@ -3,6 +3,7 @@ columns heads of a row; fewer waves to a workgroup; workgroups that take several
 import pytest
 import torch
 
+from replisense_rfq_amd import ops
 from tests.kernels.test_mix_keep_bits_gpu import _both, _near
 from tests.kernels.test_mix_keep_mfma_gpu import _check
 
@@ -49,3 +50,21 @@ def test_many_rows_of_few_sequences():
     for H, G, E, vd, shared in ((32, 8, 128, 128, False), (20, 1, 192, 128, True), (4, 1, 576, 512, True)):
         _check(H, G, E, vd, shared, seqs=[(90, 32), (33, 1), (40, 20)], softcap=20.0)
     _check(32, 8, 128, 128, False, seqs=[(33, 1)] * 70 + [(90, 32)])
+
+
+def test_more_column_tiles_than_a_grid_holds():
+    """One sequence of 33,000 rows with 32 heads, as a decode section and as a prompt."""
+    T, H, E, BS = 33000, 32, 32, 32
+    g = torch.Generator().manual_seed(1)
+    q = torch.randn(T, H, E, generator=g).cuda()
+    nb = (T + BS - 1) // BS
+    k, v = (torch.randn(nb, 1, BS, E, generator=g).bfloat16().cuda() for _ in range(2))
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device="cuda")  # noqa: E731
+    blocks = list(range((T + 31) // 32))
+    out = []
+    for short in (T, 0):
+        out.append(torch.zeros(T, H * E, dtype=torch.bfloat16, device="cuda"))
+        ops.attn_keep_window(q, k, v, E, i32([list(range(nb))]), i32([0]), i32([T]), i32([T]), i32([0] * len(blocks)),
+                             i32(blocks), None, None, out[-1], E ** -0.5, window=40, short_rows=short)
+    # both round the same sums to bf16: neighbouring values at a tie
+    torch.testing.assert_close(out[0].float(), out[1].float(), atol=1e-3, rtol=2.0 ** -7)
