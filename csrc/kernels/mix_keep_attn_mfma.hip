@@ -5,31 +5,36 @@
 // the values may be the leading entries of the key rows themselves (latent attention).
 // Decode rows have a kernel of their own (mix_keep_split.hip).
 //
-// One workgroup per (work item, HPW heads of one key/value head); a work item is (sequence, block of
-// 32 queries).  Its 2 HPW waves are (16 queries) x (head): a wave keeps the running maximum and sum of
-// its 16 query columns and the weighted values O^T [vdim x 16] in registers.  A key tile is one page,
-// staged in LDS for all heads of the workgroup, the next page while this one is multiplied; one barrier
-// per page.  Pages between the kept first tokens and the window are never read.
+// One workgroup per (work item, HPW heads of one key/value head); a work item is (sequence, block of 32 queries).
+// A wave has the 32 queries of a head: it keeps the running maximum and sum of its query columns and the weighted
+// values O^T [vdim x 32] in registers.  A key tile is one page, staged in LDS for all heads of the workgroup, the
+// next ones while this one is multiplied; one barrier per page.  Pages between the kept first tokens and the window
+// are never read.
 //
-//   S^T[key, query] = K[key, :] . Q[query, :]   v_mfma_f32_16x16x32_bf16, A = key rows from LDS,
-//                     B = the queries in registers as bf16 hi (+ lo for keys of up to 320
-//                     entries: they arrive in fp32 and are not rounded a second time), up to 192
-//                     entries already times the scale and log2 e
+//   S^T[key, query] = K[key, :] . Q[query, :]   v_mfma_f32_32x32x16_bf16, A = key rows from LDS, B = the queries in
+//                     registers as bf16 hi + lo (they arrive in fp32 and are not rounded a second time), already
+//                     times the scale and log2 e
 //   cap, mask, weights per query column in fp32, base 2
-//   O^T[dv, query] += V^T[dv, keys] . P^T[keys, query]   A = two transposed reads of V
-//                     (ds_read_tr16_b64), B = the weights straight from the score registers as bf16
-//                     hi + lo parts (two MFMAs), so the weights keep fp32's precision
+//   O^T[dv, query] += V^T[dv, keys] . P^T[keys, query]   A = two transposed reads of V (ds_read_tr16_b64), B = the
+//                     weights straight from the score registers as bf16 hi + lo parts (two MFMAs), so the weights
+//                     keep fp32's precision
 //
-// What bounds it: the vector instructions between the products, and their latency.  Pages without an
-// edge inside skip the masks, the maximum moves only when a score passes it by 2^11 (so the
-// accumulators are rarely rescaled), rows meet by lane swaps instead of LDS, one barrier a page, and a
-// sequence's last blocks, which see the most keys, start first.  Measured with the append before it,
-// without -> with these: prompts of 2,048 and 600 tokens (32 heads over 8 of 128, softcap) 234 -> 223 us,
-// five ragged prompts with sigmoid weights and a window of 1,024 125 -> 87 us, one prompt of 2,048 with
-// 64 heads and a window 268 -> 174 us.  What is left of the first is the longest block's chain of 64
-// pages.  32 x 32 tiles, a wave per 32 queries, took 217 and 116 us there and lost 20 % on prompts of a
-// few hundred tokens; two waves sharing such a wave's pages 251 and 119.
+// What bounds it: the vector instructions between the products (five and one and a half transcendental ones to an
+// MFMA) and how well they hide behind them.  A SIMD issues one in four clocks beside an MFMA of 32, one wave alone in
+// six to seven; so the order is fixed piece by piece (sched_barrier): the products of the next page's scores stand
+// beside this page's weights, those of this page's values beside the next page's caps and maximum, one product to
+// every four or five others, operands from LDS two products ahead, page copies as LDS-DMA that nothing waits for but
+// the barrier.  The maximum is looked at lane by lane and moves only when a score passes it by 2^11, pages without an
+// edge inside skip the masks.  A block's workgroups lie side by side and blocks with the most keys start first, in
+// front of the others on their SIMD (s_setprio): the longest block's chain of pages is the end of a short step.
+// Measured, the attention alone, against 16 x 16 tiles with a wave per 16 queries, compiler's order and heads one
+// after the other: prompts of 2,048 and 600 tokens (32 heads over 8 of 128, softcap) 194 -> 90 us, five ragged
+// prompts with sigmoid weights and a window of 1,024 72 -> 52 us, one prompt of 2,048 over 192-wide latents (32
+// heads) 177 -> 96 us; a workgroup alone takes 0.86 us a page, a full chip 1.1 us a page and CU.  Two pages to a
+// barrier, two score chains, or operands four products ahead changed nothing.
 #include <algorithm>
+#include <type_traits>
+#include <utility>
 
 #include "common.h"
 #include "mix_common.h"
@@ -37,6 +42,8 @@
 namespace rfqmix {
 
 using rfq::as_bf16x8;
+using rfq::f32x16;
+using rfq::u32x4;
 using rfq::f32x4;
 using rfq::s16x4;
 using rfq::s16x8;
@@ -66,10 +73,6 @@ __device__ __forceinline__ float both_halves_sum(float x) {
   return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
 
-template <int DK, int DV, bool SHARED>
-constexpr int keep_page_shorts() {
-  return WBS * (32 * DK + 8) + (SHARED ? 0 : WBS * (16 * DV + 8));
-}
 }  // namespace
 
 struct KeepArgs {
@@ -133,17 +136,81 @@ __device__ __forceinline__ void store_rows(const KeepArgs& a, f32x4 (&o)[DV], fl
   }
 }
 
-// DK = E / 32, DV = vdim / 16, HPW heads per workgroup, SHARED: values = leading entries of the
-// key rows, MODE: 0 softmax, 1 softmax of capped scores, 2 sigmoid, 3 sigmoid of capped scores.
-// Two heads a workgroup: three waves a SIMD, which the compiler left to itself spends on 180 registers for
-// two (16 chunks of 230 rows after 416, 12 heads over 2 of 128, softcap: 92 -> 70 us a pass).
+// lane (col, half) of a 32 x 32 tile holds value channels 32 m + 8 b + 4 half .. + 3 of its query: 8-byte stores
+template <int VM, int MODE>
+__device__ __forceinline__ void store_rows32(const KeepArgs& a, const f32x16 (&o)[VM], float lrun, int64_t t, int hh,
+                                             int half, bool qlive) {
+  constexpr int vdim = 32 * VM;
+  const float l = both_halves_sum(lrun);
+  if (!qlive) return;
+  const bf16_t* gate = static_cast<const bf16_t*>(a.gate);
+  float mul = MODE >= 2 ? a.out_mult : (l > 0.f ? a.out_mult / l : 0.f);
+  if (gate != nullptr && a.gate_w == 1) mul /= 1.0f + __expf(-ldf(gate + t * a.gate_stride + hh));
+  // a gate column per output: four neighbouring logits, 8-byte reads
+  const bf16_t* grow = gate != nullptr && a.gate_w > 1 ? gate + t * a.gate_stride + (int64_t)hh * vdim + half * 4 : nullptr;
+  bf16_t* orow = static_cast<bf16_t*>(a.out) + t * a.out_stride + (int64_t)hh * vdim + half * 4;
+#pragma unroll
+  for (int m = 0; m < VM; ++m)
+#pragma unroll
+    for (int b = 0; b < 4; ++b) {
+      float y[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) y[i] = o[m][4 * b + i] * mul;
+      if (grow != nullptr) {
+        const uint2 gu = *reinterpret_cast<const uint2*>(grow + m * 32 + b * 8);
+        y[0] /= 1.0f + __expf(-__uint_as_float(gu.x << 16));
+        y[1] /= 1.0f + __expf(-__uint_as_float(gu.x & 0xffff0000u));
+        y[2] /= 1.0f + __expf(-__uint_as_float(gu.y << 16));
+        y[3] /= 1.0f + __expf(-__uint_as_float(gu.y & 0xffff0000u));
+      }
+      *reinterpret_cast<uint2*>(orow + m * 32 + b * 8) = make_uint2(rfq::pack_bf16x2(y[0], y[1]), rfq::pack_bf16x2(y[2], y[3]));
+    }
+}
+
+// 64 lanes' pieces of 16 bytes from base + offset (per lane) to LDS, one after another from byte `to` (the same for
+// the wave) on.  Written out: behind the builtin the compiler waits for the copy before any later LDS read through a
+// builtin, here for the next page in the middle of this one.  The caller waits with s_waitcnt vmcnt(0).  Nothing
+// else in a kernel that uses it may rely on M0.
+__device__ __forceinline__ void lds_copy16(const void* base, uint32_t offset, uint32_t to) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
+               ::"v"(offset), "s"(base), "s"(__builtin_amdgcn_readfirstlane(to)) : "memory");
+#endif
+}
+__device__ __forceinline__ uint32_t lds_byte(const unsigned char* smem) {      // where the dynamic LDS begins
+  return (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const unsigned char*)smem;
+}
+
+// DK = E / 32, DV = vdim / 16, HPW heads per workgroup, SHARED: values = leading entries of the key rows, MODE: 0
+// softmax, 1 softmax of capped scores, 2 sigmoid, 3 sigmoid of capped scores.
+//
+// A row's 16-byte pieces are permuted inside it, and rows of 256 bytes lie 16 bytes apart after every four, so
+// that the pieces that one LDS access takes together (K: a piece of 16 neighbouring rows; V, transposed: 64
+// bytes of four neighbouring rows) lie on different banks.
+template <int E>
+__device__ __forceinline__ int page_swizzle(int r) {
+  if constexpr (E == 128) return (r & 3) << 2;
+  if constexpr (E != 128 && E % 64 == 0) return ((r >> 1) & 1) << 2 | ((r >> 2) & 3);
+  return (r >> 2) & 3;
+}
+template <int E>
+constexpr int page_row(int r) { return r * E + (E == 128 ? (r >> 2) * 8 : 0); }     // shorts before row r
+// f(0), f(1) .. f(N - 1) with constants: loops whose bodies have loops over parts of their index are unrolled for sure
+template <int... I, typename F>
+__device__ __forceinline__ void each_of(std::integer_sequence<int, I...>, F f) { (f(std::integral_constant<int, I>{}), ...); }
+template <int N, typename F>
+__device__ __forceinline__ void each(F f) { each_of(std::make_integer_sequence<int, N>{}, f); }
+template <int DK, int DV, bool SHARED>
+constexpr int tile_lds_shorts() { return SHARED ? 3 * page_row<32 * DK>(WBS) : 2 * (page_row<32 * DK>(WBS) + page_row<16 * DV>(WBS)); }
+
 template <int DK, int DV, int HPW, bool SHARED, int MODE>
-__global__ __launch_bounds__(128 * HPW, HPW == 2 ? 3 : 1) void attn_keep_mfma_kernel(const KeepArgs a) {
-  constexpr int E = 32 * DK, vdim = 16 * DV, NT = 128 * HPW;
-  constexpr int KRS = E + 8;                       // shorts per key row in LDS (+ 16 bytes)
-  constexpr int VRS = SHARED ? KRS : vdim + 8;     // shorts per value row
-  constexpr int PGS = keep_page_shorts<DK, DV, SHARED>();
-  const int item = gridDim.x - 1 - blockIdx.x;     // a sequence's later blocks see the most keys: they start first
+__global__ __launch_bounds__(64 * HPW, 2) void attn_keep_tile_kernel(const KeepArgs a) {
+  constexpr int E = 32 * DK, vdim = 16 * DV, KS = 2 * DK, VM = DV / 2, NT = 64 * HPW;
+  constexpr int VR = SHARED ? E : vdim;                      // shorts per row of the values' image
+  constexpr int KP = page_row<E>(WBS), VP = page_row<VR>(WBS);
+  const int groups = a.H / HPW;
+  const int at = gridDim.x - 1 - blockIdx.x;       // a sequence's later blocks see the most keys: they start first
+  const int item = at / groups, hg = at - item * groups;
   const int s = a.work_seq[item];
   if (s < 0) return;
   const int ql = a.q_len[s];
@@ -151,204 +218,314 @@ __global__ __launch_bounds__(128 * HPW, HPW == 2 ? 3 : 1) void attn_keep_mfma_ke
   if (i0 >= ql) return;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int col = lane & 15, grp = lane >> 4;
-  const int g = ((int)blockIdx.y * HPW) / (a.H / a.G);
-  const int hh = (int)blockIdx.y * HPW + (wid >> 1);
+  const int col = lane & 31, half = lane >> 5;
+  const int hh = hg * HPW + wid, g = hg * HPW / (a.H / a.G);
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-  short* const pages = reinterpret_cast<short*>(smem);       // two of them
+  const uint32_t lds0 = lds_byte(smem);
+  short* const kpages = reinterpret_cast<short*>(smem);
+  short* const vpages = SHARED ? kpages : kpages + 2 * KP;
 
   const int nq = min(WQB, ql - i0);
   const int p0 = a.kv_len[s] - ql + i0, plast = p0 + nq - 1;
   const int window = a.window, keep_first = a.keep_first;
   const int jwin = window > 0 ? max(0, p0 - window + 1) : 0;
   const int kf = window > 0 ? min(keep_first, jwin) : 0;     // kept keys before the window
-  const int row = (wid & 1) * 16 + col, pi = p0 + row;       // this lane's query
-  const bool qlive = row < nq;
-  const int64_t t = a.q_start[s] + i0 + (qlive ? row : 0);
+  const int pi = p0 + col;                                   // this lane's query
+  const bool qlive = col < nq;
+  const int64_t t = a.q_start[s] + i0 + (qlive ? col : 0);
   typedef const __attribute__((address_space(4))) int32_t const_i32;
   const_i32* bt = (const_i32*)(uintptr_t)(a.bt + (int64_t)s * a.maxb);
+
+  // pages [0, n_keep) hold the kept first tokens, pages [pg_win, pg_last] the window
+  const int pg_last = plast / WBS, pg_win = jwin / WBS;
+  const int n_keep = min((kf + WBS - 1) / WBS, pg_win), skip = pg_win - n_keep, turns = pg_last + 1 - skip;
+  // Long chains in front of the short ones that share their SIMD (2,048 and 600 tokens: 97 us without, 92 with).
+  if (turns >= 32) __builtin_amdgcn_s_setprio(3);
+  else if (turns >= 20) __builtin_amdgcn_s_setprio(2);
+  else if (turns >= 10) __builtin_amdgcn_s_setprio(1);
+  auto page_at = [&](int i) { return i < n_keep ? i : i + skip; };
+  auto number = [&](int i) { return bt[page_at(min(i, turns - 1))]; };
+
+  // ---- staging: LDS-DMA, 64 pieces of 16 bytes a time, permuted at the source
+  constexpr int NPK = WBS * E / 512, NPV = SHARED ? 0 : WBS * vdim / 512;
+  constexpr int NK = (NPK + HPW - 1) / HPW, NV = (NPV + HPW - 1) / HPW;
+  uint32_t ksrc[NK], vsrc[NV > 0 ? NV : 1];
+#pragma unroll
+  for (int i = 0; i < NK; ++i) {
+    const int x = (wid + i * HPW) * 64 + lane, r = x / (E / 8), c = x - r * (E / 8);
+    ksrc[i] = (r * E + (c ^ page_swizzle<E>(r)) * 8) * 2;
+  }
+#pragma unroll
+  for (int i = 0; i < NV; ++i) {
+    const int x = (wid + i * HPW) * 64 + lane, r = x / (vdim / 8), c = x - r * (vdim / 8);
+    vsrc[i] = (r * (int)a.vrs + (c ^ page_swizzle<vdim>(r)) * 8) * 2;
+  }
+  auto fetch_k = [&](int page, int buf) {
+    const char* kb = static_cast<const char*>(a.k_cache) + ((int64_t)page * a.G + g) * WBS * E * 2;
+#pragma unroll
+    for (int i = 0; i < NK; ++i) {
+      const int piece = wid + i * HPW;
+      if ((i + 1) * HPW <= NPK || piece < NPK)
+        lds_copy16(kb, ksrc[i], lds0 + 2 * (buf * KP + piece * (E == 128 ? 520 : 512)));
+    }
+  };
+  auto fetch_v = [&](int page, int buf) {
+    if constexpr (!SHARED) {
+      const char* vb = static_cast<const char*>(a.v_cache) + ((int64_t)page * a.G + g) * WBS * a.vrs * 2;
+#pragma unroll
+      for (int i = 0; i < NV; ++i) {
+        const int piece = wid + i * HPW;
+        if ((i + 1) * HPW <= NPV || piece < NPV)
+          lds_copy16(vb, vsrc[i], lds0 + 2 * (2 * KP + buf * VP + piece * (vdim == 128 ? 520 : 512)));
+      }
+    }
+  };
+  int32_t n0 = number(0), n1 = number(1), n2 = number(2);    // numbers of the pages of this turn, the next two
+  fetch_k(n0, 0);
+  fetch_v(n0, 0);
+  if (turns > 1) fetch_k(n1, 1);
 
   // scores arrive as exponents of 2: s log2 e; 2 s log2 e / cap; -s log2 e (sigmoid, no cap)
   const float qmul = a.scale * (MODE % 2 == 1 ? 2.f * kLog2e / a.softcap : MODE == 2 ? -kLog2e : kLog2e);
   const float cap2 = MODE % 2 == 1 ? a.softcap * kLog2e : 0.f;
-  s16x8 qhi[DK], qlo[DK];
+  s16x8 qhi[KS], qlo[KS];
   {
-    const float* qp = a.q + (t * a.H + hh) * E + grp * 8;
+    const float* qp = a.q + (t * a.H + hh) * E + half * 8;
 #pragma unroll
-    for (int ks = 0; ks < DK; ++ks) {
-      const float4 x = *reinterpret_cast<const float4*>(qp + ks * 32);
-      const float4 y = *reinterpret_cast<const float4*>(qp + ks * 32 + 4);
+    for (int ks = 0; ks < KS; ++ks) {
+      const float4 x = *reinterpret_cast<const float4*>(qp + ks * 16);
+      const float4 y = *reinterpret_cast<const float4*>(qp + ks * 16 + 4);
       const float f[8] = {x.x * qmul, x.y * qmul, x.z * qmul, x.w * qmul, y.x * qmul, y.y * qmul, y.z * qmul, y.w * qmul};
       split_bf16w(f, qhi[ks], qlo[ks]);
     }
   }
-  f32x4 o[DV];
+  f32x16 o[VM];
 #pragma unroll
-  for (int m = 0; m < DV; ++m) o[m] = (f32x4){0.f, 0.f, 0.f, 0.f};
+  for (int m = 0; m < VM; ++m)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) o[m][i] = 0.f;
   const float hb = a.head_bias != nullptr ? a.head_bias[hh] * kLog2e : 0.f;
   const bool sink = MODE < 2 && a.head_bias != nullptr;
   // the sink is one more entry of the row: it starts the maximum, and one lane's part of the sum
-  float mrun = sink ? hb : kNegInfW, lrun = sink && grp == 0 ? 1.f : 0.f;
+  float mrun = sink ? hb : kNegInfW, lrun = sink && half == 0 ? 1.f : 0.f;
 
-  // ---- staging
-  constexpr int NKV = (WBS * E / 8 + NT - 1) / NT;
-  constexpr int NVV = SHARED ? 1 : (WBS * vdim / 8 + NT - 1) / NT;
-  s16x8 kreg[NKV], vreg[NVV];
-  auto fetch = [&](int page) {
-    const int64_t at = ((int64_t)page * a.G + g) * WBS;      // the page's first slot
-    const bf16_t* kb = static_cast<const bf16_t*>(a.k_cache) + at * E;
+  // keys: row col, entries 16 ks + 8 half ..; values, transposed: rows 16 t + 8 j + 4 half + lane % 16 / 4,
+  // channels 32 m + 16 (lane / 16 % 2) + 4 (lane % 4) ..
+  constexpr int KA = E % 64 == 0 ? 4 : 2, KI = E == 128 ? 2 : 1;       // KI neighbouring pieces at a fixed distance
+  constexpr int VA = VR == 128 ? 4 : VR % 64 == 0 ? 2 : 1, VJ = VR == 128 ? 1 : 2;
+  int kat[KA], vat[VJ][VA];
 #pragma unroll
-    for (int i = 0; i < NKV; ++i) {
-      const int x = tid + i * NT;
-      if (x < WBS * E / 8) kreg[i] = reinterpret_cast<const s16x8*>(kb)[x];
-    }
-    if constexpr (!SHARED) {
-      const bf16_t* vb = static_cast<const bf16_t*>(a.v_cache) + at * a.vrs;
+  for (int i = 0; i < KA; ++i) kat[i] = page_row<E>(col) + ((2 * KI * i + half) ^ page_swizzle<E>(col)) * 8;
 #pragma unroll
-      for (int i = 0; i < NVV; ++i) {
-        const int x = tid + i * NT;
-        if (x < WBS * vdim / 8) {
-          const int jj = x / (vdim / 8), c = x - jj * (vdim / 8);
-          vreg[i] = *reinterpret_cast<const s16x8*>(vb + jj * a.vrs + c * 8);
-        }
-      }
-    }
-  };
-  // Rows past the sequence's end were never written and may hold anything: zeros.
-  auto stage = [&](int jb, int buf) {
-    short* Ks = pages + buf * PGS;
-    short* Vs = SHARED ? Ks : Ks + WBS * KRS;
-    const bool tail = jb + WBS - 1 > plast;
+  for (int j = 0; j < VJ; ++j)
 #pragma unroll
-    for (int i = 0; i < NKV; ++i) {
-      const int x = tid + i * NT;
-      if (x < WBS * E / 8) {
-        const int jj = x / (E / 8), c = x - jj * (E / 8);
-        s16x8 v = kreg[i];
-        if (SHARED && tail && jb + jj > plast) v = (s16x8){0, 0, 0, 0, 0, 0, 0, 0};
-        *reinterpret_cast<s16x8*>(Ks + jj * KRS + c * 8) = v;
-      }
+    for (int i = 0; i < VA; ++i) {
+      const int r = 8 * j + 4 * half + ((lane & 15) >> 2);
+      vat[j][i] = page_row<VR>(r) + ((4 * i + 2 * ((lane >> 4) & 1) + ((lane & 3) >> 1)) ^ page_swizzle<VR>(r)) * 8 + (lane & 1) * 4;
     }
-    if constexpr (!SHARED) {
-#pragma unroll
-      for (int i = 0; i < NVV; ++i) {
-        const int x = tid + i * NT;
-        if (x < WBS * vdim / 8) {
-          const int jj = x / (vdim / 8), c = x - jj * (vdim / 8);
-          s16x8 v = vreg[i];
-          if (tail && jb + jj > plast) v = (s16x8){0, 0, 0, 0, 0, 0, 0, 0};
-          *reinterpret_cast<s16x8*>(Vs + jj * VRS + c * 8) = v;
-        }
-      }
-    }
-  };
-  const int kat = col * KRS + grp * 8;
-  // transposed reads: a 16-lane group takes 4 key rows x 16 value columns, lane `col` receives its
-  // column (keys 4 grp .. 4 grp + 3 of each 16-key half)
-  const int vat = (4 * grp + (col >> 2)) * VRS + 4 * (col & 3);
 
-  // pages [0 .. pg_keep] hold the kept first tokens, pages [pg_win .. pg_last] the window
-  const int pg_last = plast / WBS;
-  const int pg_keep = kf > 0 ? (kf - 1) / WBS : -1;
-  const int pg_win = jwin / WBS;
-  auto next_page = [&](int pg) { return (pg == pg_keep && pg_win > pg) ? pg_win : pg + 1; };
-  int pg = kf > 0 ? 0 : pg_win, buf = 0;
-  fetch(bt[pg]);
-  stage(pg * WBS, 0);
-  int pn = next_page(pg);
-  if (pn <= pg_last) fetch(bt[pn]);
-  __syncthreads();
-  while (pg <= pg_last) {
-    const int jb = pg * WBS;
-    const short* Ks = pages + buf * PGS;
-    const short* Vs = SHARED ? Ks : Ks + WBS * KRS;
-    f32x4 sc[2][2];                                          // two chains per half page
+  auto key = [&](const short* Ks, int ks) {
+    return *reinterpret_cast<const s16x8*>(Ks + kat[ks / KI % KA] + (ks % KI) * 16 + (ks / (KI * KA)) * KI * KA * 16);
+  };
+  auto value = [&](const short* Vs, int c) {                 // 16 keys (c / VM) x 32 channels (c % VM)
+    const int u = c / VM, m = c % VM;
+    const short* vp = Vs + (m / VA) * VA * 32 + vat[0][m % VA] + page_row<VR>(16 * u);
+    const short* vq = Vs + (m / VA) * VA * 32 + vat[VJ - 1][m % VA] + page_row<VR>(16 * u + (VJ == 1 ? 8 : 0));
+    const s16x4 a0 = rfq::ds_read_tr16(vp), a1 = rfq::ds_read_tr16(vq);
+    return (s16x8){a0[0], a0[1], a0[2], a0[3], a1[0], a1[1], a1[2], a1[3]};
+  };
+  float p[16], top = kNegInfW;
+  // What a score becomes before the maximum is known.  Capped: cap2 - 2 cap2 / (2^x + 1), here the quotient,
+  // which falls where the score rises; sigmoid: the weight itself.
+  auto prepare = [&](int i, float x) {
+    if constexpr (MODE % 2 == 1) x = __builtin_amdgcn_rcpf(__builtin_amdgcn_exp2f(x) + 1.f);
+    if constexpr (MODE == 3) x = 2.f * cap2 * x - cap2;
+    if constexpr (MODE >= 2) x = __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(x - hb));
+    p[i] = x;
+    if constexpr (MODE < 2) top = i == 0 ? x : MODE == 1 ? fminf(top, x) : fmaxf(top, x);
+  };
+  auto mask = [&](int jb) {                                  // a page with an edge inside
+    if (jb + WBS - 1 <= p0 && (window <= 0 || plast - jb < window || jb + WBS <= keep_first)) return;
+    const int at = jb + half * 4, hi = pi - at, lo = window > 0 ? hi - window : -WBS, kept = keep_first - at;
 #pragma unroll
-    for (int kt = 0; kt < 2; ++kt) {
-      sc[kt][0] = sc[kt][1] = (f32x4){0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int ks = 0; ks < DK; ++ks) {
-        const s16x8 k = *reinterpret_cast<const s16x8*>(Ks + kat + kt * 16 * KRS + ks * 32);
-        sc[kt][0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(k), as_bf16x8(qhi[ks]), sc[kt][0], 0, 0, 0);
-        sc[kt][1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(k), as_bf16x8(qlo[ks]), sc[kt][1], 0, 0, 0);
-      }
-    }
-    float p[8];
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      float x = sc[i >> 2][0][i & 3] + sc[i >> 2][1][i & 3];
-      if constexpr (MODE % 2 == 1) x = cap2 - 2.f * cap2 * __builtin_amdgcn_rcpf(__builtin_amdgcn_exp2f(x) + 1.f);
-      if constexpr (MODE >= 2) x = __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f((MODE == 3 ? -x : x) - hb));
+    for (int i = 0; i < 16; ++i) {
+      const int j = (i >> 2) * 8 + (i & 3);
+      const bool ok = (j <= hi) & ((j > lo) | (j < kept));
+      const float x = ok ? p[i] : MODE >= 2 ? 0.f : MODE == 1 ? -kNegInfW : kNegInfW;
       p[i] = x;
+      if constexpr (MODE < 2) top = i == 0 ? x : MODE == 1 ? fminf(top, x) : fmaxf(top, x);
     }
-    if (!(jb + WBS - 1 <= p0 && (window <= 0 || plast - jb < window || jb + WBS <= keep_first))) {
-#pragma unroll
-      for (int i = 0; i < 8; ++i) {                          // an edge inside the page
-        const int j = jb + (i >> 2) * 16 + grp * 4 + (i & 3);
-        const bool ok = j <= pi && (window <= 0 || pi - j < window || j < keep_first);
-        p[i] = ok ? p[i] : MODE >= 2 ? 0.f : kNegInfW;
-      }
-    }
-    if constexpr (MODE < 2) {
-      float mx = fmaxf(fmaxf(fmaxf(p[0], p[1]), fmaxf(p[2], p[3])), fmaxf(fmaxf(p[4], p[5]), fmaxf(p[6], p[7])));
-      mx = other_half_max(other_row_max(mx));
-      const bool moves = mx > mrun + kDeferW;                // also for the first keys: mrun = -inf
-      if (__builtin_amdgcn_ballot_w64(moves) != 0ull) {
-        const float mn = moves ? mx : mrun;
-        const float alpha = moves ? __builtin_amdgcn_exp2f(mrun - mn) : 1.f;
-        mrun = mn;
-        lrun *= alpha;
-#pragma unroll
-        for (int m = 0; m < DV; ++m) o[m] *= alpha;
-      }
-      const float mu = mrun == kNegInfW ? 0.f : mrun;        // no visible key so far: every weight 0
-      float l0 = 0.f, l1 = 0.f;
-#pragma unroll
-      for (int i = 0; i < 8; i += 2) {
-        p[i] = __builtin_amdgcn_exp2f(p[i] - mu);
-        p[i + 1] = __builtin_amdgcn_exp2f(p[i + 1] - mu);
-        l0 += p[i];
-        l1 += p[i + 1];
-      }
-      lrun += l0 + l1;
-    }
-    s16x8 phi, plo;
-    split_bf16w(p, phi, plo);
-    constexpr int MG = DV % 4 == 0 ? 4 : 2;                  // value blocks taken together
-#pragma unroll
-    for (int m = 0; m < DV; m += MG) {
-      s16x8 v[MG];
-#pragma unroll
-      for (int u = 0; u < MG; ++u) {
-        const s16x4 a0 = rfq::ds_read_tr16(Vs + vat + 16 * (m + u));
-        const s16x4 a1 = rfq::ds_read_tr16(Vs + vat + 16 * VRS + 16 * (m + u));
-        v[u] = (s16x8){a0[0], a0[1], a0[2], a0[3], a1[0], a1[1], a1[2], a1[3]};
-      }
-#pragma unroll
-      for (int u = 0; u < MG; ++u)
-        o[m + u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(v[u]), as_bf16x8(phi), o[m + u], 0, 0, 0);
-#pragma unroll
-      for (int u = 0; u < MG; ++u)
-        o[m + u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(v[u]), as_bf16x8(plo), o[m + u], 0, 0, 0);
-    }
-    pg = pn;
-    if (pg <= pg_last) {
-      stage(pg * WBS, buf ^ 1);          // it has been on its way since the last page
-      pn = next_page(pg);
-      if (pn <= pg_last) fetch(bt[pn]);
-    }
+  };
+  auto passes = [&]() { return MODE == 1 ? cap2 - 2.f * cap2 * top : top; };   // this lane's largest score
+
+  auto landed = [] {
+    __builtin_amdgcn_s_waitcnt(0x0F70);                      // vmcnt(0)
     __syncthreads();
-    buf ^= 1;
+  };
+  // One turn: the weighted values of page i, whose scores p has, and the scores of page i + 1.  The order is
+  // kept piece by piece: products of the next page's scores beside the weights of this one, products of this
+  // page's values beside the next page's caps and maximum.
+  auto turn = [&](int i, auto next_c) {
+    constexpr bool NEXT = next_c;                            // there is a next page
+    const short* Kn = kpages + (SHARED ? (i + 1) % 3 : (i + 1) & 1) * KP;
+    const short* Vs = vpages + (SHARED ? i % 3 : i & 1) * VP;
+    // operands are read that many pieces ahead
+    constexpr int AK = DK > 4 ? 1 : 2, AV = AK;
+    s16x8 kc[AK], vc[AV];
+    if constexpr (NEXT) {
+#pragma unroll
+      for (int x = 0; x < AK; ++x) kc[x] = key(Kn, x);
+    }
+    const float mu = mrun == kNegInfW ? 0.f : mrun;          // no visible key so far: every weight 0
+    const float top0 = cap2 - mu;
+    u32x4 phi[2], plo[2];
+    // the weights of keys 2 e and 2 e + 1, in two steps
+    auto weigh = [&](int e) {
+      if constexpr (MODE < 2) {
+        p[2 * e] = __builtin_amdgcn_exp2f(MODE == 1 ? top0 - 2.f * cap2 * p[2 * e] : p[2 * e] - mu);
+        p[2 * e + 1] = __builtin_amdgcn_exp2f(MODE == 1 ? top0 - 2.f * cap2 * p[2 * e + 1] : p[2 * e + 1] - mu);
+      }
+    };
+    auto parts = [&](int e) {
+      const float x = p[2 * e], y = p[2 * e + 1];
+      if constexpr (MODE < 2) lrun += x + y;
+      const uint32_t h = rfq::pack_bf16x2(x, y);
+      phi[e >> 2][e & 3] = h;
+      plo[e >> 2][e & 3] = rfq::pack_bf16x2(x - __uint_as_float(h << 16), y - __uint_as_float(h & 0xffff0000u));
+    };
+    auto add = [&](const s16x8& v, int c, const u32x4& w) {
+      o[c % VM] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf16x8(v), __builtin_bit_cast(rfq::bf16x8, w), o[c % VM], 0, 0, 0);
+    };
+    f32x16 sn;
+    constexpr int C = 2 * VM;
+    if constexpr (NEXT) {
+#pragma unroll
+      for (int e = 0; e < 16; ++e) sn[e] = 0.f;
+      each<KS>([&](auto step) {
+        constexpr int ks = step, e0 = 8 * ks / KS, e1 = 8 * (ks + 1) / KS;
+        const s16x8 k = kc[ks % AK];
+        if constexpr (ks + AK < KS) kc[ks % AK] = key(Kn, ks + AK);
+        if constexpr (ks + AV >= KS) vc[ks + AV - KS] = value(Vs, ks + AV - KS);
+        sn = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf16x8(k), as_bf16x8(qhi[ks]), sn, 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+        each<e1 - e0>([&](auto e) { weigh(e0 + e); });
+        __builtin_amdgcn_sched_barrier(0);
+        sn = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf16x8(k), as_bf16x8(qlo[ks]), sn, 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+        each<e1 - e0>([&](auto e) { parts(e0 + e); });
+        __builtin_amdgcn_sched_barrier(0);
+      });
+    } else {
+#pragma unroll
+      for (int x = 0; x < AV; ++x) vc[x] = value(Vs, x);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) weigh(e);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) parts(e);
+    }
+    // two products a piece of values, the second beside the next piece's first; from the third product on the
+    // next page's scores are there
+    s16x8 before;
+    constexpr int Q = VM > 1 ? 4 * VM - 2 : 1;
+    auto some = [&](auto nc) {
+      if constexpr (NEXT) {
+        if constexpr (nc >= 0) {
+          constexpr int e0 = 16 * nc / Q, e1 = 16 * (nc + 1) / Q;
+          each<e1 - e0>([&](auto e) { prepare(e0 + e, sn[e0 + e]); });
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    };
+    each<C>([&](auto step) {
+      constexpr int c = step;
+      const s16x8 v = vc[c % AV];
+      if constexpr (c + AV < C) vc[c % AV] = value(Vs, c + AV);
+      if constexpr (VM == 1 && c > 0) {
+        add(before, c - 1, plo[(c - 1) / VM]);
+        some(std::integral_constant<int, 2 * c - 3>{});
+      }
+      add(v, c, phi[c / VM]);
+      some(std::integral_constant<int, 2 * c - 2>{});
+      if constexpr (VM > 1 && c > 0) {
+        add(before, c - 1, plo[(c - 1) / VM]);
+        some(std::integral_constant<int, 2 * c - 1>{});
+      }
+      before = v;
+    });
+    add(before, C - 1, plo[1]);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+
+  // K of page i + 1 and V of page i have landed for everyone, and everyone is done with K of page i and V of
+  // page i - 1, whose places the next ones take.
+  auto next = [&](int i) {
+    landed();
+    if (i + 2 < turns) fetch_k(n2, SHARED ? (i + 2) % 3 : i & 1);
+    fetch_v(n1, (i + 1) & 1);
+    n1 = n2;
+    n2 = number(i + 3);
+  };
+  // rows past the sequence's end were never written: zeros
+  auto last = [&]() {
+    landed();
+    const int jb = page_at(turns - 1) * WBS;
+    if (jb + WBS - 1 > plast) {
+      short* Vs = vpages + (SHARED ? (turns - 1) % 3 : (turns - 1) & 1) * VP;
+      for (int x = max(0, plast + 1 - jb) * (VR / 8) + tid; x < WBS * (VR / 8); x += NT)
+        *reinterpret_cast<s16x8*>(Vs + page_row<VR>(x / (VR / 8)) + x % (VR / 8) * 8) = (s16x8){0, 0, 0, 0, 0, 0, 0, 0};
+      __syncthreads();
+    }
+  };
+  landed();
+  {
+    f32x16 sc;
+#pragma unroll
+    for (int e = 0; e < 16; ++e) sc[e] = 0.f;
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) {
+      const s16x8 k = key(kpages, ks);
+      sc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf16x8(k), as_bf16x8(qhi[ks]), sc, 0, 0, 0);
+      sc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf16x8(k), as_bf16x8(qlo[ks]), sc, 0, 0, 0);
+    }
+#pragma unroll
+    for (int e = 0; e < 16; ++e) prepare(e, sc[e]);
+    mask(page_at(0) * WBS);
   }
-  store_rows<DV, MODE>(a, o, lrun, t, hh, grp, qlive);
+  int i = 0;
+  while (true) {
+    if constexpr (MODE < 2) {                                // the maximum moves; also for the first keys: mrun = -inf
+      const float mx = other_half_max(passes());
+      const bool moves = mx > mrun + kDeferW;
+      const float mn = moves ? mx : mrun;
+      const float alpha = moves ? __builtin_amdgcn_exp2f(mrun - mn) : 1.f;
+      mrun = mn;
+      lrun *= alpha;
+#pragma unroll
+      for (int m = 0; m < VM; ++m) o[m] *= alpha;
+    }
+    bool stays = true;
+    while (stays && i + 1 < turns) {
+      next(i);
+      turn(i, std::true_type{});
+      ++i;
+      mask(page_at(i) * WBS);
+      if constexpr (MODE < 2) stays = __builtin_amdgcn_ballot_w64(passes() > mrun + kDeferW) == 0ull;
+    }
+    if (stays) break;
+  }
+  last();
+  turn(i, std::false_type{});
+  store_rows32<VM, MODE>(a, o, lrun, t, hh, half, qlive);
 }
 
 // Wide latents: keys of 320 or 576 entries whose first 256 or 512 are the values.  32 queries' results
 // (256 registers at 512 values) and the queries themselves (144) leave no room for the rest, so a wave
 // has 16 queries on 16x16x32 tiles, two waves a head, and the page's LDS reads are what bounds it (K
 // rows 36 x 1 KB, V 64 x 512 B a wave and page: 4,350 clocks for eight waves against 3,200 of MFMA).
-// One prompt of 2,048 over 576 (32 heads) took 904 us a pass on the kernel above, 420 here; four of
-// them with 64 heads 3,249 and 1,402.  Pages come by LDS-DMA, the next one during this one; their rows lie unpadded, 16-byte pieces
+// One prompt of 2,048 over 576 (32 heads) took 904 us a pass on tiles with padded pages, 420 here; the attention of
+// four of them 1,262 us with a head's blocks one after the other, 968 with a block's heads side by side (the last
+// heads' long blocks started at seven eighths of the time).  Alone a workgroup takes 2.7 us a page.  One wave a SIMD
+// with 32 queries, half the LDS reads, took 3.2 us: it cannot issue what two can.  Pages come by LDS-DMA, the next one during this one; their rows lie unpadded, 16-byte pieces
 // permuted inside each 128 bytes by wide_swizzle(row).
 // DEC: decode rows.  A wave's columns are 16 heads of one row, so that a workgroup reads a page once for up to
 // 128 heads; the pages come one after another, which pays once every CU has a workgroup (launch_split_waves).
@@ -364,7 +541,10 @@ __global__ __launch_bounds__(128 * HPW, DEC && HPW == 1 ? 1 : 2) void attn_keep_
   constexpr int E = 32 * DK, vdim = 16 * DV, NWV = 2 * HPW, NP = WBS * E / 512, ND = (NP + NWV - 1) / NWV;
   constexpr bool QLO = DK <= 10;
   static_assert(E % 64 == 0 && DV % 4 == 0, "whole 128-byte lines");
-  const int item = gridDim.x - 1 - blockIdx.x;     // a sequence's later blocks see the most keys: they start first
+  // prompts: a block's workgroups lie side by side, a sequence's later blocks, which see the most keys, start first
+  constexpr int HW = DEC ? 16 * NWV : HPW;                    // heads of a workgroup
+  const int rep = a.H / a.G, per = (rep + HW - 1) / HW;       // workgroups of a key head, the last partly idle
+  const int at = gridDim.x - 1 - blockIdx.x, item = DEC ? at : at / (a.G * per), hg = DEC ? (int)blockIdx.y : at - item * a.G * per;
   const int s = DEC ? item : a.work_seq[item];
   if (s < 0) return;
   const int ql = a.q_len[s];
@@ -373,9 +553,7 @@ __global__ __launch_bounds__(128 * HPW, DEC && HPW == 1 ? 1 : 2) void attn_keep_
   const int tid = threadIdx.x, lane = tid & 63;
   const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int col = lane & 15, grp = lane >> 4;
-  constexpr int HW = DEC ? 16 * NWV : HPW;                    // heads of a workgroup
-  const int rep = a.H / a.G, per = (rep + HW - 1) / HW;       // workgroups of a key head, the last partly idle
-  const int g = (int)blockIdx.y / per, h0 = ((int)blockIdx.y - g * per) * HW;
+  const int g = hg / per, h0 = (hg - g * per) * HW;
   const int hd = DEC ? h0 + wid * 16 + col : h0 + (wid >> 1);
   const bool idle = DEC && h0 + wid * 16 >= rep;             // a wave that only copies pages
   const int hh = g * rep + min(hd, rep - 1);                 // past the last head: it once more, not stored
@@ -422,6 +600,7 @@ __global__ __launch_bounds__(128 * HPW, DEC && HPW == 1 ? 1 : 2) void attn_keep_
     const int p = (wid + i * NWV) * 64 + lane, r = p / (E / 8), c = p - r * (E / 8);
     src[i] = (r * E + ((c & ~7) | ((c & 7) ^ wide_swizzle(r))) * 8) * 2;
   }
+  const uint32_t lds0 = lds_byte(smem);
   auto fetch = [&](int page, int buf) {
     const char* kb = static_cast<const char*>(a.k_cache) + ((int64_t)page * a.G + g) * WBS * E * 2;
 #pragma unroll
@@ -430,8 +609,7 @@ __global__ __launch_bounds__(128 * HPW, DEC && HPW == 1 ? 1 : 2) void attn_keep_
       uint32_t at = src[i];
       asm("" : "+v"(at));      // widened here: hoisted out of the loop the offsets are pairs of registers, spilled
       if ((i + 1) * NWV <= NP || piece < NP)
-        rfq::glds16(reinterpret_cast<const bf16_t*>(kb + at),
-                    reinterpret_cast<bf16_t*>(pages + buf * WBS * E + piece * 512));
+        lds_copy16(kb, at, lds0 + 2 * (buf * WBS * E + piece * 512));
     }
   };
   // The page has landed for everyone, and everyone is done with the one before it, whose place the next
@@ -575,7 +753,7 @@ bool keep_mfma_ok(int E, int vdim, int BS, bool shared) {
 template <int DK, int DV, int HPW, bool SHARED, int MODE>
 static void launch_keep_mfma_one(const KeepArgs& a) {
   constexpr bool WIDE = SHARED && DK >= 10;
-  constexpr size_t lds = (size_t)2 * (WIDE ? WBS * 32 * DK : keep_page_shorts<DK, DV, SHARED>()) * sizeof(short);
+  constexpr size_t lds = (size_t)(WIDE ? 2 * WBS * 32 * DK : tile_lds_shorts<DK, DV, SHARED>()) * sizeof(short);
   static_assert(lds <= 160 * 1024, "LDS of a CU");
   static bool attr = false;
   auto run = [&](auto kernel, int threads) {
@@ -585,10 +763,16 @@ static void launch_keep_mfma_one(const KeepArgs& a) {
       attr = true;
     }
     const int rep = a.H / a.G;
-    hipLaunchKernelGGL(kernel, dim3(a.W, a.G * ((rep + HPW - 1) / HPW)), dim3(threads), lds, a.s, a);
+    const int groups = a.G * ((rep + HPW - 1) / HPW), most = std::max(1, (1 << 22) / groups);   // threads in 32 bits
+    for (int w = 0; w < a.W; w += most) {
+      KeepArgs part = a;
+      part.work_seq += w;
+      part.work_qblk += w;
+      hipLaunchKernelGGL(kernel, dim3((unsigned)std::min(most, a.W - w) * groups), dim3(threads), lds, a.s, part);
+    }
   };
   if constexpr (WIDE) run(&attn_keep_wide_kernel<DK, DV, HPW, MODE, false>, 128 * HPW);
-  else run(&attn_keep_mfma_kernel<DK, DV, HPW, SHARED, MODE>, 128 * HPW);
+  else run(&attn_keep_tile_kernel<DK, DV, HPW, SHARED, MODE>, 64 * HPW);
 }
 
 template <int DK, int DV, int HPW, bool SHARED>

@@ -108,6 +108,15 @@ def test_prompt_rows(H, G, E, vd, shared):
     _check(H, G, E, vd, shared, seqs=PROMPTS, prompt=True, window=64, keep_first=40)
 
 
+@pytest.mark.parametrize("H,G,E,vd,shared", [(4, 1, 128, 128, False), (2, 1, 64, 64, False), (1, 1, 32, 32, False),
+                                             (4, 1, 96, 64, True), (2, 1, 192, 128, True), (4, 1, 576, 512, True)])
+def test_long_chains_of_pages(H, G, E, vd, shared):
+    """More pages than any buffer holds, odd and even numbers of them, short blocks beside long ones."""
+    seqs = [(1100, 40), (991, 33), (640, 64), (97, 97)]
+    _check(H, G, E, vd, shared, seqs=seqs, prompt=True, softcap=20.0)
+    _check(H, G, E, vd, shared, seqs=seqs, prompt=True, window=400, keep_first=70, sigmoid=True, bias=True)
+
+
 def test_prompt_rows_with_rising_scores():
     """Every page moves the maximum by far: the accumulators are rescaled each time."""
     for shared, E, vd in ((False, 128, 128), (True, 576, 512)):
