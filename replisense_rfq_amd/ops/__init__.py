@@ -6,6 +6,7 @@ if it cannot be.  CPU tensors use :mod:`.reference` (tests / CPU engine).
 """
 from __future__ import annotations
 
+import functools
 import os
 
 import torch
@@ -502,9 +503,47 @@ def qkv_rope(x, w, positions, cos_sin, slot_mapping, k_cache, v_cache, Hq, Hkv):
                 _native.ops().skinny_gemm_rope(x, w, qkv, positions, cos_sin, slot_mapping,
                                                k_cache, v_cache, Hq, Hkv, cfg)
             return qkv
-    qkv = linear(x, w)
+    head = _round_rows(x, w)
+    if head > 0:
+        qkv = torch.empty((x.shape[0], w.shape[0]), dtype=x.dtype, device=x.device)
+        torch.matmul(x[:head], w.t(), out=qkv[:head])
+        torch.matmul(x[head:], w.t(), out=qkv[head:])
+    else:
+        qkv = linear(x, w)
     rope_kv(qkv, positions, cos_sin, slot_mapping, k_cache, v_cache, Hq, Hkv)
     return qkv
+
+
+@functools.lru_cache(maxsize=None)
+def _cus(index: int) -> int:
+    return torch.cuda.get_device_properties(index).multi_processor_count
+
+
+def _round_rows(x, w) -> int:
+    """Rows of x w^T that make whole rounds of 256 x 256 tiles over the chip, where the library takes
+    less time for them and for the others than for all of them; 0 where it does not, or where a
+    start-up plan, a tiled copy or a derivative has the word.
+
+    The library gives a grid that does not fill its last round tiles of another size, or half a chip of
+    work: 2,767 rows by 6,144 x 4,096 take 210 us, 2,560 of them 85 and the others 24.  Up to half a
+    round beyond the first one the two products were faster for all three classes of decoders, by 0 - 84
+    percent (3,072 x 2,048: 5,377 rows 71 -> 60 us, 8,064: 86 -> 84; 6,144 x 4,096: 2,561: 115 -> 103, 3,840:
+    153 -> 153; 10,240 x 8,192: 1,537: 244 -> 202, 2,304: 308 -> 291); beyond it they are even or lose (6,144 x
+    4,096: 4,385 rows 168 and 170).  After more rounds they lose with up to 4,096 terms (5,300 rows: 183 and
+    203), and gain with 8,192 up to seven tenths after two to four (10,240 x 8,192: 3,742 rows 641 -> 455, 4,826:
+    778 -> 578, 6,556: 927 -> 769), not after five (7,764: 870 and 911)."""
+    M, N, K = x.shape[0], w.shape[0], x.shape[1]
+    if (not _gpu(x) or x.dtype != torch.bfloat16 or w.dtype != torch.bfloat16 or N % 256 != 0 or N == 0 or K < 2048
+            or x.stride(1) != 1 or w.stride(1) != 1 or (N, K) in _SPLIT_PLAN or tiled_only(w)
+            or linear_plan(M, N, K) >= 0 or not _plain(x, w)):
+        return 0
+    per = _cus(x.device.index) // (N // 256) * 256           # rows of a round
+    if per == 0:
+        return 0
+    rounds, rest = M // per, M % per
+    if rest and ((rounds == 1 and 2 * rest <= per) or (K >= 8192 and 2 <= rounds <= 4 and 10 * rest <= 7 * per)):
+        return rounds * per
+    return 0
 
 
 def attn_decode_merge(part_o, part_ml, out, Hq, num_splits):

@@ -1209,3 +1209,27 @@ def test_linear_zero_rows_with_rows_plan(gpu):
         _close(ops.linear(x1, w), x1.float() @ w.float().t(), atol=2e-2, rtol=2e-2, what="M=1 rows")
     finally:
         ops.reset_plans()
+
+
+@pytest.mark.parametrize("M,parts", [(2560, 1), (2561, 2), (3840, 2), (3841, 1)])
+def test_qkv_rope_in_two_products(M, parts):
+    """Steps just over a whole round of the library's tiles take two products: the same rows and caches."""
+    Hq, Hkv, K = 32, 8, 2048
+    N = (Hq + 2 * Hkv) * 128
+    g = torch.Generator().manual_seed(M)
+    x = torch.randn(M, K, generator=g).to("cuda", torch.bfloat16)
+    w = (torch.randn(N, K, generator=g) * K ** -0.5).to("cuda", torch.bfloat16)
+    ops.reset_plans()
+    assert ops._round_rows(x, w) == (2560 if parts == 2 else 0) or ops._cus(0) != 256
+    pos = torch.arange(M, dtype=torch.int32, device="cuda") % 512
+    ang = torch.arange(512)[:, None] * 1e4 ** (-torch.arange(0, 128, 2) / 128)
+    cs = torch.cat([ang.cos(), ang.sin()], -1).float().cuda()
+    slots = torch.randperm(4096, generator=g)[:M].to("cuda", torch.int32)
+    kc, vc, kr, vr = (torch.zeros(128, Hkv, 32, 128, dtype=torch.bfloat16, device="cuda") for _ in range(4))
+    got = ops.qkv_rope(x, w, pos, cs, slots, kc, vc, Hq, Hkv)
+    want = (x.float() @ w.float().t()).bfloat16()
+    ops.rope_kv(want, pos, cs, slots, kr, vr, Hq, Hkv)
+    for a, b in ((got[:, :Hq * 128], want[:, :Hq * 128]), (kc, kr), (vc, vr)):
+        # both round a product of unit variance to bf16, the rotation's result once more: a spacing each
+        assert float((a.float() - b.float()).abs().max()) <= 3 * 2.0 ** -8 * float(b.float().abs().max())
+        assert float((a.float() - b.float()).norm() / b.float().norm()) <= 2.0 ** -8
