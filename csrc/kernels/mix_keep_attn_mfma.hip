@@ -531,10 +531,12 @@ __global__ __launch_bounds__(64 * HPW, 2) void attn_keep_tile_kernel(const KeepA
 // 128 heads; the pages come one after another, which pays once every CU has a workgroup (launch_split_waves).
 // 256 sequences of 300 tokens with 64 heads of 576 entries 44 us, 32 of 500 with four rows each 50; split over
 // waves 116 and 129.
-// Sixteen rows of one piece (a K read) and four neighbouring rows of a pair of pieces beside the next
-// four (a transposed V read) then lie on different banks: the row's parity picks a half of them, bits
-// 1 and 2 the pair, bit 3 the order inside it.
-__device__ __forceinline__ int wide_swizzle(int r) { return ((r >> 1) & 1) << 2 | ((r >> 2) & 1) << 1 | ((r >> 3) & 1); }
+// Pieces that one LDS access takes together then lie on different banks: of a K read rows 0..3 and 12..15 of one
+// piece with rows 4..11 of its neighbour, or the other way round (sixteen rows of one piece are not what it takes: a
+// permutation that parts those alone cost 1,150 clocks a page of eight waves), of a transposed V read four
+// neighbouring rows of a pair of pieces beside the next four.  The row's parity picks a half of the banks, bit 1 the
+// half of that, the row's quad the order inside it.
+__device__ __forceinline__ int wide_swizzle(int r) { return ((r >> 1) & 1) << 2 | ((4 - (r >> 2)) & 3); }
 
 template <int DK, int DV, int HPW, int MODE, bool DEC>
 __global__ __launch_bounds__(128 * HPW, DEC && HPW == 1 ? 1 : 2) void attn_keep_wide_kernel(const KeepArgs a) {
