@@ -93,6 +93,11 @@ void launch_attn_keep_split(const float*, const void*, const void*, int64_t, con
                             const int32_t*, const int32_t*, int, int, int, const float*, const void*, int64_t, int,
                             void*, int64_t, float, int, int, bool, int, int, int, int, bool, float, float,
                             hipStream_t);
+int keep_streams(int, int, int, int, int, int, bool, int);
+int64_t keep_streams_floats(int, int, int, int);
+void launch_attn_keep_streams(const float*, const void*, int64_t, const int32_t*, int, const int32_t*, const int32_t*,
+                              const int32_t*, int, int, int, const float*, const void*, int64_t, int, void*, int64_t, float,
+                              int, int, bool, int, int, float, float, float*, hipStream_t);
 bool launch_attn_keep_mfma(const float*, const void*, const void*, int64_t, const int32_t*, int,
                            const int32_t*, const int32_t*, const int32_t*, const int32_t*,
                            const int32_t*, int, const float*, const void*, int64_t, int, void*,
@@ -839,7 +844,16 @@ void attn_keep_window(const Tensor& q, const Tensor& k_cache, const Tensor& v_ca
                      (gw == 1 || (gs % 4 == 0 && reinterpret_cast<uintptr_t>(gp) % 8 == 0));
   TORCH_CHECK(short_rows >= 0 && short_rows <= 65535 && G <= 65535, "attn_keep_window: short_rows");
   if (short_rows > 0 && tiles) {
-    // sequences of at most short_rows rows each (decode section): their pages split over waves
+    // sequences of at most short_rows rows each (decode section): their pages split over waves, or over
+    // workgroups, whose parts meet in scratch memory
+    if (const int S = rfqmix::keep_streams(T, NB, H, G, E, (int)vdim, shared, (int)bt.size(1)); S > 0 && T > 0) {
+      const Tensor part = at::empty({rfqmix::keep_streams_floats(T, S, H, (int)vdim)}, q.options());
+      return rfqmix::launch_attn_keep_streams(
+          f32p(q, "q"), k_cache.data_ptr(), vrs, i32p(bt, "block_tables", 0), (int)bt.size(1),
+          i32p(q_start, "q_start", NB), i32p(q_len, "q_len", NB), i32p(kv_len, "kv_len", NB), T, NB, S, hb, gp, gs, gw,
+          out.data_ptr(), out.stride(0), (float)scale, (int)window, (int)keep_first, sigmoid, H, G, (float)softcap,
+          (float)out_mult, part.data_ptr<float>(), stream());
+    }
     return rfqmix::launch_attn_keep_split(
         f32p(q, "q"), k_cache.data_ptr(), v_cache.data_ptr(), vrs, i32p(bt, "block_tables", 0),
         (int)bt.size(1), i32p(q_start, "q_start", NB), i32p(q_len, "q_len", NB), i32p(kv_len, "kv_len", NB),

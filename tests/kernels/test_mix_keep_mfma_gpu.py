@@ -94,6 +94,20 @@ def test_a_key_outside_the_window_may_hold_infinities():
     _check(16, 1, 576, 512, True, seqs=seqs, spoil=20, window=64, keep_first=4)
 
 
+# a row a sequence on the average: pages around the streams of one and of several workgroups
+STREAMS = [(1, 1), (32, 1), (33, 1), (128, 1), (129, 1), (300, 2), (40, 0), (512, 1), (513, 1), (700, 1), (1500, 1)]
+
+
+@pytest.mark.parametrize("H,G", [(17, 1), (32, 1), (33, 1), (64, 1), (48, 2)])
+def test_wide_rows_in_streams(H, G):
+    _check(H, G, 576, 512, True, seqs=STREAMS, bias=True, gate="head")
+    _check(H, G, 576, 512, True, seqs=STREAMS, softcap=20.0, out_mult=0.6, gate="output")
+    _check(H, G, 576, 512, True, seqs=STREAMS[5:], window=100, keep_first=40, spoil=50, bias=True)   # no row sees 50
+    _check(H, G, 576, 512, True, seqs=STREAMS, window=64, keep_first=5, sigmoid=True, bias=True)
+    _check(H, G, 576, 512, True, seqs=STREAMS[4:5], sigmoid=True, softcap=15.0, bias=True)
+    _check(H, G, 576, 512, True, seqs=STREAMS[-1:])
+
+
 PROMPTS = [(1, 1), (31, 31), (32, 32), (33, 33), (100, 70), (300, 45), (40, 0), (161, 97)]
 
 
