@@ -524,9 +524,10 @@ __global__ __launch_bounds__(64 * HPW, 2) void attn_keep_tile_kernel(const KeepA
 // rows 36 x 1 KB, V 64 x 512 B a wave and page: 4,350 clocks for eight waves against 3,200 of MFMA).
 // One prompt of 2,048 over 576 (32 heads) took 904 us a pass on tiles with padded pages, 420 here; the attention of
 // four of them 1,262 us with a head's blocks one after the other, 968 with a block's heads side by side (the last
-// heads' long blocks started at seven eighths of the time).  Alone a workgroup takes 2.7 us a page.  One wave a SIMD
-// with 32 queries, half the LDS reads, took 3.2 us: it cannot issue what two can.  Pages come by LDS-DMA, the next one during this one; their rows lie unpadded, 16-byte pieces
-// permuted inside each 128 bytes by wide_swizzle(row).
+// heads' long blocks started at seven eighths of the time), 948 without conflicts in the key reads.  Alone a workgroup
+// takes 2.7 us a page.  One wave a SIMD with 32 queries, half the LDS reads, took 3.2 us: it cannot issue what two
+// can.  Pages come by LDS-DMA, the next one during this one; their rows lie unpadded, 16-byte pieces permuted inside
+// each 128 bytes by wide_swizzle(row).
 // DEC: decode rows.  A wave's columns are 16 heads of one row, so that a workgroup reads a page once for up to
 // 128 heads; the pages come one after another, which pays once every CU has a workgroup (launch_split_waves).
 // 256 sequences of 300 tokens with 64 heads of 576 entries 44 us, 32 of 500 with four rows each 50; split over
