@@ -739,7 +739,7 @@ __global__ __launch_bounds__(128 * HPW, DEC && HPW == 1 ? 1 : 2) void attn_keep_
   }
 }
 
-// Decode rows of a wide latent with more than 16 heads a key head, few sequences: a sequence's pages are shared by
+// Decode rows of a wide latent with more than 16 heads a key head, few sequences: a row's pages are shared by
 // S workgroups of four streams, a stream being two waves (16 heads each) and a page of its own in LDS.  Streams meet
 // in LDS, workgroups in attn_keep_streams_merge_kernel, by way of `part` ([T, S, H] of vdim weighted values each,
 // then as many pairs of maximum, in base 2, and sum; -inf: no key).
@@ -752,11 +752,26 @@ __global__ __launch_bounds__(128 * HPW, DEC && HPW == 1 ? 1 : 2) void attn_keep_
 // one of 611 37 -> 21, eight of 2,000 90 -> 29, 64 of 2,000 95 -> 51, 32 of 600 with 64 heads 40 -> 32.
 constexpr int kStreams = 4;
 
+// The sequence that has row t of the step, -1: none (rows of a captured step beyond those of its sequences).  A row a
+// sequence, as most steps have it, is seen at once.
+__device__ __forceinline__ int row_owner(const int32_t* q_start, const int32_t* q_len, int NA, int t) {
+  if (t < NA && q_start[t] == t && q_len[t] > 0) return t;
+  for (int b = 0; b < NA; b += 64) {
+    const int i = b + (threadIdx.x & 63), from = i < NA ? q_start[i] : 0, n = i < NA ? q_len[i] : 0;
+    const uint64_t m = __builtin_amdgcn_ballot_w64(from <= t && t < from + n);
+    if (m != 0) return b + __builtin_ctzll(m);
+  }
+  return -1;
+}
+
 template <int DK, int DV, int MODE>
-__global__ __launch_bounds__(128 * kStreams, 2) void attn_keep_streams_kernel(const KeepArgs a, float* part, int T) {
+__global__ __launch_bounds__(128 * kStreams, 2) void attn_keep_streams_kernel(const KeepArgs a, float* part, int T,
+                                                                                int NA) {
   constexpr int E = 32 * DK, vdim = 16 * DV, PGS = WBS * E, ND = WBS * E / 1024, S16 = vdim / 2 + 4;
   static_assert(DK > 10 && E % 64 == 0 && WBS * E % 1024 == 0 && 2 * kStreams * 16 * S16 * 4 <= kStreams * PGS * 2, "the partial results take the pages' place");
-  const int s = blockIdx.x, ql = a.q_len[s];
+  const int64_t t = blockIdx.x;
+  const int s = row_owner(a.q_start, a.q_len, NA, (int)t);
+  if (s < 0) return;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wid = __builtin_amdgcn_readfirstlane(tid >> 6), st = wid >> 1;
   const int col = lane & 15, grp = lane >> 4;
@@ -780,257 +795,253 @@ __global__ __launch_bounds__(128 * kStreams, 2) void attn_keep_streams_kernel(co
   const float hb = MODE >= 2 && a.head_bias != nullptr ? a.head_bias[hh] * kLog2e : 0.f;
   const int ksw = wide_swizzle(col), vrow = 4 * grp + (col >> 2), vsw = wide_swizzle(vrow);
 
-  for (int r = 0; r < ql; ++r) {
-    const int pi = a.kv_len[s] - ql + r;                      // the row's query
-    const int window = a.window;
-    const int jwin = window > 0 ? max(0, pi - window + 1) : 0;
-    const int kf = window > 0 ? min(a.keep_first, jwin) : 0;
-    const int64_t t = a.q_start[s] + r;
-    // pages [0, n_keep) hold the kept first tokens, pages [pg_win, pg_last] the window
-    const int pg_last = pi / WBS, pg_win = jwin / WBS;
-    const int n_keep = min((kf + WBS - 1) / WBS, pg_win), skip = pg_win - n_keep, pages = pg_last + 1 - skip;
-    const int turns = max(0, (pages - z * kStreams + S * kStreams - 1) / (S * kStreams));
-    constexpr int NQ = (DK + kStreams - 1) / kStreams;
-    float4 qx[NQ], qy[NQ];                                    // on their way before the page is
-    {
-      const float* qp = a.q + (t * a.H + hh) * E + grp * 8;
-#pragma unroll
-      for (int x = 0; x < NQ; ++x) {
-        const int ks = min(x * kStreams + st, DK - 1);
-        qx[x] = *reinterpret_cast<const float4*>(qp + ks * 32);
-        qy[x] = *reinterpret_cast<const float4*>(qp + ks * 32 + 4);
-      }
-    }
-    auto offset = [&](int x, int l) {                         // bytes from the page's first, of load x of this wave
-      const int p = ((wid & 1) + 2 * x) * 64 + l, rw = p / (E / 8), c = p - rw * (E / 8);
-      return (uint32_t)(rw * E + ((c & ~7) | ((c & 7) ^ wide_swizzle(rw))) * 8) * 2;
-    };
-    auto page_at = [&](int i) {
-      return static_cast<const char*>(a.k_cache) + ((int64_t)bt[i < n_keep ? i : i + skip] * a.G + g) * PGS * 2;
-    };
-    {
-      uint32_t from[ND];                                      // computed while the page's number is on its way
-      int l = lane;
-      asm volatile("" : "+v"(l));                             // and here: before the loop they would be spilled
-#pragma unroll
-      for (int x = 0; x < ND; ++x) {
-        from[x] = offset(x, l);
-        asm volatile("" : "+v"(from[x]));
-      }
-      if (z * kStreams + st < pages) {
-        const char* kb = page_at(z * kStreams + st);
-#pragma unroll
-        for (int x = 0; x < ND; ++x)
-          rfq::glds16(reinterpret_cast<const bf16_t*>(kb + from[x]), reinterpret_cast<bf16_t*>(P + ((wid & 1) + 2 * x) * 512));
-      }
-    }
-    auto fetch = [&](int i) {
-      const char* kb = page_at(i);
-      int l = lane;
-      asm volatile("" : "+v"(l));                             // the offsets are computed here, not kept
-#pragma unroll
-      for (int x = 0; x < ND; ++x)
-        rfq::glds16(reinterpret_cast<const bf16_t*>(kb + offset(x, l)), reinterpret_cast<bf16_t*>(P + ((wid & 1) + 2 * x) * 512));
-    };
-    // a stream packs every fourth piece of the queries and leaves it for the others
-    s16x8 q[DK];
+  const int pi = a.kv_len[s] - a.q_len[s] + (int)t - a.q_start[s];     // the row's query
+  const int window = a.window;
+  const int jwin = window > 0 ? max(0, pi - window + 1) : 0;
+  const int kf = window > 0 ? min(a.keep_first, jwin) : 0;
+  // pages [0, n_keep) hold the kept first tokens, pages [pg_win, pg_last] the window
+  const int pg_last = pi / WBS, pg_win = jwin / WBS;
+  const int n_keep = min((kf + WBS - 1) / WBS, pg_win), skip = pg_win - n_keep, pages = pg_last + 1 - skip;
+  const int turns = max(0, (pages - z * kStreams + S * kStreams - 1) / (S * kStreams));
+  constexpr int NQ = (DK + kStreams - 1) / kStreams;
+  float4 qx[NQ], qy[NQ];                                    // on their way before the page is
+  {
+    const float* qp = a.q + (t * a.H + hh) * E + grp * 8;
 #pragma unroll
     for (int x = 0; x < NQ; ++x) {
-      const float f[8] = {qx[x].x, qx[x].y, qx[x].z, qx[x].w, qy[x].x, qy[x].y, qy[x].z, qy[x].w};
-      if (x > 0) __syncthreads();
-      *reinterpret_cast<s16x8*>(qs + ((wid & 1) * kStreams + st) * 1024 + lane * 16) = rfq::pack8(f);
-      __syncthreads();
-#pragma unroll
-      for (int u = 0; u < kStreams; ++u)
-        if (x * kStreams + u < DK)
-          q[x * kStreams + u] = *reinterpret_cast<const s16x8*>(qs + ((wid & 1) * kStreams + u) * 1024 + lane * 16);
+      const int ks = min(x * kStreams + st, DK - 1);
+      qx[x] = *reinterpret_cast<const float4*>(qp + ks * 32);
+      qy[x] = *reinterpret_cast<const float4*>(qp + ks * 32 + 4);
     }
-    f32x4 o[DV];
+  }
+  auto offset = [&](int x, int l) {                         // bytes from the page's first, of load x of this wave
+    const int p = ((wid & 1) + 2 * x) * 64 + l, rw = p / (E / 8), c = p - rw * (E / 8);
+    return (uint32_t)(rw * E + ((c & ~7) | ((c & 7) ^ wide_swizzle(rw))) * 8) * 2;
+  };
+  auto page_at = [&](int i) {
+    return static_cast<const char*>(a.k_cache) + ((int64_t)bt[i < n_keep ? i : i + skip] * a.G + g) * PGS * 2;
+  };
+  {
+    uint32_t from[ND];                                      // computed while the page's number is on its way
+    int l = lane;
+    asm volatile("" : "+v"(l));                             // and here: before the loop they would be spilled
 #pragma unroll
-    for (int m = 0; m < DV; ++m) o[m] = (f32x4){0.f, 0.f, 0.f, 0.f};
-    float mrun = kNegInfW, lrun = 0.f;
-    for (int k = 0; k < turns; ++k) {
-      const int i = (k * S + z) * kStreams + st, jb = (i < n_keep ? i : i + skip) * WBS;
-      const bool live = i < pages;
-      __builtin_amdgcn_s_waitcnt(0x0F70);                     // vmcnt(0)
-      __syncthreads();
-      // rows past the query were never written, rows out of its sight may hold infinities: zeros
-      const bool edge = live && (jb + WBS - 1 > pi || (jb < jwin && jb + WBS > kf));
-      if (edge)
-        for (int x = (wid & 1) * 64 + lane; x < WBS * (E / 8); x += 128) {
-          const int j = jb + x / (E / 8);
-          if (j > pi || (j < jwin && j >= kf)) *reinterpret_cast<s16x8*>(P + x * 8) = (s16x8){0, 0, 0, 0, 0, 0, 0, 0};
+    for (int x = 0; x < ND; ++x) {
+      from[x] = offset(x, l);
+      asm volatile("" : "+v"(from[x]));
+    }
+    if (z * kStreams + st < pages) {
+      const char* kb = page_at(z * kStreams + st);
+#pragma unroll
+      for (int x = 0; x < ND; ++x)
+        rfq::glds16(reinterpret_cast<const bf16_t*>(kb + from[x]), reinterpret_cast<bf16_t*>(P + ((wid & 1) + 2 * x) * 512));
+    }
+  }
+  auto fetch = [&](int i) {
+    const char* kb = page_at(i);
+    int l = lane;
+    asm volatile("" : "+v"(l));                             // the offsets are computed here, not kept
+#pragma unroll
+    for (int x = 0; x < ND; ++x)
+      rfq::glds16(reinterpret_cast<const bf16_t*>(kb + offset(x, l)), reinterpret_cast<bf16_t*>(P + ((wid & 1) + 2 * x) * 512));
+  };
+  // a stream packs every fourth piece of the queries and leaves it for the others
+  s16x8 q[DK];
+#pragma unroll
+  for (int x = 0; x < NQ; ++x) {
+    const float f[8] = {qx[x].x, qx[x].y, qx[x].z, qx[x].w, qy[x].x, qy[x].y, qy[x].z, qy[x].w};
+    if (x > 0) __syncthreads();
+    *reinterpret_cast<s16x8*>(qs + ((wid & 1) * kStreams + st) * 1024 + lane * 16) = rfq::pack8(f);
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < kStreams; ++u)
+      if (x * kStreams + u < DK)
+        q[x * kStreams + u] = *reinterpret_cast<const s16x8*>(qs + ((wid & 1) * kStreams + u) * 1024 + lane * 16);
+  }
+  f32x4 o[DV];
+#pragma unroll
+  for (int m = 0; m < DV; ++m) o[m] = (f32x4){0.f, 0.f, 0.f, 0.f};
+  float mrun = kNegInfW, lrun = 0.f;
+  for (int k = 0; k < turns; ++k) {
+    const int i = (k * S + z) * kStreams + st, jb = (i < n_keep ? i : i + skip) * WBS;
+    const bool live = i < pages;
+    __builtin_amdgcn_s_waitcnt(0x0F70);                     // vmcnt(0)
+    __syncthreads();
+    // rows past the query were never written, rows out of its sight may hold infinities: zeros
+    const bool edge = live && (jb + WBS - 1 > pi || (jb < jwin && jb + WBS > kf));
+    if (edge)
+      for (int x = (wid & 1) * 64 + lane; x < WBS * (E / 8); x += 128) {
+        const int j = jb + x / (E / 8);
+        if (j > pi || (j < jwin && j >= kf)) *reinterpret_cast<s16x8*>(P + x * 8) = (s16x8){0, 0, 0, 0, 0, 0, 0, 0};
+      }
+    __syncthreads();
+    if (live && !idle) {
+      f32x4 sc[2][2];                                       // two chains per half page
+#pragma unroll
+      for (int kt = 0; kt < 2; ++kt) {
+        sc[kt][0] = sc[kt][1] = (f32x4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int ks = 0; ks < DK; ++ks) {
+          const s16x8 kv = *reinterpret_cast<const s16x8*>(P + col * E + ((4 * (ks & 1) + grp) ^ ksw) * 8 + kt * 16 * E + (ks >> 1) * 64);
+          f32x4& acc = sc[kt][ks & 1];
+          acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(kv), as_bf16x8(q[ks]), acc, 0, 0, 0);
         }
-      __syncthreads();
-      if (live && !idle) {
-        f32x4 sc[2][2];                                       // two chains per half page
+      }
+      float p[8];
 #pragma unroll
-        for (int kt = 0; kt < 2; ++kt) {
-          sc[kt][0] = sc[kt][1] = (f32x4){0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-          for (int ks = 0; ks < DK; ++ks) {
-            const s16x8 kv = *reinterpret_cast<const s16x8*>(P + col * E + ((4 * (ks & 1) + grp) ^ ksw) * 8 + kt * 16 * E + (ks >> 1) * 64);
-            f32x4& acc = sc[kt][ks & 1];
-            acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(kv), as_bf16x8(q[ks]), acc, 0, 0, 0);
-          }
-        }
-        float p[8];
+      for (int e = 0; e < 8; ++e) {
+        float x = (sc[e >> 2][0][e & 3] + sc[e >> 2][1][e & 3]) * qmul;
+        if constexpr (MODE % 2 == 1) x = cap2 - 2.f * cap2 * __builtin_amdgcn_rcpf(__builtin_amdgcn_exp2f(x) + 1.f);
+        if constexpr (MODE >= 2) x = __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f((MODE == 3 ? -x : x) - hb));
+        p[e] = x;
+      }
+      if (edge) {
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
-          float x = (sc[e >> 2][0][e & 3] + sc[e >> 2][1][e & 3]) * qmul;
-          if constexpr (MODE % 2 == 1) x = cap2 - 2.f * cap2 * __builtin_amdgcn_rcpf(__builtin_amdgcn_exp2f(x) + 1.f);
-          if constexpr (MODE >= 2) x = __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f((MODE == 3 ? -x : x) - hb));
-          p[e] = x;
-        }
-        if (edge) {
-#pragma unroll
-          for (int e = 0; e < 8; ++e) {
-            const int j = jb + (e >> 2) * 16 + grp * 4 + (e & 3);
-            const bool ok = (j <= pi) & ((j >= jwin) | (j < kf));
-            p[e] = ok ? p[e] : MODE >= 2 ? 0.f : kNegInfW;
-          }
-        }
-        if constexpr (MODE < 2) {
-          float mx = fmaxf(fmaxf(fmaxf(p[0], p[1]), fmaxf(p[2], p[3])), fmaxf(fmaxf(p[4], p[5]), fmaxf(p[6], p[7])));
-          mx = other_half_max(other_row_max(mx));
-          const bool moves = mx > mrun + kDeferW;             // also for the first keys: mrun = -inf
-          if (__builtin_amdgcn_ballot_w64(moves) != 0ull) {
-            const float mn = moves ? mx : mrun;
-            const float alpha = moves ? __builtin_amdgcn_exp2f(mrun - mn) : 1.f;
-            mrun = mn;
-            lrun *= alpha;
-#pragma unroll
-            for (int m = 0; m < DV; ++m) o[m] *= alpha;
-          }
-          const float mu = mrun == kNegInfW ? 0.f : mrun;     // no visible key so far: every weight 0
-          float l0 = 0.f, l1 = 0.f;
-#pragma unroll
-          for (int e = 0; e < 8; e += 2) {
-            p[e] = __builtin_amdgcn_exp2f(p[e] - mu);
-            p[e + 1] = __builtin_amdgcn_exp2f(p[e + 1] - mu);
-            l0 += p[e];
-            l1 += p[e + 1];
-          }
-          lrun += l0 + l1;
-        }
-        s16x8 phi, plo;
-        split_bf16w(p, phi, plo);
-#pragma unroll
-        for (int m = 0; m < DV; m += 4) {
-          s16x8 v[4];
-#pragma unroll
-          for (int u = 0; u < 4; ++u) {
-            const short* vp = P + vrow * E + ((2 * u + ((col >> 1) & 1)) ^ vsw) * 8 + (col & 1) * 4 + (m >> 2) * 64;
-            const s16x4 a0 = rfq::ds_read_tr16(vp), a1 = rfq::ds_read_tr16(vp + 16 * E);
-            v[u] = (s16x8){a0[0], a0[1], a0[2], a0[3], a1[0], a1[1], a1[2], a1[3]};
-          }
-#pragma unroll
-          for (int u = 0; u < 4; ++u)
-            o[m + u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(v[u]), as_bf16x8(phi), o[m + u], 0, 0, 0);
-#pragma unroll
-          for (int u = 0; u < 4; ++u)
-            o[m + u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(v[u]), as_bf16x8(plo), o[m + u], 0, 0, 0);
+          const int j = jb + (e >> 2) * 16 + grp * 4 + (e & 3);
+          const bool ok = (j <= pi) & ((j >= jwin) | (j < kf));
+          p[e] = ok ? p[e] : MODE >= 2 ? 0.f : kNegInfW;
         }
       }
-      __syncthreads();                                        // both waves are done with the page
-      if (const int n = i + S * kStreams; n < pages) fetch(n);
-    }
-    // ---- streams meet, half the channels at a time
-    const float l = both_halves_sum(both_rows_sum(lrun));
-    if (grp == 0) {
-      // scores that are no numbers leave the maximum at -inf, which marks a stream without visible keys
-      ml[wid * 16 + col] = MODE >= 2 ? (turns > 0 ? 0.f : kNegInfW) : l != 0.f && mrun == kNegInfW ? 0.f : mrun;
-      ml[(2 * kStreams + wid) * 16 + col] = l;
-    }
-    float* const part_ml = part + (int64_t)T * S * a.H * vdim;
+      if constexpr (MODE < 2) {
+        float mx = fmaxf(fmaxf(fmaxf(p[0], p[1]), fmaxf(p[2], p[3])), fmaxf(fmaxf(p[4], p[5]), fmaxf(p[6], p[7])));
+        mx = other_half_max(other_row_max(mx));
+        const bool moves = mx > mrun + kDeferW;             // also for the first keys: mrun = -inf
+        if (__builtin_amdgcn_ballot_w64(moves) != 0ull) {
+          const float mn = moves ? mx : mrun;
+          const float alpha = moves ? __builtin_amdgcn_exp2f(mrun - mn) : 1.f;
+          mrun = mn;
+          lrun *= alpha;
 #pragma unroll
-    for (int mp = 0; mp < 2; ++mp) {
-      if (mp > 0) __syncthreads();
+          for (int m = 0; m < DV; ++m) o[m] *= alpha;
+        }
+        const float mu = mrun == kNegInfW ? 0.f : mrun;     // no visible key so far: every weight 0
+        float l0 = 0.f, l1 = 0.f;
 #pragma unroll
-      for (int m = 0; m < DV / 2; ++m)
-        *reinterpret_cast<f32x4*>(meet + (wid * 16 + col) * S16 + 16 * m + 4 * grp) = o[mp * (DV / 2) + m];
+        for (int e = 0; e < 8; e += 2) {
+          p[e] = __builtin_amdgcn_exp2f(p[e] - mu);
+          p[e + 1] = __builtin_amdgcn_exp2f(p[e + 1] - mu);
+          l0 += p[e];
+          l1 += p[e + 1];
+        }
+        lrun += l0 + l1;
+      }
+      s16x8 phi, plo;
+      split_bf16w(p, phi, plo);
+#pragma unroll
+      for (int m = 0; m < DV; m += 4) {
+        s16x8 v[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          const short* vp = P + vrow * E + ((2 * u + ((col >> 1) & 1)) ^ vsw) * 8 + (col & 1) * 4 + (m >> 2) * 64;
+          const s16x4 a0 = rfq::ds_read_tr16(vp), a1 = rfq::ds_read_tr16(vp + 16 * E);
+          v[u] = (s16x8){a0[0], a0[1], a0[2], a0[3], a1[0], a1[1], a1[2], a1[3]};
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+          o[m + u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(v[u]), as_bf16x8(phi), o[m + u], 0, 0, 0);
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+          o[m + u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(v[u]), as_bf16x8(plo), o[m + u], 0, 0, 0);
+      }
+    }
+    __syncthreads();                                        // both waves are done with the page
+    if (const int n = i + S * kStreams; n < pages) fetch(n);
+  }
+  // ---- streams meet, half the channels at a time
+  const float l = both_halves_sum(both_rows_sum(lrun));
+  if (grp == 0) {
+    // scores that are no numbers leave the maximum at -inf, which marks a stream without visible keys
+    ml[wid * 16 + col] = MODE >= 2 ? (turns > 0 ? 0.f : kNegInfW) : l != 0.f && mrun == kNegInfW ? 0.f : mrun;
+    ml[(2 * kStreams + wid) * 16 + col] = l;
+  }
+  float* const part_ml = part + (int64_t)T * S * a.H * vdim;
+#pragma unroll
+  for (int mp = 0; mp < 2; ++mp) {
+    if (mp > 0) __syncthreads();
+#pragma unroll
+    for (int m = 0; m < DV / 2; ++m)
+      *reinterpret_cast<f32x4*>(meet + (wid * 16 + col) * S16 + 16 * m + 4 * grp) = o[mp * (DV / 2) + m];
+    __syncthreads();
+    if (mp == 0) {
+      // what the streams' parts count, and the workgroup's own maximum and sum: a thread per head and stream
+      if (tid < 32 * kStreams) {
+        const int c = tid >> 2, u = tid & 3, w = 2 * u + (c >> 4);
+        const float mu = ml[w * 16 + (c & 15)];
+        float top = fmaxf(mu, __shfl_xor(mu, 1, 64));
+        top = fmaxf(top, __shfl_xor(top, 2, 64));
+        const float f = mu == kNegInfW ? 0.f : MODE >= 2 ? 1.f : __builtin_amdgcn_exp2f(mu - top);
+        float sum = f == 0.f ? 0.f : f * ml[(2 * kStreams + w) * 16 + (c & 15)];
+        sum += __shfl_xor(sum, 1, 64);
+        sum += __shfl_xor(sum, 2, 64);
+        share[c * 4 + u] = mu == kNegInfW ? 0.f : f;
+        if (u == 0 && h0 + c < rep)
+          *reinterpret_cast<float2*>(part_ml + 2 * ((t * S + z) * a.H + g * rep + h0 + c)) = make_float2(top, sum);
+      }
       __syncthreads();
-      if (mp == 0) {
-        // what the streams' parts count, and the workgroup's own maximum and sum: a thread per head and stream
-        if (tid < 32 * kStreams) {
-          const int c = tid >> 2, u = tid & 3, w = 2 * u + (c >> 4);
-          const float mu = ml[w * 16 + (c & 15)];
-          float top = fmaxf(mu, __shfl_xor(mu, 1, 64));
-          top = fmaxf(top, __shfl_xor(top, 2, 64));
-          const float f = mu == kNegInfW ? 0.f : MODE >= 2 ? 1.f : __builtin_amdgcn_exp2f(mu - top);
-          float sum = f == 0.f ? 0.f : f * ml[(2 * kStreams + w) * 16 + (c & 15)];
-          sum += __shfl_xor(sum, 1, 64);
-          sum += __shfl_xor(sum, 2, 64);
-          share[c * 4 + u] = mu == kNegInfW ? 0.f : f;
-          if (u == 0 && h0 + c < rep)
-            *reinterpret_cast<float2*>(part_ml + 2 * ((t * S + z) * a.H + g * rep + h0 + c)) = make_float2(top, sum);
-        }
-        __syncthreads();
-      }
-      constexpr int NX = 32 * (vdim / 8) / (128 * kStreams);  // pieces of four channels a thread
-      static_assert(NX * 128 * kStreams == 32 * (vdim / 8), "");
-#pragma unroll 2
-      for (int n = 0; n < NX; ++n) {
-        const int x = tid + n * 128 * kStreams, c = x / (vdim / 8), dp = (x - c * (vdim / 8)) * 4;
-        const float4 f = *reinterpret_cast<const float4*>(share + 4 * c);
-        const float fs[4] = {f.x, f.y, f.z, f.w};
-        float y[4] = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int u = 0; u < kStreams; ++u) {
-          const float4 v = *reinterpret_cast<const float4*>(meet + ((2 * u + (c >> 4)) * 16 + (c & 15)) * S16 + dp);
-          y[0] += fs[u] * v.x; y[1] += fs[u] * v.y; y[2] += fs[u] * v.z; y[3] += fs[u] * v.w;
-        }
-        if (h0 + c < rep)
-          *reinterpret_cast<float4*>(part + ((t * S + z) * a.H + g * rep + h0 + c) * vdim + mp * (vdim / 2) + dp) =
-              make_float4(y[0], y[1], y[2], y[3]);
-      }
     }
-    __syncthreads();                                          // the next row's pages take this place
+    constexpr int NX = 32 * (vdim / 8) / (128 * kStreams);  // pieces of four channels a thread
+    static_assert(NX * 128 * kStreams == 32 * (vdim / 8), "");
+#pragma unroll 2
+    for (int n = 0; n < NX; ++n) {
+      const int x = tid + n * 128 * kStreams, c = x / (vdim / 8), dp = (x - c * (vdim / 8)) * 4;
+      const float4 f = *reinterpret_cast<const float4*>(share + 4 * c);
+      const float fs[4] = {f.x, f.y, f.z, f.w};
+      float y[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int u = 0; u < kStreams; ++u) {
+        const float4 v = *reinterpret_cast<const float4*>(meet + ((2 * u + (c >> 4)) * 16 + (c & 15)) * S16 + dp);
+        y[0] += fs[u] * v.x; y[1] += fs[u] * v.y; y[2] += fs[u] * v.z; y[3] += fs[u] * v.w;
+      }
+      if (h0 + c < rep)
+        *reinterpret_cast<float4*>(part + ((t * S + z) * a.H + g * rep + h0 + c) * vdim + mp * (vdim / 2) + dp) =
+            make_float4(y[0], y[1], y[2], y[3]);
+    }
   }
 }
 
-// One wave per sequence and head: the workgroups' parts of its rows, the sink, the gate.
+// One wave per row and head: the workgroups' parts, the sink, the gate.
 template <int DV, int MODE>
-__global__ __launch_bounds__(64) void attn_keep_streams_merge_kernel(const KeepArgs a, const float* part, int T, int S) {
+__global__ __launch_bounds__(64) void attn_keep_streams_merge_kernel(const KeepArgs a, const float* part, int T, int S,
+                                                                      int NA) {
   constexpr int vdim = 16 * DV, NC = vdim / 256;              // pieces of four channels a lane
-  const int s = blockIdx.x, hx = blockIdx.y, lane = threadIdx.x, ql = a.q_len[s];
-  for (int r = 0; r < ql; ++r) {
-    const int64_t t = a.q_start[s] + r;
-    const float2* ml = reinterpret_cast<const float2*>(part + (int64_t)T * S * a.H * vdim);
-    const bool sink = MODE < 2 && a.head_bias != nullptr;
-    float top = sink ? a.head_bias[hx] * kLog2e : kNegInfW, l = 0.f;
-    for (int z = 0; z < S; ++z) top = fmaxf(top, ml[(t * S + z) * a.H + hx].x);
-    if (sink) l = __builtin_amdgcn_exp2f(a.head_bias[hx] * kLog2e - top);
-    float y[NC][4];
+  const int64_t t = blockIdx.x;
+  const int hx = blockIdx.y, lane = threadIdx.x;
+  if (row_owner(a.q_start, a.q_len, NA, (int)t) < 0) return;
+  const float2* ml = reinterpret_cast<const float2*>(part + (int64_t)T * S * a.H * vdim);
+  const bool sink = MODE < 2 && a.head_bias != nullptr;
+  float top = sink ? a.head_bias[hx] * kLog2e : kNegInfW, l = 0.f;
+  for (int z = 0; z < S; ++z) top = fmaxf(top, ml[(t * S + z) * a.H + hx].x);
+  if (sink) l = __builtin_amdgcn_exp2f(a.head_bias[hx] * kLog2e - top);
+  float y[NC][4];
 #pragma unroll
-    for (int n = 0; n < NC; ++n) y[n][0] = y[n][1] = y[n][2] = y[n][3] = 0.f;
-    for (int z = 0; z < S; ++z) {
-      const int64_t at = (t * S + z) * a.H + hx;
-      const float2 m = ml[at];
-      if (m.x == kNegInfW) continue;                          // a workgroup without visible keys
-      const float f = MODE >= 2 ? 1.f : __builtin_amdgcn_exp2f(m.x - top);
-      l += f * m.y;
-#pragma unroll
-      for (int n = 0; n < NC; ++n) {
-        const float4 v = *reinterpret_cast<const float4*>(part + at * vdim + 256 * n + 4 * lane);
-        y[n][0] += f * v.x; y[n][1] += f * v.y; y[n][2] += f * v.z; y[n][3] += f * v.w;
-      }
-    }
-    const bf16_t* gate = static_cast<const bf16_t*>(a.gate);
-    float mul = MODE >= 2 ? a.out_mult : (l > 0.f ? a.out_mult / l : 0.f);
-    if (gate != nullptr && a.gate_w == 1) mul /= 1.0f + __expf(-ldf(gate + t * a.gate_stride + hx));
+  for (int n = 0; n < NC; ++n) y[n][0] = y[n][1] = y[n][2] = y[n][3] = 0.f;
+  for (int z = 0; z < S; ++z) {
+    const int64_t at = (t * S + z) * a.H + hx;
+    const float2 m = ml[at];
+    if (m.x == kNegInfW) continue;                          // a workgroup without visible keys
+    const float f = MODE >= 2 ? 1.f : __builtin_amdgcn_exp2f(m.x - top);
+    l += f * m.y;
 #pragma unroll
     for (int n = 0; n < NC; ++n) {
-      const int dv = 256 * n + 4 * lane;
-      float f[4];
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        f[e] = y[n][e] * mul;
-        if (gate != nullptr && a.gate_w > 1) f[e] /= 1.0f + __expf(-ldf(gate + t * a.gate_stride + (int64_t)hx * vdim + dv + e));
-      }
-      *reinterpret_cast<uint2*>(static_cast<bf16_t*>(a.out) + t * a.out_stride + (int64_t)hx * vdim + dv) =
-          make_uint2(rfq::pack_bf16x2(f[0], f[1]), rfq::pack_bf16x2(f[2], f[3]));
+      const float4 v = *reinterpret_cast<const float4*>(part + at * vdim + 256 * n + 4 * lane);
+      y[n][0] += f * v.x; y[n][1] += f * v.y; y[n][2] += f * v.z; y[n][3] += f * v.w;
     }
+  }
+  const bf16_t* gate = static_cast<const bf16_t*>(a.gate);
+  float mul = MODE >= 2 ? a.out_mult : (l > 0.f ? a.out_mult / l : 0.f);
+  if (gate != nullptr && a.gate_w == 1) mul /= 1.0f + __expf(-ldf(gate + t * a.gate_stride + hx));
+#pragma unroll
+  for (int n = 0; n < NC; ++n) {
+    const int dv = 256 * n + 4 * lane;
+    float f[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      f[e] = y[n][e] * mul;
+      if (gate != nullptr && a.gate_w > 1) f[e] /= 1.0f + __expf(-ldf(gate + t * a.gate_stride + (int64_t)hx * vdim + dv + e));
+    }
+    *reinterpret_cast<uint2*>(static_cast<bf16_t*>(a.out) + t * a.out_stride + (int64_t)hx * vdim + dv) =
+        make_uint2(rfq::pack_bf16x2(f[0], f[1]), rfq::pack_bf16x2(f[2], f[3]));
   }
 }
 
@@ -1140,10 +1151,11 @@ void launch_attn_keep_wide_rows(const float* q, const void* k_cache, int64_t vrs
 #undef ROWS_GO
 }
 
-// How many workgroups share a sequence's pages, 0 where the streams are not the way: more than the 16 heads of one
-// wave, room for two workgroups or more a sequence and pages for them (128 sequences of 600 with 32 heads, two each: 43
-// -> 40 us; up to four pages: even), and a row a sequence, as rows follow one another (64 sequences of 600 with two rows
-// each: 59 us, 42 where their columns lie side by side).
+// How many workgroups share a row's pages, 0 where the streams are not the way: more than the 16 heads of one wave,
+// room for two workgroups or more a row and pages for them (128 sequences of 600 with 32 heads, two each: 43 -> 40 us;
+// up to four pages: even).  Of up to NA rows a sequence may have several: each has workgroups of its own, as in a
+// captured step rows of an extend stand where other sequences are padding (one sequence of 600 tokens with 16 rows, 16
+// of one and 15 without: 143 us split over waves, 269 with an extend's rows one after another, 23 side by side).
 int keep_streams(int T, int NA, int H, int G, int E, int vdim, bool shared, int maxb) {
   const int rep = H / G;
   if (!shared || E != 576 || vdim != 512 || rep <= 16 || NA <= 0 || H > 65535) return 0;
@@ -1169,8 +1181,8 @@ void launch_attn_keep_streams(const float* q, const void* k_cache, int64_t vrs, 
                                 160 * 1024);
       attr = true;
     }
-    hipLaunchKernelGGL(kernel, dim3(NA, G * ((H / G + 31) / 32), S), dim3(128 * kStreams), lds, s, a, part, T);
-    hipLaunchKernelGGL(merge, dim3(NA, H), dim3(64), 0, s, a, part, T, S);
+    hipLaunchKernelGGL(kernel, dim3(T, G * ((H / G + 31) / 32), S), dim3(128 * kStreams), lds, s, a, part, T, NA);
+    hipLaunchKernelGGL(merge, dim3(T, H), dim3(64), 0, s, a, part, T, S, NA);
   };
   const bool cap = softcap > 0.f;
   if (sigmoid && cap) go(&attn_keep_streams_kernel<18, 32, 3>, &attn_keep_streams_merge_kernel<32, 3>);

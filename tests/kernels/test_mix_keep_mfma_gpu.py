@@ -14,7 +14,7 @@ DEV, BS = "cuda", 32
 SEQS = [(1, 1), (31, 1), (32, 1), (33, 1), (129, 1), (257, 1), (300, 5), (40, 0), (700, 1), (70, 33)]
 
 
-def _check(H, G, E, vd, shared, seqs=SEQS, spoil=None, prompt=False, **opt):
+def _check(H, G, E, vd, shared, seqs=SEQS, spoil=None, prompt=False, spare=0, **opt):
     g = torch.Generator().manual_seed(H + E + vd)
     need = [(n + BS - 1) // BS for n, _ in seqs]
     perm = torch.randperm(sum(need), generator=g).tolist()
@@ -45,6 +45,10 @@ def _check(H, G, E, vd, shared, seqs=SEQS, spoil=None, prompt=False, **opt):
     ref.attn_keep_window(q, kc, vc, *args("cpu"), bias, gate, out, E ** -0.5, opt.get("window", 0),
                          opt.get("keep_first", 0), opt.get("sigmoid", False), opt.get("softcap", 0.0),
                          opt.get("out_mult", 1.0))
+    if spare:                                    # a captured step's rows beyond those of its sequences
+        q = torch.cat([q, torch.full((spare, H, E), float("nan"))])
+        out = torch.cat([out, torch.full((spare, H * vd), 7.0, dtype=torch.bfloat16)])
+        gate = None if gate is None else torch.cat([gate, gate[:1].expand(spare, -1)])
     got = torch.full_like(out, 7.0).to(DEV)
     kd = k.to(DEV)
     m = lambda x: None if x is None else x.to(DEV)  # noqa: E731
@@ -106,6 +110,45 @@ def test_wide_rows_in_streams(H, G):
     _check(H, G, 576, 512, True, seqs=STREAMS, window=64, keep_first=5, sigmoid=True, bias=True)
     _check(H, G, 576, 512, True, seqs=STREAMS[4:5], sigmoid=True, softcap=15.0, bias=True)
     _check(H, G, 576, 512, True, seqs=STREAMS[-1:])
+
+
+# as many rows as sequences, and fewer, but several of one sequence: an extend beside padding in a captured step
+EXTENDS = [(300, 1), (40, 0), (600, 16), (64, 1), (33, 5), (90, 0), (161, 2)] + [(40, 0)] * 20
+
+
+@pytest.mark.parametrize("H,G", [(17, 1), (32, 1), (64, 1), (48, 2)])
+def test_wide_rows_of_one_sequence_in_streams(H, G):
+    _check(H, G, 576, 512, True, seqs=EXTENDS, bias=True, gate="head")
+    _check(H, G, 576, 512, True, seqs=EXTENDS, softcap=20.0, gate="output", spare=2)
+    _check(H, G, 576, 512, True, seqs=EXTENDS, window=64, keep_first=5, sigmoid=True, bias=True, spare=1)
+    _check(H, G, 576, 512, True, seqs=[(40, 0)] * 63 + [(200, 32)], spare=9)
+
+
+def test_wide_rows_of_one_sequence_side_by_side():
+    """Sixteen rows of one sequence beside padding take about what a row each of sixteen sequences takes (17 us more a
+    row when they follow one another)."""
+    H, E, vd, n, nb = 32, 576, 512, 16, 20
+    g = torch.Generator().manual_seed(0)
+    k = torch.randn(n * nb, 1, BS, E, generator=g).bfloat16().to(DEV)
+    q = torch.randn(n, H, E, generator=g).to(DEV)
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=DEV)  # noqa: E731
+    tables, items = torch.randperm(n * nb, generator=g).int().view(n, nb).to(DEV), i32(range(n))
+    out = torch.empty(n, H * vd, dtype=torch.bfloat16, device=DEV)
+
+    def time(rows):
+        meta = (vd, tables, i32([sum(rows[:i]) for i in range(n)]), i32(rows), i32([nb * BS] * n), items, i32([0] * n))
+        ev = [torch.cuda.Event(enable_timing=True) for _ in range(2)]
+        best = float("inf")
+        for _ in range(6):
+            ev[0].record()
+            for _ in range(10):
+                ops.attn_keep_window(q, k, k, *meta, None, None, out, E ** -0.5, short_rows=32)
+            ev[1].record()
+            torch.cuda.synchronize()
+            best = min(best, ev[0].elapsed_time(ev[1]))
+        return best
+
+    assert time([16] + [0] * 15) <= 3 * time([1] * 16)
 
 
 PROMPTS = [(1, 1), (31, 31), (32, 32), (33, 33), (100, 70), (300, 45), (40, 0), (161, 97)]
