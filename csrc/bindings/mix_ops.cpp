@@ -93,7 +93,7 @@ void launch_attn_keep_split(const float*, const void*, const void*, int64_t, con
                             const int32_t*, const int32_t*, int, int, int, const float*, const void*, int64_t, int,
                             void*, int64_t, float, int, int, bool, int, int, int, int, bool, float, float,
                             hipStream_t);
-int keep_streams(int, int, int, int, int, int, bool, int);
+int keep_streams(int, int, int, int, int, int, bool, int, int, int);
 int64_t keep_streams_floats(int, int, int, int);
 void launch_attn_keep_streams(const float*, const void*, int64_t, const int32_t*, int, const int32_t*, const int32_t*,
                               const int32_t*, int, int, int, const float*, const void*, int64_t, int, void*, int64_t, float,
@@ -846,7 +846,8 @@ void attn_keep_window(const Tensor& q, const Tensor& k_cache, const Tensor& v_ca
   if (short_rows > 0 && tiles) {
     // sequences of at most short_rows rows each (decode section): their pages split over waves, or over
     // workgroups, whose parts meet in scratch memory
-    if (const int S = rfqmix::keep_streams(T, NB, H, G, E, (int)vdim, shared, (int)bt.size(1)); S > 0 && T > 0) {
+    if (const int S = rfqmix::keep_streams(T, NB, H, G, E, (int)vdim, shared, (int)bt.size(1), (int)window,
+                                           (int)keep_first); S > 0 && T > 0) {
       const Tensor part = at::empty({rfqmix::keep_streams_floats(T, S, H, (int)vdim)}, q.options());
       return rfqmix::launch_attn_keep_streams(
           f32p(q, "q"), k_cache.data_ptr(), vrs, i32p(bt, "block_tables", 0), (int)bt.size(1),

@@ -752,35 +752,90 @@ __global__ __launch_bounds__(128 * HPW, DEC && HPW == 1 ? 1 : 2) void attn_keep_
 // one of 611 37 -> 21, eight of 2,000 90 -> 29, 64 of 2,000 95 -> 51, 32 of 600 with 64 heads 40 -> 32.
 constexpr int kStreams = 4;
 
-// The sequence that has row t of the step, -1: none (rows of a captured step beyond those of its sequences).  A row a
-// sequence, as most steps have it, is seen at once.
-__device__ __forceinline__ int row_owner(const int32_t* q_start, const int32_t* q_len, int NA, int t) {
-  if (t < NA && q_start[t] == t && q_len[t] > 0) return t;
-  for (int b = 0; b < NA; b += 64) {
-    const int i = b + (threadIdx.x & 63), from = i < NA ? q_start[i] : 0, n = i < NA ? q_len[i] : 0;
-    const uint64_t m = __builtin_amdgcn_ballot_w64(from <= t && t < from + n);
-    if (m != 0) return b + __builtin_ctzll(m);
+// What a row of the step sees: pages [0, n_keep) of its sequence s (-1: none, a row of a captured step beyond those of
+// its sequences) hold the kept first tokens, `skip` pages follow that are not read, then those of the window up to the
+// row's own.
+struct RowPages {
+  int s, pi, jwin, kf, n_keep, skip, pages;                   // pi: query, jwin: window's first key, kf: kept keys before it
+};
+// Most steps have a row a sequence: then row t is sequence t's, whose numbers are on their way at once.
+__device__ __forceinline__ RowPages row_pages(const KeepArgs& a, int NA, int t) {
+  RowPages r;
+  const int i = min(t, NA - 1);
+  int from = a.q_start[i], n = a.q_len[i], kv = a.kv_len[i];
+  r.s = i;
+  if (from > t || from + n <= t) {
+    r.s = -1;
+    for (int b = 0; b < NA && r.s < 0; b += 64) {
+      const int x = b + (threadIdx.x & 63), xf = x < NA ? a.q_start[x] : 0, xn = x < NA ? a.q_len[x] : 0;
+      const uint64_t m = __builtin_amdgcn_ballot_w64(xf <= t && t < xf + xn);
+      if (m != 0) r.s = b + __builtin_ctzll(m);
+    }
+    if (r.s < 0) return r;
+    from = a.q_start[r.s];
+    n = a.q_len[r.s];
+    kv = a.kv_len[r.s];
   }
-  return -1;
+  r.pi = kv - n + t - from;
+  r.jwin = a.window > 0 ? max(0, r.pi - a.window + 1) : 0;
+  r.kf = a.window > 0 ? min(a.keep_first, r.jwin) : 0;
+  const int pg_win = r.jwin / WBS;
+  r.n_keep = min((r.kf + WBS - 1) / WBS, pg_win);
+  r.skip = pg_win - r.n_keep;
+  r.pages = r.pi / WBS + 1 - r.skip;
+  return r;
 }
+// What a row's weighted values of head h are multiplied by, given the maximum and sum of all its keys: the sink's part
+// of the sum, a gate per head.
+template <int MODE>
+__device__ __forceinline__ float whole(const KeepArgs& a, int64_t t, int h, float top, float sum) {
+  float f = 1.f, l = sum;
+  if constexpr (MODE < 2) {
+    const float sink = a.head_bias != nullptr ? a.head_bias[h] * kLog2e : kNegInfW, m = fmaxf(top, sink);
+    f = top == kNegInfW ? 0.f : __builtin_amdgcn_exp2f(top - m);
+    l = (top == kNegInfW ? 0.f : f * sum) + (sink == kNegInfW ? 0.f : __builtin_amdgcn_exp2f(sink - m));
+  }
+  float mul = MODE >= 2 ? a.out_mult : (l > 0.f ? a.out_mult / l : 0.f);
+  if (a.gate != nullptr && a.gate_w == 1)
+    mul /= 1.0f + __expf(-ldf(static_cast<const bf16_t*>(a.gate) + t * a.gate_stride + h));
+  return f * mul;
+}
+// Four neighbouring outputs of head h, through a gate per output
+template <int vdim>
+__device__ __forceinline__ void store_gated(const KeepArgs& a, float (&y)[4], int64_t t, int h, int dv) {
+  if (a.gate != nullptr && a.gate_w > 1) {
+    const float4 x = ld4(static_cast<const bf16_t*>(a.gate) + t * a.gate_stride + (int64_t)h * vdim + dv);
+    y[0] /= 1.0f + __expf(-x.x);
+    y[1] /= 1.0f + __expf(-x.y);
+    y[2] /= 1.0f + __expf(-x.z);
+    y[3] /= 1.0f + __expf(-x.w);
+  }
+  *reinterpret_cast<uint2*>(static_cast<bf16_t*>(a.out) + t * a.out_stride + (int64_t)h * vdim + dv) =
+      make_uint2(rfq::pack_bf16x2(y[0], y[1]), rfq::pack_bf16x2(y[2], y[3]));
+}
+// How many of S workgroups have a part in the row: those with pages, the first in any case
+__device__ __forceinline__ int row_shares(const RowPages& r, int S) { return min(S, max(1, (r.pages + kStreams - 1) / kStreams)); }
 
 template <int DK, int DV, int MODE>
 __global__ __launch_bounds__(128 * kStreams, 2) void attn_keep_streams_kernel(const KeepArgs a, float* part, int T,
                                                                                 int NA) {
   constexpr int E = 32 * DK, vdim = 16 * DV, PGS = WBS * E, ND = WBS * E / 1024, S16 = vdim / 2 + 4;
   static_assert(DK > 10 && E % 64 == 0 && WBS * E % 1024 == 0 && 2 * kStreams * 16 * S16 * 4 <= kStreams * PGS * 2, "the partial results take the pages' place");
-  const int64_t t = blockIdx.x;
-  const int s = row_owner(a.q_start, a.q_len, NA, (int)t);
-  if (s < 0) return;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wid = __builtin_amdgcn_readfirstlane(tid >> 6), st = wid >> 1;
+  const int64_t t = blockIdx.x;
+  const int S = gridDim.z, z = blockIdx.z;
+  const RowPages row = row_pages(a, NA, (int)t);
+  if (row.s < 0) return;
+  const int pi = row.pi, jwin = row.jwin, kf = row.kf, n_keep = row.n_keep, skip = row.skip, pages = row.pages;
+  const int shares = row_shares(row, S);
+  if (z >= shares) return;                                    // no page for this workgroup
   const int col = lane & 15, grp = lane >> 4;
   const int rep = a.H / a.G, per = (rep + 31) / 32;
   const int g = (int)blockIdx.y / per, h0 = ((int)blockIdx.y - g * per) * 32;
   const int hd = h0 + (wid & 1) * 16 + col;
   const bool idle = h0 + (wid & 1) * 16 >= rep;               // a wave that only copies pages
   const int hh = g * rep + min(hd, rep - 1);                  // past the last head: it once more, not stored
-  const int S = gridDim.z, z = blockIdx.z;
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   short* const P = reinterpret_cast<short*>(smem) + st * PGS; // this stream's page
   float* const meet = reinterpret_cast<float*>(smem);         // later [wave][16][S16]
@@ -788,21 +843,14 @@ __global__ __launch_bounds__(128 * kStreams, 2) void attn_keep_streams_kernel(co
   float* const share = ml + 4 * kStreams * 16;                // [head][stream]
   unsigned char* const qs = reinterpret_cast<unsigned char*>(share + 32 * kStreams);   // [half][stream] KB of queries
   typedef const __attribute__((address_space(4))) int32_t const_i32;
-  const_i32* bt = (const_i32*)(uintptr_t)(a.bt + (int64_t)s * a.maxb);
+  const_i32* bt = (const_i32*)(uintptr_t)(a.bt + (int64_t)row.s * a.maxb);
   const float qmul = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(
       a.scale * (MODE % 2 == 1 ? 2.f * kLog2e / a.softcap : MODE == 2 ? -kLog2e : kLog2e))));
   const float cap2 = MODE % 2 == 1 ? a.softcap * kLog2e : 0.f;
   const float hb = MODE >= 2 && a.head_bias != nullptr ? a.head_bias[hh] * kLog2e : 0.f;
   const int ksw = wide_swizzle(col), vrow = 4 * grp + (col >> 2), vsw = wide_swizzle(vrow);
 
-  const int pi = a.kv_len[s] - a.q_len[s] + (int)t - a.q_start[s];     // the row's query
-  const int window = a.window;
-  const int jwin = window > 0 ? max(0, pi - window + 1) : 0;
-  const int kf = window > 0 ? min(a.keep_first, jwin) : 0;
-  // pages [0, n_keep) hold the kept first tokens, pages [pg_win, pg_last] the window
-  const int pg_last = pi / WBS, pg_win = jwin / WBS;
-  const int n_keep = min((kf + WBS - 1) / WBS, pg_win), skip = pg_win - n_keep, pages = pg_last + 1 - skip;
-  const int turns = max(0, (pages - z * kStreams + S * kStreams - 1) / (S * kStreams));
+  const int turns = (pages - z * kStreams + S * kStreams - 1) / (S * kStreams);
   constexpr int NQ = (DK + kStreams - 1) / kStreams;
   float4 qx[NQ], qy[NQ];                                    // on their way before the page is
   {
@@ -950,9 +998,20 @@ __global__ __launch_bounds__(128 * kStreams, 2) void attn_keep_streams_kernel(co
   }
   // ---- streams meet, half the channels at a time
   const float l = both_halves_sum(both_rows_sum(lrun));
+  // scores that are no numbers leave the maximum at -inf, which marks a stream without visible keys
+  const float mx = MODE >= 2 || (l != 0.f && mrun == kNegInfW) ? 0.f : mrun;
+  if (pages == 1) {                                           // nobody to meet
+    if (st > 0 || hd >= rep) return;
+    const float f = whole<MODE>(a, t, hh, mx, l);
+#pragma unroll
+    for (int m = 0; m < DV; ++m) {
+      float y[4] = {o[m][0] * f, o[m][1] * f, o[m][2] * f, o[m][3] * f};
+      store_gated<vdim>(a, y, t, hh, 16 * m + 4 * grp);
+    }
+    return;
+  }
   if (grp == 0) {
-    // scores that are no numbers leave the maximum at -inf, which marks a stream without visible keys
-    ml[wid * 16 + col] = MODE >= 2 ? (turns > 0 ? 0.f : kNegInfW) : l != 0.f && mrun == kNegInfW ? 0.f : mrun;
+    ml[wid * 16 + col] = mx;
     ml[(2 * kStreams + wid) * 16 + col] = l;
   }
   float* const part_ml = part + (int64_t)T * S * a.H * vdim;
@@ -974,9 +1033,13 @@ __global__ __launch_bounds__(128 * kStreams, 2) void attn_keep_streams_kernel(co
         float sum = f == 0.f ? 0.f : f * ml[(2 * kStreams + w) * 16 + (c & 15)];
         sum += __shfl_xor(sum, 1, 64);
         sum += __shfl_xor(sum, 2, 64);
-        share[c * 4 + u] = mu == kNegInfW ? 0.f : f;
-        if (u == 0 && h0 + c < rep)
-          *reinterpret_cast<float2*>(part_ml + 2 * ((t * S + z) * a.H + g * rep + h0 + c)) = make_float2(top, sum);
+        if (shares > 1) {
+          share[c * 4 + u] = f;
+          if (u == 0 && h0 + c < rep)
+            *reinterpret_cast<float2*>(part_ml + 2 * ((t * S + z) * a.H + g * rep + h0 + c)) = make_float2(top, sum);
+        } else {                                              // no other part: what the merge would do
+          share[c * 4 + u] = f * whole<MODE>(a, t, g * rep + min(h0 + c, rep - 1), top, sum);
+        }
       }
       __syncthreads();
     }
@@ -993,9 +1056,10 @@ __global__ __launch_bounds__(128 * kStreams, 2) void attn_keep_streams_kernel(co
         const float4 v = *reinterpret_cast<const float4*>(meet + ((2 * u + (c >> 4)) * 16 + (c & 15)) * S16 + dp);
         y[0] += fs[u] * v.x; y[1] += fs[u] * v.y; y[2] += fs[u] * v.z; y[3] += fs[u] * v.w;
       }
-      if (h0 + c < rep)
-        *reinterpret_cast<float4*>(part + ((t * S + z) * a.H + g * rep + h0 + c) * vdim + mp * (vdim / 2) + dp) =
-            make_float4(y[0], y[1], y[2], y[3]);
+      const int hc = g * rep + h0 + c, dv = mp * (vdim / 2) + dp;
+      if (h0 + c >= rep) continue;
+      if (shares > 1) *reinterpret_cast<float4*>(part + ((t * S + z) * a.H + hc) * vdim + dv) = make_float4(y[0], y[1], y[2], y[3]);
+      else store_gated<vdim>(a, y, t, hc, dv);
     }
   }
 }
@@ -1007,16 +1071,17 @@ __global__ __launch_bounds__(64) void attn_keep_streams_merge_kernel(const KeepA
   constexpr int vdim = 16 * DV, NC = vdim / 256;              // pieces of four channels a lane
   const int64_t t = blockIdx.x;
   const int hx = blockIdx.y, lane = threadIdx.x;
-  if (row_owner(a.q_start, a.q_len, NA, (int)t) < 0) return;
+  const RowPages row = row_pages(a, NA, (int)t);
+  if (row.s < 0) return;
+  const int shares = row_shares(row, S);
+  if (shares == 1) return;                                    // its workgroup has stored the row itself
   const float2* ml = reinterpret_cast<const float2*>(part + (int64_t)T * S * a.H * vdim);
-  const bool sink = MODE < 2 && a.head_bias != nullptr;
-  float top = sink ? a.head_bias[hx] * kLog2e : kNegInfW, l = 0.f;
-  for (int z = 0; z < S; ++z) top = fmaxf(top, ml[(t * S + z) * a.H + hx].x);
-  if (sink) l = __builtin_amdgcn_exp2f(a.head_bias[hx] * kLog2e - top);
+  float top = kNegInfW, l = 0.f;
+  for (int z = 0; z < shares; ++z) top = fmaxf(top, ml[(t * S + z) * a.H + hx].x);
   float y[NC][4];
 #pragma unroll
   for (int n = 0; n < NC; ++n) y[n][0] = y[n][1] = y[n][2] = y[n][3] = 0.f;
-  for (int z = 0; z < S; ++z) {
+  for (int z = 0; z < shares; ++z) {
     const int64_t at = (t * S + z) * a.H + hx;
     const float2 m = ml[at];
     if (m.x == kNegInfW) continue;                          // a workgroup without visible keys
@@ -1028,20 +1093,12 @@ __global__ __launch_bounds__(64) void attn_keep_streams_merge_kernel(const KeepA
       y[n][0] += f * v.x; y[n][1] += f * v.y; y[n][2] += f * v.z; y[n][3] += f * v.w;
     }
   }
-  const bf16_t* gate = static_cast<const bf16_t*>(a.gate);
-  float mul = MODE >= 2 ? a.out_mult : (l > 0.f ? a.out_mult / l : 0.f);
-  if (gate != nullptr && a.gate_w == 1) mul /= 1.0f + __expf(-ldf(gate + t * a.gate_stride + hx));
+  const float mul = whole<MODE>(a, t, hx, top, l);
 #pragma unroll
   for (int n = 0; n < NC; ++n) {
-    const int dv = 256 * n + 4 * lane;
-    float f[4];
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      f[e] = y[n][e] * mul;
-      if (gate != nullptr && a.gate_w > 1) f[e] /= 1.0f + __expf(-ldf(gate + t * a.gate_stride + (int64_t)hx * vdim + dv + e));
-    }
-    *reinterpret_cast<uint2*>(static_cast<bf16_t*>(a.out) + t * a.out_stride + (int64_t)hx * vdim + dv) =
-        make_uint2(rfq::pack_bf16x2(f[0], f[1]), rfq::pack_bf16x2(f[2], f[3]));
+    for (int e = 0; e < 4; ++e) y[n][e] *= mul;
+    store_gated<vdim>(a, y[n], t, hx, 256 * n + 4 * lane);
   }
 }
 
@@ -1152,16 +1209,22 @@ void launch_attn_keep_wide_rows(const float* q, const void* k_cache, int64_t vrs
 }
 
 // How many workgroups share a row's pages, 0 where the streams are not the way: more than the 16 heads of one wave,
-// room for two workgroups or more a row and pages for them (128 sequences of 600 with 32 heads, two each: 43 -> 40 us;
-// up to four pages: even).  Of up to NA rows a sequence may have several: each has workgroups of its own, as in a
-// captured step rows of an extend stand where other sequences are padding (one sequence of 600 tokens with 16 rows, 16
-// of one and 15 without: 143 us split over waves, 269 with an extend's rows one after another, 23 side by side).
-int keep_streams(int T, int NA, int H, int G, int E, int vdim, bool shared, int maxb) {
+// room for two workgroups or more a row (128 sequences of 600 with 32 heads, two each: 43 -> 40 us), and more than 20
+// pages that a row may see, by its table and window.  With fewer the scratch and the second launch cost a layer's pass
+// that the host bounds 4 us (32 heads, 1 - 64 sequences of 400 tokens, tables as wide: 47 us split over waves, 51 in
+// streams; of 600 49 - 52 and 51; of 900 60 - 64 and 51.5).  Captured steps have wide tables over any number of pages:
+// there a row of one page takes 14.8 us either way, four pages 18.8 and 17.1, nineteen 23 - 38 and 19 - 29.
+// Of up to NA rows a sequence may have several: each has workgroups of its own, as in a captured step rows of an extend
+// stand where other sequences are padding (one sequence of 600 tokens with 16 rows, 16 of one and 15 without: 143 us
+// split over waves, 269 with an extend's rows one after another, 23 side by side).
+int keep_streams(int T, int NA, int H, int G, int E, int vdim, bool shared, int maxb, int window, int keep_first) {
   const int rep = H / G;
   if (!shared || E != 576 || vdim != 512 || rep <= 16 || NA <= 0 || H > 65535) return 0;
   const int64_t wgs = (int64_t)NA * G * ((rep + 31) / 32);
-  const int S = (int)std::min<int64_t>(256 / std::max<int64_t>(wgs, 1), std::min((maxb + kStreams - 1) / kStreams, 16));
-  return S >= 2 && T <= NA ? S : 0;
+  // pages that a row can see: of its table, of the window and of the kept first tokens
+  const int64_t most = window > 0 ? std::min<int64_t>(maxb, ((int64_t)window + WBS - 2) / WBS + 1 + ((int64_t)keep_first + WBS - 1) / WBS) : maxb;
+  const int S = (int)std::min(256 / std::max<int64_t>(wgs, 1), std::min<int64_t>((most + kStreams - 1) / kStreams, 16));
+  return S >= 2 && most > 20 && T <= NA ? S : 0;
 }
 int64_t keep_streams_floats(int T, int S, int H, int vdim) { return (int64_t)T * S * H * (vdim + 2); }
 
