@@ -1228,6 +1228,21 @@ int keep_streams(int T, int NA, int H, int G, int E, int vdim, bool shared, int 
 }
 int64_t keep_streams_floats(int T, int S, int H, int vdim) { return (int64_t)T * S * H * (vdim + 2); }
 
+template <int DK, int DV, int MODE>
+static void launch_streams_one(const KeepArgs& a, int T, int NA, int S, float* part) {
+  constexpr size_t lds = (size_t)kStreams * WBS * 32 * DK * 2 + (4 * kStreams * 16 + 32 * kStreams) * sizeof(float) + 2 * kStreams * 1024;
+  static_assert(lds <= 160 * 1024, "LDS of a CU");
+  static bool attr = false;
+  if (!attr) {
+    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&attn_keep_streams_kernel<DK, DV, MODE>),
+                              hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+    attr = true;
+  }
+  hipLaunchKernelGGL((attn_keep_streams_kernel<DK, DV, MODE>), dim3(T, a.G * ((a.H / a.G + 31) / 32), S), dim3(128 * kStreams),
+                     lds, a.s, a, part, T, NA);
+  hipLaunchKernelGGL((attn_keep_streams_merge_kernel<DV, MODE>), dim3(T, a.H), dim3(64), 0, a.s, a, part, T, S, NA);
+}
+
 void launch_attn_keep_streams(const float* q, const void* k_cache, int64_t vrs, const int32_t* bt, int maxb,
                               const int32_t* q_start, const int32_t* q_len, const int32_t* kv_len, int T, int NA, int S,
                               const float* head_bias, const void* gate, int64_t gate_stride, int gate_w, void* out,
@@ -1236,22 +1251,11 @@ void launch_attn_keep_streams(const float* q, const void* k_cache, int64_t vrs, 
   const KeepArgs a{q, k_cache, k_cache, vrs, bt, maxb, q_start, q_len, kv_len, nullptr, nullptr,
                    0, head_bias, gate, gate_stride, gate_w, out, out_stride, scale, window, keep_first,
                    sigmoid, H, G, softcap, out_mult, s};
-  auto go = [&](auto kernel, auto merge) {
-    constexpr size_t lds = (size_t)kStreams * WBS * 576 * 2 + (4 * kStreams * 16 + 32 * kStreams) * sizeof(float) + 2 * kStreams * 1024;
-    static bool attr = false;
-    if (!attr) {
-      (void)hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                160 * 1024);
-      attr = true;
-    }
-    hipLaunchKernelGGL(kernel, dim3(T, G * ((H / G + 31) / 32), S), dim3(128 * kStreams), lds, s, a, part, T, NA);
-    hipLaunchKernelGGL(merge, dim3(T, H), dim3(64), 0, s, a, part, T, S, NA);
-  };
   const bool cap = softcap > 0.f;
-  if (sigmoid && cap) go(&attn_keep_streams_kernel<18, 32, 3>, &attn_keep_streams_merge_kernel<32, 3>);
-  else if (sigmoid) go(&attn_keep_streams_kernel<18, 32, 2>, &attn_keep_streams_merge_kernel<32, 2>);
-  else if (cap) go(&attn_keep_streams_kernel<18, 32, 1>, &attn_keep_streams_merge_kernel<32, 1>);
-  else go(&attn_keep_streams_kernel<18, 32, 0>, &attn_keep_streams_merge_kernel<32, 0>);
+  if (sigmoid && cap) launch_streams_one<18, 32, 3>(a, T, NA, S, part);
+  else if (sigmoid) launch_streams_one<18, 32, 2>(a, T, NA, S, part);
+  else if (cap) launch_streams_one<18, 32, 1>(a, T, NA, S, part);
+  else launch_streams_one<18, 32, 0>(a, T, NA, S, part);
 }
 
 bool launch_attn_keep_mfma(const float* q, const void* k_cache, const void* v_cache, int64_t vrs,
