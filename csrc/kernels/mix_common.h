@@ -33,6 +33,20 @@ __device__ __forceinline__ float wave_max(float v) {
   return v;
 }
 
+// 64 lanes' pieces of 16 bytes from base + offset (per lane) to LDS, one after another from byte `to` (the same for
+// the wave) on.  Written out: behind the builtin the compiler waits for the copy before any later LDS read through a
+// builtin.  The caller waits with s_waitcnt vmcnt(0).  M0 is named as overwritten, so that a builtin's copy behind it
+// sets its own; the compiler warns of such a name because it saves no value there, and none is kept in M0 across.
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"
+__device__ __forceinline__ void lds_copy16(const void* base, uint32_t offset, uint32_t to) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
+               ::"v"(offset), "s"(base), "s"(__builtin_amdgcn_readfirstlane(to)) : "memory", "m0");
+#endif
+}
+#pragma clang diagnostic pop
+
 // Sum over each aligned group of L neighbouring lanes (L = 4, 8, .. 64, the same for the whole wave);
 // every lane of the group receives it.  The first four steps stay inside a row of 16 lanes.
 __device__ __forceinline__ float group_sum(float v, int L) {

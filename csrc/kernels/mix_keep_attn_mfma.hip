@@ -167,16 +167,6 @@ __device__ __forceinline__ void store_rows32(const KeepArgs& a, const f32x16 (&o
     }
 }
 
-// 64 lanes' pieces of 16 bytes from base + offset (per lane) to LDS, one after another from byte `to` (the same for
-// the wave) on.  Written out: behind the builtin the compiler waits for the copy before any later LDS read through a
-// builtin, here for the next page in the middle of this one.  The caller waits with s_waitcnt vmcnt(0).  Nothing
-// else in a kernel that uses it may rely on M0.
-__device__ __forceinline__ void lds_copy16(const void* base, uint32_t offset, uint32_t to) {
-#if defined(__HIP_DEVICE_COMPILE__)
-  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
-               ::"v"(offset), "s"(base), "s"(__builtin_amdgcn_readfirstlane(to)) : "memory");
-#endif
-}
 __device__ __forceinline__ uint32_t lds_byte(const unsigned char* smem) {      // where the dynamic LDS begins
   return (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const unsigned char*)smem;
 }
