@@ -519,6 +519,9 @@ def _cus(index: int) -> int:
     return torch.cuda.get_device_properties(index).multi_processor_count
 
 
+_ROUND_MIN_ROWS, _ROUND_MAX_N = 1024, 14336     # a round of 256 CUs has at least 1,024 rows up to 14,336 columns
+
+
 def _round_rows(x, w) -> int:
     """Rows of x w^T that make whole rounds of 256 x 256 tiles over the chip, where the library takes
     less time for them and for the others than for all of them; 0 where it does not, or where a
@@ -532,9 +535,12 @@ def _round_rows(x, w) -> int:
     4,096: 4,385 rows 168 and 170).  After more rounds they lose with up to 4,096 terms (5,300 rows: 183 and
     203), and gain with 8,192 up to seven tenths after two to four (10,240 x 8,192: 3,742 rows 641 -> 455, 4,826:
     778 -> 578, 6,556: 927 -> 769), not after five (7,764: 870 and 911)."""
-    M, N, K = x.shape[0], w.shape[0], x.shape[1]
-    if (not _gpu(x) or x.dtype != torch.bfloat16 or w.dtype != torch.bfloat16 or N % 256 != 0 or N == 0 or K < 2048
-            or x.stride(1) != 1 or w.stride(1) != 1 or (N, K) in _SPLIT_PLAN or tiled_only(w)
+    M = x.shape[0]
+    if M <= _ROUND_MIN_ROWS:                                 # steps of few rows are bound by the host: nothing else first
+        return 0
+    N, K = w.shape[0], x.shape[1]
+    if (not _gpu(x) or x.dtype != torch.bfloat16 or w.dtype != torch.bfloat16 or N % 256 != 0 or not 0 < N <= _ROUND_MAX_N
+            or K < 2048 or x.stride(1) != 1 or w.stride(1) != 1 or (N, K) in _SPLIT_PLAN or tiled_only(w)
             or linear_plan(M, N, K) >= 0 or not _plain(x, w)):
         return 0
     per = _cus(x.device.index) // (N // 256) * 256           # rows of a round
