@@ -527,29 +527,38 @@ def _round_rows(x, w) -> int:
     less time for them and for the others than for all of them; 0 where it does not, or where a
     start-up plan, a tiled copy or a derivative has the word.
 
-    The library gives a grid that does not fill its last round tiles of another size, or half a chip of
-    work: 2,767 rows by 6,144 x 4,096 take 210 us, 2,560 of them 85 and the others 24.  Up to half a
-    round beyond the first one the two products were faster for all three classes of decoders, by 0 - 84
-    percent (3,072 x 2,048: 5,377 rows 71 -> 60 us, 8,064: 86 -> 84; 6,144 x 4,096: 2,561: 115 -> 103, 3,840:
-    153 -> 153; 10,240 x 8,192: 1,537: 244 -> 202, 2,304: 308 -> 291); beyond it they are even or lose (6,144 x
-    4,096: 4,385 rows 168 and 170).  After more rounds they lose with up to 4,096 terms (5,300 rows: 183 and
-    203), and gain with 8,192 up to seven tenths after two to four (10,240 x 8,192: 3,742 rows 641 -> 455, 4,826:
-    778 -> 578, 6,556: 927 -> 769), not after five (7,764: 870 and 911)."""
+    The library gives a grid that just passes a whole round tiles of another size, or half a chip of
+    work: 2,767 rows by 6,144 x 4,096 take 210 us, 2,560 of them 85 and the others 24.  The bounds are
+    where the two products were never slower (one product's time over theirs, one MI355X, 2,048 to 14,336
+    columns and 2,048 to 16,384 terms):
+    one round that keeps 15/16 of the CUs busy and up to a tenth more, from 3,072 terms on (from 2,048 up to
+    4,096 columns): 1.00 - 2.3, on the average 1.35 (with 2,048 terms 0.97 for 4,608 and 6,144 columns; an
+    eighth more 0.98; a quarter 0.89 for 9,216; rounds of 238 tiles 0.91, of 224 0.78);
+    two to four rounds and up to six tenths more, 8,192 to 9,216 terms, 7,168 to 11,264 columns, unless the
+    tiles of all rows fit as many rounds: 0.99 - 1.8, on the average 1.20 (tiles that fit 0.86 - 0.99; 10,240
+    terms 0.55 - 1.8)."""
     M = x.shape[0]
     if M <= _ROUND_MIN_ROWS:                                 # steps of few rows are bound by the host: nothing else first
         return 0
     N, K = w.shape[0], x.shape[1]
-    if (not _gpu(x) or x.dtype != torch.bfloat16 or w.dtype != torch.bfloat16 or N % 256 != 0 or not 0 < N <= _ROUND_MAX_N
-            or K < 2048 or x.stride(1) != 1 or w.stride(1) != 1 or (N, K) in _SPLIT_PLAN or tiled_only(w)
-            or linear_plan(M, N, K) >= 0 or not _plain(x, w)):
+    if N % 256 or not 2048 <= N <= _ROUND_MAX_N or not 2048 <= K <= 16384 or not _gpu(x):
         return 0
-    per = _cus(x.device.index) // (N // 256) * 256           # rows of a round
+    cus, cols = _cus(x.device.index), N // 256
+    per = cus // cols * 256                                  # rows of a round
     if per == 0:
         return 0
     rounds, rest = M // per, M % per
-    if rest and ((rounds == 1 and 2 * rest <= per) or (K >= 8192 and 2 <= rounds <= 4 and 10 * rest <= 7 * per)):
-        return rounds * per
-    return 0
+    if rest == 0:
+        return 0
+    if rounds == 1:
+        ok = 10 * rest <= per and 16 * (cus // cols * cols) >= 15 * cus and (K >= 3072 or N <= 4096)
+    else:
+        ok = (2 <= rounds <= 4 and 10 * rest <= 6 * per and 8192 <= K <= 9216 and 7168 <= N <= 11264
+              and -(-M // 256) * cols > rounds * cus)
+    if (not ok or x.dtype != torch.bfloat16 or w.dtype != torch.bfloat16 or x.stride(1) != 1 or w.stride(1) != 1
+            or (N, K) in _SPLIT_PLAN or tiled_only(w) or linear_plan(M, N, K) >= 0 or not _plain(x, w)):
+        return 0
+    return rounds * per
 
 
 def attn_decode_merge(part_o, part_ml, out, Hq, num_splits):

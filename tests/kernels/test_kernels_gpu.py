@@ -1211,16 +1211,18 @@ def test_linear_zero_rows_with_rows_plan(gpu):
         ops.reset_plans()
 
 
-@pytest.mark.parametrize("M,parts", [(2560, 1), (2561, 2), (3840, 2), (3841, 1)])
-def test_qkv_rope_in_two_products(M, parts):
-    """Steps just over a whole round of the library's tiles take two products: the same rows and caches."""
-    Hq, Hkv, K = 32, 8, 2048
+@pytest.mark.parametrize("M,head,Hq,K", [(2560, 0, 32, 3072), (2561, 2560, 32, 3072), (2816, 2560, 32, 3072),
+                                         (2817, 0, 32, 3072), (3073, 3072, 64, 8192), (3993, 3072, 64, 8192),
+                                         (3994, 0, 64, 8192)])
+def test_qkv_rope_in_two_products(M, head, Hq, K):
+    """Steps just over whole rounds of the library's tiles take two products: the same rows and caches."""
+    Hkv = 8
     N = (Hq + 2 * Hkv) * 128
     g = torch.Generator().manual_seed(M)
     x = torch.randn(M, K, generator=g).to("cuda", torch.bfloat16)
     w = (torch.randn(N, K, generator=g) * K ** -0.5).to("cuda", torch.bfloat16)
     ops.reset_plans()
-    assert ops._round_rows(x, w) == (2560 if parts == 2 else 0) or ops._cus(0) != 256
+    assert ops._round_rows(x, w) == head or ops._cus(0) != 256
     pos = torch.arange(M, dtype=torch.int32, device="cuda") % 512
     ang = torch.arange(512)[:, None] * 1e4 ** (-torch.arange(0, 128, 2) / 128)
     cs = torch.cat([ang.cos(), ang.sin()], -1).float().cuda()
