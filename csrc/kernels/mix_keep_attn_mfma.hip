@@ -239,14 +239,16 @@ __global__ __launch_bounds__(64 * HPW, 2) void attn_keep_tile_kernel(const KeepA
   // ---- staging: LDS-DMA, 64 pieces of 16 bytes a time, permuted at the source
   constexpr int NPK = WBS * E / 512, NPV = SHARED ? 0 : WBS * vdim / 512;
   constexpr int NK = (NPK + HPW - 1) / HPW, NV = (NPV + HPW - 1) / HPW;
-  uint32_t ksrc[NK], vsrc[NV > 0 ? NV : 1];
+  // rows 16 apart are permuted alike: a wave whose pieces lie so needs the offsets of half of them
+  constexpr int UK = NPK % (2 * HPW) == 0 ? NK / 2 : NK, UV = NPV % (2 * HPW) == 0 ? NV / 2 : NV;
+  uint32_t ksrc[UK], vsrc[UV > 0 ? UV : 1];
 #pragma unroll
-  for (int i = 0; i < NK; ++i) {
+  for (int i = 0; i < UK; ++i) {
     const int x = (wid + i * HPW) * 64 + lane, r = x / (E / 8), c = x - r * (E / 8);
     ksrc[i] = (r * E + (c ^ page_swizzle<E>(r)) * 8) * 2;
   }
 #pragma unroll
-  for (int i = 0; i < NV; ++i) {
+  for (int i = 0; i < UV; ++i) {
     const int x = (wid + i * HPW) * 64 + lane, r = x / (vdim / 8), c = x - r * (vdim / 8);
     vsrc[i] = (r * (int)a.vrs + (c ^ page_swizzle<vdim>(r)) * 8) * 2;
   }
@@ -256,7 +258,7 @@ __global__ __launch_bounds__(64 * HPW, 2) void attn_keep_tile_kernel(const KeepA
     for (int i = 0; i < NK; ++i) {
       const int piece = wid + i * HPW;
       if ((i + 1) * HPW <= NPK || piece < NPK)
-        lds_copy16(kb, ksrc[i], lds0 + 2 * (buf * KP + piece * (E == 128 ? 520 : 512)));
+        lds_copy16(kb + i / UK * (WBS * E), ksrc[i % UK], lds0 + 2 * (buf * KP + piece * (E == 128 ? 520 : 512)));
     }
   };
   auto fetch_v = [&](int page, int buf) {
@@ -266,7 +268,7 @@ __global__ __launch_bounds__(64 * HPW, 2) void attn_keep_tile_kernel(const KeepA
       for (int i = 0; i < NV; ++i) {
         const int piece = wid + i * HPW;
         if ((i + 1) * HPW <= NPV || piece < NPV)
-          lds_copy16(vb, vsrc[i], lds0 + 2 * (2 * KP + buf * VP + piece * (vdim == 128 ? 520 : 512)));
+          lds_copy16(vb + i / UV * (WBS * a.vrs), vsrc[i % UV], lds0 + 2 * (2 * KP + buf * VP + piece * (vdim == 128 ? 520 : 512)));
       }
     }
   };
