@@ -136,6 +136,226 @@ __device__ __forceinline__ void store_rows(const KeepArgs& a, f32x4 (&o)[DV], fl
   }
 }
 
+template <int DK, int DV, bool SHARED>
+constexpr int keep_page_shorts() {
+  return WBS * (32 * DK + 8) + (SHARED ? 0 : WBS * (16 * DV + 8));
+}
+
+// DK = E / 32, DV = vdim / 16, HPW heads per workgroup, SHARED: values = leading entries of the key rows, MODE: 0
+// softmax, 1 softmax of capped scores, 2 sigmoid, 3 sigmoid of capped scores.
+//
+// Groups of one or two heads where the chip is not full (small_groups): a wave has 16 queries of a head on 16 x 16
+// tiles, so that a head's 32 queries are two waves side by side, with half the weights to make each; pages come through
+// registers into padded rows.  The tiles of 32 queries below leave half of the SIMDs idle there, and sigmoid weights,
+// two transcendental instructions each and no maximum to wait for, are their time (eight prompts of 200, 12 heads over
+// 2 of 128, sigmoid: 15 us against 17 there).  Two heads a workgroup: three waves a SIMD, which the compiler left to
+// itself spends on 180 registers for two.
+template <int DK, int DV, int HPW, bool SHARED, int MODE>
+__global__ __launch_bounds__(128 * HPW, HPW == 2 ? 3 : 1) void attn_keep_mfma_kernel(const KeepArgs a) {
+  constexpr int E = 32 * DK, vdim = 16 * DV, NT = 128 * HPW;
+  constexpr int KRS = E + 8;                       // shorts per key row in LDS (+ 16 bytes)
+  constexpr int VRS = SHARED ? KRS : vdim + 8;     // shorts per value row
+  constexpr int PGS = keep_page_shorts<DK, DV, SHARED>();
+  const int item = gridDim.x - 1 - blockIdx.x;     // a sequence's later blocks see the most keys: they start first
+  const int s = a.work_seq[item];
+  if (s < 0) return;
+  const int ql = a.q_len[s];
+  const int i0 = a.work_qblk[item] * WQB;
+  if (i0 >= ql) return;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int col = lane & 15, grp = lane >> 4;
+  const int g = ((int)blockIdx.y * HPW) / (a.H / a.G);
+  const int hh = (int)blockIdx.y * HPW + (wid >> 1);
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  short* const pages = reinterpret_cast<short*>(smem);       // two of them
+
+  const int nq = min(WQB, ql - i0);
+  const int p0 = a.kv_len[s] - ql + i0, plast = p0 + nq - 1;
+  const int window = a.window, keep_first = a.keep_first;
+  const int jwin = window > 0 ? max(0, p0 - window + 1) : 0;
+  const int kf = window > 0 ? min(keep_first, jwin) : 0;     // kept keys before the window
+  const int row = (wid & 1) * 16 + col, pi = p0 + row;       // this lane's query
+  const bool qlive = row < nq;
+  const int64_t t = a.q_start[s] + i0 + (qlive ? row : 0);
+  typedef const __attribute__((address_space(4))) int32_t const_i32;
+  const_i32* bt = (const_i32*)(uintptr_t)(a.bt + (int64_t)s * a.maxb);
+
+  // scores arrive as exponents of 2: s log2 e; 2 s log2 e / cap; -s log2 e (sigmoid, no cap)
+  const float qmul = a.scale * (MODE % 2 == 1 ? 2.f * kLog2e / a.softcap : MODE == 2 ? -kLog2e : kLog2e);
+  const float cap2 = MODE % 2 == 1 ? a.softcap * kLog2e : 0.f;
+  s16x8 qhi[DK], qlo[DK];
+  {
+    const float* qp = a.q + (t * a.H + hh) * E + grp * 8;
+#pragma unroll
+    for (int ks = 0; ks < DK; ++ks) {
+      const float4 x = *reinterpret_cast<const float4*>(qp + ks * 32);
+      const float4 y = *reinterpret_cast<const float4*>(qp + ks * 32 + 4);
+      const float f[8] = {x.x * qmul, x.y * qmul, x.z * qmul, x.w * qmul, y.x * qmul, y.y * qmul, y.z * qmul, y.w * qmul};
+      split_bf16w(f, qhi[ks], qlo[ks]);
+    }
+  }
+  f32x4 o[DV];
+#pragma unroll
+  for (int m = 0; m < DV; ++m) o[m] = (f32x4){0.f, 0.f, 0.f, 0.f};
+  const float hb = a.head_bias != nullptr ? a.head_bias[hh] * kLog2e : 0.f;
+  const bool sink = MODE < 2 && a.head_bias != nullptr;
+  // the sink is one more entry of the row: it starts the maximum, and one lane's part of the sum
+  float mrun = sink ? hb : kNegInfW, lrun = sink && grp == 0 ? 1.f : 0.f;
+
+  // ---- staging
+  constexpr int NKV = (WBS * E / 8 + NT - 1) / NT;
+  constexpr int NVV = SHARED ? 1 : (WBS * vdim / 8 + NT - 1) / NT;
+  s16x8 kreg[NKV], vreg[NVV];
+  auto fetch = [&](int page) {
+    const int64_t at = ((int64_t)page * a.G + g) * WBS;      // the page's first slot
+    const bf16_t* kb = static_cast<const bf16_t*>(a.k_cache) + at * E;
+#pragma unroll
+    for (int i = 0; i < NKV; ++i) {
+      const int x = tid + i * NT;
+      if (x < WBS * E / 8) kreg[i] = reinterpret_cast<const s16x8*>(kb)[x];
+    }
+    if constexpr (!SHARED) {
+      const bf16_t* vb = static_cast<const bf16_t*>(a.v_cache) + at * a.vrs;
+#pragma unroll
+      for (int i = 0; i < NVV; ++i) {
+        const int x = tid + i * NT;
+        if (x < WBS * vdim / 8) {
+          const int jj = x / (vdim / 8), c = x - jj * (vdim / 8);
+          vreg[i] = *reinterpret_cast<const s16x8*>(vb + jj * a.vrs + c * 8);
+        }
+      }
+    }
+  };
+  // Rows past the sequence's end were never written and may hold anything: zeros.
+  auto stage = [&](int jb, int buf) {
+    short* Ks = pages + buf * PGS;
+    short* Vs = SHARED ? Ks : Ks + WBS * KRS;
+    const bool tail = jb + WBS - 1 > plast;
+#pragma unroll
+    for (int i = 0; i < NKV; ++i) {
+      const int x = tid + i * NT;
+      if (x < WBS * E / 8) {
+        const int jj = x / (E / 8), c = x - jj * (E / 8);
+        s16x8 v = kreg[i];
+        if (SHARED && tail && jb + jj > plast) v = (s16x8){0, 0, 0, 0, 0, 0, 0, 0};
+        *reinterpret_cast<s16x8*>(Ks + jj * KRS + c * 8) = v;
+      }
+    }
+    if constexpr (!SHARED) {
+#pragma unroll
+      for (int i = 0; i < NVV; ++i) {
+        const int x = tid + i * NT;
+        if (x < WBS * vdim / 8) {
+          const int jj = x / (vdim / 8), c = x - jj * (vdim / 8);
+          s16x8 v = vreg[i];
+          if (tail && jb + jj > plast) v = (s16x8){0, 0, 0, 0, 0, 0, 0, 0};
+          *reinterpret_cast<s16x8*>(Vs + jj * VRS + c * 8) = v;
+        }
+      }
+    }
+  };
+  const int kat = col * KRS + grp * 8;
+  // transposed reads: a 16-lane group takes 4 key rows x 16 value columns, lane `col` receives its
+  // column (keys 4 grp .. 4 grp + 3 of each 16-key half)
+  const int vat = (4 * grp + (col >> 2)) * VRS + 4 * (col & 3);
+
+  // pages [0 .. pg_keep] hold the kept first tokens, pages [pg_win .. pg_last] the window
+  const int pg_last = plast / WBS;
+  const int pg_keep = kf > 0 ? (kf - 1) / WBS : -1;
+  const int pg_win = jwin / WBS;
+  auto next_page = [&](int pg) { return (pg == pg_keep && pg_win > pg) ? pg_win : pg + 1; };
+  int pg = kf > 0 ? 0 : pg_win, buf = 0;
+  fetch(bt[pg]);
+  stage(pg * WBS, 0);
+  int pn = next_page(pg);
+  if (pn <= pg_last) fetch(bt[pn]);
+  __syncthreads();
+  while (pg <= pg_last) {
+    const int jb = pg * WBS;
+    const short* Ks = pages + buf * PGS;
+    const short* Vs = SHARED ? Ks : Ks + WBS * KRS;
+    f32x4 sc[2][2];                                          // two chains per half page
+#pragma unroll
+    for (int kt = 0; kt < 2; ++kt) {
+      sc[kt][0] = sc[kt][1] = (f32x4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int ks = 0; ks < DK; ++ks) {
+        const s16x8 k = *reinterpret_cast<const s16x8*>(Ks + kat + kt * 16 * KRS + ks * 32);
+        sc[kt][0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(k), as_bf16x8(qhi[ks]), sc[kt][0], 0, 0, 0);
+        sc[kt][1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(k), as_bf16x8(qlo[ks]), sc[kt][1], 0, 0, 0);
+      }
+    }
+    float p[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      float x = sc[i >> 2][0][i & 3] + sc[i >> 2][1][i & 3];
+      if constexpr (MODE % 2 == 1) x = cap2 - 2.f * cap2 * __builtin_amdgcn_rcpf(__builtin_amdgcn_exp2f(x) + 1.f);
+      if constexpr (MODE >= 2) x = __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f((MODE == 3 ? -x : x) - hb));
+      p[i] = x;
+    }
+    if (!(jb + WBS - 1 <= p0 && (window <= 0 || plast - jb < window || jb + WBS <= keep_first))) {
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {                          // an edge inside the page
+        const int j = jb + (i >> 2) * 16 + grp * 4 + (i & 3);
+        const bool ok = j <= pi && (window <= 0 || pi - j < window || j < keep_first);
+        p[i] = ok ? p[i] : MODE >= 2 ? 0.f : kNegInfW;
+      }
+    }
+    if constexpr (MODE < 2) {
+      float mx = fmaxf(fmaxf(fmaxf(p[0], p[1]), fmaxf(p[2], p[3])), fmaxf(fmaxf(p[4], p[5]), fmaxf(p[6], p[7])));
+      mx = other_half_max(other_row_max(mx));
+      const bool moves = mx > mrun + kDeferW;                // also for the first keys: mrun = -inf
+      if (__builtin_amdgcn_ballot_w64(moves) != 0ull) {
+        const float mn = moves ? mx : mrun;
+        const float alpha = moves ? __builtin_amdgcn_exp2f(mrun - mn) : 1.f;
+        mrun = mn;
+        lrun *= alpha;
+#pragma unroll
+        for (int m = 0; m < DV; ++m) o[m] *= alpha;
+      }
+      const float mu = mrun == kNegInfW ? 0.f : mrun;        // no visible key so far: every weight 0
+      float l0 = 0.f, l1 = 0.f;
+#pragma unroll
+      for (int i = 0; i < 8; i += 2) {
+        p[i] = __builtin_amdgcn_exp2f(p[i] - mu);
+        p[i + 1] = __builtin_amdgcn_exp2f(p[i + 1] - mu);
+        l0 += p[i];
+        l1 += p[i + 1];
+      }
+      lrun += l0 + l1;
+    }
+    s16x8 phi, plo;
+    split_bf16w(p, phi, plo);
+    constexpr int MG = DV % 4 == 0 ? 4 : 2;                  // value blocks taken together
+#pragma unroll
+    for (int m = 0; m < DV; m += MG) {
+      s16x8 v[MG];
+#pragma unroll
+      for (int u = 0; u < MG; ++u) {
+        const s16x4 a0 = rfq::ds_read_tr16(Vs + vat + 16 * (m + u));
+        const s16x4 a1 = rfq::ds_read_tr16(Vs + vat + 16 * VRS + 16 * (m + u));
+        v[u] = (s16x8){a0[0], a0[1], a0[2], a0[3], a1[0], a1[1], a1[2], a1[3]};
+      }
+#pragma unroll
+      for (int u = 0; u < MG; ++u)
+        o[m + u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(v[u]), as_bf16x8(phi), o[m + u], 0, 0, 0);
+#pragma unroll
+      for (int u = 0; u < MG; ++u)
+        o[m + u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(v[u]), as_bf16x8(plo), o[m + u], 0, 0, 0);
+    }
+    pg = pn;
+    if (pg <= pg_last) {
+      stage(pg * WBS, buf ^ 1);          // it has been on its way since the last page
+      pn = next_page(pg);
+      if (pn <= pg_last) fetch(bt[pn]);
+    }
+    __syncthreads();
+    buf ^= 1;
+  }
+  store_rows<DV, MODE>(a, o, lrun, t, hh, grp, qlive);
+}
+
 // lane (col, half) of a 32 x 32 tile holds value channels 32 m + 8 b + 4 half .. + 3 of its query: 8-byte stores
 template <int VM, int MODE>
 __device__ __forceinline__ void store_rows32(const KeepArgs& a, const f32x16 (&o)[VM], float lrun, int64_t t, int hh,
@@ -171,9 +391,6 @@ __device__ __forceinline__ uint32_t lds_byte(const unsigned char* smem) {      /
   return (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const unsigned char*)smem;
 }
 
-// DK = E / 32, DV = vdim / 16, HPW heads per workgroup, SHARED: values = leading entries of the key rows, MODE: 0
-// softmax, 1 softmax of capped scores, 2 sigmoid, 3 sigmoid of capped scores.
-//
 // A row's 16-byte pieces are permuted inside it, and rows of 256 bytes lie 16 bytes apart after every four, so
 // that the pieces that one LDS access takes together (K: a piece of 16 neighbouring rows; V, transposed: 64
 // bytes of four neighbouring rows) lie on different banks.
@@ -1133,13 +1350,39 @@ static void launch_keep_mfma_one(const KeepArgs& a) {
   else run(&attn_keep_tile_kernel<DK, DV, HPW, SHARED, MODE>, 64 * HPW);
 }
 
+// Groups of fewer than four heads a workgroup whose 32 queries are better two waves: rows of up to three pages, where
+// the way to the first page is the time (one prompt of 33 tokens, two heads a group: 0.91 - 0.97 of the other kernel's
+// time; of one head a group only sigmoid weights of latents, 0.88 - 0.97), and sigmoid weights of two heads a workgroup
+// up to 1,024 workgroups, four waves to a CU of the other kernel (1 - 32 prompts of 33 - 1,200 tokens: 0.75 - 1.0 of its
+// time, where it has fewer than 512; from 1,024 on the other is as fast or takes down to 0.6 of this one's).
+template <int HPW, bool SHARED, int MODE>
+static bool small_groups(const KeepArgs& a) {
+  if constexpr (HPW == 1 && SHARED && MODE >= 2) return a.maxb <= 3;
+  if constexpr (HPW == 2) return a.maxb <= 3 || (MODE >= 2 && (int64_t)a.W * (a.H / HPW) < 1024);
+  return false;
+}
+
+template <int DK, int DV, int HPW, bool SHARED, int MODE>
+static void launch_keep_small_one(const KeepArgs& a) {
+  constexpr size_t lds = (size_t)2 * keep_page_shorts<DK, DV, SHARED>() * sizeof(short);
+  static_assert(lds <= 64 * 1024, "LDS without an allowance");
+  hipLaunchKernelGGL((attn_keep_mfma_kernel<DK, DV, HPW, SHARED, MODE>), dim3(a.W, a.H / HPW), dim3(128 * HPW), lds, a.s, a);
+}
+
+template <int DK, int DV, int HPW, bool SHARED, int MODE>
+static void launch_keep_mfma_any(const KeepArgs& a) {
+  if constexpr (!(SHARED && DK >= 10) && (HPW == 2 || (HPW == 1 && SHARED && MODE >= 2)))
+    if (small_groups<HPW, SHARED, MODE>(a)) return launch_keep_small_one<DK, DV, HPW, SHARED, MODE>(a);
+  launch_keep_mfma_one<DK, DV, HPW, SHARED, MODE>(a);
+}
+
 template <int DK, int DV, int HPW, bool SHARED>
 static void launch_keep_mfma_mode(const KeepArgs& a) {
   const bool cap = a.softcap > 0.f;
-  if (a.sigmoid && cap) launch_keep_mfma_one<DK, DV, HPW, SHARED, 3>(a);
-  else if (a.sigmoid) launch_keep_mfma_one<DK, DV, HPW, SHARED, 2>(a);
-  else if (cap) launch_keep_mfma_one<DK, DV, HPW, SHARED, 1>(a);
-  else launch_keep_mfma_one<DK, DV, HPW, SHARED, 0>(a);
+  if (a.sigmoid && cap) launch_keep_mfma_any<DK, DV, HPW, SHARED, 3>(a);
+  else if (a.sigmoid) launch_keep_mfma_any<DK, DV, HPW, SHARED, 2>(a);
+  else if (cap) launch_keep_mfma_any<DK, DV, HPW, SHARED, 1>(a);
+  else launch_keep_mfma_any<DK, DV, HPW, SHARED, 0>(a);
 }
 
 template <int DK, int DV, bool SHARED>

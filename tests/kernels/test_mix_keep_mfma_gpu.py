@@ -184,6 +184,22 @@ def test_prompt_rows(H, G, E, vd, shared):
     _check(H, G, E, vd, shared, seqs=PROMPTS, prompt=True, window=64, keep_first=40)
 
 
+@pytest.mark.parametrize("H,G,E,vd,shared", [(2, 1, 128, 128, False), (24, 4, 64, 64, False), (12, 2, 32, 128, False),
+                                             (6, 1, 96, 64, True), (3, 1, 192, 128, True), (4, 2, 160, 128, True)])
+def test_prompt_rows_of_small_groups(H, G, E, vd, shared):
+    """Both sides of where groups of one and two heads change kernels: three pages and four, 1,024 workgroups."""
+    for n in (96, 97):
+        seqs = [(n, n), (1, 1), (33, 33), (40, 7), (40, 0)]
+        _check(H, G, E, vd, shared, seqs=seqs, prompt=True, bias=True, gate="head")
+        _check(H, G, E, vd, shared, seqs=seqs, prompt=True, softcap=20.0, window=37, keep_first=5)
+        _check(H, G, E, vd, shared, seqs=seqs, prompt=True, sigmoid=True, bias=True, gate="output")
+    per = H // 2 if H // G % 2 == 0 else H
+    for items in (1023 // per - 1, 1024 // per):             # one more item is padding
+        seqs = [(70, 70)] * (items // 3) + [(32, 32)] * (items % 3)
+        _check(H, G, E, vd, shared, seqs=seqs, prompt=True, sigmoid=True, bias=True)
+        _check(H, G, E, vd, shared, seqs=seqs, prompt=True, sigmoid=True, bias=True, softcap=20.0)
+
+
 @pytest.mark.parametrize("H,G,E,vd,shared", [(4, 1, 128, 128, False), (2, 1, 64, 64, False), (1, 1, 32, 32, False),
                                              (4, 1, 96, 64, True), (2, 1, 192, 128, True), (4, 1, 576, 512, True)])
 def test_long_chains_of_pages(H, G, E, vd, shared):
