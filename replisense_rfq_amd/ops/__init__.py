@@ -525,7 +525,7 @@ _ROUND_MIN_ROWS, _ROUND_MAX_N = 1024, 14336     # a round of 256 CUs has at leas
 def _round_rows(x, w) -> int:
     """Rows of x w^T that make whole rounds of 256 x 256 tiles over the chip, where the library takes
     less time for them and for the others than for all of them; 0 where it does not, or where a
-    start-up plan, a tiled copy or a derivative has the word.
+    start-up plan, a tiled copy, autocast or a derivative has the word.
 
     The library gives a grid that just passes a whole round tiles of another size, or half a chip of
     work: 2,767 rows by 6,144 x 4,096 take 210 us, 2,560 of them 85 and the others 24.  The bounds are
@@ -556,7 +556,8 @@ def _round_rows(x, w) -> int:
         ok = (2 <= rounds <= 4 and 10 * rest <= 6 * per and 8192 <= K <= 9216 and 7168 <= N <= 11264
               and -(-M // 256) * cols > rounds * cus)
     if (not ok or x.dtype != torch.bfloat16 or w.dtype != torch.bfloat16 or x.stride(1) != 1 or w.stride(1) != 1
-            or (N, K) in _SPLIT_PLAN or tiled_only(w) or linear_plan(M, N, K) >= 0 or not _plain(x, w)):
+            or (N, K) in _SPLIT_PLAN or tiled_only(w) or linear_plan(M, N, K) >= 0 or torch.is_autocast_enabled("cuda")
+            or not _plain(x, w)):
         return 0
     return rounds * per
 

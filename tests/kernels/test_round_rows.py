@@ -54,3 +54,11 @@ def test_plans_copies_types_and_derivatives_have_the_word(chip):
     ops._SPLIT_PLAN.clear()
     chip.setattr(ops, "tiled_only", lambda t: True)
     assert ops._round_rows(x, w) == 0
+
+
+def test_autocast_has_the_word(chip):
+    """Under autocast to another type one product would give rows of that type, which the append refuses."""
+    x, w = _pair(2561, 6144, 4096)
+    assert ops._round_rows(x, w) == 2560
+    chip.setattr(torch, "is_autocast_enabled", lambda device: device == "cuda")      # no GPU, no autocast
+    assert ops._round_rows(x, w) == 0
