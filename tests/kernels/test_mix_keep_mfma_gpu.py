@@ -14,7 +14,7 @@ DEV, BS = "cuda", 32
 SEQS = [(1, 1), (31, 1), (32, 1), (33, 1), (129, 1), (257, 1), (300, 5), (40, 0), (700, 1), (70, 33)]
 
 
-def _check(H, G, E, vd, shared, seqs=SEQS, spoil=None, prompt=False, spare=0, **opt):
+def _check(H, G, E, vd, shared, seqs=SEQS, spoil=None, prompt=False, spare=0, rising=0.0, **opt):
     g = torch.Generator().manual_seed(H + E + vd)
     need = [(n + BS - 1) // BS for n, _ in seqs]
     perm = torch.randperm(sum(need), generator=g).tolist()
@@ -24,6 +24,8 @@ def _check(H, G, E, vd, shared, seqs=SEQS, spoil=None, prompt=False, spare=0, **
         at += nb
     nb = sum(need) + 1
     k = torch.randn(nb, G, BS, E, generator=g).bfloat16()
+    for t in tables if rising else ():           # later pages' scores are larger
+        k[t] = (k[t].float() * (1 + rising * torch.arange(len(t))[:, None, None, None])).bfloat16()
     v = k if shared else torch.randn(nb, G, BS, vd, generator=g).bfloat16()
     i32 = lambda x: torch.tensor(x, dtype=torch.int32)  # noqa: E731
     ql, kl, bt = i32([r for _, r in seqs]), i32([n for n, _ in seqs]), i32(tables)
@@ -36,6 +38,7 @@ def _check(H, G, E, vd, shared, seqs=SEQS, spoil=None, prompt=False, spare=0, **
                 x[tables[i][spoil // BS], :, spoil % BS] = float("inf")
     qs, T = torch.cumsum(ql, 0).int() - ql, int(ql.sum())
     q = torch.randn(T, H, E, generator=g) * 2
+    q = q.bfloat16().float() if rising else q    # large scores: no part of what is compared is their queries' rounding
     gate = opt.pop("gate", None)
     gate = None if gate is None else torch.randn(T, H * (vd if gate == "output" else 1), generator=g).bfloat16()
     bias = torch.randn(H, generator=g) - 1 if opt.pop("bias", False) else None
@@ -162,6 +165,16 @@ def test_wide_rows_in_streams_with_a_window(H, G):
         _check(H, G, 576, 512, True, seqs=seqs[9:], window=641, keep_first=0, spoil=50, bias=True, gate="head")  # no row sees 50
         _check(H, G, 576, 512, True, seqs=seqs, window=700, keep_first=40, softcap=20.0, gate="output")
         _check(H, G, 576, 512, True, seqs=seqs, window=610, keep_first=70, sigmoid=True, bias=True)
+
+
+@pytest.mark.parametrize("H,G,n", [(64, 1, 64), (32, 1, 128), (17, 1, 85)])
+def test_wide_rows_in_streams_of_many_turns(H, G, n):
+    """Two or three workgroups a row, up to eight turns of four pages each; the maximum moves in most of them."""
+    seqs = [(2016, 1), (1999, 1), (1300, 1), (257, 2), (33, 1)]
+    seqs += [(40, 0)] * (n - len(seqs))
+    _check(H, G, 576, 512, True, seqs=seqs, rising=0.1, bias=True, gate="head")
+    _check(H, G, 576, 512, True, seqs=seqs, rising=0.05, softcap=20.0, gate="output")
+    _check(H, G, 576, 512, True, seqs=seqs, window=1000, keep_first=70, sigmoid=True, bias=True)
 
 
 def test_few_pages_under_a_wide_table():
