@@ -95,6 +95,7 @@ struct KeepArgs {
   int H, G;
   float softcap, out_mult;
   hipStream_t s;
+  bool turned = false;                             // attn_keep_tile_kernel: a block's heads begin where the block says
 };
 
 // the same over lanes 16 away
@@ -417,7 +418,9 @@ __global__ __launch_bounds__(64 * HPW, 2) void attn_keep_tile_kernel(const KeepA
   constexpr int KP = page_row<E>(WBS), VP = page_row<VR>(WBS);
   const int groups = a.H / HPW;
   const int at = gridDim.x - 1 - blockIdx.x;       // a sequence's later blocks see the most keys: they start first
-  const int item = at / groups, hg = at - item * groups;
+  const int item = at / groups;
+  int hg = at - item * groups;
+  if (a.turned && (hg += item % groups) >= groups) hg -= groups;
   const int s = a.work_seq[item];
   if (s < 0) return;
   const int ql = a.q_len[s];
@@ -1339,8 +1342,15 @@ static void launch_keep_mfma_one(const KeepArgs& a) {
     }
     const int rep = a.H / a.G;
     const int groups = a.G * ((rep + HPW - 1) / HPW), most = std::max(1, (1 << 22) / groups);   // threads in 32 bits
+    // Heads side by side put a head group's blocks on one XCD where there are eight of them: each reads only its key
+    // heads' pages (32 heads over 8 of 128, sigmoid: 400 tokens 29.4 us a pass with the append, 32.1 with the groups
+    // turned by one from block to block), but its L2 sees an eighth of every row's columns, which costs the kernel
+    // that writes the next rows up to 4 us while queries and results just fill the L2s (780 tokens 46.5 against 42.9,
+    // 900 50.8 and 47.2; 64 heads, 500 tokens 40.8 and 38.8).  From 24 MB of queries on neither matters.
+    const int64_t queries = (int64_t)a.W * WQB * a.H * 32 * DK * sizeof(float);
     for (int w = 0; w < a.W; w += most) {
       KeepArgs part = a;
+      part.turned = queries > (8 << 20) && queries <= (24 << 20);
       part.work_seq += w;
       part.work_qblk += w;
       hipLaunchKernelGGL(kernel, dim3((unsigned)std::min(most, a.W - w) * groups), dim3(threads), lds, a.s, part);

@@ -222,6 +222,14 @@ def test_long_chains_of_pages(H, G, E, vd, shared):
     _check(H, G, E, vd, shared, seqs=seqs, prompt=True, window=400, keep_first=70, sigmoid=True, bias=True)
 
 
+@pytest.mark.parametrize("H,G", [(32, 8), (24, 6), (16, 4)])
+def test_blocks_whose_heads_are_turned(H, G):
+    """More than 8 MB of queries: the heads of a block begin where its number says."""
+    seqs = [(33, 33), (64 * 512 // H // 2, 64 * 512 // H // 2), (90, 17)]
+    _check(H, G, 128, 128, False, seqs=seqs, prompt=True, softcap=20.0, gate="head")
+    _check(H, G, 128, 128, False, seqs=seqs, prompt=True, window=100, keep_first=40, sigmoid=True, bias=True)
+
+
 def test_prompt_rows_with_rising_scores():
     """Every page moves the maximum by far: the accumulators are rescaled each time."""
     for shared, E, vd in ((False, 128, 128), (True, 576, 512)):
