@@ -3,7 +3,8 @@
 // tokens; softmax, softmax with a sink, or unnormalised sigmoid weights; optional output gate
 // (a column per head, or gate_w = vdim: one per output, rows 8-byte aligned);
 // the values may be the leading entries of the key rows themselves (latent attention).
-// Decode rows have a kernel of their own (mix_keep_split.hip).
+// Decode rows have kernels of their own: mix_keep_split.hip, and here those of wide latents in streams over several
+// workgroups (attn_keep_streams_kernel) and many heads at a time (attn_keep_wide_kernel, DEC).
 //
 // One workgroup per (work item, HPW heads of one key/value head); a work item is (sequence, block of 32 queries).
 // A wave has the 32 queries of a head: it keeps the running maximum and sum of its query columns and the weighted
@@ -27,10 +28,12 @@
 // the barrier.  The maximum is looked at lane by lane and moves only when a score passes it by 2^11, pages without an
 // edge inside skip the masks.  A block's workgroups lie side by side and blocks with the most keys start first, in
 // front of the others on their SIMD (s_setprio): the longest block's chain of pages is the end of a short step.
+// Groups of one or two heads a workgroup and short rows keep 16 queries a wave where the chip is not full
+// (small_groups).
 // Measured, the attention alone, against 16 x 16 tiles with a wave per 16 queries, compiler's order and heads one
 // after the other: prompts of 2,048 and 600 tokens (32 heads over 8 of 128, softcap) 194 -> 90 us, five ragged
-// prompts with sigmoid weights and a window of 1,024 72 -> 52 us, one prompt of 2,048 over 192-wide latents (32
-// heads) 177 -> 96 us; a workgroup alone takes 0.86 us a page, a full chip 1.1 us a page and CU.  Two pages to a
+// prompts with sigmoid weights and a window of 1,024 72 -> 51 us, one prompt of 2,048 over 192-wide latents (32
+// heads) 177 -> 96 us, sixteen chunks of 230 rows after 416 over two 192-wide latents of one head each 40 -> 27 us; a workgroup alone takes 0.86 us a page, a full chip 1.1 us a page and CU.  Two pages to a
 // barrier, two score chains, or operands four products ahead changed nothing.
 #include <algorithm>
 #include <type_traits>
@@ -145,8 +148,8 @@ constexpr int keep_page_shorts() {
 // DK = E / 32, DV = vdim / 16, HPW heads per workgroup, SHARED: values = leading entries of the key rows, MODE: 0
 // softmax, 1 softmax of capped scores, 2 sigmoid, 3 sigmoid of capped scores.
 //
-// Groups of one or two heads where the chip is not full (small_groups): a wave has 16 queries of a head on 16 x 16
-// tiles, so that a head's 32 queries are two waves side by side, with half the weights to make each; pages come through
+// Groups of one or two heads, and short rows, where the chip is not full (small_groups): a wave has 16 queries of a
+// head on 16 x 16 tiles, so that a head's 32 queries are two waves side by side, with half the weights to make each; pages come through
 // registers into padded rows.  The tiles of 32 queries below leave half of the SIMDs idle there, and sigmoid weights,
 // two transcendental instructions each and no maximum to wait for, are their time (eight prompts of 200, 12 heads over
 // 2 of 128, sigmoid: 15 us against 17 there).  Two heads a workgroup: three waves a SIMD, which the compiler left to
@@ -449,7 +452,9 @@ __global__ __launch_bounds__(64 * HPW, 2) void attn_keep_tile_kernel(const KeepA
   // pages [0, n_keep) hold the kept first tokens, pages [pg_win, pg_last] the window
   const int pg_last = plast / WBS, pg_win = jwin / WBS;
   const int n_keep = min((kf + WBS - 1) / WBS, pg_win), skip = pg_win - n_keep, turns = pg_last + 1 - skip;
-  // Long chains in front of the short ones that share their SIMD (2,048 and 600 tokens: 97 us without, 92 with).
+  // Long chains in front of the short ones that share their SIMD.  Over fourteen mixes of prompts, three head counts and
+  // three sizes it is worth half a percent: up to 11 % where long and short prompts or odd numbers of blocks meet, and
+  // 3 - 8 % lost on prompts of one length and on 192-wide rows.
   if (turns >= 32) __builtin_amdgcn_s_setprio(3);
   else if (turns >= 20) __builtin_amdgcn_s_setprio(2);
   else if (turns >= 10) __builtin_amdgcn_s_setprio(1);
@@ -958,10 +963,13 @@ __global__ __launch_bounds__(128 * HPW, DEC && HPW == 1 ? 1 : 2) void attn_keep_
 // What bounds it: the way to the first page (some 2 us for the step's numbers, 5 - 9 for page and queries), a page's
 // products (3 us), and 2 us for the streams to meet; so as many streams as the chip has room for, one workgroup to a
 // CU.  The queries are read once a workgroup and shared through LDS: read by every stream they held the pages up
-// (34 us for what takes 28 now).  A workgroup per 16 heads whose four waves took half a page a turn, copied through
-// registers (attn_keep_split_kernel), left half the CUs idle.  576 entries, before -> after with the merge: 64
-// sequences of 300 - 900 tokens with 32 heads 51 -> 35 us (alone; 61 -> 52 a layer's pass, which the host now bounds),
-// one of 611 37 -> 21, eight of 2,000 90 -> 29, 64 of 2,000 95 -> 51, 32 of 600 with 64 heads 40 -> 32.
+// (34 us for what took 28 without).  A workgroup has one row: a loop over a sequence's rows cost 10 - 17 spilled registers.
+// Workgroups without a page leave, a row that one workgroup has whole needs no merge, a row of one page no meeting.
+// A workgroup per 16 heads whose four waves took half a page a turn, copied through registers (attn_keep_split_kernel),
+// left half the CUs idle.  576 entries, before -> after with the merge: 64 sequences of 300 - 900 tokens with 32 heads
+// 51 -> 31 us (alone; 61 -> 51 a layer's pass, which the host now bounds), one of 600 36 -> 19, eight of 600 37 -> 18, 64
+// of 600 39 -> 30, with 64 heads 39 -> 33; 16 of 2,000 90 -> 32, 64 of them 91 -> 46, through a window of 1,024
+// 53 -> 36.
 constexpr int kStreams = 4;
 
 // What a row of the step sees: pages [0, n_keep) of its sequence s (-1: none, a row of a captured step beyond those of
@@ -1346,11 +1354,12 @@ static void launch_keep_mfma_one(const KeepArgs& a) {
     // heads' pages (32 heads over 8 of 128, sigmoid: 400 tokens 29.4 us a pass with the append, 32.1 with the groups
     // turned by one from block to block), but its L2 sees an eighth of every row's columns, which costs the kernel
     // that writes the next rows up to 4 us while queries and results just fill the L2s (780 tokens 46.5 against 42.9,
-    // 900 50.8 and 47.2; 64 heads, 500 tokens 40.8 and 38.8).  From 24 MB of queries on neither matters.
+    // 900 50.8 and 47.2; 64 heads, 500 tokens 40.8 and 38.8).  From 24 MB of queries on neither matters, with softmax
+    // weights they are even, and under eight pages the blocks' common pages count for more (16 prompts of 64 30.2, 31.5).
     const int64_t queries = (int64_t)a.W * WQB * a.H * 32 * DK * sizeof(float);
     for (int w = 0; w < a.W; w += most) {
       KeepArgs part = a;
-      part.turned = queries > (8 << 20) && queries <= (24 << 20);
+      part.turned = MODE >= 2 && a.maxb >= 8 && queries > (8 << 20) && queries <= (24 << 20);
       part.work_seq += w;
       part.work_qblk += w;
       hipLaunchKernelGGL(kernel, dim3((unsigned)std::min(most, a.W - w) * groups), dim3(threads), lds, a.s, part);
@@ -1360,16 +1369,22 @@ static void launch_keep_mfma_one(const KeepArgs& a) {
   else run(&attn_keep_tile_kernel<DK, DV, HPW, SHARED, MODE>, 64 * HPW);
 }
 
-// Groups of fewer than four heads a workgroup whose 32 queries are better two waves: rows of up to three pages, where
-// the way to the first page is the time (one prompt of 33 tokens, two heads a group: 0.91 - 0.97 of the other kernel's
-// time; of one head a group only sigmoid weights of latents, 0.88 - 0.97), and sigmoid weights of two heads a workgroup
-// up to 1,024 workgroups, four waves to a CU of the other kernel (1 - 32 prompts of 33 - 1,200 tokens: 0.75 - 1.0 of its
-// time, where it has fewer than 512; from 1,024 on the other is as fast or takes down to 0.6 of this one's).
+// Steps whose 32 queries of a head are better two waves, by the heads of a workgroup and its number `wgs`.
+// One or two heads: rows of up to three pages, where the way to the first page is the time (one prompt of 33 tokens,
+// two heads a group: 0.91 - 0.97 of the other kernel's time; of one head a group only sigmoid weights of latents, 0.88 -
+// 0.97), and sigmoid weights of two heads up to 1,024 workgroups, four waves to a CU of the other kernel (1 - 32 prompts
+// of 33 - 1,200 tokens: 0.75 - 1.0 of its time, where it has fewer than 512; from 1,024 on the other is as fast or takes
+// down to 0.6 of this one's).
+// Four heads are eight waves here, a workgroup to a CU: where that is one round, sigmoid weights over up to four pages,
+// over up to eight if most CUs have one, and any weights over two (passes with the append, 16 heads over 4 of 128: 8
+// prompts of 64 17.9 us against 19.3, 32 of them 28.2 and 31.0, softcap 34.3 and 35.7; 32 over 8, 4 of 200: 29.7 and
+// 32.0, 8 of 128 29.4 and 31.7; longer prompts 0 - 6 % the other way round).
 template <int HPW, bool SHARED, int MODE>
 static bool small_groups(const KeepArgs& a) {
-  if constexpr (HPW == 1 && SHARED && MODE >= 2) return a.maxb <= 3;
-  if constexpr (HPW == 2) return a.maxb <= 3 || (MODE >= 2 && (int64_t)a.W * (a.H / HPW) < 1024);
-  return false;
+  const int64_t wgs = (int64_t)a.W * (a.H / HPW);
+  if constexpr (HPW == 1) return SHARED && MODE >= 2 && a.maxb <= 3;
+  if constexpr (HPW == 2) return a.maxb <= 3 || (MODE >= 2 && wgs < 1024);
+  return wgs <= 256 && ((MODE >= 2 && a.maxb <= 4) || (wgs > 192 && a.maxb <= (MODE >= 2 ? 8 : 2)));
 }
 
 template <int DK, int DV, int HPW, bool SHARED, int MODE>
@@ -1381,7 +1396,7 @@ static void launch_keep_small_one(const KeepArgs& a) {
 
 template <int DK, int DV, int HPW, bool SHARED, int MODE>
 static void launch_keep_mfma_any(const KeepArgs& a) {
-  if constexpr (!(SHARED && DK >= 10) && (HPW == 2 || (HPW == 1 && SHARED && MODE >= 2)))
+  if constexpr (!(SHARED && DK >= 10) && (HPW > 1 || (SHARED && MODE >= 2)))
     if (small_groups<HPW, SHARED, MODE>(a)) return launch_keep_small_one<DK, DV, HPW, SHARED, MODE>(a);
   launch_keep_mfma_one<DK, DV, HPW, SHARED, MODE>(a);
 }

@@ -225,9 +225,23 @@ def test_long_chains_of_pages(H, G, E, vd, shared):
 @pytest.mark.parametrize("H,G", [(32, 8), (24, 6), (16, 4)])
 def test_blocks_whose_heads_are_turned(H, G):
     """More than 8 MB of queries: the heads of a block begin where its number says."""
-    seqs = [(33, 33), (64 * 512 // H // 2, 64 * 512 // H // 2), (90, 17)]
+    seqs = [(33, 33), (64 * 512 // H // 2, 64 * 512 // H // 2), (90, 17)]          # sigmoid weights only
     _check(H, G, 128, 128, False, seqs=seqs, prompt=True, softcap=20.0, gate="head")
     _check(H, G, 128, 128, False, seqs=seqs, prompt=True, window=100, keep_first=40, sigmoid=True, bias=True)
+
+
+@pytest.mark.parametrize("H,G,E,vd,shared", [(16, 4, 128, 128, False), (8, 2, 64, 32, False), (4, 1, 192, 128, True)])
+def test_short_rows_of_four_heads(H, G, E, vd, shared):
+    """Both sides of where four heads a workgroup change kernels: pages, and 192 and 256 workgroups."""
+    for n in (64, 65, 128, 129):
+        seqs = [(n, n), (1, 1), (33, 33), (40, 7), (40, 0)]
+        _check(H, G, E, vd, shared, seqs=seqs, prompt=True, sigmoid=True, bias=True, gate="output")
+    for wgs in (192, 193, 256, 257):
+        items = -(-wgs // (H // 4)) - 1                      # one more item is padding
+        for n, opt in ((64, {}), (65, {"softcap": 20.0}), (256, {"sigmoid": True, "bias": True}),
+                       (257, {"sigmoid": True, "bias": True, "softcap": 20.0})):
+            left = items - (n + 31) // 32
+            _check(H, G, E, vd, shared, seqs=[(n, n)] + [(32, 5)] * left, prompt=True, window=90, keep_first=40, **opt)
 
 
 def test_prompt_rows_with_rising_scores():
