@@ -33,8 +33,9 @@
 // Measured, the attention alone, against 16 x 16 tiles with a wave per 16 queries, compiler's order and heads one
 // after the other: prompts of 2,048 and 600 tokens (32 heads over 8 of 128, softcap) 194 -> 90 us, five ragged
 // prompts with sigmoid weights and a window of 1,024 72 -> 51 us, one prompt of 2,048 over 192-wide latents (32
-// heads) 177 -> 96 us, sixteen chunks of 230 rows after 416 over two 192-wide latents of one head each 40 -> 27 us; a workgroup alone takes 0.86 us a page, a full chip 1.1 us a page and CU.  Two pages to a
-// barrier, two score chains, or operands four products ahead changed nothing.
+// heads) 177 -> 96 us, sixteen chunks of 230 rows after 416 over two 192-wide latents of one head each 40 -> 27 us; a
+// workgroup alone takes 0.86 us a page, a full chip 1.1 us a page and CU.  Two pages to a barrier, two score chains, or
+// operands four products ahead changed nothing.
 #include <algorithm>
 #include <type_traits>
 #include <utility>
@@ -149,11 +150,11 @@ constexpr int keep_page_shorts() {
 // softmax, 1 softmax of capped scores, 2 sigmoid, 3 sigmoid of capped scores.
 //
 // Groups of one or two heads, and short rows, where the chip is not full (small_groups): a wave has 16 queries of a
-// head on 16 x 16 tiles, so that a head's 32 queries are two waves side by side, with half the weights to make each; pages come through
-// registers into padded rows.  The tiles of 32 queries below leave half of the SIMDs idle there, and sigmoid weights,
-// two transcendental instructions each and no maximum to wait for, are their time (eight prompts of 200, 12 heads over
-// 2 of 128, sigmoid: 15 us against 17 there).  Two heads a workgroup: three waves a SIMD, which the compiler left to
-// itself spends on 180 registers for two.
+// head on 16 x 16 tiles, so that a head's 32 queries are two waves side by side, with half the weights to make each;
+// pages come through registers into padded rows.  The tiles of 32 queries below leave half of the SIMDs idle there, and
+// sigmoid weights, two transcendental instructions each and no maximum to wait for, are their time (eight prompts of
+// 200, 12 heads over 2 of 128, sigmoid: 15 us against 17 there).  Two heads a workgroup: three waves a SIMD, which the
+// compiler left to itself spends on 180 registers for two.
 template <int DK, int DV, int HPW, bool SHARED, int MODE>
 __global__ __launch_bounds__(128 * HPW, HPW == 2 ? 3 : 1) void attn_keep_mfma_kernel(const KeepArgs a) {
   constexpr int E = 32 * DK, vdim = 16 * DV, NT = 128 * HPW;
@@ -1034,7 +1035,9 @@ __device__ __forceinline__ void store_gated(const KeepArgs& a, float (&y)[4], in
       make_uint2(rfq::pack_bf16x2(y[0], y[1]), rfq::pack_bf16x2(y[2], y[3]));
 }
 // How many of S workgroups have a part in the row: those with pages, the first in any case
-__device__ __forceinline__ int row_shares(const RowPages& r, int S) { return min(S, max(1, (r.pages + kStreams - 1) / kStreams)); }
+__device__ __forceinline__ int row_shares(const RowPages& r, int S) {
+  return min(S, max(1, (r.pages + kStreams - 1) / kStreams));
+}
 
 template <int DK, int DV, int MODE>
 __global__ __launch_bounds__(128 * kStreams, 2) void attn_keep_streams_kernel(const KeepArgs a, float* part, int T,
@@ -1278,8 +1281,10 @@ __global__ __launch_bounds__(128 * kStreams, 2) void attn_keep_streams_kernel(co
       }
       const int hc = g * rep + h0 + c, dv = mp * (vdim / 2) + dp;
       if (h0 + c >= rep) continue;
-      if (shares > 1) *reinterpret_cast<float4*>(part + ((t * S + z) * a.H + hc) * vdim + dv) = make_float4(y[0], y[1], y[2], y[3]);
-      else store_gated<vdim>(a, y, t, hc, dv);
+      if (shares > 1)
+        *reinterpret_cast<float4*>(part + ((t * S + z) * a.H + hc) * vdim + dv) = make_float4(y[0], y[1], y[2], y[3]);
+      else
+        store_gated<vdim>(a, y, t, hc, dv);
     }
   }
 }
@@ -1482,7 +1487,8 @@ int keep_streams(int T, int NA, int H, int G, int E, int vdim, bool shared, int 
   if (!shared || E != 576 || vdim != 512 || rep <= 16 || NA <= 0 || H > 65535) return 0;
   const int64_t wgs = (int64_t)NA * G * ((rep + 31) / 32);
   // pages that a row can see: of its table, of the window and of the kept first tokens
-  const int64_t most = window > 0 ? std::min<int64_t>(maxb, ((int64_t)window + WBS - 2) / WBS + 1 + ((int64_t)keep_first + WBS - 1) / WBS) : maxb;
+  const int64_t seen = ((int64_t)window + WBS - 2) / WBS + 1 + ((int64_t)keep_first + WBS - 1) / WBS;
+  const int64_t most = window > 0 ? std::min<int64_t>(maxb, seen) : maxb;
   const int S = (int)std::min(256 / std::max<int64_t>(wgs, 1), std::min<int64_t>((most + kStreams - 1) / kStreams, 16));
   return S >= 2 && most > 20 && T <= NA ? S : 0;
 }

@@ -9,8 +9,8 @@
 // MFMA operands, its value rows through the wave's own piece of LDS (read back transposed), the next
 // rows are in flight meanwhile, and no wave waits for another until the partial results (running
 // maximum, sum, weighted values) meet in LDS at the end.  Measured: 37 us (4.5 TB/s), 15 us and 54 us.  (Steps of the
-// 576-wide latent with more than 16 heads and no more rows than sequences do not come here while CUs are free: a
-// row's pages are split over workgroups as well, attn_keep_streams_kernel.)
+// 576-wide latent with more than 16 heads, no more rows than sequences and more than 20 pages to see do not come here
+// while CUs are free: a row's pages are split over workgroups as well, attn_keep_streams_kernel.)
 //
 // The 16 MFMA columns are (row, head) pairs of one key/value head, so the rows of a short extend and
 // the heads of a group share one pass.
@@ -458,10 +458,10 @@ static void launch_split_one(const KeepSplitArgs& a, int NA, int z, hipStream_t 
 // Eight waves to a workgroup where sequences and heads alone leave CUs idle: a wave's chain of pages is the
 // time then.  The wide latent's staged page leaves room for four, one workgroup to a CU; once there are more
 // workgroups than CUs the prompts' kernel takes its rows, which reads a page once for all heads, not for every
-// 16 of them (64 heads of 576: 128 sequences of 600 tokens 78 us split, 54 there; 64 of them 40 and 53, which
-// as steps of no more rows than sequences have gone to keep_streams' workgroups before).  Many workgroups of large groups in plain
-// sizes: two waves, or one, whose partial results need no merge (512 sequences of 100 tokens, 32 heads over 2 of
-// 128: 23 us with four waves, 20 with one; of 1,000: 100 and 99).
+// 16 of them (64 heads of 576: 128 sequences of 600 tokens 78 us split, 54 there; 64 of them 40 and 53; where rows may
+// see more than 20 pages, steps of no more rows than sequences have gone to keep_streams' workgroups before).  Many
+// workgroups of large groups in plain sizes: two waves, or one, whose partial results need no merge (512 sequences of
+// 100 tokens, 32 heads over 2 of 128: 23 us with four waves, 20 with one; of 1,000: 100 and 99).
 // Column tiles side by side: as many as the sequences have on the average, more where CUs would idle (one
 // sequence of 600 tokens with 33 rows, 64 heads: 1,130 us with four side by side, 38 with all).
 template <int DK, int DV, bool SHARED, bool EXACT>
