@@ -1387,6 +1387,7 @@ static void launch_keep_mfma_one(const KeepArgs& a) {
 template <int HPW, bool SHARED, int MODE>
 static bool small_groups(const KeepArgs& a) {
   const int64_t wgs = (int64_t)a.W * (a.H / HPW);
+  if (a.W > (1 << 22)) return false;               // a grid's threads in 32 bits; the other kernel's launches are cut
   if constexpr (HPW == 1) return SHARED && MODE >= 2 && a.maxb <= 3;
   if constexpr (HPW == 2) return a.maxb <= 3 || (MODE >= 2 && wgs < 1024);
   return wgs <= 256 && ((MODE >= 2 && a.maxb <= 4) || (wgs > 192 && a.maxb <= (MODE >= 2 ? 8 : 2)));
