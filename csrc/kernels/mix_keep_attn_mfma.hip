@@ -3,6 +3,7 @@
 // tokens; softmax, softmax with a sink, or unnormalised sigmoid weights; optional output gate
 // (a column per head, or gate_w = vdim: one per output, rows 8-byte aligned);
 // the values may be the leading entries of the key rows themselves (latent attention).
+// Prompt rows of 576-wide latents with groups of four heads: mix_keep_latent.hip.
 // Decode rows have kernels of their own: mix_keep_split.hip, and here those of wide latents in streams over several
 // workgroups (attn_keep_streams_kernel) and many heads at a time (attn_keep_wide_kernel, DEC).
 //
@@ -38,69 +39,12 @@
 // operands four products ahead changed nothing.
 #include <algorithm>
 #include <type_traits>
-#include <utility>
 
 #include "common.h"
 #include "mix_common.h"
+#include "mix_keep_mfma.h"
 
 namespace rfqmix {
-
-using rfq::as_bf16x8;
-using rfq::f32x16;
-using rfq::u32x4;
-using rfq::f32x4;
-using rfq::s16x4;
-using rfq::s16x8;
-
-namespace {
-constexpr int WQB = 32;                 // queries per work item
-constexpr int WBS = 32;                 // keys per tile = page size
-constexpr float kNegInfW = -__builtin_huge_valf();
-constexpr float kLog2e = 1.44269504088896f;
-constexpr float kDeferW = 11.f;         // base 2
-
-__device__ __forceinline__ void split_bf16w(const float* f, s16x8& hi, s16x8& lo) {
-  float r[8];
-  hi = rfq::pack8(f);
-#pragma unroll
-  for (int i = 0; i < 8; ++i) r[i] = f[i] - rfq::bf2f_s(hi[i]);
-  lo = rfq::pack8(r);
-}
-
-// the value of the lane 32 away beside one's own
-__device__ __forceinline__ float other_half_max(float x) {
-  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-  return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
-}
-__device__ __forceinline__ float both_halves_sum(float x) {
-  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
-}
-
-}  // namespace
-
-struct KeepArgs {
-  const float* q;
-  const void *k_cache, *v_cache;
-  int64_t vrs;
-  const int32_t* bt;
-  int maxb;
-  const int32_t *q_start, *q_len, *kv_len, *work_seq, *work_qblk;
-  int W;
-  const float* head_bias;
-  const void* gate;
-  int64_t gate_stride;
-  int gate_w;
-  void* out;
-  int64_t out_stride;
-  float scale;
-  int window, keep_first;
-  bool sigmoid;
-  int H, G;
-  float softcap, out_mult;
-  hipStream_t s;
-  bool turned = false;                             // attn_keep_tile_kernel: a block's heads begin where the block says
-};
 
 // the same over lanes 16 away
 __device__ __forceinline__ float other_row_max(float x) {
@@ -361,41 +305,6 @@ __global__ __launch_bounds__(128 * HPW, HPW == 2 ? 3 : 1) void attn_keep_mfma_ke
   store_rows<DV, MODE>(a, o, lrun, t, hh, grp, qlive);
 }
 
-// lane (col, half) of a 32 x 32 tile holds value channels 32 m + 8 b + 4 half .. + 3 of its query: 8-byte stores
-template <int VM, int MODE>
-__device__ __forceinline__ void store_rows32(const KeepArgs& a, const f32x16 (&o)[VM], float lrun, int64_t t, int hh,
-                                             int half, bool qlive) {
-  constexpr int vdim = 32 * VM;
-  const float l = both_halves_sum(lrun);
-  if (!qlive) return;
-  const bf16_t* gate = static_cast<const bf16_t*>(a.gate);
-  float mul = MODE >= 2 ? a.out_mult : (l > 0.f ? a.out_mult / l : 0.f);
-  if (gate != nullptr && a.gate_w == 1) mul /= 1.0f + __expf(-ldf(gate + t * a.gate_stride + hh));
-  // a gate column per output: four neighbouring logits, 8-byte reads
-  const bf16_t* grow = gate != nullptr && a.gate_w > 1 ? gate + t * a.gate_stride + (int64_t)hh * vdim + half * 4 : nullptr;
-  bf16_t* orow = static_cast<bf16_t*>(a.out) + t * a.out_stride + (int64_t)hh * vdim + half * 4;
-#pragma unroll
-  for (int m = 0; m < VM; ++m)
-#pragma unroll
-    for (int b = 0; b < 4; ++b) {
-      float y[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) y[i] = o[m][4 * b + i] * mul;
-      if (grow != nullptr) {
-        const uint2 gu = *reinterpret_cast<const uint2*>(grow + m * 32 + b * 8);
-        y[0] /= 1.0f + __expf(-__uint_as_float(gu.x << 16));
-        y[1] /= 1.0f + __expf(-__uint_as_float(gu.x & 0xffff0000u));
-        y[2] /= 1.0f + __expf(-__uint_as_float(gu.y << 16));
-        y[3] /= 1.0f + __expf(-__uint_as_float(gu.y & 0xffff0000u));
-      }
-      *reinterpret_cast<uint2*>(orow + m * 32 + b * 8) = make_uint2(rfq::pack_bf16x2(y[0], y[1]), rfq::pack_bf16x2(y[2], y[3]));
-    }
-}
-
-__device__ __forceinline__ uint32_t lds_byte(const unsigned char* smem) {      // where the dynamic LDS begins
-  return (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const unsigned char*)smem;
-}
-
 // A row's 16-byte pieces are permuted inside it, and rows of 256 bytes lie 16 bytes apart after every four, so
 // that the pieces that one LDS access takes together (K: a piece of 16 neighbouring rows; V, transposed: 64
 // bytes of four neighbouring rows) lie on different banks.
@@ -407,11 +316,6 @@ __device__ __forceinline__ int page_swizzle(int r) {
 }
 template <int E>
 constexpr int page_row(int r) { return r * E + (E == 128 ? (r >> 2) * 8 : 0); }     // shorts before row r
-// f(0), f(1) .. f(N - 1) with constants: loops whose bodies have loops over parts of their index are unrolled for sure
-template <int... I, typename F>
-__device__ __forceinline__ void each_of(std::integer_sequence<int, I...>, F f) { (f(std::integral_constant<int, I>{}), ...); }
-template <int N, typename F>
-__device__ __forceinline__ void each(F f) { each_of(std::make_integer_sequence<int, N>{}, f); }
 template <int DK, int DV, bool SHARED>
 constexpr int tile_lds_shorts() { return SHARED ? 3 * page_row<32 * DK>(WBS) : 2 * (page_row<32 * DK>(WBS) + page_row<16 * DV>(WBS)); }
 
@@ -733,30 +637,20 @@ __global__ __launch_bounds__(64 * HPW, 2) void attn_keep_tile_kernel(const KeepA
   }
   last();
   turn(i, std::false_type{});
-  store_rows32<VM, MODE>(a, o, lrun, t, hh, half, qlive);
+  store_tiles32<VM>(a, o, row_factor<MODE>(a, both_halves_sum(lrun), t, hh), t, hh, vdim, 0, half, qlive);
 }
 
-// Wide latents: keys of 320 or 576 entries whose first 256 or 512 are the values.  32 queries' results
-// (256 registers at 512 values) and the queries themselves (144) leave no room for the rest, so a wave
-// has 16 queries on 16x16x32 tiles, two waves a head, and the page's LDS reads are what bounds it (K
-// rows 36 x 1 KB, V 64 x 512 B a wave and page: 4,350 clocks for eight waves against 3,200 of MFMA).
-// One prompt of 2,048 over 576 (32 heads) took 904 us a pass on tiles with padded pages, 420 here; the attention of
-// four of them 1,262 us with a head's blocks one after the other, 968 with a block's heads side by side (the last
-// heads' long blocks started at seven eighths of the time), 948 without conflicts in the key reads.  Alone a workgroup
-// takes 2.7 us a page.  One wave a SIMD with 32 queries, half the LDS reads, took 3.2 us: it cannot issue what two
-// can.  Pages come by LDS-DMA, the next one during this one; their rows lie unpadded, 16-byte pieces permuted inside
-// each 128 bytes by wide_swizzle(row).
+// Wide latents: keys of 320 entries whose first 256 are the values; of 576 and 512 in groups of two heads or of one
+// (groups of four and odd ones: mix_keep_latent.hip).  32 queries' results (256 registers at 512 values) and the queries
+// themselves (144) leave no room for the rest, so a wave has 16 queries on 16x16x32 tiles, two waves a head: a page's
+// LDS reads are K rows 36 x 1 KB, V 64 x 512 B a wave at 576.  A block's heads lie side by side: one after the other the
+// last heads' long blocks started at seven eighths of the time.  Pages come by LDS-DMA, the next one during this one;
+// their rows lie unpadded, 16-byte pieces permuted inside each 128 bytes by wide_swizzle(row).  576 entries in groups
+// of two, 16 heads over 8, two prompts of 2,048: 237 us; a workgroup of four heads, half of them idle, took 358.
 // DEC: decode rows.  A wave's columns are 16 heads of one row, so that a workgroup reads a page once for up to
 // 128 heads; the pages come one after another, which pays once every CU has a workgroup (launch_split_waves).
 // 256 sequences of 300 tokens with 64 heads of 576 entries 44 us, 32 of 500 with four rows each 50; split over
 // waves 116 and 129.
-// Pieces that one LDS access takes together then lie on different banks: of a K read rows 0..3 and 12..15 of one
-// piece with rows 4..11 of its neighbour, or the other way round (sixteen rows of one piece are not what it takes: a
-// permutation that parts those alone cost 1,150 clocks a page of eight waves), of a transposed V read four
-// neighbouring rows of a pair of pieces beside the next four.  The row's parity picks a half of the banks, bit 1 the
-// half of that, the row's quad the order inside it.
-__device__ __forceinline__ int wide_swizzle(int r) { return ((r >> 1) & 1) << 2 | ((4 - (r >> 2)) & 3); }
-
 template <int DK, int DV, int HPW, int MODE, bool DEC>
 __global__ __launch_bounds__(128 * HPW, DEC && HPW == 1 ? 1 : 2) void attn_keep_wide_kernel(const KeepArgs a) {
   constexpr int E = 32 * DK, vdim = 16 * DV, NWV = 2 * HPW, NP = WBS * E / 512, ND = (NP + NWV - 1) / NWV;
@@ -1370,7 +1264,8 @@ static void launch_keep_mfma_one(const KeepArgs& a) {
       hipLaunchKernelGGL(kernel, dim3((unsigned)std::min(most, a.W - w) * groups), dim3(threads), lds, a.s, part);
     }
   };
-  if constexpr (WIDE) run(&attn_keep_wide_kernel<DK, DV, HPW, MODE, false>, 128 * HPW);
+  if constexpr (DK == 18 && HPW == 4) return launch_attn_keep_latent(a);
+  else if constexpr (WIDE) run(&attn_keep_wide_kernel<DK, DV, HPW, MODE, false>, 128 * HPW);
   else run(&attn_keep_tile_kernel<DK, DV, HPW, SHARED, MODE>, 64 * HPW);
 }
 

@@ -254,6 +254,17 @@ def test_short_rows_of_four_heads(H, G, E, vd, shared):
             _check(H, G, E, vd, shared, seqs=[(n, n)] + [(32, 5)] * left, prompt=True, window=90, keep_first=40, **opt)
 
 
+@pytest.mark.parametrize("H,G", [(4, 1), (16, 2), (5, 1)])
+def test_latent_prompt_rows(H, G):
+    """Waves of scores and waves of values: one page and up to six, blocks of one row, eight rows and nine, whole ones,
+    gates of either kind, all weights, the maximum moving at every page."""
+    seqs = [(1, 1), (8, 8), (9, 9), (32, 32), (33, 33), (70, 8), (97, 41), (160, 9), (161, 40), (40, 0)]
+    _check(H, G, 576, 512, True, seqs=seqs, prompt=True, rising=0.3, bias=True, gate="head")
+    _check(H, G, 576, 512, True, seqs=seqs, prompt=True, rising=0.3, softcap=20.0, out_mult=0.6, gate="output")
+    _check(H, G, 576, 512, True, seqs=seqs, prompt=True, window=37, keep_first=5, sigmoid=True, bias=True)
+    _check(H, G, 576, 512, True, seqs=seqs, prompt=True, window=64, keep_first=40, sigmoid=True, softcap=15.0, bias=True)
+
+
 def test_prompt_rows_with_rising_scores():
     """Every page moves the maximum by far: the accumulators are rescaled each time."""
     for shared, E, vd in ((False, 128, 128), (True, 576, 512)):
