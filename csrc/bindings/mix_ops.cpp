@@ -10,6 +10,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <functional>
+
 #include "../kernels/mix_linrec.h"
 #include "../kernels/mix_mlstm.h"
 
@@ -63,7 +65,7 @@ void launch_wkv_recurrence(bool, const void*, const void*, const void*, const vo
                            int64_t, int64_t, int64_t, int64_t, int64_t, const float*, const float*,
                            const float*, float, float*, const int32_t*, const int32_t*,
                            const int32_t*, const int32_t*, const int32_t*, int, void*, int, int, int,
-                           int, hipStream_t);
+                           int, const std::function<float*(int64_t)>&, hipStream_t);
 void launch_moe_route_grouped(const float*, const float*, int, int, int, int, int, int32_t*, float*,
                               hipStream_t);
 void launch_moe_pair_up(bool, const void*, int64_t, const int32_t*, const void*, void*, int, int,
@@ -473,6 +475,15 @@ Tensor matmul_short_meta(const Tensor& x, const Tensor& w, bool out_f32) {
   return at::empty({x.size(0), w.size(0)}, x.options().dtype(out_f32 ? at::kFloat : x.scalar_type()));
 }
 
+// Scratch memory for a launcher, on the tensor's device from the caching allocator: `held` keeps it until the launches
+// are queued.
+std::function<float*(int64_t)> scratch_floats(const Tensor& like, Tensor& held) {
+  return [&](int64_t n) {
+    held = at::empty({n}, like.options().dtype(at::kFloat));
+    return held.data_ptr<float>();
+  };
+}
+
 void wkv_recurrence(const Tensor& r, const Tensor& k, const Tensor& v, const Tensor& zw,
                     const Tensor& w0, const Tensor& u, const Tensor& gate, const Tensor& norm_w,
                     double eps, const Tensor& state, const Tensor& row_state,
@@ -490,6 +501,7 @@ void wkv_recurrence(const Tensor& r, const Tensor& k, const Tensor& v, const Ten
   TORCH_CHECK(state.dim() == 4 && state.size(0) % 2 == 0 && state.size(1) == H &&
               state.size(2) == N && state.size(3) == N, "wkv_recurrence: state [2 slots, H, N, N]");
   TORCH_CHECK(rfqmix::wkv_ok(N) && H <= 65535, "wkv_recurrence: head size outside the kernel's range");
+  Tensor part;
   rfqmix::launch_wkv_recurrence(
       f32, r.data_ptr(), k.data_ptr(), v.data_ptr(), zw.data_ptr(), gate.data_ptr(), r.stride(0),
       k.stride(0), v.stride(0), zw.stride(0), gate.stride(0), f32p(w0, "w0", HN), f32p(u, "u", HN),
@@ -497,7 +509,7 @@ void wkv_recurrence(const Tensor& r, const Tensor& k, const Tensor& v, const Ten
       i32p(row_state, "row_state", T), i32p(row_back, "row_back", T), i32p(row_fwd, "row_fwd", T),
       i32p(pos, "positions", T), run_rows.has_value() ? i32p(*run_rows, "run_rows", 0) : nullptr,
       run_rows.has_value() ? (int)run_rows->numel() : 0, out.data_ptr(), T, H, N,
-      (int)state.size(0) / 2, stream());
+      (int)state.size(0) / 2, scratch_floats(out, part), stream());
 }
 
 // Latent attention on MFMA tiles: q [T, H, R] bf16 (the queries carried into the latent space;
@@ -977,7 +989,8 @@ void gated_linear_recurrence(const Tensor& q, const Tensor& k, const Tensor& v, 
   a.runs = run_rows.has_value() ? (int)run_rows->numel() : 0;
   a.out = out.data_ptr(); a.os = out.stride(0);
   a.T = T; a.H = H; a.rep = H / Hq; a.dim = dim; a.vdim = vdim; a.slots = (int)state.size(0) / 2;
-  rfqmix::launch_gated_linrec(in_f32, a_f32, beta.has_value(), a, stream());
+  Tensor part;
+  rfqmix::launch_gated_linrec(in_f32, a_f32, beta.has_value(), a, scratch_floats(out, part), stream());
 }
 
 void moe_route_topk(const Tensor& z, const OptT& bias, int64_t top, const Tensor& ids,

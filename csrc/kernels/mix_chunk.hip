@@ -26,6 +26,12 @@
 // registers, an fp32 operand is never narrowed.  Measured, two runs of 2,048 tokens in bf16: wkv with
 // 64 heads of 64 x 64 5,353 -> 203 us; delta rule with 32 heads of 64 x 128 741 (decays and scan) ->
 // 301 us; gla in fp32, five ragged runs of up to 1,031, 32 heads, 447 -> 121 us.
+//
+// Without the delta rule a run's chain is cut where workgroups leave CUs idle (chunk_seg_rows): chunk_segment_kernel
+// makes what every segment's rows leave of a state of zeros and the products of its decays, all segments at once, and a
+// segment's workgroup begins from the state of before the run carried through those in front of it.  wkv, two runs of
+// 2,048 with 64 heads: 204 -> 26 + 118 us.  What bounds the first kernel: exponentials (22 instructions a decay, 38 of gla)
+// and the way to its first rows and out, 10 us of a workgroup.
 #include <algorithm>
 #include <type_traits>
 
@@ -126,13 +132,46 @@ __device__ __forceinline__ void lower_product(const float* m, const f32x4& x, in
 }
 }  // namespace
 
-// 64 value channels, from z64 on, of head h of the run that begins at row t0.
+// A run's segment `seg` (the slot-th of the step): rows [t0, t0 + n) of the run from row run0 on.
+struct ChunkSegment {
+  int run0, t0, n, seg, slot;
+  bool last;
+};
+__device__ __forceinline__ ChunkSegment whole_run(const ChunkArgs& a, int t0) {
+  return {t0, t0, a.row_fwd[t0] + 1, 0, 0, true};
+}
+// The slot-th segment of the step's runs in their order, every wave for itself; n = 0: there are fewer.
+__device__ __forceinline__ ChunkSegment find_segment(const ChunkArgs& a, int slot, int lane) {
+  int left = slot;
+  for (int base = 0; base < a.runs; base += 64) {
+    const int r = base + lane < a.runs ? a.run_rows[base + lane] : -1;
+    const int n = r >= 0 && a.row_back[r] == 0 ? a.row_fwd[r] + 1 : 0;
+    const int mine = (n + a.seg_rows - 1) / a.seg_rows;
+    int upto = mine;                                       // segments of the runs up to this lane's
+#pragma unroll
+    for (int o = 1; o < 64; o *= 2) {
+      const int x = __shfl_up(upto, o, 64);
+      if (lane >= o) upto += x;
+    }
+    const uint64_t m = __builtin_amdgcn_ballot_w64(left < upto);
+    if (m != 0) {
+      const int at = __builtin_ctzll(m);
+      const int seg = left - __builtin_amdgcn_readlane(upto - mine, at), rows = __builtin_amdgcn_readlane(n, at);
+      const int run0 = __builtin_amdgcn_readlane(r, at), from = seg * a.seg_rows;
+      return {run0, run0 + from, min(rows - from, a.seg_rows), seg, slot, from + a.seg_rows >= rows};
+    }
+    left -= __builtin_amdgcn_readlane(upto, 63);
+  }
+  return {0, 0, 0, 0, 0, false};
+}
+
+// 64 value channels, from z64 on, of head h of a run or of a segment of one.
 template <typename TI, typename TG, int MODE>
-__device__ __forceinline__ void chunk_run(const ChunkArgs& a, const int t0, const int h, const int z64, const int tid) {
+__device__ __forceinline__ void chunk_run(const ChunkArgs& a, const ChunkSegment& sg, const int h, const int z64, const int tid) {
   constexpr bool WKV = MODE == kChunkWkv, DELTA = MODE == kChunkDelta;
   const int lane = tid & 63, col = lane & 15, grp = lane >> 4;
-  const int n = a.row_fwd[t0] + 1, nc = (n + CT - 1) / CT;
-  const int code = a.row_state[t0];
+  const int t0 = sg.t0, n = sg.n, nc = (n + CT - 1) / CT;
+  const int code = a.row_state[sg.run0];
   const int H = a.H, dim = a.dim, vdim = a.vdim;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int role = wave >> 2, w = wave & 3;               // 0 consumers, 1 decays, 2 A and T, 3 wkv's norm and gate
@@ -155,7 +194,7 @@ __device__ __forceinline__ void chunk_run(const ChunkArgs& a, const int t0, cons
   // ---- consumers: 16 value channels, S[16 i + 4 grp + r][column]
   const int vcol = z64 + 16 * w + col;
   const bool vlive = vcol < vdim;
-  const bool from_state = code >= 0 && a.pos[t0] > 0;
+  const bool from_state = code >= 0 && a.pos[sg.run0] > 0;
   const int64_t hsz = (int64_t)dim * vdim;
   f32x4 st[4];
   TI vreg[4];
@@ -212,6 +251,20 @@ __device__ __forceinline__ void chunk_run(const ChunkArgs& a, const int t0, cons
         st[i][r] = (from_state && vlive && c < dim) ? rd[(int64_t)c * vdim + vcol] : 0.f;
       }
     fetch_v(0);
+    if constexpr (!DELTA) {
+      const int64_t slots = a.runs + a.T / max(a.seg_rows, 1);
+      for (int j = sg.slot - sg.seg; j < sg.slot; ++j) {     // the run's segments before this one
+        const float* left = a.seg + ((int64_t)j * H + h) * hsz + vcol;
+        const float* kept = a.seg + slots * H * hsz + ((int64_t)j * H + h) * dim;
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const int c = 16 * i + 4 * grp + r;
+            st[i][r] = fmaf(kept[c], st[i][r], left[(int64_t)c * vdim]);
+          }
+      }
+    }
   } else if (role == 1) {
     offsets(qo, a.qs, 4 * grp, sizeof(TI), 0);
     offsets(ko, a.ks, 4 * grp, sizeof(TI), 0);
@@ -573,7 +626,7 @@ do {                                                                            
     }
   }
 
-  if (role == 0 && code >= 0 && vlive) {
+  if (role == 0 && code >= 0 && vlive && sg.last) {
     float* wr = a.state + (((int64_t)(1 - (code & 1)) * a.slots + (code >> 1)) * H + h) * hsz;
 #pragma unroll
     for (int i = 0; i < 4; ++i)
@@ -589,7 +642,193 @@ do {                                                                            
 template <typename TI, typename TG, int MODE>
 __global__ __launch_bounds__(chunk_threads(MODE)) void chunk_recurrence_kernel(const ChunkArgs a) {
   const int t0 = a.run_rows[blockIdx.x];
-  if (t0 >= 0 && a.row_back[t0] == 0) chunk_run<TI, TG, MODE>(a, t0, blockIdx.y, blockIdx.z * 64, threadIdx.x);
+  if (t0 >= 0 && a.row_back[t0] == 0) chunk_run<TI, TG, MODE>(a, whole_run(a, t0), blockIdx.y, blockIdx.z * 64, threadIdx.x);
+}
+
+// Two and four neighbouring entries in flight, and their values where they are needed (see `arrived`).
+__device__ __forceinline__ void raw4(const float* base, uint32_t bytes, uint4& x) { x = load_at(reinterpret_cast<const uint4*>(base), bytes); }
+__device__ __forceinline__ void raw4(const bf16_t* base, uint32_t bytes, uint2& x) { x = load_at(reinterpret_cast<const uint2*>(base), bytes); }
+__device__ __forceinline__ void raw2(const float* base, uint32_t bytes, uint2& x) { x = load_at(reinterpret_cast<const uint2*>(base), bytes); }
+__device__ __forceinline__ void raw2(const bf16_t* base, uint32_t bytes, uint32_t& x) { x = load_at(reinterpret_cast<const uint32_t*>(base), bytes); }
+__device__ __forceinline__ void arrived2(uint2 x, float* f) {
+  asm volatile("" : "+v"(x.x), "+v"(x.y));
+  f[0] = __uint_as_float(x.x);
+  f[1] = __uint_as_float(x.y);
+}
+__device__ __forceinline__ void arrived2(uint32_t x, float* f) {
+  asm volatile("" : "+v"(x));
+  f[0] = __uint_as_float(x << 16);
+  f[1] = __uint_as_float(x & 0xffff0000u);
+}
+__device__ __forceinline__ void arrived4(uint4 x, float* f) {
+  asm volatile("" : "+v"(x.x), "+v"(x.y), "+v"(x.z), "+v"(x.w));
+  f[0] = __uint_as_float(x.x);
+  f[1] = __uint_as_float(x.y);
+  f[2] = __uint_as_float(x.z);
+  f[3] = __uint_as_float(x.w);
+}
+__device__ __forceinline__ void arrived4(uint2 x, float* f) {
+  asm volatile("" : "+v"(x.x), "+v"(x.y));
+  f[0] = __uint_as_float(x.x << 16);
+  f[1] = __uint_as_float(x.x & 0xffff0000u);
+  f[2] = __uint_as_float(x.y << 16);
+  f[3] = __uint_as_float(x.y & 0xffff0000u);
+}
+
+// What a segment's rows leave of a state of zeros, and the products of its decays: for every segment but a run's last,
+// one workgroup per segment, head, 32 key and 64 value channels.  A wave has an eighth (a sixteenth) of the rows and goes through them
+// from the last chunk to the first, the keys times all decays behind them: nothing is rescaled, and the lane that makes
+// such a product (four tokens of two key channels) has it as the MFMA operand.  No LDS but to add the waves' parts up.
+constexpr int kSegKeys = 32;
+template <typename TI, int MODE, int kSegWaves>
+__global__ __launch_bounds__(64 * kSegWaves, 4) void chunk_segment_kernel(const ChunkArgs a) {
+  constexpr bool WKV = MODE == kChunkWkv;
+  typedef typename std::conditional<WKV, TI, float>::type TZ;
+  typedef typename std::conditional<sizeof(TI) == 2, uint2, uint4>::type RV;
+  typedef typename std::conditional<sizeof(TI) == 2, uint32_t, uint2>::type RK;
+  typedef typename std::conditional<sizeof(TZ) == 2, uint32_t, uint2>::type RZ;
+  const int tid = threadIdx.x, lane = tid & 63, col = lane & 15, grp = lane >> 4;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const ChunkSegment sg = find_segment(a, blockIdx.z, lane);
+  if (sg.n == 0 || sg.last) return;
+  __shared__ __attribute__((aligned(16))) float sums[kSegWaves / 2][kSegKeys * NC];
+  const int h = blockIdx.x, z64 = (blockIdx.y >> 1) * 64, c0 = (blockIdx.y & 1) * kSegKeys, H = a.H, vdim = a.vdim, hq = h / a.rep;
+  const int rows = a.seg_rows / kSegWaves;
+  // the wave's last chunk; a lane's tokens by their offsets in bytes
+  const int64_t at = sg.t0 + (w + 1) * rows - CT;
+  const TI* kb = static_cast<const TI*>(a.k) + at * a.ks + (int64_t)hq * NC + c0;
+  const TI* vb = static_cast<const TI*>(a.v) + at * a.vs + (int64_t)h * vdim + z64;
+  const TZ* zb = static_cast<const TZ*>(a.z) + at * a.zs + (int64_t)h * NC + c0;
+  uint32_t ko[4], vo[4], zo[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    ko[i] = (uint32_t)((4 * grp + i) * a.ks + 2 * col) * (uint32_t)sizeof(TI);
+    vo[i] = (uint32_t)((4 * grp + i) * a.vs + 4 * col) * (uint32_t)sizeof(TI);
+    zo[i] = (uint32_t)((4 * grp + i) * a.zs + 2 * col) * (uint32_t)sizeof(TZ);
+  }
+  RK kr[4];
+  RV vr[4];
+  RZ zr[4];
+  auto fetch = [&]() {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      raw2(zb, zo[i], zr[i]);
+      raw2(kb, ko[i], kr[i]);
+      raw4(vb, vo[i], vr[i]);
+    }
+    kb -= CT * a.ks;
+    vb -= CT * a.vs;
+    zb -= CT * a.zs;
+  };
+  fetch();
+  const float bias[2] = {a.zbias[h * NC + c0 + 2 * col], a.zbias[h * NC + c0 + 2 * col + 1]};
+  const float rate = WKV ? 0.f : a.rate[h];
+  f32x4 st[2][4];                                            // [key channel % 2][value channel % 4]
+#pragma unroll
+  for (int x = 0; x < 2; ++x)
+#pragma unroll
+    for (int y = 0; y < 4; ++y) st[x][y] = (f32x4){0.f, 0.f, 0.f, 0.f};
+  float behind[2] = {1.f, 1.f};                              // products of the decays behind the chunk
+  for (int c = rows / CT; c > 0; --c) {
+    float k[4][2], d[4][2], v[4][4];                         // [token][channel % 2 or 4]
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      arrived2(zr[i], d[i]);
+      arrived2(kr[i], k[i]);
+      arrived4(vr[i], v[i]);
+    }
+    if (c > 1) fetch();
+#pragma unroll
+    for (int x = 0; x < 2; ++x) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float z = d[i][x] + bias[x];
+        d[i][x] = WKV ? exp_c(-exp_c(z > 80.f ? 80.f : z)) : exp_c(-rate * softplus_c(a.zsign * z));
+      }
+      const float a2 = d[3][x], a1 = d[2][x] * a2, a0 = d[1][x] * a1, up = d[0][x] * a0;
+      const float b1 = __shfl_xor(up, 16, 64), b2 = __shfl_xor(up, 32, 64), b3 = __shfl_xor(b1, 32, 64);
+      const float b23 = b2 * b3;
+      const float post = ((grp & 1) ? 1.f : b1) * ((grp & 2) ? 1.f : b23) * behind[x];
+      behind[x] *= (up * b1) * b23;
+      k[0][x] *= a0 * post;
+      k[1][x] *= a1 * post;
+      k[2][x] *= a2 * post;
+      k[3][x] *= post;
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int y = 0; y < 4; ++y) st[x][y] = __builtin_amdgcn_mfma_f32_16x16x4f32(k[i][x], v[i][y], st[x][y], 0, 0, 0);
+    }
+  }
+  // a wave's part times the decays of those behind it
+  float* decays = &sums[0][0];
+  if (grp == 0) *reinterpret_cast<float2*>(decays + w * kSegKeys + 2 * col) = make_float2(behind[0], behind[1]);
+  __syncthreads();
+  if (blockIdx.y < 2 && tid < kSegKeys) {
+    float f = decays[tid];
+#pragma unroll
+    for (int u = 1; u < kSegWaves; ++u) f *= decays[u * kSegKeys + tid];
+    a.seg[(a.runs + a.T / a.seg_rows) * (int64_t)(H * NC) * vdim + ((int64_t)sg.slot * H + h) * NC + c0 + tid] = f;
+  }
+  float4 f[2];                                               // of channels 8 grp ..
+  f[0] = f[1] = make_float4(1.f, 1.f, 1.f, 1.f);
+  for (int u = w + 1; u < kSegWaves; ++u)
+#pragma unroll
+    for (int r = 0; r < 2; ++r) f[r] = mul4(f[r], ld4(decays + u * kSegKeys + 8 * grp + 4 * r));
+#pragma unroll
+  for (int r = 0; r < 2; ++r)
+#pragma unroll
+    for (int y = 0; y < 4; ++y) {
+      st[0][y][2 * r] *= f[r].x;
+      st[1][y][2 * r] *= f[r].y;
+      st[0][y][2 * r + 1] *= f[r].z;
+      st[1][y][2 * r + 1] *= f[r].w;
+    }
+  constexpr int half = kSegWaves / 2;
+  auto place = [&](int x, int r) { return &sums[w & (half - 1)][(2 * (4 * grp + r) + x) * NC + 4 * col]; };
+#pragma unroll
+  for (int part = 0; part < 2; ++part) {                     // the later half's parts to the earlier half's, those out
+    __syncthreads();
+    if ((w >= half) == (part == 0)) {
+#pragma unroll
+      for (int x = 0; x < 2; ++x)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) st4(place(x, r), make_float4(st[x][0][r], st[x][1][r], st[x][2][r], st[x][3][r]));
+    }
+    __syncthreads();
+    if (part == 0 && w < half) {
+#pragma unroll
+      for (int x = 0; x < 2; ++x)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const float4 o = ld4(place(x, r));
+          st[x][0][r] += o.x;
+          st[x][1][r] += o.y;
+          st[x][2][r] += o.z;
+          st[x][3][r] += o.w;
+        }
+    }
+  }
+  float* out = a.seg + (((int64_t)sg.slot * H + h) * NC + c0) * vdim + z64;
+#pragma unroll
+  for (int i = 0; i < kSegKeys * NC / (128 * kSegWaves); ++i) {
+    const int e = (i * 64 * kSegWaves + tid) * 2;
+    float2 y = make_float2(0.f, 0.f);
+#pragma unroll
+    for (int u = 0; u < half; u += 2) {
+      const float2 p = *reinterpret_cast<const float2*>(&sums[u][e]), q = *reinterpret_cast<const float2*>(&sums[u + 1][e]);
+      y.x += p.x + q.x;
+      y.y += p.y + q.y;
+    }
+    *reinterpret_cast<float2*>(out + (int64_t)(e / NC) * vdim + e % NC) = y;
+  }
+}
+
+// A workgroup per segment, head and 64 value channels, behind chunk_segment_kernel.
+template <typename TI, typename TG, int MODE>
+__global__ __launch_bounds__(chunk_threads(MODE)) void chunk_recurrence_segments_kernel(const ChunkArgs a) {
+  const ChunkSegment sg = find_segment(a, blockIdx.z, threadIdx.x & 63);
+  if (sg.n > 0) chunk_run<TI, TG, MODE>(a, sg, blockIdx.x, blockIdx.y * 64, threadIdx.x);
 }
 
 // Workgroups, one to a CU at most, that share the runs of min_run rows or more, which every wave counts for
@@ -622,7 +861,7 @@ __global__ __launch_bounds__(chunk_threads(MODE)) void chunk_recurrence_share_ke
     const_args* p = (const_args*)__builtin_amdgcn_kernarg_segment_ptr();
     int tid = threadIdx.x;
     asm volatile("" : "+v"(tid), "+s"(p));
-    chunk_run<TI, TG, MODE>(*(const ChunkArgs*)p, t0, part - z * a.H, z * 64, tid);
+    chunk_run<TI, TG, MODE>(*(const ChunkArgs*)p, whole_run(*(const ChunkArgs*)p, t0), part - z * a.H, z * 64, tid);
   }
 }
 
@@ -650,6 +889,43 @@ int chunk_min_run(int mode, int T, const ChunkArgs& a) {
   return T - a.runs + 1 >= from ? from : kNever;          // no run can be longer than that
 }
 
+// Segments instead of whole runs where they leave fewer or shorter rounds of one workgroup a CU, by the times of
+// the kernels below (us): a workgroup's start and end and its chunks, as many rounds as workgroups ask for; the same of
+// chunk_segment_kernel, whose workgroups of eight waves stand two to a CU.  Runs are taken as equally long, the
+// case that gains least.  Two runs of 2,048 tokens in bf16, whole -> in segments: wkv, 64 heads 204 -> 145 us, 32
+// heads 194 -> 89; gla, 16 heads of 128 218 -> 112; one run of 2,048, 64 heads, 190 -> 81.  The delta rule's decays are
+// matrices: its runs stay whole.
+int chunk_seg_rows(int mode, bool in_f32, int T, const ChunkArgs& a) {
+  if (mode == kChunkDelta || chunk_min_run(mode, T, a) != 1 || a.dim != NC || a.vdim % 64 != 0) return 0;
+  const uintptr_t wide = in_f32 ? 16 : 8, zwide = mode == kChunkWkv && !in_f32 ? 4 : 8;     // loads of four, of two
+  for (const void* p : {a.k, a.v})
+    if (reinterpret_cast<uintptr_t>(p) % wide != 0) return 0;
+  if (reinterpret_cast<uintptr_t>(a.z) % zwide != 0) return 0;
+  for (int64_t st : {a.ks, a.vs, a.zs})
+    if (st % 4 != 0) return 0;
+  const int64_t per = (int64_t)a.H * (a.vdim / 64);
+  const int c = (T + CT * a.runs - 1) / (CT * a.runs);    // chunks of a run
+  const double turn = mode == kChunkWkv ? 1.65 : 1.85;
+  auto rounds = [](int64_t wgs, int at_once) { return (double)((wgs + at_once - 1) / at_once); };
+  double best = 0.9 * rounds(a.runs * per, 256) * (6 + turn * c) - 5;
+  int rows = 0;
+  for (int s = 2; s <= 16; ++s) {
+    int cs = ((c + s - 1) / s + 7) / 8 * 8;               // chunks of a segment
+    if (cs >= 64) cs = (cs + 15) / 16 * 16;
+    const int64_t n = (c + cs - 1) / cs, w1 = a.runs * (n - 1) * per * (NC / kSegKeys);
+    const double t = 6 + (cs >= 64 ? rounds(w1, 256) * (8 + 3.3 * cs / 16) : rounds(w1, 512) * (6 + 2.0 * cs / 8)) +
+                     rounds(a.runs * n * per, 256) * (6 + turn * cs);
+    if (n > 1 && t < best) {
+      best = t;
+      rows = cs * CT;
+    }
+  }
+  return rows;
+}
+int64_t chunk_seg_floats(int T, const ChunkArgs& a) {
+  return (a.runs + (int64_t)T / a.seg_rows) * a.H * a.dim * (a.vdim + 1);
+}
+
 template <typename TI, typename TG, int MODE>
 static void launch_chunk_one(int T, const ChunkArgs& a, hipStream_t s) {
   static bool attr = false;
@@ -660,6 +936,22 @@ static void launch_chunk_one(int T, const ChunkArgs& a, hipStream_t s) {
   }
   static_assert(sizeof(ChunkLds<MODE>) <= 160 * 1024, "LDS of a CU");
   const int cols = (a.vdim + 63) / 64;
+  if constexpr (MODE != kChunkDelta)
+    if (a.seg != nullptr) {
+      static bool seg_attr = false;
+      if (!seg_attr) {
+        (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&chunk_recurrence_segments_kernel<TI, TG, MODE>),
+                                  hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+        seg_attr = true;
+      }
+      const dim3 grid(a.H, cols, a.runs + T / a.seg_rows);
+      const dim3 parts(a.H, cols * (NC / kSegKeys), grid.z);
+      if (a.seg_rows >= 64 * CT) hipLaunchKernelGGL((chunk_segment_kernel<TI, MODE, 16>), parts, dim3(1024), 0, s, a);
+      else hipLaunchKernelGGL((chunk_segment_kernel<TI, MODE, 8>), parts, dim3(512), 0, s, a);
+      hipLaunchKernelGGL((chunk_recurrence_segments_kernel<TI, TG, MODE>), grid, dim3(chunk_threads(MODE)),
+                         sizeof(ChunkLds<MODE>), s, a);
+      return;
+    }
   if (a.min_run <= 1)
     hipLaunchKernelGGL((chunk_recurrence_kernel<TI, TG, MODE>), dim3(a.runs, a.H, cols), dim3(chunk_threads(MODE)),
                        sizeof(ChunkLds<MODE>), s, a);

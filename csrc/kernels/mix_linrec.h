@@ -4,6 +4,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <functional>
+
 namespace rfqmix {
 
 struct LinrecArgs {
@@ -31,6 +33,8 @@ struct LinrecArgs {
 };
 
 bool linrec_ok(int dim, int vdim);
-void launch_gated_linrec(bool in_f32, bool act_f32, bool delta, const LinrecArgs& a, hipStream_t s);
+// scratch(n): n floats that stay until the launches are queued
+void launch_gated_linrec(bool in_f32, bool act_f32, bool delta, const LinrecArgs& a,
+                         const std::function<float*(int64_t)>& scratch, hipStream_t s);
 
 }  // namespace rfqmix

@@ -492,7 +492,7 @@ bool linrec_ok(int dim, int vdim) {
 
 // in_f32: q, k, v are fp32 (else bf16); act_f32: beta, gate and out are fp32 (else bf16).
 void launch_gated_linrec(bool in_f32, bool act_f32, bool delta, const LinrecArgs& args,
-                         hipStream_t s) {
+                         const std::function<float*(int64_t)>& scratch, hipStream_t s) {
   LinrecArgs a = args;
   if (a.T == 0 || (a.run_rows != nullptr && a.runs == 0)) return;
   int above = 0;                // runs of up to that many rows are finished by their own kernel
@@ -504,9 +504,10 @@ void launch_gated_linrec(bool in_f32, bool act_f32, bool delta, const LinrecArgs
     c.raw = a.raw; c.state = a.state;
     c.row_state = a.row_state; c.row_back = a.row_back; c.row_fwd = a.row_fwd; c.pos = a.pos;
     c.run_rows = a.run_rows; c.runs = a.runs; c.H = a.H; c.rep = a.rep; c.dim = a.dim; c.vdim = a.vdim;
-    c.slots = a.slots;
+    c.slots = a.slots; c.T = a.T;
     const int mode = delta ? kChunkDelta : kChunkGla;
     a.below = c.min_run = chunk_min_run(mode, a.T, c);
+    if ((c.seg_rows = chunk_seg_rows(mode, in_f32, a.T, c)) > 0) c.seg = scratch(chunk_seg_floats(a.T, c));
     if (c.min_run < INT32_MAX) launch_chunk(mode, in_f32, act_f32, a.T, c, s);
     // Below them: the scan's fixed cost is the larger one (64 decode rows, gla: 41 us against 72),
     // its tokens are the cheaper ones where each has two sums (delta, 64 runs of 8: 106 us against

@@ -9,6 +9,8 @@
 // (-1: none), row_back = index of the row inside its run, row_fwd = rows of the run after it.
 // State pools are double buffered: a run reads its sequence's half and writes the other, and
 // a run that starts at position 0 reads nothing (the slot may hold another sequence's rest).
+#include <functional>
+
 #include "mix_chunk.h"
 #include "mix_common.h"
 
@@ -246,7 +248,7 @@ void launch_wkv_recurrence(bool f32, const void* r, const void* k, const void* v
                            float eps, float* state, const int32_t* row_state,
                            const int32_t* row_back, const int32_t* row_fwd, const int32_t* pos,
                            const int32_t* run_rows, int runs, void* out, int Trows, int H, int N,
-                           int slots, hipStream_t s) {
+                           int slots, const std::function<float*(int64_t)>& scratch, hipStream_t s) {
   if (Trows == 0 || (run_rows != nullptr && runs == 0)) return;
   ChunkArgs a{};
   a.q = r; a.k = k; a.v = v; a.z = zw; a.gate = gate;
@@ -254,8 +256,9 @@ void launch_wkv_recurrence(bool f32, const void* r, const void* k, const void* v
   a.zbias = w0; a.u = u; a.norm_w = norm_w; a.eps = eps; a.q_scale = 1.f;
   a.out = out; a.state = state;
   a.row_state = row_state; a.row_back = row_back; a.row_fwd = row_fwd; a.pos = pos; a.run_rows = run_rows;
-  a.runs = runs; a.H = H; a.rep = 1; a.dim = a.vdim = N; a.slots = slots;
+  a.runs = runs; a.H = H; a.rep = 1; a.dim = a.vdim = N; a.slots = slots; a.T = Trows;
   const int below = a.min_run = chunk_min_run(kChunkWkv, Trows, a);
+  if ((a.seg_rows = chunk_seg_rows(kChunkWkv, f32, Trows, a)) > 0) a.seg = scratch(chunk_seg_floats(Trows, a));
   if (below < INT32_MAX) launch_chunk(kChunkWkv, f32, f32, Trows, a, s);
   if (below == 1) return;
 #define WKV_GO(TT, NRR)                                                                         \

@@ -34,10 +34,10 @@ def _close(got, want, tol):
     assert float((got[ok] - want[ok]).square().mean().sqrt()) <= tol * float(scale)
 
 
-def _linrec(mode, H, Hq, dim, vdim, dtype, shift, lens=LENS, spoil=None):
+def _linrec(mode, H, Hq, dim, vdim, dtype, shift, lens=LENS, spoil=None, pad=3):
     g = torch.Generator().manual_seed(H * 1000 + dim + vdim)
     T = sum(lens)
-    wide = torch.randn(T, 2 * Hq * dim + H * vdim + 3, generator=g)              # columns of wider rows
+    wide = torch.randn(T, 2 * Hq * dim + H * vdim + pad, generator=g)              # columns of wider rows
     qk = wide[:, :2 * Hq * dim].unflatten(1, (2 * Hq, dim))
     qk /= qk.square().sum(-1, keepdim=True).sqrt() / (2.0 if mode == "gla" else 1.0)   # unit vectors: delta rule
     if spoil is not None:
@@ -98,8 +98,8 @@ def test_a_non_finite_value_stays_out_of_earlier_tokens(mode, value):
     _close(out[sum(LENS[:8]):], out_w[sum(LENS[:8]):], 1e-5)  # and no other run sees it
 
 
-def _wkv(dtype, shift, spoil=None):
-    H, N, lens = 3, 64, LENS
+def _wkv(dtype, shift, spoil=None, lens=LENS):
+    H, N = 3, 64
     g = torch.Generator().manual_seed(5)
     T = sum(lens)
     r, k, v, zw, gate = (torch.randn(T, H * N, generator=g) for _ in range(5))
@@ -132,6 +132,44 @@ def test_wkv_non_finite_value_stays_out_of_earlier_tokens():
     (out, _), (out_w, _) = _wkv(torch.float32, -2.0, (first + 9, 3, float("inf")))
     _close(out[:first + 9], out_w[:first + 9], 1e-5)
     _close(out[sum(LENS[:8]):], out_w[sum(LENS[:8]):], 1e-5)
+
+
+# Runs in segments of 128 tokens (a state's way into a segment is one more sum and product a segment): ends just before,
+# at and behind a segment's end, runs that begin and that go on, states of several segments back; rows of wider
+# tensors that a segment's loads of four fit (a pad of 4) and that they do not (3: whole runs).
+SEGMENTS = [700, 1, 129, 128, 255, 257, 400]
+
+
+@pytest.mark.parametrize("shift", [-6.0, 0.0, 60.0])      # decays near one over segments, ordinary, all but zero
+@pytest.mark.parametrize("H,Hq,vdim,pad", [(2, 2, 64, 4), (4, 2, 128, 0), (2, 2, 64, 3)])
+def test_linear_recurrence_in_segments(H, Hq, vdim, pad, shift):
+    (out, st), (out_w, st_w) = _linrec("gla", H, Hq, 64, vdim, torch.float32, shift, lens=SEGMENTS, pad=pad)
+    _close(out, out_w, 1e-5)
+    _close(st, st_w, 1e-5)
+
+
+@pytest.mark.parametrize("lens", [SEGMENTS, [4096 + 40]])     # 4,136: segments of a sixteenth a wave where heads are many
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_wkv_in_segments(dtype, lens):
+    # 1e-5 is for sums of up to 150 tokens; where decays are near one, roundings add up with the root of their number,
+    # in the reference (one sum a token) as here
+    tol = 1e-5 * (max(lens) / 150) ** 0.5
+    for shift in (-6.0, -2.0, 5.0):
+        (out, st), (out_w, st_w) = _wkv(dtype, shift, lens=lens)
+        _close(out, out_w, tol if dtype == torch.float32 else 2.0 ** -8)
+        _close(st, st_w, tol)
+
+
+def test_linear_recurrence_in_segments_bf16():
+    (out, st), (out_w, st_w) = _linrec("gla", 2, 2, 64, 128, torch.bfloat16, 0.0, lens=SEGMENTS, pad=4)
+    _close(out, out_w, 2.0 ** -8)
+    _close(st, st_w, 1e-5)
+
+
+def test_a_non_finite_value_stays_out_of_earlier_segments():
+    (out, _), (out_w, _) = _linrec("gla", 2, 2, 64, 64, torch.float32, 0.0, lens=SEGMENTS, spoil=(300, 3, float("inf")), pad=4)
+    _close(out[:300], out_w[:300], 1e-5)
+    _close(out[700:], out_w[700:], 1e-5)
 
 
 # 40 rows: chunks; 6: token by token; 200 without a list of runs: the scan
