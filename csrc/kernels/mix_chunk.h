@@ -28,17 +28,18 @@ struct ChunkArgs {
   const int32_t *row_state, *row_back, *row_fwd, *pos, *run_rows;
   int runs, H, rep, dim, vdim, slots, T;
   int min_run;                      // shorter runs are left alone
-  int seg_rows = 0;                 // > 0: runs are shared in segments of so many rows, a multiple of 128
-  float* seg = nullptr;             // of every segment but a run's last: [segments, H, dim, vdim] what its rows leave
-                                    // of a state of zeros, then [segments, H, dim] products of its decays
+  int cap = 0, per = 0, unit = 0;   // segments of runs that the step is shared in at most (0: whole runs), workgroups of
+                                    // each, and what divides their rows
+  float* seg = nullptr;             // scratch of cap segments: [cap, H, dim, vdim] what a segment's rows leave of a state of
+                                    // zeros, then [cap, H, dim] products of its decays (delta rule: see delta_seg)
 };
 
 // How a step of T rows is shared: runs of at least this many rows go to the chunked kernel, the
 // others to the token-by-token one (1: all in chunks, INT32_MAX: none).
 int chunk_min_run(int mode, int T, const ChunkArgs& a);
-// Rows of a segment where the step's runs are shared so, else 0, and the scratch floats that they take.
-int chunk_seg_rows(int mode, bool in_f32, int T, const ChunkArgs& a);
-int64_t chunk_seg_floats(int T, const ChunkArgs& a);
+// Segments that the step's runs are shared in at most where they are, else 0 (sets a.per and a.unit), and the scratch floats of a.cap.
+int chunk_seg_cap(int mode, bool in_f32, int T, ChunkArgs& a);
+int64_t chunk_seg_floats(int mode, const ChunkArgs& a);
 // in_f32: q, k, v (and wkv's z, gate, out) are fp32, else bf16; act_f32: beta's type.
 // T: rows of the step.
 void launch_chunk(int mode, bool in_f32, bool act_f32, int T, const ChunkArgs& a, hipStream_t s);

@@ -15,24 +15,28 @@
 // blocks factor at the block's edge: (a_{block} .. a_t) from the reader's side, (a_{s+1} ..) from
 // the writer's, both at most 1; pairs inside a block multiply their decays directly.
 //
-// What bounds it: the chain over a run's chunks, and inside a chunk the instructions of the waves
-// that share a SIMD.  Token by token the chain was 0.2 - 2.6 us a token (LDS round trips, 64 x 64
-// FMAs on one or four waves); here a chunk's chain is 36 (wkv, gla) or 56 (delta) MFMAs of 16x16x4
-// per wave, 1.6 - 2.3 us.  One workgroup per (run, head, 64 value channels): four consumer waves hold
-// 64 x 16 of the state in accumulators, which are MFMA operands as they lie (a lane holds channels
-// 16 i + 4 grp + r of its column: exactly the K slices that step (i, r) of Qd S takes); the other
-// waves work ahead: decays and their products for chunk c + 3, A for chunk c + 2, T for chunk c + 1,
-// wkv's norm and gate for chunk c - 1; one barrier per chunk.  A state operand never leaves the
-// registers, an fp32 operand is never narrowed.  Measured, two runs of 2,048 tokens in bf16: wkv with
-// 64 heads of 64 x 64 5,353 -> 203 us; delta rule with 32 heads of 64 x 128 741 (decays and scan) ->
-// 301 us; gla in fp32, five ragged runs of up to 1,031, 32 heads, 447 -> 121 us.
+// What bounds it: the vector instructions of the waves that share a SIMD, 60 - 70 % of its cycles, and their order inside
+// a chunk.  (fp32 MFMA 16x16x4 hold a SIMD's vector unit for their 32 clocks, other waves' instructions as well: with the
+// state's products in it the decay waves stood for as long as they took, 2.3 us a chunk of the delta rule.)  The state's
+// products, 48 of 56 a wave, therefore go to the matrix cores in bf16: an fp32 operand is the exact sum of three bf16, six
+// products of them leave out less than 2^-26 of each (split3).  Those inside a chunk stay in fp32 MFMA.  Errors against
+// 64 bits: state of the delta rule 6.3e-8 for 6.4e-8 before, outputs of gla in fp32 5.7e-7 and of wkv 2.0e-7, the same.
+// One workgroup per (run, head, 64 or 128 value channels): four consumer waves hold 64 x 16 of the state, or twice that, in
+// accumulators, which are MFMA operands as they lie (a lane holds channels 16 i + 4 grp + r of its column); the other
+// waves work ahead: decays, their products and parts for chunk c + 3, A for chunk c + 2, T for chunk c + 1, wkv's norm
+// and gate for chunk c - 1; one barrier per chunk.  The state never leaves the registers.  A chunk takes 2.1 us with 64
+// channels (delta; gla 1.65, wkv 1.45) and 2.7 with 128 (gla 2.0), for which the other waves' work is done once.
+// Measured, two runs of 2,048 tokens in bf16, all kernels of the recurrence: delta rule with 32 heads of 64 x 128 301 ->
+// 190 us, wkv with 64 heads of 64 x 64 203 -> 136; gla in fp32, five ragged runs of up to 1,031, 32 heads, 121 -> 85.
 //
-// Without the delta rule a run's chain is cut where workgroups leave CUs idle (chunk_seg_rows): chunk_segment_kernel
-// makes what every segment's rows leave of a state of zeros and the products of its decays, all segments at once, and a
-// segment's workgroup begins from the state of before the run carried through those in front of it.  wkv, two runs of
-// 2,048 with 64 heads: 204 -> 26 + 118 us.  What bounds the first kernel: exponentials (22 instructions a decay, 38 of gla)
-// and the way to its first rows and out, 10 us of a workgroup.
+// A run's chain is cut where workgroups leave CUs idle (chunk_seg_cap, segment_rows).  Without the delta rule
+// chunk_segment_kernel makes what every segment's rows leave of a state of zeros and the products of its decays, all
+// segments at once, and a segment's workgroup begins from the state of before the run carried through those in front of
+// it.  What bounds the first kernel: exponentials (22 instructions a decay, 38 of gla) and the way to its first rows and
+// out, 10 us of a workgroup.  The delta rule's first kernel makes matrices of 64 x 64 in place of the products
+// (chunk_delta_first_kernel).  One run of 4,096: delta, 32 heads, 665 -> 299 us a pass, gla 430 -> 172, wkv, 64, 423 -> 196.
 #include <algorithm>
+#include <cmath>
 #include <type_traits>
 
 #include "common.h"
@@ -47,7 +51,9 @@ namespace {
 constexpr int CT = 16;                  // tokens per chunk
 constexpr int NC = kChunkDim;           // key channels (those past dim are zeros)
 constexpr int RS = NC + 4;              // floats per token row in LDS
-constexpr int TS = CT + 4;              // floats per row of a 16 x 16 tile, of Kd^T
+constexpr int TS = CT + 4;              // floats per row of a 16 x 16 tile
+constexpr int PS = NC + 8;              // bf16 per token row of a part of Qd or Kk, per channel row of Kd^T's parts
+constexpr float kTurnMost = 1.001f;     // see chunk_delta_later_kernel
 
 // four consumers, four waves for the decays, four for A (and T), wkv: four for norm and gate
 constexpr int chunk_threads(int mode) { return mode == kChunkWkv ? 1024 : 768; }
@@ -63,9 +69,11 @@ __device__ __forceinline__ float ror_add(float v) {   // sum over the 16 lanes o
 template <int MODE>
 struct ChunkLds {
   static constexpr bool DELTA = MODE == kChunkDelta;
-  float qd[4][CT * RS];                 // four chunks in flight between producers and consumers
-  float kk[DELTA ? 4 : 1][DELTA ? CT * RS : 4];
-  float kd[4][NC * TS];                 // Kd^T
+  // four chunks in flight between producers and consumers; parts as split3 makes them
+  uint16_t qd[4][3][CT * PS];           // [part][token][operand_at(channel)]
+  uint16_t kk[DELTA ? 4 : 1][3][DELTA ? CT * PS : 8];
+  uint16_t kd[4][NC * PS];   // Kd^T: [channel][four tokens: two parts of four, first and third again]
+  uint32_t odd[4][4];                   // of each wave: operands that are split otherwise, see odd_split
   float dec[4][NC];
   float beta[4][CT];
   float aq[4][CT * TS];
@@ -78,6 +86,47 @@ struct ChunkLds {
   float o[2][MODE == kChunkWkv ? CT * RS : 4];
 };
 
+// fp32 as a sum of three bf16, h + m + l, each the rounding of what is left: the sum is exact (8 bits each and two signs).
+// Products of two such sums without m l, l m and l l, of which each is below 2^-26 of the whole product, take six products
+// on the matrix cores, 2.7 times the rate of fp32 MFMA and, other than those, beside the vector instructions of other
+// waves.  Packed in twos: a in the low half.
+struct Split2 {
+  uint32_t h, m, l;
+};
+__device__ __forceinline__ float lo_f(uint32_t x) { return __uint_as_float(x << 16); }
+__device__ __forceinline__ float hi_f(uint32_t x) { return __uint_as_float(x & 0xffff0000u); }
+__device__ __forceinline__ Split2 split3(float a, float b) {
+  Split2 s;
+  s.h = rfq::pack_bf16x2(a, b);
+  a -= lo_f(s.h);
+  b -= hi_f(s.h);
+  s.m = rfq::pack_bf16x2(a, b);
+  s.l = rfq::pack_bf16x2(a - lo_f(s.m), b - hi_f(s.m));
+  return s;
+}
+// The same cut instead of rounded: for values that the rounding takes to infinity; infinities and NaN are h alone.
+constexpr float kSplitMost = 3.38e38f;
+__device__ __forceinline__ Split2 odd_split(float a, float b) {
+  uint32_t p[3][2];
+  float f[2] = {a, b};
+#pragma unroll
+  for (int e = 0; e < 2; ++e) {
+    const uint32_t all = __float_as_uint(f[e]);
+    const bool whole = (all & 0x7f800000u) != 0x7f800000u;
+    p[0][e] = all >> 16 | (!whole && (all & 0xffffu) != 0 ? 1u : 0u);       // a NaN stays one
+    const float r = f[e] - __uint_as_float(all & 0xffff0000u);
+    p[1][e] = whole ? __float_as_uint(r) >> 16 : 0;
+    p[2][e] = whole ? __float_as_uint(r - __uint_as_float(__float_as_uint(r) & 0xffff0000u)) >> 16 : 0;
+  }
+  return {p[0][0] | p[0][1] << 16, p[1][0] | p[1][1] << 16, p[2][0] | p[2][1] << 16};
+}
+// Where a row of an operand's parts holds channel c: a lane's eight of a 16x16x32 product are channels 4 grp + r of two
+// neighbouring tiles of sixteen, as the accumulators of the state hold them.
+__device__ __forceinline__ int operand_at(int c) { return (c & 32) | (c & 12) << 1 | (c & 16) >> 2 | (c & 3); }
+__device__ __forceinline__ f32x4 mma32(const uint4& a, const uint4& b, const f32x4& c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(rfq::bf16x8, a), __builtin_bit_cast(rfq::bf16x8, b), c, 0, 0, 0);
+}
+__device__ __forceinline__ uint4 ld8(const uint16_t* p) { return *reinterpret_cast<const uint4*>(p); }
 __device__ __forceinline__ float4 mul4(float4 x, float4 y) {
   return make_float4(x.x * y.x, x.y * y.y, x.z * y.z, x.w * y.w);
 }
@@ -136,39 +185,89 @@ __device__ __forceinline__ void lower_product(const float* m, const f32x4& x, in
 struct ChunkSegment {
   int run0, t0, n, seg, slot;
   bool last;
+  int rows;                             // of the step's segments but a run's last
 };
 __device__ __forceinline__ ChunkSegment whole_run(const ChunkArgs& a, int t0) {
-  return {t0, t0, a.row_fwd[t0] + 1, 0, 0, true};
-}
-// The slot-th segment of the step's runs in their order, every wave for itself; n = 0: there are fewer.
-__device__ __forceinline__ ChunkSegment find_segment(const ChunkArgs& a, int slot, int lane) {
-  int left = slot;
-  for (int base = 0; base < a.runs; base += 64) {
-    const int r = base + lane < a.runs ? a.run_rows[base + lane] : -1;
-    const int n = r >= 0 && a.row_back[r] == 0 ? a.row_fwd[r] + 1 : 0;
-    const int mine = (n + a.seg_rows - 1) / a.seg_rows;
-    int upto = mine;                                       // segments of the runs up to this lane's
-#pragma unroll
-    for (int o = 1; o < 64; o *= 2) {
-      const int x = __shfl_up(upto, o, 64);
-      if (lane >= o) upto += x;
-    }
-    const uint64_t m = __builtin_amdgcn_ballot_w64(left < upto);
-    if (m != 0) {
-      const int at = __builtin_ctzll(m);
-      const int seg = left - __builtin_amdgcn_readlane(upto - mine, at), rows = __builtin_amdgcn_readlane(n, at);
-      const int run0 = __builtin_amdgcn_readlane(r, at), from = seg * a.seg_rows;
-      return {run0, run0 + from, min(rows - from, a.seg_rows), seg, slot, from + a.seg_rows >= rows};
-    }
-    left -= __builtin_amdgcn_readlane(upto, 63);
-  }
-  return {0, 0, 0, 0, 0, false};
+  return {t0, t0, a.row_fwd[t0] + 1, 0, 0, true, 0};
 }
 
-// 64 value channels, from z64 on, of head h of a run or of a segment of one.
-template <typename TI, typename TG, int MODE>
-__device__ __forceinline__ void chunk_run(const ChunkArgs& a, const ChunkSegment& sg, const int h, const int z64, const int tid) {
+// How long the step's segments are: only the device knows its runs (64 at most).  Lane l tries the longest run in l + 1
+// equal parts (of whole chunks, a.unit rows where the first kernel shares a segment over its waves); of those that make no
+// more than a.cap segments (workgroups of one of the delta rule's kernels) the one takes over that the times below (us, as measured) say is done first.  The same for
+// every wave of both kernels.
+template <int MODE, int NV>
+__device__ __forceinline__ int segment_rows(const ChunkArgs& a, int n, int lane) {
+  constexpr bool DELTA = MODE == kChunkDelta;
+  int longest = n;
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) longest = max(longest, __shfl_xor(longest, o, 64));
+  const int rows = (int)((uint32_t)(longest + lane) / (uint32_t)(lane + 1) + a.unit - 1) / a.unit * a.unit;
+  int all = 0, cut = 0, runs = 0, most = 0;                  // segments, runs of more than one, runs, segments of one
+  for (int r = 0; r < a.runs; ++r) {
+    const int m = __builtin_amdgcn_readlane(n, r);
+    const int parts = rows > 0 ? (int)((uint32_t)(m + rows - 1) / (uint32_t)rows) : 0;
+    all += parts;
+    cut += parts > 1;
+    most = max(most, parts);
+    runs += m > 0;
+  }
+  auto rounds = [&](int segments) { return (float)((segments * a.per + 255) / 256); };
+  const float c = (float)((min(rows, longest) + CT - 1) / CT);
+  float t;
+  if constexpr (DELTA) t = rounds(all - cut) * (9.f + 2.7f * c) + (all > runs ? 3.f + rounds(all - runs) * (11.f + 2.8f * c) + 3.f * (most - 2) : 0.f);
+  else t = rounds(all) * (6.f + (MODE == kChunkWkv ? 1.45f : NV == 1 ? 1.65f : 2.f) * c) + (all > runs ? 10.f + 0.25f * c + 0.8f * most : 0.f);
+  uint32_t best = (DELTA ? all - cut : all) <= a.cap ? (__float_as_uint(t) & ~63u) | (uint32_t)lane : ~0u;
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) best = min(best, (uint32_t)__shfl_xor((int)best, o, 64));
+  return __builtin_amdgcn_readlane(rows, (int)(best & 63u));
+}
+// The item-th segment of the step's runs in their order that the kernel has work for, every wave for itself; n = 0: there
+// are fewer.  Items without a gap: where workgroups that leave at once lie between others, those of one remainder are
+// left for the same few CUs, which then take two rounds (240 on 256 CUs: 72 us for 36).
+enum SegmentKind { kAllSegments, kFirstSegments, kLaterSegments };   // all; a run's only one or all but its last; but its first
+template <int MODE, int NV, int KIND>
+__device__ __forceinline__ ChunkSegment find_segment(const ChunkArgs& a, int item, int lane) {
+  const int r = lane < a.runs ? a.run_rows[lane] : -1;
+  const int n = r >= 0 && a.row_back[r] == 0 ? a.row_fwd[r] + 1 : 0;
+  const int size = segment_rows<MODE, NV>(a, n, lane);
+  if (size == 0) return {0, 0, 0, 0, 0, false, 0};
+  const int parts = (n + size - 1) / size;
+  const int mine = parts - (KIND == kLaterSegments ? parts > 0 : KIND == kFirstSegments ? parts > 1 : 0);
+  int upto = mine;                                         // items of the runs up to this lane's
+#pragma unroll
+  for (int o = 1; o < 64; o *= 2) {
+    const int x = __shfl_up(upto, o, 64);
+    if (lane >= o) upto += x;
+  }
+  const uint64_t m = __builtin_amdgcn_ballot_w64(item < upto);
+  if (m == 0) return {0, 0, 0, 0, 0, false, 0};
+  const uint64_t single = __builtin_amdgcn_ballot_w64(parts == 1);
+  const int at = __builtin_ctzll(m);
+  const int before = __builtin_amdgcn_readlane(upto - mine, at), rows = __builtin_amdgcn_readlane(n, at);
+  const int seg = item - before + (KIND == kLaterSegments ? 1 : 0);
+  // the slot is the item of all or of the first segments
+  const int slot = KIND == kLaterSegments ? before + __builtin_popcountll(single & ((1ull << at) - 1)) + seg : item;
+  const int run0 = __builtin_amdgcn_readlane(r, at), from = seg * size;
+  return {run0, run0 + from, min(rows - from, size), seg, slot, from + size >= rows, size};
+}
+
+// Scratch of the delta rule's segments: what a segment leaves of a state of zeros (a run's first one: the state itself),
+// [slots, H, dim, vdim]; what it makes of a state, [slots, H, NC, NC]; whether that is bounded, [slots, H, 4].
+struct DeltaSeg {
+  float *left, *turn, *wild;
+};
+__device__ __forceinline__ DeltaSeg delta_seg(const ChunkArgs& a, int slot, int h) {
+  const int64_t n = (int64_t)a.cap * a.H, at = (int64_t)slot * a.H + h, hsz = (int64_t)NC * a.vdim;
+  return {a.seg + at * hsz, a.seg + n * hsz + at * NC * NC, a.seg + n * (hsz + NC * NC) + at * 4};
+}
+
+// 64 NV value channels, from zv on, of head h of a run or of a segment of one.  TURN: beside what the rows leave of a
+// state of zeros, what they make of any: the state's own columns are 64 more, which begin as the unit matrix and take no
+// values; there are no read-outs.
+template <typename TI, typename TG, int MODE, int NV = 1, bool TURN = false>
+__device__ __forceinline__ void chunk_run(const ChunkArgs& a, const ChunkSegment& sg, const int h, const int zv, const int tid) {
   constexpr bool WKV = MODE == kChunkWkv, DELTA = MODE == kChunkDelta;
+  constexpr int NT = NV + (TURN ? 1 : 0);                 // tiles of 16 columns a consumer wave holds
   const int lane = tid & 63, col = lane & 15, grp = lane >> 4;
   const int t0 = sg.t0, n = sg.n, nc = (n + CT - 1) / CT;
   const int code = a.row_state[sg.run0];
@@ -185,26 +284,35 @@ __device__ __forceinline__ void chunk_run(const ChunkArgs& a, const ChunkSegment
       (&L.tt[0][0])[x] = 0.f;
     }
 
-  // Row offsets inside a chunk in bytes (the launcher bounds 16 rows by 2^31); a chunk's first row
-  // is a wave-uniform pointer.  Rows past the run's end are read as its last row and left out later.
-  auto offsets = [&](uint32_t (&o)[4], int64_t stride, int first, int esz, int c) {
+  // Offsets inside a chunk in bytes (the launcher bounds 16 rows by 2^31), of a lane's four rows and its column; a chunk's
+  // first row is a wave-uniform pointer, which goes on from chunk to chunk: a product for every turn's address costs the
+  // wave more than the load.  Rows past the run's end are read as its last row and left out later.
+  auto offsets = [&](uint32_t (&o)[4], int64_t stride, int column, int esz, int c) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) o[i] = (uint32_t)min(first + i, n - 1 - c * CT) * (uint32_t)(stride * esz);
+    for (int i = 0; i < 4; ++i) o[i] = (uint32_t)min(4 * grp + i, n - 1 - c * CT) * (uint32_t)(stride * esz) + (uint32_t)(column * esz);
   };
-  // ---- consumers: 16 value channels, S[16 i + 4 grp + r][column]
-  const int vcol = z64 + 16 * w + col;
-  const bool vlive = vcol < vdim;
+  // ---- consumers: tiles of 16 value channels, S[16 i + 4 grp + r][column]
+  const int vcol = zv + 16 * NV * w + col;                // of the first tile
+  auto vlive = [&](int j) { return vcol + 16 * j < vdim; };
   const bool from_state = code >= 0 && a.pos[sg.run0] > 0;
   const int64_t hsz = (int64_t)dim * vdim;
-  f32x4 st[4];
-  TI vreg[4];
+  f32x4 st[NT][4];
+  TI vreg[NV][4];
   uint32_t vo[4];
-  const TI* vb = static_cast<const TI*>(a.v) + t0 * a.vs + (int64_t)h * vdim;
-  auto fetch_v = [&](int c) {
-    if (c * CT + CT > n) offsets(vo, a.vs, 4 * grp, sizeof(TI), c);   // the last, partial chunk
-    const TI* base = vb + (int64_t)c * CT * a.vs;
+  const TI* vb = static_cast<const TI*>(a.v) + t0 * a.vs + (int64_t)h * vdim;     // of the chunk in flight
+  int cf = 0;
+  auto next_v = [&]() {                                   // behind the last chunk: that again
+    if (cf + 1 < nc) {
+      ++cf;
+      vb += CT * a.vs;
+      if (cf * CT + CT > n) offsets(vo, a.vs, min(vcol, vdim - 1), sizeof(TI), cf);   // the last, partial chunk
+    }
+  };
+  auto fetch_v = [&]() {
 #pragma unroll
-    for (int r = 0; r < 4; ++r) vreg[r] = load_at(base, vo[r] + (uint32_t)(min(vcol, vdim - 1) * sizeof(TI)));
+    for (int r = 0; r < 4; ++r)
+#pragma unroll
+      for (int j = 0; j < NV; ++j) vreg[j][r] = load_at(vb, vo[r] + (uint32_t)((min(vcol + 16 * j, vdim - 1) - min(vcol, vdim - 1)) * sizeof(TI)));
   };
   // ---- producers: a lane has four tokens of one key channel
   const int ch = 16 * w + col, chl = min(ch, dim - 1);
@@ -221,55 +329,122 @@ __device__ __forceinline__ void chunk_run(const ChunkArgs& a, const ChunkSegment
   const TZ* zb = static_cast<const TZ*>(a.z) + t0 * a.zs + (int64_t)h * dim;
   const TG* bb = DELTA ? static_cast<const TG*>(a.beta) + t0 * a.bs + h : nullptr;
   const TI* gb = WKV ? static_cast<const TI*>(a.gate) + t0 * a.gs + (int64_t)h * vdim : nullptr;
-  auto fetch = [&](int c) {
-    if (c * CT + CT > n) {
-      offsets(qo, a.qs, 4 * grp, sizeof(TI), c);
-      offsets(ko, a.ks, 4 * grp, sizeof(TI), c);
-      offsets(zo, a.zs, 4 * grp, sizeof(TZ), c);
+  auto next = [&]() {                                     // behind the last chunk: that again
+    if (cf + 1 < nc) {
+      ++cf;
+      qb += CT * a.qs;
+      kb += CT * a.ks;
+      zb += CT * a.zs;
+      if (cf * CT + CT > n) {
+        offsets(qo, a.qs, chl, sizeof(TI), cf);
+        offsets(ko, a.ks, chl, sizeof(TI), cf);
+        offsets(zo, a.zs, chl, sizeof(TZ), cf);
+      }
     }
-    const TI *q = qb + (int64_t)c * CT * a.qs, *k = kb + (int64_t)c * CT * a.ks;
-    const TZ* z = zb + (int64_t)c * CT * a.zs;
+  };
+  auto fetch = [&]() {
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      rq[i] = load_at(q, qo[i] + (uint32_t)(chl * sizeof(TI)));
-      rk[i] = load_at(k, ko[i] + (uint32_t)(chl * sizeof(TI)));
-      rz[i] = load_at(z, zo[i] + (uint32_t)(chl * sizeof(TZ)));
+      if constexpr (!TURN) rq[i] = load_at(qb, qo[i]);
+      rk[i] = load_at(kb, ko[i]);
+      rz[i] = load_at(zb, zo[i]);
     }
-    if constexpr (DELTA) rb = load_at(bb + (int64_t)min(c * CT + col, n - 1) * a.bs, 0);
+    if constexpr (DELTA) rb = load_at(bb + (int64_t)min(cf * CT + col, n - 1) * a.bs, 0);
   };
   float4 nw = {}, bonus = {};
   float zbias = 0.f, rate = 0.f;
 
   if (role == 0) {
-    offsets(vo, a.vs, 4 * grp, sizeof(TI), 0);
+    offsets(vo, a.vs, min(vcol, vdim - 1), sizeof(TI), 0);
     const float* rd = a.state + (((int64_t)(code & 1) * a.slots + (code >> 1)) * H + h) * hsz;
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+    for (int j = 0; j < NT; ++j)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int c = 16 * i + 4 * grp + r;
-        st[i][r] = (from_state && vlive && c < dim) ? rd[(int64_t)c * vdim + vcol] : 0.f;
-      }
-    fetch_v(0);
-    if constexpr (!DELTA) {
-      const int64_t slots = a.runs + a.T / max(a.seg_rows, 1);
-      for (int j = sg.slot - sg.seg; j < sg.slot; ++j) {     // the run's segments before this one
-        const float* left = a.seg + ((int64_t)j * H + h) * hsz + vcol;
-        const float* kept = a.seg + slots * H * hsz + ((int64_t)j * H + h) * dim;
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int c = 16 * i + 4 * grp + r;
+          if constexpr (TURN) st[j][i][r] = j == NV && c == 16 * w + col ? 1.f : 0.f;
+          else st[j][i][r] = (from_state && vlive(j) && c < dim) ? rd[(int64_t)c * vdim + vcol + 16 * j] : 0.f;
+        }
+    fetch_v();
+    if constexpr (DELTA && !TURN) {
+      if (sg.seg > 0) {
+        // from the state behind the run's first segment through the others before this one
+        const uint32_t lo = (uint32_t)(4 * grp * vdim + vcol) * 4, to = (uint32_t)(col * NC + 4 * grp) * 4;
+        const float* left = delta_seg(a, sg.slot - sg.seg, h).left;
 #pragma unroll
         for (int i = 0; i < 4; ++i)
 #pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            const int c = 16 * i + 4 * grp + r;
-            st[i][r] = fmaf(kept[c], st[i][r], left[(int64_t)c * vdim]);
+          for (int r = 0; r < 4; ++r)
+#pragma unroll
+            for (int j = 0; j < NT; ++j) st[j][i][r] = load_at(left + (16 * i + r) * vdim, lo + 64 * j);
+#pragma unroll 1
+        for (int s = sg.slot - sg.seg + 1; s < sg.slot; ++s) {
+          const DeltaSeg d = delta_seg(a, s, h);
+          f32x4 sum[NT][4];
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+#pragma unroll
+              for (int j = 0; j < NT; ++j) sum[j][i][r] = load_at(d.left + (16 * i + r) * vdim, lo + 64 * j);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            float4 m[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) m[i] = load_at(reinterpret_cast<const float4*>(d.turn + 16 * i * NC + 16 * e), to);
+#define CHUNK_TURN(r, f)                                                                                \
+  do {                                                                                                  \
+    _Pragma("unroll") for (int j = 0; j < NT; ++j)                                                      \
+      _Pragma("unroll") for (int i = 0; i < 4; ++i)                                                     \
+        sum[j][i] = __builtin_amdgcn_mfma_f32_16x16x4f32(m[i].f, st[j][e][r], sum[j][i], 0, 0, 0);      \
+  } while (0)
+            CHUNK_TURN(0, x);
+            CHUNK_TURN(1, y);
+            CHUNK_TURN(2, z);
+            CHUNK_TURN(3, w);
+#undef CHUNK_TURN
+          }
+#pragma unroll
+          for (int j = 0; j < NT; ++j)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) st[j][i] = sum[j][i];
+        }
+      }
+    }
+    if constexpr (!DELTA) {
+      const uint32_t lo = (uint32_t)(4 * grp * vdim + vcol) * 4;
+#pragma unroll 1
+      for (int s = sg.slot - sg.seg; s < sg.slot; ++s) {     // through the run's segments before this one
+        const float* left = a.seg + ((int64_t)s * H + h) * hsz;
+        const float* kept = a.seg + (int64_t)a.cap * H * hsz + ((int64_t)s * H + h) * dim + 4 * grp;
+        float x[NT][4][4];
+        float4 f[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          f[i] = ld4(kept + 16 * i);
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+#pragma unroll
+            for (int j = 0; j < NT; ++j) x[j][i][r] = load_at(left + (16 * i + r) * vdim, lo + 64 * j);
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+          for (int j = 0; j < NT; ++j) {
+            st[j][i][0] = fmaf(f[i].x, st[j][i][0], x[j][i][0]);
+            st[j][i][1] = fmaf(f[i].y, st[j][i][1], x[j][i][1]);
+            st[j][i][2] = fmaf(f[i].z, st[j][i][2], x[j][i][2]);
+            st[j][i][3] = fmaf(f[i].w, st[j][i][3], x[j][i][3]);
           }
       }
     }
   } else if (role == 1) {
-    offsets(qo, a.qs, 4 * grp, sizeof(TI), 0);
-    offsets(ko, a.ks, 4 * grp, sizeof(TI), 0);
-    offsets(zo, a.zs, 4 * grp, sizeof(TZ), 0);
-    fetch(0);
+    offsets(qo, a.qs, chl, sizeof(TI), 0);
+    offsets(ko, a.ks, chl, sizeof(TI), 0);
+    offsets(zo, a.zs, chl, sizeof(TZ), 0);
+    fetch();
     zbias = a.zbias[h * dim + chl];
     if constexpr (!WKV) rate = a.rate[h];
   } else if constexpr (WKV) {
@@ -283,114 +458,183 @@ __device__ __forceinline__ void chunk_run(const ChunkArgs& a, const ChunkSegment
   const int turns = nc + (WKV ? 1 : 0);                   // and three turns ahead of them
   if (role == 0) {
     for (int i = 0; i < 3; ++i) __syncthreads();
-    // The operands of the next chunk are there a turn ahead: they are read into registers behind the
-    // products that use the present ones.
-    float4 qa[4], ka[DELTA ? 4 : 1], kh[4], dc[4], aa;
-    auto queries = [&](int b) {
+    // The next chunk's values are waited for before this chunk's read-outs are stored: a wait at the top of the turn
+    // would be one for the stores, which are counted with the loads and in order.
+    float v[NV][4];
+    auto values = [&](int c) {
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        qa[i] = ld4(&L.qd[b][col * RS + 16 * i + 4 * grp]);
-        if constexpr (DELTA) ka[i] = ld4(&L.kk[b][col * RS + 16 * i + 4 * grp]);
+      for (int j = 0; j < NV; ++j)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) v[j][r] = arrived(vreg[j][r]);
+      if (!vlive(NV - 1) || c * CT + CT > n) {
+#pragma unroll
+        for (int j = 0; j < NV; ++j)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) v[j][r] = vlive(j) && c * CT + 4 * grp + r < n ? v[j][r] : 0.f;
       }
     };
-    auto keys = [&](int b) {
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        kh[i] = ld4(&L.kd[b][(16 * i + col) * TS + 4 * grp]);
-        dc[i] = ld4(&L.dec[b][16 * i + 4 * grp]);
-      }
-      aa = ld4(&L.aq[b][col * TS + 4 * grp]);
-    };
-    queries(0);
-    keys(0);
+    values(0);
+    float* rw = WKV || TURN ? nullptr : a.raw + ((int64_t)t0 * H + h) * vdim;
+    const uint32_t ro = (uint32_t)(4 * grp * H * vdim + vcol);
     for (int it = 0; it < nc; ++it) {
       const int b = it & 3;
-      float v[4];
+      next_v();
+      fetch_v();
+      f32x4 o[NT], u[NT], y[NT];
+      const uint16_t *qp = &L.qd[b][0][col * PS + 8 * grp], *kp = &L.kk[DELTA ? b : 0][0][col * PS + 8 * grp];
+      const uint16_t* sp = &L.kd[b][col * PS + 16 * grp];
 #pragma unroll
-      for (int r = 0; r < 4; ++r) v[r] = arrived(vreg[r]);
-      fetch_v(min(it + 1, nc - 1));
-      if (!vlive || it * CT + CT > n) {
+      for (int j = 0; j < NT; ++j) o[j] = y[j] = (f32x4){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int r = 0; r < 4; ++r) v[r] = vlive && it * CT + 4 * grp + r < n ? v[r] : 0.f;
+      for (int e = 0; e < 2; ++e) {
+        uint4 qa[3], ka[3];
+#pragma unroll
+        for (int p = 0; p < 3; ++p) {
+          if constexpr (DELTA) ka[p] = ld8(kp + p * CT * PS + 32 * e);
+          if constexpr (!TURN) qa[p] = ld8(qp + p * CT * PS + 32 * e);
+        }
+#pragma unroll
+        for (int j = 0; j < NT; ++j) {
+          const f32x4 &s0 = st[j][2 * e], &s1 = st[j][2 * e + 1];
+          const Split2 x0 = split3(s0[0], s0[1]), x1 = split3(s0[2], s0[3]), x2 = split3(s1[0], s1[1]), x3 = split3(s1[2], s1[3]);
+          const uint4 h = make_uint4(x0.h, x1.h, x2.h, x3.h), m = make_uint4(x0.m, x1.m, x2.m, x3.m),
+                      l = make_uint4(x0.l, x1.l, x2.l, x3.l);
+          auto product = [&](const uint4 (&a)[3], f32x4& to) {
+            to = mma32(a[2], h, to);
+            to = mma32(a[0], l, to);
+            to = mma32(a[1], m, to);
+            to = mma32(a[1], h, to);
+            to = mma32(a[0], m, to);
+            to = mma32(a[0], h, to);
+          };
+          if constexpr (DELTA) product(ka, y[j]);
+          if constexpr (!TURN) product(qa, o[j]);
+        }
       }
-      f32x4 o = (f32x4){0.f, 0.f, 0.f, 0.f}, u;
+      __builtin_amdgcn_sched_barrier(0);                  // operands of later products wait: registers
+      const uint4 oddw = *reinterpret_cast<const uint4*>(L.odd[b]);
+      bool plain = (oddw.x | oddw.y | oddw.z | oddw.w) == 0;
+#pragma unroll
+      for (int j = 0; j < NT; ++j) plain = plain && finite4(o[j]) && finite4(y[j]);
+      // Infinities, NaN, and values that a part cannot hold: in fp32 products
+      const bool odd = __builtin_amdgcn_ballot_w64(!plain) != 0ull;
+      if (odd) {
+#pragma unroll
+        for (int j = 0; j < NT; ++j) o[j] = y[j] = (f32x4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const int at = 32 * (i >> 1) + 4 * (i & 1) + r;
+            auto whole = [&](const uint16_t* p) { return (ldf(p + at) + ldf(p + at + CT * PS)) + ldf(p + at + 2 * CT * PS); };
+#pragma unroll
+            for (int j = 0; j < NT; ++j) {
+              if constexpr (DELTA) y[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(whole(kp), st[j][i][r], y[j], 0, 0, 0);
+              if constexpr (!TURN) o[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(whole(qp), st[j][i][r], o[j], 0, 0, 0);
+            }
+          }
+      }
       if constexpr (DELTA) {
         const float4 bt = ld4(&L.beta[b][4 * grp]), ta = ld4(&L.tt[it & 1][col * TS + 4 * grp]);
-        f32x4 y = (f32x4){0.f, 0.f, 0.f, 0.f};
+        f32x4 x[NT];
+        bool whole = true;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          y = __builtin_amdgcn_mfma_f32_16x16x4f32(ka[i].x, st[i][0], y, 0, 0, 0);
-          o = __builtin_amdgcn_mfma_f32_16x16x4f32(qa[i].x, st[i][0], o, 0, 0, 0);
-          y = __builtin_amdgcn_mfma_f32_16x16x4f32(ka[i].y, st[i][1], y, 0, 0, 0);
-          o = __builtin_amdgcn_mfma_f32_16x16x4f32(qa[i].y, st[i][1], o, 0, 0, 0);
-          y = __builtin_amdgcn_mfma_f32_16x16x4f32(ka[i].z, st[i][2], y, 0, 0, 0);
-          o = __builtin_amdgcn_mfma_f32_16x16x4f32(qa[i].z, st[i][2], o, 0, 0, 0);
-          y = __builtin_amdgcn_mfma_f32_16x16x4f32(ka[i].w, st[i][3], y, 0, 0, 0);
-          o = __builtin_amdgcn_mfma_f32_16x16x4f32(qa[i].w, st[i][3], o, 0, 0, 0);
+        for (int j = 0; j < NT; ++j) {
+          const f32x4 own = j < NV ? (f32x4){v[j % NV][0], v[j % NV][1], v[j % NV][2], v[j % NV][3]} : (f32x4){0.f, 0.f, 0.f, 0.f};
+          x[j] = (f32x4){bt.x * (own[0] - y[j][0]), bt.y * (own[1] - y[j][1]), bt.z * (own[2] - y[j][2]), bt.w * (own[3] - y[j][3])};
+          u[j] = (f32x4){0.f, 0.f, 0.f, 0.f};
+          whole = whole && finite4(x[j]);
         }
-        const f32x4 x = {bt.x * (v[0] - y[0]), bt.y * (v[1] - y[1]), bt.z * (v[2] - y[2]), bt.w * (v[3] - y[3])};
-        u = (f32x4){0.f, 0.f, 0.f, 0.f};
-        if (__builtin_amdgcn_ballot_w64(!finite4(x)) == 0ull) {
-          u = __builtin_amdgcn_mfma_f32_16x16x4f32(ta.x, x[0], u, 0, 0, 0);
-          u = __builtin_amdgcn_mfma_f32_16x16x4f32(ta.y, x[1], u, 0, 0, 0);
-          u = __builtin_amdgcn_mfma_f32_16x16x4f32(ta.z, x[2], u, 0, 0, 0);
-          u = __builtin_amdgcn_mfma_f32_16x16x4f32(ta.w, x[3], u, 0, 0, 0);
+        if (__builtin_amdgcn_ballot_w64(!whole) == 0ull) {
+#pragma unroll
+          for (int j = 0; j < NT; ++j) u[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(ta.x, x[j][0], u[j], 0, 0, 0);
+#pragma unroll
+          for (int j = 0; j < NT; ++j) u[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(ta.y, x[j][1], u[j], 0, 0, 0);
+#pragma unroll
+          for (int j = 0; j < NT; ++j) u[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(ta.z, x[j][2], u[j], 0, 0, 0);
+#pragma unroll
+          for (int j = 0; j < NT; ++j) u[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(ta.w, x[j][3], u[j], 0, 0, 0);
         } else {
-          lower_product(L.tt[it & 1], x, col, grp, u);
+#pragma unroll
+          for (int j = 0; j < NT; ++j) lower_product(L.tt[it & 1], x[j], col, grp, u[j]);
         }
       } else {
-        f32x4 o2 = (f32x4){0.f, 0.f, 0.f, 0.f};           // two independent chains
 #pragma unroll
-        for (int i = 0; i < 4; i += 2) {
-          o = __builtin_amdgcn_mfma_f32_16x16x4f32(qa[i].x, st[i][0], o, 0, 0, 0);
-          o2 = __builtin_amdgcn_mfma_f32_16x16x4f32(qa[i + 1].x, st[i + 1][0], o2, 0, 0, 0);
-          o = __builtin_amdgcn_mfma_f32_16x16x4f32(qa[i].y, st[i][1], o, 0, 0, 0);
-          o2 = __builtin_amdgcn_mfma_f32_16x16x4f32(qa[i + 1].y, st[i + 1][1], o2, 0, 0, 0);
-          o = __builtin_amdgcn_mfma_f32_16x16x4f32(qa[i].z, st[i][2], o, 0, 0, 0);
-          o2 = __builtin_amdgcn_mfma_f32_16x16x4f32(qa[i + 1].z, st[i + 1][2], o2, 0, 0, 0);
-          o = __builtin_amdgcn_mfma_f32_16x16x4f32(qa[i].w, st[i][3], o, 0, 0, 0);
-          o2 = __builtin_amdgcn_mfma_f32_16x16x4f32(qa[i + 1].w, st[i + 1][3], o2, 0, 0, 0);
-        }
-        o += o2;
-        u = (f32x4){v[0], v[1], v[2], v[3]};
+        for (int j = 0; j < NT; ++j) u[j] = (f32x4){v[j][0], v[j][1], v[j][2], v[j][3]};
       }
-      queries((it + 1) & 3);
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        st[i][0] *= dc[i].x;
-        st[i][1] *= dc[i].y;
-        st[i][2] *= dc[i].z;
-        st[i][3] *= dc[i].w;
+        const float4 dc = ld4(&L.dec[b][16 * i + 4 * grp]);
+#pragma unroll
+        for (int j = 0; j < NT; ++j) {
+          st[j][i][0] *= dc.x;
+          st[j][i][1] *= dc.y;
+          st[j][i][2] *= dc.z;
+          st[j][i][3] *= dc.w;
+        }
       }
-#define CHUNK_STATE(r, f)                                                           \
-do {                                                                              \
-  st[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(kh[0].f, u[r], st[0], 0, 0, 0);    \
-  st[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(kh[1].f, u[r], st[1], 0, 0, 0);    \
-  st[2] = __builtin_amdgcn_mfma_f32_16x16x4f32(kh[2].f, u[r], st[2], 0, 0, 0);    \
-  st[3] = __builtin_amdgcn_mfma_f32_16x16x4f32(kh[3].f, u[r], st[3], 0, 0, 0);    \
-} while (0)
-      if (__builtin_amdgcn_ballot_w64(!finite4(u)) != 0ull) {
-        lower_product(L.aq[b], u, col, grp, o);
+      bool small = true;                                  // within what a part can hold
+#pragma unroll
+      for (int j = 0; j < NT; ++j) small = small && (fabsf(u[j][0]) + fabsf(u[j][1])) + (fabsf(u[j][2]) + fabsf(u[j][3])) < kSplitMost;
+      if (odd || __builtin_amdgcn_ballot_w64(!small) != 0ull) {
+#pragma unroll
+        for (int j = 0; j < NT; ++j) {
+          if constexpr (!TURN) lower_product(L.aq[b], u[j], col, grp, o[j]);
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+              const uint16_t* p = sp + 16 * i * PS + r;
+              const float k = (ldf(p) + ldf(p + 4)) + ldf(p + 12);
+              st[j][i] = __builtin_amdgcn_mfma_f32_16x16x4f32(k, u[j][r], st[j][i], 0, 0, 0);
+            }
+        }
       } else {
-        o = __builtin_amdgcn_mfma_f32_16x16x4f32(aa.x, u[0], o, 0, 0, 0);
-        o = __builtin_amdgcn_mfma_f32_16x16x4f32(aa.y, u[1], o, 0, 0, 0);
-        o = __builtin_amdgcn_mfma_f32_16x16x4f32(aa.z, u[2], o, 0, 0, 0);
-        o = __builtin_amdgcn_mfma_f32_16x16x4f32(aa.w, u[3], o, 0, 0, 0);
+        if constexpr (!TURN) {
+          const float4 aa = ld4(&L.aq[b][col * TS + 4 * grp]);
+#pragma unroll
+          for (int j = 0; j < NT; ++j) o[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(aa.x, u[j][0], o[j], 0, 0, 0);
+#pragma unroll
+          for (int j = 0; j < NT; ++j) o[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(aa.y, u[j][1], o[j], 0, 0, 0);
+#pragma unroll
+          for (int j = 0; j < NT; ++j) o[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(aa.z, u[j][2], o[j], 0, 0, 0);
+#pragma unroll
+          for (int j = 0; j < NT; ++j) o[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(aa.w, u[j][3], o[j], 0, 0, 0);
+        }
+        // a lane's eight are two parts of four tokens: (l h + h l), (h m + m m), (h h + m h)
+        uint4 kh[4][2];
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+          for (int p = 0; p < 2; ++p) kh[i][p] = ld8(sp + 16 * i * PS + 8 * p);
+#pragma unroll
+        for (int j = 0; j < NT; ++j) {
+          const Split2 p = split3(u[j][0], u[j][1]), q = split3(u[j][2], u[j][3]);
+          const uint4 lh = make_uint4(p.l, q.l, p.h, q.h), mm = make_uint4(p.m, q.m, p.m, q.m), hh = make_uint4(p.h, q.h, p.h, q.h);
+#pragma unroll
+          for (int i = 0; i < 4; ++i) st[j][i] = mma32(kh[i][1], lh, st[j][i]);
+#pragma unroll
+          for (int i = 0; i < 4; ++i) st[j][i] = mma32(kh[i][0], mm, st[j][i]);
+#pragma unroll
+          for (int i = 0; i < 4; ++i) st[j][i] = mma32(kh[i][0], hh, st[j][i]);
+        }
       }
-      CHUNK_STATE(0, x);
-      CHUNK_STATE(1, y);
-      CHUNK_STATE(2, z);
-      CHUNK_STATE(3, w);
-#undef CHUNK_STATE
-      keys((it + 1) & 3);
+      values(min(it + 1, nc - 1));
+      __builtin_amdgcn_sched_barrier(0);
       if constexpr (WKV) {
 #pragma unroll
-        for (int r = 0; r < 4; ++r) L.o[it & 1][(4 * grp + r) * RS + 16 * w + col] = o[r];
-      } else {
-        float* rw = a.raw + ((int64_t)(t0 + it * CT + 4 * grp) * H + h) * vdim + vcol;
+        for (int r = 0; r < 4; ++r) L.o[it & 1][(4 * grp + r) * RS + 16 * w + col] = o[0][r];
+      } else if constexpr (!TURN) {
+        float* row = rw;                                  // of the chunk's first row, then the next
+        const bool all = it * CT + CT <= n && zv + 64 * NV <= vdim;
 #pragma unroll
-        for (int r = 0; r < 4; ++r)
-          if (vlive && it * CT + 4 * grp + r < n) rw[(int64_t)r * H * vdim] = o[r] * a.q_scale;
+        for (int r = 0; r < 4; ++r) {
+#pragma unroll
+          for (int j = 0; j < NT; ++j)
+            if (all || (vlive(j) && it * CT + 4 * grp + r < n)) row[ro + 16 * j] = o[j][r] * a.q_scale;
+          row += H * vdim;
+        }
+        rw += (int64_t)CT * H * vdim;
       }
       __syncthreads();
     }
@@ -400,12 +644,14 @@ do {                                                                            
       float q[4], k[4], d[4], bt = 0.f;
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        q[i] = arrived(rq[i]);
+        q[i] = 0.f;
+        if constexpr (!TURN) q[i] = arrived(rq[i]);
         k[i] = arrived(rk[i]);
         d[i] = arrived(rz[i]) + zbias;
       }
       if constexpr (DELTA) bt = arrived(rb);
-      fetch(min(it + 4, nc - 1));
+      next();
+      fetch();
       if (const int c = it + 3; c < nc) {                 // decays and their products of chunk c
         const int b = c & 3, e = c & 1;
 #pragma unroll
@@ -437,27 +683,54 @@ do {                                                                            
         const float post = ((grp & 1) ? 1.f : b1) * ((grp & 2) ? 1.f : b23);
         if (grp == 0) L.dec[b][ch] = up[3] * post;
         L.blk[e][grp * NC + ch] = up[3];
-        float4 kd;
-        float* kdp = reinterpret_cast<float*>(&kd);
+        float qd[4], kk[4], kd[4], most = 0.f;
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           const int at = (4 * grp + i) * RS + ch;
           const float ql = WKV ? (i == 0 ? q[0] : q[i] * up[i - 1]) : q[i] * up[i];
           const float kl = k[i] * after[i];
-          L.qd[b][at] = ql * pre;
-          kdp[i] = kl * post;
-          L.q[e][at] = q[i];
+          kd[i] = kl * post;
+          qd[i] = ql * pre;
+          kk[i] = 0.f;
+          most += fabsf(kd[i]) + fabsf(qd[i]);
+          if constexpr (!TURN) {
+            L.q[e][at] = q[i];
+            L.ql[e][at] = ql;
+          }
           L.k[e][at] = k[i];
           L.a[e][at] = d[i];
-          L.ql[e][at] = ql;
           L.kl[e][at] = kl;
           if constexpr (DELTA) {
             const float kb = k[i] * up[i];
             L.kb[e][at] = kb;
-            L.kk[b][at] = kb * pre;
+            kk[i] = kb * pre;
+            most += fabsf(kk[i]);
           }
         }
-        *reinterpret_cast<float4*>(&L.kd[b][ch * TS + 4 * grp]) = kd;
+        const bool odd = __builtin_amdgcn_ballot_w64(!(most < kSplitMost)) != 0ull;
+        if (lane == 0) L.odd[b][w] = odd;
+        auto put = [&](auto split) {
+          const Split2 p = split(kd[0], kd[1]), q = split(kd[2], kd[3]);
+          uint4* to = reinterpret_cast<uint4*>(&L.kd[b][ch * PS + 16 * grp]);
+          to[0] = make_uint4(p.h, q.h, p.m, q.m);
+          to[1] = make_uint4(p.h, q.h, p.l, q.l);
+          const int at = 4 * grp * PS + operand_at(ch);
+#pragma unroll
+          for (int i = 0; i < 4; i += 2) {
+            auto rows = [&](uint16_t (&part)[3][CT * PS], const Split2& x) {
+              const uint32_t f[3] = {x.h, x.m, x.l};
+#pragma unroll
+              for (int y = 0; y < 3; ++y) {
+                part[y][at + i * PS] = (uint16_t)f[y];
+                part[y][at + (i + 1) * PS] = (uint16_t)(f[y] >> 16);
+              }
+            };
+            if constexpr (!TURN) rows(L.qd[b], split(qd[i], qd[i + 1]));
+            if constexpr (DELTA) rows(L.kk[b], split(kk[i], kk[i + 1]));
+          }
+        };
+        if (odd) put([](float x, float y) { return odd_split(x, y); });
+        else put([](float x, float y) { return split3(x, y); });
       }
       __syncthreads();
     }
@@ -493,7 +766,7 @@ do {                                                                            
         const int b = c & 1;
         auto product = [&](auto far_c, auto rows_c) {     // rows: 0 q, 1 k, 2 both
           constexpr int far = far_c, rows = rows_c;
-          const float* src = rows == 1 || (rows == 2 && col >= 8) ? L.kb[DELTA ? b : 0] : L.ql[b];
+          const float* src = TURN || rows == 1 || (rows == 2 && col >= 8) ? L.kb[DELTA ? b : 0] : L.ql[b];
           const int tr = rows == 2 ? 8 + (col & 7) : col;
           float4 q[4], k[4], g[4], g2[4];
 #pragma unroll
@@ -517,7 +790,7 @@ do {                                                                            
           x += y;
           const int tb = rows == 2 ? 2 + (grp & 1) : grp;  // this lane's block of rows, its column's block
           float* to = rows == 1 || (rows == 2 && grp >= 2) ? L.ak[DELTA ? b : 0] : L.aq[c & 3];
-          if (tb - (col >> 2) == far) {
+          if (tb - (col >> 2) == far && !(TURN && rows == 2 && grp < 2)) {
 #pragma unroll
             for (int r = 0; r < 4; ++r) to[(4 * tb + r) * TS + col] = x[r];
           }
@@ -526,10 +799,13 @@ do {                                                                            
         constexpr std::integral_constant<int, 1> i1{};
         constexpr std::integral_constant<int, 2> i2{};
         constexpr std::integral_constant<int, 3> i3{};
-        if constexpr (DELTA) {
+        if constexpr (TURN) {                             // pairs of keys alone
+          if (w == 1) { product(i1, i1); product(i3, i2); }
+          else if (w == 2) product(i2, i2);
+        } else if constexpr (DELTA) {
           if (w == 0) product(i1, i0);
-          else if (w == 1) product(i1, i1);
-          else if (w == 2) { product(i2, i2); product(i3, i2); }
+          else if (w == 1) { product(i1, i1); product(i3, i2); }
+          else if (w == 2) product(i2, i2);
         } else {
           if (w == 0) product(i1, i0);
           else if (w == 1) product(i2, i0);
@@ -541,7 +817,7 @@ do {                                                                            
 #pragma unroll
           for (int i = 0; i < 4; ++i) {
             const int at = (4 * grp + i) * RS + 4 * col;
-            q[i] = ld4(&L.q[b][at]);
+            if constexpr (!TURN) q[i] = ld4(&L.q[b][at]);
             k[i] = ld4(&L.k[b][at]);
             d[i] = ld4(&L.a[b][at]);
           }
@@ -559,14 +835,16 @@ do {                                                                            
           } else {
             const float4 e10 = mul4(d[1], k[0]), e21 = mul4(d[2], k[1]), e32 = mul4(d[3], k[2]);
             const float4 e20 = mul4(d[2], e10), e31 = mul4(d[3], e21), e30 = mul4(d[3], e20);
-            acc[1] = dot4(q[1], e10);
-            acc[3] = dot4(q[2], e20);
-            acc[4] = dot4(q[2], e21);
-            acc[6] = dot4(q[3], e30);
-            acc[7] = dot4(q[3], e31);
-            acc[8] = dot4(q[3], e32);
+            if constexpr (!TURN) {
+              acc[1] = dot4(q[1], e10);
+              acc[3] = dot4(q[2], e20);
+              acc[4] = dot4(q[2], e21);
+              acc[6] = dot4(q[3], e30);
+              acc[7] = dot4(q[3], e31);
+              acc[8] = dot4(q[3], e32);
 #pragma unroll
-            for (int i = 0; i < 4; ++i) acc[i * (i + 3) / 2] = dot4(q[i], k[i]);
+              for (int i = 0; i < 4; ++i) acc[i * (i + 3) / 2] = dot4(q[i], k[i]);
+            }
             if constexpr (DELTA) {
               ack[0] = dot4(k[1], e10);
               ack[1] = dot4(k[2], e20);
@@ -576,15 +854,17 @@ do {                                                                            
               ack[5] = dot4(k[3], e32);
             }
           }
-          float* ao = &L.aq[c & 3][4 * grp * TS + 4 * grp];
+          if constexpr (!TURN) {
+            float* ao = &L.aq[c & 3][4 * grp * TS + 4 * grp];
 #pragma unroll
-          for (int i = 0; i < 10; ++i) acc[i] = ror_add(acc[i]);
-          if (col == 0) {
-            ao[0] = acc[0];
-            *reinterpret_cast<float2*>(ao + TS) = make_float2(acc[1], acc[2]);
-            *reinterpret_cast<float2*>(ao + 2 * TS) = make_float2(acc[3], acc[4]);
-            ao[2 * TS + 2] = acc[5];
-            *reinterpret_cast<float4*>(ao + 3 * TS) = make_float4(acc[6], acc[7], acc[8], acc[9]);
+            for (int i = 0; i < 10; ++i) acc[i] = ror_add(acc[i]);
+            if (col == 0) {
+              ao[0] = acc[0];
+              *reinterpret_cast<float2*>(ao + TS) = make_float2(acc[1], acc[2]);
+              *reinterpret_cast<float2*>(ao + 2 * TS) = make_float2(acc[3], acc[4]);
+              ao[2 * TS + 2] = acc[5];
+              *reinterpret_cast<float4*>(ao + 3 * TS) = make_float4(acc[6], acc[7], acc[8], acc[9]);
+            }
           }
           if constexpr (DELTA) {
             float* ko4 = &L.ak[b][4 * grp * TS + 4 * grp];
@@ -626,15 +906,41 @@ do {                                                                            
     }
   }
 
-  if (role == 0 && code >= 0 && vlive && sg.last) {
+  if constexpr (DELTA) {
+    if (role == 0 && !sg.last) {                          // a segment: dim is NC and all channels are there
+      const DeltaSeg d = delta_seg(a, sg.slot, h);
+#pragma unroll
+      for (int j = 0; j < NV; ++j)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) d.left[(16 * i + 4 * grp + r) * vdim + vcol + 16 * j] = st[j][i][r];
+      if constexpr (TURN)
+        if (zv == 0) {
+          bool ok = true;
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+              d.turn[(16 * i + 4 * grp + r) * NC + 16 * w + col] = st[NV][i][r];
+              ok = ok && fabsf(st[NV][i][r]) <= kTurnMost;
+            }
+          const uint64_t all = __builtin_amdgcn_ballot_w64(ok);
+          if (lane == 0) d.wild[w] = all == ~0ull ? 0.f : 1.f;
+        }
+    }
+  }
+  if (role == 0 && code >= 0 && sg.last) {
     float* wr = a.state + (((int64_t)(1 - (code & 1)) * a.slots + (code >> 1)) * H + h) * hsz;
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+    for (int j = 0; j < NV; ++j)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int c = 16 * i + 4 * grp + r;
-        if (c < dim) wr[(int64_t)c * vdim + vcol] = st[i][r];
-      }
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int c = 16 * i + 4 * grp + r;
+          if (c < dim && vlive(j)) wr[(int64_t)c * vdim + vcol + 16 * j] = st[j][i][r];
+        }
   }
 }
 
@@ -680,7 +986,7 @@ __device__ __forceinline__ void arrived4(uint2 x, float* f) {
 // from the last chunk to the first, the keys times all decays behind them: nothing is rescaled, and the lane that makes
 // such a product (four tokens of two key channels) has it as the MFMA operand.  No LDS but to add the waves' parts up.
 constexpr int kSegKeys = 32;
-template <typename TI, int MODE, int kSegWaves>
+template <typename TI, int MODE, int NV, int kSegWaves>
 __global__ __launch_bounds__(64 * kSegWaves, 4) void chunk_segment_kernel(const ChunkArgs a) {
   constexpr bool WKV = MODE == kChunkWkv;
   typedef typename std::conditional<WKV, TI, float>::type TZ;
@@ -689,11 +995,11 @@ __global__ __launch_bounds__(64 * kSegWaves, 4) void chunk_segment_kernel(const 
   typedef typename std::conditional<sizeof(TZ) == 2, uint32_t, uint2>::type RZ;
   const int tid = threadIdx.x, lane = tid & 63, col = lane & 15, grp = lane >> 4;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const ChunkSegment sg = find_segment(a, blockIdx.z, lane);
+  const ChunkSegment sg = find_segment<MODE, NV, kAllSegments>(a, blockIdx.z, lane);
   if (sg.n == 0 || sg.last) return;
   __shared__ __attribute__((aligned(16))) float sums[kSegWaves / 2][kSegKeys * NC];
   const int h = blockIdx.x, z64 = (blockIdx.y >> 1) * 64, c0 = (blockIdx.y & 1) * kSegKeys, H = a.H, vdim = a.vdim, hq = h / a.rep;
-  const int rows = a.seg_rows / kSegWaves;
+  const int rows = sg.rows / kSegWaves;
   // the wave's last chunk; a lane's tokens by their offsets in bytes
   const int64_t at = sg.t0 + (w + 1) * rows - CT;
   const TI* kb = static_cast<const TI*>(a.k) + at * a.ks + (int64_t)hq * NC + c0;
@@ -768,7 +1074,7 @@ __global__ __launch_bounds__(64 * kSegWaves, 4) void chunk_segment_kernel(const 
     float f = decays[tid];
 #pragma unroll
     for (int u = 1; u < kSegWaves; ++u) f *= decays[u * kSegKeys + tid];
-    a.seg[(a.runs + a.T / a.seg_rows) * (int64_t)(H * NC) * vdim + ((int64_t)sg.slot * H + h) * NC + c0 + tid] = f;
+    a.seg[a.cap * (int64_t)(H * NC) * vdim + ((int64_t)sg.slot * H + h) * NC + c0 + tid] = f;
   }
   float4 f[2];                                               // of channels 8 grp ..
   f[0] = f[1] = make_float4(1.f, 1.f, 1.f, 1.f);
@@ -824,26 +1130,68 @@ __global__ __launch_bounds__(64 * kSegWaves, 4) void chunk_segment_kernel(const 
   }
 }
 
-// A workgroup per segment, head and 64 value channels, behind chunk_segment_kernel.
-template <typename TI, typename TG, int MODE>
+// A workgroup per segment, head and 64 NV value channels, behind chunk_segment_kernel.
+template <typename TI, typename TG, int MODE, int NV>
 __global__ __launch_bounds__(chunk_threads(MODE)) void chunk_recurrence_segments_kernel(const ChunkArgs a) {
-  const ChunkSegment sg = find_segment(a, blockIdx.z, threadIdx.x & 63);
-  if (sg.n > 0) chunk_run<TI, TG, MODE>(a, sg, blockIdx.x, blockIdx.y * 64, threadIdx.x);
+  const ChunkSegment sg = find_segment<MODE, NV, kAllSegments>(a, blockIdx.z, threadIdx.x & 63);
+  if (sg.n > 0) chunk_run<TI, TG, MODE, NV>(a, sg, blockIdx.x, blockIdx.y * 64 * NV, threadIdx.x);
+}
+
+// The delta rule's segments.  Before: a run's first segment to its end, read-outs and all, and of the others but a run's
+// last what their rows leave of a state of zeros and the 64 x 64 turn that they make of any, by the same chunks with 64
+// more columns.  After it the later segments, from the state that the turns carry to them.  A workgroup per segment,
+// head and 128 value channels: the producers' work, which 64 channels cost as much, is done half as often.
+// Two runs of 2,048 with 32 heads: 301 -> 89 + 95 us.  Error of the state against 64 bits as with whole runs (6.3e-8 to
+// 6.5e-8).  Unit keys and betas of at most 1 turn a state no larger.  Where an entry passes that (other keys, whose turns may
+// grow or overflow though the state does not), a run's second segment goes through to its end in sequence.
+template <typename TI, typename TG>
+__global__ __launch_bounds__(chunk_threads(kChunkDelta)) void chunk_delta_first_kernel(const ChunkArgs a) {
+  const ChunkSegment sg = find_segment<kChunkDelta, 2, kFirstSegments>(a, blockIdx.z, threadIdx.x & 63);
+  if (sg.n == 0) return;
+  if (sg.seg == 0) chunk_run<TI, TG, kChunkDelta, 2>(a, sg, blockIdx.x, blockIdx.y * 128, threadIdx.x);
+  else chunk_run<TI, TG, kChunkDelta, 2, true>(a, sg, blockIdx.x, blockIdx.y * 128, threadIdx.x);
+}
+template <typename TI, typename TG>
+__global__ __launch_bounds__(chunk_threads(kChunkDelta)) void chunk_delta_later_kernel(const ChunkArgs a) {
+  const int lane = threadIdx.x & 63, h = blockIdx.x;
+  ChunkSegment sg = find_segment<kChunkDelta, 2, kLaterSegments>(a, blockIdx.z, lane);
+  if (sg.n == 0) return;
+  const int rows = a.row_fwd[sg.run0] + 1, turns = (rows + sg.rows - 1) / sg.rows - 2;
+  const float* wild = delta_seg(a, sg.slot - sg.seg + 1, h).wild;        // of the run's second segment
+  uint64_t any = 0;
+  for (int x = lane; x < 4 * turns; x += 64) any |= wild[(int64_t)(x >> 2) * a.H * 4 + (x & 3)] != 0.f;
+  if (__builtin_amdgcn_ballot_w64(any != 0) != 0ull) {
+    if (sg.seg > 1) return;
+    sg.n = rows - sg.rows;
+    sg.last = true;
+  }
+  chunk_run<TI, TG, kChunkDelta, 2>(a, sg, h, blockIdx.y * 128, threadIdx.x);
 }
 
 // Workgroups, one to a CU at most, that share the runs of min_run rows or more, which every wave counts for
-// itself: one for every run that the step has room for costs 16 us where there is none (64 runs of 16, wkv).
+// itself: one for every run that the step has room for costs 16 us where there is none (64 runs of 16, wkv).  Where those
+// runs are more than one round, a workgroup takes 128 value channels at a time, 1.25 of the time for twice the work.
 template <typename TI, typename TG, int MODE>
 __global__ __launch_bounds__(chunk_threads(MODE)) void chunk_recurrence_share_kernel(const ChunkArgs a) {
-  const int lane = threadIdx.x & 63, cols = (a.vdim + 63) >> 6, per = a.H * cols;
+  const int lane = threadIdx.x & 63;
+  auto fits = [&](int base, int& r) {
+    r = base + lane < a.runs ? a.run_rows[base + lane] : -1;
+    return __builtin_amdgcn_ballot_w64(r >= 0 && a.row_back[r] == 0 && a.row_fwd[r] + 1 >= a.min_run);
+  };
+  int width = 64, r;
+  if constexpr (MODE != kChunkWkv)
+    if (a.vdim > 64) {
+      int all = 0;
+      for (int base = 0; base < a.runs; base += 64) all += __builtin_popcountll(fits(base, r));
+      if ((int64_t)all * a.H * ((a.vdim + 63) / 64) > gridDim.x) width = 128;
+    }
+  const int per = a.H * ((a.vdim + width - 1) / width);
 #pragma unroll 1
   for (int item = blockIdx.x;; item += gridDim.x) {
     int left = item / per, t0 = -1;
     const int part = item - left * per, z = part / a.H;
     for (int base = 0; base < a.runs; base += 64) {
-      const int r = base + lane < a.runs ? a.run_rows[base + lane] : -1;
-      const bool fits = r >= 0 && a.row_back[r] == 0 && a.row_fwd[r] + 1 >= a.min_run;
-      uint64_t m = __builtin_amdgcn_ballot_w64(fits);
+      uint64_t m = fits(base, r);
       const int c = __builtin_popcountll(m);
       if (left < c) {
         for (; left > 0; --left) m &= m - 1;
@@ -861,12 +1209,15 @@ __global__ __launch_bounds__(chunk_threads(MODE)) void chunk_recurrence_share_ke
     const_args* p = (const_args*)__builtin_amdgcn_kernarg_segment_ptr();
     int tid = threadIdx.x;
     asm volatile("" : "+v"(tid), "+s"(p));
-    chunk_run<TI, TG, MODE>(*(const ChunkArgs*)p, whole_run(*(const ChunkArgs*)p, t0), part - z * a.H, z * 64, tid);
+    if (MODE == kChunkWkv || width == 64)
+      chunk_run<TI, TG, MODE>(*(const ChunkArgs*)p, whole_run(*(const ChunkArgs*)p, t0), part - z * a.H, z * 64, tid);
+    else if constexpr (MODE != kChunkWkv)
+      chunk_run<TI, TG, MODE, 2>(*(const ChunkArgs*)p, whole_run(*(const ChunkArgs*)p, t0), part - z * a.H, z * 128, tid);
   }
 }
 
 // ------------------------------------------------------------------ launcher
-// A workgroup costs some 8 us before its first chunk is out and 1.6 - 2.3 us a chunk, one to a CU; the
+// A workgroup costs some 8 us before its first chunk is out and 1.6 - 2.3 us a chunk (now 1.45 - 2.1), one to a CU; the
 // token-by-token kernels some 6 us and 0.2 (64 runs) - 2.6 us a token, many to a CU.  Times below are of whole
 // steps, 32 heads of 64 x 128 (wkv: 64 of 64 x 64), chunks against tokens.
 // Two workgroups to a CU or fewer: everything in chunks from 8 rows a run on (one run of 8: gla 14 us against 25,
@@ -889,76 +1240,93 @@ int chunk_min_run(int mode, int T, const ChunkArgs& a) {
   return T - a.runs + 1 >= from ? from : kNever;          // no run can be longer than that
 }
 
-// Segments instead of whole runs where they leave fewer or shorter rounds of one workgroup a CU, by the times of
-// the kernels below (us): a workgroup's start and end and its chunks, as many rounds as workgroups ask for; the same of
-// chunk_segment_kernel, whose workgroups of eight waves stand two to a CU.  Runs are taken as equally long, the
-// case that gains least.  Two runs of 2,048 tokens in bf16, whole -> in segments: wkv, 64 heads 204 -> 145 us, 32
-// heads 194 -> 89; gla, 16 heads of 128 218 -> 112; one run of 2,048, 64 heads, 190 -> 81.  The delta rule's decays are
-// matrices: its runs stay whole.
-int chunk_seg_rows(int mode, bool in_f32, int T, const ChunkArgs& a) {
-  if (mode == kChunkDelta || chunk_min_run(mode, T, a) != 1 || a.dim != NC || a.vdim % 64 != 0) return 0;
-  const uintptr_t wide = in_f32 ? 16 : 8, zwide = mode == kChunkWkv && !in_f32 ? 4 : 8;     // loads of four, of two
-  for (const void* p : {a.k, a.v})
-    if (reinterpret_cast<uintptr_t>(p) % wide != 0) return 0;
-  if (reinterpret_cast<uintptr_t>(a.z) % zwide != 0) return 0;
-  for (int64_t st : {a.ks, a.vs, a.zs})
-    if (st % 4 != 0) return 0;
-  const int64_t per = (int64_t)a.H * (a.vdim / 64);
-  const int c = (T + CT * a.runs - 1) / (CT * a.runs);    // chunks of a run
-  const double turn = mode == kChunkWkv ? 1.65 : 1.85;
-  auto rounds = [](int64_t wgs, int at_once) { return (double)((wgs + at_once - 1) / at_once); };
-  double best = 0.9 * rounds(a.runs * per, 256) * (6 + turn * c) - 5;
-  int rows = 0;
-  for (int s = 2; s <= 16; ++s) {
-    int cs = ((c + s - 1) / s + 7) / 8 * 8;               // chunks of a segment
-    if (cs >= 64) cs = (cs + 15) / 16 * 16;
-    const int64_t n = (c + cs - 1) / cs, w1 = a.runs * (n - 1) * per * (NC / kSegKeys);
-    const double t = 6 + (cs >= 64 ? rounds(w1, 256) * (8 + 3.3 * cs / 16) : rounds(w1, 512) * (6 + 2.0 * cs / 8)) +
-                     rounds(a.runs * n * per, 256) * (6 + turn * cs);
-    if (n > 1 && t < best) {
-      best = t;
-      rows = cs * CT;
-    }
+// Segments instead of whole runs, which the kernels place where that is faster (segment_rows; only they know the runs):
+// from steps on whose runs, taken as equally long, gain a tenth by it by the same times (a first kernel that finds nothing
+// to cut costs 5 - 10 us: gla, 16 heads, 8 runs of 128, 32 us for 45), and in all steps whose whole runs are more than
+// one round of workgroups of 64 value channels, for workgroups of 128 are no more than one then (gla, 32 heads, 8 runs of
+// 512: 156 -> 110).  Room is for as many segments as the chip has CUs; for twice the runs where these fill it alone, from 40
+// chunks a run on.  183 steps of 72 to 4,096 tokens, 16 to 64 heads, against whole runs of 64 channels in fp32 products:
+// 1.34 times as fast on the average, 5.8 at the most, six of them (72 or 128 tokens a run) 1 - 2 % slower.
+int chunk_seg_cap(int mode, bool in_f32, int T, ChunkArgs& a) {
+  if (chunk_min_run(mode, T, a) != 1 || a.dim != NC || a.runs > 64) return 0;
+  const int wide = a.vdim % 128 == 0 ? 2 : 1;             // 64 value channels to a workgroup
+  if (mode == kChunkDelta) {
+    if (wide == 1) return 0;
+  } else {
+    if (a.vdim % 64 != 0) return 0;
+    const uintptr_t v4 = in_f32 ? 16 : 8, z2 = mode == kChunkWkv && !in_f32 ? 4 : 8;     // loads of four, of two
+    for (const void* p : {a.k, a.v})
+      if (reinterpret_cast<uintptr_t>(p) % v4 != 0) return 0;
+    if (reinterpret_cast<uintptr_t>(a.z) % z2 != 0) return 0;
+    for (int64_t st : {a.ks, a.vs, a.zs})
+      if (st % 4 != 0) return 0;
   }
-  return rows;
+  const int64_t narrow = (int64_t)a.H * (a.vdim / 64);
+  a.per = (int)(narrow / wide);
+  const int room = std::max(256 / a.per, a.runs), parts = room / a.runs;
+  // sixteen waves to a segment of chunk_segment_kernel where it is that long, else eight
+  a.unit = mode == kChunkDelta ? CT : CT * (T / std::min(room, 2 * a.runs) >= 64 * CT && T / room >= 48 * CT ? 16 : 8);
+  const double c = (double)T / (CT * a.runs);             // chunks of a run
+  if (room == a.runs) return wide == 1 ? 0 : c >= 40 ? 2 * room : a.runs * narrow > 256 ? room : 0;
+  if (a.runs * narrow <= 256) {
+    const double turn = mode == kChunkDelta ? 2.1 : mode == kChunkWkv ? 1.45 : 1.65;
+    double cut = 1e9;
+    for (int n = 2; n <= std::min(parts + (mode == kChunkDelta), 64); ++n)
+      cut = std::min(cut, mode == kChunkDelta ? 20 + 5.5 * std::ceil(c / n) + 3 * (n - 2)
+                                              : 18 + (0.25 + (wide == 1 ? turn : 2.)) * std::max(std::ceil(c / n), 8.) + 0.8 * n);
+    if (cut > 0.9 * (6 + turn * c)) return 0;
+  }
+  return room;
 }
-int64_t chunk_seg_floats(int T, const ChunkArgs& a) {
-  return (a.runs + (int64_t)T / a.seg_rows) * a.H * a.dim * (a.vdim + 1);
+int64_t chunk_seg_floats(int mode, const ChunkArgs& a) {
+  return (int64_t)a.cap * a.H * (mode == kChunkDelta ? NC * a.vdim + NC * NC + 4 : a.dim * (a.vdim + 1));
+}
+
+// Dynamic LDS above 64 KB has to be allowed per kernel, once.
+template <auto kernel>
+static void allow_lds() {
+  static bool done = false;
+  if (!done) (void)hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+  done = true;
+}
+
+template <typename TI, typename TG, int MODE, int NV>
+static void launch_chunk_segments(const ChunkArgs& a, hipStream_t s) {
+  constexpr int lds = sizeof(ChunkLds<MODE>);
+  const dim3 grid(a.H, a.vdim / (64 * NV), a.cap), wg(chunk_threads(MODE));
+  if constexpr (MODE == kChunkDelta) {
+    allow_lds<&chunk_delta_first_kernel<TI, TG>>();
+    allow_lds<&chunk_delta_later_kernel<TI, TG>>();
+    hipLaunchKernelGGL((chunk_delta_first_kernel<TI, TG>), grid, wg, lds, s, a);
+    if (a.cap > a.runs) hipLaunchKernelGGL((chunk_delta_later_kernel<TI, TG>), grid, wg, lds, s, a);
+  } else {
+    allow_lds<&chunk_recurrence_segments_kernel<TI, TG, MODE, NV>>();
+    const dim3 parts(a.H, a.vdim / 64 * (NC / kSegKeys), a.cap);
+    if (a.cap > a.runs && a.unit > 8 * CT) hipLaunchKernelGGL((chunk_segment_kernel<TI, MODE, NV, 16>), parts, dim3(1024), 0, s, a);
+    else if (a.cap > a.runs) hipLaunchKernelGGL((chunk_segment_kernel<TI, MODE, NV, 8>), parts, dim3(512), 0, s, a);
+    hipLaunchKernelGGL((chunk_recurrence_segments_kernel<TI, TG, MODE, NV>), grid, wg, lds, s, a);
+  }
 }
 
 template <typename TI, typename TG, int MODE>
 static void launch_chunk_one(int T, const ChunkArgs& a, hipStream_t s) {
-  static bool attr = false;
-  if (!attr) {          // dynamic LDS above 64 KB has to be allowed per kernel, once
-    for (auto* k : {&chunk_recurrence_kernel<TI, TG, MODE>, &chunk_recurrence_share_kernel<TI, TG, MODE>})
-      (void)hipFuncSetAttribute(reinterpret_cast<const void*>(k), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
-    attr = true;
-  }
-  static_assert(sizeof(ChunkLds<MODE>) <= 160 * 1024, "LDS of a CU");
+  constexpr int lds = sizeof(ChunkLds<MODE>);
+  static_assert(lds <= 160 * 1024, "LDS of a CU");
   const int cols = (a.vdim + 63) / 64;
-  if constexpr (MODE != kChunkDelta)
-    if (a.seg != nullptr) {
-      static bool seg_attr = false;
-      if (!seg_attr) {
-        (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&chunk_recurrence_segments_kernel<TI, TG, MODE>),
-                                  hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
-        seg_attr = true;
-      }
-      const dim3 grid(a.H, cols, a.runs + T / a.seg_rows);
-      const dim3 parts(a.H, cols * (NC / kSegKeys), grid.z);
-      if (a.seg_rows >= 64 * CT) hipLaunchKernelGGL((chunk_segment_kernel<TI, MODE, 16>), parts, dim3(1024), 0, s, a);
-      else hipLaunchKernelGGL((chunk_segment_kernel<TI, MODE, 8>), parts, dim3(512), 0, s, a);
-      hipLaunchKernelGGL((chunk_recurrence_segments_kernel<TI, TG, MODE>), grid, dim3(chunk_threads(MODE)),
-                         sizeof(ChunkLds<MODE>), s, a);
-      return;
-    }
-  if (a.min_run <= 1)
-    hipLaunchKernelGGL((chunk_recurrence_kernel<TI, TG, MODE>), dim3(a.runs, a.H, cols), dim3(chunk_threads(MODE)),
-                       sizeof(ChunkLds<MODE>), s, a);
-  else                        // no more long runs than rows allow
+  const dim3 wg(chunk_threads(MODE));
+  if (a.seg != nullptr) {
+    if constexpr (MODE != kChunkWkv)
+      if (a.vdim % 128 == 0) return launch_chunk_segments<TI, TG, MODE, 2>(a, s);
+    if constexpr (MODE != kChunkDelta) launch_chunk_segments<TI, TG, MODE, 1>(a, s);
+  } else if (a.min_run <= 1) {
+    allow_lds<&chunk_recurrence_kernel<TI, TG, MODE>>();
+    hipLaunchKernelGGL((chunk_recurrence_kernel<TI, TG, MODE>), dim3(a.runs, a.H, cols), wg, lds, s, a);
+  } else {                    // no more long runs than rows allow
+    allow_lds<&chunk_recurrence_share_kernel<TI, TG, MODE>>();
     hipLaunchKernelGGL((chunk_recurrence_share_kernel<TI, TG, MODE>),
-                       dim3((unsigned)std::min<int64_t>((int64_t)std::min(a.runs, T / a.min_run) * a.H * cols, 256)),
-                       dim3(chunk_threads(MODE)), sizeof(ChunkLds<MODE>), s, a);
+                       dim3((unsigned)std::min<int64_t>((int64_t)std::min(a.runs, T / a.min_run) * a.H * cols, 256)), wg,
+                       lds, s, a);
+  }
 }
 
 void launch_chunk(int mode, bool in_f32, bool act_f32, int T, const ChunkArgs& a, hipStream_t s) {

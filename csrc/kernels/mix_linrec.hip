@@ -507,7 +507,7 @@ void launch_gated_linrec(bool in_f32, bool act_f32, bool delta, const LinrecArgs
     c.slots = a.slots; c.T = a.T;
     const int mode = delta ? kChunkDelta : kChunkGla;
     a.below = c.min_run = chunk_min_run(mode, a.T, c);
-    if ((c.seg_rows = chunk_seg_rows(mode, in_f32, a.T, c)) > 0) c.seg = scratch(chunk_seg_floats(a.T, c));
+    if ((c.cap = chunk_seg_cap(mode, in_f32, a.T, c)) > 0) c.seg = scratch(chunk_seg_floats(mode, c));
     if (c.min_run < INT32_MAX) launch_chunk(mode, in_f32, act_f32, a.T, c, s);
     // Below them: the scan's fixed cost is the larger one (64 decode rows, gla: 41 us against 72),
     // its tokens are the cheaper ones where each has two sums (delta, 64 runs of 8: 106 us against

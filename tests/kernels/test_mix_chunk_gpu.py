@@ -34,12 +34,14 @@ def _close(got, want, tol):
     assert float((got[ok] - want[ok]).square().mean().sqrt()) <= tol * float(scale)
 
 
-def _linrec(mode, H, Hq, dim, vdim, dtype, shift, lens=LENS, spoil=None, pad=3):
+def _linrec(mode, H, Hq, dim, vdim, dtype, shift, lens=LENS, spoil=None, pad=3, keys=None):
     g = torch.Generator().manual_seed(H * 1000 + dim + vdim)
     T = sum(lens)
     wide = torch.randn(T, 2 * Hq * dim + H * vdim + pad, generator=g)              # columns of wider rows
     qk = wide[:, :2 * Hq * dim].unflatten(1, (2 * Hq, dim))
     qk /= qk.square().sum(-1, keepdim=True).sqrt() / (2.0 if mode == "gla" else 1.0)   # unit vectors: delta rule
+    if keys is not None:
+        keys(qk[:, Hq:], wide[:, 2 * Hq * dim:])
     if spoil is not None:
         wide[spoil[0], 2 * Hq * dim + spoil[1]] = float(spoil[2])
     wide = wide.to(dtype)
@@ -170,6 +172,53 @@ def test_a_non_finite_value_stays_out_of_earlier_segments():
     (out, _), (out_w, _) = _linrec("gla", 2, 2, 64, 64, torch.float32, 0.0, lens=SEGMENTS, spoil=(300, 3, float("inf")), pad=4)
     _close(out[:300], out_w[:300], 1e-5)
     _close(out[700:], out_w[700:], 1e-5)
+
+
+# The delta rule's segments are whole chunks, as many as the chip has room for: runs of several, of one, of less than one
+# and of a chunk, a single long one; states carried through turns of 64 x 64
+@pytest.mark.parametrize("shift", [-6.0, 0.0, 60.0])
+@pytest.mark.parametrize("H,Hq,vdim,lens", [(2, 2, 128, [1500, 33, 16, 700]), (4, 2, 128, [2100]), (1, 1, 256, [513, 1024])])
+def test_delta_rule_in_segments(H, Hq, vdim, lens, shift):
+    (out, st), (out_w, st_w) = _linrec("delta", H, Hq, 64, vdim, torch.float32, shift, lens=lens)
+    tol = 1e-5 * (max(lens) / 150) ** 0.5 if shift < 0 else 1e-5        # as for wkv above
+    _close(out, out_w, tol)
+    _close(st, st_w, tol)
+
+
+@pytest.mark.parametrize("size,row", [(3.0, 2100), (1e20, 1000)])
+def test_delta_rule_turns_that_grow(size, row):
+    """Keys that turn a state into a larger one, or a state of zeros into what no fp32 holds, leave segments to be done in
+    sequence.  Few keys are not zero, so that the growth is not undone; the large one meets a channel that holds nothing."""
+    def keys(k, v):
+        keep = torch.zeros(len(k), dtype=torch.bool)
+        keep[::97] = True
+        k[~keep] = 0.0
+        k[:1500, :, 0] = 0.0
+        k[row], v[row] = 0.0, 0.0
+        k[row, :, 0] = size
+
+    (out, st), (out_w, st_w) = _linrec("delta", 2, 2, 64, 128, torch.float32, -9.0, lens=[1500, 900], keys=keys)
+    # a norm of size^2 on a difference: 9 times the roundings of the state it reads
+    _close(out, out_w, 1e-4)
+    _close(st, st_w, 1e-4)
+
+
+@pytest.mark.parametrize("mode", ["gla", "delta"])
+def test_many_long_runs_share_workgroups_of_128_channels(mode):
+    (out, st), (out_w, st_w) = _linrec(mode, 8, 4, 64, 192, torch.float32, 0.0, lens=[81 + i % 7 for i in range(24)] + [3, 16])
+    _close(out, out_w, 1e-5)
+    _close(st, st_w, 1e-5)
+
+
+@pytest.mark.parametrize("value", [3.395e38, 1e-37])         # a part of three would round to infinity; parts below 2^-126
+@pytest.mark.parametrize("mode", ["gla", "delta"])
+def test_states_at_the_ends_of_fp32(mode, value):
+    first = sum(LENS[:7])
+    (_, st), (_, st_w) = _linrec(mode, 2, 2, 64, 64, torch.float32, 0.0, spoil=(first + 9, 3, value))
+    assert torch.equal(torch.isfinite(st.cpu()), torch.isfinite(st_w))
+    for i in range(len(LENS)):                               # every run against its own size
+        if i != 7 or value < 1:
+            _close(st[i::len(LENS)], st_w[i::len(LENS)], 1e-5)
 
 
 # 40 rows: chunks; 6: token by token; 200 without a list of runs: the scan
