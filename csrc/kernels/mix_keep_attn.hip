@@ -374,6 +374,233 @@ __global__ __launch_bounds__(1024) void qk_norm_rotary_append_kernel(
   }
 }
 
+// The same for steps of many rows whose norms are of whole projections: a workgroup takes several neighbouring rows one
+// after another.  A thread has two chunks of eight columns for all of them and keeps these columns' weights (of the
+// convolution, the norms, the bias) and the rows above in registers; with a workgroup a row every row read 100 KB of
+// weights and three rows from the L2s for its own 12, which bounded it.  Two rows on are on their way while one is made;
+// they are waited for before a row's stores, which are counted with the loads and in order.
+struct QknRows {
+  const void* proj;
+  int64_t stride;
+  const float *bias, *q_norm_w, *k_norm_w;
+  float eps;
+  const int32_t* pos;
+  const float* inv_freq;
+  int nrot;
+  float rot_mult;
+  int q_rot_off, k_rot_off;
+  const int32_t* slots;
+  void *k_cache, *v_cache;
+  int T, H, G, qw, kw, vdim, BS;
+  int64_t pool_slots;
+  float* q_out;
+  int64_t q_ts, q_hs;
+  const float* conv_w;                  // [4][W], or none
+  float* conv_state;
+  int state_slots;
+  const int32_t *row_state, *row_back, *row_fwd;
+  int rows;                             // of a workgroup
+};
+constexpr int kQknThreads = 640, kQknTaps = 4, kQknRows = 16;
+template <typename T, bool CONV, int N>
+__global__ __launch_bounds__(N == 1 ? 1024 : kQknThreads) void qk_norm_rotary_append_rows_kernel(const QknRows a) {
+  constexpr int K = kQknTaps - 1;
+  constexpr bool DEEP = !CONV || N == 1;                            // two rows on the way, else one: registers
+  extern __shared__ __attribute__((aligned(16))) float lds[];
+  const int tid = threadIdx.x, nthr = blockDim.x, lane = tid & 63, wid = tid >> 6, nw = nthr >> 6;
+  const int t0 = blockIdx.x * a.rows, n = min(a.rows, a.T - t0);
+  const int nq = a.H * a.qw, nk = a.G * a.kw, W = nq + nk + a.G * a.vdim;
+  float* cs = lds;                                        // (cos, sin) of every row
+  float* sums = cs + 2 * a.nrot * a.rows;                 // [2][q, k][wave]
+  int32_t* meta = reinterpret_cast<int32_t*>(sums + 4 * nw);     // [rows][slot, back, fwd, state, position]
+  if (tid < n) {
+    const int t = t0 + tid;
+    meta[5 * tid] = a.slots[t];
+    meta[5 * tid + 1] = CONV ? a.row_back[t] : 0;
+    meta[5 * tid + 2] = CONV ? a.row_fwd[t] : 0;
+    meta[5 * tid + 3] = CONV ? a.row_state[t] : -1;
+    meta[5 * tid + 4] = a.pos[t];
+  }
+  const T* proj = static_cast<const T*>(a.proj);
+  int col[N];                                             // chunks past the row are read as its last one
+  bool live[N];
+#pragma unroll
+  for (int j = 0; j < N; ++j) {
+    col[j] = (tid + j * nthr) * 8;
+    live[j] = col[j] < W;
+    if (!live[j]) col[j] = W - 8;
+  }
+  Bits<8> raw[N], next[DEEP ? N : 1], above[CONV ? K : 1][N];
+  auto fetch = [&](auto& to, int r) {
+    const T* src = proj + (int64_t)(t0 + min(max(r, -t0), n - 1)) * a.stride;
+#pragma unroll
+    for (int j = 0; j < N; ++j) to[j].load(src + col[j]);
+  };
+  fetch(raw, 0);
+  if constexpr (DEEP) fetch(next, 1);
+  float taps[CONV ? kQknTaps : 1][N][8], bias[CONV ? 1 : N][8], norm[N][8];
+  if constexpr (CONV) {
+#pragma unroll
+    for (int d = 0; d < K; ++d) fetch(above[d], -1 - d);
+#pragma unroll
+    for (int d = 0; d < kQknTaps; ++d)
+#pragma unroll
+      for (int j = 0; j < N; ++j) ld_chunk<8>(a.conv_w + (int64_t)d * W + col[j], taps[d][j]);
+  }
+  // a chunk's place: 0 q, 1 k, 2 v; its head and the entry in it; the rotation of its head
+  int kind[N], head[N], entry[N], turn[N];                // turn: (cos, sin) pairs by which it turns, or -1
+  bool first[N];                                          // of the rotation's two halves
+#pragma unroll
+  for (int j = 0; j < N; ++j) {
+    kind[j] = col[j] < nq ? 0 : col[j] < nq + nk ? 1 : 2;
+    const int y = col[j] - (kind[j] == 0 ? 0 : kind[j] == 1 ? nq : nq + nk), w = kind[j] == 0 ? a.qw : kind[j] == 1 ? a.kw : a.vdim;
+    head[j] = y / w;
+    entry[j] = y - head[j] * w;
+    const int r0 = entry[j] - (kind[j] == 0 ? a.q_rot_off : a.k_rot_off);
+    first[j] = r0 < a.nrot;
+    turn[j] = kind[j] < 2 && r0 >= 0 && r0 < 2 * a.nrot ? (first[j] ? r0 : r0 - a.nrot) : -1;
+    const float* wn = kind[j] == 0 ? a.q_norm_w : kind[j] == 1 ? a.k_norm_w : nullptr;
+    if (wn != nullptr) ld_chunk<8>(wn + y, norm[j]);
+    else
+#pragma unroll
+      for (int i = 0; i < 8; ++i) norm[j][i] = 1.f;
+    if constexpr (!CONV)
+      if (a.bias != nullptr) ld_chunk<8>(a.bias + col[j], bias[j]);
+  }
+  __syncthreads();
+  for (int x = tid; x < n * a.nrot; x += nthr) {
+    const int r = x / a.nrot, i = x - r * a.nrot;
+    float sn, c;
+    sincosf((float)meta[5 * r + 4] * a.inv_freq[i], &sn, &c);
+    cs[2 * x] = c * a.rot_mult;
+    cs[2 * x + 1] = sn * a.rot_mult;
+  }
+  for (int r = 0; r < n; ++r) {
+    const int slot = __builtin_amdgcn_readfirstlane(meta[5 * r]);
+    float f[N][8];
+#pragma unroll
+    for (int j = 0; j < N; ++j) raw[j].template get<T>(f[j]);
+    if constexpr (CONV) {
+      const int back = __builtin_amdgcn_readfirstlane(meta[5 * r + 1]), fwd = __builtin_amdgcn_readfirstlane(meta[5 * r + 2]);
+      const int code = __builtin_amdgcn_readfirstlane(meta[5 * r + 3]), pt = __builtin_amdgcn_readfirstlane(meta[5 * r + 4]);
+      if (fwd < K && code >= 0) {                         // the run's last rows go to the other half
+        const float* rd = a.conv_state + ((int64_t)((code & 1) * a.state_slots + (code >> 1)) * K) * W;
+        float* wr = a.conv_state + ((int64_t)((1 - (code & 1)) * a.state_slots + (code >> 1)) * K) * W;
+#pragma unroll
+        for (int j = 0; j < N; ++j)
+          if (live[j]) {
+            st_chunk<8>(wr + (int64_t)(K - 1 - fwd) * W + col[j], f[j]);
+            if (back == 0)                                // a run shorter than the taps: older inputs move up
+              for (int e = 0; e < K - (fwd + 1); ++e) {
+                float u[8];
+                ld_chunk<8>(rd + (int64_t)(e + fwd + 1) * W + col[j], u);
+                st_chunk<8>(wr + (int64_t)e * W + col[j], u);
+              }
+          }
+      }
+#pragma unroll
+      for (int j = 0; j < N; ++j)
+#pragma unroll
+        for (int i = 0; i < 8; ++i) f[j][i] *= taps[K][j][i];
+      if (back >= K) {
+#pragma unroll
+        for (int d = 0; d < K; ++d)
+#pragma unroll
+          for (int j = 0; j < N; ++j) {
+            float u[8];
+            above[d][j].template get<T>(u);
+#pragma unroll
+            for (int i = 0; i < 8; ++i) f[j][i] += taps[K - 1 - d][j][i] * u[i];
+          }
+      } else {
+#pragma unroll
+        for (int d = 0; d < K; ++d) {
+          const bool own = d < back;
+          if (!own && (pt - d - 1 < 0 || code < 0)) break;
+          const float* rd = a.conv_state + ((int64_t)((code & 1) * a.state_slots + (code >> 1)) * K + (K + back - d - 1)) * W;
+#pragma unroll
+          for (int j = 0; j < N; ++j) {
+            float u[8];
+            if (own) above[d][j].template get<T>(u);
+            else ld_chunk<8>(rd + col[j], u);
+#pragma unroll
+            for (int i = 0; i < 8; ++i) f[j][i] += taps[K - 1 - d][j][i] * u[i];
+          }
+        }
+      }
+#pragma unroll
+      for (int j = 0; j < N; ++j) {
+#pragma unroll
+        for (int d = K - 1; d > 0; --d) above[d][j] = above[d - 1][j];
+        above[0][j] = raw[j];
+      }
+    }
+    if constexpr (DEEP) {
+#pragma unroll
+      for (int j = 0; j < N; ++j) raw[j] = next[j];
+      fetch(next, r + 2);
+    } else {
+      fetch(raw, r + 1);
+    }
+    float sq = 0.f, sk = 0.f;
+#pragma unroll
+    for (int j = 0; j < N; ++j) {
+      if constexpr (!CONV)
+        if (a.bias != nullptr) {
+#pragma unroll
+          for (int i = 0; i < 8; ++i) f[j][i] += bias[j][i];
+        }
+      float ss = 0.f;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) ss += f[j][i] * f[j][i];
+      sq += live[j] && kind[j] == 0 ? ss : 0.f;
+      sk += live[j] && kind[j] == 1 ? ss : 0.f;
+    }
+    float* sum = sums + (r & 1) * 2 * nw;
+    sq = group_sum(sq, 64);
+    sk = group_sum(sk, 64);
+    if (lane == 0) {
+      sum[wid] = sq;
+      sum[nw + wid] = sk;
+    }
+    __syncthreads();                                      // the first: the sines too
+    const int part = lane & 15;
+    const float qs = group_sum(part < nw ? sum[part] : 0.f, 16), ks = group_sum(part < nw ? sum[nw + part] : 0.f, 16);
+    const float fq = a.q_norm_w != nullptr ? 1.0f / sqrtf(qs / (float)nq + a.eps) : 1.f;
+    const float fk = a.k_norm_w != nullptr ? 1.0f / sqrtf(ks / (float)nk + a.eps) : 1.f;
+#pragma unroll
+    for (int j = 0; j < N; ++j) {
+      const float fc = kind[j] == 0 ? fq : kind[j] == 1 ? fk : 1.f;
+#pragma unroll
+      for (int i = 0; i < 8; i += 2) {
+        f[j][i] *= fc * norm[j][i];
+        f[j][i + 1] *= fc * norm[j][i + 1];
+        const float u0 = __shfl_xor(f[j][i], a.nrot >> 3, 64), u1 = __shfl_xor(f[j][i + 1], a.nrot >> 3, 64);   // the partner's
+        if (turn[j] >= 0) {
+          const float4 c = ld4(cs + 2 * (r * a.nrot + turn[j] + i));
+          f[j][i] = first[j] ? f[j][i] * c.x - u0 * c.y : f[j][i] * c.x + u0 * c.y;
+          f[j][i + 1] = first[j] ? f[j][i + 1] * c.z - u1 * c.w : f[j][i + 1] * c.z + u1 * c.w;
+        }
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < N; ++j)
+#pragma unroll
+      for (int i = 0; i < (sizeof(T) == 4 ? 8 : 4); ++i) asm volatile("" : "+v"(raw[j].u[i]));
+    const bool keep = slot >= 0 && slot < a.pool_slots;
+    const int64_t page_row = keep ? ((int64_t)(slot / a.BS) * a.G) * a.BS + slot % a.BS : 0;   // + g * BS
+#pragma unroll
+    for (int j = 0; j < N; ++j)
+      if (live[j]) {
+        if (kind[j] == 0) st_chunk<8>(a.q_out + (t0 + r) * a.q_ts + head[j] * a.q_hs + entry[j], f[j]);
+        else if (keep) {
+          T* cache = static_cast<T*>(kind[j] == 1 ? a.k_cache : a.v_cache);
+          st_chunk<8>(cache + (page_row + (int64_t)head[j] * a.BS) * (kind[j] == 1 ? a.kw : a.vdim) + entry[j], f[j]);
+        }
+      }
+  }
+}
+
 // ------------------------------------------------------------------ prompt rows
 // Work item (work_seq[w], work_qblk[w]) x head.  Thread (ti, tj) of the 16 x 16 grid owns score
 // rows ti, ti + 16 and columns tj + 16 k of a 64-key tile; queries and keys pass through LDS in
@@ -784,6 +1011,40 @@ bool launch_qk_norm_rotary_append(bool f32, const void* proj, int64_t stride, co
                    al16(k_norm_w) && al16(k_cache) && al16(v_cache) && al16(q_out) && al16(v_in) &&
                    al16(v_out) && al16(conv_w) && al16(conv_state) && q_ts % 8 == 0 && q_hs % 8 == 0 &&
                    q_from % 8 == 0;
+  // A partner of the rotation lies as many lanes away as chunks: nrot / 8, a power of two, and heads and rotations begin at
+  // multiples of both halves.
+  const int turn = 2 * nrot;
+  const bool lanes = nrot == 0 || (turn <= 512 && (nrot & (nrot - 1)) == 0 && q_rot_off % turn == 0 && k_rot_off % turn == 0 &&
+                                   qw % turn == 0 && kw % turn == 0);
+  // Two chunks a thread, one where a thread keeps the convolution's weights for it (two spill 30 registers).  Of rows beyond
+  // 8,192 columns, convolved, few are faster in the other kernel (80 heads of 128: 257 rows 15.0 us for 16.5, 1,024 34.2
+  // for 31.2); all others gain at every size.  32 + 8 + 8 heads of 128 in bf16: convolved 1 row 8.1 -> 7.3 us, 64 rows 9.3
+  // -> 7.9, 512 12.6 -> 9.5, 2,648 40.5 -> 29.3 (3.0 TB/s), 8,192 103 -> 85; with a bias 2,648 rows 28.7 -> 21.5.
+  const int per = conv_w != nullptr && W <= 8 * 1024 ? 1 : 2;
+  const int wide = (int)((W / 8 + per - 1) / per + 63) / 64 * 64;
+  if (vec && lanes && norm_all && G > 0 && v_mode == 0 && v_in == nullptr && v_out == nullptr && q_from == 0 && !neighbours &&
+      (conv_w == nullptr || (taps == kQknTaps && bias == nullptr)) && wide <= (per == 1 ? 1024 : kQknThreads) &&
+      (conv_w == nullptr || per == 1 || T >= 1024)) {
+    QknRows a{proj, stride, bias, q_norm_w, k_norm_w, eps, pos, inv_freq, nrot, rot_mult, q_rot_off, k_rot_off, slots, k_cache,
+              v_cache, T, H, G, qw, kw, vdim, BS, pool_slots, q_out, q_ts, q_hs, conv_w, conv_state, state_slots, row_state,
+              row_back, row_fwd, 0};
+    const int at_once = 256 * std::max(1, 12 * 64 / wide);
+    a.rows = std::min(kQknRows, (T + at_once - 1) / at_once);
+    const size_t bytes = (size_t)(2 * nrot * a.rows + 4 * (wide / 64) + 5 * a.rows) * 4;
+    const dim3 grid((T + a.rows - 1) / a.rows);
+#define QKN_ROWS(TT, C, N) hipLaunchKernelGGL((qk_norm_rotary_append_rows_kernel<TT, C, N>), grid, dim3(wide), bytes, s, a)
+    if (f32) {
+      if (conv_w == nullptr) QKN_ROWS(float, false, 2);
+      else if (per == 1) QKN_ROWS(float, true, 1);
+      else QKN_ROWS(float, true, 2);
+    } else {
+      if (conv_w == nullptr) QKN_ROWS(bf16_t, false, 2);
+      else if (per == 1) QKN_ROWS(bf16_t, true, 1);
+      else QKN_ROWS(bf16_t, true, 2);
+    }
+#undef QKN_ROWS
+    return true;
+  }
   // Up to a row per CU its chain of loads is what counts: a chunk per thread, a wave for the sines
   // beside them (32 + 8 + 8 heads of 128, convolved: one row 10.7 -> 8.2 us, 64 rows 14.2 -> 11.4).
   // More rows share a CU and fill it from blocks of 256 (512 rows: a pass of 23.7 us against 24.8;

@@ -93,3 +93,36 @@ def test_norm_and_rotation_by_number_of_rows(taps, norm_all, H, G, dim, T):
     # of up to six products of at most 25
     for a, b in zip(got, want):
         torch.testing.assert_close(a.cpu(), b, atol=3e-5, rtol=1e-5)
+
+
+# Several rows a workgroup, two chunks a thread or one: rows that its groups do not divide, runs that begin and end inside
+# a group, rotated parts behind plain ones, rows of one wave's chunks and of ten, columns that no thread has alone
+@pytest.mark.parametrize("T", [1, 66, 1030, 2101])
+@pytest.mark.parametrize("H,G,dim,nrot,off", [(2, 1, 64, 16, 32), (20, 3, 64, 32, 0), (64, 8, 128, 32, 64), (5, 5, 40, 0, 0)])
+@pytest.mark.parametrize("conv", [False, True])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_norm_and_rotation_of_rows_one_after_another(dtype, conv, H, G, dim, nrot, off, T):
+    g = torch.Generator().manual_seed(T + H)
+    W, lens, page = (H + 2 * G) * dim, _lens(T) if T > 45 else [T], 32
+    wide, state = torch.randn(T, W + 8, generator=g).to(dtype), torch.randn(2 * len(lens), 3, W, generator=g)
+    qn, kn, bias = (torch.randn(n, generator=g) for n in (H * dim, G * dim, W))
+    w, freq = torch.randn(4, W, generator=g), 1000.0 ** -torch.linspace(0, 1, nrot)
+    rows, pages = _rows(lens), T // page + 2
+    slots = torch.randperm(pages * page, generator=g)[:T].to(torch.int32)
+    if T > 5:
+        slots[5] = -1
+
+    def call(dev, f, st):
+        m = lambda x: x.to(dev)  # noqa: E731
+        q = torch.empty(T, H, dim, device=dev)
+        kc, vc = (torch.full((pages, G, page, dim), 7.0, device=dev, dtype=dtype) for _ in range(2))
+        rs, rb, rf, pos = (m(r) for r in rows)
+        f(m(wide)[:, 8:], None if conv else m(bias), m(qn), m(kn), True, dim, 1e-5, pos, m(freq), 1.5, off, off, m(slots), kc,
+          vc, H, G, dim, dim, dim, 0, q, conv=(m(w), st, rs, rb, rf) if conv else None)
+        return q, kc, vc, st
+
+    got, want = call(DEV, ops.qk_norm_rotary_append, state.to(DEV)), call("cpu", ref.qk_norm_rotary_append, state.clone())
+    # as above; angles of up to 2,100 radians round by 1.2e-4 of them: 30 times the sine's error of 2^-13; bf16 pages: the
+    # neighbouring value, up to 2^-7 away
+    for a, b, rel in zip(got, want, (0.0, 2.0 ** -7, 2.0 ** -7, 0.0)):
+        torch.testing.assert_close(a.cpu().float(), b.float(), atol=3e-5 if T < 100 else 4e-3, rtol=1e-5 + (rel if dtype == torch.bfloat16 else 0.0))
