@@ -55,6 +55,8 @@ void launch_token_shift_mix(bool, const float*, const float*, float*, const int3
                             int, hipStream_t);
 bool wkv_ok(int);
 bool rank_product_ok(int64_t, int64_t, int64_t);
+bool rank_product_f32_ok(int64_t, int64_t, int64_t);
+void launch_rank_product_f32(const float*, int64_t, const float*, int64_t, float*, int, int, int, hipStream_t);
 void launch_rank_product(bool, const void*, int64_t, const void*, int64_t, void*, int, int, int, hipStream_t);
 bool latent_mfma_ok(int, int);
 bool launch_attn_latent_mfma(const void*, int64_t, int64_t, const void*, const int32_t*, int,
@@ -446,21 +448,28 @@ void token_shift_mix(const Tensor& x, const Tensor& mu, const Tensor& prev, cons
                                  out.data_ptr(), T, d, NS, (int)prev.size(0) / 2, stream());
 }
 
-// x . w^T for the short and small products; the caller sends no others.  Memory from elsewhere may
-// begin at any address: such an operand is copied.
+// x . w^T for the short and small products, bf16 or fp32 (of that result); the caller sends no others.  Memory from
+// elsewhere may begin at any address: such an operand is copied.
 Tensor matmul_short(const Tensor& x, const Tensor& w, bool out_f32) {
-  TORCH_CHECK(x.is_cuda() && x.dim() == 2 && w.dim() == 2 && x.scalar_type() == at::kBFloat16 &&
-              w.scalar_type() == at::kBFloat16 && x.device() == w.device() && x.size(1) == w.size(1) &&
-              rfqmix::rank_product_ok(x.size(0), w.size(0), x.size(1)), "matmul_short: x [M, K], w [N, K] bf16");
+  const bool f32 = x.scalar_type() == at::kFloat;
+  TORCH_CHECK(x.is_cuda() && x.dim() == 2 && w.dim() == 2 && (f32 ? out_f32 : x.scalar_type() == at::kBFloat16) &&
+              w.scalar_type() == x.scalar_type() && x.device() == w.device() && x.size(1) == w.size(1) &&
+              (f32 ? rfqmix::rank_product_f32_ok(x.size(0), w.size(0), x.size(1))
+                   : rfqmix::rank_product_ok(x.size(0), w.size(0), x.size(1))),
+              "matmul_short: x [M, K], w [N, K] bf16 or fp32");
   const c10::DeviceGuard on(x.device());
-  auto rows = [](const Tensor& t) {
-    TORCH_CHECK(t.stride(1) == 1 && t.stride(0) % 8 == 0, "matmul_short: rows of whole 16-byte pieces");
+  auto rows = [f32](const Tensor& t) {
+    TORCH_CHECK(t.stride(1) == 1 && t.stride(0) % (f32 ? 4 : 8) == 0, "matmul_short: rows of whole 16-byte pieces");
     return reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0 ? t : t.clone(at::MemoryFormat::Contiguous);
   };
   const Tensor xr = rows(x), wr = rows(w);
   Tensor y = at::empty({x.size(0), w.size(0)}, x.options().dtype(out_f32 ? at::kFloat : at::kBFloat16));
-  rfqmix::launch_rank_product(out_f32, xr.data_ptr(), xr.stride(0), wr.data_ptr(), wr.stride(0), y.data_ptr(),
-                              (int)x.size(0), (int)w.size(0), (int)x.size(1), stream());
+  if (f32)
+    rfqmix::launch_rank_product_f32(xr.data_ptr<float>(), xr.stride(0), wr.data_ptr<float>(), wr.stride(0), y.data_ptr<float>(),
+                                    (int)x.size(0), (int)w.size(0), (int)x.size(1), stream());
+  else
+    rfqmix::launch_rank_product(out_f32, xr.data_ptr(), xr.stride(0), wr.data_ptr(), wr.stride(0), y.data_ptr(),
+                                (int)x.size(0), (int)w.size(0), (int)x.size(1), stream());
   return y;
 }
 

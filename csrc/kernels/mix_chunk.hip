@@ -42,6 +42,7 @@
 #include "common.h"
 #include "mix_common.h"
 #include "mix_chunk.h"
+#include "mix_split.h"
 
 namespace rfqmix {
 
@@ -86,26 +87,7 @@ struct ChunkLds {
   float o[2][MODE == kChunkWkv ? CT * RS : 4];
 };
 
-// fp32 as a sum of three bf16, h + m + l, each the rounding of what is left: the sum is exact (8 bits each and two signs).
-// Products of two such sums without m l, l m and l l, of which each is below 2^-26 of the whole product, take six products
-// on the matrix cores, 2.7 times the rate of fp32 MFMA and, other than those, beside the vector instructions of other
-// waves.  Packed in twos: a in the low half.
-struct Split2 {
-  uint32_t h, m, l;
-};
-__device__ __forceinline__ float lo_f(uint32_t x) { return __uint_as_float(x << 16); }
-__device__ __forceinline__ float hi_f(uint32_t x) { return __uint_as_float(x & 0xffff0000u); }
-__device__ __forceinline__ Split2 split3(float a, float b) {
-  Split2 s;
-  s.h = rfq::pack_bf16x2(a, b);
-  a -= lo_f(s.h);
-  b -= hi_f(s.h);
-  s.m = rfq::pack_bf16x2(a, b);
-  s.l = rfq::pack_bf16x2(a - lo_f(s.m), b - hi_f(s.m));
-  return s;
-}
-// The same cut instead of rounded: for values that the rounding takes to infinity; infinities and NaN are h alone.
-constexpr float kSplitMost = 3.38e38f;
+// split3 cut instead of rounded: for values that the rounding takes to infinity; infinities and NaN are h alone.
 __device__ __forceinline__ Split2 odd_split(float a, float b) {
   uint32_t p[3][2];
   float f[2] = {a, b};
@@ -123,9 +105,6 @@ __device__ __forceinline__ Split2 odd_split(float a, float b) {
 // Where a row of an operand's parts holds channel c: a lane's eight of a 16x16x32 product are channels 4 grp + r of two
 // neighbouring tiles of sixteen, as the accumulators of the state hold them.
 __device__ __forceinline__ int operand_at(int c) { return (c & 32) | (c & 12) << 1 | (c & 16) >> 2 | (c & 3); }
-__device__ __forceinline__ f32x4 mma32(const uint4& a, const uint4& b, const f32x4& c) {
-  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(rfq::bf16x8, a), __builtin_bit_cast(rfq::bf16x8, b), c, 0, 0, 0);
-}
 __device__ __forceinline__ uint4 ld8(const uint16_t* p) { return *reinterpret_cast<const uint4*>(p); }
 __device__ __forceinline__ float4 mul4(float4 x, float4 y) {
   return make_float4(x.x * y.x, x.y * y.y, x.z * y.z, x.w * y.w);

@@ -11,8 +11,11 @@
 // No LDS: a wave has the W rows of 64 columns, all K of them, and 16 rows of X straight from memory in
 // 16-byte pieces.  Y comes out transposed in the accumulators (A = W, B = X), so a lane holds
 // neighbouring entries of a row.
+#include <algorithm>
+
 #include "common.h"
 #include "mix_common.h"
+#include "mix_split.h"
 
 namespace rfqmix {
 
@@ -68,6 +71,90 @@ __global__ __launch_bounds__(256) void rank_product_kernel(const bf16_t* __restr
   }
 }
 
+// The same in fp32, X, W and Y.  Up to 64 terms an eager call takes 8 us for the library's 19, and the device's time is no
+// longer from 2^22 entries on, where it counts: 2,067 x 2,048 (K = 64) 31 -> 13 us, 4,096 x 4,096 33 -> 24, 4,096 x 8,192
+// 55 -> 33 (4.2 TB/s of results); 64 x 2,048 4.8 -> 3.6, 1,000 x 2,048 8.0 -> 9.4 of the device's time.  With more terms the
+// library's tiles are better above 2^18 entries (1,000 x 2,048, K = 96 9.0 us for 13.1).  Error against 64 bits: 4.6e-8 for
+// the library's 1.4e-7 (K = 64).
+// By operands of three bf16 parts (split3): six products on the matrix cores take 96 clocks for the 256
+// that fp32 MFMA hold the vector unit.  A wave keeps its 16 NT columns' W rows as parts and goes through `blocks` times 16 rows
+// of X, the next ones on their way meanwhile.  Infinities, NaN and values that a part cannot hold go through fp32 MFMA.
+template <int KS, int NT>
+__global__ __launch_bounds__(256) void rank_product_f32_kernel(const float* __restrict__ x, int64_t xs, const float* __restrict__ w,
+                                                               int64_t ws, float* __restrict__ y, int M, int N, int blocks) {
+  const int lane = threadIdx.x & 63, col = lane & 15, grp = lane >> 4;
+  const int n0 = (blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6)) * (16 * NT);
+  if (n0 >= N) return;
+  float4 next[2 * KS];                                       // a lane's K entries: 32 k + 8 grp ..
+  auto parts = [](const float4& p, const float4& q, uint4 (&to)[3]) {
+    const Split2 s0 = split3(p.x, p.y), s1 = split3(p.z, p.w), s2 = split3(q.x, q.y), s3 = split3(q.z, q.w);
+    to[0] = make_uint4(s0.h, s1.h, s2.h, s3.h);
+    to[1] = make_uint4(s0.m, s1.m, s2.m, s3.m);
+    to[2] = make_uint4(s0.l, s1.l, s2.l, s3.l);
+    return ((fabsf(p.x) + fabsf(p.y)) + (fabsf(p.z) + fabsf(p.w))) + ((fabsf(q.x) + fabsf(q.y)) + (fabsf(q.z) + fabsf(q.w)));
+  };
+  auto fetch = [&](int m) {
+    const float* xr = x + (int64_t)min(m, M - 1) * xs + 8 * grp;
+#pragma unroll
+    for (int k = 0; k < 2 * KS; ++k) next[k] = ld4(xr + 32 * (k >> 1) + 4 * (k & 1));
+  };
+  const int first = blockIdx.y * blocks * 16 + col;
+  fetch(first);
+  uint4 a[NT][KS][3];
+  float large = 0.f;
+#pragma unroll
+  for (int i = 0; i < NT; ++i) {
+    const float* wr = w + (int64_t)min(n0 + 16 * i + col, N - 1) * ws + 8 * grp;
+#pragma unroll
+    for (int k = 0; k < KS; ++k) large += parts(ld4(wr + 32 * k), ld4(wr + 32 * k + 4), a[i][k]);
+  }
+  for (int t = 0; t < blocks; ++t) {
+    const int m = first + 16 * t;
+    uint4 b[KS][3];
+    float size = large;
+#pragma unroll
+    for (int k = 0; k < KS; ++k) size += parts(next[2 * k], next[2 * k + 1], b[k]);
+    if (t + 1 < blocks) fetch(m + 16);
+    f32x4 c[NT];
+#pragma unroll
+    for (int i = 0; i < NT; ++i) c[i] = (f32x4){0.f, 0.f, 0.f, 0.f};
+    if (__builtin_amdgcn_ballot_w64(!(size < kSplitMost)) == 0ull) {
+      auto product = [&](int p, int q) {                     // the small ones first
+#pragma unroll
+        for (int k = 0; k < KS; ++k)
+#pragma unroll
+          for (int i = 0; i < NT; ++i) c[i] = mma32(a[i][k][p], b[k][q], c[i]);
+      };
+      product(2, 0);
+      product(0, 2);
+      product(1, 1);
+      product(1, 0);
+      product(0, 1);
+      product(0, 0);
+    } else {
+      const float* xr = x + (int64_t)min(m, M - 1) * xs + 4 * grp;
+#pragma unroll 1
+      for (int k = 0; k < 32 * KS; k += 16) {
+        const float4 xv = ld4(xr + k);
+#pragma unroll
+        for (int i = 0; i < NT; ++i) {
+          const float4 wv = ld4(w + (int64_t)min(n0 + 16 * i + col, N - 1) * ws + 4 * grp + k);
+          c[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(wv.x, xv.x, c[i], 0, 0, 0);
+          c[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(wv.y, xv.y, c[i], 0, 0, 0);
+          c[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(wv.z, xv.z, c[i], 0, 0, 0);
+          c[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(wv.w, xv.w, c[i], 0, 0, 0);
+        }
+      }
+    }
+    if (m < M) {
+      float* const to = y + (int64_t)m * N + n0 + 4 * grp;
+#pragma unroll
+      for (int i = 0; i < NT; ++i)
+        if (n0 + 16 * i + 4 * grp < N) st4(to + 16 * i, make_float4(c[i][0], c[i][1], c[i][2], c[i][3]));   // N: a multiple of four
+    }
+  }
+}
+
 // ------------------------------------------------------------------ launcher
 bool rank_product_ok(int64_t M, int64_t N, int64_t K) {
   return M >= 1 && K >= 32 && K <= 128 && K % 32 == 0 && N >= 4 && N % 4 == 0 && M <= (1 << (K > 96 ? 20 : 21)) / N;
@@ -88,6 +175,33 @@ void launch_rank_product(bool out_f32, const void* x, int64_t xs, const void* w,
   } while (0)
   if (out_f32) RANK_ALL(float);
   else RANK_ALL(bf16_t);
+#undef RANK_ALL
+#undef RANK_GO
+}
+
+bool rank_product_f32_ok(int64_t M, int64_t N, int64_t K) {
+  return M >= 1 && M <= 1 << 20 && K >= 32 && K <= 128 && K % 32 == 0 && N >= 4 && N % 4 == 0 && M <= (1 << (K > 64 ? 18 : 26)) / N;
+}
+
+void launch_rank_product_f32(const float* x, int64_t xs, const float* w, int64_t ws, float* y, int M, int N, int K, hipStream_t s) {
+  // 64 columns to a wave, fewer where that leaves SIMDs without one (64 x 2,048, K = 64: 3.6 us for 5.8; 300 x 4,096 7.6 for
+  // 8.5), and up to sixteen times 16 rows (4,096 x 2,048: 8 blocks 15 us, one 26)
+  const int64_t waves = (int64_t)((N + 63) / 64) * ((M + 15) / 16);
+  const int blocks = (int)std::min<int64_t>(16, std::max<int64_t>(1, waves / 1024));
+  const int nt = waves <= 640 || K > 64 ? 1 : waves < 1536 ? 2 : 4;
+  const dim3 grid((N + 64 * nt - 1) / (64 * nt), (M + 16 * blocks - 1) / (16 * blocks));
+#define RANK_GO(KS, NT) \
+  hipLaunchKernelGGL((rank_product_f32_kernel<KS, NT>), grid, dim3(256), 0, s, x, xs, w, ws, y, M, N, blocks)
+#define RANK_ALL(KS)              \
+  do {                            \
+    if (nt == 1) RANK_GO(KS, 1);  \
+    else if (nt == 2) RANK_GO(KS, 2); \
+    else RANK_GO(KS, 4);          \
+  } while (0)
+  if (K == 32) RANK_ALL(1);
+  else if (K == 64) RANK_ALL(2);
+  else if (K == 96) RANK_GO(3, 1);
+  else RANK_GO(4, 1);
 #undef RANK_ALL
 #undef RANK_GO
 }

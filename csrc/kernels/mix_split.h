@@ -1,0 +1,31 @@
+// fp32 operands on the bf16 matrix cores.
+#pragma once
+#include "common.h"
+
+namespace rfqmix {
+
+// fp32 as a sum of three bf16, h + m + l, each the rounding of what is left: the sum is exact (8 bits each and two signs).
+// Products of two such sums without m l, l m and l l, of which each is below 2^-26 of the whole product, take six products
+// on the matrix cores, 2.7 times the rate of fp32 MFMA and, other than those, beside the vector instructions of other
+// waves.  Packed in twos: a in the low half.
+struct Split2 {
+  uint32_t h, m, l;
+};
+__device__ __forceinline__ float lo_f(uint32_t x) { return __uint_as_float(x << 16); }
+__device__ __forceinline__ float hi_f(uint32_t x) { return __uint_as_float(x & 0xffff0000u); }
+__device__ __forceinline__ Split2 split3(float a, float b) {
+  Split2 s;
+  s.h = rfq::pack_bf16x2(a, b);
+  a -= lo_f(s.h);
+  b -= hi_f(s.h);
+  s.m = rfq::pack_bf16x2(a, b);
+  s.l = rfq::pack_bf16x2(a - lo_f(s.m), b - hi_f(s.m));
+  return s;
+}
+// The largest value that split3 takes: larger ones may round to infinity.
+constexpr float kSplitMost = 3.38e38f;
+__device__ __forceinline__ rfq::f32x4 mma32(const uint4& a, const uint4& b, const rfq::f32x4& c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(rfq::bf16x8, a), __builtin_bit_cast(rfq::bf16x8, b), c, 0, 0, 0);
+}
+
+}  // namespace rfqmix
