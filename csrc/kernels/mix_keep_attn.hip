@@ -374,8 +374,8 @@ __global__ __launch_bounds__(1024) void qk_norm_rotary_append_kernel(
   }
 }
 
-// The same for steps of many rows whose norms are of whole projections: a workgroup takes several neighbouring rows one
-// after another.  A thread has two chunks of eight columns for all of them and keeps these columns' weights (of the
+// The same where norms are of whole projections, of a single key head or none: a workgroup takes several neighbouring rows
+// one after another.  A thread has two chunks of eight columns for all of them and keeps these columns' weights (of the
 // convolution, the norms, the bias) and the rows above in registers; with a workgroup a row every row read 100 KB of
 // weights and three rows from the L2s for its own 12, which bounded it.  Two rows on are on their way while one is made;
 // they are waited for before a row's stores, which are counted with the loads and in order.
@@ -391,7 +391,8 @@ struct QknRows {
   int q_rot_off, k_rot_off;
   const int32_t* slots;
   void *k_cache, *v_cache;
-  int T, H, G, qw, kw, vdim, BS;
+  int T, H, G, qw, kw, vdim, BS;        // vdim 0: no values
+  int q_from, k_norm_n, neighbours;     // k_norm_n: of kw entries (whole projections: all)
   int64_t pool_slots;
   float* q_out;
   int64_t q_ts, q_hs;
@@ -422,19 +423,20 @@ __global__ __launch_bounds__(N == 1 ? 1024 : kQknThreads) void qk_norm_rotary_ap
     meta[5 * tid + 4] = a.pos[t];
   }
   const T* proj = static_cast<const T*>(a.proj);
-  int col[N];                                             // chunks past the row are read as its last one
+  int col[N], at[N];                                      // columns here and in proj; chunks past the row: its last one
   bool live[N];
 #pragma unroll
   for (int j = 0; j < N; ++j) {
     col[j] = (tid + j * nthr) * 8;
     live[j] = col[j] < W;
     if (!live[j]) col[j] = W - 8;
+    at[j] = CONV ? col[j] : col[j] + a.q_from * (col[j] < nq ? col[j] / a.qw + 1 : a.H);
   }
   Bits<8> raw[N], next[DEEP ? N : 1], above[CONV ? K : 1][N];
   auto fetch = [&](auto& to, int r) {
     const T* src = proj + (int64_t)(t0 + min(max(r, -t0), n - 1)) * a.stride;
 #pragma unroll
-    for (int j = 0; j < N; ++j) to[j].load(src + col[j]);
+    for (int j = 0; j < N; ++j) to[j].load(src + at[j]);
   };
   fetch(raw, 0);
   if constexpr (DEEP) fetch(next, 1);
@@ -447,7 +449,7 @@ __global__ __launch_bounds__(N == 1 ? 1024 : kQknThreads) void qk_norm_rotary_ap
 #pragma unroll
       for (int j = 0; j < N; ++j) ld_chunk<8>(a.conv_w + (int64_t)d * W + col[j], taps[d][j]);
   }
-  // a chunk's place: 0 q, 1 k, 2 v; its head and the entry in it; the rotation of its head
+  // a chunk's place: 0 q, 1 k, 2 v, 3 k without norm; its head and the entry in it; the rotation of its head
   int kind[N], head[N], entry[N], turn[N];                // turn: (cos, sin) pairs by which it turns, or -1
   bool first[N];                                          // of the rotation's two halves
 #pragma unroll
@@ -458,7 +460,8 @@ __global__ __launch_bounds__(N == 1 ? 1024 : kQknThreads) void qk_norm_rotary_ap
     entry[j] = y - head[j] * w;
     const int r0 = entry[j] - (kind[j] == 0 ? a.q_rot_off : a.k_rot_off);
     first[j] = r0 < a.nrot;
-    turn[j] = kind[j] < 2 && r0 >= 0 && r0 < 2 * a.nrot ? (first[j] ? r0 : r0 - a.nrot) : -1;
+    turn[j] = kind[j] < 2 && r0 >= 0 && r0 < 2 * a.nrot ? (a.neighbours ? r0 >> 1 : first[j] ? r0 : r0 - a.nrot) : -1;
+    if (kind[j] == 1 && entry[j] >= a.k_norm_n) kind[j] = 3;          // a key's entries that are not normed
     const float* wn = kind[j] == 0 ? a.q_norm_w : kind[j] == 1 ? a.k_norm_w : nullptr;
     if (wn != nullptr) ld_chunk<8>(wn + y, norm[j]);
     else
@@ -567,7 +570,7 @@ __global__ __launch_bounds__(N == 1 ? 1024 : kQknThreads) void qk_norm_rotary_ap
     const int part = lane & 15;
     const float qs = group_sum(part < nw ? sum[part] : 0.f, 16), ks = group_sum(part < nw ? sum[nw + part] : 0.f, 16);
     const float fq = a.q_norm_w != nullptr ? 1.0f / sqrtf(qs / (float)nq + a.eps) : 1.f;
-    const float fk = a.k_norm_w != nullptr ? 1.0f / sqrtf(ks / (float)nk + a.eps) : 1.f;
+    const float fk = a.k_norm_w != nullptr ? 1.0f / sqrtf(ks / (float)(a.G * a.k_norm_n) + a.eps) : 1.f;
 #pragma unroll
     for (int j = 0; j < N; ++j) {
       const float fc = kind[j] == 0 ? fq : kind[j] == 1 ? fk : 1.f;
@@ -575,6 +578,15 @@ __global__ __launch_bounds__(N == 1 ? 1024 : kQknThreads) void qk_norm_rotary_ap
       for (int i = 0; i < 8; i += 2) {
         f[j][i] *= fc * norm[j][i];
         f[j][i + 1] *= fc * norm[j][i + 1];
+        if (a.neighbours) {
+          if (turn[j] >= 0) {
+            const float2 c = *reinterpret_cast<const float2*>(cs + 2 * (r * a.nrot + turn[j]) + i);
+            const float x = f[j][i] * c.x - f[j][i + 1] * c.y;
+            f[j][i + 1] = f[j][i + 1] * c.x + f[j][i] * c.y;
+            f[j][i] = x;
+          }
+          continue;
+        }
         const float u0 = __shfl_xor(f[j][i], a.nrot >> 3, 64), u1 = __shfl_xor(f[j][i + 1], a.nrot >> 3, 64);   // the partner's
         if (turn[j] >= 0) {
           const float4 c = ld4(cs + 2 * (r * a.nrot + turn[j] + i));
@@ -594,8 +606,8 @@ __global__ __launch_bounds__(N == 1 ? 1024 : kQknThreads) void qk_norm_rotary_ap
       if (live[j]) {
         if (kind[j] == 0) st_chunk<8>(a.q_out + (t0 + r) * a.q_ts + head[j] * a.q_hs + entry[j], f[j]);
         else if (keep) {
-          T* cache = static_cast<T*>(kind[j] == 1 ? a.k_cache : a.v_cache);
-          st_chunk<8>(cache + (page_row + (int64_t)head[j] * a.BS) * (kind[j] == 1 ? a.kw : a.vdim) + entry[j], f[j]);
+          T* cache = static_cast<T*>(kind[j] != 2 ? a.k_cache : a.v_cache);
+          st_chunk<8>(cache + (page_row + (int64_t)head[j] * a.BS) * (kind[j] != 2 ? a.kw : a.vdim) + entry[j], f[j]);
         }
       }
   }
@@ -1014,19 +1026,21 @@ bool launch_qk_norm_rotary_append(bool f32, const void* proj, int64_t stride, co
   // A partner of the rotation lies as many lanes away as chunks: nrot / 8, a power of two, and heads and rotations begin at
   // multiples of both halves.
   const int turn = 2 * nrot;
-  const bool lanes = nrot == 0 || (turn <= 512 && (nrot & (nrot - 1)) == 0 && q_rot_off % turn == 0 && k_rot_off % turn == 0 &&
+  const bool lanes = nrot == 0 || neighbours || (turn <= 512 && (nrot & (nrot - 1)) == 0 && q_rot_off % turn == 0 && k_rot_off % turn == 0 &&
                                    qw % turn == 0 && kw % turn == 0);
   // Two chunks a thread, one where a thread keeps the convolution's weights for it (two spill 30 registers).  Of rows beyond
   // 8,192 columns, convolved, few are faster in the other kernel (80 heads of 128: 257 rows 15.0 us for 16.5, 1,024 34.2
   // for 31.2); all others gain at every size.  32 + 8 + 8 heads of 128 in bf16: convolved 1 row 8.1 -> 7.3 us, 64 rows 9.3
   // -> 7.9, 512 12.6 -> 9.5, 2,648 40.5 -> 29.3 (3.0 TB/s), 8,192 103 -> 85; with a bias 2,648 rows 28.7 -> 21.5.
+  // Latents (64 rotated entries of 32 heads, 576 of the key): 2,067 rows 15.2 -> 11.3, 8,192 44.3 -> 28.2.
   const int per = conv_w != nullptr && W <= 8 * 1024 ? 1 : 2;
   const int wide = (int)((W / 8 + per - 1) / per + 63) / 64 * 64;
-  if (vec && lanes && norm_all && G > 0 && v_mode == 0 && v_in == nullptr && v_out == nullptr && q_from == 0 && !neighbours &&
-      (conv_w == nullptr || (taps == kQknTaps && bias == nullptr)) && wide <= (per == 1 ? 1024 : kQknThreads) &&
+  const bool one = norm_all || (q_norm_w == nullptr && (k_norm_w == nullptr || G == 1));     // norm of a kind's columns
+  if (vec && lanes && one && G > 0 && v_mode != 1 && v_in == nullptr && v_out == nullptr &&
+      (conv_w == nullptr || (taps == kQknTaps && bias == nullptr && q_from == 0)) && wide <= (per == 1 ? 1024 : kQknThreads) &&
       (conv_w == nullptr || per == 1 || T >= 1024)) {
     QknRows a{proj, stride, bias, q_norm_w, k_norm_w, eps, pos, inv_freq, nrot, rot_mult, q_rot_off, k_rot_off, slots, k_cache,
-              v_cache, T, H, G, qw, kw, vdim, BS, pool_slots, q_out, q_ts, q_hs, conv_w, conv_state, state_slots, row_state,
+              v_cache, T, H, G, qw, kw, v_mode == 0 ? vdim : 0, BS, q_from, norm_all ? kw : k_norm_n, (int)neighbours, pool_slots, q_out, q_ts, q_hs, conv_w, conv_state, state_slots, row_state,
               row_back, row_fwd, 0};
     const int at_once = 256 * std::max(1, 12 * 64 / wide);
     a.rows = std::min(kQknRows, (T + at_once - 1) / at_once);

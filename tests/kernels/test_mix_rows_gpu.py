@@ -126,3 +126,28 @@ def test_norm_and_rotation_of_rows_one_after_another(dtype, conv, H, G, dim, nro
     # neighbouring value, up to 2^-7 away
     for a, b, rel in zip(got, want, (0.0, 2.0 ** -7, 2.0 ** -7, 0.0)):
         torch.testing.assert_close(a.cpu().float(), b.float(), atol=3e-5 if T < 100 else 4e-3, rtol=1e-5 + (rel if dtype == torch.bfloat16 else 0.0))
+
+
+# The same without values: the rotated ends of query heads, one key of which only the leading entries are normed
+@pytest.mark.parametrize("T", [3, 1030])
+@pytest.mark.parametrize("neighbours", [False, True])
+@pytest.mark.parametrize("H,qw,latent,rot", [(5, 48, 96, 16), (32, 192, 512, 64)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_rotated_ends_and_a_partly_normed_key(dtype, H, qw, latent, rot, neighbours, T):
+    g = torch.Generator().manual_seed(T + H)
+    E, page, pages = latent + rot, 32, T // 32 + 2
+    proj = torch.randn(T, H * qw + E + 8, generator=g).to(dtype)
+    kn, freq = torch.randn(latent, generator=g), 1000.0 ** -torch.linspace(0, 1, rot // 2)
+    pos, slots = torch.arange(7, T + 7, dtype=torch.int32), torch.randperm(pages * page, generator=g)[:T].to(torch.int32)
+    slots[1] = -1
+
+    def call(dev, f):
+        m = lambda x: x.to(dev)  # noqa: E731
+        q, pool = torch.full((T, H, E), 3.0, device=dev), torch.full((pages, 1, page, E), 7.0, device=dev, dtype=dtype)
+        f(m(proj), None, None, m(kn), False, latent, 1e-5, m(pos), m(freq), 1.5, qw - rot, latent, m(slots), pool, None, H, 1,
+          qw, E, 0, 2, q[:, :, latent:], neighbours=neighbours)
+        return q, pool
+
+    # as above
+    for a, b, rel in zip(call(DEV, ops.qk_norm_rotary_append), call("cpu", ref.qk_norm_rotary_append), (0.0, 2.0 ** -7)):
+        torch.testing.assert_close(a.cpu().float(), b.float(), atol=3e-5 if T < 100 else 4e-3, rtol=1e-5 + (rel if dtype == torch.bfloat16 else 0.0))
