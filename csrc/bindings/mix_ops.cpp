@@ -56,6 +56,9 @@ void launch_token_shift_mix(bool, const float*, const float*, float*, const int3
 bool wkv_ok(int);
 bool rank_product_ok(int64_t, int64_t, int64_t);
 bool rank_product_f32_ok(int64_t, int64_t, int64_t);
+bool batch_product_ok(int64_t, int64_t, int64_t, int64_t);
+void launch_batch_product(const void*, int64_t, int64_t, const void*, int64_t, int64_t, float*, int64_t, int64_t, int, int, int,
+                          int, hipStream_t);
 void launch_rank_product_f32(const float*, int64_t, const float*, int64_t, float*, int, int, int, hipStream_t);
 void launch_rank_product(bool, const void*, int64_t, const void*, int64_t, void*, int, int, int, hipStream_t);
 bool latent_mfma_ok(int, int);
@@ -472,6 +475,29 @@ Tensor matmul_short(const Tensor& x, const Tensor& w, bool out_f32) {
                                 (int)x.size(0), (int)w.size(0), (int)x.size(1), stream());
   return y;
 }
+
+// out = a . b for a batch, bf16 into fp32; the caller sends only what the kernel takes.  Operands that begin at any address
+// are copied; a result at such a place, or in an operand's memory, is made beside it.
+void bmm_short(const Tensor& a, const Tensor& b, const Tensor& out) {
+  TORCH_CHECK(a.is_cuda() && a.dim() == 3 && b.dim() == 3 && out.dim() == 3 && a.scalar_type() == at::kBFloat16 &&
+              b.scalar_type() == at::kBFloat16 && out.scalar_type() == at::kFloat && a.device() == b.device() &&
+              a.device() == out.device(), "bmm_short: a, b bf16, out fp32");
+  const int64_t B = a.size(0), M = a.size(1), K = a.size(2), N = b.size(2);
+  TORCH_CHECK(b.size(0) == B && b.size(1) == K && out.size(0) == B && out.size(1) == M && out.size(2) == N &&
+              rfqmix::batch_product_ok(B, M, N, K), "bmm_short: a [B, M, K], b [B, K, N], out [B, M, N]");
+  for (const Tensor& t : {a, b, out})
+    TORCH_CHECK(t.stride(2) == 1 && (t.stride(0) | t.stride(1)) % (t.element_size() == 2 ? 8 : 4) == 0,
+                "bmm_short: rows of whole 16-byte pieces");
+  const c10::DeviceGuard on(a.device());
+  auto whole = [](const Tensor& t) { return reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0; };
+  const Tensor x = whole(a) ? a : a.clone(at::MemoryFormat::Contiguous), w = whole(b) ? b : b.clone(at::MemoryFormat::Contiguous);
+  const bool own = whole(out) && !out.is_alias_of(a) && !out.is_alias_of(b);
+  const Tensor y = own ? out : at::empty({B, M, N}, out.options());
+  rfqmix::launch_batch_product(x.data_ptr(), x.stride(0), x.stride(1), w.data_ptr(), w.stride(0), w.stride(1),
+                               y.data_ptr<float>(), y.stride(0), y.stride(1), (int)B, (int)M, (int)N, (int)K, stream());
+  if (!own) out.copy_(y);
+}
+void bmm_short_meta(const Tensor&, const Tensor&, const Tensor&) {}
 
 // under vmap: the library's product, which has a batched form; in fp32, as batched bf16 products with a
 // transposed right side are not safe on this hardware
@@ -1233,6 +1259,7 @@ TORCH_LIBRARY(rfq_mix, m) {
   m.def("silu_mul_any(Tensor gate_up, Tensor(a!) out) -> ()");
   m.def("softcap(Tensor(a!) x, float cap) -> ()");
   m.def("matmul_short(Tensor x, Tensor w, bool out_f32) -> Tensor");
+  m.def("bmm_short(Tensor a, Tensor b, Tensor(c!) out) -> ()");
   m.def("token_shift_mix(Tensor x, Tensor mu, Tensor(a!) prev, Tensor row_state, Tensor row_back, Tensor row_fwd, Tensor pos, Tensor(b!) out) -> ()");
   m.def("wkv_recurrence(Tensor r, Tensor k, Tensor v, Tensor zw, Tensor w0, Tensor u, Tensor gate, Tensor norm_w, float eps, Tensor(a!) state, Tensor row_state, Tensor row_back, Tensor row_fwd, Tensor pos, Tensor? run_rows, Tensor(b!) out) -> ()");
   m.def("moe_route_grouped(Tensor z, Tensor correction, int top, int groups, int keep, Tensor(a!) ids, Tensor(b!) weights) -> ()");
@@ -1277,6 +1304,7 @@ TORCH_LIBRARY_IMPL(rfq_mix, CUDA, m) {
   m.impl("softcap", &softcap);
   m.impl("token_shift_mix", &token_shift_mix);
   m.impl("matmul_short", &matmul_short);
+  m.impl("bmm_short", &bmm_short);
   m.impl("wkv_recurrence", &wkv_recurrence);
   m.impl("moe_route_grouped", &moe_route_grouped);
   m.impl("moe_pair_up", &moe_pair_up);
@@ -1294,4 +1322,7 @@ TORCH_LIBRARY_IMPL(rfq_mix, CUDA, m) {
 }
 
 TORCH_LIBRARY_IMPL(rfq_mix, FuncTorchBatched, m) { m.impl("matmul_short", &matmul_short_batched); }
-TORCH_LIBRARY_IMPL(rfq_mix, Meta, m) { m.impl("matmul_short", &matmul_short_meta); }
+TORCH_LIBRARY_IMPL(rfq_mix, Meta, m) {
+  m.impl("matmul_short", &matmul_short_meta);
+  m.impl("bmm_short", &bmm_short_meta);
+}

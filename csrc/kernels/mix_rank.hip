@@ -155,6 +155,71 @@ __global__ __launch_bounds__(256) void rank_product_f32_kernel(const float* __re
   }
 }
 
+// Y[b] = X[b] . W[b] for a batch, W[b] [K, N] as it lies, bf16 operands, Y in fp32: queries of decode rows carried into a
+// latent space, head by head, into slices of wider rows.  A wave makes 16 rows of 64 columns: their W passes through its
+// piece of LDS, 64 terms at a time, and is read back transposed.  What bounds it: launch and three trips to memory, 4 - 5 us;
+// the library's takes 5 - 6 and 18 us of the host, 9 here, which bounded a decode step (64 rows of 32 heads, 128 to
+// 512: 5.6 -> 4.7 us, the pass 49 -> 41).  From 2^20 results on the library's tiles are better (64 heads 6.8 us for 7.9).
+template <int KS>
+__global__ __launch_bounds__(256) void batch_product_kernel(const bf16_t* __restrict__ x, int64_t xb, int64_t xs,
+                                                            const bf16_t* __restrict__ w, int64_t wb, int64_t ws,
+                                                            float* __restrict__ y, int64_t yb, int64_t ys, int M, int N) {
+  constexpr int WR = 64 + 8, KH = KS < 2 ? 32 : 64;          // shorts per row in LDS, rows
+  __shared__ __attribute__((aligned(16))) short slab[4][KH * WR];
+  const int lane = threadIdx.x & 63, col = lane & 15, grp = lane >> 4, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int n0 = (blockIdx.x * 4 + wave) * 64;
+  if (n0 >= N) return;
+  x += blockIdx.z * xb;
+  w += blockIdx.z * wb + n0;
+  y += blockIdx.z * yb + n0;
+  const int m = blockIdx.y * 16 + col;
+  const bf16_t* xr = x + (int64_t)min(m, M - 1) * xs + 8 * grp;
+  s16x8 b[KS];
+#pragma unroll
+  for (int k = 0; k < KS; ++k) b[k] = *reinterpret_cast<const s16x8*>(xr + 32 * k);
+  s16x8 a[4][KS];
+  short* S = slab[wave];
+#pragma unroll
+  for (int h = 0; h < KS; h += 2) {
+    constexpr int pieces = KH / 8;                           // eight rows to a load of the wave
+    s16x8 raw[pieces];
+#pragma unroll
+    for (int i = 0; i < pieces; ++i)
+      if (h * 32 + 8 * i < KS * 32)
+        raw[i] = *reinterpret_cast<const s16x8*>(w + (int64_t)(h * 32 + 8 * i + (lane >> 3)) * ws + 8 * (lane & 7));
+#pragma unroll
+    for (int i = 0; i < pieces; ++i)
+      if (h * 32 + 8 * i < KS * 32) *reinterpret_cast<s16x8*>(S + (8 * i + (lane >> 3)) * WR + 8 * (lane & 7)) = raw[i];
+    // a wave's LDS accesses are in order: this keeps the compiler's
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll
+    for (int k = h; k < h + 2 && k < KS; ++k)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const short* p = S + (32 * (k - h) + 8 * grp + (col >> 2)) * WR + 16 * i + 4 * (col & 3);
+        const rfq::s16x4 lo = rfq::ds_read_tr16(p), hi = rfq::ds_read_tr16(p + 4 * WR);
+        a[i][k] = (s16x8){lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+      }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  }
+  f32x4 c[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) c[i] = (f32x4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int k = 0; k < KS; ++k)
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      c[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(a[i][k]), as_bf16x8(b[k]), c[i], 0, 0, 0);
+  if (m >= M) return;
+  float* const to = y + (int64_t)m * ys + 4 * grp;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) st4(to + 16 * i, make_float4(c[i][0], c[i][1], c[i][2], c[i][3]));
+}
+
 // ------------------------------------------------------------------ launcher
 bool rank_product_ok(int64_t M, int64_t N, int64_t K) {
   return M >= 1 && K >= 32 && K <= 128 && K % 32 == 0 && N >= 4 && N % 4 == 0 && M <= (1 << (K > 96 ? 20 : 21)) / N;
@@ -204,6 +269,24 @@ void launch_rank_product_f32(const float* x, int64_t xs, const float* w, int64_t
   else RANK_GO(4, 1);
 #undef RANK_ALL
 #undef RANK_GO
+}
+
+bool batch_product_ok(int64_t B, int64_t M, int64_t N, int64_t K) {
+  return B >= 1 && B <= 65535 && M >= 1 && N >= 64 && N % 64 == 0 && N <= 1 << 20 && M <= (1 << 20) / N && B <= (1 << 20) / (M * N) &&
+         K >= 32 && K <= 128 && K % 32 == 0;
+}
+
+void launch_batch_product(const void* x, int64_t xb, int64_t xs, const void* w, int64_t wb, int64_t ws, float* y, int64_t yb,
+                          int64_t ys, int B, int M, int N, int K, hipStream_t s) {
+  const dim3 grid((N + 255) / 256, (M + 15) / 16, B);
+#define BATCH_GO(KS)                                                                                                    \
+  hipLaunchKernelGGL((batch_product_kernel<KS>), grid, dim3(256), 0, s, (const bf16_t*)x, xb, xs, (const bf16_t*)w, wb, \
+                     ws, y, yb, ys, M, N)
+  if (K == 32) BATCH_GO(1);
+  else if (K == 64) BATCH_GO(2);
+  else if (K == 96) BATCH_GO(3);
+  else BATCH_GO(4);
+#undef BATCH_GO
 }
 
 }  // namespace rfqmix

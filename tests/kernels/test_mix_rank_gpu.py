@@ -92,3 +92,44 @@ def test_fp32_products_keep_autocast_and_derivatives():
     torch.testing.assert_close(x.grad, w.sum(0, keepdim=True).expand(8, 64), atol=1e-4, rtol=1e-4)
     y = torch.func.vmap(lambda a: ops.matmul_nt(a, w))(torch.ones(3, 5, 64, device=DEV))
     torch.testing.assert_close(y, w.sum(1).expand(3, 5, 12), atol=1e-4, rtol=1e-4)
+
+
+# rows and columns around a wave's tile, slices of wider rows on all sides, results of rows in either order; what stays with
+# the library: 2^20 results and one row, columns that are no whole tiles, 40 terms, a result in memory of an operand
+@pytest.mark.parametrize("B,M,N", [(1, 1, 64), (3, 17, 320), (32, 64, 512), (32, 65, 512), (2, 5, 72)])
+@pytest.mark.parametrize("K", [32, 64, 96, 128, 40])
+@pytest.mark.parametrize("rows_first", [False, True])
+def test_batches_of_short_products(B, M, N, K, rows_first):
+    g = torch.Generator().manual_seed(B * M + K)
+    x = torch.randn(M, B, K + 24, generator=g).to(DEV, torch.bfloat16)[:, :, 8:8 + K].transpose(0, 1)
+    w = torch.randn(B, K, N + 8, generator=g).to(DEV, torch.bfloat16)[:, :, :N]
+    wide = torch.full((M, B, N + 64) if rows_first else (B, M, N + 64), 7.0, device=DEV)
+    out = wide[:, :, :N].transpose(0, 1) if rows_first else wide[:, :, :N]
+    assert ops.bmm_f32(x, w, out=out) is out
+    xd, wd = x.double().cpu(), w.double().cpu()
+    tol = K * 2.0 ** -24 * (xd.abs() @ wd.abs())             # as above
+    assert bool(((out.double().cpu() - xd @ wd).abs() <= tol).all()) and bool((wide[:, :, N:] == 7.0).all())
+
+
+def test_batches_that_the_kernel_leaves_alone():
+    x, w = torch.randn(2, 4, 64, device=DEV).bfloat16(), torch.randn(2, 64, 64, device=DEV).bfloat16()
+    out = torch.empty(2, 4, 64, device=DEV)
+    ok = lambda *a: ops._short_batch(*a)  # noqa: E731
+    assert ok(x, w, out) and not ok(x, w, out.bfloat16()) and not ok(x[:, :, 1:33], w[:, :32], out)
+    assert not ok(x, w.transpose(1, 2), out) and not ok(x, w, out[:, :1].expand(2, 4, 64)) and not ok(x, w[:1], out)
+    assert not ok(x[:, :0], w, out[:, :0]) and not ok(x, w, torch.empty(2, 5, 64, device=DEV))
+    # a result beside an operand in the same memory, operands at odd addresses, and shapes alone
+    both = torch.zeros(2, 4, 96 + 64, device=DEV)
+    a = both.view(torch.bfloat16)[:, :, :64].copy_(x)
+    ops.bmm_f32(a, w, out=both[:, :, 96:])
+    torch.testing.assert_close(both[:, :, 96:], x.float() @ w.float(), atol=1e-4, rtol=1e-4)
+    assert torch.equal(both.view(torch.bfloat16)[:, :, :64], x)
+    odd = torch.zeros(2 * 4 * 64 + 1, device=DEV, dtype=torch.bfloat16)[1:].view(2, 4, 64).copy_(x)
+    torch.testing.assert_close(ops.bmm_f32(odd, w, out=out), x.float() @ w.float(), atol=1e-4, rtol=1e-4)
+    from torch._subclasses.fake_tensor import FakeTensorMode
+    with FakeTensorMode():
+        fake = [torch.empty(2, 4, 64, device=DEV, dtype=torch.bfloat16), torch.empty(2, 64, 64, device=DEV, dtype=torch.bfloat16)]
+        assert ops.bmm_f32(*fake, out=torch.empty(2, 4, 64, device=DEV)).shape == (2, 4, 64)
+        assert ops.matmul_nt(torch.empty(4, 64, device=DEV), torch.empty(8, 64, device=DEV)).shape == (4, 8)
+    y = torch.func.vmap(lambda a: ops.bmm_f32(a, w))(torch.stack([x, x]))
+    torch.testing.assert_close(y[1], x.float() @ w.float(), atol=1e-3, rtol=1e-4)
