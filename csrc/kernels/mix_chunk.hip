@@ -886,7 +886,8 @@ __device__ __forceinline__ void chunk_run(const ChunkArgs& a, const ChunkSegment
   }
 
   if constexpr (DELTA) {
-    if (role == 0 && !sg.last) {                          // a segment: dim is NC and all channels are there
+    // what the later kernel reads: never written by it, whose workgroups begin and end at any time
+    if (role == 0 && !sg.last && (TURN || sg.seg == 0)) { // a segment: dim is NC and all channels are there
       const DeltaSeg d = delta_seg(a, sg.slot, h);
 #pragma unroll
       for (int j = 0; j < NV; ++j)

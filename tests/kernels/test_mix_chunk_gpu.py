@@ -185,6 +185,38 @@ def test_delta_rule_in_segments(H, Hq, vdim, lens, shift):
     _close(st, st_w, tol)
 
 
+def test_segments_beside_other_work():
+    """Workgroups that begin late, between others that are done, read the same: products on another stream hold CUs meanwhile.
+    Decays near one, and other inputs in between, so that a state from elsewhere would show."""
+    steps = []
+    for seed, lens in ((1, [1500, 900]), (2, [2400])):
+        g = torch.Generator().manual_seed(seed)
+        T, H = sum(lens), 16
+        q, k = (torch.nn.functional.normalize(torch.randn(T, H, 64, generator=g), dim=-1).to(DEV) for _ in range(2))
+        v, z = torch.randn(T, H, 128, generator=g).to(DEV), torch.randn(T, H * 64, generator=g).to(DEV)
+        beta, gate = torch.randn(T, H, generator=g).to(DEV), torch.randn(T, H * 128, generator=g).to(DEV)
+        rows, runs = _rows(lens, 23)
+        steps.append((q, k, v, z, beta, gate, torch.randn(2 * len(lens), H, 64, 128, generator=g).to(DEV), [r.to(DEV) for r in rows], runs.to(DEV)))
+
+    def call(q, k, v, z, beta, gate, st, rows, runs):
+        out, st = torch.empty_like(gate), st.clone()
+        ops.gated_linear_recurrence(q, k, v, z, torch.full((16,), 0.01, device=DEV), torch.full((16 * 64,), -4.0, device=DEV), 1.0, beta,
+                                    gate, True, torch.ones(128, device=DEV), 1e-5, 0.125, st, *rows, out, run_rows=runs)
+        return out, st
+
+    alone = [call(*s) for s in steps]
+    side, m = torch.cuda.Stream(), torch.randn(2048, 2048, device=DEV)
+    torch.cuda.synchronize()
+    for i in range(12):
+        with torch.cuda.stream(side):
+            for _ in range(1 + i % 4):
+                m @ m
+        for s, want in zip(steps, alone):
+            got = call(*s)
+            assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1]), i
+    torch.cuda.synchronize()
+
+
 @pytest.mark.parametrize("size,row", [(3.0, 2100), (1e20, 1000)])
 def test_delta_rule_turns_that_grow(size, row):
     """Keys that turn a state into a larger one, or a state of zeros into what no fp32 holds, leave segments to be done in
