@@ -19,15 +19,16 @@
 // a chunk.  (fp32 MFMA 16x16x4 hold a SIMD's vector unit for their 32 clocks, other waves' instructions as well: with the
 // state's products in it the decay waves stood for as long as they took, 2.3 us a chunk of the delta rule.)  The state's
 // products, 48 of 56 a wave, therefore go to the matrix cores in bf16: an fp32 operand is the exact sum of three bf16, six
-// products of them leave out less than 2^-26 of each (split3).  Those inside a chunk stay in fp32 MFMA.  Errors against
-// 64 bits: state of the delta rule 6.3e-8 for 6.4e-8 before, outputs of gla in fp32 5.7e-7 and of wkv 2.0e-7, the same.
+// products of them leave out less than 2^-26 of each (split3).  Those inside a chunk stay in fp32 MFMA: pairs of blocks on
+// tiles of 4x4x1, whose sixteen side by side take 64 channels of one pair in 32 clocks (16x16x4 made all pairs of a distance
+// and sixteen more each, 512: wkv 172 -> 164 us a pass, delta 276 -> 265).  Errors against 64 bits: state of the delta rule 6.3e-8 for 6.4e-8 before, outputs of gla in fp32 5.7e-7 and of wkv 2.0e-7, the same.
 // One workgroup per (run, head, 64 or 128 value channels): four consumer waves hold 64 x 16 of the state, or twice that, in
 // accumulators, which are MFMA operands as they lie (a lane holds channels 16 i + 4 grp + r of its column); the other
 // waves work ahead: decays, their products and parts for chunk c + 3, A for chunk c + 2, T for chunk c + 1, wkv's norm
 // and gate for chunk c - 1; one barrier per chunk.  The state never leaves the registers.  A chunk takes 2.1 us with 64
 // channels (delta; gla 1.65, wkv 1.45) and 2.7 with 128 (gla 2.0), for which the other waves' work is done once.
 // Measured, two runs of 2,048 tokens in bf16, all kernels of the recurrence: delta rule with 32 heads of 64 x 128 301 ->
-// 190 us, wkv with 64 heads of 64 x 64 203 -> 136; gla in fp32, five ragged runs of up to 1,031, 32 heads, 121 -> 85.
+// 171 us, wkv with 64 heads of 64 x 64 203 -> 128; gla in fp32, five ragged runs of up to 1,031, 32 heads, 121 -> 82.
 //
 // A run's chain is cut where workgroups leave CUs idle (chunk_seg_cap, segment_rows).  Without the delta rule
 // chunk_segment_kernel makes what every segment's rows leave of a state of zeros and the products of its decays, all
@@ -66,24 +67,38 @@ __device__ __forceinline__ float ror_add(float v) {   // sum over the 16 lanes o
   v += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x121, 0xf, 0xf, true));
   return v;
 }
+// Sixteen tiles of 4x4 added up: lane 16 i + j (and those 4, 8, 12 further) gets entry (i, j).
+__device__ __forceinline__ float tiles_sum(const f32x4& x) {
+  auto swap32 = [](float p, float q) {                    // lanes below 32: p's two halves, above: q's
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(p), __float_as_uint(q), false, false);
+    return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+  };
+  const float e = swap32(x[0], x[2]), o = swap32(x[1], x[3]);
+  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(e), __float_as_uint(o), false, false);
+  float v = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+  v += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x128, 0xf, 0xf, true));
+  v += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x124, 0xf, 0xf, true));
+  return v;
+}
 // What a chunk's producers leave in LDS.
 template <int MODE>
 struct ChunkLds {
   static constexpr bool DELTA = MODE == kChunkDelta;
-  // four chunks in flight between producers and consumers; parts as split3 makes them
-  uint16_t qd[4][3][CT * PS];           // [part][token][operand_at(channel)]
-  uint16_t kk[DELTA ? 4 : 1][3][DELTA ? CT * PS : 8];
-  uint16_t kd[4][NC * PS];   // Kd^T: [channel][four tokens: two parts of four, first and third again]
-  uint32_t odd[4][4];                   // of each wave: operands that are split otherwise, see odd_split
-  float dec[4][NC];
-  float beta[4][CT];
+  // What is written in small pieces comes first: its places are constants of LDS instructions, up to 64 KB.
   float aq[4][CT * TS];
   float ak[2][DELTA ? CT * TS : 4];
   float tt[2][DELTA ? CT * TS : 4];
-  float q[2][CT * RS], k[2][CT * RS], a[2][CT * RS];      // operands of A: raw,
-  float ql[2][CT * RS], kl[2][CT * RS];                   // times the block's products up to / after
-  float kb[2][DELTA ? CT * RS : 4];
+  float dec[4][NC];
+  float beta[4][CT];
+  uint32_t odd[4][4];                   // of each wave: operands that are split otherwise, see odd_split
   float blk[2][4 * NC];                 // product of a block's decays
+  float ql[2][CT * RS], kl[2][CT * RS];                   // operands of A: times the block's products up to / after,
+  float kb[2][DELTA ? CT * RS : 4];
+  float q[2][CT * RS], k[2][CT * RS], a[2][CT * RS];      // raw
+  // four chunks in flight between producers and consumers; parts as split3 makes them
+  uint16_t qd[4][3][CT * PS];           // [part][token][operand_at(channel)]
+  uint16_t kk[DELTA ? 4 : 1][3][DELTA ? CT * PS : 8];
+  uint16_t kd[4][NC * PS];              // Kd^T: [channel][four tokens: two parts of four, first and third again]
   float o[2][MODE == kChunkWkv ? CT * RS : 4];
 };
 
@@ -738,57 +753,38 @@ __device__ __forceinline__ void chunk_run(const ChunkArgs& a, const ChunkSegment
         }
       }
       if (const int c = it + 2; c >= 0 && c < nc) {
-        // A of chunk c.  Pairs of blocks `far` apart: one 16 x 16 product of the readers' rows with
-        // the writers' rows times the blocks between them, of which those pairs are kept.  The delta
-        // rule's keys as readers take the same columns: beside q's rows where they fit (rows 0..7 q,
-        // 8..15 k of the last two blocks), else in a product of their own.
-        const int b = c & 1;
-        auto product = [&](auto far_c, auto rows_c) {     // rows: 0 q, 1 k, 2 both
-          constexpr int far = far_c, rows = rows_c;
-          const float* src = TURN || rows == 1 || (rows == 2 && col >= 8) ? L.kb[DELTA ? b : 0] : L.ql[b];
-          const int tr = rows == 2 ? 8 + (col & 7) : col;
-          float4 q[4], k[4], g[4], g2[4];
-#pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            const int at = 16 * i + 4 * grp;
-            q[i] = ld4(src + tr * RS + at);
-            k[i] = ld4(&L.kl[b][col * RS + at]);
-            if constexpr (far > 1) g[i] = ld4(&L.blk[b][min((col >> 2) + 1, 3) * NC + at]);
-            if constexpr (far > 2) g2[i] = ld4(&L.blk[b][min((col >> 2) + 2, 3) * NC + at]);
-          }
-          f32x4 x = (f32x4){0.f, 0.f, 0.f, 0.f}, y = x;
-#pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            if constexpr (far > 1) k[i] = mul4(k[i], g[i]);
-            if constexpr (far > 2) k[i] = mul4(k[i], g2[i]);
-            x = __builtin_amdgcn_mfma_f32_16x16x4f32(q[i].x, k[i].x, x, 0, 0, 0);
-            y = __builtin_amdgcn_mfma_f32_16x16x4f32(q[i].y, k[i].y, y, 0, 0, 0);
-            x = __builtin_amdgcn_mfma_f32_16x16x4f32(q[i].z, k[i].z, x, 0, 0, 0);
-            y = __builtin_amdgcn_mfma_f32_16x16x4f32(q[i].w, k[i].w, y, 0, 0, 0);
-          }
-          x += y;
-          const int tb = rows == 2 ? 2 + (grp & 1) : grp;  // this lane's block of rows, its column's block
-          float* to = rows == 1 || (rows == 2 && grp >= 2) ? L.ak[DELTA ? b : 0] : L.aq[c & 3];
-          if (tb - (col >> 2) == far && !(TURN && rows == 2 && grp < 2)) {
-#pragma unroll
-            for (int r = 0; r < 4; ++r) to[(4 * tb + r) * TS + col] = x[r];
-          }
+        // A of chunk c.  A pair of blocks: the readers' rows with the writers' rows times the blocks between them, on tiles
+        // of 4x4x1, of which sixteen side by side take four key channels each.
+        const int b = c & 1, at = lane & ~3;
+        auto pair = [&](auto tb_c, auto sb_c) {
+          constexpr int tb = tb_c, sb = sb_c;
+          float4 k = ld4(&L.kl[b][(4 * sb + (lane & 3)) * RS + at]);
+          if constexpr (tb > sb + 1) k = mul4(k, ld4(&L.blk[b][(sb + 1) * NC + at]));
+          if constexpr (tb > sb + 2) k = mul4(k, ld4(&L.blk[b][(sb + 2) * NC + at]));
+          auto product = [&](const float* rows, float* to) {
+            const float4 q = ld4(rows + (4 * tb + (lane & 3)) * RS + at);
+            f32x4 x = (f32x4){0.f, 0.f, 0.f, 0.f};
+            x = __builtin_amdgcn_mfma_f32_4x4x1f32(q.x, k.x, x, 0, 0, 0);
+            x = __builtin_amdgcn_mfma_f32_4x4x1f32(q.y, k.y, x, 0, 0, 0);
+            x = __builtin_amdgcn_mfma_f32_4x4x1f32(q.z, k.z, x, 0, 0, 0);
+            x = __builtin_amdgcn_mfma_f32_4x4x1f32(q.w, k.w, x, 0, 0, 0);
+            const float y = tiles_sum(x);
+            if ((lane & 12) == 0) to[(4 * tb + grp) * TS + 4 * sb + (lane & 3)] = y;
+          };
+          if constexpr (!TURN) product(L.ql[b], L.aq[c & 3]);
+          if constexpr (DELTA) product(L.kb[b], L.ak[b]);
         };
         constexpr std::integral_constant<int, 0> i0{};
         constexpr std::integral_constant<int, 1> i1{};
         constexpr std::integral_constant<int, 2> i2{};
         constexpr std::integral_constant<int, 3> i3{};
-        if constexpr (TURN) {                             // pairs of keys alone
-          if (w == 1) { product(i1, i1); product(i3, i2); }
-          else if (w == 2) product(i2, i2);
-        } else if constexpr (DELTA) {
-          if (w == 0) product(i1, i0);
-          else if (w == 1) { product(i1, i1); product(i3, i2); }
-          else if (w == 2) product(i2, i2);
+        if constexpr (DELTA) {
+          if (w == 1) { pair(i1, i0); pair(i2, i1); pair(i3, i0); }
+          else if (w == 2) { pair(i3, i2); pair(i2, i0); pair(i3, i1); }
         } else {
-          if (w == 0) product(i1, i0);
-          else if (w == 1) product(i2, i0);
-          else if (w == 2) product(i3, i0);
+          if (w == 0) { pair(i1, i0); pair(i2, i0); }
+          else if (w == 1) { pair(i2, i1); pair(i3, i1); }
+          else if (w == 2) { pair(i3, i2); pair(i3, i0); }
         }
         if (w == (DELTA ? 0 : 3)) {
           // pairs inside a block: sixteen lanes per block, four key channels each
@@ -1121,7 +1117,7 @@ __global__ __launch_bounds__(chunk_threads(MODE)) void chunk_recurrence_segments
 // last what their rows leave of a state of zeros and the 64 x 64 turn that they make of any, by the same chunks with 64
 // more columns.  After it the later segments, from the state that the turns carry to them.  A workgroup per segment,
 // head and 128 value channels: the producers' work, which 64 channels cost as much, is done half as often.
-// Two runs of 2,048 with 32 heads: 301 -> 89 + 95 us.  Error of the state against 64 bits as with whole runs (6.3e-8 to
+// Two runs of 2,048 with 32 heads: 301 -> 82 + 89 us.  Error of the state against 64 bits as with whole runs (6.3e-8 to
 // 6.5e-8).  Unit keys and betas of at most 1 turn a state no larger.  Where an entry passes that (other keys, whose turns may
 // grow or overflow though the state does not), a run's second segment goes through to its end in sequence.
 template <typename TI, typename TG>
