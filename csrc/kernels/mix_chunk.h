@@ -40,6 +40,8 @@ int chunk_min_run(int mode, int T, const ChunkArgs& a);
 // Segments that the step's runs are shared in at most where they are, else 0 (sets a.per and a.unit), and the scratch floats of a.cap.
 int chunk_seg_cap(int mode, bool in_f32, int T, ChunkArgs& a);
 int64_t chunk_seg_floats(int mode, const ChunkArgs& a);
+// Whether the kernels may cut a run: the device's choice of segments and the launches that it needs go by this alone.
+__host__ __device__ inline bool chunk_may_cut(const ChunkArgs& a) { return a.cap > a.runs; }
 // in_f32: q, k, v (and wkv's z, gate, out) are fp32, else bf16; act_f32: beta's type.
 // T: rows of the step.
 void launch_chunk(int mode, bool in_f32, bool act_f32, int T, const ChunkArgs& a, hipStream_t s);

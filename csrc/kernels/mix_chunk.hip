@@ -187,8 +187,9 @@ __device__ __forceinline__ ChunkSegment whole_run(const ChunkArgs& a, int t0) {
 
 // How long the step's segments are: only the device knows its runs (64 at most).  Lane l tries the longest run in l + 1
 // equal parts (of whole chunks, a.unit rows where the first kernel shares a segment over its waves); of those that make no
-// more than a.cap segments (workgroups of one of the delta rule's kernels) the one takes over that the times below (us, as measured) say is done first.  The same for
-// every wave of both kernels.
+// more than a.cap segments (workgroups of one of the delta rule's kernels) the one takes over that the times below (us, as
+// measured) say is done first.  The same for every wave of both kernels.  Where only one of them is launched runs stay
+// whole: entries without a run leave a.cap room that nobody may take then.
 template <int MODE, int NV>
 __device__ __forceinline__ int segment_rows(const ChunkArgs& a, int n, int lane) {
   constexpr bool DELTA = MODE == kChunkDelta;
@@ -210,7 +211,8 @@ __device__ __forceinline__ int segment_rows(const ChunkArgs& a, int n, int lane)
   float t;
   if constexpr (DELTA) t = rounds(all - cut) * (9.f + 2.7f * c) + (all > runs ? 3.f + rounds(all - runs) * (11.f + 2.8f * c) + 3.f * (most - 2) : 0.f);
   else t = rounds(all) * (6.f + (MODE == kChunkWkv ? 1.45f : NV == 1 ? 1.65f : 2.f) * c) + (all > runs ? 10.f + 0.25f * c + 0.8f * most : 0.f);
-  uint32_t best = (DELTA ? all - cut : all) <= a.cap ? (__float_as_uint(t) & ~63u) | (uint32_t)lane : ~0u;
+  const bool may = lane == 0 || (chunk_may_cut(a) && (DELTA ? all - cut : all) <= a.cap);
+  uint32_t best = may ? (__float_as_uint(t) & ~63u) | (uint32_t)lane : ~0u;
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) best = min(best, (uint32_t)__shfl_xor((int)best, o, 64));
   return __builtin_amdgcn_readlane(rows, (int)(best & 63u));
@@ -1274,12 +1276,12 @@ static void launch_chunk_segments(const ChunkArgs& a, hipStream_t s) {
     allow_lds<&chunk_delta_first_kernel<TI, TG>>();
     allow_lds<&chunk_delta_later_kernel<TI, TG>>();
     hipLaunchKernelGGL((chunk_delta_first_kernel<TI, TG>), grid, wg, lds, s, a);
-    if (a.cap > a.runs) hipLaunchKernelGGL((chunk_delta_later_kernel<TI, TG>), grid, wg, lds, s, a);
+    if (chunk_may_cut(a)) hipLaunchKernelGGL((chunk_delta_later_kernel<TI, TG>), grid, wg, lds, s, a);
   } else {
     allow_lds<&chunk_recurrence_segments_kernel<TI, TG, MODE, NV>>();
     const dim3 parts(a.H, a.vdim / 64 * (NC / kSegKeys), a.cap);
-    if (a.cap > a.runs && a.unit > 8 * CT) hipLaunchKernelGGL((chunk_segment_kernel<TI, MODE, NV, 16>), parts, dim3(1024), 0, s, a);
-    else if (a.cap > a.runs) hipLaunchKernelGGL((chunk_segment_kernel<TI, MODE, NV, 8>), parts, dim3(512), 0, s, a);
+    if (chunk_may_cut(a) && a.unit > 8 * CT) hipLaunchKernelGGL((chunk_segment_kernel<TI, MODE, NV, 16>), parts, dim3(1024), 0, s, a);
+    else if (chunk_may_cut(a)) hipLaunchKernelGGL((chunk_segment_kernel<TI, MODE, NV, 8>), parts, dim3(512), 0, s, a);
     hipLaunchKernelGGL((chunk_recurrence_segments_kernel<TI, TG, MODE, NV>), grid, wg, lds, s, a);
   }
 }

@@ -34,7 +34,7 @@ def _close(got, want, tol):
     assert float((got[ok] - want[ok]).square().mean().sqrt()) <= tol * float(scale)
 
 
-def _linrec(mode, H, Hq, dim, vdim, dtype, shift, lens=LENS, spoil=None, pad=3, keys=None):
+def _linrec(mode, H, Hq, dim, vdim, dtype, shift, lens=LENS, spoil=None, pad=3, keys=None, spare=0):
     g = torch.Generator().manual_seed(H * 1000 + dim + vdim)
     T = sum(lens)
     wide = torch.randn(T, 2 * Hq * dim + H * vdim + pad, generator=g)              # columns of wider rows
@@ -52,6 +52,7 @@ def _linrec(mode, H, Hq, dim, vdim, dtype, shift, lens=LENS, spoil=None, pad=3, 
     nw = torch.randn(vdim, generator=g)
     st = torch.randn(2 * len(lens), H, dim, vdim, generator=g) * 0.3
     rows, runs = _rows(lens, 23)
+    runs = torch.cat([runs, torch.full((spare,), -1, dtype=torch.int32)])
 
     def call(dev, f, w, zz, s, **more):
         out = torch.empty(T, H * vdim, dtype=dtype, device=dev)
@@ -181,6 +182,19 @@ def test_a_non_finite_value_stays_out_of_earlier_segments():
 def test_delta_rule_in_segments(H, Hq, vdim, lens, shift):
     (out, st), (out_w, st_w) = _linrec("delta", H, Hq, 64, vdim, torch.float32, shift, lens=lens)
     tol = 1e-5 * (max(lens) / 150) ** 0.5 if shift < 0 else 1e-5        # as for wkv above
+    _close(out, out_w, tol)
+    _close(st, st_w, tol)
+
+
+# As many entries as the chip has room for segments: whole runs, however many of the entries are empty (the one that every
+# list here has and `spare`).  Cut into segments all the same, three of five runs, or every one, would begin from states
+# that no kernel had made.
+@pytest.mark.parametrize("mode,H,lens,spare", [("gla", 32, [1031, 77, 345, 1, 613], 2), ("gla", 64, [700, 800], 1),
+                                               ("delta", 16, [600] * 4, 11), ("delta", 32, [1300, 900], 5)])
+def test_empty_entries_leave_runs_whole(mode, H, lens, spare):
+    # decays near one: what a segment begins from stays in its rows
+    (out, st), (out_w, st_w) = _linrec(mode, H, H, 64, 128, torch.float32, -6.0, lens=lens, pad=4, spare=spare)
+    tol = 1e-5 * (max(lens) / 150) ** 0.5                    # as for wkv above
     _close(out, out_w, tol)
     _close(st, st_w, tol)
 
