@@ -102,7 +102,7 @@ struct ChunkLds {
   float o[2][MODE == kChunkWkv ? CT * RS : 4];
 };
 
-// split3 cut instead of rounded: for values that the rounding takes to infinity; infinities and NaN are h alone.
+// split3 cut instead of rounded: for values that are added up in fp32 (kSplitMost); infinities and NaN are h alone.
 __device__ __forceinline__ Split2 odd_split(float a, float b) {
   uint32_t p[3][2];
   float f[2] = {a, b};
@@ -512,7 +512,7 @@ __device__ __forceinline__ void chunk_run(const ChunkArgs& a, const ChunkSegment
       bool plain = (oddw.x | oddw.y | oddw.z | oddw.w) == 0;
 #pragma unroll
       for (int j = 0; j < NT; ++j) plain = plain && finite4(o[j]) && finite4(y[j]);
-      // Infinities, NaN, and values that a part cannot hold: in fp32 products
+      // Infinities, NaN, and values too large for products of parts: in fp32 products
       const bool odd = __builtin_amdgcn_ballot_w64(!plain) != 0ull;
       if (odd) {
 #pragma unroll
@@ -569,7 +569,7 @@ __device__ __forceinline__ void chunk_run(const ChunkArgs& a, const ChunkSegment
           st[j][i][3] *= dc.w;
         }
       }
-      bool small = true;                                  // within what a part can hold
+      bool small = true;                                  // enough for products of parts
 #pragma unroll
       for (int j = 0; j < NT; ++j) small = small && (fabsf(u[j][0]) + fabsf(u[j][1])) + (fabsf(u[j][2]) + fabsf(u[j][3])) < kSplitMost;
       if (odd || __builtin_amdgcn_ballot_w64(!small) != 0ull) {

@@ -78,7 +78,7 @@ __global__ __launch_bounds__(256) void rank_product_kernel(const bf16_t* __restr
 // the library's 1.4e-7 (K = 64).
 // By operands of three bf16 parts (split3): six products on the matrix cores take 96 clocks for the 256
 // that fp32 MFMA hold the vector unit.  A wave keeps its 16 NT columns' W rows as parts and goes through `blocks` times 16 rows
-// of X, the next ones on their way meanwhile.  Infinities, NaN and values that a part cannot hold go through fp32 MFMA.
+// of X, the next ones on their way meanwhile.  Infinities, NaN and values too large for products of parts go through fp32 MFMA.
 template <int KS, int NT>
 __global__ __launch_bounds__(256) void rank_product_f32_kernel(const float* __restrict__ x, int64_t xs, const float* __restrict__ w,
                                                                int64_t ws, float* __restrict__ y, int M, int N, int blocks) {

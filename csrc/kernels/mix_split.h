@@ -22,8 +22,9 @@ __device__ __forceinline__ Split2 split3(float a, float b) {
   s.l = rfq::pack_bf16x2(a - lo_f(s.m), b - hi_f(s.m));
   return s;
 }
-// The largest value that split3 takes: larger ones may round to infinity.
-constexpr float kSplitMost = 3.38e38f;
+// Sums of sizes from here on are not for products of parts: above 2^127 h itself may round to infinity, and a product of two
+// h may pass the end of fp32 where that of the values does not (both 2^64 - 2^55).
+constexpr float kSplitMost = 0x1p60f;
 __device__ __forceinline__ rfq::f32x4 mma32(const uint4& a, const uint4& b, const rfq::f32x4& c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(rfq::bf16x8, a), __builtin_bit_cast(rfq::bf16x8, b), c, 0, 0, 0);
 }

@@ -267,6 +267,18 @@ def test_states_at_the_ends_of_fp32(mode, value):
             _close(st[i::len(LENS)], st_w[i::len(LENS)], 1e-5)
 
 
+def test_products_that_end_just_below_the_range():
+    """(2^64 - 2^55)^2 is a number of fp32, the square of what it rounds to in bf16 is not: a key's entry and a value in the
+    last row of the longest run."""
+    def keys(k, v):
+        k[-1], v[-1] = 0.0, 0.0
+        k[-1, :, 0] = v[-1, 3] = 2.0 ** 64 - 2.0 ** 55
+
+    (_, st), (_, st_w) = _linrec("gla", 2, 2, 64, 64, torch.float32, 0.0, keys=keys)
+    assert bool(torch.isfinite(st_w).all())
+    _close(st, st_w, 1e-5)
+
+
 # 40 rows: chunks; 6: token by token; 200 without a list of runs: the scan
 @pytest.mark.parametrize("n", [40, 6, 200])
 @pytest.mark.parametrize("mode", ["gla", "delta"])

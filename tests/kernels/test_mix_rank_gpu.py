@@ -83,6 +83,16 @@ def test_fp32_products_at_the_ends_of_the_range(value):
     torch.testing.assert_close(y.cpu(), want, atol=0, rtol=1e-6, equal_nan=True)
 
 
+@pytest.mark.parametrize("M,N,K", [(40, 72, 64), (2100, 2052, 64), (64, 512, 128)])
+def test_fp32_products_that_end_just_below_the_range(M, N, K):
+    """(2^64 - 2^55)^2 is a number of fp32; the square of what it rounds to in bf16 is not."""
+    x, w = torch.zeros(M, K, device=DEV), torch.zeros(N, K, device=DEV)
+    x[::3, 5] = w[::2, 5] = 2.0 ** 64 - 2.0 ** 55
+    _check_f32(x, w)
+    x[::2, 7], w[::2, 7] = 2.0 ** 63, -(2.0 ** 63)           # finite sums of both signs
+    _check_f32(x, w)
+
+
 def test_fp32_products_keep_autocast_and_derivatives():
     x, w = (torch.randn(n, 64, device=DEV) for n in (8, 12))
     with torch.autocast("cuda", torch.bfloat16):
