@@ -78,7 +78,8 @@ __global__ __launch_bounds__(256) void rank_product_kernel(const bf16_t* __restr
 // the library's 1.4e-7 (K = 64).
 // By operands of three bf16 parts (split3): six products on the matrix cores take 96 clocks for the 256
 // that fp32 MFMA hold the vector unit.  A wave keeps its 16 NT columns' W rows as parts and goes through `blocks` times 16 rows
-// of X, the next ones on their way meanwhile.  Infinities, NaN and values too large for products of parts go through fp32 MFMA.
+// of X, the next ones on their way meanwhile.  Infinities, NaN and rows too large or too small for products of parts go
+// through fp32 MFMA.
 template <int KS, int NT>
 __global__ __launch_bounds__(256) void rank_product_f32_kernel(const float* __restrict__ x, int64_t xs, const float* __restrict__ w,
                                                                int64_t ws, float* __restrict__ y, int M, int N, int blocks) {
@@ -101,24 +102,26 @@ __global__ __launch_bounds__(256) void rank_product_f32_kernel(const float* __re
   const int first = blockIdx.y * blocks * 16 + col;
   fetch(first);
   uint4 a[NT][KS][3];
-  float large = 0.f;
+  bool fits = true;
 #pragma unroll
   for (int i = 0; i < NT; ++i) {
     const float* wr = w + (int64_t)min(n0 + 16 * i + col, N - 1) * ws + 8 * grp;
+    float size = 0.f;
 #pragma unroll
-    for (int k = 0; k < KS; ++k) large += parts(ld4(wr + 32 * k), ld4(wr + 32 * k + 4), a[i][k]);
+    for (int k = 0; k < KS; ++k) size += parts(ld4(wr + 32 * k), ld4(wr + 32 * k + 4), a[i][k]);
+    fits &= split_fits(size);
   }
   for (int t = 0; t < blocks; ++t) {
     const int m = first + 16 * t;
     uint4 b[KS][3];
-    float size = large;
+    float size = 0.f;
 #pragma unroll
     for (int k = 0; k < KS; ++k) size += parts(next[2 * k], next[2 * k + 1], b[k]);
     if (t + 1 < blocks) fetch(m + 16);
     f32x4 c[NT];
 #pragma unroll
     for (int i = 0; i < NT; ++i) c[i] = (f32x4){0.f, 0.f, 0.f, 0.f};
-    if (__builtin_amdgcn_ballot_w64(!(size < kSplitMost)) == 0ull) {
+    if (__builtin_amdgcn_ballot_w64(!(fits & split_fits(size))) == 0ull) {
       auto product = [&](int p, int q) {                     // the small ones first
 #pragma unroll
         for (int k = 0; k < KS; ++k)

@@ -93,6 +93,19 @@ def test_fp32_products_that_end_just_below_the_range(M, N, K):
     _check_f32(x, w)
 
 
+@pytest.mark.parametrize("a,b", [(1e-36, 1.0), (1.0, 1e-36), (1e10, 1e-36), (1e-33, 1e-4)])
+@pytest.mark.parametrize("M,N,K", [(40, 72, 64), (2100, 2052, 32), (64, 512, 128)])
+def test_fp32_products_of_small_operands(M, N, K, a, b):
+    """Entries whose third part bf16 does not hold, of all rows and of every third, keep the precision that others have."""
+    g = torch.Generator().manual_seed(M)
+    x, w = (torch.randn(n, K, generator=g).to(DEV) for n in (M, N))
+    _check_f32(x * a, w * b)
+    x[1::3] *= a
+    w[::3] *= b
+    x[5] = 0.0
+    _check_f32(x, w)
+
+
 def test_fp32_products_keep_autocast_and_derivatives():
     x, w = (torch.randn(n, 64, device=DEV) for n in (8, 12))
     with torch.autocast("cuda", torch.bfloat16):
