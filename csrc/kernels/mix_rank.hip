@@ -72,10 +72,10 @@ __global__ __launch_bounds__(256) void rank_product_kernel(const bf16_t* __restr
 }
 
 // The same in fp32, X, W and Y.  Up to 64 terms an eager call takes 8 us for the library's 19, and the device's time is no
-// longer from 2^22 entries on, where it counts: 2,067 x 2,048 (K = 64) 31 -> 13 us, 4,096 x 4,096 33 -> 24, 4,096 x 8,192
-// 55 -> 33 (4.2 TB/s of results); 64 x 2,048 4.8 -> 3.6, 1,000 x 2,048 8.0 -> 9.4 of the device's time.  With more terms the
-// library's tiles are better above 2^18 entries (1,000 x 2,048, K = 96 9.0 us for 13.1).  Error against 64 bits: 4.6e-8 for
-// the library's 1.4e-7 (K = 64).
+// longer either (K = 64: 64 x 2,048 3.2 us for 4.3, 1,000 x 2,048 6.8 for 7.2, 2,067 x 2,048 10.7 for 30.5, 4,096 x 4,096
+// 23.9 for 31.0, 4,096 x 8,192 35.3 for 54.8; 4,096 x 1,024, the worst of 34 sizes, 11.3 for 11.1).  With more terms the
+// library's tiles are better above 2^18 entries (1,000 x 2,048, K = 96 9.0 us for 13.1) and along sides beyond 2^14 (K = 128,
+// 4 x 65,536 7.3 for 9.0).  Error against 64 bits: 4.6e-8 for the library's 1.4e-7 (K = 64).
 // By operands of three bf16 parts (split3): six products on the matrix cores take 96 clocks for the 256
 // that fp32 MFMA hold the vector unit.  A wave keeps its 16 NT columns' W rows as parts and goes through `blocks` times 16 rows
 // of X, the next ones on their way meanwhile.  Infinities, NaN and rows too large or too small for products of parts go
@@ -248,15 +248,20 @@ void launch_rank_product(bool out_f32, const void* x, int64_t xs, const void* w,
 }
 
 bool rank_product_f32_ok(int64_t M, int64_t N, int64_t K) {
-  return M >= 1 && M <= 1 << 20 && K >= 32 && K <= 128 && K % 32 == 0 && N >= 4 && N % 4 == 0 && M <= (1 << (K > 64 ? 18 : 26)) / N;
+  return M >= 1 && M <= 1 << (K > 64 ? 14 : 20) && K >= 32 && K <= 128 && K % 32 == 0 && N >= 4 && N % 4 == 0 &&
+         (K <= 64 || N <= 1 << 14) && M <= (1 << (K > 64 ? 18 : 26)) / N;
 }
 
 void launch_rank_product_f32(const float* x, int64_t xs, const float* w, int64_t ws, float* y, int M, int N, int K, hipStream_t s) {
-  // 64 columns to a wave, fewer where that leaves SIMDs without one (64 x 2,048, K = 64: 3.6 us for 5.8; 300 x 4,096 7.6 for
-  // 8.5), and up to sixteen times 16 rows (4,096 x 2,048: 8 blocks 15 us, one 26)
-  const int64_t waves = (int64_t)((N + 63) / 64) * ((M + 15) / 16);
-  const int blocks = (int)std::min<int64_t>(16, std::max<int64_t>(1, waves / 1024));
-  const int nt = waves <= 640 || K > 64 ? 1 : waves < 1536 ? 2 : 4;
+  // Tiles of 16 x 16 in one round of a wave to every SIMD where up to sixteen blocks of rows a wave allow it: a wave splits
+  // its columns' W once, so 16 (K above 64: registers), 32 or 64 columns by what a wave then has, and as few blocks as
+  // make the round.  K = 64, the library's times beside: 1,000 x 2,048 (columns 32, blocks 4) 6.7 us of the device for 7.2,
+  // 300 x 4,096 (32, 3) 5.6 for 6.9, 2,067 x 2,048 (64, 5) 11 for 31, 65,536 x 16 (16, 4) 5.4 for 6.1, 4 x 2^20 48 for 75.
+  // By waves alone, with blocks in place of rows that are not there: 8.6, 7.0, 12.7, 7.3 and 177.
+  const int64_t tx = (N + 15) / 16, ty = (M + 15) / 16, want = tx * ty / 1024;
+  const int nt = K > 64 || tx < 2 || want < 2 ? 1 : tx < 4 || want <= 8 ? 2 : 4;
+  const int64_t across = (tx + nt - 1) / nt, down = std::max<int64_t>(1, 1024 / across);     // waves
+  const int blocks = (int)std::min<int64_t>(16, (ty + down - 1) / down);
   const dim3 grid((N + 64 * nt - 1) / (64 * nt), (M + 16 * blocks - 1) / (16 * blocks));
 #define RANK_GO(KS, NT) \
   hipLaunchKernelGGL((rank_product_f32_kernel<KS, NT>), grid, dim3(256), 0, s, x, xs, w, ws, y, M, N, blocks)

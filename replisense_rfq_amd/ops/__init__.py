@@ -1085,7 +1085,7 @@ def _short_f32(x, w) -> bool:
     """The same for fp32 operands, up to where the library is as fast."""
     M, K, N = x.shape[0], x.shape[1], w.shape[0]
     return (32 <= K <= SHORT_K and K % 32 == 0 and w.shape[1] == K and 1 <= M <= 1 << 20 and N >= 4 and N % 4 == 0
-            and M * N <= 1 << (18 if K > 64 else 26) and x.device == w.device and x.stride(1) == 1 and w.stride(1) == 1
+            and (M * N <= 1 << 26 if K <= 64 else M * N <= 1 << 18 and max(M, N) <= 1 << 14) and x.device == w.device and x.stride(1) == 1 and w.stride(1) == 1
             and x.stride(0) % 4 == 0 and w.stride(0) % 4 == 0
             and x.storage_offset() % 4 == 0 and w.storage_offset() % 4 == 0)
 

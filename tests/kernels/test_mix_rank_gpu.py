@@ -60,9 +60,11 @@ def _check_f32(x, w):
     assert bool(((y.double().cpu() - xd @ wd.t()).abs() <= tol).all())
 
 
-# a wave with 16, 32 (from 641 tiles of 64 x 16 on) and 64 columns (1,536), one block of rows and several (2,048); tiles that
-# are cut, columns slices of wider rows, rows at odd addresses (there the library, or a copy)
-@pytest.mark.parametrize("M,N", [(1, 4), (17, 60), (64, 2048), (129, 68), (645, 1028), (1540, 1030 * 2), (2100, 2052), (9000, 1024)])
+# a wave with 16, 32 (from 2,048 tiles of 16 x 16 on) and 64 columns (9,216), one block of rows (64 x 2,048) to sixteen
+# (300,000 x 4), fewer columns than a wave takes otherwise (20, 36), more than a round of them beside each other (70,000); tiles
+# that are cut, columns slices of wider rows, rows at odd addresses (there the library, or a copy)
+@pytest.mark.parametrize("M,N", [(1, 4), (17, 60), (64, 2048), (129, 68), (645, 1028), (1540, 1030 * 2), (2100, 2052), (9000, 1024),
+                                 (40000, 20), (20000, 36), (300000, 4), (33, 70000)])
 @pytest.mark.parametrize("K", [32, 64, 96, 128, 40])
 def test_short_fp32_products(M, N, K):
     g = torch.Generator().manual_seed(M + K)
