@@ -19,7 +19,8 @@
 // a chunk.  (fp32 MFMA 16x16x4 hold a SIMD's vector unit for their 32 clocks, other waves' instructions as well: with the
 // state's products in it the decay waves stood for as long as they took, 2.3 us a chunk of the delta rule.)  The state's
 // products, 48 of 56 a wave, therefore go to the matrix cores in bf16: an fp32 operand is the exact sum of three bf16, six
-// products of them leave out less than 2^-26 of each (split3).  Those inside a chunk stay in fp32 MFMA: pairs of blocks on
+// products of them leave out at most 2^-24 of each (split3).  Operands at the ends of bf16's range have ways of their own
+// (kUp, kSplitLeast, odd_split), which cost 2 us of wkv's 100.  Those inside a chunk stay in fp32 MFMA: pairs of blocks on
 // tiles of 4x4x1, whose sixteen side by side take 64 channels of one pair in 32 clocks (16x16x4 made all pairs of a distance
 // and sixteen more each, 512: wkv 172 -> 164 us a pass, delta 276 -> 265).  Errors against 64 bits: state of the delta rule 6.3e-8 for 6.4e-8 before, outputs of gla in fp32 5.7e-7 and of wkv 2.0e-7, the same.
 // One workgroup per (run, head, 64 or 128 value channels): four consumer waves hold 64 x 16 of the state, or twice that, in
@@ -56,6 +57,14 @@ constexpr int RS = NC + 4;              // floats per token row in LDS
 constexpr int TS = CT + 4;              // floats per row of a 16 x 16 tile
 constexpr int PS = NC + 8;              // bf16 per token row of a part of Qd or Kk, per channel row of Kd^T's parts
 constexpr float kTurnMost = 1.001f;     // see chunk_delta_later_kernel
+// Operands of products of parts that bf16's range would cut (kSplitLeast).  Qd and Kk, which decays make as small as they
+// please, are split times kUp, and products with them come out that much larger.  Kd, u and the state are sums of their own
+// along 16 or 64 entries: where all of these are too small, the products are in fp32, of Kd's parts split times kUpKd.
+constexpr float kUp = 0x1p32f, kDown = 0x1p-32f, kUpKd = 0x1p64f, kDownKd = 0x1p-64f;
+// What a column of the state all of whose entries are below kSplitLeast cannot make with four rows of Qd (each entry
+// below kSplitMost).
+constexpr float kReadLeast = 0x1p-28f;
+constexpr uint32_t kOddLarge = 1, kOddSmall = 2;
 
 // four consumers, four waves for the decays, four for A (and T), wkv: four for norm and gate
 constexpr int chunk_threads(int mode) { return mode == kChunkWkv ? 1024 : 768; }
@@ -90,7 +99,8 @@ struct ChunkLds {
   float tt[2][DELTA ? CT * TS : 4];
   float dec[4][NC];
   float beta[4][CT];
-  uint32_t odd[4][4];                   // of each wave: operands that are split otherwise, see odd_split
+  uint32_t odd[4][4];                   // of each wave: operands that are split otherwise (kOddLarge: odd_split, without
+                                        // kUp; kOddSmall: Kd times kUpKd)
   float blk[2][4 * NC];                 // product of a block's decays
   float ql[2][CT * RS], kl[2][CT * RS];                   // operands of A: times the block's products up to / after,
   float kb[2][DELTA ? CT * RS : 4];
@@ -152,8 +162,21 @@ __device__ __forceinline__ float arrived(bf16_t bits) {
 
 namespace {
 __device__ __forceinline__ bool finite4(const f32x4& x) {      // no infinity, no NaN among them
-  return fabsf((fabsf(x[0]) + fabsf(x[1])) + (fabsf(x[2]) + fabsf(x[3]))) < __builtin_huge_valf();
+  return (fabsf(x[0]) + fabsf(x[1])) + (fabsf(x[2]) + fabsf(x[3])) < __builtin_huge_valf();
 }
+
+// Whether the sixteen lanes' columns that a wave's lanes 16 grp + col hold in fours are too small for products of parts.
+__device__ __forceinline__ bool small_column(float most) {
+  most = fmaxf(most, __shfl_xor(most, 16, 64));
+  most = fmaxf(most, __shfl_xor(most, 32, 64));
+  return most > 0.f && most < kSplitLeast;
+}
+// lo <= x < hi, of numbers that are not negative
+__device__ __forceinline__ bool within(float x, float lo, float hi) {
+  return __float_as_uint(x) - __float_as_uint(lo) < __float_as_uint(hi) - __float_as_uint(lo);
+}
+__device__ __forceinline__ float sum_of_sizes(const f32x4& x) { return (fabsf(x[0]) + fabsf(x[1])) + (fabsf(x[2]) + fabsf(x[3])); }
+__device__ __forceinline__ float largest(const f32x4& x) { return fmaxf(fmaxf(fabsf(x[0]), fabsf(x[1])), fmaxf(fabsf(x[2]), fabsf(x[3]))); }
 
 // o[t] += sum_{s<=t} m[t][s] x[s] with the pairs s > t left out instead of multiplied by zero: a
 // token's infinity or NaN stays out of the tokens before it.  (Also taken, with the same result,
@@ -264,6 +287,7 @@ template <typename TI, typename TG, int MODE, int NV = 1, bool TURN = false>
 __device__ __forceinline__ void chunk_run(const ChunkArgs& a, const ChunkSegment& sg, const int h, const int zv, const int tid) {
   constexpr bool WKV = MODE == kChunkWkv, DELTA = MODE == kChunkDelta;
   constexpr int NT = NV + (TURN ? 1 : 0);                 // tiles of 16 columns a consumer wave holds
+  constexpr bool BF16U = !DELTA && sizeof(TI) == 2;       // u, the values, is of one part
   const int lane = tid & 63, col = lane & 15, grp = lane >> 4;
   const int t0 = sg.t0, n = sg.n, nc = (n + CT - 1) / CT;
   const int code = a.row_state[sg.run0];
@@ -349,6 +373,7 @@ __device__ __forceinline__ void chunk_run(const ChunkArgs& a, const ChunkSegment
   };
   float4 nw = {}, bonus = {};
   float zbias = 0.f, rate = 0.f;
+  const float least = grp == 3 ? kSplitLeast : 0.f;       // of a lane's keys
 
   if (role == 0) {
     offsets(vo, a.vs, min(vcol, vdim - 1), sizeof(TI), 0);
@@ -509,27 +534,48 @@ __device__ __forceinline__ void chunk_run(const ChunkArgs& a, const ChunkSegment
       }
       __builtin_amdgcn_sched_barrier(0);                  // operands of later products wait: registers
       const uint4 oddw = *reinterpret_cast<const uint4*>(L.odd[b]);
-      bool plain = (oddw.x | oddw.y | oddw.z | oddw.w) == 0;
+      const bool flagged = (oddw.x | oddw.y | oddw.z | oddw.w) != 0;
+      // Infinities, NaN, and values too large or too small for products of parts: in fp32 products
+      bool plain = !flagged;
 #pragma unroll
-      for (int j = 0; j < NT; ++j) plain = plain && finite4(o[j]) && finite4(y[j]);
-      // Infinities, NaN, and values too large for products of parts: in fp32 products
-      const bool odd = __builtin_amdgcn_ballot_w64(!plain) != 0ull;
+      for (int j = 0; j < NT; ++j) {
+        plain &= j < NV ? within(sum_of_sizes(TURN ? y[j] : o[j]), kReadLeast, __builtin_huge_valf()) : finite4(y[j]);
+        if constexpr (DELTA && !TURN) plain &= finite4(y[j]);
+      }
+      bool odd = false;
+      if (__builtin_amdgcn_ballot_w64(!plain) != 0ull) {
+        bool bad = flagged;
+#pragma unroll
+        for (int j = 0; j < NT; ++j) {
+          float most = 0.f;                               // a turn's columns may be as small as they are: they began as one
+#pragma unroll
+          for (int i = 0; i < 4; ++i) most = j < NV ? fmaxf(most, largest(st[j][i])) : 0.f;
+          bad |= !finite4(o[j]) | !finite4(y[j]) | small_column(most);
+        }
+        odd = __builtin_amdgcn_ballot_w64(bad) != 0ull;
+      }
       if (odd) {
 #pragma unroll
         for (int j = 0; j < NT; ++j) o[j] = y[j] = (f32x4){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
+        for (int i = 0; i < 4; ++i) {
+          const float down = L.odd[b][i] == kOddLarge ? 1.f : kDown;
 #pragma unroll
           for (int r = 0; r < 4; ++r) {
             const int at = 32 * (i >> 1) + 4 * (i & 1) + r;
-            auto whole = [&](const uint16_t* p) { return (ldf(p + at) + ldf(p + at + CT * PS)) + ldf(p + at + 2 * CT * PS); };
+            auto whole = [&](const uint16_t* p) { return ((ldf(p + at) + ldf(p + at + CT * PS)) + ldf(p + at + 2 * CT * PS)) * down; };
 #pragma unroll
             for (int j = 0; j < NT; ++j) {
               if constexpr (DELTA) y[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(whole(kp), st[j][i][r], y[j], 0, 0, 0);
               if constexpr (!TURN) o[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(whole(qp), st[j][i][r], o[j], 0, 0, 0);
             }
           }
+        }
       }
+      const float down = odd ? 1.f : kDown;
+      if constexpr (!TURN)
+#pragma unroll
+        for (int j = 0; j < NT; ++j) o[j] *= down;
       if constexpr (DELTA) {
         const float4 bt = ld4(&L.beta[b][4 * grp]), ta = ld4(&L.tt[it & 1][col * TS + 4 * grp]);
         f32x4 x[NT];
@@ -537,7 +583,8 @@ __device__ __forceinline__ void chunk_run(const ChunkArgs& a, const ChunkSegment
 #pragma unroll
         for (int j = 0; j < NT; ++j) {
           const f32x4 own = j < NV ? (f32x4){v[j % NV][0], v[j % NV][1], v[j % NV][2], v[j % NV][3]} : (f32x4){0.f, 0.f, 0.f, 0.f};
-          x[j] = (f32x4){bt.x * (own[0] - y[j][0]), bt.y * (own[1] - y[j][1]), bt.z * (own[2] - y[j][2]), bt.w * (own[3] - y[j][3])};
+          x[j] = (f32x4){bt.x * fmaf(-down, y[j][0], own[0]), bt.y * fmaf(-down, y[j][1], own[1]),
+                         bt.z * fmaf(-down, y[j][2], own[2]), bt.w * fmaf(-down, y[j][3], own[3])};
           u[j] = (f32x4){0.f, 0.f, 0.f, 0.f};
           whole = whole && finite4(x[j]);
         }
@@ -569,21 +616,30 @@ __device__ __forceinline__ void chunk_run(const ChunkArgs& a, const ChunkSegment
           st[j][i][3] *= dc.w;
         }
       }
-      bool small = true;                                  // enough for products of parts
+      bool fits = !odd;                                   // for products of parts
 #pragma unroll
-      for (int j = 0; j < NT; ++j) small = small && (fabsf(u[j][0]) + fabsf(u[j][1])) + (fabsf(u[j][2]) + fabsf(u[j][3])) < kSplitMost;
-      if (odd || __builtin_amdgcn_ballot_w64(!small) != 0ull) {
+      for (int j = 0; j < NT; ++j)
+        fits &= j < NV && !BF16U ? within(sum_of_sizes(u[j]), kSplitLeast, kSplitMost) : sum_of_sizes(u[j]) < kSplitMost;
+      auto bad = [&]() {
+        bool any = odd;
+#pragma unroll
+        for (int j = 0; j < NT; ++j) any |= !(sum_of_sizes(u[j]) < kSplitMost) | small_column(j < NV && !BF16U ? largest(u[j]) : 0.f);
+        return __builtin_amdgcn_ballot_w64(any) != 0ull;
+      };
+      if (__builtin_amdgcn_ballot_w64(!fits) != 0ull && bad()) {
 #pragma unroll
         for (int j = 0; j < NT; ++j) {
           if constexpr (!TURN) lower_product(L.aq[b], u[j], col, grp, o[j]);
 #pragma unroll
-          for (int i = 0; i < 4; ++i)
+          for (int i = 0; i < 4; ++i) {
+            const float down = L.odd[b][i] == kOddSmall ? kDownKd : 1.f;
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
               const uint16_t* p = sp + 16 * i * PS + r;
-              const float k = (ldf(p) + ldf(p + 4)) + ldf(p + 12);
+              const float k = ((ldf(p) + ldf(p + 4)) + ldf(p + 12)) * down;
               st[j][i] = __builtin_amdgcn_mfma_f32_16x16x4f32(k, u[j][r], st[j][i], 0, 0, 0);
             }
+          }
         }
       } else {
         if constexpr (!TURN) {
@@ -605,12 +661,20 @@ __device__ __forceinline__ void chunk_run(const ChunkArgs& a, const ChunkSegment
           for (int p = 0; p < 2; ++p) kh[i][p] = ld8(sp + 16 * i * PS + 8 * p);
 #pragma unroll
         for (int j = 0; j < NT; ++j) {
-          const Split2 p = split3(u[j][0], u[j][1]), q = split3(u[j][2], u[j][3]);
+          Split2 p{}, q{};
+          if constexpr (BF16U) {
+            p.h = rfq::pack_bf16x2(u[j][0], u[j][1]);
+            q.h = rfq::pack_bf16x2(u[j][2], u[j][3]);
+          } else {
+            p = split3(u[j][0], u[j][1]);
+            q = split3(u[j][2], u[j][3]);
+          }
           const uint4 lh = make_uint4(p.l, q.l, p.h, q.h), mm = make_uint4(p.m, q.m, p.m, q.m), hh = make_uint4(p.h, q.h, p.h, q.h);
 #pragma unroll
           for (int i = 0; i < 4; ++i) st[j][i] = mma32(kh[i][1], lh, st[j][i]);
+          if constexpr (!BF16U)
 #pragma unroll
-          for (int i = 0; i < 4; ++i) st[j][i] = mma32(kh[i][0], mm, st[j][i]);
+            for (int i = 0; i < 4; ++i) st[j][i] = mma32(kh[i][0], mm, st[j][i]);
 #pragma unroll
           for (int i = 0; i < 4; ++i) st[j][i] = mma32(kh[i][0], hh, st[j][i]);
         }
@@ -675,11 +739,11 @@ __device__ __forceinline__ void chunk_run(const ChunkArgs& a, const ChunkSegment
         // the products of the blocks grp ^ 1, grp ^ 2, grp ^ 3 from the lanes that hold them
         const float b1 = __shfl_xor(up[3], 16, 64), b2 = __shfl_xor(up[3], 32, 64), b3 = __shfl_xor(b1, 32, 64);
         const float b23 = b2 * b3;
-        const float pre = ((grp & 1) ? b1 : 1.f) * ((grp & 2) ? b23 : 1.f);
+        const float pre = ((grp & 1) ? b1 * kUp : kUp) * ((grp & 2) ? b23 : 1.f);
         const float post = ((grp & 1) ? 1.f : b1) * ((grp & 2) ? 1.f : b23);
         if (grp == 0) L.dec[b][ch] = up[3] * post;
         L.blk[e][grp * NC + ch] = up[3];
-        float qd[4], kk[4], kd[4], most = 0.f;
+        float qd[4], kk[4], kd[4], sizes = 0.f, most = 0.f;
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           const int at = (4 * grp + i) * RS + ch;
@@ -688,7 +752,8 @@ __device__ __forceinline__ void chunk_run(const ChunkArgs& a, const ChunkSegment
           kd[i] = kl * post;
           qd[i] = ql * pre;
           kk[i] = 0.f;
-          most += fabsf(kd[i]) + fabsf(qd[i]);
+          sizes += fabsf(kd[i]);
+          most += fabsf(qd[i]);
           if constexpr (!TURN) {
             L.q[e][at] = q[i];
             L.ql[e][at] = ql;
@@ -703,7 +768,23 @@ __device__ __forceinline__ void chunk_run(const ChunkArgs& a, const ChunkSegment
             most += fabsf(kk[i]);
           }
         }
-        const bool odd = __builtin_amdgcn_ballot_w64(!(most < kSplitMost)) != 0ull;
+        // as a rule the last four tokens say that a channel's keys are not too small
+        uint32_t odd = 0;
+        if (__builtin_amdgcn_ballot_w64(!((sizes + most < kSplitMost) & (sizes >= least))) != 0ull) {
+          if (__builtin_amdgcn_ballot_w64(!(sizes + most < kSplitMost)) != 0ull) {
+            odd = kOddLarge;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+              const int at = (4 * grp + i) * RS + ch;
+              if constexpr (!TURN) qd[i] = L.ql[e][at] * (pre * kDown);
+              if constexpr (DELTA) kk[i] = L.kb[e][at] * (pre * kDown);
+            }
+          } else if (__builtin_amdgcn_ballot_w64(small_column(sizes)) != 0ull) {
+            odd = kOddSmall;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) kd[i] *= kUpKd;
+          }
+        }
         if (lane == 0) L.odd[b][w] = odd;
         auto put = [&](auto split) {
           const Split2 p = split(kd[0], kd[1]), q = split(kd[2], kd[3]);
@@ -725,7 +806,7 @@ __device__ __forceinline__ void chunk_run(const ChunkArgs& a, const ChunkSegment
             if constexpr (DELTA) rows(L.kk[b], split(kk[i], kk[i + 1]));
           }
         };
-        if (odd) put([](float x, float y) { return odd_split(x, y); });
+        if (odd == kOddLarge) put([](float x, float y) { return odd_split(x, y); });
         else put([](float x, float y) { return split3(x, y); });
       }
       __syncthreads();

@@ -34,7 +34,8 @@ def _close(got, want, tol):
     assert float((got[ok] - want[ok]).square().mean().sqrt()) <= tol * float(scale)
 
 
-def _linrec(mode, H, Hq, dim, vdim, dtype, shift, lens=LENS, spoil=None, pad=3, keys=None, spare=0):
+def _linrec(mode, H, Hq, dim, vdim, dtype, shift, lens=LENS, spoil=None, pad=3, keys=None, spare=0,
+            sizes=(1.0, 1.0, 1.0, 1.0)):
     g = torch.Generator().manual_seed(H * 1000 + dim + vdim)
     T = sum(lens)
     wide = torch.randn(T, 2 * Hq * dim + H * vdim + pad, generator=g)              # columns of wider rows
@@ -42,6 +43,8 @@ def _linrec(mode, H, Hq, dim, vdim, dtype, shift, lens=LENS, spoil=None, pad=3, 
     qk /= qk.square().sum(-1, keepdim=True).sqrt() / (2.0 if mode == "gla" else 1.0)   # unit vectors: delta rule
     if keys is not None:
         keys(qk[:, Hq:], wide[:, 2 * Hq * dim:])
+    for part, size in zip((qk[:, :Hq], qk[:, Hq:], wide[:, 2 * Hq * dim:]), sizes):
+        part *= size
     if spoil is not None:
         wide[spoil[0], 2 * Hq * dim + spoil[1]] = float(spoil[2])
     wide = wide.to(dtype)
@@ -50,7 +53,7 @@ def _linrec(mode, H, Hq, dim, vdim, dtype, shift, lens=LENS, spoil=None, pad=3, 
     beta = torch.randn(T, H, generator=g).to(dtype) if mode == "delta" else None
     gate = torch.randn(T, H * vdim, generator=g).to(dtype)
     nw = torch.randn(vdim, generator=g)
-    st = torch.randn(2 * len(lens), H, dim, vdim, generator=g) * 0.3
+    st = torch.randn(2 * len(lens), H, dim, vdim, generator=g) * (0.3 * sizes[3])
     rows, runs = _rows(lens, 23)
     runs = torch.cat([runs, torch.full((spare,), -1, dtype=torch.int32)])
 
@@ -101,16 +104,17 @@ def test_a_non_finite_value_stays_out_of_earlier_tokens(mode, value):
     _close(out[sum(LENS[:8]):], out_w[sum(LENS[:8]):], 1e-5)  # and no other run sees it
 
 
-def _wkv(dtype, shift, spoil=None, lens=LENS):
+def _wkv(dtype, shift, spoil=None, lens=LENS, sizes=(1.0, 1.0, 1.0, 1.0)):
     H, N = 3, 64
     g = torch.Generator().manual_seed(5)
     T = sum(lens)
     r, k, v, zw, gate = (torch.randn(T, H * N, generator=g) for _ in range(5))
+    r, k, v = (x * size for x, size in zip((r, k, v), sizes))
     if spoil is not None:
         v[spoil[0], spoil[1]] = spoil[2]
     r, k, v, zw, gate = (x.to(dtype) for x in (r, k, v, zw, gate))
     w0, u = torch.randn(H * N, generator=g) + shift, torch.randn(H, N, generator=g)
-    nw, st = torch.randn(H * N, generator=g), torch.randn(2 * len(lens), H, N, N, generator=g) * 0.3
+    nw, st = torch.randn(H * N, generator=g), torch.randn(2 * len(lens), H, N, N, generator=g) * (0.3 * sizes[3])
     rows, runs = _rows(lens, 23)
 
     def call(dev, f, s, **more):
@@ -254,6 +258,46 @@ def test_many_long_runs_share_workgroups_of_128_channels(mode):
     (out, st), (out_w, st_w) = _linrec(mode, 8, 4, 64, 192, torch.float32, 0.0, lens=[81 + i % 7 for i in range(24)] + [3, 16])
     _close(out, out_w, 1e-5)
     _close(st, st_w, 1e-5)
+
+
+# Entries of queries, keys and states, values and states whose second and third parts bf16 does not hold: the precision is
+# that of others, relative to what comes out (of about 1e-36: fp32 itself ends at 2^-149, 1e-9 of it)
+@pytest.mark.parametrize("sizes", [(1e-36, 1.0, 1.0, 1.0), (1.0, 1e-36, 1.0, 1e-36), (1.0, 1.0, 1e-36, 1e-36)])
+@pytest.mark.parametrize("mode,H,vdim,lens", [("gla", 2, 64, LENS), ("delta", 2, 64, LENS), ("gla", 8, 128, [2100]),
+                                              ("delta", 8, 128, [2100]), ("wkv", 3, 64, LENS), ("wkv bf16", 3, 64, LENS)])
+def test_small_operands(mode, H, vdim, lens, sizes):
+    if mode[:3] == "wkv":
+        (out, st), (out_w, st_w) = _wkv(torch.float32 if mode == "wkv" else torch.bfloat16, -2.0, sizes=sizes)
+    else:
+        (out, st), (out_w, st_w) = _linrec(mode, H, H, 64, vdim, torch.float32, 0.0, lens=lens, pad=4, sizes=sizes)
+    for got, want in ((out, out_w), (st, st_w)):
+        new = want.double().square().mean().sqrt()
+        _close(got.double() / float(new), want.double() / float(new), 1e-5 if got.dtype == torch.float32 else 2.0 ** -8)
+
+
+@pytest.mark.parametrize("mode", ["gla", "delta"])
+def test_small_operands_that_decays_leave(mode):
+    """Sixteen tokens without values read a state that decays take to 1e-37 of itself, each row to the precision of the first.
+    (Delta rule: without keys too, so that the rule leaves the state alone.)"""
+    g, H = torch.Generator().manual_seed(3), 2
+    q, k, v = torch.randn(16, H, 64, generator=g), torch.randn(16, H, 64, generator=g), torch.zeros(16, H, 64)
+    if mode == "delta":
+        k *= 0.0
+    z, st = torch.full((16, H * 64), 5.3), torch.randn(2, H, 64, 64, generator=g)
+    rows, runs = _rows([16], 23)
+    rows[3][:] += 23                                         # the run goes on from the state
+    beta = torch.zeros(16, H) if mode == "delta" else None
+
+    def call(dev, f, **more):
+        m = lambda x: None if x is None else x.to(dev)  # noqa: E731
+        out, s = torch.empty(16, H * 64, device=dev), m(st.clone())
+        f(m(q), m(k), m(v), m(z), m(torch.ones(H)), m(torch.zeros(H * 64)), 1.0, m(beta), m(torch.ones(16, H * 64)), mode == "delta",
+          m(torch.ones(64)), 1e-5, 1.0, s, *(m(r) for r in rows), out, **more)
+        return out.cpu().double()
+
+    got, want = call(DEV, ops.gated_linear_recurrence, run_rows=runs.to(DEV)), call("cpu", ref.gated_linear_recurrence)
+    # sixteen decays of e^-5.3, each to 2^-21 (exponent and exponential): 1e-5; the last row's 6e-37 ends at 2^-149
+    assert bool(((got - want).norm(dim=1) <= 2e-5 * want.norm(dim=1)).all())
 
 
 @pytest.mark.parametrize("value", [3.395e38, 1e-37])         # a part of three would round to infinity; parts below 2^-126
