@@ -1202,7 +1202,10 @@ __global__ __launch_bounds__(chunk_threads(MODE)) void chunk_recurrence_segments
 // head and 128 value channels: the producers' work, which 64 channels cost as much, is done half as often.
 // Two runs of 2,048 with 32 heads: 301 -> 82 + 89 us.  Error of the state against 64 bits as with whole runs (6.3e-8 to
 // 6.5e-8).  Unit keys and betas of at most 1 turn a state no larger.  Where an entry passes that (other keys, whose turns may
-// grow or overflow though the state does not), a run's second segment goes through to its end in sequence.
+// grow or overflow though the state does not), the rest of the run is gone through in sequence, by the workgroups of its second
+// segment and of its third (there is one: turns are of segments between others), 64 channels each, which take 2.1 us a chunk
+// for 128 channels' 2.7: two runs of 2,048 with 32 heads 284 us a call, one of 4,096 491 (as whole runs in fp32 products 319
+// and 596, in one go of 128 channels 352 and 638); four of 600 with 16 heads 106, 103 as whole runs.
 template <typename TI, typename TG>
 __global__ __launch_bounds__(chunk_threads(kChunkDelta)) void chunk_delta_first_kernel(const ChunkArgs a) {
   const ChunkSegment sg = find_segment<kChunkDelta, 2, kFirstSegments>(a, blockIdx.z, threadIdx.x & 63);
@@ -1219,12 +1222,17 @@ __global__ __launch_bounds__(chunk_threads(kChunkDelta)) void chunk_delta_later_
   const float* wild = delta_seg(a, sg.slot - sg.seg + 1, h).wild;        // of the run's second segment
   uint64_t any = 0;
   for (int x = lane; x < 4 * turns; x += 64) any |= wild[(int64_t)(x >> 2) * a.H * 4 + (x & 3)] != 0.f;
-  if (__builtin_amdgcn_ballot_w64(any != 0) != 0ull) {
-    if (sg.seg > 1) return;
+  if (__builtin_amdgcn_ballot_w64(any != 0) == 0ull) {
+    chunk_run<TI, TG, kChunkDelta, 2>(a, sg, h, blockIdx.y * 128, threadIdx.x);
+  } else if (sg.seg <= 2) {
+    const int part = sg.seg - 1;
+    sg.slot -= part;
+    sg.seg = 1;
+    sg.t0 = sg.run0 + sg.rows;
     sg.n = rows - sg.rows;
     sg.last = true;
+    chunk_run<TI, TG, kChunkDelta>(a, sg, h, blockIdx.y * 128 + 64 * part, threadIdx.x);
   }
-  chunk_run<TI, TG, kChunkDelta, 2>(a, sg, h, blockIdx.y * 128, threadIdx.x);
 }
 
 // Workgroups, one to a CU at most, that share the runs of min_run rows or more, which every wave counts for

@@ -235,8 +235,8 @@ def test_segments_beside_other_work():
     torch.cuda.synchronize()
 
 
-@pytest.mark.parametrize("size,row", [(3.0, 2100), (1e20, 1000)])
-def test_delta_rule_turns_that_grow(size, row):
+@pytest.mark.parametrize("size,row,vdim", [(3.0, 2100, 128), (1e20, 1000, 128), (3.0, 700, 256)])
+def test_delta_rule_turns_that_grow(size, row, vdim):
     """Keys that turn a state into a larger one, or a state of zeros into what no fp32 holds, leave segments to be done in
     sequence.  Few keys are not zero, so that the growth is not undone; the large one meets a channel that holds nothing."""
     def keys(k, v):
@@ -247,7 +247,7 @@ def test_delta_rule_turns_that_grow(size, row):
         k[row], v[row] = 0.0, 0.0
         k[row, :, 0] = size
 
-    (out, st), (out_w, st_w) = _linrec("delta", 2, 2, 64, 128, torch.float32, -9.0, lens=[1500, 900], keys=keys)
+    (out, st), (out_w, st_w) = _linrec("delta", 2, 2, 64, vdim, torch.float32, -9.0, lens=[1500, 900], keys=keys)
     # a norm of size^2 on a difference: 9 times the roundings of the state it reads
     _close(out, out_w, 1e-4)
     _close(st, st_w, 1e-4)
