@@ -1043,8 +1043,10 @@ bool launch_qk_norm_rotary_append(bool f32, const void* proj, int64_t stride, co
               v_cache, T, H, G, qw, kw, v_mode == 0 ? vdim : 0, BS, q_from, norm_all ? kw : k_norm_n, (int)neighbours, pool_slots, q_out, q_ts, q_hs, conv_w, conv_state, state_slots, row_state,
               row_back, row_fwd, 0};
     const int at_once = 256 * std::max(1, 12 * 64 / wide);
+    auto bytes_of = [&](int rows) { return (size_t)(2 * nrot * rows + 4 * (wide / 64) + 5 * rows) * 4; };
     a.rows = std::min(kQknRows, (T + at_once - 1) / at_once);
-    const size_t bytes = (size_t)(2 * nrot * a.rows + 4 * (wide / 64) + 5 * a.rows) * 4;
+    while (a.rows > 1 && bytes_of(a.rows) > (size_t)64 * 1024) --a.rows;     // a row's sines: 40 KB at most (10,240 columns)
+    const size_t bytes = bytes_of(a.rows);
     const dim3 grid((T + a.rows - 1) / a.rows);
 #define QKN_ROWS(TT, C, N) hipLaunchKernelGGL((qk_norm_rotary_append_rows_kernel<TT, C, N>), grid, dim3(wide), bytes, s, a)
     if (f32) {

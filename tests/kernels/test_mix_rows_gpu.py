@@ -151,3 +151,22 @@ def test_rotated_ends_and_a_partly_normed_key(dtype, H, qw, latent, rot, neighbo
     # as above
     for a, b, rel in zip(call(DEV, ops.qk_norm_rotary_append), call("cpu", ref.qk_norm_rotary_append), (0.0, 2.0 ** -7)):
         torch.testing.assert_close(a.cpu().float(), b.float(), atol=3e-5 if T < 100 else 4e-3, rtol=1e-5 + (rel if dtype == torch.bfloat16 else 0.0))
+
+
+def test_rotations_of_wide_heads_in_long_steps():
+    """512 sines a row of a step with sixteen rows a workgroup: they leave room for fewer."""
+    H, w, T, page = 8, 1024, 3850, 32
+    g = torch.Generator().manual_seed(1)
+    W, pages, slots = (H + 2) * w, T // page + 1, torch.arange(T, dtype=torch.int32)
+    proj, freq, pos = torch.randn(T, W, generator=g).bfloat16(), 1000.0 ** -torch.linspace(0, 1, w // 2), torch.arange(T, dtype=torch.int32) % 100
+
+    def call(dev, f):
+        m = lambda x: x.to(dev)  # noqa: E731
+        q = torch.empty(T, H, w, device=dev)
+        kc, vc = (torch.zeros(pages, 1, page, w, device=dev, dtype=torch.bfloat16) for _ in range(2))
+        f(m(proj), None, None, None, False, w, 1e-5, m(pos), m(freq), 1.0, 0, 0, m(slots), kc, vc, H, 1, w, w, w, 0, q, neighbours=True)
+        return q, kc, vc
+
+    # as above, angles of up to 100 radians
+    for a, b, rel in zip(call(DEV, ops.qk_norm_rotary_append), call("cpu", ref.qk_norm_rotary_append), (0.0, 2.0 ** -7, 2.0 ** -7)):
+        torch.testing.assert_close(a.cpu().float(), b.float(), atol=3e-4, rtol=1e-5 + rel)
