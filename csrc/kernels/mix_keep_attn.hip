@@ -1028,33 +1028,49 @@ bool launch_qk_norm_rotary_append(bool f32, const void* proj, int64_t stride, co
   const int turn = 2 * nrot;
   const bool lanes = nrot == 0 || neighbours || (turn <= 512 && (nrot & (nrot - 1)) == 0 && q_rot_off % turn == 0 && k_rot_off % turn == 0 &&
                                    qw % turn == 0 && kw % turn == 0);
-  // Two chunks a thread, one where a thread keeps the convolution's weights for it (two spill 30 registers).  Of rows beyond
-  // 8,192 columns, convolved, few are faster in the other kernel (80 heads of 128: 257 rows 15.0 us for 16.5, 1,024 34.2
-  // for 31.2); all others gain at every size.  32 + 8 + 8 heads of 128 in bf16: convolved 1 row 8.1 -> 7.3 us, 64 rows 9.3
-  // -> 7.9, 512 12.6 -> 9.5, 2,648 40.5 -> 29.3 (3.0 TB/s), 8,192 103 -> 85; with a bias 2,648 rows 28.7 -> 21.5.
-  // Latents (64 rotated entries of 32 heads, 576 of the key): 2,067 rows 15.2 -> 11.3, 8,192 44.3 -> 28.2.
-  const int per = conv_w != nullptr && W <= 8 * 1024 ? 1 : 2;
+  // Two chunks a thread, one where a thread keeps the convolution's weights for it (two spill 30 registers in bf16, 70 in
+  // fp32).  32 + 8 + 8 heads of 128 in bf16: convolved 1 row 8.1 -> 7.3 us, 64 rows 9.3 -> 7.9, 512 12.6 -> 9.5, 2,648 40.5 ->
+  // 29.3 (3.0 TB/s), 4,654 64 -> 55, 8,192 103 -> 85; with a bias 2,648 rows 28.7 -> 21.5.  Latents (64 rotated entries of 32
+  // heads, 576 of the key): 2,067 rows 15.2 -> 11.3, 8,192 44.3 -> 28.2.  Where it does not pay, measured from 256 to 10,240
+  // columns and 1 to 8,192 rows:
+  //   convolved, two chunks a thread: in fp32 never (64 + 8 + 8 heads, 2,067 rows 99 us for 73), in bf16 up to 9,216 columns
+  //   (4,654 rows 108 for 96) and few rows (10,240 columns: 257 rows 16.5 for 15.0, 1,024 31.2 for 34.2)
+  //   convolved in fp32, a single row of 6,144 columns and more: up to 1.09 times the other kernel's time
+  //   no norm, little to sum up: 64 rows of 3,072 columns 4.7 us for 4.4
+  //   fp32 without a convolution, four to eight waves of 134 registers, one such workgroup a CU: 824 rows of 6,144 columns 16.2
+  //   for 13.4, 2,067 32 for 26; ten waves 40 for 44
+  const bool conv = conv_w != nullptr;
+  const int per = conv && W <= 8 * 1024 ? 1 : 2;
   const int wide = (int)((W / 8 + per - 1) / per + 63) / 64 * 64;
   const bool one = norm_all || (q_norm_w == nullptr && (k_norm_w == nullptr || G == 1));     // norm of a kind's columns
+  auto pays = [&]() {
+    if (conv) return per == 1 ? !f32 || T >= 8 || W < 6144 : !f32 && W > 9216 && T >= 1024;
+    if (q_norm_w == nullptr && k_norm_w == nullptr &&
+        !(f32 ? T >= 2048 : T >= 1024 || (int64_t)T * (int64_t)W >= 1 << 20 || W >= 7168)) return false;
+    return !f32 || T <= 256 || wide <= 192 || W > 9216 || (wide >= 576 && T >= 2048);
+  };
   if (vec && lanes && one && G > 0 && v_mode != 1 && v_in == nullptr && v_out == nullptr &&
-      (conv_w == nullptr || (taps == kQknTaps && bias == nullptr && q_from == 0)) && wide <= (per == 1 ? 1024 : kQknThreads) &&
-      (conv_w == nullptr || per == 1 || T >= 1024)) {
+      (!conv || (taps == kQknTaps && bias == nullptr && q_from == 0)) && wide <= (per == 1 ? 1024 : kQknThreads) && pays()) {
     QknRows a{proj, stride, bias, q_norm_w, k_norm_w, eps, pos, inv_freq, nrot, rot_mult, q_rot_off, k_rot_off, slots, k_cache,
-              v_cache, T, H, G, qw, kw, v_mode == 0 ? vdim : 0, BS, q_from, norm_all ? kw : k_norm_n, (int)neighbours, pool_slots, q_out, q_ts, q_hs, conv_w, conv_state, state_slots, row_state,
-              row_back, row_fwd, 0};
-    const int at_once = 256 * std::max(1, 12 * 64 / wide);
+              v_cache, T, H, G, qw, kw, v_mode == 0 ? vdim : 0, BS, q_from, norm_all ? kw : k_norm_n, (int)neighbours, pool_slots,
+              q_out, q_ts, q_hs, conv_w, conv_state, state_slots, row_state, row_back, row_fwd, 0};
+    // Whole rounds of what the CUs take at a time (four waves a SIMD by their registers, three of those with 134), and rows
+    // of a workgroup so that the last round is full: 4,654 rows of 32 + 8 + 8 heads, convolved, ten by ten 55 us, in sixteens,
+    // 291 workgroups on 256 CUs, 77.
+    const int waves = wide / 64, simd = f32 && !conv ? 3 : 4;
+    const int at_once = 256 * std::max(1, waves < 4 ? 4 * simd / waves : simd / ((waves + 3) / 4));
+    const int rounds = (T + at_once * kQknRows - 1) / (at_once * kQknRows);
+    a.rows = (T + at_once * rounds - 1) / (at_once * rounds);
     auto bytes_of = [&](int rows) { return (size_t)(2 * nrot * rows + 4 * (wide / 64) + 5 * rows) * 4; };
-    a.rows = std::min(kQknRows, (T + at_once - 1) / at_once);
     while (a.rows > 1 && bytes_of(a.rows) > (size_t)64 * 1024) --a.rows;     // a row's sines: 40 KB at most (10,240 columns)
     const size_t bytes = bytes_of(a.rows);
     const dim3 grid((T + a.rows - 1) / a.rows);
 #define QKN_ROWS(TT, C, N) hipLaunchKernelGGL((qk_norm_rotary_append_rows_kernel<TT, C, N>), grid, dim3(wide), bytes, s, a)
     if (f32) {
-      if (conv_w == nullptr) QKN_ROWS(float, false, 2);
-      else if (per == 1) QKN_ROWS(float, true, 1);
-      else QKN_ROWS(float, true, 2);
+      if (conv) QKN_ROWS(float, true, 1);
+      else QKN_ROWS(float, false, 2);
     } else {
-      if (conv_w == nullptr) QKN_ROWS(bf16_t, false, 2);
+      if (!conv) QKN_ROWS(bf16_t, false, 2);
       else if (per == 1) QKN_ROWS(bf16_t, true, 1);
       else QKN_ROWS(bf16_t, true, 2);
     }

@@ -128,6 +128,12 @@ def test_norm_and_rotation_of_rows_one_after_another(dtype, conv, H, G, dim, nro
         torch.testing.assert_close(a.cpu().float(), b.float(), atol=3e-5 if T < 100 else 4e-3, rtol=1e-5 + (rel if dtype == torch.bfloat16 else 0.0))
 
 
+# More rows than one round of workgroups takes in sixteens: two rounds of eight or nine
+@pytest.mark.parametrize("T", [4096, 4104])
+def test_norm_and_rotation_of_rows_in_rounds(T):
+    test_norm_and_rotation_of_rows_one_after_another(torch.bfloat16, False, 64, 8, 128, 32, 64, T)
+
+
 # The same without values: the rotated ends of query heads, one key of which only the leading entries are normed
 @pytest.mark.parametrize("T", [3, 1030])
 @pytest.mark.parametrize("neighbours", [False, True])
