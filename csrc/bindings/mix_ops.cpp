@@ -12,6 +12,7 @@
 
 #include <functional>
 
+#include "../kernels/mix_chunk.h"
 #include "../kernels/mix_linrec.h"
 #include "../kernels/mix_mlstm.h"
 
@@ -517,6 +518,19 @@ std::function<float*(int64_t)> scratch_floats(const Tensor& like, Tensor& held) 
     held = at::empty({n}, like.options().dtype(at::kFloat));
     return held.data_ptr<float>();
   };
+}
+
+// How a step whose rows' places and strides all suit is shared: segments that its runs may be cut into at most (0: runs stay
+// whole), and waves that share one of them in the kernel before the recurrence's (delta rule: 1).
+std::vector<int64_t> recurrence_segments(int64_t mode, int64_t rows, int64_t runs, int64_t heads, int64_t dim, int64_t vdim) {
+  TORCH_CHECK(mode >= rfqmix::kChunkWkv && mode <= rfqmix::kChunkDelta && rows >= 1 && runs >= 1 && heads >= 1 && dim >= 1 && vdim >= 1,
+              "recurrence_segments: mode 0 wkv, 1 gated, 2 delta rule; sizes");
+  const int32_t none = -1;
+  rfqmix::ChunkArgs a{};
+  a.run_rows = &none;                                     // there is a list; nobody reads it here
+  a.runs = (int)runs; a.H = (int)heads; a.dim = (int)dim; a.vdim = (int)vdim;
+  a.cap = rfqmix::chunk_seg_cap((int)mode, true, (int)rows, a);
+  return {rfqmix::chunk_may_cut(a) ? a.cap : 0, a.unit / rfqmix::kChunkRows};
 }
 
 void wkv_recurrence(const Tensor& r, const Tensor& k, const Tensor& v, const Tensor& zw,
@@ -1259,6 +1273,7 @@ TORCH_LIBRARY(rfq_mix, m) {
   m.def("silu_mul_any(Tensor gate_up, Tensor(a!) out) -> ()");
   m.def("softcap(Tensor(a!) x, float cap) -> ()");
   m.def("matmul_short(Tensor x, Tensor w, bool out_f32) -> Tensor");
+  m.def("recurrence_segments(int mode, int rows, int runs, int heads, int dim, int vdim) -> int[]", &recurrence_segments);
   m.def("bmm_short(Tensor a, Tensor b, Tensor(c!) out) -> ()");
   m.def("token_shift_mix(Tensor x, Tensor mu, Tensor(a!) prev, Tensor row_state, Tensor row_back, Tensor row_fwd, Tensor pos, Tensor(b!) out) -> ()");
   m.def("wkv_recurrence(Tensor r, Tensor k, Tensor v, Tensor zw, Tensor w0, Tensor u, Tensor gate, Tensor norm_w, float eps, Tensor(a!) state, Tensor row_state, Tensor row_back, Tensor row_fwd, Tensor pos, Tensor? run_rows, Tensor(b!) out) -> ()");

@@ -6,6 +6,7 @@
 namespace rfqmix {
 
 constexpr int kChunkDim = 64;          // most key channels
+constexpr int kChunkRows = 16;         // tokens of a chunk
 enum ChunkMode { kChunkWkv = 0, kChunkGla = 1, kChunkDelta = 2 };
 
 struct ChunkArgs {

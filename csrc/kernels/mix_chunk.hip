@@ -51,7 +51,7 @@ namespace rfqmix {
 using rfq::f32x4;
 
 namespace {
-constexpr int CT = 16;                  // tokens per chunk
+constexpr int CT = kChunkRows;          // tokens per chunk
 constexpr int NC = kChunkDim;           // key channels (those past dim are zeros)
 constexpr int RS = NC + 4;              // floats per token row in LDS
 constexpr int TS = CT + 4;              // floats per row of a 16 x 16 tile

@@ -104,8 +104,8 @@ def test_a_non_finite_value_stays_out_of_earlier_tokens(mode, value):
     _close(out[sum(LENS[:8]):], out_w[sum(LENS[:8]):], 1e-5)  # and no other run sees it
 
 
-def _wkv(dtype, shift, spoil=None, lens=LENS, sizes=(1.0, 1.0, 1.0, 1.0)):
-    H, N = 3, 64
+def _wkv(dtype, shift, spoil=None, lens=LENS, sizes=(1.0, 1.0, 1.0, 1.0), H=3):
+    N = 64
     g = torch.Generator().manual_seed(5)
     T = sum(lens)
     r, k, v, zw, gate = (torch.randn(T, H * N, generator=g) for _ in range(5))
@@ -141,51 +141,101 @@ def test_wkv_non_finite_value_stays_out_of_earlier_tokens():
     _close(out[sum(LENS[:8]):], out_w[sum(LENS[:8]):], 1e-5)
 
 
-# Runs in segments of 128 tokens (a state's way into a segment is one more sum and product a segment): ends just before,
-# at and behind a segment's end, runs that begin and that go on, states of several segments back; rows of wider
-# tensors that a segment's loads of four fit (a pad of 4) and that they do not (3: whole runs).
-SEGMENTS = [700, 1, 129, 128, 255, 257, 400]
+def _cut(mode, H, vdim, lens, waves=8):
+    """The host lets the step's runs be cut (the list of runs has an entry of -1 more); waves of the kernel before the
+    recurrence's that share a segment."""
+    kind = {"wkv": 0, "gla": 1, "delta": 2}[mode]
+    got = torch.ops.rfq_mix.recurrence_segments(kind, sum(lens), len(lens) + 1, H, 64, vdim)
+    return got[0] > len(lens) + 1 and got[1] == (1 if mode == "delta" else waves)
+
+
+# 1e-5 is for sums of up to 150 tokens; where decays are near one, roundings add up with the root of their number, in the
+# reference (one sum a token) as here
+def _tol(lens, shift):
+    return 1e-5 * max(1.0, max(lens) / 150) ** 0.5 if shift < 0 else 1e-5
+
+
+# Runs in segments of 128 tokens, which is what the device takes for SEGMENTS and as few heads as here (a state's way into a
+# segment is one more sum and product a segment): ends just before, at and behind a segment's end, runs that begin and that
+# go on, states of several segments back; rows of wider tensors that a segment's loads of four fit (a pad of 4) and that they
+# do not (3: whole runs).  WHOLE: too short, on the average, for the host to cut.
+SEGMENTS = [1535, 256, 513, 129, 127]
+WHOLE = [700, 1, 129, 128, 255, 257, 400]
+
+
+def test_which_steps_are_cut():
+    for H, vdim in ((2, 64), (4, 128)):
+        assert _cut("gla", H, vdim, SEGMENTS) and not _cut("gla", H, vdim, WHOLE)
+    assert _cut("wkv", 3, 64, SEGMENTS) and not _cut("wkv", 3, 64, WHOLE)
+    assert not _cut("gla", 2, 96, SEGMENTS) and not _cut("delta", 2, 64, SEGMENTS)
+    got = torch.ops.rfq_mix.recurrence_segments(1, 2070, 8, 32, 64, 128)
+    assert got[0] == 0                                        # as many entries as segments fit: runs stay whole
 
 
 @pytest.mark.parametrize("shift", [-6.0, 0.0, 60.0])      # decays near one over segments, ordinary, all but zero
 @pytest.mark.parametrize("H,Hq,vdim,pad", [(2, 2, 64, 4), (4, 2, 128, 0), (2, 2, 64, 3)])
-def test_linear_recurrence_in_segments(H, Hq, vdim, pad, shift):
-    (out, st), (out_w, st_w) = _linrec("gla", H, Hq, 64, vdim, torch.float32, shift, lens=SEGMENTS, pad=pad)
-    _close(out, out_w, 1e-5)
-    _close(st, st_w, 1e-5)
+@pytest.mark.parametrize("lens", [SEGMENTS, WHOLE])
+def test_linear_recurrence_in_segments(lens, H, Hq, vdim, pad, shift):
+    (out, st), (out_w, st_w) = _linrec("gla", H, Hq, 64, vdim, torch.float32, shift, lens=lens, pad=pad)
+    _close(out, out_w, _tol(lens, shift))
+    _close(st, st_w, _tol(lens, shift))
 
 
-@pytest.mark.parametrize("lens", [SEGMENTS, [4096 + 40]])     # 4,136: segments of a sixteenth a wave where heads are many
+@pytest.mark.parametrize("lens", [SEGMENTS, WHOLE, [4096 + 40]])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_wkv_in_segments(dtype, lens):
-    # 1e-5 is for sums of up to 150 tokens; where decays are near one, roundings add up with the root of their number,
-    # in the reference (one sum a token) as here
-    tol = 1e-5 * (max(lens) / 150) ** 0.5
+    tol = 1e-5 * (max(lens) / 150) ** 0.5                    # as above, whatever the decays
     for shift in (-6.0, -2.0, 5.0):
         (out, st), (out_w, st_w) = _wkv(dtype, shift, lens=lens)
         _close(out, out_w, tol if dtype == torch.float32 else 2.0 ** -8)
         _close(st, st_w, tol)
 
 
-def test_linear_recurrence_in_segments_bf16():
-    (out, st), (out_w, st_w) = _linrec("gla", 2, 2, 64, 128, torch.bfloat16, 0.0, lens=SEGMENTS, pad=4)
+# Sixteen waves to a segment (heads are many, runs long): segments of 1,280 rows, whose last ones are shorter
+@pytest.mark.parametrize("mode,H,vdim,lens,dtype", [("wkv", 64, 64, [4136], torch.bfloat16), ("wkv", 40, 64, [3333, 2900], torch.float32),
+                                                    ("gla", 64, 128, [4136], torch.bfloat16), ("gla", 40, 64, [3333, 2900], torch.float32)])
+def test_segments_of_sixteen_waves(mode, H, vdim, lens, dtype):
+    assert _cut(mode, H, vdim, lens, 16)
+    for shift in (-6.0, 0.0):
+        (out, st), (out_w, st_w) = (_wkv(dtype, shift, lens=lens, H=H) if mode == "wkv" else
+                                    _linrec(mode, H, H, 64, vdim, dtype, shift, lens=lens, pad=4))
+        tol = 1e-5 * (max(lens) / 150) ** 0.5
+        if dtype == torch.float32:
+            _close(out, out_w, tol)
+        else:
+            # 34 million values up to 10 times the rms: where two sums round to different sides, the neighbouring bf16 value,
+            # up to 2^-7 of the value away; the sums' own difference is 8 tol of the rms as in fp32
+            got, want = out.cpu().double(), out_w.double()
+            rms = float(want.square().mean().sqrt())
+            assert bool(((got - want).abs() <= 2.0 ** -7 * want.abs() + 8 * tol * max(1.0, rms)).all())
+            assert float((got - want).square().mean().sqrt()) <= 2.0 ** -8 * rms
+        _close(st, st_w, tol)
+
+
+@pytest.mark.parametrize("mode,H,vdim,lens", [("gla", 2, 128, SEGMENTS), ("gla", 2, 64, SEGMENTS), ("delta", 2, 128, [1500, 33, 700])])
+def test_linear_recurrence_in_segments_bf16(mode, H, vdim, lens):
+    assert _cut(mode, H, vdim, lens)
+    (out, st), (out_w, st_w) = _linrec(mode, H, H, 64, vdim, torch.bfloat16, 0.0, lens=lens, pad=4)
     _close(out, out_w, 2.0 ** -8)
     _close(st, st_w, 1e-5)
 
 
-def test_a_non_finite_value_stays_out_of_earlier_segments():
-    (out, _), (out_w, _) = _linrec("gla", 2, 2, 64, 64, torch.float32, 0.0, lens=SEGMENTS, spoil=(300, 3, float("inf")), pad=4)
+@pytest.mark.parametrize("lens,other", [(SEGMENTS, 1535), (WHOLE, 700)])
+def test_a_non_finite_value_stays_out_of_earlier_segments(lens, other):
+    (out, _), (out_w, _) = _linrec("gla", 2, 2, 64, 64, torch.float32, 0.0, lens=lens, spoil=(300, 3, float("inf")), pad=4)
     _close(out[:300], out_w[:300], 1e-5)
-    _close(out[700:], out_w[700:], 1e-5)
+    _close(out[other:], out_w[other:], 1e-5)
 
 
 # The delta rule's segments are whole chunks, as many as the chip has room for: runs of several, of one, of less than one
-# and of a chunk, a single long one; states carried through turns of 64 x 64
+# and of a chunk, a single long one, all of them whole (the first list); states carried through turns of 64 x 64
 @pytest.mark.parametrize("shift", [-6.0, 0.0, 60.0])
-@pytest.mark.parametrize("H,Hq,vdim,lens", [(2, 2, 128, [1500, 33, 16, 700]), (4, 2, 128, [2100]), (1, 1, 256, [513, 1024])])
+@pytest.mark.parametrize("H,Hq,vdim,lens", [(2, 2, 128, [1500, 33, 16, 700]), (2, 2, 128, [1500, 33, 700]), (2, 2, 128, [1600, 16]),
+                                            (4, 2, 128, [2100]), (1, 1, 256, [513, 1024])])
 def test_delta_rule_in_segments(H, Hq, vdim, lens, shift):
+    assert _cut("delta", H, vdim, lens) == (len(lens) < 4)
     (out, st), (out_w, st_w) = _linrec("delta", H, Hq, 64, vdim, torch.float32, shift, lens=lens)
-    tol = 1e-5 * (max(lens) / 150) ** 0.5 if shift < 0 else 1e-5        # as for wkv above
+    tol = _tol(lens, shift)
     _close(out, out_w, tol)
     _close(st, st_w, tol)
 
