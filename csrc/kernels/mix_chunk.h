@@ -27,7 +27,7 @@ struct ChunkArgs {
   void* out;                        // [T, H vdim] contiguous (wkv)
   float* state;                     // [2 slots, H, dim, vdim]
   const int32_t *row_state, *row_back, *row_fwd, *pos, *run_rows;
-  int runs, H, rep, dim, vdim, slots, T;
+  int runs, H, rep, dim, vdim, slots;
   int min_run;                      // shorter runs are left alone
   int cap = 0, per = 0, unit = 0;   // segments of runs that the step is shared in at most (0: whole runs), workgroups of
                                     // each, and what divides their rows

@@ -504,7 +504,7 @@ void launch_gated_linrec(bool in_f32, bool act_f32, bool delta, const LinrecArgs
     c.raw = a.raw; c.state = a.state;
     c.row_state = a.row_state; c.row_back = a.row_back; c.row_fwd = a.row_fwd; c.pos = a.pos;
     c.run_rows = a.run_rows; c.runs = a.runs; c.H = a.H; c.rep = a.rep; c.dim = a.dim; c.vdim = a.vdim;
-    c.slots = a.slots; c.T = a.T;
+    c.slots = a.slots;
     const int mode = delta ? kChunkDelta : kChunkGla;
     a.below = c.min_run = chunk_min_run(mode, a.T, c);
     if ((c.cap = chunk_seg_cap(mode, in_f32, a.T, c)) > 0) c.seg = scratch(chunk_seg_floats(mode, c));

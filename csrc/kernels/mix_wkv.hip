@@ -256,7 +256,7 @@ void launch_wkv_recurrence(bool f32, const void* r, const void* k, const void* v
   a.zbias = w0; a.u = u; a.norm_w = norm_w; a.eps = eps; a.q_scale = 1.f;
   a.out = out; a.state = state;
   a.row_state = row_state; a.row_back = row_back; a.row_fwd = row_fwd; a.pos = pos; a.run_rows = run_rows;
-  a.runs = runs; a.H = H; a.rep = 1; a.dim = a.vdim = N; a.slots = slots; a.T = Trows;
+  a.runs = runs; a.H = H; a.rep = 1; a.dim = a.vdim = N; a.slots = slots;
   const int below = a.min_run = chunk_min_run(kChunkWkv, Trows, a);
   if ((a.cap = chunk_seg_cap(kChunkWkv, f32, Trows, a)) > 0) a.seg = scratch(chunk_seg_floats(kChunkWkv, a));
   if (below < INT32_MAX) launch_chunk(kChunkWkv, f32, f32, Trows, a, s);
