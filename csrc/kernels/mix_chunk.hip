@@ -573,18 +573,18 @@ __device__ __forceinline__ void chunk_run(const ChunkArgs& a, const ChunkSegment
         }
       }
       const float down = odd ? 1.f : kDown;
-      if constexpr (!TURN)
+      f32x4 own[NT];                                      // read-outs of the chunk's own tokens
 #pragma unroll
-        for (int j = 0; j < NT; ++j) o[j] *= down;
+      for (int j = 0; j < NT; ++j) own[j] = (f32x4){0.f, 0.f, 0.f, 0.f};
       if constexpr (DELTA) {
         const float4 bt = ld4(&L.beta[b][4 * grp]), ta = ld4(&L.tt[it & 1][col * TS + 4 * grp]);
         f32x4 x[NT];
         bool whole = true;
 #pragma unroll
         for (int j = 0; j < NT; ++j) {
-          const f32x4 own = j < NV ? (f32x4){v[j % NV][0], v[j % NV][1], v[j % NV][2], v[j % NV][3]} : (f32x4){0.f, 0.f, 0.f, 0.f};
-          x[j] = (f32x4){bt.x * fmaf(-down, y[j][0], own[0]), bt.y * fmaf(-down, y[j][1], own[1]),
-                         bt.z * fmaf(-down, y[j][2], own[2]), bt.w * fmaf(-down, y[j][3], own[3])};
+          const f32x4 val = j < NV ? (f32x4){v[j % NV][0], v[j % NV][1], v[j % NV][2], v[j % NV][3]} : (f32x4){0.f, 0.f, 0.f, 0.f};
+          x[j] = (f32x4){bt.x * fmaf(-down, y[j][0], val[0]), bt.y * fmaf(-down, y[j][1], val[1]),
+                         bt.z * fmaf(-down, y[j][2], val[2]), bt.w * fmaf(-down, y[j][3], val[3])};
           u[j] = (f32x4){0.f, 0.f, 0.f, 0.f};
           whole = whole && finite4(x[j]);
         }
@@ -629,7 +629,7 @@ __device__ __forceinline__ void chunk_run(const ChunkArgs& a, const ChunkSegment
       if (__builtin_amdgcn_ballot_w64(!fits) != 0ull && bad()) {
 #pragma unroll
         for (int j = 0; j < NT; ++j) {
-          if constexpr (!TURN) lower_product(L.aq[b], u[j], col, grp, o[j]);
+          if constexpr (!TURN) lower_product(L.aq[b], u[j], col, grp, own[j]);
 #pragma unroll
           for (int i = 0; i < 4; ++i) {
             const float down = L.odd[b][i] == kOddSmall ? kDownKd : 1.f;
@@ -645,13 +645,13 @@ __device__ __forceinline__ void chunk_run(const ChunkArgs& a, const ChunkSegment
         if constexpr (!TURN) {
           const float4 aa = ld4(&L.aq[b][col * TS + 4 * grp]);
 #pragma unroll
-          for (int j = 0; j < NT; ++j) o[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(aa.x, u[j][0], o[j], 0, 0, 0);
+          for (int j = 0; j < NT; ++j) own[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(aa.x, u[j][0], own[j], 0, 0, 0);
 #pragma unroll
-          for (int j = 0; j < NT; ++j) o[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(aa.y, u[j][1], o[j], 0, 0, 0);
+          for (int j = 0; j < NT; ++j) own[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(aa.y, u[j][1], own[j], 0, 0, 0);
 #pragma unroll
-          for (int j = 0; j < NT; ++j) o[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(aa.z, u[j][2], o[j], 0, 0, 0);
+          for (int j = 0; j < NT; ++j) own[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(aa.z, u[j][2], own[j], 0, 0, 0);
 #pragma unroll
-          for (int j = 0; j < NT; ++j) o[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(aa.w, u[j][3], o[j], 0, 0, 0);
+          for (int j = 0; j < NT; ++j) own[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(aa.w, u[j][3], own[j], 0, 0, 0);
         }
         // a lane's eight are two parts of four tokens: (l h + h l), (h m + m m), (h h + m h)
         uint4 kh[4][2];
@@ -679,6 +679,11 @@ __device__ __forceinline__ void chunk_run(const ChunkArgs& a, const ChunkSegment
           for (int i = 0; i < 4; ++i) st[j][i] = mma32(kh[i][0], hh, st[j][i]);
         }
       }
+      if constexpr (!TURN)
+#pragma unroll
+        for (int j = 0; j < NT; ++j)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) o[j][r] = fmaf(o[j][r], down, own[j][r]);
       values(min(it + 1, nc - 1));
       __builtin_amdgcn_sched_barrier(0);
       if constexpr (WKV) {
@@ -739,7 +744,7 @@ __device__ __forceinline__ void chunk_run(const ChunkArgs& a, const ChunkSegment
         // the products of the blocks grp ^ 1, grp ^ 2, grp ^ 3 from the lanes that hold them
         const float b1 = __shfl_xor(up[3], 16, 64), b2 = __shfl_xor(up[3], 32, 64), b3 = __shfl_xor(b1, 32, 64);
         const float b23 = b2 * b3;
-        const float pre = ((grp & 1) ? b1 * kUp : kUp) * ((grp & 2) ? b23 : 1.f);
+        const float pre = ((grp & 1) ? b1 : 1.f) * ((grp & 2) ? b23 : 1.f);
         const float post = ((grp & 1) ? 1.f : b1) * ((grp & 2) ? 1.f : b23);
         if (grp == 0) L.dec[b][ch] = up[3] * post;
         L.blk[e][grp * NC + ch] = up[3];
@@ -770,15 +775,10 @@ __device__ __forceinline__ void chunk_run(const ChunkArgs& a, const ChunkSegment
         }
         // as a rule the last four tokens say that a channel's keys are not too small
         uint32_t odd = 0;
-        if (__builtin_amdgcn_ballot_w64(!((sizes + most < kSplitMost) & (sizes >= least))) != 0ull) {
-          if (__builtin_amdgcn_ballot_w64(!(sizes + most < kSplitMost)) != 0ull) {
+        const float all = fmaf(most, kUp, sizes);
+        if (__builtin_amdgcn_ballot_w64(!((all < kSplitMost) & (sizes >= least))) != 0ull) {
+          if (__builtin_amdgcn_ballot_w64(!(all < kSplitMost)) != 0ull) {
             odd = kOddLarge;
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-              const int at = (4 * grp + i) * RS + ch;
-              if constexpr (!TURN) qd[i] = L.ql[e][at] * (pre * kDown);
-              if constexpr (DELTA) kk[i] = L.kb[e][at] * (pre * kDown);
-            }
           } else if (__builtin_amdgcn_ballot_w64(small_column(sizes)) != 0ull) {
             odd = kOddSmall;
 #pragma unroll
@@ -786,7 +786,7 @@ __device__ __forceinline__ void chunk_run(const ChunkArgs& a, const ChunkSegment
           }
         }
         if (lane == 0) L.odd[b][w] = odd;
-        auto put = [&](auto split) {
+        auto put = [&](auto split, float up) {
           const Split2 p = split(kd[0], kd[1]), q = split(kd[2], kd[3]);
           uint4* to = reinterpret_cast<uint4*>(&L.kd[b][ch * PS + 16 * grp]);
           to[0] = make_uint4(p.h, q.h, p.m, q.m);
@@ -802,12 +802,12 @@ __device__ __forceinline__ void chunk_run(const ChunkArgs& a, const ChunkSegment
                 part[y][at + (i + 1) * PS] = (uint16_t)(f[y] >> 16);
               }
             };
-            if constexpr (!TURN) rows(L.qd[b], split(qd[i], qd[i + 1]));
-            if constexpr (DELTA) rows(L.kk[b], split(kk[i], kk[i + 1]));
+            if constexpr (!TURN) rows(L.qd[b], split(qd[i] * up, qd[i + 1] * up));
+            if constexpr (DELTA) rows(L.kk[b], split(kk[i] * up, kk[i + 1] * up));
           }
         };
-        if (odd == kOddLarge) put([](float x, float y) { return odd_split(x, y); });
-        else put([](float x, float y) { return split3(x, y); });
+        if (odd == kOddLarge) put([](float x, float y) { return odd_split(x, y); }, 1.f);
+        else put([](float x, float y) { return split3(x, y); }, kUp);
       }
       __syncthreads();
     }
