@@ -523,8 +523,8 @@ std::function<float*(int64_t)> scratch_floats(const Tensor& like, Tensor& held) 
 // How a step whose rows' places and strides all suit is shared: segments that its runs may be cut into at most (0: runs stay
 // whole), and waves that share one of them in the kernel before the recurrence's (delta rule: 1).
 std::vector<int64_t> recurrence_segments(int64_t mode, int64_t rows, int64_t runs, int64_t heads, int64_t dim, int64_t vdim) {
-  TORCH_CHECK(mode >= rfqmix::kChunkWkv && mode <= rfqmix::kChunkDelta && rows >= 1 && runs >= 1 && heads >= 1 && dim >= 1 && vdim >= 1,
-              "recurrence_segments: mode 0 wkv, 1 gated, 2 delta rule; sizes");
+  TORCH_CHECK(mode >= rfqmix::kChunkWkv && mode <= rfqmix::kChunkDelta, "recurrence_segments: mode 0 wkv, 1 gated, 2 delta rule");
+  for (int64_t n : {rows, runs, heads, dim, vdim}) TORCH_CHECK(n >= 1 && n <= INT32_MAX, "recurrence_segments: sizes");
   const int32_t none = -1;
   rfqmix::ChunkArgs a{};
   a.run_rows = &none;                                     // there is a list; nobody reads it here

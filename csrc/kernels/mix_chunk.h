@@ -38,7 +38,8 @@ struct ChunkArgs {
 // How a step of T rows is shared: runs of at least this many rows go to the chunked kernel, the
 // others to the token-by-token one (1: all in chunks, INT32_MAX: none).
 int chunk_min_run(int mode, int T, const ChunkArgs& a);
-// Segments that the step's runs are shared in at most where they are, else 0 (sets a.per and a.unit), and the scratch floats of a.cap.
+// Segments that the step's runs are shared in at most where they are, else 0 (sets a.per and a.unit), and the scratch floats
+// of a.cap.
 int chunk_seg_cap(int mode, bool in_f32, int T, ChunkArgs& a);
 int64_t chunk_seg_floats(int mode, const ChunkArgs& a);
 // Whether the kernels may cut a run: the device's choice of segments and the launches that it needs go by this alone.

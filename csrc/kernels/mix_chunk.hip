@@ -20,9 +20,10 @@
 // state's products in it the decay waves stood for as long as they took, 2.3 us a chunk of the delta rule.)  The state's
 // products, 48 of 56 a wave, therefore go to the matrix cores in bf16: an fp32 operand is the exact sum of three bf16, six
 // products of them leave out at most 2^-24 of each (split3).  Operands at the ends of bf16's range have ways of their own
-// (kUp, kSplitLeast, odd_split), which cost 2 us of wkv's 100.  Those inside a chunk stay in fp32 MFMA: pairs of blocks on
-// tiles of 4x4x1, whose sixteen side by side take 64 channels of one pair in 32 clocks (16x16x4 made all pairs of a distance
-// and sixteen more each, 512: wkv 172 -> 164 us a pass, delta 276 -> 265).  Errors against 64 bits: state of the delta rule 6.3e-8 for 6.4e-8 before, outputs of gla in fp32 5.7e-7 and of wkv 2.0e-7, the same.
+// (kUp, kSplitLeast, odd_split), which cost 1 us of wkv's 100.  Those inside a chunk stay in fp32 MFMA: pairs of blocks on
+// tiles of 4x4x1, whose sixteen side by side take 64 channels of one pair in 32 clocks (16x16x4, which made all pairs of a
+// distance and sixteen more each in 512: 4 - 5 % more a pass).  Errors against 64 bits: state of the delta rule 6.3e-8 for
+// 6.4e-8 in fp32 products, outputs of gla in fp32 5.7e-7 and of wkv 2.0e-7, the same.
 // One workgroup per (run, head, 64 or 128 value channels): four consumer waves hold 64 x 16 of the state, or twice that, in
 // accumulators, which are MFMA operands as they lie (a lane holds channels 16 i + 4 grp + r of its column); the other
 // waves work ahead: decays, their products and parts for chunk c + 3, A for chunk c + 2, T for chunk c + 1, wkv's norm
@@ -36,7 +37,8 @@
 // segments at once, and a segment's workgroup begins from the state of before the run carried through those in front of
 // it.  What bounds the first kernel: exponentials (22 instructions a decay, 38 of gla) and the way to its first rows and
 // out, 10 us of a workgroup.  The delta rule's first kernel makes matrices of 64 x 64 in place of the products
-// (chunk_delta_first_kernel).  One run of 4,096: delta, 32 heads, 665 -> 299 us a pass, gla 430 -> 172, wkv, 64, 423 -> 196.
+// (chunk_delta_first_kernel).  One run of 4,096, whole runs in fp32 products before, all kernels of a layer's pass: delta, 32
+// heads, 668 -> 295 us, gla in fp32 449 -> 182, wkv, 64 heads, 425 -> 182.
 #include <algorithm>
 #include <cmath>
 #include <type_traits>
@@ -176,7 +178,9 @@ __device__ __forceinline__ bool within(float x, float lo, float hi) {
   return __float_as_uint(x) - __float_as_uint(lo) < __float_as_uint(hi) - __float_as_uint(lo);
 }
 __device__ __forceinline__ float sum_of_sizes(const f32x4& x) { return (fabsf(x[0]) + fabsf(x[1])) + (fabsf(x[2]) + fabsf(x[3])); }
-__device__ __forceinline__ float largest(const f32x4& x) { return fmaxf(fmaxf(fabsf(x[0]), fabsf(x[1])), fmaxf(fabsf(x[2]), fabsf(x[3]))); }
+__device__ __forceinline__ float largest(const f32x4& x) {
+  return fmaxf(fmaxf(fabsf(x[0]), fabsf(x[1])), fmaxf(fabsf(x[2]), fabsf(x[3])));
+}
 
 // o[t] += sum_{s<=t} m[t][s] x[s] with the pairs s > t left out instead of multiplied by zero: a
 // token's infinity or NaN stays out of the tokens before it.  (Also taken, with the same result,
@@ -232,8 +236,12 @@ __device__ __forceinline__ int segment_rows(const ChunkArgs& a, int n, int lane)
   auto rounds = [&](int segments) { return (float)((segments * a.per + 255) / 256); };
   const float c = (float)((min(rows, longest) + CT - 1) / CT);
   float t;
-  if constexpr (DELTA) t = rounds(all - cut) * (9.f + 2.7f * c) + (all > runs ? 3.f + rounds(all - runs) * (11.f + 2.8f * c) + 3.f * (most - 2) : 0.f);
-  else t = rounds(all) * (6.f + (MODE == kChunkWkv ? 1.45f : NV == 1 ? 1.65f : 2.f) * c) + (all > runs ? 10.f + 0.25f * c + 0.8f * most : 0.f);
+  if constexpr (DELTA)
+    t = rounds(all - cut) * (9.f + 2.7f * c) +
+        (all > runs ? 3.f + rounds(all - runs) * (11.f + 2.8f * c) + 3.f * (most - 2) : 0.f);
+  else
+    t = rounds(all) * (6.f + (MODE == kChunkWkv ? 1.45f : NV == 1 ? 1.65f : 2.f) * c) +
+        (all > runs ? 10.f + 0.25f * c + 0.8f * most : 0.f);
   const bool may = lane == 0 || (chunk_may_cut(a) && (DELTA ? all - cut : all) <= a.cap);
   uint32_t best = may ? (__float_as_uint(t) & ~63u) | (uint32_t)lane : ~0u;
 #pragma unroll
@@ -332,7 +340,8 @@ __device__ __forceinline__ void chunk_run(const ChunkArgs& a, const ChunkSegment
 #pragma unroll
     for (int r = 0; r < 4; ++r)
 #pragma unroll
-      for (int j = 0; j < NV; ++j) vreg[j][r] = load_at(vb, vo[r] + (uint32_t)((min(vcol + 16 * j, vdim - 1) - min(vcol, vdim - 1)) * sizeof(TI)));
+      for (int j = 0; j < NV; ++j)
+        vreg[j][r] = load_at(vb, vo[r] + (uint32_t)((min(vcol + 16 * j, vdim - 1) - min(vcol, vdim - 1)) * sizeof(TI)));
   };
   // ---- producers: a lane has four tokens of one key channel
   const int ch = 16 * w + col, chl = min(ch, dim - 1);
@@ -1041,9 +1050,9 @@ __device__ __forceinline__ void arrived4(uint2 x, float* f) {
 }
 
 // What a segment's rows leave of a state of zeros, and the products of its decays: for every segment but a run's last,
-// one workgroup per segment, head, 32 key and 64 value channels.  A wave has an eighth (a sixteenth) of the rows and goes through them
-// from the last chunk to the first, the keys times all decays behind them: nothing is rescaled, and the lane that makes
-// such a product (four tokens of two key channels) has it as the MFMA operand.  No LDS but to add the waves' parts up.
+// one workgroup per segment, head, 32 key and 64 value channels.  A wave has an eighth (a sixteenth) of the rows and goes
+// through them from the last chunk to the first, the keys times all decays behind them: nothing is rescaled, and the lane
+// that makes such a product (four tokens of two key channels) has it as the MFMA operand.  No LDS but to add the waves' parts.
 constexpr int kSegKeys = 32;
 template <typename TI, int MODE, int NV, int kSegWaves>
 __global__ __launch_bounds__(64 * kSegWaves, 4) void chunk_segment_kernel(const ChunkArgs a) {
@@ -1202,10 +1211,10 @@ __global__ __launch_bounds__(chunk_threads(MODE)) void chunk_recurrence_segments
 // head and 128 value channels: the producers' work, which 64 channels cost as much, is done half as often.
 // Two runs of 2,048 with 32 heads: 301 -> 82 + 89 us.  Error of the state against 64 bits as with whole runs (6.3e-8 to
 // 6.5e-8).  Unit keys and betas of at most 1 turn a state no larger.  Where an entry passes that (other keys, whose turns may
-// grow or overflow though the state does not), the rest of the run is gone through in sequence, by the workgroups of its second
-// segment and of its third (there is one: turns are of segments between others), 64 channels each, which take 2.1 us a chunk
-// for 128 channels' 2.7: two runs of 2,048 with 32 heads 284 us a call, one of 4,096 491 (as whole runs in fp32 products 319
-// and 596, in one go of 128 channels 352 and 638); four of 600 with 16 heads 106, 103 as whole runs.
+// grow or overflow though the state does not), the rest of the run is gone through in sequence, by the workgroups of its
+// second segment and of its third (there is one: turns are of segments between others), 64 channels each, which take 2.1 us
+// a chunk for 128 channels' 2.7: two runs of 2,048 with 32 heads 284 us a call, one of 4,096 491 (as whole runs in fp32
+// products 319 and 596, in one go of 128 channels 352 and 638); four of 600 with 16 heads 106, 103 as whole runs.
 template <typename TI, typename TG>
 __global__ __launch_bounds__(chunk_threads(kChunkDelta)) void chunk_delta_first_kernel(const ChunkArgs a) {
   const ChunkSegment sg = find_segment<kChunkDelta, 2, kFirstSegments>(a, blockIdx.z, threadIdx.x & 63);
@@ -1284,9 +1293,10 @@ __global__ __launch_bounds__(chunk_threads(MODE)) void chunk_recurrence_share_ke
 }
 
 // ------------------------------------------------------------------ launcher
-// A workgroup costs some 8 us before its first chunk is out and 1.6 - 2.3 us a chunk (now 1.45 - 2.1), one to a CU; the
-// token-by-token kernels some 6 us and 0.2 (64 runs) - 2.6 us a token, many to a CU.  Times below are of whole
-// steps, 32 heads of 64 x 128 (wkv: 64 of 64 x 64), chunks against tokens.
+// A workgroup costs some 8 us before its first chunk is out and 1.45 - 2.1 us a chunk (1.6 - 2.3 with the state's products
+// in fp32, which the times below are of: the lines are on the safe side), one to a CU; the token-by-token kernels some 6 us
+// and 0.2 (64 runs) - 2.6 us a token, many to a CU.  Times of whole steps, 32 heads of 64 x 128 (wkv: 64 of 64 x 64), chunks
+// against tokens.
 // Two workgroups to a CU or fewer: everything in chunks from 8 rows a run on (one run of 8: gla 14 us against 25,
 // delta 14 against 28, wkv 8 against 24).
 // More: a step's runs, decode rows beside prompts as a rule, are shared by their length (64 decode rows beside

@@ -1026,8 +1026,9 @@ bool launch_qk_norm_rotary_append(bool f32, const void* proj, int64_t stride, co
   // A partner of the rotation lies as many lanes away as chunks: nrot / 8, a power of two, and heads and rotations begin at
   // multiples of both halves.
   const int turn = 2 * nrot;
-  const bool lanes = nrot == 0 || neighbours || (turn <= 512 && (nrot & (nrot - 1)) == 0 && q_rot_off % turn == 0 && k_rot_off % turn == 0 &&
-                                   qw % turn == 0 && kw % turn == 0);
+  const bool lanes = nrot == 0 || neighbours ||
+                     (turn <= 512 && (nrot & (nrot - 1)) == 0 && q_rot_off % turn == 0 && k_rot_off % turn == 0 &&
+                      qw % turn == 0 && kw % turn == 0);
   // Two chunks a thread, one where a thread keeps the convolution's weights for it (two spill 30 registers in bf16, 70 in
   // fp32).  32 + 8 + 8 heads of 128 in bf16: convolved 1 row 8.1 -> 7.3 us, 64 rows 9.3 -> 7.9, 512 12.6 -> 9.5, 2,648 40.5 ->
   // 29.3 (3.0 TB/s), 4,654 64 -> 55, 8,192 103 -> 85; with a bias 2,648 rows 28.7 -> 21.5.  Latents (64 rotated entries of 32

@@ -19,9 +19,10 @@
 // shorter, without the lo parts 22 %.  Beside it 870 MB of queries and results where a step has 8,192 rows of 32 heads.
 // A page a workgroup takes 2.4 us; on 16 x 16 tiles, 16 queries a wave and every wave with all of a page, twice the LDS
 // reads, it took 3.0.  Queries come by LDS-DMA in whole lines, results leave by way of LDS: as the tiles have them, 32
-// bytes and 8 bytes of 32 rows to an access, these took 15 and 10 us a workgroup.  Attention alone, 32 heads: four
-// prompts of 2,048 851 -> 714 us, one 212 -> 180, one of 77 23.7 -> 13.3, eight chunks of 96 - 740 rows after
-// 416 227 -> 181; 187 steps of 1 to 8,192 rows, 3 to 64 heads, all kinds of weights and windows 1.02 - 2.1 times as fast.
+// bytes and 8 bytes of 32 rows to an access, these took 15 and 10 us a workgroup.  Attention alone, call after call, 32
+// heads: four prompts of 2,048 854 -> 725 us (772 and more where it is traced behind a pass's large products), one 213 -> 181,
+// one of 77 24.2 -> 13.5, eight chunks of 96 - 740 rows after 416 227 -> 181; 187 steps of 1 to 8,192 rows, 3 to 64 heads, all
+// kinds of weights and windows 1.02 - 2.1 times as fast.
 // Four tiles of values beside the scores take 2.8 us a page; with two the other wave's fourteen spill.
 #include <algorithm>
 #include <type_traits>

@@ -6,8 +6,8 @@ namespace rfqmix {
 
 // fp32 as a sum of three bf16, h + m + l, each the rounding of what is left: the sum is exact (8 bits each and two signs).
 // Products of two such sums without m l, l m (up to 2^-25 of the whole product each) and l l, together up to 2^-24, fp32's own
-// rounding, and a quarter of that on the average, take six products on the matrix cores, 2.7 times the rate of fp32 MFMA and, other than those, beside the vector instructions of other
-// waves.  Packed in twos: a in the low half.
+// rounding, and a quarter of that on the average, take six products on the matrix cores, 2.7 times the rate of fp32 MFMA and,
+// other than those, beside the vector instructions of other waves.  Packed in twos: a in the low half.
 struct Split2 {
   uint32_t h, m, l;
 };

@@ -1085,7 +1085,8 @@ def _short_f32(x, w) -> bool:
     """The same for fp32 operands, up to where the library is as fast."""
     M, K, N = x.shape[0], x.shape[1], w.shape[0]
     return (32 <= K <= SHORT_K and K % 32 == 0 and w.shape[1] == K and 1 <= M <= 1 << 20 and N >= 4 and N % 4 == 0
-            and (M * N <= 1 << 26 if K <= 64 else M * N <= 1 << 18 and max(M, N) <= 1 << 14) and x.device == w.device and x.stride(1) == 1 and w.stride(1) == 1
+            and (M * N <= 1 << 26 if K <= 64 else M * N <= 1 << 18 and max(M, N) <= 1 << 14)
+            and x.device == w.device and x.stride(1) == 1 and w.stride(1) == 1
             and x.stride(0) % 4 == 0 and w.stride(0) % 4 == 0
             and x.storage_offset() % 4 == 0 and w.storage_offset() % 4 == 0)
 
@@ -1095,7 +1096,8 @@ def matmul_nt(x, w, out_dtype=None):
     operands); ``out_dtype`` float32 keeps the accumulator's precision for bf16 operands.  Short
     bf16 products (a low-rank projection's second factor) of few rows run on a kernel: the
     library's host work, 20 us a call, is what bounds them.  fp32 ones of up to 64 terms run on
-    a kernel at all sizes, whose error is a third of the library's."""
+    a kernel up to 2^26 results (of 96 and 128 terms up to 2^18), whose error is a third of the
+    library's."""
     if (x.is_cuda and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and x.dim() == 2 and w.dim() == 2
             and out_dtype in (None, torch.bfloat16, torch.float32) and _short(x, w) and _plain(x, w)):
         return _native.mix_ops().matmul_short(x, w, out_dtype == torch.float32)

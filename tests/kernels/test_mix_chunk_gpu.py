@@ -192,8 +192,9 @@ def test_wkv_in_segments(dtype, lens):
 
 
 # Sixteen waves to a segment (heads are many, runs long): segments of 1,280 rows, whose last ones are shorter
-@pytest.mark.parametrize("mode,H,vdim,lens,dtype", [("wkv", 64, 64, [4136], torch.bfloat16), ("wkv", 40, 64, [3333, 2900], torch.float32),
-                                                    ("gla", 64, 128, [4136], torch.bfloat16), ("gla", 40, 64, [3333, 2900], torch.float32)])
+@pytest.mark.parametrize("mode,H,vdim,lens,dtype", [
+    ("wkv", 64, 64, [4136], torch.bfloat16), ("wkv", 40, 64, [3333, 2900], torch.float32),
+    ("gla", 64, 128, [4136], torch.bfloat16), ("gla", 40, 64, [3333, 2900], torch.float32)])
 def test_segments_of_sixteen_waves(mode, H, vdim, lens, dtype):
     assert _cut(mode, H, vdim, lens, 16)
     for shift in (-6.0, 0.0):
@@ -212,7 +213,8 @@ def test_segments_of_sixteen_waves(mode, H, vdim, lens, dtype):
         _close(st, st_w, tol)
 
 
-@pytest.mark.parametrize("mode,H,vdim,lens", [("gla", 2, 128, SEGMENTS), ("gla", 2, 64, SEGMENTS), ("delta", 2, 128, [1500, 33, 700])])
+@pytest.mark.parametrize("mode,H,vdim,lens", [("gla", 2, 128, SEGMENTS), ("gla", 2, 64, SEGMENTS),
+                                              ("delta", 2, 128, [1500, 33, 700])])
 def test_linear_recurrence_in_segments_bf16(mode, H, vdim, lens):
     assert _cut(mode, H, vdim, lens)
     (out, st), (out_w, st_w) = _linrec(mode, H, H, 64, vdim, torch.bfloat16, 0.0, lens=lens, pad=4)
@@ -264,12 +266,14 @@ def test_segments_beside_other_work():
         v, z = torch.randn(T, H, 128, generator=g).to(DEV), torch.randn(T, H * 64, generator=g).to(DEV)
         beta, gate = torch.randn(T, H, generator=g).to(DEV), torch.randn(T, H * 128, generator=g).to(DEV)
         rows, runs = _rows(lens, 23)
-        steps.append((q, k, v, z, beta, gate, torch.randn(2 * len(lens), H, 64, 128, generator=g).to(DEV), [r.to(DEV) for r in rows], runs.to(DEV)))
+        st = torch.randn(2 * len(lens), H, 64, 128, generator=g).to(DEV)
+        steps.append((q, k, v, z, beta, gate, st, [r.to(DEV) for r in rows], runs.to(DEV)))
 
     def call(q, k, v, z, beta, gate, st, rows, runs):
         out, st = torch.empty_like(gate), st.clone()
-        ops.gated_linear_recurrence(q, k, v, z, torch.full((16,), 0.01, device=DEV), torch.full((16 * 64,), -4.0, device=DEV), 1.0, beta,
-                                    gate, True, torch.ones(128, device=DEV), 1e-5, 0.125, st, *rows, out, run_rows=runs)
+        rate, zb = torch.full((16,), 0.01, device=DEV), torch.full((16 * 64,), -4.0, device=DEV)
+        ops.gated_linear_recurrence(q, k, v, z, rate, zb, 1.0, beta, gate, True, torch.ones(128, device=DEV), 1e-5, 0.125, st, *rows,
+                                    out, run_rows=runs)
         return out, st
 
     alone = [call(*s) for s in steps]
