@@ -17,7 +17,8 @@
 // The state pool is double buffered: a run reads its sequence's half and writes the other, and
 // a run that starts at position 0 reads nothing (the slot may hold another sequence's rest).
 //
-// Long runs with up to 64 key channels go in chunks (mix_chunk.hip).  Below: token by token.  One
+// Long runs with up to 64 key channels go in chunks (mix_chunk.hip), decode rows keep a head's state in the registers of a
+// workgroup (mix_state_rows.hip).  Below: token by token.  One
 // workgroup per (run, head); thread j owns value channel j: column j of S lives in
 // registers when dim is a compile-time size, else in LDS.  q, k and the decay of a token reach
 // all threads through LDS (one 16-byte read per key channel); the next token's operands are
@@ -531,7 +532,19 @@ void launch_gated_linrec(bool in_f32, bool act_f32, bool delta, const LinrecArgs
     LinrecArgs b = a;
     b.raw = nullptr;
     if (above > 0) b.below = above + 1;
-    LINREC_ALL();
+    const int mode = delta ? kChunkDelta : kChunkGla;
+    StateRows r{};
+    r.q = b.q; r.k = b.k; r.v = b.v; r.z = b.z; r.beta = b.beta; r.gate = b.gate;
+    r.qs = b.qs; r.ks = b.ks; r.vs = b.vs; r.zs = b.zs; r.bs = b.bs; r.gs = b.gs;
+    r.rate = b.rate; r.zbias = b.zbias; r.norm_w = b.norm_w;
+    r.zsign = b.zsign; r.eps = b.eps; r.q_scale = b.q_scale; r.gate_sigmoid = b.gate_sigmoid;
+    r.state = b.state;
+    r.row_state = b.row_state; r.row_back = b.row_back; r.row_fwd = b.row_fwd; r.pos = b.pos; r.run_rows = b.run_rows;
+    r.runs = b.run_rows != nullptr ? b.runs : b.T;
+    r.out = b.out; r.os = b.os;
+    r.H = b.H; r.rep = b.rep; r.dim = b.dim; r.vdim = b.vdim; r.slots = b.slots; r.below = b.below;
+    if (state_rows_ok(mode, in_f32, b.T, r)) launch_state_rows(mode, in_f32, act_f32, r, s);
+    else LINREC_ALL();
   }
   if (a.raw != nullptr && above + 1 < a.below) {
     const LinrecArgs& b = a;

@@ -13,6 +13,7 @@
 
 #include "mix_chunk.h"
 #include "mix_common.h"
+#include "mix_linrec.h"
 
 namespace rfqmix {
 
@@ -84,7 +85,7 @@ __global__ __launch_bounds__(256) void token_shift_mix_vec_kernel(
   }
 }
 
-// Token by token (long runs of 64 x 64 heads go in chunks: mix_chunk.hip).  One workgroup per
+// Token by token (long runs of 64 x 64 heads go in chunks: mix_chunk.hip; their decode rows: mix_state_rows.hip).  One workgroup per
 // (row, head); only a run's first row works: it walks the run.  Thread j owns value channel j: column j of S lives in LDS (st[i * N + j]: lanes hit
 // consecutive banks), or in registers when N is the compile-time NR.  r, k and the decay of
 // the next token are fetched while the current one is computed.
@@ -261,6 +262,16 @@ void launch_wkv_recurrence(bool f32, const void* r, const void* k, const void* v
   if ((a.cap = chunk_seg_cap(kChunkWkv, f32, Trows, a)) > 0) a.seg = scratch(chunk_seg_floats(kChunkWkv, a));
   if (below < INT32_MAX) launch_chunk(kChunkWkv, f32, f32, Trows, a, s);
   if (below == 1) return;
+  StateRows st{};
+  st.q = r; st.k = k; st.v = v; st.z = zw; st.gate = gate;
+  st.qs = rs; st.ks = ks; st.vs = vs; st.zs = zs; st.gs = gs;
+  st.zbias = w0; st.u = u; st.norm_w = norm_w; st.eps = eps; st.q_scale = 1.f;
+  st.state = state;
+  st.row_state = row_state; st.row_back = row_back; st.row_fwd = row_fwd; st.pos = pos; st.run_rows = run_rows;
+  st.runs = run_rows != nullptr ? runs : Trows;
+  st.out = out; st.os = (int64_t)H * N;
+  st.H = H; st.rep = 1; st.dim = st.vdim = N; st.slots = slots; st.below = below;
+  if (state_rows_ok(kChunkWkv, f32, Trows, st)) return launch_state_rows(kChunkWkv, f32, f32, st, s);
 #define WKV_GO(TT, NRR)                                                                         \
   launch_wkv_one<TT, NRR>(r, k, v, zw, gate, rs, ks, vs, zs, gs, w0, u, norm_w, eps, state,     \
                           row_state, row_back, row_fwd, pos, run_rows, runs, out, Trows, H, N,  \
