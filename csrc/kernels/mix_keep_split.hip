@@ -8,9 +8,11 @@
 // tiles, 121 us.  Here every wave takes every NW-th piece: its key rows go from memory straight into
 // MFMA operands, its value rows through the wave's own piece of LDS (read back transposed), the next
 // rows are in flight meanwhile, and no wave waits for another until the partial results (running
-// maximum, sum, weighted values) meet in LDS at the end.  Measured: 37 us (4.5 TB/s), 15 us and 54 us.  (Steps of the
-// 576-wide latent with more than 16 heads, no more rows than sequences and more than 20 pages to see do not come here
-// while CUs are free: a row's pages are split over workgroups as well, attn_keep_streams_kernel.)
+// maximum, sum, weighted values) meet in LDS at the end.  Measured: 37 us (4.5 TB/s; 44 where no cache holds the pages),
+// 15 us and 54 us.  (Groups of up to eight heads with keys and values of 64 or 128, no more rows than sequences, do not
+// come here: mix_keep_row.hip.  Nor do steps of the 576-wide latent with more than 16 heads, no more rows than sequences
+// and more than 20 pages to see while CUs are free: a row's pages are split over workgroups as well,
+// attn_keep_streams_kernel.)
 //
 // The 16 MFMA columns are (row, head) pairs of one key/value head, so the rows of a short extend and
 // the heads of a group share one pass.
@@ -25,61 +27,11 @@
 
 #include "common.h"
 #include "mix_common.h"
+#include "mix_keep_split.h"
 
 namespace rfqmix {
 
-using rfq::as_bf16x8;
-using rfq::f32x4;
-using rfq::s16x4;
-using rfq::s16x8;
-
 namespace {
-constexpr int PG = 32;                  // tokens per page
-constexpr float kNegInfS = -__builtin_huge_valf();
-// The maximum that weights are taken against moves only when a score passes it by this much (weights
-// stay below e^8): most turns then leave the accumulators alone.
-constexpr float kDefer = 8.f;
-
-// f as a sum of N bf16 values: three hold all 24 bits, two 16.  INF: f may be infinite, as one of them.
-template <bool INF, int N>
-__device__ __forceinline__ void split_parts(const float* f, s16x8 (&p)[N]) {
-  float r[8];
-#pragma unroll
-  for (int i = 0; i < 8; ++i) r[i] = f[i];
-#pragma unroll
-  for (int n = 0; n < N; ++n) {
-    p[n] = rfq::pack8(r);
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const float h = rfq::bf2f_s(p[n][i]);
-      r[i] = INF && fabsf(h) == -kNegInfS ? 0.f : r[i] - h;
-    }
-  }
-}
-template <bool EXACT>
-__device__ __forceinline__ float exp_of(float x) { return EXACT ? expf(x) : __expf(x); }
-// tanh to 1.6 units in the last place, without tanhf's branches (64 sequences of 300 - 900 tokens: 58.5 us a
-// pass with it, 57.5 with this, 56.4 with the wide groups' form).  Below 0.7 an odd
-// polynomial, fitted to a relative error of 1.6e-8; above, 1 - 2 / (exp(2 |x|) + 1).
-__device__ __forceinline__ float tanh_of(float x) {
-  const float u = x * x, ax = fabsf(x);
-  float p = -0.0051386617f;
-  p = p * u + 0.02009197f;
-  p = p * u - 0.05355886f;
-  p = p * u + 0.13329111f;
-  p = p * u - 0.3333319f;
-  const float big = 1.f - 2.f * __builtin_amdgcn_rcpf(__builtin_amdgcn_exp2f(ax * 2.88539008f) + 1.f);
-  return ax < 0.7f ? x + x * u * p : copysignf(big, x);
-}
-
-// Lanes read here what others of their wave wrote to LDS.  The hardware keeps a wave's LDS accesses in
-// order, this keeps the compiler's; no instruction comes of it.
-__device__ __forceinline__ void wave_lds_order() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // keys per turn: a page, or half of one where queries and results of a wide latent fill the registers
 template <int DK, bool SHARED>
 constexpr int turn_keys() { return SHARED && DK >= 10 ? 16 : PG; }
@@ -105,23 +57,6 @@ constexpr int wave_lds() {
 void launch_attn_keep_wide_rows(const float*, const void*, int64_t, const int32_t*, int, const int32_t*, const int32_t*,
                                 const int32_t*, int, int, const float*, const void*, int64_t, int, void*, int64_t, float,
                                 int, int, bool, int, int, int, float, float, hipStream_t);   // mix_keep_attn_mfma.hip
-
-struct KeepSplitArgs {
-  const float* q;
-  const bf16_t *k_cache, *v_cache;
-  int64_t vrs;
-  const int32_t* bt;
-  int maxb;
-  const int32_t *q_start, *q_len, *kv_len;
-  const float* head_bias;
-  const bf16_t* gate;
-  int64_t gate_stride;
-  int gate_w;
-  bf16_t* out;
-  int64_t out_stride;
-  float scale, softcap, out_mult;
-  int window, keep_first, sigmoid, H, G;
-};
 
 // EXACT (groups of fewer than 16 heads): queries, weights and their functions in full fp32.
 template <int DK, int DV, bool SHARED, int NW, bool EXACT>
@@ -496,6 +431,7 @@ void launch_attn_keep_split(const float* q, const void* k_cache, const void* v_c
   const KeepSplitArgs a{q, (const bf16_t*)k_cache, (const bf16_t*)v_cache, vrs, bt, maxb, q_start, q_len, kv_len,
                         head_bias, (const bf16_t*)gate, gate_stride, gate_w, (bf16_t*)out, out_stride,
                         scale, softcap, out_mult, window, keep_first, (int)sigmoid, H, G};
+  if (keep_row_ok(T, NA, H, G, E, vdim, shared)) return launch_attn_keep_row(a, NA, E, s);
   const int DK = E / 32, DV = vdim / 16;
   const bool exact = H / G < 16;
   const int tiles = (int)(((int64_t)std::min(short_rows, T) * (H / G) + 15) / 16);   // at most, of a sequence
