@@ -1235,3 +1235,37 @@ def test_qkv_rope_in_two_products(M, head, Hq, K):
         # both round a product of unit variance to bf16, the rotation's result once more: a spacing each
         assert float((a.float() - b.float()).abs().max()) <= 3 * 2.0 ** -8 * float(b.float().abs().max())
         assert float((a.float() - b.float()).norm() / b.float().norm()) <= 2.0 ** -8
+
+
+@pytest.mark.parametrize("Hq,Hkv", [(32, 8), (8, 1), (64, 8), (3, 3), (16, 1)])
+@pytest.mark.parametrize("splits,single", [(1, False), (3, False), (2, True), (16, True)])
+@pytest.mark.parametrize("tiles", [1, 2])
+def test_attn_decode_rows(gpu, Hq, Hkv, splits, single, tiles):
+    """Steps of no more rows than work items (csrc/kernels/attn_decode_rows.hip): contexts around pages, splits and
+    waves, what was never written, a sequence of several rows and one without any."""
+    torch.manual_seed(6)
+    G = Hq // Hkv
+    qlens, kvlens = [1, 1, 1, 1, 1, 0, 2, 1, 1], [1, 31, 32, 33, 700, 50, 70, 257, 2049]
+    k, v = _paged_cache(512, Hkv, gpu, seed=5)
+    bt = _block_tables(kvlens, 512, gpu)
+    for i, n in enumerate(kvlens):
+        if n % 32:
+            k[bt[i, n // 32].long(), :, n % 32:] = v[bt[i, n // 32].long(), :, n % 32:] = float("nan")
+    T = sum(qlens)
+    qs = [sum(qlens[:i]) for i in range(len(qlens))]
+    work = [(i, ct) for i, n in enumerate(qlens) for ct in range(((n * G + 15) // 16 + tiles - 1) // tiles)]
+    work += [(-1, 0)] * max(1, T - len(work))
+    i32 = lambda a: torch.tensor(a, dtype=torch.int32, device=gpu)  # noqa: E731
+    q = torch.randn(T, Hq * 128, device=gpu, dtype=BF)
+    po = torch.full((T * Hq * splits * 128,), float("nan"), device=gpu)
+    pm = torch.full((T * Hq * splits * 2,), float("nan"), device=gpu)
+    tickets = torch.zeros(len(work) * Hkv, dtype=torch.int32, device=gpu) if single else None
+    exp = torch.zeros(T, Hq * 128, dtype=BF)
+    ref.attn_prefill(q.cpu(), k.cpu().nan_to_num(), v.cpu().nan_to_num(), bt.cpu(), torch.tensor(qs), torch.tensor(qlens),
+                     torch.tensor(kvlens), None, None, exp, Hq, Hkv, 128 ** -0.5)
+    for it in range(3 if single else 1):
+        out = torch.full((T, Hq * 128), float("nan"), device=gpu, dtype=BF)
+        ops.attn_decode(q, k, v, bt, i32(qs), i32(qlens), i32(kvlens), i32([x[0] for x in work]), i32([x[1] for x in work]),
+                        out, po, pm, Hq, Hkv, 128 ** -0.5, splits, tiles, tickets)
+        assert not single or int(tickets.abs().sum()) == 0
+        _close(out, exp, 2e-2, 0, f"attn_decode rows Hq={Hq} splits={splits} tiles={tiles} it={it}")
