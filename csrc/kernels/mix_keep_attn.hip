@@ -91,6 +91,17 @@ __device__ __forceinline__ void st_chunk(bf16_t* p, const float* f) {
     stf(p, f[0]);
   }
 }
+// Sum over the wave in every lane, without a way through LDS
+__device__ __forceinline__ float wave_total(float v) {
+  v = group_sum(v, 16);
+  const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  v = __uint_as_float(a[0]) + __uint_as_float(a[1]);
+  const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return __uint_as_float(b[0]) + __uint_as_float(b[1]);
+}
+__device__ __forceinline__ float lane_of(float v, int lane) {
+  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane));
+}
 // A chunk as loaded, for operands that several loads bring in together: converted at its use.
 template <int CW>
 struct Bits {
@@ -376,9 +387,14 @@ __global__ __launch_bounds__(1024) void qk_norm_rotary_append_kernel(
 
 // The same where norms are of whole projections, of a single key head or none: a workgroup takes several neighbouring rows
 // one after another.  A thread has two chunks of eight columns for all of them and keeps these columns' weights (of the
-// convolution, the norms, the bias) and the rows above in registers; with a workgroup a row every row read 100 KB of
-// weights and three rows from the L2s for its own 12, which bounded it.  Two rows on are on their way while one is made;
-// they are waited for before a row's stores, which are counted with the loads and in order.
+// convolution, the norms, the bias) in registers; with a workgroup a row every row read 100 KB of weights and three rows
+// from the L2s for its own 12, which bounded it.  Two rows on are on their way while one is made; they are waited for before
+// a row's stores, which are counted with the loads and in order.
+// What bounds it: vector instructions (twelve waves a CU at 32 + 8 + 8 heads, 70 % of the clocks before), then the writes of
+// q, so a row's work is kept small: with one chunk a thread a row adds its parts to sums for the three rows below it when it
+// is converted, once, instead of being converted again for each of them; waves without columns of q, of k or of a rotation
+// leave their sums and exchanges out; both factors' roots are made at once, in two rows of lanes.  2,648 rows of 6,144
+// columns 30.6 -> 25.0 us; two, three or four rows to a barrier instead changed nothing there and cost narrow rows a third.
 struct QknRows {
   const void* proj;
   int64_t stride;
@@ -407,20 +423,20 @@ template <typename T, bool CONV, int N>
 __global__ __launch_bounds__(N == 1 ? 1024 : kQknThreads) void qk_norm_rotary_append_rows_kernel(const QknRows a) {
   constexpr int K = kQknTaps - 1;
   constexpr bool DEEP = !CONV || N == 1;                            // two rows on the way, else one: registers
+  constexpr bool SUMS = CONV && N == 1;                             // a row's part of the K rows below it is summed up
   extern __shared__ __attribute__((aligned(16))) float lds[];
   const int tid = threadIdx.x, nthr = blockDim.x, lane = tid & 63, wid = tid >> 6, nw = nthr >> 6;
   const int t0 = blockIdx.x * a.rows, n = min(a.rows, a.T - t0);
   const int nq = a.H * a.qw, nk = a.G * a.kw, W = nq + nk + a.G * a.vdim;
-  float* cs = lds;                                        // (cos, sin) of every row
+  int32_t* meta = reinterpret_cast<int32_t*>(lds);        // [rows][slot, back, fwd, state]
+  float* cs = lds + 4 * a.rows;                           // (cos, sin) of every row
   float* sums = cs + 2 * a.nrot * a.rows;                 // [2][q, k][wave]
-  int32_t* meta = reinterpret_cast<int32_t*>(sums + 4 * nw);     // [rows][slot, back, fwd, state, position]
+  int32_t* pos = reinterpret_cast<int32_t*>(sums + 4 * nw);          // [rows]
   if (tid < n) {
     const int t = t0 + tid;
-    meta[5 * tid] = a.slots[t];
-    meta[5 * tid + 1] = CONV ? a.row_back[t] : 0;
-    meta[5 * tid + 2] = CONV ? a.row_fwd[t] : 0;
-    meta[5 * tid + 3] = CONV ? a.row_state[t] : -1;
-    meta[5 * tid + 4] = a.pos[t];
+    *reinterpret_cast<int4*>(meta + 4 * tid) = make_int4(a.slots[t], CONV ? a.row_back[t] : 0, CONV ? a.row_fwd[t] : 0,
+                                                         CONV ? a.row_state[t] : -1);
+    pos[tid] = a.pos[t];
   }
   const T* proj = static_cast<const T*>(a.proj);
   int col[N], at[N];                                      // columns here and in proj; chunks past the row: its last one
@@ -450,18 +466,20 @@ __global__ __launch_bounds__(N == 1 ? 1024 : kQknThreads) void qk_norm_rotary_ap
       for (int j = 0; j < N; ++j) ld_chunk<8>(a.conv_w + (int64_t)d * W + col[j], taps[d][j]);
   }
   // a chunk's place: 0 q, 1 k, 2 v, 3 k without norm; its head and the entry in it; the rotation of its head
-  int kind[N], head[N], entry[N], turn[N];                // turn: (cos, sin) pairs by which it turns, or -1
+  int kind[N], turn[N];                                   // turn: (cos, sin) pairs by which it turns, or -1
+  int64_t put[N];                                         // where it goes in a row of q, in a page from the row's slot on
   bool first[N];                                          // of the rotation's two halves
+  bool has_q = false, has_k = false, turns = false;       // this wave, in any lane
 #pragma unroll
   for (int j = 0; j < N; ++j) {
     kind[j] = col[j] < nq ? 0 : col[j] < nq + nk ? 1 : 2;
     const int y = col[j] - (kind[j] == 0 ? 0 : kind[j] == 1 ? nq : nq + nk), w = kind[j] == 0 ? a.qw : kind[j] == 1 ? a.kw : a.vdim;
-    head[j] = y / w;
-    entry[j] = y - head[j] * w;
-    const int r0 = entry[j] - (kind[j] == 0 ? a.q_rot_off : a.k_rot_off);
+    const int head = y / w, entry = y - head * w;
+    put[j] = kind[j] == 0 ? head * a.q_hs + entry : (int64_t)head * a.BS * w + entry;
+    const int r0 = entry - (kind[j] == 0 ? a.q_rot_off : a.k_rot_off);
     first[j] = r0 < a.nrot;
     turn[j] = kind[j] < 2 && r0 >= 0 && r0 < 2 * a.nrot ? (a.neighbours ? r0 >> 1 : first[j] ? r0 : r0 - a.nrot) : -1;
-    if (kind[j] == 1 && entry[j] >= a.k_norm_n) kind[j] = 3;          // a key's entries that are not normed
+    if (kind[j] == 1 && entry >= a.k_norm_n) kind[j] = 3;            // a key's entries that are not normed
     const float* wn = kind[j] == 0 ? a.q_norm_w : kind[j] == 1 ? a.k_norm_w : nullptr;
     if (wn != nullptr) ld_chunk<8>(wn + y, norm[j]);
     else
@@ -469,23 +487,55 @@ __global__ __launch_bounds__(N == 1 ? 1024 : kQknThreads) void qk_norm_rotary_ap
       for (int i = 0; i < 8; ++i) norm[j][i] = 1.f;
     if constexpr (!CONV)
       if (a.bias != nullptr) ld_chunk<8>(a.bias + col[j], bias[j]);
+    has_q |= __builtin_amdgcn_ballot_w64(live[j] && kind[j] == 0) != 0ull;
+    has_k |= __builtin_amdgcn_ballot_w64(live[j] && kind[j] == 1) != 0ull;
+    turns |= __builtin_amdgcn_ballot_w64(turn[j] >= 0) != 0ull;
   }
+  const int partner = (lane ^ a.nrot >> 3) * 4;           // of the rotation: that lane's byte
   __syncthreads();
   for (int x = tid; x < n * a.nrot; x += nthr) {
     const int r = x / a.nrot, i = x - r * a.nrot;
     float sn, c;
-    sincosf((float)meta[5 * r + 4] * a.inv_freq[i], &sn, &c);
+    sincosf((float)pos[r] * a.inv_freq[i], &sn, &c);
     cs[2 * x] = c * a.rot_mult;
     cs[2 * x + 1] = sn * a.rot_mult;
   }
+  // What the rows above row r of its run add to it and the two below.  `back` of them are in the projection (registers:
+  // r = 0), older ones in the state that the run began with.
+  float acc[SUMS ? K : 1][8];
+  auto begin = [&](int r, const int4& m) {
+    const int pt = __builtin_amdgcn_readfirstlane(pos[r]);
+    const int half = (m.w & 1) * a.state_slots + (m.w >> 1);
+#pragma unroll
+    for (int e = 0; e < K; ++e)
+#pragma unroll
+      for (int i = 0; i < 8; ++i) acc[e][i] = 0.f;
+#pragma unroll
+    for (int d = K - 1; d >= 0; --d) {
+      const bool own = d < m.y;
+      if (!own && (pt - d - 1 < 0 || m.w < 0)) continue;
+      float u[8];
+      if (own) above[d][0].template get<T>(u);
+      else ld_chunk<8>(a.conv_state + ((int64_t)half * K + (K + m.y - d - 1)) * W + col[0], u);
+#pragma unroll
+      for (int e = 0; e < K - d; ++e)
+#pragma unroll
+        for (int i = 0; i < 8; ++i) acc[e][i] += taps[K - 1 - d - e][0][i] * u[i];
+    }
+  };
+  auto numbers = [&](int r) {                             // a row's slot, back, fwd, state
+    const int4 m = *reinterpret_cast<const int4*>(meta + 4 * r);
+    return make_int4(__builtin_amdgcn_readfirstlane(m.x), __builtin_amdgcn_readfirstlane(m.y),
+                     __builtin_amdgcn_readfirstlane(m.z), __builtin_amdgcn_readfirstlane(m.w));
+  };
+  if constexpr (SUMS) begin(0, numbers(0));
   for (int r = 0; r < n; ++r) {
-    const int slot = __builtin_amdgcn_readfirstlane(meta[5 * r]);
+    const int4 m = numbers(r);
+    const int slot = m.x, back = m.y, fwd = m.z, code = m.w;
     float f[N][8];
 #pragma unroll
     for (int j = 0; j < N; ++j) raw[j].template get<T>(f[j]);
     if constexpr (CONV) {
-      const int back = __builtin_amdgcn_readfirstlane(meta[5 * r + 1]), fwd = __builtin_amdgcn_readfirstlane(meta[5 * r + 2]);
-      const int code = __builtin_amdgcn_readfirstlane(meta[5 * r + 3]), pt = __builtin_amdgcn_readfirstlane(meta[5 * r + 4]);
       if (fwd < K && code >= 0) {                         // the run's last rows go to the other half
         const float* rd = a.conv_state + ((int64_t)((code & 1) * a.state_slots + (code >> 1)) * K) * W;
         float* wr = a.conv_state + ((int64_t)((1 - (code & 1)) * a.state_slots + (code >> 1)) * K) * W;
@@ -501,41 +551,54 @@ __global__ __launch_bounds__(N == 1 ? 1024 : kQknThreads) void qk_norm_rotary_ap
               }
           }
       }
+      if constexpr (SUMS) {
+        if (back == 0 && r > 0) begin(r, m);
 #pragma unroll
-      for (int j = 0; j < N; ++j)
+        for (int i = 0; i < 8; ++i) {
+          const float x = f[0][i];
+          f[0][i] = fmaf(taps[K][0][i], x, acc[0][i]);
 #pragma unroll
-        for (int i = 0; i < 8; ++i) f[j][i] *= taps[K][j][i];
-      if (back >= K) {
-#pragma unroll
-        for (int d = 0; d < K; ++d)
-#pragma unroll
-          for (int j = 0; j < N; ++j) {
-            float u[8];
-            above[d][j].template get<T>(u);
-#pragma unroll
-            for (int i = 0; i < 8; ++i) f[j][i] += taps[K - 1 - d][j][i] * u[i];
-          }
+          for (int e = 0; e < K - 1; ++e) acc[e][i] = fmaf(taps[K - 1 - e][0][i], x, acc[e + 1][i]);
+          acc[K - 1][i] = taps[0][0][i] * x;
+        }
       } else {
 #pragma unroll
-        for (int d = 0; d < K; ++d) {
-          const bool own = d < back;
-          if (!own && (pt - d - 1 < 0 || code < 0)) break;
-          const float* rd = a.conv_state + ((int64_t)((code & 1) * a.state_slots + (code >> 1)) * K + (K + back - d - 1)) * W;
+        for (int j = 0; j < N; ++j)
 #pragma unroll
-          for (int j = 0; j < N; ++j) {
-            float u[8];
-            if (own) above[d][j].template get<T>(u);
-            else ld_chunk<8>(rd + col[j], u);
+          for (int i = 0; i < 8; ++i) f[j][i] *= taps[K][j][i];
+        if (back >= K) {
 #pragma unroll
-            for (int i = 0; i < 8; ++i) f[j][i] += taps[K - 1 - d][j][i] * u[i];
+          for (int d = 0; d < K; ++d)
+#pragma unroll
+            for (int j = 0; j < N; ++j) {
+              float u[8];
+              above[d][j].template get<T>(u);
+#pragma unroll
+              for (int i = 0; i < 8; ++i) f[j][i] += taps[K - 1 - d][j][i] * u[i];
+            }
+        } else {
+          const int pt = __builtin_amdgcn_readfirstlane(pos[r]);
+#pragma unroll
+          for (int d = 0; d < K; ++d) {
+            const bool own = d < back;
+            if (!own && (pt - d - 1 < 0 || code < 0)) break;
+            const float* rd = a.conv_state + ((int64_t)((code & 1) * a.state_slots + (code >> 1)) * K + (K + back - d - 1)) * W;
+#pragma unroll
+            for (int j = 0; j < N; ++j) {
+              float u[8];
+              if (own) above[d][j].template get<T>(u);
+              else ld_chunk<8>(rd + col[j], u);
+#pragma unroll
+              for (int i = 0; i < 8; ++i) f[j][i] += taps[K - 1 - d][j][i] * u[i];
+            }
           }
         }
-      }
 #pragma unroll
-      for (int j = 0; j < N; ++j) {
+        for (int j = 0; j < N; ++j) {
 #pragma unroll
-        for (int d = K - 1; d > 0; --d) above[d][j] = above[d - 1][j];
-        above[0][j] = raw[j];
+          for (int d = K - 1; d > 0; --d) above[d][j] = above[d - 1][j];
+          above[0][j] = raw[j];
+        }
       }
     }
     if constexpr (DEEP) {
@@ -560,38 +623,54 @@ __global__ __launch_bounds__(N == 1 ? 1024 : kQknThreads) void qk_norm_rotary_ap
       sk += live[j] && kind[j] == 1 ? ss : 0.f;
     }
     float* sum = sums + (r & 1) * 2 * nw;
-    sq = group_sum(sq, 64);
-    sk = group_sum(sk, 64);
+    if (has_q) sq = wave_total(sq);
+    if (has_k) sk = wave_total(sk);
     if (lane == 0) {
       sum[wid] = sq;
       sum[nw + wid] = sk;
     }
     __syncthreads();                                      // the first: the sines too
+    // q's factor in the first of four rows of lanes, k's in the second
     const int part = lane & 15;
-    const float qs = group_sum(part < nw ? sum[part] : 0.f, 16), ks = group_sum(part < nw ? sum[nw + part] : 0.f, 16);
-    const float fq = a.q_norm_w != nullptr ? 1.0f / sqrtf(qs / (float)nq + a.eps) : 1.f;
-    const float fk = a.k_norm_w != nullptr ? 1.0f / sqrtf(ks / (float)(a.G * a.k_norm_n) + a.eps) : 1.f;
+    const bool of_k = (lane & 16) != 0;
+    const float all = group_sum(part < nw ? sum[(of_k ? nw : 0) + part] : 0.f, 16);
+    const float fac = 1.0f / sqrtf(all / (float)(of_k ? a.G * a.k_norm_n : nq) + a.eps);
+    const float fq = a.q_norm_w != nullptr ? lane_of(fac, 0) : 1.f, fk = a.k_norm_w != nullptr ? lane_of(fac, 16) : 1.f;
 #pragma unroll
     for (int j = 0; j < N; ++j) {
       const float fc = kind[j] == 0 ? fq : kind[j] == 1 ? fk : 1.f;
 #pragma unroll
-      for (int i = 0; i < 8; i += 2) {
-        f[j][i] *= fc * norm[j][i];
-        f[j][i + 1] *= fc * norm[j][i + 1];
-        if (a.neighbours) {
-          if (turn[j] >= 0) {
-            const float2 c = *reinterpret_cast<const float2*>(cs + 2 * (r * a.nrot + turn[j]) + i);
-            const float x = f[j][i] * c.x - f[j][i + 1] * c.y;
-            f[j][i + 1] = f[j][i + 1] * c.x + f[j][i] * c.y;
+      for (int i = 0; i < 8; ++i) f[j][i] *= fc * norm[j][i];
+      if (!turns) continue;
+      const float* c = cs + 2 * (r * a.nrot + max(turn[j], 0));
+      if (a.neighbours) {
+        if (turn[j] >= 0) {
+          const float4 c0 = ld4(c), c1 = ld4(c + 4);
+          const float cc[8] = {c0.x, c0.y, c0.z, c0.w, c1.x, c1.y, c1.z, c1.w};
+#pragma unroll
+          for (int i = 0; i < 8; i += 2) {
+            const float x = f[j][i] * cc[i] - f[j][i + 1] * cc[i + 1];
+            f[j][i + 1] = f[j][i + 1] * cc[i] + f[j][i] * cc[i + 1];
             f[j][i] = x;
           }
-          continue;
         }
-        const float u0 = __shfl_xor(f[j][i], a.nrot >> 3, 64), u1 = __shfl_xor(f[j][i + 1], a.nrot >> 3, 64);   // the partner's
-        if (turn[j] >= 0) {
-          const float4 c = ld4(cs + 2 * (r * a.nrot + turn[j] + i));
-          f[j][i] = first[j] ? f[j][i] * c.x - u0 * c.y : f[j][i] * c.x + u0 * c.y;
-          f[j][i + 1] = first[j] ? f[j][i + 1] * c.z - u1 * c.w : f[j][i + 1] * c.z + u1 * c.w;
+      } else {
+        constexpr int SH = CONV && N == 2 ? 2 : 8;        // at a time: registers
+#pragma unroll
+        for (int i0 = 0; i0 < 8; i0 += SH) {
+          float u[SH];
+#pragma unroll
+          for (int i = 0; i < SH; ++i)
+            u[i] = __int_as_float(__builtin_amdgcn_ds_bpermute(partner, __float_as_int(f[j][i0 + i])));
+          if (turn[j] >= 0) {
+#pragma unroll
+            for (int i = 0; i < SH; i += 2) {
+              const float4 cc = ld4(c + 2 * (i0 + i));
+              float* const y = f[j] + i0 + i;
+              y[0] = y[0] * cc.x + u[i] * (first[j] ? -cc.y : cc.y);
+              y[1] = y[1] * cc.z + u[i + 1] * (first[j] ? -cc.w : cc.w);
+            }
+          }
         }
       }
     }
@@ -604,10 +683,10 @@ __global__ __launch_bounds__(N == 1 ? 1024 : kQknThreads) void qk_norm_rotary_ap
 #pragma unroll
     for (int j = 0; j < N; ++j)
       if (live[j]) {
-        if (kind[j] == 0) st_chunk<8>(a.q_out + (t0 + r) * a.q_ts + head[j] * a.q_hs + entry[j], f[j]);
+        if (kind[j] == 0) st_chunk<8>(a.q_out + (t0 + r) * a.q_ts + put[j], f[j]);
         else if (keep) {
           T* cache = static_cast<T*>(kind[j] != 2 ? a.k_cache : a.v_cache);
-          st_chunk<8>(cache + (page_row + (int64_t)head[j] * a.BS) * (kind[j] != 2 ? a.kw : a.vdim) + entry[j], f[j]);
+          st_chunk<8>(cache + page_row * (kind[j] != 2 ? a.kw : a.vdim) + put[j], f[j]);
         }
       }
   }
@@ -1029,13 +1108,14 @@ bool launch_qk_norm_rotary_append(bool f32, const void* proj, int64_t stride, co
   const bool lanes = nrot == 0 || neighbours ||
                      (turn <= 512 && (nrot & (nrot - 1)) == 0 && q_rot_off % turn == 0 && k_rot_off % turn == 0 &&
                       qw % turn == 0 && kw % turn == 0);
-  // Two chunks a thread, one where a thread keeps the convolution's weights for it (two spill 30 registers in bf16, 70 in
-  // fp32).  32 + 8 + 8 heads of 128 in bf16: convolved 1 row 8.1 -> 7.3 us, 64 rows 9.3 -> 7.9, 512 12.6 -> 9.5, 2,648 40.5 ->
-  // 29.3 (3.0 TB/s), 4,654 64 -> 55, 8,192 103 -> 85; with a bias 2,648 rows 28.7 -> 21.5.  Latents (64 rotated entries of 32
-  // heads, 576 of the key): 2,067 rows 15.2 -> 11.3, 8,192 44.3 -> 28.2.  Where it does not pay, measured from 256 to 10,240
-  // columns and 1 to 8,192 rows:
-  //   convolved, two chunks a thread: in fp32 never (64 + 8 + 8 heads, 2,067 rows 99 us for 73), in bf16 up to 9,216 columns
-  //   (4,654 rows 108 for 96) and few rows (10,240 columns: 257 rows 16.5 for 15.0, 1,024 31.2 for 34.2)
+  // Two chunks a thread, one where a thread keeps the convolution's weights for it (two spill 20 registers in bf16, 70 in
+  // fp32).  32 + 8 + 8 heads of 128 in bf16, against a workgroup a row and against these rows before the sums were kept:
+  // convolved 1 row 8.1, 7.2, now 6.6 us, 64 rows 9.3, 8.4, 7.8, 2,648 40.5, 30.6, 25.0 (3.4 TB/s), 8,192 103, 87, 66; with a
+  // bias 2,648 rows 28.7, 23.1, 21.5.  Latents (64 rotated entries of 32 heads, 576 of the key): 2,067 rows 15.2, 10.3, 10.0,
+  // 8,192 44.3, 29.5, 28.2.  Where it does not pay, measured from 256 to 10,240 columns and 1 to 8,192 rows:
+  //   convolved, two chunks a thread: in fp32 never (64 + 8 + 8 heads, 2,067 rows 99 us for 73), in bf16 up to a row a CU
+  //   (10,240 columns: 64 rows 14.0 us for 12.5, 256 13.3 for 10.9, 300 15.2 for 16.9, 700 21.1 for 22.3) and up to 9,216
+  //   columns from three rows a CU (9,216: 513 rows 19.2 for 18.3, 700 20.3 for 20.5, 1,031 26.6 for 32.9, 512 16.8 for 18.0)
   //   convolved in fp32, a single row of 6,144 columns and more: up to 1.09 times the other kernel's time
   //   no norm, little to sum up: 64 rows of 3,072 columns 4.7 us for 4.4
   //   fp32 without a convolution, four to eight waves of 134 registers, one such workgroup a CU: 824 rows of 6,144 columns 16.2
@@ -1045,7 +1125,7 @@ bool launch_qk_norm_rotary_append(bool f32, const void* proj, int64_t stride, co
   const int wide = (int)((W / 8 + per - 1) / per + 63) / 64 * 64;
   const bool one = norm_all || (q_norm_w == nullptr && (k_norm_w == nullptr || G == 1));     // norm of a kind's columns
   auto pays = [&]() {
-    if (conv) return per == 1 ? !f32 || T >= 8 || W < 6144 : !f32 && W > 9216 && T >= 1024;
+    if (conv) return per == 1 ? !f32 || T >= 8 || W < 6144 : !f32 && T > 256 && (W > 9216 || T <= 512 || T >= 700);
     if (q_norm_w == nullptr && k_norm_w == nullptr &&
         !(f32 ? T >= 2048 : T >= 1024 || (int64_t)T * (int64_t)W >= 1 << 20 || W >= 7168)) return false;
     return !f32 || T <= 256 || wide <= 192 || W > 9216 || (wide >= 576 && T >= 2048);

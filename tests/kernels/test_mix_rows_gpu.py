@@ -128,6 +128,16 @@ def test_norm_and_rotation_of_rows_one_after_another(dtype, conv, H, G, dim, nro
         torch.testing.assert_close(a.cpu().float(), b.float(), atol=3e-5 if T < 100 else 4e-3, rtol=1e-5 + (rel if dtype == torch.bfloat16 else 0.0))
 
 
+# Runs of one to seven rows everywhere: workgroups that begin at any row of a run, with and without a state
+@pytest.mark.parametrize("T,H,G,dim", [(2101, 20, 3, 64), (1030, 40, 8, 128), (300, 64, 8, 128), (1030, 56, 8, 128)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_convolved_rows_of_short_runs(monkeypatch, dtype, T, H, G, dim):
+    lens = [1 + i % 7 for i in range(T // 4)]
+    lens = lens[:next(i for i in range(len(lens)) if sum(lens[:i + 1]) >= T - 7) + 1]
+    monkeypatch.setitem(globals(), "_lens", lambda total: lens + [total - sum(lens)] * (total > sum(lens)))
+    test_norm_and_rotation_of_rows_one_after_another(dtype, True, H, G, dim, 32, 0, T)
+
+
 # More rows than one round of workgroups takes in sixteens: two rounds of eight or nine
 @pytest.mark.parametrize("T", [4096, 4104])
 def test_norm_and_rotation_of_rows_in_rounds(T):
