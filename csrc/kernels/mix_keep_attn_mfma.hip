@@ -4,8 +4,8 @@
 // (a column per head, or gate_w = vdim: one per output, rows 8-byte aligned);
 // the values may be the leading entries of the key rows themselves (latent attention).
 // Prompt rows of 576-wide latents with groups of four heads: mix_keep_latent.hip.
-// Decode rows have kernels of their own: mix_keep_split.hip, and here those of wide latents in streams over several
-// workgroups (attn_keep_streams_kernel) and many heads at a time (attn_keep_wide_kernel, DEC).
+// Decode rows have kernels of their own: mix_keep_split.hip, mix_keep_streams.hip (wide latents, pages shared by several
+// workgroups), and here those of wide latents with many heads at a time (attn_keep_wide_kernel, DEC).
 //
 // One workgroup per (work item, HPW heads of one key/value head); a work item is (sequence, block of 32 queries).
 // A wave has the 32 queries of a head: it keeps the running maximum and sum of its query columns and the weighted
@@ -45,16 +45,6 @@
 #include "mix_keep_mfma.h"
 
 namespace rfqmix {
-
-// the same over lanes 16 away
-__device__ __forceinline__ float other_row_max(float x) {
-  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-  return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
-}
-__device__ __forceinline__ float both_rows_sum(float x) {
-  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
-}
 
 // lane (col, grp) holds value channels 16 m + 4 grp .. + 3 of its query: 8-byte stores
 template <int DV, int MODE>
@@ -851,376 +841,6 @@ __global__ __launch_bounds__(128 * HPW, DEC && HPW == 1 ? 1 : 2) void attn_keep_
   }
 }
 
-// Decode rows of a wide latent with more than 16 heads a key head, few sequences: a row's pages are shared by
-// S workgroups of four streams, a stream being two waves (16 heads each) and a page of its own in LDS.  Streams meet
-// in LDS, workgroups in attn_keep_streams_merge_kernel, by way of `part` ([T, S, H] of vdim weighted values each,
-// then as many pairs of maximum, in base 2, and sum; -inf: no key).
-// What bounds it: the way to the first page (some 2 us for the step's numbers, 5 - 9 for page and queries), a page's
-// products (3 us), and 2 us for the streams to meet; so as many streams as the chip has room for, one workgroup to a
-// CU.  The queries are read once a workgroup and shared through LDS: read by every stream they held the pages up
-// (34 us for what took 28 without).  A workgroup has one row: a loop over a sequence's rows cost 10 - 17 spilled registers.
-// Workgroups without a page leave, a row that one workgroup has whole needs no merge, a row of one page no meeting.
-// A workgroup per 16 heads whose four waves took half a page a turn, copied through registers (attn_keep_split_kernel),
-// left half the CUs idle.  576 entries, before -> after with the merge: 64 sequences of 300 - 900 tokens with 32 heads
-// 51 -> 31 us (alone; 61 -> 51 a layer's pass, which the host now bounds), one of 600 36 -> 19, eight of 600 37 -> 18, 64
-// of 600 39 -> 30, with 64 heads 39 -> 33; 16 of 2,000 90 -> 32, 64 of them 91 -> 46, through a window of 1,024
-// 53 -> 36.
-constexpr int kStreams = 4;
-
-// What a row of the step sees: pages [0, n_keep) of its sequence s (-1: none, a row of a captured step beyond those of
-// its sequences) hold the kept first tokens, `skip` pages follow that are not read, then those of the window up to the
-// row's own.
-struct RowPages {
-  int s, pi, jwin, kf, n_keep, skip, pages;                   // pi: query, jwin: window's first key, kf: kept keys before it
-};
-// Most steps have a row a sequence: then row t is sequence t's, whose numbers are on their way at once.
-__device__ __forceinline__ RowPages row_pages(const KeepArgs& a, int NA, int t) {
-  RowPages r;
-  const int i = min(t, NA - 1);
-  int from = a.q_start[i], n = a.q_len[i], kv = a.kv_len[i];
-  r.s = i;
-  if (from > t || from + n <= t) {
-    r.s = -1;
-    for (int b = 0; b < NA && r.s < 0; b += 64) {
-      const int x = b + (threadIdx.x & 63), xf = x < NA ? a.q_start[x] : 0, xn = x < NA ? a.q_len[x] : 0;
-      const uint64_t m = __builtin_amdgcn_ballot_w64(xf <= t && t < xf + xn);
-      if (m != 0) r.s = b + __builtin_ctzll(m);
-    }
-    if (r.s < 0) return r;
-    from = a.q_start[r.s];
-    n = a.q_len[r.s];
-    kv = a.kv_len[r.s];
-  }
-  r.pi = kv - n + t - from;
-  r.jwin = a.window > 0 ? max(0, r.pi - a.window + 1) : 0;
-  r.kf = a.window > 0 ? min(a.keep_first, r.jwin) : 0;
-  const int pg_win = r.jwin / WBS;
-  r.n_keep = min((r.kf + WBS - 1) / WBS, pg_win);
-  r.skip = pg_win - r.n_keep;
-  r.pages = r.pi / WBS + 1 - r.skip;
-  return r;
-}
-// What a row's weighted values of head h are multiplied by, given the maximum and sum of all its keys: the sink's part
-// of the sum, a gate per head.
-template <int MODE>
-__device__ __forceinline__ float whole(const KeepArgs& a, int64_t t, int h, float top, float sum) {
-  float f = 1.f, l = sum;
-  if constexpr (MODE < 2) {
-    const float sink = a.head_bias != nullptr ? a.head_bias[h] * kLog2e : kNegInfW, m = fmaxf(top, sink);
-    f = top == kNegInfW ? 0.f : __builtin_amdgcn_exp2f(top - m);
-    l = (top == kNegInfW ? 0.f : f * sum) + (sink == kNegInfW ? 0.f : __builtin_amdgcn_exp2f(sink - m));
-  }
-  float mul = MODE >= 2 ? a.out_mult : (l > 0.f ? a.out_mult / l : 0.f);
-  if (a.gate != nullptr && a.gate_w == 1)
-    mul /= 1.0f + __expf(-ldf(static_cast<const bf16_t*>(a.gate) + t * a.gate_stride + h));
-  return f * mul;
-}
-// Four neighbouring outputs of head h, through a gate per output
-template <int vdim>
-__device__ __forceinline__ void store_gated(const KeepArgs& a, float (&y)[4], int64_t t, int h, int dv) {
-  if (a.gate != nullptr && a.gate_w > 1) {
-    const float4 x = ld4(static_cast<const bf16_t*>(a.gate) + t * a.gate_stride + (int64_t)h * vdim + dv);
-    y[0] /= 1.0f + __expf(-x.x);
-    y[1] /= 1.0f + __expf(-x.y);
-    y[2] /= 1.0f + __expf(-x.z);
-    y[3] /= 1.0f + __expf(-x.w);
-  }
-  *reinterpret_cast<uint2*>(static_cast<bf16_t*>(a.out) + t * a.out_stride + (int64_t)h * vdim + dv) =
-      make_uint2(rfq::pack_bf16x2(y[0], y[1]), rfq::pack_bf16x2(y[2], y[3]));
-}
-// How many of S workgroups have a part in the row: those with pages, the first in any case
-__device__ __forceinline__ int row_shares(const RowPages& r, int S) {
-  return min(S, max(1, (r.pages + kStreams - 1) / kStreams));
-}
-
-template <int DK, int DV, int MODE>
-__global__ __launch_bounds__(128 * kStreams, 2) void attn_keep_streams_kernel(const KeepArgs a, float* part, int T,
-                                                                                int NA) {
-  constexpr int E = 32 * DK, vdim = 16 * DV, PGS = WBS * E, ND = WBS * E / 1024, S16 = vdim / 2 + 4;
-  static_assert(DK > 10 && E % 64 == 0 && WBS * E % 1024 == 0 && 2 * kStreams * 16 * S16 * 4 <= kStreams * PGS * 2, "the partial results take the pages' place");
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int wid = __builtin_amdgcn_readfirstlane(tid >> 6), st = wid >> 1;
-  const int64_t t = blockIdx.x;
-  const int S = gridDim.z, z = blockIdx.z;
-  const RowPages row = row_pages(a, NA, (int)t);
-  if (row.s < 0) return;
-  const int pi = row.pi, jwin = row.jwin, kf = row.kf, n_keep = row.n_keep, skip = row.skip, pages = row.pages;
-  const int shares = row_shares(row, S);
-  if (z >= shares) return;                                    // no page for this workgroup
-  const int col = lane & 15, grp = lane >> 4;
-  const int rep = a.H / a.G, per = (rep + 31) / 32;
-  const int g = (int)blockIdx.y / per, h0 = ((int)blockIdx.y - g * per) * 32;
-  const int hd = h0 + (wid & 1) * 16 + col;
-  const bool idle = h0 + (wid & 1) * 16 >= rep;               // a wave that only copies pages
-  const int hh = g * rep + min(hd, rep - 1);                  // past the last head: it once more, not stored
-  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-  short* const P = reinterpret_cast<short*>(smem) + st * PGS; // this stream's page
-  float* const meet = reinterpret_cast<float*>(smem);         // later [wave][16][S16]
-  float* const ml = reinterpret_cast<float*>(smem + kStreams * PGS * 2);     // [wave][16] maxima, as many sums
-  float* const share = ml + 4 * kStreams * 16;                // [head][stream]
-  unsigned char* const qs = reinterpret_cast<unsigned char*>(share + 32 * kStreams);   // [half][stream] KB of queries
-  typedef const __attribute__((address_space(4))) int32_t const_i32;
-  const_i32* bt = (const_i32*)(uintptr_t)(a.bt + (int64_t)row.s * a.maxb);
-  const float qmul = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(
-      a.scale * (MODE % 2 == 1 ? 2.f * kLog2e / a.softcap : MODE == 2 ? -kLog2e : kLog2e))));
-  const float cap2 = MODE % 2 == 1 ? a.softcap * kLog2e : 0.f;
-  const float hb = MODE >= 2 && a.head_bias != nullptr ? a.head_bias[hh] * kLog2e : 0.f;
-  const int ksw = wide_swizzle(col), vrow = 4 * grp + (col >> 2), vsw = wide_swizzle(vrow);
-
-  const int turns = (pages - z * kStreams + S * kStreams - 1) / (S * kStreams);
-  constexpr int NQ = (DK + kStreams - 1) / kStreams;
-  float4 qx[NQ], qy[NQ];                                    // on their way before the page is
-  {
-    const float* qp = a.q + (t * a.H + hh) * E + grp * 8;
-#pragma unroll
-    for (int x = 0; x < NQ; ++x) {
-      const int ks = min(x * kStreams + st, DK - 1);
-      qx[x] = *reinterpret_cast<const float4*>(qp + ks * 32);
-      qy[x] = *reinterpret_cast<const float4*>(qp + ks * 32 + 4);
-    }
-  }
-  auto offset = [&](int x, int l) {                         // bytes from the page's first, of load x of this wave
-    const int p = ((wid & 1) + 2 * x) * 64 + l, rw = p / (E / 8), c = p - rw * (E / 8);
-    return (uint32_t)(rw * E + ((c & ~7) | ((c & 7) ^ wide_swizzle(rw))) * 8) * 2;
-  };
-  auto page_at = [&](int i) {
-    return static_cast<const char*>(a.k_cache) + ((int64_t)bt[i < n_keep ? i : i + skip] * a.G + g) * PGS * 2;
-  };
-  {
-    uint32_t from[ND];                                      // computed while the page's number is on its way
-    int l = lane;
-    asm volatile("" : "+v"(l));                             // and here: before the loop they would be spilled
-#pragma unroll
-    for (int x = 0; x < ND; ++x) {
-      from[x] = offset(x, l);
-      asm volatile("" : "+v"(from[x]));
-    }
-    if (z * kStreams + st < pages) {
-      const char* kb = page_at(z * kStreams + st);
-#pragma unroll
-      for (int x = 0; x < ND; ++x)
-        rfq::glds16(reinterpret_cast<const bf16_t*>(kb + from[x]), reinterpret_cast<bf16_t*>(P + ((wid & 1) + 2 * x) * 512));
-    }
-  }
-  auto fetch = [&](int i) {
-    const char* kb = page_at(i);
-    int l = lane;
-    asm volatile("" : "+v"(l));                             // the offsets are computed here, not kept
-#pragma unroll
-    for (int x = 0; x < ND; ++x)
-      rfq::glds16(reinterpret_cast<const bf16_t*>(kb + offset(x, l)), reinterpret_cast<bf16_t*>(P + ((wid & 1) + 2 * x) * 512));
-  };
-  // a stream packs every fourth piece of the queries and leaves it for the others
-  s16x8 q[DK];
-#pragma unroll
-  for (int x = 0; x < NQ; ++x) {
-    const float f[8] = {qx[x].x, qx[x].y, qx[x].z, qx[x].w, qy[x].x, qy[x].y, qy[x].z, qy[x].w};
-    if (x > 0) __syncthreads();
-    *reinterpret_cast<s16x8*>(qs + ((wid & 1) * kStreams + st) * 1024 + lane * 16) = rfq::pack8(f);
-    __syncthreads();
-#pragma unroll
-    for (int u = 0; u < kStreams; ++u)
-      if (x * kStreams + u < DK)
-        q[x * kStreams + u] = *reinterpret_cast<const s16x8*>(qs + ((wid & 1) * kStreams + u) * 1024 + lane * 16);
-  }
-  f32x4 o[DV];
-#pragma unroll
-  for (int m = 0; m < DV; ++m) o[m] = (f32x4){0.f, 0.f, 0.f, 0.f};
-  float mrun = kNegInfW, lrun = 0.f;
-  for (int k = 0; k < turns; ++k) {
-    const int i = (k * S + z) * kStreams + st, jb = (i < n_keep ? i : i + skip) * WBS;
-    const bool live = i < pages;
-    __builtin_amdgcn_s_waitcnt(0x0F70);                     // vmcnt(0)
-    __syncthreads();
-    // rows past the query were never written, rows out of its sight may hold infinities: zeros
-    const bool edge = live && (jb + WBS - 1 > pi || (jb < jwin && jb + WBS > kf));
-    if (edge)
-      for (int x = (wid & 1) * 64 + lane; x < WBS * (E / 8); x += 128) {
-        const int j = jb + x / (E / 8);
-        if (j > pi || (j < jwin && j >= kf)) *reinterpret_cast<s16x8*>(P + x * 8) = (s16x8){0, 0, 0, 0, 0, 0, 0, 0};
-      }
-    __syncthreads();
-    if (live && !idle) {
-      f32x4 sc[2][2];                                       // two chains per half page
-#pragma unroll
-      for (int kt = 0; kt < 2; ++kt) {
-        sc[kt][0] = sc[kt][1] = (f32x4){0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int ks = 0; ks < DK; ++ks) {
-          const s16x8 kv = *reinterpret_cast<const s16x8*>(P + col * E + ((4 * (ks & 1) + grp) ^ ksw) * 8 + kt * 16 * E + (ks >> 1) * 64);
-          f32x4& acc = sc[kt][ks & 1];
-          acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(kv), as_bf16x8(q[ks]), acc, 0, 0, 0);
-        }
-      }
-      float p[8];
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        float x = (sc[e >> 2][0][e & 3] + sc[e >> 2][1][e & 3]) * qmul;
-        if constexpr (MODE % 2 == 1) x = cap2 - 2.f * cap2 * __builtin_amdgcn_rcpf(__builtin_amdgcn_exp2f(x) + 1.f);
-        if constexpr (MODE >= 2) x = __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f((MODE == 3 ? -x : x) - hb));
-        p[e] = x;
-      }
-      if (edge) {
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          const int j = jb + (e >> 2) * 16 + grp * 4 + (e & 3);
-          const bool ok = (j <= pi) & ((j >= jwin) | (j < kf));
-          p[e] = ok ? p[e] : MODE >= 2 ? 0.f : kNegInfW;
-        }
-      }
-      if constexpr (MODE < 2) {
-        float mx = fmaxf(fmaxf(fmaxf(p[0], p[1]), fmaxf(p[2], p[3])), fmaxf(fmaxf(p[4], p[5]), fmaxf(p[6], p[7])));
-        mx = other_half_max(other_row_max(mx));
-        const bool moves = mx > mrun + kDeferW;             // also for the first keys: mrun = -inf
-        if (__builtin_amdgcn_ballot_w64(moves) != 0ull) {
-          const float mn = moves ? mx : mrun;
-          const float alpha = moves ? __builtin_amdgcn_exp2f(mrun - mn) : 1.f;
-          mrun = mn;
-          lrun *= alpha;
-#pragma unroll
-          for (int m = 0; m < DV; ++m) o[m] *= alpha;
-        }
-        const float mu = mrun == kNegInfW ? 0.f : mrun;     // no visible key so far: every weight 0
-        float l0 = 0.f, l1 = 0.f;
-#pragma unroll
-        for (int e = 0; e < 8; e += 2) {
-          p[e] = __builtin_amdgcn_exp2f(p[e] - mu);
-          p[e + 1] = __builtin_amdgcn_exp2f(p[e + 1] - mu);
-          l0 += p[e];
-          l1 += p[e + 1];
-        }
-        lrun += l0 + l1;
-      }
-      s16x8 phi, plo;
-      split_bf16w(p, phi, plo);
-#pragma unroll
-      for (int m = 0; m < DV; m += 4) {
-        s16x8 v[4];
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-          const short* vp = P + vrow * E + ((2 * u + ((col >> 1) & 1)) ^ vsw) * 8 + (col & 1) * 4 + (m >> 2) * 64;
-          const s16x4 a0 = rfq::ds_read_tr16(vp), a1 = rfq::ds_read_tr16(vp + 16 * E);
-          v[u] = (s16x8){a0[0], a0[1], a0[2], a0[3], a1[0], a1[1], a1[2], a1[3]};
-        }
-#pragma unroll
-        for (int u = 0; u < 4; ++u)
-          o[m + u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(v[u]), as_bf16x8(phi), o[m + u], 0, 0, 0);
-#pragma unroll
-        for (int u = 0; u < 4; ++u)
-          o[m + u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(v[u]), as_bf16x8(plo), o[m + u], 0, 0, 0);
-      }
-    }
-    __syncthreads();                                        // both waves are done with the page
-    if (const int n = i + S * kStreams; n < pages) fetch(n);
-  }
-  // ---- streams meet, half the channels at a time
-  const float l = both_halves_sum(both_rows_sum(lrun));
-  // scores that are no numbers leave the maximum at -inf, which marks a stream without visible keys
-  const float mx = MODE >= 2 || (l != 0.f && mrun == kNegInfW) ? 0.f : mrun;
-  if (pages == 1) {                                           // nobody to meet
-    if (st > 0 || hd >= rep) return;
-    const float f = whole<MODE>(a, t, hh, mx, l);
-#pragma unroll
-    for (int m = 0; m < DV; ++m) {
-      float y[4] = {o[m][0] * f, o[m][1] * f, o[m][2] * f, o[m][3] * f};
-      store_gated<vdim>(a, y, t, hh, 16 * m + 4 * grp);
-    }
-    return;
-  }
-  if (grp == 0) {
-    ml[wid * 16 + col] = mx;
-    ml[(2 * kStreams + wid) * 16 + col] = l;
-  }
-  float* const part_ml = part + (int64_t)T * S * a.H * vdim;
-#pragma unroll
-  for (int mp = 0; mp < 2; ++mp) {
-    if (mp > 0) __syncthreads();
-#pragma unroll
-    for (int m = 0; m < DV / 2; ++m)
-      *reinterpret_cast<f32x4*>(meet + (wid * 16 + col) * S16 + 16 * m + 4 * grp) = o[mp * (DV / 2) + m];
-    __syncthreads();
-    if (mp == 0) {
-      // what the streams' parts count, and the workgroup's own maximum and sum: a thread per head and stream
-      if (tid < 32 * kStreams) {
-        const int c = tid >> 2, u = tid & 3, w = 2 * u + (c >> 4);
-        const float mu = ml[w * 16 + (c & 15)];
-        float top = fmaxf(mu, __shfl_xor(mu, 1, 64));
-        top = fmaxf(top, __shfl_xor(top, 2, 64));
-        const float f = mu == kNegInfW ? 0.f : MODE >= 2 ? 1.f : __builtin_amdgcn_exp2f(mu - top);
-        float sum = f == 0.f ? 0.f : f * ml[(2 * kStreams + w) * 16 + (c & 15)];
-        sum += __shfl_xor(sum, 1, 64);
-        sum += __shfl_xor(sum, 2, 64);
-        if (shares > 1) {
-          share[c * 4 + u] = f;
-          if (u == 0 && h0 + c < rep)
-            *reinterpret_cast<float2*>(part_ml + 2 * ((t * S + z) * a.H + g * rep + h0 + c)) = make_float2(top, sum);
-        } else {                                              // no other part: what the merge would do
-          share[c * 4 + u] = f * whole<MODE>(a, t, g * rep + min(h0 + c, rep - 1), top, sum);
-        }
-      }
-      __syncthreads();
-    }
-    constexpr int NX = 32 * (vdim / 8) / (128 * kStreams);  // pieces of four channels a thread
-    static_assert(NX * 128 * kStreams == 32 * (vdim / 8), "");
-#pragma unroll 2
-    for (int n = 0; n < NX; ++n) {
-      const int x = tid + n * 128 * kStreams, c = x / (vdim / 8), dp = (x - c * (vdim / 8)) * 4;
-      const float4 f = *reinterpret_cast<const float4*>(share + 4 * c);
-      const float fs[4] = {f.x, f.y, f.z, f.w};
-      float y[4] = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int u = 0; u < kStreams; ++u) {
-        const float4 v = *reinterpret_cast<const float4*>(meet + ((2 * u + (c >> 4)) * 16 + (c & 15)) * S16 + dp);
-        y[0] += fs[u] * v.x; y[1] += fs[u] * v.y; y[2] += fs[u] * v.z; y[3] += fs[u] * v.w;
-      }
-      const int hc = g * rep + h0 + c, dv = mp * (vdim / 2) + dp;
-      if (h0 + c >= rep) continue;
-      if (shares > 1)
-        *reinterpret_cast<float4*>(part + ((t * S + z) * a.H + hc) * vdim + dv) = make_float4(y[0], y[1], y[2], y[3]);
-      else
-        store_gated<vdim>(a, y, t, hc, dv);
-    }
-  }
-}
-
-// One wave per row and head: the workgroups' parts, the sink, the gate.
-template <int DV, int MODE>
-__global__ __launch_bounds__(64) void attn_keep_streams_merge_kernel(const KeepArgs a, const float* part, int T, int S,
-                                                                      int NA) {
-  constexpr int vdim = 16 * DV, NC = vdim / 256;              // pieces of four channels a lane
-  const int64_t t = blockIdx.x;
-  const int hx = blockIdx.y, lane = threadIdx.x;
-  const RowPages row = row_pages(a, NA, (int)t);
-  if (row.s < 0) return;
-  const int shares = row_shares(row, S);
-  if (shares == 1) return;                                    // its workgroup has stored the row itself
-  const float2* ml = reinterpret_cast<const float2*>(part + (int64_t)T * S * a.H * vdim);
-  float top = kNegInfW, l = 0.f;
-  for (int z = 0; z < shares; ++z) top = fmaxf(top, ml[(t * S + z) * a.H + hx].x);
-  float y[NC][4];
-#pragma unroll
-  for (int n = 0; n < NC; ++n) y[n][0] = y[n][1] = y[n][2] = y[n][3] = 0.f;
-  for (int z = 0; z < shares; ++z) {
-    const int64_t at = (t * S + z) * a.H + hx;
-    const float2 m = ml[at];
-    if (m.x == kNegInfW) continue;                          // a workgroup without visible keys
-    const float f = MODE >= 2 ? 1.f : __builtin_amdgcn_exp2f(m.x - top);
-    l += f * m.y;
-#pragma unroll
-    for (int n = 0; n < NC; ++n) {
-      const float4 v = *reinterpret_cast<const float4*>(part + at * vdim + 256 * n + 4 * lane);
-      y[n][0] += f * v.x; y[n][1] += f * v.y; y[n][2] += f * v.z; y[n][3] += f * v.w;
-    }
-  }
-  const float mul = whole<MODE>(a, t, hx, top, l);
-#pragma unroll
-  for (int n = 0; n < NC; ++n) {
-#pragma unroll
-    for (int e = 0; e < 4; ++e) y[n][e] *= mul;
-    store_gated<vdim>(a, y[n], t, hx, 256 * n + 4 * lane);
-  }
-}
-
 // ------------------------------------------------------------------ launcher
 namespace {
 bool plain_sizes(int DK, int DV) { return DK >= 1 && DK <= 4 && (DV == 2 || DV == 4 || DV == 8); }
@@ -1367,57 +987,6 @@ void launch_attn_keep_wide_rows(const float* q, const void* k_cache, int64_t vrs
   if (E == 576) ROWS_GO(18, 32);
   else ROWS_GO(10, 16);
 #undef ROWS_GO
-}
-
-// How many workgroups share a row's pages, 0 where the streams are not the way: more than the 16 heads of one wave,
-// room for two workgroups or more a row (128 sequences of 600 with 32 heads, two each: 43 -> 40 us), and more than 20
-// pages that a row may see, by its table and window.  With fewer the scratch and the second launch cost a layer's pass
-// that the host bounds 4 us (32 heads, 1 - 64 sequences of 400 tokens, tables as wide: 47 us split over waves, 51 in
-// streams; of 600 49 - 52 and 51; of 900 60 - 64 and 51.5).  Captured steps have wide tables over any number of pages:
-// there a row of one page takes 14.8 us either way, four pages 18.8 and 17.1, nineteen 23 - 38 and 19 - 29.
-// Of up to NA rows a sequence may have several: each has workgroups of its own, as in a captured step rows of an extend
-// stand where other sequences are padding (one sequence of 600 tokens with 16 rows, 16 of one and 15 without: 143 us
-// split over waves, 269 with an extend's rows one after another, 23 side by side).
-int keep_streams(int T, int NA, int H, int G, int E, int vdim, bool shared, int maxb, int window, int keep_first) {
-  const int rep = H / G;
-  if (!shared || E != 576 || vdim != 512 || rep <= 16 || NA <= 0 || H > 65535) return 0;
-  const int64_t wgs = (int64_t)NA * G * ((rep + 31) / 32);
-  // pages that a row can see: of its table, of the window and of the kept first tokens
-  const int64_t seen = ((int64_t)window + WBS - 2) / WBS + 1 + ((int64_t)keep_first + WBS - 1) / WBS;
-  const int64_t most = window > 0 ? std::min<int64_t>(maxb, seen) : maxb;
-  const int S = (int)std::min(256 / std::max<int64_t>(wgs, 1), std::min<int64_t>((most + kStreams - 1) / kStreams, 16));
-  return S >= 2 && most > 20 && T <= NA ? S : 0;
-}
-int64_t keep_streams_floats(int T, int S, int H, int vdim) { return (int64_t)T * S * H * (vdim + 2); }
-
-template <int DK, int DV, int MODE>
-static void launch_streams_one(const KeepArgs& a, int T, int NA, int S, float* part) {
-  constexpr size_t lds = (size_t)kStreams * WBS * 32 * DK * 2 + (4 * kStreams * 16 + 32 * kStreams) * sizeof(float) + 2 * kStreams * 1024;
-  static_assert(lds <= 160 * 1024, "LDS of a CU");
-  static bool attr = false;
-  if (!attr) {
-    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&attn_keep_streams_kernel<DK, DV, MODE>),
-                              hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
-    attr = true;
-  }
-  hipLaunchKernelGGL((attn_keep_streams_kernel<DK, DV, MODE>), dim3(T, a.G * ((a.H / a.G + 31) / 32), S), dim3(128 * kStreams),
-                     lds, a.s, a, part, T, NA);
-  hipLaunchKernelGGL((attn_keep_streams_merge_kernel<DV, MODE>), dim3(T, a.H), dim3(64), 0, a.s, a, part, T, S, NA);
-}
-
-void launch_attn_keep_streams(const float* q, const void* k_cache, int64_t vrs, const int32_t* bt, int maxb,
-                              const int32_t* q_start, const int32_t* q_len, const int32_t* kv_len, int T, int NA, int S,
-                              const float* head_bias, const void* gate, int64_t gate_stride, int gate_w, void* out,
-                              int64_t out_stride, float scale, int window, int keep_first, bool sigmoid, int H, int G,
-                              float softcap, float out_mult, float* part, hipStream_t s) {
-  const KeepArgs a{q, k_cache, k_cache, vrs, bt, maxb, q_start, q_len, kv_len, nullptr, nullptr,
-                   0, head_bias, gate, gate_stride, gate_w, out, out_stride, scale, window, keep_first,
-                   sigmoid, H, G, softcap, out_mult, s};
-  const bool cap = softcap > 0.f;
-  if (sigmoid && cap) launch_streams_one<18, 32, 3>(a, T, NA, S, part);
-  else if (sigmoid) launch_streams_one<18, 32, 2>(a, T, NA, S, part);
-  else if (cap) launch_streams_one<18, 32, 1>(a, T, NA, S, part);
-  else launch_streams_one<18, 32, 0>(a, T, NA, S, part);
 }
 
 bool launch_attn_keep_mfma(const float* q, const void* k_cache, const void* v_cache, int64_t vrs,

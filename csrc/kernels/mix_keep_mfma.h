@@ -1,4 +1,5 @@
-// What the kernels of attn_keep_window on MFMA tiles share (mix_keep_attn_mfma.hip, mix_keep_latent.hip).
+// What the kernels of attn_keep_window on MFMA tiles share (mix_keep_attn_mfma.hip, mix_keep_latent.hip,
+// mix_keep_streams.hip).
 #pragma once
 #include <utility>
 
@@ -36,6 +37,15 @@ __device__ __forceinline__ float other_half_max(float x) {
 }
 __device__ __forceinline__ float both_halves_sum(float x) {
   const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+// the same over lanes 16 away
+__device__ __forceinline__ float other_row_max(float x) {
+  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+__device__ __forceinline__ float both_rows_sum(float x) {
+  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
   return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
 

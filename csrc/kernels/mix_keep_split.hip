@@ -11,8 +11,7 @@
 // maximum, sum, weighted values) meet in LDS at the end.  Measured: 37 us (4.5 TB/s; 44 where no cache holds the pages),
 // 15 us and 54 us.  (Groups of up to eight heads with keys and values of 64 or 128, no more rows than sequences, do not
 // come here: mix_keep_row.hip.  Nor do steps of the 576-wide latent with more than 16 heads, no more rows than sequences
-// and more than 20 pages to see while CUs are free: a row's pages are split over workgroups as well,
-// attn_keep_streams_kernel.)
+// and more than 13 pages to see while CUs are free: a row's pages are split over workgroups as well, mix_keep_streams.hip.)
 //
 // The 16 MFMA columns are (row, head) pairs of one key/value head, so the rows of a short extend and
 // the heads of a group share one pass.
@@ -394,7 +393,7 @@ static void launch_split_one(const KeepSplitArgs& a, int NA, int z, hipStream_t 
 // time then.  The wide latent's staged page leaves room for four, one workgroup to a CU; once there are more
 // workgroups than CUs the prompts' kernel takes its rows, which reads a page once for all heads, not for every
 // 16 of them (64 heads of 576: 128 sequences of 600 tokens 78 us split, 54 there; 64 of them 40 and 53; where rows may
-// see more than 20 pages, steps of no more rows than sequences have gone to keep_streams' workgroups before).  Many
+// see more than 13 to 20 pages, steps of no more rows than sequences have gone to keep_streams' workgroups before).  Many
 // workgroups of large groups in plain sizes: two waves, or one, whose partial results need no merge (512 sequences of
 // 100 tokens, 32 heads over 2 of 128: 23 us with four waves, 20 with one; of 1,000: 100 and 99).
 // Column tiles side by side: as many as the sequences have on the average, more where CUs would idle (one

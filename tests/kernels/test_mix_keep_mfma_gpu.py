@@ -187,6 +187,22 @@ def test_wide_rows_in_streams_of_many_turns(H, G, n):
     _check(H, G, 576, 512, True, seqs=seqs, window=1000, keep_first=70, sigmoid=True, bias=True)
 
 
+@pytest.mark.parametrize("H,G,n", [(33, 1, 100), (64, 1, 128), (48, 1, 90), (128, 2, 40)])
+def test_wide_rows_of_64_heads_together(H, G, n):
+    """Two workgroups a row only where 64 heads share one: one to six pages a workgroup, a last tile without heads."""
+    seqs = [(353, 1), (352, 1), (32, 1), (33, 1), (65, 1), (300, 2), (97, 1), (450, 1), (1, 1)]
+    seqs += [(40, 0)] * (n - len(seqs))
+    _check(H, G, 576, 512, True, seqs=seqs + [(700, 0)], rising=0.1, bias=True, gate="head")
+    _check(H, G, 576, 512, True, seqs=seqs + [(700, 0)], softcap=20.0, gate="output", out_mult=0.6)
+    _check(H, G, 576, 512, True, seqs=seqs[1:] + [(800, 1)], window=700, keep_first=70, sigmoid=True, bias=True)
+
+
+# Shares of one page and more from fourteen pages to see on
+@pytest.mark.parametrize("kv", [417, 448, 449, 480])
+def test_wide_rows_of_few_pages_in_streams(kv):
+    _check(32, 1, 576, 512, True, seqs=[(kv, 1), (1, 1), (64, 1), (65, 1), (129, 1), (40, 0)], bias=True, gate="head")
+
+
 def test_few_pages_under_a_wide_table():
     """Workgroups without a page cost nothing: 20 tokens take about as long where the table has room for 8,192 (14.5
     us both; 21.5 when all of them took part)."""
