@@ -12,6 +12,7 @@
 // 16-byte pieces.  Y comes out transposed in the accumulators (A = W, B = X), so a lane holds
 // neighbouring entries of a row.
 #include <algorithm>
+#include <type_traits>
 
 #include "common.h"
 #include "mix_common.h"
@@ -162,7 +163,7 @@ __global__ __launch_bounds__(256) void rank_product_f32_kernel(const float* __re
 // latent space, head by head, into slices of wider rows.  A wave makes 16 rows of 64 columns: their W passes through its
 // piece of LDS, 64 terms at a time, and is read back transposed.  What bounds it: launch and three trips to memory, 4 - 5 us;
 // the library's takes 5 - 6 and 18 us of the host, 9 here, which bounded a decode step (64 rows of 32 heads, 128 to
-// 512: 5.6 -> 4.7 us, the pass 49 -> 41).  From 2^20 results on the library's tiles are better (64 heads 6.8 us for 7.9).
+// 512: 5.6 -> 4.7 us, the pass 49 -> 41).  Up to 2^20 results (64 heads 7.9 us for the library's 6.8).
 template <int KS>
 __global__ __launch_bounds__(256) void batch_product_kernel(const bf16_t* __restrict__ x, int64_t xb, int64_t xs,
                                                             const bf16_t* __restrict__ w, int64_t wb, int64_t ws,
@@ -223,6 +224,87 @@ __global__ __launch_bounds__(256) void batch_product_kernel(const bf16_t* __rest
   for (int i = 0; i < 4; ++i) st4(to + 16 * i, make_float4(c[i][0], c[i][1], c[i][2], c[i][3]));
 }
 
+// The same for many rows: a wave keeps its 64 columns' W and goes through blocks of 16 rows, every gridDim.y-th, the next
+// one's X on its way meanwhile; the workgroup's columns of a block leave by way of LDS, 1 KB to an access, many results past the
+// caches (PAST).
+// What bounds it: the results' bytes.  32 heads, 8,192 rows, 128 to 512 (537 MB): 97 us, 5.5 TB/s, as fast as they can be
+// filled with a number (102); the library's product 153.  Stored as the tiles lie, 64 bytes of 16 rows to an access, 206; 256
+// bytes of a row 171; 1 KB 158; past the caches 97.  2,067 rows 30.2 for 43.1, 1,031 18.3 for 23.1, 600 13.6 for 15.4.
+constexpr int kBatchWaves = 8;
+template <int KS, bool PAST>
+__global__ __launch_bounds__(64 * kBatchWaves, 4) void batch_rows_kernel(const bf16_t* __restrict__ x, int64_t xb, int64_t xs,
+                                                                         const bf16_t* __restrict__ w, int64_t wb, int64_t ws,
+                                                                         float* __restrict__ y, int64_t yb, int64_t ys, int M) {
+  constexpr int WR = 64 + 8;                                 // shorts per row of a wave's W in LDS
+  extern __shared__ __attribute__((aligned(16))) float blocks[];     // [2][16][columns + 4]
+  const int lane = threadIdx.x & 63, col = lane & 15, grp = lane >> 4, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int nthr = blockDim.x, n0 = blockIdx.x * nthr, FR = nthr + 4;      // a column per thread
+  x += blockIdx.z * xb;
+  w += blockIdx.z * wb + n0 + 64 * wave;
+  y += blockIdx.z * yb + n0;
+  auto fetch = [&](s16x8 (&b)[KS], int m) {
+    const bf16_t* xr = x + (int64_t)min(m + col, M - 1) * xs + 8 * grp;
+#pragma unroll
+    for (int k = 0; k < KS; ++k) b[k] = *reinterpret_cast<const s16x8*>(xr + 32 * k);
+  };
+  const int step = 16 * gridDim.y;
+  s16x8 b[KS];
+  fetch(b, 16 * blockIdx.y);
+  s16x8 a[4][KS];
+  short* S = reinterpret_cast<short*>(blocks) + wave * 32 * WR;
+#pragma unroll
+  for (int k = 0; k < KS; ++k) {
+    s16x8 raw[4];                                            // eight rows to a load of the wave
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      raw[i] = *reinterpret_cast<const s16x8*>(w + (int64_t)(k * 32 + 8 * i + (lane >> 3)) * ws + 8 * (lane & 7));
+#pragma unroll
+    for (int i = 0; i < 4; ++i) *reinterpret_cast<s16x8*>(S + (8 * i + (lane >> 3)) * WR + 8 * (lane & 7)) = raw[i];
+    // a wave's LDS accesses are in order: this keeps the compiler's
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const short* p = S + (8 * grp + (col >> 2)) * WR + 16 * i + 4 * (col & 3);
+      const rfq::s16x4 lo = rfq::ds_read_tr16(p), hi = rfq::ds_read_tr16(p + 4 * WR);
+      a[i][k] = (s16x8){lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+    }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  }
+  __syncthreads();                                           // every wave has its W: blocks take its place
+  int buf = 0, m = 16 * blockIdx.y;
+  auto block = [&](auto whole) {
+    f32x4 c[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) c[i] = (f32x4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int k = 0; k < KS; ++k)
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        c[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(a[i][k]), as_bf16x8(b[k]), c[i], 0, 0, 0);
+    float* const F = blocks + buf * 16 * FR;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) *reinterpret_cast<f32x4*>(F + col * FR + 64 * wave + 16 * i + 4 * grp) = c[i];
+    if constexpr (whole) fetch(b, m + step);                 // past the last row: that one again
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int p = threadIdx.x + j * nthr, r = p / (nthr / 4), e = (p - r * (nthr / 4)) * 4;
+      f32x4* const to = reinterpret_cast<f32x4*>(y + (int64_t)(m + r) * ys + e);
+      const f32x4 v = *reinterpret_cast<const f32x4*>(F + r * FR + e);
+      if (!whole && m + r >= M) continue;
+      if constexpr (PAST) __builtin_nontemporal_store(v, to);
+      else *to = v;
+    }
+  };
+  // only whole blocks in the loop: behind a store that may be left out the compiler waits for all of them, not for X alone
+  for (; m + 16 <= M; m += step, buf ^= 1) block(std::true_type{});
+  if (m < M) block(std::false_type{});
+}
+
 // ------------------------------------------------------------------ launcher
 bool rank_product_ok(int64_t M, int64_t N, int64_t K) {
   return M >= 1 && K >= 32 && K <= 128 && K % 32 == 0 && N >= 4 && N % 4 == 0 && M <= (1 << (K > 96 ? 20 : 21)) / N;
@@ -279,13 +361,48 @@ void launch_rank_product_f32(const float* x, int64_t xs, const float* w, int64_t
 #undef RANK_GO
 }
 
+// Up to 2^20 results a launch is what counts.  Above, the kernel for many rows is slower than the library's in two places,
+// measured from 1 to 128 matrices, 64 to 4,096 columns, 64 to 8,192 rows: 128 terms with fewer rows than repay W's way into
+// registers (32 x 512 columns, 300 rows 10.2 us for 9.4, 64 x 512, 100 rows 8.5 for 8.2), and results of 2 GB (630 for 593).
+static bool few_results(int64_t B, int64_t M, int64_t N) { return M <= (1 << 20) / N && B <= (1 << 20) / (M * N); }
 bool batch_product_ok(int64_t B, int64_t M, int64_t N, int64_t K) {
-  return B >= 1 && B <= 65535 && M >= 1 && N >= 64 && N % 64 == 0 && N <= 1 << 20 && M <= (1 << 20) / N && B <= (1 << 20) / (M * N) &&
-         K >= 32 && K <= 128 && K % 32 == 0;
+  if (!(B >= 1 && B <= 65535 && M >= 1 && N >= 64 && N % 64 == 0 && N <= 1 << 20 && K >= 32 && K <= 128 && K % 32 == 0)) return false;
+  return few_results(B, M, N) || (M <= (1 << 28) / N && B <= (1 << 28) / (M * N) && (K <= 96 || M >= 500));
 }
 
 void launch_batch_product(const void* x, int64_t xb, int64_t xs, const void* w, int64_t wb, int64_t ws, float* y, int64_t yb,
                           int64_t ys, int B, int M, int N, int K, hipStream_t s) {
+  if (!few_results(B, M, N)) {
+    // a workgroup of eight waves to a CU: two take 107 us for the 97
+    int waves = kBatchWaves;
+    while (N / 64 % waves != 0) --waves;
+    const int across = N / 64 / waves;
+    const int64_t down = std::max<int64_t>(1, 256 * kBatchWaves / waves / ((int64_t)across * B));
+    const dim3 g2(across, std::min<int64_t>((M + 15) / 16, down), B);
+    const size_t lds = std::max<size_t>((size_t)2 * 16 * (64 * waves + 4) * 4, (size_t)waves * 32 * 72 * 2);
+    // more than half of the last cache holds go past it; of fewer the next kernel reads some there (a layer's passes with 64 -
+    // 200 MB of results are 0 - 2 % shorter so, those with more 0 - 1.5 % longer)
+    const bool past = (int64_t)B * M * N > 1 << 25;
+#define ROWS_AS(KS, PAST)                                                                                                        \
+  do {                                                                                                                           \
+    static bool attr = false;                                                                                                    \
+    if (!attr) {                                                                                                                 \
+      (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&batch_rows_kernel<KS, PAST>),                                     \
+                                hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);                                         \
+      attr = true;                                                                                                               \
+    }                                                                                                                            \
+    hipLaunchKernelGGL((batch_rows_kernel<KS, PAST>), g2, dim3(64 * waves), lds, s, (const bf16_t*)x, xb, xs, (const bf16_t*)w, wb, \
+                       ws, y, yb, ys, M);                                                                                        \
+  } while (0)
+#define ROWS_GO(KS) do { if (past) ROWS_AS(KS, true); else ROWS_AS(KS, false); } while (0)
+    if (K == 32) ROWS_GO(1);
+    else if (K == 64) ROWS_GO(2);
+    else if (K == 96) ROWS_GO(3);
+    else ROWS_GO(4);
+#undef ROWS_GO
+#undef ROWS_AS
+    return;
+  }
   const dim3 grid((N + 255) / 256, (M + 15) / 16, B);
 #define BATCH_GO(KS)                                                                                                    \
   hipLaunchKernelGGL((batch_product_kernel<KS>), grid, dim3(256), 0, s, (const bf16_t*)x, xb, xs, (const bf16_t*)w, wb, \

@@ -1244,7 +1244,8 @@ def _short_batch(a, b, out) -> bool:
     (B, M, K), N = a.shape, b.shape[2]
     (x0, x1, x2), (w0, w1, w2), (y0, y1, y2) = a.stride(), b.stride(), out.stride()
     lo, hi, n = (y1, y0, M) if y1 <= y0 else (y0, y1, B)
-    return (1 <= B <= 65535 and M >= 1 and K in (32, 64, 96, 128) and N % 64 == 0 and N >= 64 and B * M * N <= 1 << 20
+    return (1 <= B <= 65535 and M >= 1 and K in (32, 64, 96, 128) and N % 64 == 0 and N >= 64
+            and B * M * N <= 1 << (28 if K <= 96 or M >= 500 else 20) and N <= 1 << 20
             and b.shape == (B, K, N) and out.shape == (B, M, N) and x2 == w2 == y2 == 1 and lo >= N and hi >= n * lo
             and not (x0 | x1 | w0 | w1 | a.storage_offset() | b.storage_offset()) & 7 and not (y0 | y1 | out.storage_offset()) & 3
             and a.device == b.device == out.device)
@@ -1252,8 +1253,9 @@ def _short_batch(a, b, out) -> bool:
 
 def bmm_f32(a, b, out=None):
     """Batched a[B, M, K] . b[B, K, N] on the vendor library with an fp32 result (the
-    accumulator's precision is kept for bf16 operands); ``out`` may be a slice of wider rows.  Few
-    sums of up to 128 terms into ``out`` run on a kernel: the library's host work, 18 us, bounds them."""
+    accumulator's precision is kept for bf16 operands); ``out`` may be a slice of wider rows.  Sums of
+    up to 128 terms into ``out`` run on a kernel: few are bound by the library's host work, 18 us,
+    many by the results' way to memory, which the kernel writes faster."""
     if (out is not None and a.is_cuda and _short_batch(a, b, out) and _plain(a, b) and _plain(out, out)
             and not torch.is_autocast_enabled("cuda")):
         _native.mix_ops().bmm_short(a, b, out)

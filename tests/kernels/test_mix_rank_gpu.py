@@ -120,7 +120,7 @@ def test_fp32_products_keep_autocast_and_derivatives():
 
 
 # rows and columns around a wave's tile, slices of wider rows on all sides, results of rows in either order; what stays with
-# the library: 2^20 results and one row, columns that are no whole tiles, 40 terms, a result in memory of an operand
+# the library: 2^20 results and one row of 128 terms, columns that are no whole tiles, 40 terms, a result in memory of an operand
 @pytest.mark.parametrize("B,M,N", [(1, 1, 64), (3, 17, 320), (32, 64, 512), (32, 65, 512), (2, 5, 72)])
 @pytest.mark.parametrize("K", [32, 64, 96, 128, 40])
 @pytest.mark.parametrize("rows_first", [False, True])
@@ -134,6 +134,15 @@ def test_batches_of_short_products(B, M, N, K, rows_first):
     xd, wd = x.double().cpu(), w.double().cpu()
     tol = K * 2.0 ** -24 * (xd.abs() @ wd.abs())             # as above
     assert bool(((out.double().cpu() - xd @ wd).abs() <= tol).all()) and bool((wide[:, :, N:] == 7.0).all())
+
+
+# more than 2^20 results: workgroups of one, three and eight waves, several columns' workgroups, rows that blocks do not divide,
+# more blocks than workgroups and fewer; 128 terms and fewer than 500 rows stay with the library
+@pytest.mark.parametrize("B,M,N,K", [(70, 501, 64, 128), (9, 500, 576, 96), (9, 499, 576, 128), (2, 2100, 512, 128), (1, 600, 4096, 32),
+                                     (300, 65, 128, 64), (32, 130, 512, 32), (5, 4097, 128, 64)])
+@pytest.mark.parametrize("rows_first", [False, True])
+def test_batches_of_many_rows(B, M, N, K, rows_first):
+    test_batches_of_short_products(B, M, N, K, rows_first)
 
 
 def test_batches_that_the_kernel_leaves_alone():
