@@ -328,12 +328,21 @@ __global__ __launch_bounds__(256) void conv_act_heads_vec_kernel(
   for (int cc = unit_here * dim + threadIdx.x; cc < nc; cc += blockDim.x) o[cc] = ys[cc];
 }
 
+// x / (1 + e^-x), the quotient's rest added once: rounded as a division, for divisors and quotients in the middle of the range.
+// An infinite divisor gives 0, and NaN for -inf.
+__device__ __forceinline__ float silu_p(float x) {
+  const float d = x < -87.f ? __builtin_huge_valf() : 1.f + exp_c(-x), r = __builtin_amdgcn_rcpf(d), q = x * r;
+  return __builtin_amdgcn_div_fixupf(fmaf(fmaf(-d, q, x), r, q), d, x);
+}
+
 // The same for heads of 16, 32, 64, 128 or 256 channels: a wave has 256 channels, four a lane, so a head
 // is a group of dim / 4 lanes and its sum needs no LDS; a thread takes R rows below one another, whose
 // earlier inputs and taps stay in registers.  (Positions rise by one inside a run, so what precedes a
-// row is what preceded the row above, shifted.)  Bound by memory and the fp32 divides: 4,096 rows of 8,192
-// channels, 4 taps, from bf16 took 97 us with a row a block, its taps read again for each and the heads'
-// sums through LDS; 49 us here (4.1 TB/s).
+// row is what preceded the row above, shifted.)  Bound by memory and vector instructions, some 110 a row of 256
+// channels: 4,096 rows of 8,192 channels, 4 taps, from bf16 took 97 us with a row a block, its taps read again for
+// each and the heads' sums through LDS; 45.4 us with expf and a divide (25 instructions for the 16 of silu_p) and
+// with lengths in waves without unit heads, 41.3 now (4.9 TB/s; a layer's pass 264.5 -> 261).  Stored past the
+// caches 8,192 rows take a fifth less, which the kernel that reads them loses again.
 template <typename T, int TAPS, int R>
 __global__ __launch_bounds__(256) void conv_act_heads_rows_kernel(
     const T* __restrict__ x, int64_t x_stride, const float* __restrict__ w,
@@ -344,7 +353,7 @@ __global__ __launch_bounds__(256) void conv_act_heads_rows_kernel(
   constexpr int K = TAPS - 1;
   const int t0 = blockIdx.x * R, c = (blockIdx.y * 256 + threadIdx.x) * 4;
   if (c >= C) return;                                    // whole heads: C is a multiple of dim
-  const bool unit = c < n_unit * dim;
+  const bool unit = c < n_unit * dim, units = __builtin_amdgcn_ballot_w64(unit) != 0ull;
   float wc[4 * TAPS];                                    // [4][taps], read in 16-byte pieces
 #pragma unroll
   for (int k = 0; k < TAPS; ++k) *reinterpret_cast<float4*>(wc + 4 * k) = ld4(w + (int64_t)c * TAPS + 4 * k);
@@ -376,9 +385,8 @@ __global__ __launch_bounds__(256) void conv_act_heads_rows_kernel(
       a2 += wc[2 * TAPS + K - dl] * h[dl - 1].z;
       a3 += wc[3 * TAPS + K - dl] * h[dl - 1].w;
     }
-    float4 y = make_float4(a0 / (1.0f + expf(-a0)), a1 / (1.0f + expf(-a1)), a2 / (1.0f + expf(-a2)),
-                           a3 / (1.0f + expf(-a3)));
-    if (n_unit > 0) {
+    float4 y = make_float4(silu_p(a0), silu_p(a1), silu_p(a2), silu_p(a3));
+    if (units) {
       const float m = 1.0f / sqrtf(group_sum(y.x * y.x + y.y * y.y + y.z * y.z + y.w * y.w, dim >> 2) + unit_eps);
       if (unit) y = make_float4(y.x * m, y.y * m, y.z * m, y.w * m);
     }
