@@ -44,11 +44,33 @@ __global__ __launch_bounds__(256) void token_shift_mix_kernel(
   }
 }
 
+// Four neighbouring entries, PAST: past the caches
+template <bool PAST>
+__device__ __forceinline__ void st4_as(float* p, float4 v) {
+  typedef float f32x4 __attribute__((ext_vector_type(4)));
+  if constexpr (PAST) __builtin_nontemporal_store((f32x4){v.x, v.y, v.z, v.w}, reinterpret_cast<f32x4*>(p));
+  else st4(p, v);
+}
+template <bool PAST>
+__device__ __forceinline__ void st4_as(bf16_t* p, float4 v) {
+  if constexpr (PAST) {
+    typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+    union { bf16_t h[4]; u32x2 w; } u;
+    stf(u.h, v.x);
+    stf(u.h + 1, v.y);
+    stf(u.h + 2, v.z);
+    stf(u.h + 3, v.w);
+    __builtin_nontemporal_store(u.w, reinterpret_cast<u32x2*>(p));
+  } else {
+    st4(p, v);
+  }
+}
+
 // The same, four channels a thread and R rows below one another (d a multiple of 4, rows 16-byte
 // aligned): a row is read once and stays for the row below it, a mix's coefficients are read once for
 // R rows, stores are 8 or 16 bytes.  Bound by memory: 4,096 rows of 4,096 with five mixes in bf16 move
-// 235 MB in 47 us (5.0 TB/s); a channel a lane with two-byte stores took 110 us.
-template <typename T, int R>
+// 235 MB in 45 us (5.2 TB/s; 37.5 call after call); a channel a lane with two-byte stores took 110 us.
+template <typename T, int R, bool PAST>
 __global__ __launch_bounds__(256) void token_shift_mix_vec_kernel(
     const float* __restrict__ x, const float* __restrict__ mu, float* __restrict__ prev,
     const int32_t* __restrict__ row_state, const int32_t* __restrict__ row_back,
@@ -80,8 +102,8 @@ __global__ __launch_bounds__(256) void token_shift_mix_vec_kernel(
 #pragma unroll
     for (int r = 0; r < R; ++r)
       if (t0 + r < Trows)
-        st4(o + (int64_t)r * d, make_float4(a[r].x + b[r].x * m.x, a[r].y + b[r].y * m.y, a[r].z + b[r].z * m.z,
-                                            a[r].w + b[r].w * m.w));
+        st4_as<PAST>(o + (int64_t)r * d, make_float4(a[r].x + b[r].x * m.x, a[r].y + b[r].y * m.y, a[r].z + b[r].z * m.z,
+                                                     a[r].w + b[r].w * m.w));
   }
 }
 
@@ -206,10 +228,16 @@ void launch_token_shift_mix(bool out_f32, const float* x, const float* mu, float
 #define SHIFT_GO(KERNEL, GRID, TT)                                                               \
   hipLaunchKernelGGL(KERNEL, GRID, dim3(256), 0, s, x, mu, prev, row_state, row_back, row_fwd,   \
                      pos, (TT*)out, T, d, NS, slots)
+  // More than half of the last cache holds go past it: the products that read them take as long either way, and what a layer's
+  // other kernels read stays there.  4,096 rows of 4,096, five mixes in bf16 (168 MB): 37.5 us both, a pass with the
+  // recurrence 166 -> 155, with five products 507 -> 505; fp32, 336 MB, 80 -> 69.  Fewer: 2,048 rows of 2,048 with the products
+  // 118 -> 128.
+  const bool past = (int64_t)NS * T * d * (out_f32 ? 4 : 2) > (int64_t)128 << 20;
 #define SHIFT_ALL(TT)                                                                            \
   do {                                                                                           \
-    if (vec && rows4) SHIFT_GO((token_shift_mix_vec_kernel<TT, 4>), dim3((T + 3) / 4, cols), TT); \
-    else if (vec) SHIFT_GO((token_shift_mix_vec_kernel<TT, 1>), dim3(T, cols), TT);              \
+    if (vec && rows4 && past) SHIFT_GO((token_shift_mix_vec_kernel<TT, 4, true>), dim3((T + 3) / 4, cols), TT); \
+    else if (vec && rows4) SHIFT_GO((token_shift_mix_vec_kernel<TT, 4, false>), dim3((T + 3) / 4, cols), TT); \
+    else if (vec) SHIFT_GO((token_shift_mix_vec_kernel<TT, 1, false>), dim3(T, cols), TT);              \
     else SHIFT_GO(token_shift_mix_kernel<TT>, dim3(T), TT);                                      \
   } while (0)
   if (out_f32) SHIFT_ALL(float);
