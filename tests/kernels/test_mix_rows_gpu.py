@@ -50,7 +50,21 @@ def test_convolution_by_groups_of_lanes(dtype, taps, dim, heads, n_unit, togethe
     assert torch.equal(got_s.cpu(), want_s)
 
 
-@pytest.mark.parametrize("T,d", [(47, 4), (50, 2052), (1371, 2052), (4099, 64)])     # the last two: four rows a thread
+def test_convolution_at_the_ends_of_the_range():
+    """What a sigmoid makes of infinities, NaN and where its exponential ends."""
+    x = torch.tensor([float("inf"), -float("inf"), float("nan"), 3e38, -3e38, 86.9, -86.9, -87.1, -88.5, -104.0, 0.0, 1e-40,
+                      20.0, -20.0, 5.0, -1e-5]).repeat(4)[None].contiguous()
+    w, state, i = torch.zeros(64, 4), torch.zeros(2, 3, 64), torch.zeros(1, dtype=torch.int32)
+    w[:, 3] = 1.0
+    got, want = torch.empty(1, 64, device=DEV), torch.empty(1, 64)
+    ops.conv_act_heads(x.to(DEV), w.to(DEV), state.to(DEV), *(r.to(DEV) for r in (i, i, i, i)), 0, 16, 1e-6, got)
+    ref.conv_act_heads(x, w, state, i, i, i, i, 0, 16, 1e-6, want)
+    # below -87 zero for less than 87 e^-87 = 2e-36; four roundings of 2^-24, 20 of them in the reference's exponential
+    torch.testing.assert_close(got.cpu(), want, atol=2e-36, rtol=2e-6, equal_nan=True)
+
+
+# the last three: four rows a thread; the last: past the caches
+@pytest.mark.parametrize("T,d", [(47, 4), (50, 2052), (1371, 2052), (4099, 64), (3301, 4100)])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_token_shift_four_channels_a_lane(dtype, T, d):
     g = torch.Generator().manual_seed(d)
