@@ -75,8 +75,8 @@ struct KeepSplitArgs {
   int window, keep_first, sigmoid, H, G;
 };
 
-// Decode rows of groups of up to eight heads (mix_keep_row.hip), NA sequences of no more than NA rows together.
+// Decode rows of groups of up to eight heads (mix_keep_row.hip): T rows of NA sequences, no more than these.
 bool keep_row_ok(int T, int NA, int H, int G, int E, int vdim, bool shared);
-void launch_attn_keep_row(const KeepSplitArgs& a, int NA, int E, hipStream_t s);
+void launch_attn_keep_row(const KeepSplitArgs& a, int T, int NA, int E, hipStream_t s);
 
 }  // namespace rfqmix

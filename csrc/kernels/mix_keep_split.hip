@@ -430,7 +430,7 @@ void launch_attn_keep_split(const float* q, const void* k_cache, const void* v_c
   const KeepSplitArgs a{q, (const bf16_t*)k_cache, (const bf16_t*)v_cache, vrs, bt, maxb, q_start, q_len, kv_len,
                         head_bias, (const bf16_t*)gate, gate_stride, gate_w, (bf16_t*)out, out_stride,
                         scale, softcap, out_mult, window, keep_first, (int)sigmoid, H, G};
-  if (keep_row_ok(T, NA, H, G, E, vdim, shared)) return launch_attn_keep_row(a, NA, E, s);
+  if (keep_row_ok(T, NA, H, G, E, vdim, shared)) return launch_attn_keep_row(a, T, NA, E, s);
   const int DK = E / 32, DV = vdim / 16;
   const bool exact = H / G < 16;
   const int tiles = (int)(((int64_t)std::min(short_rows, T) * (H / G) + 15) / 16);   // at most, of a sequence
