@@ -52,7 +52,7 @@ void launch_embed(const int32_t*, const bf16_t*, bf16_t*, int, int, int, int, hi
 void launch_rope_kv(bf16_t*, int64_t, const int32_t*, const float*, const int32_t*, bf16_t*,
                     bf16_t*, int, int, int, int, hipStream_t);
 void launch_attn_decode(const bf16_t*, int64_t, const bf16_t*, const bf16_t*, const int32_t*, int,
-                        const int32_t*, const int32_t*, const int32_t*, const int32_t*,
+                        const int32_t*, const int32_t*, const int32_t*, int, const int32_t*,
                         const int32_t*, int, int, bf16_t*, int64_t, float*, float*, int, int,
                         float, int, int, int32_t*, hipStream_t, bool);
 void launch_attn_decode_shared(const bf16_t*, int64_t, const bf16_t*, const bf16_t*,
@@ -542,8 +542,9 @@ void attn_decode(const Tensor& q, const Tensor& k_cache, const Tensor& v_cache,
   rfq::launch_attn_decode(bp(q), q.stride(0), bp(k_cache), bp(v_cache),
                           block_tables.data_ptr<int32_t>(), block_tables.stride(0),
                           seq_q_start.data_ptr<int32_t>(), seq_q_len.data_ptr<int32_t>(),
-                          seq_kv_len.data_ptr<int32_t>(), work_seq.data_ptr<int32_t>(),
-                          work_ct.data_ptr<int32_t>(), work_seq.numel(), rows, bpm(out),
+                          seq_kv_len.data_ptr<int32_t>(), (int)seq_q_len.numel(),
+                          work_seq.data_ptr<int32_t>(), work_ct.data_ptr<int32_t>(),
+                          work_seq.numel(), rows, bpm(out),
                           out.stride(0), num_splits > 1 ? part_o.data_ptr<float>() : nullptr,
                           num_splits > 1 ? part_ml.data_ptr<float>() : nullptr, Hq, Hkv,
                           (float)scale, num_splits, tiles_per_item, tk, cur_stream(), reduce);

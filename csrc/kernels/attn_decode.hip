@@ -23,7 +23,8 @@
 //     of a 32-lane half touches 16 distinct 16-byte slots (conflict-free).
 //   * split-K partials (unnormalised O, running max, sum) are merged by
 //     attn_decode_reduce; with one split the kernel writes bf16 output directly.
-//   Steps of no more rows than work items (decode steps) run on attn_decode_rows.hip, with more waves to a split.
+//   Steps of no more rows than work items (decode steps, captured steps) run on attn_decode_rows.hip, with more waves to a
+//   split.
 //   The split size is derived per sequence from its context length on device, so a
 //   hipGraph captured with a fixed split count stays balanced as contexts grow.
 //
@@ -140,15 +141,15 @@ void launch_attn_decode_reduce(const float* part_o, const float* part_ml, bf16_t
 }
 
 void launch_attn_decode_rows(const bf16_t*, int64_t, const bf16_t*, const bf16_t*, const int32_t*, int, const int32_t*,
-                             const int32_t*, const int32_t*, const int32_t*, const int32_t*, int, int, bf16_t*, int64_t,
-                             float*, float*, int, int, float, int, int, int32_t*, hipStream_t);   // attn_decode_rows.hip
+                             const int32_t*, const int32_t*, int, const int32_t*, const int32_t*, int, int, bf16_t*,
+                             int64_t, float*, float*, int, int, float, int, int, int32_t*, hipStream_t);   // attn_decode_rows.hip
 
 // rows = number of q rows covered (for the split-K reduce), W = work items;
 // reduce = false leaves split partials for the consumer to merge (attn_decode_merge)
 void launch_attn_decode(const bf16_t* q, int64_t q_stride, const bf16_t* k_cache,
                         const bf16_t* v_cache, const int32_t* block_tables, int bt_stride,
                         const int32_t* seq_q_start, const int32_t* seq_q_len,
-                        const int32_t* seq_kv_len, const int32_t* work_seq,
+                        const int32_t* seq_kv_len, int nseq, const int32_t* work_seq,
                         const int32_t* work_ct, int W, int rows, bf16_t* out, int64_t out_stride,
                         float* part_o, float* part_ml, int Hq, int Hkv, float scale,
                         int num_splits, int tiles_per_item, int32_t* tickets, hipStream_t s,
@@ -162,11 +163,12 @@ void launch_attn_decode(const bf16_t* q, int64_t q_stride, const bf16_t* k_cache
     const char* v = getenv("RFQ_ATTN_NT");
     return v != nullptr && v[0] == '1';
   }();
-  // no more rows than work items: a decode step, one row a sequence (a longer one's further columns go one after another)
+  // no more rows than work items: decode steps, one row a sequence, and captured steps, whose lists have an item for every
+  // row.  An eager step with longer extends has fewer.
   const bool single = rows <= W;
   if (single)
     launch_attn_decode_rows(q, q_stride, k_cache, v_cache, block_tables, bt_stride, seq_q_start, seq_q_len, seq_kv_len,
-                            work_seq, work_ct, W, rows, out, out_stride, part_o, part_ml, Hq, Hkv, scale_log2, num_splits,
+                            nseq, work_seq, work_ct, W, rows, out, out_stride, part_o, part_ml, Hq, Hkv, scale_log2, num_splits,
                             tiles_per_item, tk, s);
 #define RFQ_AD_LAUNCH(T, N)                                                                     \
   attn_decode_kernel<T, 0, N><<<grid, 64, 0, s>>>(                                            \

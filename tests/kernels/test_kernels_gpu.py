@@ -1240,12 +1240,13 @@ def test_qkv_rope_in_two_products(M, head, Hq, K):
 @pytest.mark.parametrize("Hq,Hkv", [(32, 8), (8, 1), (64, 8), (3, 3), (16, 1)])
 @pytest.mark.parametrize("splits,single", [(1, False), (3, False), (2, True), (16, True)])
 @pytest.mark.parametrize("tiles", [1, 2])
-def test_attn_decode_rows(gpu, Hq, Hkv, splits, single, tiles):
+@pytest.mark.parametrize("qlens,kvlens", [([1, 1, 1, 1, 1, 0, 2, 1, 1], [1, 31, 32, 33, 700, 50, 70, 257, 2049]),
+                                          ([1, 12, 0, 30, 5, 32], [33, 700, 50, 31, 257, 64])])
+def test_attn_decode_rows(gpu, Hq, Hkv, splits, single, tiles, qlens, kvlens):
     """Steps of no more rows than work items (csrc/kernels/attn_decode_rows.hip): contexts around pages, splits and
-    waves, what was never written, a sequence of several rows and one without any."""
+    waves, what was never written, sequences of several rows and one without any, extends as in captured steps."""
     torch.manual_seed(6)
     G = Hq // Hkv
-    qlens, kvlens = [1, 1, 1, 1, 1, 0, 2, 1, 1], [1, 31, 32, 33, 700, 50, 70, 257, 2049]
     k, v = _paged_cache(512, Hkv, gpu, seed=5)
     bt = _block_tables(kvlens, 512, gpu)
     for i, n in enumerate(kvlens):
