@@ -328,21 +328,23 @@ __global__ __launch_bounds__(256) void conv_act_heads_vec_kernel(
   for (int cc = unit_here * dim + threadIdx.x; cc < nc; cc += blockDim.x) o[cc] = ys[cc];
 }
 
-// x / (1 + e^-x), the quotient's rest added once: rounded as a division, for divisors and quotients in the middle of the range.
-// An infinite divisor gives 0, and NaN for -inf.
+// x / (1 + e^-x) for x not below -87, the quotient's rest added once: rounded as a division.  Below, where the divisor's
+// reciprocal leaves the range of normal numbers, silu_low.
 __device__ __forceinline__ float silu_p(float x) {
-  const float d = x < -87.f ? __builtin_huge_valf() : 1.f + exp_c(-x), r = __builtin_amdgcn_rcpf(d), q = x * r;
+  const float d = 1.f + exp_c(-x), r = __builtin_amdgcn_rcpf(d), q = x * r;
   return __builtin_amdgcn_div_fixupf(fmaf(fmaf(-d, q, x), r, q), d, x);
 }
+__device__ __forceinline__ float silu_low(float y, float x) { return x < -87.f ? x / (1.0f + expf(-x)) : y; }
 
 // The same for heads of 16, 32, 64, 128 or 256 channels: a wave has 256 channels, four a lane, so a head
 // is a group of dim / 4 lanes and its sum needs no LDS; a thread takes R rows below one another, whose
 // earlier inputs and taps stay in registers.  (Positions rise by one inside a run, so what precedes a
 // row is what preceded the row above, shifted.)  Bound by memory and vector instructions, some 110 a row of 256
 // channels: 4,096 rows of 8,192 channels, 4 taps, from bf16 took 97 us with a row a block, its taps read again for
-// each and the heads' sums through LDS; 45.4 us with expf and a divide (25 instructions for the 16 of silu_p) and
-// with lengths in waves without unit heads, 41.3 now (4.9 TB/s; a layer's pass 264.5 -> 261).  Stored past the
-// caches 8,192 rows take a fifth less, which the kernel that reads them loses again.
+// each and the heads' sums through LDS; 45.4 us with expf and a divide (25 instructions for the 15 of silu_p) and
+// with lengths in waves without unit heads, 41.7 with a look at every sum for those below -87, 40.2 now with one at a
+// thread's four together (5.0 TB/s; a layer's pass, both sides in turn, 257.9 -> 256.2).  Stored past the caches 8,192 rows
+// take a fifth less, which the kernel that reads them loses again.
 template <typename T, int TAPS, int R>
 __global__ __launch_bounds__(256) void conv_act_heads_rows_kernel(
     const T* __restrict__ x, int64_t x_stride, const float* __restrict__ w,
@@ -386,6 +388,8 @@ __global__ __launch_bounds__(256) void conv_act_heads_rows_kernel(
       a3 += wc[3 * TAPS + K - dl] * h[dl - 1].w;
     }
     float4 y = make_float4(silu_p(a0), silu_p(a1), silu_p(a2), silu_p(a3));
+    if (__builtin_expect(__builtin_amdgcn_ballot_w64(fminf(fminf(a0, a1), fminf(a2, a3)) < -87.f) != 0ull, 0))
+      y = make_float4(silu_low(y.x, a0), silu_low(y.y, a1), silu_low(y.z, a2), silu_low(y.w, a3));
     if (units) {
       const float m = 1.0f / sqrtf(group_sum(y.x * y.x + y.y * y.y + y.z * y.z + y.w * y.w, dim >> 2) + unit_eps);
       if (unit) y = make_float4(y.x * m, y.y * m, y.z * m, y.w * m);

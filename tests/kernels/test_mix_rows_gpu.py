@@ -59,8 +59,23 @@ def test_convolution_at_the_ends_of_the_range():
     got, want = torch.empty(1, 64, device=DEV), torch.empty(1, 64)
     ops.conv_act_heads(x.to(DEV), w.to(DEV), state.to(DEV), *(r.to(DEV) for r in (i, i, i, i)), 0, 16, 1e-6, got)
     ref.conv_act_heads(x, w, state, i, i, i, i, 0, 16, 1e-6, want)
-    # below -87 zero for less than 87 e^-87 = 2e-36; four roundings of 2^-24, 20 of them in the reference's exponential
+    # below -88.7 zero for less than 88.7 e^-88.7 = 3e-37; four roundings of 2^-24, 20 of them in the reference's exponential
     torch.testing.assert_close(got.cpu(), want, atol=2e-36, rtol=2e-6, equal_nan=True)
+
+
+def test_convolution_of_far_negative_sums():
+    """Results are normal numbers down to -88.7, where the exponential ends, in all three kernels: heads of whole groups of
+    lanes, in fours, and any."""
+    for dim, C in ((16, 64), (20, 40), (3, 6)):
+        x = -torch.linspace(86.5, 88.7, C).clone()[None].contiguous()
+        x[0, 1] = 7.0                                        # beside one in the middle of the range
+        w, state, i = torch.zeros(C, 4), torch.zeros(2, 3, C), torch.zeros(1, dtype=torch.int32)
+        w[:, 3] = 1.0
+        got, want = torch.empty(1, C, device=DEV), x.double() / (1 + torch.exp(-x.double()))
+        ops.conv_act_heads(x.to(DEV), w.to(DEV), state.to(DEV), *(r.to(DEV) for r in (i, i, i, i)), 0, dim, 1e-6, got)
+        # an exponential begins with the product of -x and log2 e, between 64 and 128 and so rounded by up to 2^-18, of which
+        # ln 2 are the result's, 2.6e-6; the other four roundings, 2^-24 each, make less than the rest of 2^-18, 3.8e-6
+        assert float((got.cpu().double() / want - 1).abs().max()) <= 2.0 ** -18
 
 
 # the last three: four rows a thread; the last: past the caches
