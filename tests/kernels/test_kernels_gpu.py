@@ -1242,7 +1242,7 @@ def test_qkv_rope_in_two_products(M, head, Hq, K):
 @pytest.mark.parametrize("tiles", [1, 2])
 @pytest.mark.parametrize("qlens,kvlens", [([1, 1, 1, 1, 1, 0, 2, 1, 1], [1, 31, 32, 33, 700, 50, 70, 257, 2049]),
                                           ([1, 12, 0, 30, 5, 32], [33, 700, 50, 31, 257, 64])])
-def test_attn_decode_rows(gpu, Hq, Hkv, splits, single, tiles, qlens, kvlens):
+def test_attn_decode_rows(gpu, Hq, Hkv, splits, single, tiles, qlens, kvlens, wide=False):
     """Steps of no more rows than work items (csrc/kernels/attn_decode_rows.hip): contexts around pages, splits and
     waves, what was never written, sequences of several rows and one without any, extends as in captured steps."""
     torch.manual_seed(6)
@@ -1256,6 +1256,14 @@ def test_attn_decode_rows(gpu, Hq, Hkv, splits, single, tiles, qlens, kvlens):
     qs = [sum(qlens[:i]) for i in range(len(qlens))]
     work = [(i, ct) for i, n in enumerate(qlens) for ct in range(((n * G + 15) // 16 + tiles - 1) // tiles)]
     work += [(-1, 0)] * max(1, T - len(work))
+    if wide:                    # room for more than 96 MB, entries past a sequence's pages name one that nobody may read
+        spare = next(p for p in range(1, 512) if not bool((bt == p).any()))
+        k[spare] = v[spare] = float("nan")
+        cols = (96 << 20) // (len(work) * Hkv * 16384) + 1
+        bt = torch.cat([bt, bt.new_zeros(len(qlens), max(0, cols - bt.shape[1]))], 1)
+        for i, n in enumerate(kvlens):
+            bt[i, (n + 31) // 32:] = spare
+        assert len(work) * Hkv * bt.shape[1] * 16384 > 96 << 20
     i32 = lambda a: torch.tensor(a, dtype=torch.int32, device=gpu)  # noqa: E731
     q = torch.randn(T, Hq * 128, device=gpu, dtype=BF)
     po = torch.full((T * Hq * splits * 128,), float("nan"), device=gpu)
@@ -1270,3 +1278,14 @@ def test_attn_decode_rows(gpu, Hq, Hkv, splits, single, tiles, qlens, kvlens):
                         out, po, pm, Hq, Hkv, 128 ** -0.5, splits, tiles, tickets)
         assert not single or int(tickets.abs().sum()) == 0
         _close(out, exp, 2e-2, 0, f"attn_decode rows Hq={Hq} splits={splits} tiles={tiles} it={it}")
+
+
+# eight, four and two waves to a workgroup (ten to twelve work items), and one (up to four rows)
+@pytest.mark.parametrize("Hq,Hkv", [(32, 8), (64, 8)])
+@pytest.mark.parametrize("splits,single", [(1, False), (4, False), (16, True)])
+@pytest.mark.parametrize("tiles", [1, 2])
+@pytest.mark.parametrize("qlens,kvlens", [([1, 1, 1, 1, 1, 0, 2, 1, 1], [1, 31, 32, 33, 700, 50, 70, 257, 2049]),
+                                          ([1, 12, 0, 9, 5, 1], [33, 700, 50, 31, 257, 64]), ([1, 1, 2], [600, 33, 64])])
+def test_attn_decode_rows_past_the_caches(gpu, Hq, Hkv, splits, single, tiles, qlens, kvlens):
+    """The same with tables as wide as a captured step's, whose pages are read past the caches."""
+    test_attn_decode_rows(gpu, Hq, Hkv, splits, single, tiles, qlens, kvlens, wide=True)
