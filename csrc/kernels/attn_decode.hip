@@ -142,7 +142,7 @@ void launch_attn_decode_reduce(const float* part_o, const float* part_ml, bf16_t
 
 void launch_attn_decode_rows(const bf16_t*, int64_t, const bf16_t*, const bf16_t*, const int32_t*, int, const int32_t*,
                              const int32_t*, const int32_t*, int, const int32_t*, const int32_t*, int, int, bf16_t*,
-                             int64_t, float*, float*, int, int, float, int, int, int32_t*, hipStream_t);   // attn_decode_rows.hip
+                             int64_t, float*, float*, int, int, float, int, int, int32_t*, bool, hipStream_t);   // attn_decode_rows.hip
 
 // rows = number of q rows covered (for the split-K reduce), W = work items;
 // reduce = false leaves split partials for the consumer to merge (attn_decode_merge)
@@ -158,7 +158,8 @@ void launch_attn_decode(const bf16_t* q, int64_t q_stride, const bf16_t* k_cache
   const float scale_log2 = scale * 1.4426950408889634f;
   dim3 grid(num_splits, Hkv, W);
   int32_t* tk = num_splits > 1 ? tickets : nullptr;
-  // RFQ_ATTN_NT=1: non-temporal loads for the per-sequence KV pages (NTK above)
+  // RFQ_ATTN_NT=1: pages past the caches in every step (without it where attn_decode_rows.hip finds many), here from a
+  // sequence's page kNtFromPage on
   static const bool ntk = [] {
     const char* v = getenv("RFQ_ATTN_NT");
     return v != nullptr && v[0] == '1';
@@ -169,7 +170,7 @@ void launch_attn_decode(const bf16_t* q, int64_t q_stride, const bf16_t* k_cache
   if (single)
     launch_attn_decode_rows(q, q_stride, k_cache, v_cache, block_tables, bt_stride, seq_q_start, seq_q_len, seq_kv_len,
                             nseq, work_seq, work_ct, W, rows, out, out_stride, part_o, part_ml, Hq, Hkv, scale_log2, num_splits,
-                            tiles_per_item, tk, s);
+                            tiles_per_item, tk, ntk, s);
 #define RFQ_AD_LAUNCH(T, N)                                                                     \
   attn_decode_kernel<T, 0, N><<<grid, 64, 0, s>>>(                                            \
       q, q_stride, k_cache, v_cache, block_tables, bt_stride, seq_q_start, seq_q_len,            \

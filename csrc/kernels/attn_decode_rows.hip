@@ -337,17 +337,19 @@ void launch_attn_decode_rows(const bf16_t* q, int64_t q_stride, const bf16_t* k_
                              const int32_t* block_tables, int bt_stride, const int32_t* seq_q_start, const int32_t* seq_q_len,
                              const int32_t* seq_kv_len, int seqs, const int32_t* work_seq, const int32_t* work_ct, int W, int rows,
                              bf16_t* out, int64_t out_stride, float* part_o, float* part_ml, int Hq, int Hkv, float scale_log2,
-                             int num_splits, int tiles_per_item, int32_t* tickets, hipStream_t s) {
+                             int num_splits, int tiles_per_item, int32_t* tickets, bool past, hipStream_t s) {
   const DecodeRows a{q, k_cache, v_cache, q_stride, out_stride, block_tables, seq_q_start, seq_q_len, seq_kv_len, work_seq,
                      work_ct, tickets, out, part_o, part_ml, bt_stride, Hq, Hkv, num_splits, scale_log2};
   // As many waves to a workgroup as its LDS leaves room for with all workgroups on the chip at once: 8.5 KB of a CU's 160
   // for a wave's keys, as much for its values.  Work items of a captured step's list that none of its sequences can need
-  // are padding and leave at once.  Past the caches where the tables have room for more than 96 MB, as in
-  // mix_keep_row.hip, also where sequences share their first pages.
+  // are padding and leave at once.  Past the caches where the caller asks for it (`past`), and where the tables have room
+  // for more than 96 MB, as in mix_keep_row.hip.  A captured step's have, whatever its sequences hold.  32 heads over 8, 600
+  // tokens each, pages that no cache holds, through the caches and past them: 4 sequences 10.7 / 11.0 us, 8 12.8 / 12.4, 16
+  // 16.1 / 14.8, 64 31.6 / 31.8; with the first 13 pages in common 10.0 / 10.3, 10.6 / 11.3, 12.0 / 12.4, 20.0 / 20.1.
   const int64_t wgs = (int64_t)W * Hkv * num_splits;
   const int64_t items = std::min<int64_t>(W, seqs + (int64_t)rows * (Hq / Hkv) / (16 * tiles_per_item));
   const int64_t live = items * Hkv * num_splits;
-  const bool stream = (int64_t)W * Hkv * bt_stride * (kPage * kD * 4) > (96 << 20);
+  const bool stream = past || (int64_t)W * Hkv * bt_stride * (kPage * kD * 4) > (96 << 20);
   if (rows <= 4) return launch_rows_waves<1>(a, wgs, tiles_per_item, stream, s);   // steps that the persistent layer takes in a captured graph
   if (live <= 256) return launch_rows_waves<8>(a, wgs, tiles_per_item, stream, s);
   if (live <= 512) return launch_rows_waves<4>(a, wgs, tiles_per_item, stream, s);

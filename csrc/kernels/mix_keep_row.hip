@@ -371,7 +371,10 @@ static void launch_row_one(const KeepSplitArgs& a, int T, int NA, hipStream_t s)
 // Eight waves to a workgroup where rows and heads alone leave CUs idle: a wave's chain of pages is the time then.
 // Pages past the caches where what the tables have room for is more than 96 MB: the last-level cache, 256 MB, then holds
 // nothing of them by the time they are read again.  32 heads over 8 of 128, 300 - 900 tokens, through the caches and past
-// them: 8 sequences (of up to 1,900) 29.2 / 32.0 us, 24 24.7 / 25.7, 32 29.3 / 28.3, 48 42.2 / 37.2, 64 50.0 / 42.1.
+// them: 8 sequences (of up to 1,900) 29.2 / 32.0 us, 24 24.7 / 25.7, 32 29.3 / 28.3, 48 42.2 / 37.2, 64 50.0 / 42.1.  A
+// captured step's tables are as wide as the longest context, whatever its sequences hold.  600 tokens each, pages that no
+// cache holds: 4 sequences 11.9 / 13.3 us, 8 14.1 / 13.7, 16 15.2 / 14.3, 64 29.9 / 30.0; with the first 13 pages in common
+// 11.7 / 13.0, 12.1 / 13.1, 13.5 / 13.3, 20.6 / 20.0.
 template <int DK, int DV, int HC>
 static void launch_row_waves(const KeepSplitArgs& a, int T, int NA, hipStream_t s) {
   const int64_t wgs = (int64_t)T * a.G;
