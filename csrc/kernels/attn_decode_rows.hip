@@ -345,7 +345,8 @@ void launch_attn_decode_rows(const bf16_t* q, int64_t q_stride, const bf16_t* k_
   // are padding and leave at once.  Past the caches where the caller asks for it (`past`), and where the tables have room
   // for more than 96 MB, as in mix_keep_row.hip.  A captured step's have, whatever its sequences hold.  32 heads over 8, 600
   // tokens each, pages that no cache holds, through the caches and past them: 4 sequences 10.7 / 11.0 us, 8 12.8 / 12.4, 16
-  // 16.1 / 14.8, 64 31.6 / 31.8; with the first 13 pages in common 10.0 / 10.3, 10.6 / 11.3, 12.0 / 12.4, 20.0 / 20.1.
+  // 16.1 / 14.8, 64 31.6 / 31.8; with the first 13 pages in common 10.0 / 10.3, 10.6 / 11.3, 12.0 / 12.4, 20.0 / 20.1.  Few
+  // long ones gain: 4 of 2,000 tokens 14.7 / 13.9, 8 of 4,000 31.8 / 29.7, one of 32,000 70.4 / 58.2.
   const int64_t wgs = (int64_t)W * Hkv * num_splits;
   const int64_t items = std::min<int64_t>(W, seqs + (int64_t)rows * (Hq / Hkv) / (16 * tiles_per_item));
   const int64_t live = items * Hkv * num_splits;

@@ -1113,9 +1113,11 @@ bool launch_qk_norm_rotary_append(bool f32, const void* proj, int64_t stride, co
   // convolved 1 row 8.1, 7.2, now 6.6 us, 64 rows 9.3, 8.4, 7.8, 2,648 40.5, 30.6, 25.0 (3.4 TB/s), 8,192 103, 87, 66; with a
   // bias 2,648 rows 28.7, 23.1, 21.5.  Latents (64 rotated entries of 32 heads, 576 of the key): 2,067 rows 15.2, 10.3, 10.0,
   // 8,192 44.3, 29.5, 28.2.  Where it does not pay, measured from 256 to 10,240 columns and 1 to 8,192 rows:
-  //   convolved, two chunks a thread: in fp32 never (64 + 8 + 8 heads, 2,067 rows 99 us for 73), in bf16 up to a row a CU
-  //   (10,240 columns: 64 rows 14.0 us for 12.5, 256 13.3 for 10.9, 300 15.2 for 16.9, 700 21.1 for 22.3) and up to 9,216
-  //   columns from three rows a CU (9,216: 513 rows 19.2 for 18.3, 700 20.3 for 20.5, 1,031 26.6 for 32.9, 512 16.8 for 18.0)
+  //   convolved, two chunks a thread: in fp32 never (64 + 8 + 8 heads, 2,067 rows 99 us for 73), in bf16 for few rows, whose
+  //   runs may be short: a run's first rows wait for the state three times, one after another (10,240 columns: 600 runs of one
+  //   row 45 us for 38, one of 520 20.2 for 20.8, of 700 21.4 for 21.8; 9,216: 1,031 runs of one row 86 for 73, 300 of four 42
+  //   for 39, one of 1,031 27 for 33, 2,048 of one row 145 for 143, one of 2,067 41 for 50, of 8,000 156 for 193).  A run's
+  //   state on its way at once spills 50 registers: 1.3 to 1.6 times the time throughout
   //   convolved in fp32, a single row of 6,144 columns and more: up to 1.09 times the other kernel's time
   //   no norm, little to sum up: 64 rows of 3,072 columns 4.7 us for 4.4
   //   fp32 without a convolution, four to eight waves of 134 registers, one such workgroup a CU: 824 rows of 6,144 columns 16.2
@@ -1125,7 +1127,7 @@ bool launch_qk_norm_rotary_append(bool f32, const void* proj, int64_t stride, co
   const int wide = (int)((W / 8 + per - 1) / per + 63) / 64 * 64;
   const bool one = norm_all || (q_norm_w == nullptr && (k_norm_w == nullptr || G == 1));     // norm of a kind's columns
   auto pays = [&]() {
-    if (conv) return per == 1 ? !f32 || T >= 8 || W < 6144 : !f32 && T > 256 && (W > 9216 || T <= 512 || T >= 700);
+    if (conv) return per == 1 ? !f32 || T >= 8 || W < 6144 : !f32 && T >= (W > 9216 ? 1024 : 2048);
     if (q_norm_w == nullptr && k_norm_w == nullptr &&
         !(f32 ? T >= 2048 : T >= 1024 || (int64_t)T * (int64_t)W >= 1 << 20 || W >= 7168)) return false;
     return !f32 || T <= 256 || wide <= 192 || W > 9216 || (wide >= 576 && T >= 2048);

@@ -374,7 +374,8 @@ static void launch_row_one(const KeepSplitArgs& a, int T, int NA, hipStream_t s)
 // them: 8 sequences (of up to 1,900) 29.2 / 32.0 us, 24 24.7 / 25.7, 32 29.3 / 28.3, 48 42.2 / 37.2, 64 50.0 / 42.1.  A
 // captured step's tables are as wide as the longest context, whatever its sequences hold.  600 tokens each, pages that no
 // cache holds: 4 sequences 11.9 / 13.3 us, 8 14.1 / 13.7, 16 15.2 / 14.3, 64 29.9 / 30.0; with the first 13 pages in common
-// 11.7 / 13.0, 12.1 / 13.1, 13.5 / 13.3, 20.6 / 20.0.
+// 11.7 / 13.0, 12.1 / 13.1, 13.5 / 13.3, 20.6 / 20.0.  Few long ones gain: 4 of 2,000 tokens 28.1 / 27.5, 15 of 2,000 32.5 /
+// 30.5, one of 32,000 290 / 282.
 template <int DK, int DV, int HC>
 static void launch_row_waves(const KeepSplitArgs& a, int T, int NA, hipStream_t s) {
   const int64_t wgs = (int64_t)T * a.G;

@@ -341,7 +341,7 @@ __device__ __forceinline__ float silu_low(float y, float x) { return x < -87.f ?
 // earlier inputs and taps stay in registers.  (Positions rise by one inside a run, so what precedes a
 // row is what preceded the row above, shifted.)  Bound by memory and vector instructions, some 110 a row of 256
 // channels: 4,096 rows of 8,192 channels, 4 taps, from bf16 took 97 us with a row a block, its taps read again for
-// each and the heads' sums through LDS; 45.4 us with expf and a divide (25 instructions for the 15 of silu_p) and
+// each and the heads' sums through LDS; 45.4 us with expf and a divide (25 instructions for the 14 of silu_p) and
 // with lengths in waves without unit heads, 41.7 with a look at every sum for those below -87, 40.2 now with one at a
 // thread's four together (5.0 TB/s; a layer's pass, both sides in turn, 257.9 -> 256.2).  Stored past the caches 8,192 rows
 // take a fifth less, which the kernel that reads them loses again.

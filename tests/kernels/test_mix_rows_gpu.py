@@ -158,7 +158,7 @@ def test_norm_and_rotation_of_rows_one_after_another(dtype, conv, H, G, dim, nro
 
 
 # Runs of one to seven rows everywhere: workgroups that begin at any row of a run, with and without a state
-@pytest.mark.parametrize("T,H,G,dim", [(2101, 20, 3, 64), (1030, 40, 8, 128), (300, 64, 8, 128), (1030, 56, 8, 128)])
+@pytest.mark.parametrize("T,H,G,dim", [(2101, 20, 3, 64), (1030, 40, 8, 128), (300, 64, 8, 128), (1030, 56, 8, 128), (1030, 64, 8, 128), (2060, 56, 8, 128)])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_convolved_rows_of_short_runs(monkeypatch, dtype, T, H, G, dim):
     lens = [1 + i % 7 for i in range(T // 4)]
