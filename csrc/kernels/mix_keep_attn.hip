@@ -24,6 +24,7 @@
 // workgroup per (sequence, key/value head) over one pass through the pages for decode rows.
 // MFMA tiles for bf16 pages are in mix_keep_attn_mfma.hip.
 #include <algorithm>
+#include <type_traits>
 
 #include "mix_common.h"
 
@@ -500,10 +501,10 @@ __global__ __launch_bounds__(N == 1 ? 1024 : kQknThreads) void qk_norm_rotary_ap
     cs[2 * x] = c * a.rot_mult;
     cs[2 * x + 1] = sn * a.rot_mult;
   }
-  // What the rows above row r of its run add to it and the two below.  `back` of them are in the projection (registers:
-  // r = 0), older ones in the state that the run began with.
+  // What the rows above row r of its run add to it and the two below.  `back` of them are in the projection (registers, for
+  // the workgroup's first row: a later one is its run's first), older ones in the state that the run began with.
   float acc[SUMS ? K : 1][8];
-  auto begin = [&](int r, const int4& m) {
+  auto begin = [&](int r, const int4& m, auto first) {
     const int pt = __builtin_amdgcn_readfirstlane(pos[r]);
     const int half = (m.w & 1) * a.state_slots + (m.w >> 1);
 #pragma unroll
@@ -512,7 +513,7 @@ __global__ __launch_bounds__(N == 1 ? 1024 : kQknThreads) void qk_norm_rotary_ap
       for (int i = 0; i < 8; ++i) acc[e][i] = 0.f;
 #pragma unroll
     for (int d = K - 1; d >= 0; --d) {
-      const bool own = d < m.y;
+      const bool own = first && d < m.y;
       if (!own && (pt - d - 1 < 0 || m.w < 0)) continue;
       float u[8];
       if (own) above[d][0].template get<T>(u);
@@ -528,7 +529,7 @@ __global__ __launch_bounds__(N == 1 ? 1024 : kQknThreads) void qk_norm_rotary_ap
     return make_int4(__builtin_amdgcn_readfirstlane(m.x), __builtin_amdgcn_readfirstlane(m.y),
                      __builtin_amdgcn_readfirstlane(m.z), __builtin_amdgcn_readfirstlane(m.w));
   };
-  if constexpr (SUMS) begin(0, numbers(0));
+  if constexpr (SUMS) begin(0, numbers(0), std::true_type{});
   for (int r = 0; r < n; ++r) {
     const int4 m = numbers(r);
     const int slot = m.x, back = m.y, fwd = m.z, code = m.w;
@@ -552,7 +553,7 @@ __global__ __launch_bounds__(N == 1 ? 1024 : kQknThreads) void qk_norm_rotary_ap
           }
       }
       if constexpr (SUMS) {
-        if (back == 0 && r > 0) begin(r, m);
+        if (back == 0 && r > 0) begin(r, m, std::false_type{});
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
           const float x = f[0][i];
@@ -655,7 +656,7 @@ __global__ __launch_bounds__(N == 1 ? 1024 : kQknThreads) void qk_norm_rotary_ap
           }
         }
       } else {
-        constexpr int SH = CONV && N == 2 ? 2 : 8;        // at a time: registers
+        constexpr int SH = !CONV || (N == 1 && sizeof(T) == 2) ? 8 : N == 1 ? 4 : 2;      // at a time: registers
 #pragma unroll
         for (int i0 = 0; i0 < 8; i0 += SH) {
           float u[SH];
@@ -1109,7 +1110,8 @@ bool launch_qk_norm_rotary_append(bool f32, const void* proj, int64_t stride, co
                      (turn <= 512 && (nrot & (nrot - 1)) == 0 && q_rot_off % turn == 0 && k_rot_off % turn == 0 &&
                       qw % turn == 0 && kw % turn == 0);
   // Two chunks a thread, one where a thread keeps the convolution's weights for it (two spill 20 registers in bf16, 70 in
-  // fp32).  32 + 8 + 8 heads of 128 in bf16, against a workgroup a row and against these rows before the sums were kept:
+  // fp32; one in fp32 has none to spare, and four of them spilled cost 1,100 rows of 1,536 columns 9.1 us for 8.2, 4,100 of
+  // 8,192 65 for 56).  32 + 8 + 8 heads of 128 in bf16, against a workgroup a row and against these rows before the sums were kept:
   // convolved 1 row 8.1, 7.2, now 6.6 us, 64 rows 9.3, 8.4, 7.8, 2,648 40.5, 30.6, 25.0 (3.4 TB/s), 8,192 103, 87, 66; with a
   // bias 2,648 rows 28.7, 23.1, 21.5.  Latents (64 rotated entries of 32 heads, 576 of the key): 2,067 rows 15.2, 10.3, 10.0,
   // 8,192 44.3, 29.5, 28.2.  Where it does not pay, measured from 256 to 10,240 columns and 1 to 8,192 rows:
