@@ -362,12 +362,14 @@ void launch_rank_product_f32(const float* x, int64_t xs, const float* w, int64_t
 }
 
 // Up to 2^20 results a launch is what counts.  Above, the kernel for many rows is slower than the library's in two places,
-// measured from 1 to 128 matrices, 64 to 4,096 columns, 64 to 8,192 rows: 128 terms with fewer rows than repay W's way into
-// registers (32 x 512 columns, 300 rows 10.2 us for 9.4, 64 x 512, 100 rows 8.5 for 8.2), and results of 2 GB (630 for 593).
+// measured from 1 to 128 matrices, 64 to 4,096 columns, 64 to 8,192 rows: 128 terms with fewer rows or results than repay W's
+// way into registers (32 x 512 columns, 300 rows 10.2 us for 9.4, 500 14.6 for 13.7, 700 17.2 for 17.1, 800 18.1 for 20.3;
+// 16 x 512, 900 rows 12.7 for 11.0, 1,031 13.3 for 15.0; 8 x 512, 1,500 rows 10.4 for 9.8, 2,067 13.0 for 14.8; 64 x 512, 100
+// rows 8.5 for 8.2, 500 19.9 for 20.3), and results of 2 GB (630 for 593).
 static bool few_results(int64_t B, int64_t M, int64_t N) { return M <= (1 << 20) / N && B <= (1 << 20) / (M * N); }
 bool batch_product_ok(int64_t B, int64_t M, int64_t N, int64_t K) {
   if (!(B >= 1 && B <= 65535 && M >= 1 && N >= 64 && N % 64 == 0 && N <= 1 << 20 && K >= 32 && K <= 128 && K % 32 == 0)) return false;
-  return few_results(B, M, N) || (M <= (1 << 28) / N && B <= (1 << 28) / (M * N) && (K <= 96 || M >= 500));
+  return few_results(B, M, N) || (M <= (1 << 28) / N && B <= (1 << 28) / (M * N) && (K <= 96 || (M >= 500 && B * M * N > 1 << 23)));
 }
 
 void launch_batch_product(const void* x, int64_t xb, int64_t xs, const void* w, int64_t wb, int64_t ws, float* y, int64_t yb,

@@ -1245,7 +1245,7 @@ def _short_batch(a, b, out) -> bool:
     (x0, x1, x2), (w0, w1, w2), (y0, y1, y2) = a.stride(), b.stride(), out.stride()
     lo, hi, n = (y1, y0, M) if y1 <= y0 else (y0, y1, B)
     return (1 <= B <= 65535 and M >= 1 and K in (32, 64, 96, 128) and N % 64 == 0 and N >= 64
-            and B * M * N <= 1 << (28 if K <= 96 or M >= 500 else 20) and N <= 1 << 20
+            and B * M * N <= 1 << (28 if K <= 96 or M >= 500 and B * M * N > 1 << 23 else 20) and N <= 1 << 20
             and b.shape == (B, K, N) and out.shape == (B, M, N) and x2 == w2 == y2 == 1 and lo >= N and hi >= n * lo
             and not (x0 | x1 | w0 | w1 | a.storage_offset() | b.storage_offset()) & 7 and not (y0 | y1 | out.storage_offset()) & 3
             and a.device == b.device == out.device)

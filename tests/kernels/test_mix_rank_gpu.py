@@ -137,10 +137,11 @@ def test_batches_of_short_products(B, M, N, K, rows_first):
 
 
 # more than 2^20 results: workgroups of one, three and eight waves, several columns' workgroups, rows that blocks do not divide,
-# more blocks than workgroups and fewer, results past the caches; 128 terms and fewer than 500 rows stay with the library
+# more blocks than workgroups and fewer, results past the caches; 128 terms and fewer than 500 rows, or up to 2^23 results, stay
+# with the library
 @pytest.mark.parametrize("B,M,N,K", [(70, 501, 64, 128), (9, 500, 576, 96), (9, 499, 576, 128), (2, 2100, 512, 128), (1, 600, 4096, 32),
                                      (300, 65, 128, 64), (32, 130, 512, 32), (5, 4097, 128, 64),
-                                     (3, 21899, 512, 32)])
+                                     (3, 21899, 512, 32), (33, 501, 576, 128), (70, 1999, 64, 128), (3, 2100, 1536, 128)])
 @pytest.mark.parametrize("rows_first", [False, True])
 def test_batches_of_many_rows(B, M, N, K, rows_first):
     test_batches_of_short_products(B, M, N, K, rows_first)

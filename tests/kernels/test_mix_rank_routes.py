@@ -1,11 +1,12 @@
 """Which products of ops.matmul_nt go to the kernel for short ones, and which stay with the library."""
+import ctypes
 import types
 import warnings
 
 import pytest
 import torch
 
-from replisense_rfq_amd import ops
+from replisense_rfq_amd import _build, ops
 
 DEV = "cuda"
 
@@ -97,3 +98,22 @@ def test_a_batch_of_products_is_one(out_dtype):
                        (torch.vmap(lambda a: ops.matmul_nt(a, w[0], out_dtype))(x), x.float() @ w[0].float().t())):
             assert y.dtype == (out_dtype or torch.bfloat16)
             torch.testing.assert_close(y.float(), ref, atol=1e-3, rtol=2.0 ** -8)
+
+
+# B, M, N, K; around 2^20 results, 500 rows and 2^23 results of 128 terms, 2^28 results
+@pytest.mark.parametrize("B,M,N,K,short", [(32, 64, 512, 128, True), (32, 65, 512, 128, False), (32, 65, 512, 96, True),
+                                           (32, 499, 576, 128, False), (32, 500, 576, 128, True), (32, 512, 512, 128, False),
+                                           (32, 513, 512, 128, True), (8, 1500, 512, 128, False), (8, 2067, 512, 128, True),
+                                           (16, 900, 512, 64, True), (64, 8192, 512, 128, True), (64, 8193, 512, 128, False),
+                                           (64, 8193, 512, 32, False), (1, 1, 64, 32, True), (1, 1, 72, 32, False)])
+def test_batches_of_the_kernel(B, M, N, K, short):
+    """Where it is as fast as the library's; the operator refuses what the rule leaves out."""
+    a, b = torch.empty(B, M, K, device="meta"), torch.empty(B, K, N, device="meta")
+    a, b, out = a.bfloat16(), b.bfloat16(), torch.empty(B, M, N, device="meta")
+    assert ops._short_batch(a, b, out) == short
+    if not _build.MIX_SO.exists():
+        _build.build_mix_kernels()
+    torch.ops.load_library(str(_build.MIX_SO))
+    rule = ctypes.CDLL(str(_build.MIX_SO))["_ZN6rfqmix16batch_product_okEllll"]
+    rule.restype, rule.argtypes = ctypes.c_bool, [ctypes.c_int64] * 4
+    assert rule(B, M, N, K) == short
