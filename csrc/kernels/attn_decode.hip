@@ -165,8 +165,10 @@ void launch_attn_decode(const bf16_t* q, int64_t q_stride, const bf16_t* k_cache
     return v != nullptr && v[0] == '1';
   }();
   // no more rows than work items: decode steps, one row a sequence, and captured steps, whose lists have an item for every
-  // row.  An eager step with longer extends has fewer.
-  const bool single = rows <= W;
+  // row.  An eager step with longer extends has fewer.  Tables of one page leave nothing to share: 64 sequences of 20 tokens,
+  // 32 heads over 8, 5.5 us here and 6.1 there, 256 of 30 10.7 and 13.7; of two pages 8.6 and 7.6, 17.7 and 18.8.  Up to four
+  // rows are one wave there too.
+  const bool single = rows <= W && (bt_stride > 1 || rows <= 4);
   if (single)
     launch_attn_decode_rows(q, q_stride, k_cache, v_cache, block_tables, bt_stride, seq_q_start, seq_q_len, seq_kv_len,
                             nseq, work_seq, work_ct, W, rows, out, out_stride, part_o, part_ml, Hq, Hkv, scale_log2, num_splits,

@@ -96,7 +96,7 @@ fn = lib[name]
 fn.restype = None
 fn.argtypes = [p, l, p, p, p, i, p, p, p, i, p, p, i, i, p, l, p, p, i, i, f, i, i, p, p, b]
 for seqs, items, rows, cols, splits in ((1, 1, 1, 40, 2), (8, 8, 8, 40, 2), (32, 32, 32, 20, 2), (64, 64, 64, 11, 2), (64, 64, 64, 300, 2),
-                                        (2, 16, 16, 16, 8), (64, 80, 100, 20, 2)):
+                                        (2, 16, 16, 16, 8), (64, 80, 100, 20, 2), (8, 8, 8, 1, 1)):
     for tiles in (1, 2):
         fn(None, 4096, None, None, None, cols, None, None, None, seqs, None, None, items, rows, None, 4096, None, None, 32, 8, 0.1, splits,
            tiles, None, None, False)
@@ -108,7 +108,7 @@ print("bad", front.bad())
 @pytest.mark.skipif(shutil.which("g++") is None or shutil.which("nm") is None, reason="needs g++ and nm")
 def test_which_kernel_a_decode_step_goes_to(tmp_path):
     """attn_decode by its launches: waves by the items that the sequences can need, pages past the caches by the tables' room
-    or RFQ_ATTN_NT=1, more rows than items to the general kernel, and all of them allowed their LDS."""
+    or RFQ_ATTN_NT=1, more rows than items and tables of one page to the general kernel, and all of them allowed their LDS."""
     if not _build.C_SO.exists():
         _build.build_kernels()
     front = _front(tmp_path)
@@ -119,4 +119,4 @@ def test_which_kernel_a_decode_step_goes_to(tmp_path):
         out = _run(DECODE, front, _build.C_SO, RFQ_ATTN_NT=nt).split()
         for tiles in (1, 2):
             assert out[tiles - 1:12:2] == [rows % (w, tiles, past or nt == "1") for w, past in want[tiles - 1]], out
-        assert all(x.startswith("18attn_decode_kernel") for x in out[12:14]) and out[14:] == ["bad", "0"], out
+        assert all(x.startswith("18attn_decode_kernel") for x in out[12:16]) and out[16:] == ["bad", "0"], out
