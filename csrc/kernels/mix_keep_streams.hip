@@ -29,6 +29,7 @@ constexpr int kLatE = 576, kLatV = 512;
 constexpr int kLatPage = WBS * kLatE * 2;        // bytes
 constexpr int stream_pages(int tiles) { return tiles == 1 ? 4 : 3; }        // in LDS
 constexpr int kSharePages = 2;                   // pages of a workgroup, at least
+constexpr int kWholePages = 8;                   // rows of so many and fewer are a workgroup's, of two tiles of heads
 
 // What a row of the step sees: pages [0, n_keep) of its sequence s (-1: none, a row of a captured step beyond those of
 // its sequences) hold the kept first tokens, `skip` pages follow that are not read, then those of the window up to the
@@ -92,7 +93,9 @@ __device__ __forceinline__ void store_gated(const KeepArgs& a, float (&y)[4], in
       make_uint2(rfq::pack_bf16x2(y[0], y[1]), rfq::pack_bf16x2(y[2], y[3]));
 }
 // How many of S workgroups have a part in the row: no more than have two pages, the first in any case
+template <int HT>
 __device__ __forceinline__ int row_shares(const RowPages& r, int S) {
+  if (HT == 2 && r.pages <= kWholePages) return 1;
   return min(S, max(1, (r.pages + kSharePages - 1) / kSharePages));
 }
 
@@ -131,7 +134,7 @@ __global__ __launch_bounds__(512, 2) void attn_keep_streams_kernel(const KeepArg
   }
   const RowPages row = row_pages(a, NA, (int)t);
   if (row.s < 0) return;
-  const int shares = row_shares(row, S);
+  const int shares = row_shares<HT>(row, S);
   if (z >= shares) return;                                    // no page for this workgroup
   const int from = z * row.pages / shares, n = (z + 1) * row.pages / shares - from;
   typedef const __attribute__((address_space(4))) int32_t const_i32;
@@ -375,7 +378,7 @@ __global__ __launch_bounds__(512, 2) void attn_keep_streams_kernel(const KeepArg
 }
 
 // One wave per row and head: the workgroups' parts, the sink, the gate.
-template <int MODE>
+template <int HT, int MODE>
 __global__ __launch_bounds__(64) void attn_keep_streams_merge_kernel(const KeepArgs a, const float* part, int T, int S,
                                                                       int NA) {
   constexpr int vdim = kLatV, NC = vdim / 256, AHEAD = 4;     // pieces of four channels a lane; shares on their way at once
@@ -383,7 +386,7 @@ __global__ __launch_bounds__(64) void attn_keep_streams_merge_kernel(const KeepA
   const int hx = blockIdx.y, lane = threadIdx.x;
   const RowPages row = row_pages(a, NA, (int)t);
   if (row.s < 0) return;
-  const int shares = row_shares(row, S);
+  const int shares = row_shares<HT>(row, S);
   if (shares == 1) return;                                    // its workgroup has stored the row itself
   const float2* ml = reinterpret_cast<const float2*>(part + (int64_t)T * S * a.H * vdim);
   const int64_t at = t * S * a.H + hx;
@@ -430,7 +433,9 @@ __global__ __launch_bounds__(64) void attn_keep_streams_merge_kernel(const KeepA
 // 64 heads together, half as many reads of a page for three pages in LDS instead of four and 5 us more on the way to the
 // first: where 32 leave no two workgroups a row (100 sequences of 900 tokens with 64 heads 82 us by the prompts' kernel, 53;
 // 128 of 600 58, 45), or just two and the rows are long (64 of 2,000 60 us with 32 heads, 55.5 with 64; of 600 30 and 34; a
-// captured step's table says nothing about that).
+// captured step's table says nothing about that).  Short rows of captured steps cost more so than by the prompts' kernel: 128
+// sequences with 64 heads of 20 tokens 17.9 for 12.5, of 100 24.7 for 20.8, of 200 31 for 29, of 300 38 for 37.  Rows of up to
+// eight pages shared by two workgroups, whose parts then meet, took 29 and 35 of 100 and 200.
 // Of up to NA rows a sequence may have several: each has workgroups of its own, as in a captured step rows of an extend
 // stand where other sequences are padding (one sequence of 600 tokens with 16 rows, 16 of one and 15 without: 143 us
 // split over waves, 269 with an extend's rows one after another, 23 side by side).
@@ -471,12 +476,12 @@ static void launch_streams_tiles(const KeepArgs& a, int T, int NA, int S, float*
   }
   hipLaunchKernelGGL((attn_keep_streams_kernel<HT, MODE>), dim3(T, a.G * ((a.H / a.G + 32 * HT - 1) / (32 * HT)), S), dim3(512), lds, a.s, a,
                      part, T, NA);
+  hipLaunchKernelGGL((attn_keep_streams_merge_kernel<HT, MODE>), dim3(T, a.H), dim3(64), 0, a.s, a, part, T, S, NA);
 }
 template <int MODE>
 static void launch_streams_one(const KeepArgs& a, int T, int NA, int S, float* part) {
   if (streams_of(T, NA, a.H, a.G, a.maxb, a.window, a.keep_first).tiles == 2) launch_streams_tiles<2, MODE>(a, T, NA, S, part);
   else launch_streams_tiles<1, MODE>(a, T, NA, S, part);
-  hipLaunchKernelGGL(attn_keep_streams_merge_kernel<MODE>, dim3(T, a.H), dim3(64), 0, a.s, a, part, T, S, NA);
 }
 
 void launch_attn_keep_streams(const float* q, const void* k_cache, int64_t vrs, const int32_t* bt, int maxb,

@@ -197,6 +197,15 @@ def test_wide_rows_of_64_heads_together(H, G, n):
     _check(H, G, 576, 512, True, seqs=seqs[1:] + [(800, 1)], window=700, keep_first=70, sigmoid=True, bias=True)
 
 
+@pytest.mark.parametrize("H,G,n", [(64, 1, 128), (128, 2, 40)])
+def test_wide_rows_of_eight_pages_and_nine(H, G, n):
+    """Where 64 heads share a page, rows of up to eight pages are one workgroup's, longer ones two's; a window's pages count."""
+    seqs = [(256, 1), (257, 1), (224, 1), (288, 1), (289, 1), (255, 2)]
+    seqs += [(40, 0)] * (n - len(seqs))
+    _check(H, G, 576, 512, True, seqs=seqs + [(700, 0)], rising=0.1, bias=True, gate="output")
+    _check(H, G, 576, 512, True, seqs=[(800, 1), (815, 1), (832, 1)] + seqs[3:] + [(1000, 0)], window=650, keep_first=33, softcap=20.0)
+
+
 # Shares of one page and more from fourteen pages to see on
 @pytest.mark.parametrize("kv", [417, 448, 449, 480])
 def test_wide_rows_of_few_pages_in_streams(kv):
