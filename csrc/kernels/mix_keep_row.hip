@@ -78,12 +78,13 @@ struct RowLds {
 }  // namespace
 
 // E = 32 DK, vdim = 16 DV, HC heads to a tile of columns, NW waves; STREAM: pages past the caches.  rep: heads a group;
-// side: rows whose heads the columns hold.
+// side4: rows whose heads the columns hold, one of more than four.
 template <int DK, int DV, int HC, int NW, bool STREAM>
-__global__ __launch_bounds__(64 * NW, 2) void attn_keep_row_kernel(const KeepSplitArgs a, int NA, int rep, int side) {
+__global__ __launch_bounds__(64 * NW, 2) void attn_keep_row_kernel(const KeepSplitArgs a, int NA, int rep, int side4) {
   constexpr int E = 32 * DK, vdim = 16 * DV, NL = 16 / HC, QP = HC == 4 ? 1 : 2, NE = 8 / NL;
   typedef RowLds<DK, DV, HC> L;
   typedef const __attribute__((address_space(4))) int32_t const_i32;
+  const int side = HC == 4 ? side4 : 1;
   // a row's heads lie side by side, as their pages do
   const int64_t t = blockIdx.x / a.G;
   const int g = blockIdx.x - (int)t * a.G;
